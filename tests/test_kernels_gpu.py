@@ -132,6 +132,31 @@ def test_gemm_fma(ops, m, n, k, xd, wd, od):
         close(got, want, 1e-3, 2**-8)
 
 
+# rows and columns around a tile of 64 and the groups of 16 rows; K around the steps of 16, 32 and 64 and fewer
+# steps than groups of waves (4); form 0 is the rule's own choice
+@pytest.mark.parametrize("form", [0, 1, 2, 4])
+@pytest.mark.parametrize("m,n,k", [(1, 16, 4), (2, 3072, 2048), (16, 17, 68), (17, 33, 1028), (33, 1, 20), (63, 65, 132), (64, 128, 64),
+                                   (65, 63, 196), (129, 200, 96), (70, 6400, 36)])
+@pytest.mark.parametrize("xd,wd,od", [
+    (torch.float32, torch.float32, torch.float32),
+    (torch.bfloat16, torch.float32, torch.bfloat16),
+    (torch.float32, torch.bfloat16, torch.float32),
+])
+def test_float32_matrix_core_products(ops, form, m, n, k, xd, wd, od):
+    x = rnd((m, k + 12), xd, 41)[:, 4: 4 + k]  # rows of their own stride, starting off 16 bytes for bfloat16
+    w = rnd((n, k + 4), wd, 42)[:, :k]
+    ops.force_float32_form(form)
+    try:
+        got = ops.gemm_fma(x, w, od)
+    finally:
+        ops.force_float32_form()
+    want = x.double().cpu() @ w.double().cpu().T
+    # float32 sums of k products of about 1: each of at most k / 16 + 16 additions in a row rounds the running sum, of about
+    # sqrt(k), by 2^-24 of itself
+    atol = math.sqrt(k) * math.sqrt(k / 16 + 16) * 2.0**-24 * 8
+    close(got, want, atol, 2.0**-23 if od == torch.float32 else 2.0**-8)
+
+
 def test_gemm_fma_is_true_float32(ops):
     """Inputs that a reduced-precision matrix mode would truncate: 1 + 2^-12 has more
     mantissa bits than bfloat16 (8) or a 10-bit tensor-float mode keep, and every partial

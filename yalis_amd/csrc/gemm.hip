@@ -2,9 +2,9 @@
 //
 // Two kernels:
 //  * gemm_fma: float32 fused multiply-add accumulation for any mix of float32 /
-//    bfloat16 operands and any sizes.  This is the whole true-32-bit path (no matrix
-//    core mode with reduced-precision inputs is used) and the fallback for operands
-//    the matrix-core kernel does not take.
+//    bfloat16 operands and any sizes: what neither the float32 matrix-core kernels
+//    (gemm_f32.hip, which the entry point hands every product they take) nor the
+//    bfloat16 ones can read (sizes or strides that are no multiple of four or eight).
 //  * gemm_mfma_skinny: bfloat16 operands on the gfx950 matrix cores
 //    (v_mfma_f32_16x16x32_bf16), float32 accumulation, for few rows of x (decode and
 //    the output head): the weight is streamed once, straight from memory into the
@@ -89,6 +89,11 @@ static int launch_fma(const void* x, const void* w, void* y, int y_dtype, int M,
   return yk_check_launch("gemm_fma");
 }
 
+// the float32 products on the matrix cores (gemm_f32.hip), where the operands allow them
+bool gemm_f32_takes(const void* x, int x_dtype, const void* w, int w_dtype, int y_dtype, int M, int K, int ldx, int ldw);
+int gemm_f32(const void* x, int x_dtype, const void* w, int w_dtype, void* y, int y_dtype, int M, int N, int K, int ldx, int ldw, int ldy,
+             hipStream_t stream);
+
 extern "C" int yk_gemm_fma(const void* x, int x_dtype, const void* w, int w_dtype, void* y,
                            int y_dtype, int M, int N, int K, int ldx, int ldw, int ldy,
                            hipStream_t stream) {
@@ -96,6 +101,8 @@ extern "C" int yk_gemm_fma(const void* x, int x_dtype, const void* w, int w_dtyp
   YK_REQUIRE(ldx >= K && ldw >= K && ldy >= N, "gemm_fma: leading dimensions too small");
   YK_REQUIRE((M + FT - 1) / FT <= 65535, "gemm_fma: too many rows for one launch");
   if (M == 0) return 0;
+  if (gemm_f32_takes(x, x_dtype, w, w_dtype, y_dtype, M, K, ldx, ldw))
+    return gemm_f32(x, x_dtype, w, w_dtype, y, y_dtype, M, N, K, ldx, ldw, ldy, stream);
   if (x_dtype == YK_F32 && w_dtype == YK_F32) return launch_fma<float, float>(x, w, y, y_dtype, M, N, K, ldx, ldw, ldy, stream);
   if (x_dtype == YK_BF16 && w_dtype == YK_F32) return launch_fma<bf16_t, float>(x, w, y, y_dtype, M, N, K, ldx, ldw, ldy, stream);
   if (x_dtype == YK_F32 && w_dtype == YK_BF16) return launch_fma<float, bf16_t>(x, w, y, y_dtype, M, N, K, ldx, ldw, ldy, stream);

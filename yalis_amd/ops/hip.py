@@ -190,6 +190,7 @@ _SIGNATURES = {
         [_vp, _c_int, _vp, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp],
         _c_int,
     ),
+    "yk_gemm_f32_force": ([_c_int], _c_int),
     "yk_gemm_skinny_splits": ([_c_int, _c_int, _c_int, _c_int], _c_int),
     "yk_gemm_skinny_force": ([_c_int, _c_int, _c_int], _c_int),
     "yk_gemm_skinny_wide": ([_c_int], _c_int),
@@ -782,7 +783,14 @@ class HipOps:
         self._check(self.lib.yk_gemm_tile_force(int(slices)))
         self._answers = {k: v for k, v in self._answers.items() if k[0] != "yk_gemm_tile_splits"}
 
+    def force_float32_form(self, form: int = 0) -> None:
+        """For tests and measurements: the form of float32 products (1: few rows; 2 and 4: tiles with that many
+        groups of waves; 0: the library decides)."""
+        self._check(self.lib.yk_gemm_f32_force(int(form)))
+
     def gemm_fma(self, x, w, out_dtype):
+        """x [M, K] . w [N, K]^T with float32 arithmetic, for any types and sizes: on the float32 matrix cores where
+        an operand is float32 and rows can be read four elements at a time, else by multiply-adds."""
         m, k = x.shape
         n = w.shape[0]
         y = torch.empty((m, n), dtype=out_dtype, device=x.device)
