@@ -670,6 +670,18 @@ def _attention_case(ops, dtype, h, g, d, page, spans, window, seed, poison=True,
 SPANS = [(0, 5), (17, 1), (0, 70), (63, 2), (100, 1), (31, 34), (0, 1)]
 
 
+# enough (token, head)s for the form that makes four, two or one head a wave; windows that start inside a group of four keys
+@pytest.mark.parametrize("h,g,d,page", [(48, 12, 16, 16), (40, 20, 80, 64), (45, 15, 32, 16), (40, 5, 256, 32)])
+@pytest.mark.parametrize("window", [0, 3, 66])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_attention_generic_many_tokens(ops, h, g, d, page, window, dtype):
+    got, want = _attention_case(ops, dtype, h, g, d, page, SPANS, window, 19)
+    if dtype == torch.float32:
+        close(got, want, 2e-5, 1e-5)
+    else:
+        close(got, want, 1e-2, 2**-7)
+
+
 @pytest.mark.parametrize("h,g,d,page", [(4, 2, 16, 16), (4, 1, 32, 32), (6, 3, 48, 16), (5, 5, 80, 64), (2, 1, 256, 16)])
 @pytest.mark.parametrize("window", [0, 24])
 def test_attention_generic_f32(ops, h, g, d, page, window):

@@ -14,7 +14,7 @@
 // values of tokens that do not exist yet, or that lie below a window, are zeroed before they meet a probability.
 //
 // Two kernels:
-//  * attn_generic: one wave per (token, head), float32 arithmetic throughout, any
+//  * attn_generic: a workgroup per (token, head), float32 arithmetic throughout, any
 //    head_dim that is a multiple of 16 up to 256, float32 or bfloat16 storage.  This is
 //    the true-32-bit path and the fallback for head sizes the matrix-core kernel lacks.
 //  * attn_mfma: bfloat16 on the gfx950 matrix cores.  One wave owns 16 "columns": a few
@@ -28,74 +28,171 @@
 #include "common.h"
 
 // ---------------------------------------------------------------------------- generic
-template <typename T>
-__global__ __launch_bounds__(64) void attn_generic_kernel(
+// four elements of a row as float32 (rows of pages start at multiples of 16 elements)
+__device__ __forceinline__ float4 generic_load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 generic_load4(const bf16_t* p) {
+  const uint2 u = *reinterpret_cast<const uint2*>(p);
+  return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u));
+}
+
+// A workgroup of W waves makes HQ heads of one token that share a key/value head; its waves take the
+// blocks of 64 keys by turns and merge at the end.  In a block a lane makes one key's scores, 16 bytes of
+// the key at a time, and then adds the block's values for its own elements of the heads, four keys a load
+// (a page holds four consecutive slots of an element side by side in every layout).  Bound by latency and
+// the count of loads, which are scattered (64 keys' rows, 64 elements' rows): so wide loads, every load
+// for all heads that want it, and many waves.  32 heads of 64 elements over 8 kv heads, float32 (us a
+// layer; before: one wave a head with 4-byte loads): 2 tokens behind 200 and 311 keys 45 -> 12, 511 tokens
+// of two prompts 357 -> 74 (164 with one head a wave).
+template <typename T, int W, int HQ>
+__global__ __launch_bounds__(64 * W) void attn_generic_kernel(
     const T* __restrict__ q, int q_stride, T* __restrict__ out, const T* __restrict__ k_cache,
     const T* __restrict__ v_cache, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ token_seq, const int32_t* __restrict__ block_table, int table_width,
     int page_size, int head_dim, int n_heads, int n_kv, float scale, int window) {
   const bool tiled = cache_is_tiled(sizeof(T) == 2 ? YK_BF16 : YK_F32, head_dim, page_size);
   const size_t slab = static_cast<size_t>(page_size) * head_dim;
-  __shared__ float qs[256];
-  __shared__ float ps[64];
-  __shared__ int pbase[64];  // (page * n_kv + kv_head) per key of the tile
-  __shared__ int poff[64];
-  const int n = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  const int qpk = n_heads / n_kv, g = h / qpk;
+  __shared__ __attribute__((aligned(16))) float qs[HQ][256];
+  __shared__ __attribute__((aligned(16))) float ps[W][HQ][64];
+  __shared__ int2 where[W][16];        // (page * n_kv + kv_head, slot) of every fourth key of a wave's block
+  __shared__ float merged[W][HQ][258];  // a wave's sums, maximum and sum of weights
+  const int n = blockIdx.x, h0 = blockIdx.y * HQ, lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int qpk = n_heads / n_kv, g = h0 / qpk;
   const int pos = positions[n], seq = token_seq[n];
   const int hi = pos + 1;
   const int lo = window > 0 ? max(0, pos - window + 1) : 0;
-  const T* qrow = q + static_cast<size_t>(n) * q_stride + static_cast<size_t>(h) * head_dim;
-  for (int d = lane; d < head_dim; d += 64) qs[d] = to_f32<T>(qrow[d]);
+  const T* qrow = q + static_cast<size_t>(n) * q_stride + static_cast<size_t>(h0) * head_dim;
+  for (int d = threadIdx.x; d < HQ * head_dim; d += 64 * W) qs[d / head_dim][d % head_dim] = to_f32<T>(qrow[d]);
   __syncthreads();
   const int32_t* bt = block_table + static_cast<size_t>(seq) * table_width;
-  float m = -INFINITY, l = 0.f;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int t0 = lo; t0 < hi; t0 += 64) {
+  float m[HQ], l[HQ], acc[HQ][4];
+#pragma unroll
+  for (int e = 0; e < HQ; ++e) {
+    m[e] = -INFINITY;
+    l[e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[e][i] = 0.f;
+  }
+  // blocks start at multiples of 64: four consecutive keys of one lie in one page
+  for (int t0 = (lo / 64 + wave) * 64; t0 < hi; t0 += 64 * W) {
     const int key = t0 + lane;
-    const bool valid = key < hi;
-    float s = -INFINITY;
+    const bool valid = key >= lo && key < hi;
+    float s[HQ];
+#pragma unroll
+    for (int e = 0; e < HQ; ++e) s[e] = -INFINITY;
     int base = 0, off = 0;
     if (valid) {
-      const int page = bt[key / page_size];
+      base = bt[key / page_size] * n_kv + g;
       off = key % page_size;
-      base = page * n_kv + g;
       const T* kp = k_cache + static_cast<size_t>(base) * slab;
-      float dot = 0.f;
-      for (int d = 0; d < head_dim; ++d) dot = fmaf(qs[d], to_f32<T>(kp[cache_k_offset(tiled, page_size, head_dim, off, d)]), dot);
-      s = dot * scale;
+      float4 dot[HQ] = {};
+#pragma unroll 4
+      for (int d = 0; d < head_dim; d += 4) {
+        const float4 k4 = generic_load4(kp + cache_k_offset(tiled, page_size, head_dim, off, d));
+#pragma unroll
+        for (int e = 0; e < HQ; ++e) {
+          const float4 q4 = *reinterpret_cast<const float4*>(&qs[e][d]);
+          dot[e].x = fmaf(q4.x, k4.x, dot[e].x);
+          dot[e].y = fmaf(q4.y, k4.y, dot[e].y);
+          dot[e].z = fmaf(q4.z, k4.z, dot[e].z);
+          dot[e].w = fmaf(q4.w, k4.w, dot[e].w);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < HQ; ++e) s[e] = ((dot[e].x + dot[e].y) + (dot[e].z + dot[e].w)) * scale;
     }
-    const float m_new = fmaxf(m, wave_max(s));  // finite: the tile holds at least one key
-    const float p = valid ? expf(s - m_new) : 0.f;
-    const float alpha = expf(m - m_new);  // 0 on the first tile
-    l = l * alpha + wave_sum(p);
-    m = m_new;
-    __syncthreads();  // the previous tile's ps/pbase are no longer read
-    ps[lane] = p;
-    pbase[lane] = base;
-    poff[lane] = off;
-    __syncthreads();
-    const int count = min(64, hi - t0);
+    __builtin_amdgcn_wave_barrier();  // the block before is done with this wave's lists
+    float alpha[HQ];
+#pragma unroll
+    for (int e = 0; e < HQ; ++e) {
+      const float m_new = fmaxf(m[e], wave_max(s[e]));  // finite: the block holds at least one visible key
+      const float p = valid ? expf(s[e] - m_new) : 0.f;
+      alpha[e] = expf(m[e] - m_new);  // 0 on the first block
+      l[e] = l[e] * alpha[e] + wave_sum(p);
+      m[e] = m_new;
+      ps[wave][e][lane] = p;
+    }
+    // four keys' place is that of any of them that is visible
+    const int first = min(max(t0 + lane / 4 * 4, lo), hi - 1);
+    const int from = __shfl(base, first - t0, 64), slot = __shfl(off, first - t0, 64);
+    if (lane % 4 == 0) where[wave][lane / 4] = make_int2(from, slot & ~3);
+    __builtin_amdgcn_wave_barrier();
+    const int j0 = max(0, lo - t0) / 4, j1 = (min(64, hi - t0) + 3) / 4;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int d = lane + 64 * i;
       if (d < head_dim) {
-        float a = acc[i] * alpha;
-        for (int j = 0; j < count; ++j) {
-          const T* vp = v_cache + static_cast<size_t>(pbase[j]) * slab + cache_v_offset(tiled, page_size, head_dim, poff[j], d);
-          a = fmaf(ps[j], to_f32<T>(*vp), a);
+#pragma unroll
+        for (int e = 0; e < HQ; ++e) acc[e][i] *= alpha[e];
+#pragma unroll 4
+        for (int j = j0; j < j1; ++j) {
+          const int2 at = where[wave][j];
+          float4 v4 = generic_load4(v_cache + static_cast<size_t>(at.x) * slab + cache_v_offset(tiled, page_size, head_dim, at.y, d));
+          const int k0 = t0 + 4 * j;  // what lies in a page beside the visible keys (weight 0) is not to be read as a number
+          v4.x = k0 >= lo && k0 < hi ? v4.x : 0.f;
+          v4.y = k0 + 1 >= lo && k0 + 1 < hi ? v4.y : 0.f;
+          v4.z = k0 + 2 >= lo && k0 + 2 < hi ? v4.z : 0.f;
+          v4.w = k0 + 3 >= lo && k0 + 3 < hi ? v4.w : 0.f;
+#pragma unroll
+          for (int e = 0; e < HQ; ++e) {
+            const float4 p4 = *reinterpret_cast<const float4*>(&ps[wave][e][4 * j]);
+            acc[e][i] = fmaf(p4.w, v4.w, fmaf(p4.z, v4.z, fmaf(p4.y, v4.y, fmaf(p4.x, v4.x, acc[e][i]))));
+          }
         }
-        acc[i] = a;
       }
     }
   }
-  T* orow = out + (static_cast<size_t>(n) * n_heads + h) * head_dim;
-  const float inv = 1.f / l;
+  T* orow = out + (static_cast<size_t>(n) * n_heads + h0) * head_dim;
+  if (W == 1) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = lane + 64 * i;
-    if (d < head_dim) orow[d] = from_f32<T>(acc[i] * inv);
+    for (int e = 0; e < HQ; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int d = lane + 64 * i;
+        if (d < head_dim) orow[e * head_dim + d] = from_f32<T>(acc[e][i] * (1.f / l[e]));
+      }
+    return;
   }
+#pragma unroll
+  for (int e = 0; e < HQ; ++e) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (lane + 64 * i < head_dim) merged[wave][e][lane + 64 * i] = acc[e][i];
+    if (lane == 0) {
+      merged[wave][e][256] = m[e];  // -inf, with a sum of 0, where a wave had no block
+      merged[wave][e][257] = l[e];
+    }
+  }
+  __syncthreads();
+  for (int o = threadIdx.x; o < HQ * head_dim; o += 64 * W) {
+    const int e = o / head_dim, d = o % head_dim;
+    float top = -INFINITY, sum = 0.f, a = 0.f;
+#pragma unroll
+    for (int v = 0; v < W; ++v) top = fmaxf(top, merged[v][e][256]);
+#pragma unroll
+    for (int v = 0; v < W; ++v) {
+      const float weight = expf(merged[v][e][256] - top);
+      sum += weight * merged[v][e][257];
+      a = fmaf(weight, merged[v][e][d], a);
+    }
+    orow[o] = from_f32<T>(a * (1.f / sum));
+  }
+}
+
+// Where the (token, head)s alone fill the GPU several times over, a wave makes up to four heads that
+// share their keys; else (decoded tokens, short portions) eight waves share a head's keys.
+template <typename T>
+static void launch_generic(const T* q, int q_stride, T* out, const T* k_cache, const T* v_cache, const int32_t* positions,
+                           const int32_t* token_seq, const int32_t* block_table, int table_width, int n_tokens, int page_size, int head_dim,
+                           int n_heads, int n_kv, float scale, int window, hipStream_t stream) {
+  const int qpk = n_heads / n_kv;
+  auto with = [&](auto kernel, int waves, int heads) {
+    kernel<<<dim3(n_tokens, n_heads / heads), 64 * waves, 0, stream>>>(q, q_stride, out, k_cache, v_cache, positions, token_seq, block_table,
+                                                                       table_width, page_size, head_dim, n_heads, n_kv, scale, window);
+  };
+  if (static_cast<long long>(n_tokens) * n_heads < 4096) return with(attn_generic_kernel<T, 8, 1>, 8, 1);
+  if (qpk % 4 == 0) return with(attn_generic_kernel<T, 1, 4>, 1, 4);
+  if (qpk % 2 == 0) return with(attn_generic_kernel<T, 1, 2>, 1, 2);
+  with(attn_generic_kernel<T, 1, 1>, 1, 1);
 }
 
 extern "C" int yk_attn_generic(const void* q, int q_stride, void* out, const void* k_cache,
@@ -112,17 +209,14 @@ extern "C" int yk_attn_generic(const void* q, int q_stride, void* out, const voi
   YK_REQUIRE(n_heads <= 65535, "attention: too many heads for one launch");
   YK_REQUIRE(window >= 0, "attention: window must not be negative");
   if (n_tokens == 0) return 0;
-  dim3 grid(n_tokens, n_heads), block(64);
   if (dtype == YK_F32)
-    attn_generic_kernel<float><<<grid, block, 0, stream>>>(
-        static_cast<const float*>(q), q_stride, static_cast<float*>(out),
-        static_cast<const float*>(k_cache), static_cast<const float*>(v_cache), positions,
-        token_seq, block_table, table_width, page_size, head_dim, n_heads, n_kv, scale, window);
+    launch_generic(static_cast<const float*>(q), q_stride, static_cast<float*>(out), static_cast<const float*>(k_cache),
+                   static_cast<const float*>(v_cache), positions, token_seq, block_table, table_width, n_tokens, page_size, head_dim, n_heads,
+                   n_kv, scale, window, stream);
   else if (dtype == YK_BF16)
-    attn_generic_kernel<bf16_t><<<grid, block, 0, stream>>>(
-        static_cast<const bf16_t*>(q), q_stride, static_cast<bf16_t*>(out),
-        static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), positions,
-        token_seq, block_table, table_width, page_size, head_dim, n_heads, n_kv, scale, window);
+    launch_generic(static_cast<const bf16_t*>(q), q_stride, static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache),
+                   static_cast<const bf16_t*>(v_cache), positions, token_seq, block_table, table_width, n_tokens, page_size, head_dim, n_heads,
+                   n_kv, scale, window, stream);
   else
     return yk_fail("attention: unsupported dtype");
   return yk_check_launch("attn_generic");
