@@ -509,15 +509,23 @@ extern "C" int yk_latent_attention(const float* q_lat, const void* pages, int dt
 // take their first operand from memory as it lies there, 16 bytes a lane:
 //   S^T = K . Q^T   (first operand: 16 page rows x 32 elements; second: the queries, in registers)
 //   O^T = C^T . P^T (first operand: 16 latent columns x 32 slots of the transposed pages)
-// A wave owns 16 columns = (token, head) pairs of one tile: the heads of a token (16 at a time), or
-// several tokens' heads where a model has fewer than 16.  It walks the keys in groups of 32; within
-// a group the rows of the two score products are assigned to keys so that afterwards lane group g
-// holds the probabilities of keys 8g .. 8g + 7 in order (row i is key 8 (i / 4) + i % 4, + 4 for the
-// second product), which is the second operand of the other product as it stands.  Each lane keeps
-// its column's running maximum and sum.  The four waves of a workgroup take four tiles that follow
-// each other, so they ask for the same rows at about the same time.  With n_splits > 1 the groups of
-// keys are divided among gridDim.z workgroups, which leave unnormalised sums, maxima and sums of
-// weights for a merging kernel.
+// A workgroup owns the 64 columns = (token, head) pairs of one tile, 16 to every pair of its eight
+// waves: up to 64 heads of a token, or several tokens' heads where a model has fewer.  It walks the keys
+// in groups of 32, whose page rows and transposed latents it parks in LDS once for all waves, so memory
+// is asked for a key once per 64 columns.  The waves of a pair divide a group's work: each makes the
+// scores of 16 keys, both read all 32 of them back (float32, through LDS) and take the same softmax
+// step, and each makes the sums of one half of the latent; so a wave needs half the registers and every
+// SIMD has two waves.  The walk is skewed by a group: between two barriers a wave makes the next group's
+// scores and finishes this one's, while the loads of the rows after next and the latents after these
+// are in flight in registers.  Lane group g takes the probabilities of keys 8g .. 8g + 7 of its column:
+// the second operand of the other product as it stands.  Each lane keeps its column's running maximum
+// and sum.  With n_splits > 1 the groups of keys are divided among gridDim.z workgroups, which leave
+// unnormalised sums, maxima and sums of weights for a merging kernel.
+// Bound by the LDS reads (a group of rows of 576 and latents of 512 is read four times over, 272 KiB).
+// Before (every wave walking the pages on its own, its loads not staged) / this, 16 heads, rows of 576
+// (us): a prompt of 2,048 tokens 580 / 195, 512 tokens behind 1,536 525 / 103, eight decoded tokens behind 100 keys 42 /
+// 15, behind 1,000 46 / 18, behind 4,000 63 / 30.
+constexpr int kLatCols = 64;  // columns of a workgroup
 typedef __bf16 lat_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float lat_f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t lat_u32x4_t __attribute__((ext_vector_type(4)));
@@ -527,23 +535,61 @@ union LatFrag {
   bf16_t h[8];
 };
 
+// N products that each take a piece from LDS: the pieces are read four at a time, the next four asked
+// for before these four are used (left alone the compiler keeps one read in flight, and a wave waits for
+// the LDS at every product)
+template <int N, typename Read, typename Use>
+__device__ __forceinline__ void lat_read_ahead(Read read, Use use) {
+  constexpr int B = 4;
+  LatFrag f[2][B];
+#pragma unroll
+  for (int j = 0; j < B && j < N; ++j) f[0][j].u = read(j);
+#pragma unroll
+  for (int base = 0; base < N; base += B) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < B; ++j)
+      if (base + B + j < N) f[(base / B + 1) % 2][j].u = read(base + B + j);
+#pragma unroll
+    for (int j = 0; j < B; ++j)
+      if (base + j < N) use(base + j, f[base / B % 2][j]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 template <int KS, int CT>
-__global__ __launch_bounds__(256, 1) void latent_attention_mfma_kernel(
+constexpr size_t lat_lds_bytes() {  // two buffers each of rows, latents and scores
+  return 2 * ((32 * (32 * KS + 8) + 16 * CT * 32) * sizeof(bf16_t) + 4 * 16 * 36 * sizeof(float));
+}
+
+template <int KS, int CT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_attention_mfma_kernel(
     const float* __restrict__ q_lat, const bf16_t* __restrict__ kpages, const bf16_t* __restrict__ vpages,
-    const int32_t* __restrict__ tiles, int n_tiles, const int32_t* __restrict__ block_table, int table_width, int page_size,
+    const int32_t* __restrict__ tiles, const int32_t* __restrict__ block_table, int table_width, int page_size,
     int n_heads, float scale_log2, int n_splits, const float* __restrict__ sink, float* __restrict__ out, float* __restrict__ ws_o,
     float* __restrict__ ws_ml) {
-  constexpr int WIDTH = 32 * KS, RANK = 16 * CT;
+  constexpr int WIDTH = 32 * KS, RANK = 16 * CT, HALF = CT / 2;
+  // LDS: rows 16 bytes longer than their elements, latents' four pieces of 16 bytes turned by their
+  // column's number, scores in rows of 36: 16 lanes that read a piece of neighbouring rows meet different banks
+  constexpr int KROW = WIDTH + 8, SROW = 36;
+  constexpr int KP = 32 * WIDTH / 8, VP = RANK * 4;  // 16-byte pieces of a group: page rows, transposed latents
+  constexpr int KN = (KP + 511) / 512, VN = (VP + 511) / 512;
+  extern __shared__ __attribute__((aligned(16))) bf16_t lat_lds[];
+  auto kbuf = [&](int b) { return lat_lds + b * (32 * KROW); };
+  auto vbuf = [&](int b) { return lat_lds + 2 * 32 * KROW + b * (RANK * 32); };
+  float* sbase = reinterpret_cast<float*>(lat_lds + 2 * 32 * KROW + 2 * RANK * 32);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
-  const int tile_i = blockIdx.x * 4 + wave;
-  if (tile_i >= n_tiles) return;
+  const int pair = wave / 2, half = wave % 2;
+  auto sbuf = [&](int b) { return sbase + (b * 4 + pair) * (16 * SROW); };
+  const int tile_i = blockIdx.x;
   const int r = lane % 16, g = lane / 16;
   const int32_t* tile = tiles + 4 * tile_i;
   const int seq = tile[0], tok0 = tile[1], count = tile[2], pos0 = tile[3];
   const int chunk = blockIdx.y, split = blockIdx.z;
-  const int hpt = n_heads < 16 ? n_heads : 16;
-  const int tt = r / hpt, hh = r % hpt, head = chunk * 16 + hh;
+  const int hpt = n_heads < kLatCols ? n_heads : kLatCols;
+  const int col = 16 * pair + r, tt = col / hpt, hh = col % hpt, head = chunk * kLatCols + hh;
   const bool col_ok = tt < count && head < n_heads;
+  const bool wave_ok = 16 * pair < count * hpt;  // (a pair without columns only helps to park)
   const int my_pos = pos0 + (col_ok ? tt : 0);
   const int last = pos0 + count - 1;
 
@@ -565,91 +611,149 @@ __global__ __launch_bounds__(256, 1) void latent_attention_mfma_kernel(
   const int32_t* bt = block_table + static_cast<size_t>(seq) * table_width;
 
   float m = -INFINITY, l = 0.f;
-  lat_f32x4_t acc[CT];
+  lat_f32x4_t acc[HALF];
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) acc[ct] = lat_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int ct = 0; ct < HALF; ++ct) acc[ct] = lat_f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  for (int grp = g_lo; grp < g_hi; ++grp) {
+  lat_u32x4_t kreg[KN], vreg[VN];
+  auto page_of = [&](int grp) { return static_cast<size_t>(bt[grp * 32 / page_size]); };
+  // (a uniform base and a 32-bit offset in bytes: one register an address)
+  auto fetch_k = [&](int grp) {
     const int k0 = grp * 32;
-    const size_t page = static_cast<size_t>(bt[k0 / page_size]);
-    const int slot0 = k0 % page_size;
-    lat_f32x4_t s[2];
+    const char* kp = reinterpret_cast<const char*>(kpages + (page_of(grp) * page_size + k0 % page_size) * WIDTH);
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb) {
-      s[sb] = lat_f32x4_t{0.f, 0.f, 0.f, 0.f};
-      // the page row behind row r of this product (rows that do not exist yet: the last one that does)
-      const int kl = min(8 * (r / 4) + 4 * sb + r % 4, last - k0);
-      const bf16_t* krow = kpages + (page * page_size + slot0 + kl) * WIDTH + 8 * g;
+    for (int i = 0; i < KN; ++i) {
+      const uint32_t e = threadIdx.x + 512 * i;  // rows that do not exist yet: the last one that does
+      if (KP % 512 == 0 || e < KP)
+        kreg[i] = *reinterpret_cast<const lat_u32x4_t*>(kp + (min(e / (WIDTH / 8), static_cast<uint32_t>(last - k0)) * (WIDTH * 2) + e % (WIDTH / 8) * 16));
+    }
+  };
+  auto park_k = [&](int b) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        LatFrag kf;
-        kf.u = *reinterpret_cast<const lat_u32x4_t*>(krow + 32 * ks);
-        s[sb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.v, qf[ks].v, s[sb], 0, 0, 0);
+    for (int i = 0; i < KN; ++i) {
+      const int e = threadIdx.x + 512 * i;
+      if (KP % 512 == 0 || e < KP) *reinterpret_cast<lat_u32x4_t*>(kbuf(b) + e / (WIDTH / 8) * KROW + e % (WIDTH / 8) * 8) = kreg[i];
+    }
+  };
+  const uint32_t v_row = 2 * page_size;
+  auto fetch_v = [&](int grp) {
+    const char* vp = reinterpret_cast<const char*>(vpages + page_of(grp) * RANK * page_size + grp * 32 % page_size);
+#pragma unroll
+    for (int i = 0; i < VN; ++i) {
+      const uint32_t e = threadIdx.x + 512 * i;
+      if (VP % 512 == 0 || e < VP) vreg[i] = *reinterpret_cast<const lat_u32x4_t*>(vp + (e / 4 * v_row + e % 4 * 16));
+    }
+  };
+  auto park_v = [&](int b, int grp) {
+    const int key_max = last - grp * 32;
+#pragma unroll
+    for (int i = 0; i < VN; ++i) {
+      const int e = threadIdx.x + 512 * i;
+      if (VP % 512 == 0 || e < VP) {
+        LatFrag f;
+        f.u = vreg[i];
+        if (key_max < 31) {  // slots behind the last key hold whatever was there
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (e % 4 * 8 + j > key_max) f.h[j] = 0;
+        }
+        *reinterpret_cast<lat_u32x4_t*>(vbuf(b) + e / 4 * 32 + ((e % 4) ^ (e / 16 % 4)) * 8) = f.u;
       }
     }
-    // this lane: column r, keys k0 + 8 g + 4 sb + j
-    float tmax = -INFINITY;
+  };
+  // this wave's 16 keys of a group against its columns: lane (r, g) gets column r, keys 16 half + 4 g .. + 3
+  auto scores = [&](int b, int grp) {
+    const bf16_t* krow = kbuf(b) + (16 * half + r) * KROW + 8 * g;
+    lat_f32x4_t s0 = {0.f, 0.f, 0.f, 0.f};
+    lat_read_ahead<KS>([&](int ks) { return *reinterpret_cast<const lat_u32x4_t*>(krow + 32 * ks); },
+                       [&](int ks, const LatFrag& kf) { s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.v, qf[ks].v, s0, 0, 0, 0); });
+    const int key = grp * 32 + 16 * half + 4 * g;
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int key = k0 + 8 * g + 4 * sb + j;
-        s[sb][j] = key <= my_pos ? s[sb][j] * scale_log2 : -INFINITY;
-        tmax = fmaxf(tmax, s[sb][j]);
-      }
-    tmax = column_lanes_max(tmax);
-    const float m_new = fmaxf(m, tmax);
-    const float m_safe = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f(m - m_safe);
-    float psum = 0.f;
-    LatFrag pf;
-#pragma unroll
-    for (int sb = 0; sb < 2; ++sb) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        s[sb][j] = __builtin_amdgcn_exp2f(s[sb][j] - m_safe);
-        psum += s[sb][j];
-      }
-      pf.u[2 * sb] = pack_bf16x2(s[sb][0], s[sb][1]);
-      pf.u[2 * sb + 1] = pack_bf16x2(s[sb][2], s[sb][3]);
-    }
-    l = l * alpha + psum;
-    m = m_new;
-    const bool ragged = k0 + 32 > last + 1;  // slots behind the last key hold whatever was there
-    const bf16_t* vcol = vpages + (page * RANK + r) * page_size + slot0 + 8 * g;
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-      LatFrag vf;
-      vf.u = *reinterpret_cast<const lat_u32x4_t*>(vcol + static_cast<size_t>(16 * ct) * page_size);
-      if (ragged) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (k0 + 8 * g + e > last) vf.h[e] = 0;
-      }
-      acc[ct] *= alpha;
-      acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, acc[ct], 0, 0, 0);
-    }
+    for (int j = 0; j < 4; ++j) s0[j] = key + j <= my_pos ? s0[j] * scale_log2 : -INFINITY;
+    *reinterpret_cast<lat_f32x4_t*>(sbuf(b) + r * SROW + 16 * half + 4 * g) = s0;
+  };
+  // (nothing in the walk is conditional: behind the last group it fetches, parks and scores that group again, unread)
+  const int g_end = g_hi - 1;
+  if (g_lo < g_hi) {
+    fetch_k(g_lo);
+    fetch_v(g_lo);
+    park_k(0);
+    park_v(0, g_lo);
+    fetch_k(min(g_lo + 1, g_end));
+    __syncthreads();
+    if (wave_ok) scores(0, g_lo);
+    park_k(1);
   }
+  for (int grp = g_lo; grp < g_hi; ++grp) {
+    const int b = (grp - g_lo) & 1;
+    fetch_k(min(grp + 2, g_end));
+    fetch_v(min(grp + 1, g_end));
+    // the rows of the next group, the latents and scores of this one are parked, and every wave is done with what is
+    // written below: the rows and latents of this group's and the next one's buffers as they were two groups ago
+    __syncthreads();
+    if (wave_ok) {
+      scores(b ^ 1, grp + 1);
+      // this lane: column r, keys 8 g .. 8 g + 7 of the group
+      lat_f32x4_t s[2];
+      s[0] = *reinterpret_cast<const lat_f32x4_t*>(sbuf(b) + r * SROW + 8 * g);
+      s[1] = *reinterpret_cast<const lat_f32x4_t*>(sbuf(b) + r * SROW + 8 * g + 4);
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) tmax = fmaxf(tmax, s[sb][j]);
+      tmax = column_lanes_max(tmax);
+      const float m_new = fmaxf(m, tmax);
+      const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f(m - m_safe);
+      float psum = 0.f;
+      LatFrag pf;
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          s[sb][j] = __builtin_amdgcn_exp2f(s[sb][j] - m_safe);
+          psum += s[sb][j];
+        }
+        pf.u[2 * sb] = pack_bf16x2(s[sb][0], s[sb][1]);
+        pf.u[2 * sb + 1] = pack_bf16x2(s[sb][2], s[sb][3]);
+      }
+      const bool grew = m_new > m;
+      l = l * alpha + psum;
+      m = m_new;
+      if (__any(grew)) {
+        asm volatile("" ::: "memory");  // (a branch, not a multiplication and a select per element)
+#pragma unroll
+        for (int ct = 0; ct < HALF; ++ct) acc[ct] *= alpha;
+      }
+      const bf16_t* vcol = vbuf(b) + (16 * HALF * half + r) * 32 + (g ^ (r / 4)) * 8;
+      lat_read_ahead<HALF>([&](int ct) { return *reinterpret_cast<const lat_u32x4_t*>(vcol + 16 * ct * 32); },
+                           [&](int ct, const LatFrag& vf) { acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, acc[ct], 0, 0, 0); });
+    }
+    park_k(b);
+    park_v(b ^ 1, min(grp + 1, g_end));
+  }
+  if (!col_ok && !__any(col_ok)) return;  // (uniform: the sum below exchanges lanes)
   l = column_lanes_sum(l);
-  // acc[ct][j]: latent column 16 ct + 4 g + j of this lane's column r
+  if (!col_ok) return;
+  // acc[ct][j]: latent column 16 (HALF half + ct) + 4 g + j of this lane's column r
   if (n_splits == 1) {
-    if (!col_ok) return;
     // the sink joins the sum of weights at the end (every column has seen a key: m is finite)
     if (sink != nullptr) l += __builtin_amdgcn_exp2f(sink[head] * 1.4426950408889634f - m);
     const float inv = 1.f / l;
-    float* o = out + (static_cast<size_t>(tok0 + tt) * n_heads + head) * RANK + 4 * g;
+    float* o = out + (static_cast<size_t>(tok0 + tt) * n_heads + head) * RANK + 16 * HALF * half + 4 * g;
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
+    for (int ct = 0; ct < HALF; ++ct)
       *reinterpret_cast<float4*>(o + 16 * ct) = make_float4(acc[ct][0] * inv, acc[ct][1] * inv, acc[ct][2] * inv, acc[ct][3] * inv);
     return;
   }
   const size_t part = (static_cast<size_t>(tile_i) * gridDim.y + chunk) * n_splits + split;
-  float* o = ws_o + (part * 16 + r) * RANK + 4 * g;
+  float* o = ws_o + (part * kLatCols + col) * RANK + 16 * HALF * half + 4 * g;
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) *reinterpret_cast<float4*>(o + 16 * ct) = make_float4(acc[ct][0], acc[ct][1], acc[ct][2], acc[ct][3]);
-  if (g == 0) {
-    ws_ml[(part * 16 + r) * 2] = m;
-    ws_ml[(part * 16 + r) * 2 + 1] = l;
+  for (int ct = 0; ct < HALF; ++ct) *reinterpret_cast<float4*>(o + 16 * ct) = make_float4(acc[ct][0], acc[ct][1], acc[ct][2], acc[ct][3]);
+  if (g == 0 && half == 0) {
+    ws_ml[(part * kLatCols + col) * 2] = m;
+    ws_ml[(part * kLatCols + col) * 2 + 1] = l;
   }
 }
 
@@ -665,19 +769,19 @@ __global__ __launch_bounds__(128) void latent_attention_merge_kernel(const float
   const int tile_i = blockIdx.x, chunk = blockIdx.y, r = blockIdx.z;
   const int32_t* tile = tiles + 4 * tile_i;
   const int tok0 = tile[1], count = tile[2];
-  const int hpt = n_heads < 16 ? n_heads : 16;
-  const int tt = r / hpt, head = chunk * 16 + r % hpt;
+  const int hpt = n_heads < kLatCols ? n_heads : kLatCols;
+  const int tt = r / hpt, head = chunk * kLatCols + r % hpt;
   if (tt >= count || head >= n_heads) return;
   const size_t part0 = (static_cast<size_t>(tile_i) * gridDim.y + chunk) * n_splits;
   if (threadIdx.x < kWave) {
     float m_max = -INFINITY;
-    for (int s = threadIdx.x; s < n_splits; s += kWave) m_max = fmaxf(m_max, ws_ml[((part0 + s) * 16 + r) * 2]);
+    for (int s = threadIdx.x; s < n_splits; s += kWave) m_max = fmaxf(m_max, ws_ml[((part0 + s) * kLatCols + r) * 2]);
     m_max = wave_max(m_max);
     float den = 0.f;
     for (int s = threadIdx.x; s < n_splits; s += kWave) {
-      const float ws = exp2f(ws_ml[((part0 + s) * 16 + r) * 2] - m_max);
+      const float ws = exp2f(ws_ml[((part0 + s) * kLatCols + r) * 2] - m_max);
       w[s] = ws;
-      den = fmaf(ws, ws_ml[((part0 + s) * 16 + r) * 2 + 1], den);
+      den = fmaf(ws, ws_ml[((part0 + s) * kLatCols + r) * 2 + 1], den);
     }
     den = wave_sum(den);
     if (sink != nullptr) den += exp2f(sink[head] * 1.4426950408889634f - m_max);
@@ -691,7 +795,7 @@ __global__ __launch_bounds__(128) void latent_attention_merge_kernel(const float
       float4 v[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (s0 + j < n_splits) v[j] = *reinterpret_cast<const float4*>(ws_o + ((part0 + s0 + j) * 16 + r) * rank + c);
+        if (s0 + j < n_splits) v[j] = *reinterpret_cast<const float4*>(ws_o + ((part0 + s0 + j) * kLatCols + r) * rank + c);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         if (s0 + j < n_splits) {
@@ -714,13 +818,13 @@ extern "C" int yk_latent_mfma_ok(int kv_rank, int rot_dim, int page_size) {
   return size_ok && page_size % 32 == 0 ? 1 : 0;
 }
 
-extern "C" int yk_latent_mfma_tile_tokens(int n_heads) { return n_heads >= 16 ? 1 : 16 / n_heads; }
+extern "C" int yk_latent_mfma_tile_tokens(int n_heads) { return n_heads >= kLatCols ? 1 : kLatCols / n_heads; }
 
 // floats of workspace a launch with these tiles and splits needs
 extern "C" size_t yk_latent_mfma_workspace(int n_tiles, int n_heads, int kv_rank, int n_splits) {
   if (n_splits <= 1) return 0;
-  const size_t parts = static_cast<size_t>(n_tiles) * ((n_heads + 15) / 16) * n_splits;
-  return parts * 16 * (kv_rank + 2);
+  const size_t parts = static_cast<size_t>(n_tiles) * ((n_heads + kLatCols - 1) / kLatCols) * n_splits;
+  return parts * kLatCols * (kv_rank + 2);
 }
 
 extern "C" int yk_latent_attention_mfma(const float* q_lat, const void* kpages, const void* vpages, const int32_t* tiles,
@@ -732,15 +836,20 @@ extern "C" int yk_latent_attention_mfma(const float* q_lat, const void* kpages, 
   YK_REQUIRE(workspace_floats >= yk_latent_mfma_workspace(n_tiles, n_heads, kv_rank, n_splits) && (n_splits == 1 || workspace != nullptr),
              "latent_attention_mfma: the workspace is too small");
   if (n_tiles == 0) return 0;
-  const int chunks = (n_heads + 15) / 16;
-  dim3 grid((n_tiles + 3) / 4, chunks, n_splits);
+  const int chunks = (n_heads + kLatCols - 1) / kLatCols;
+  dim3 grid(n_tiles, chunks, n_splits);
   const float scale_log2 = scale * 1.4426950408889634f;
   float* ws_o = workspace;
-  float* ws_ml = workspace == nullptr ? nullptr : workspace + static_cast<size_t>(n_tiles) * chunks * n_splits * 16 * kv_rank;
+  float* ws_ml = workspace == nullptr ? nullptr : workspace + static_cast<size_t>(n_tiles) * chunks * n_splits * kLatCols * kv_rank;
 #define YK_CASE(KS, CT)                                                                                                      \
   if (kv_rank + rot_dim == 32 * KS && kv_rank == 16 * CT) {                                                                  \
-    latent_attention_mfma_kernel<KS, CT><<<grid, 256, 0, stream>>>(                                                          \
-        q_lat, static_cast<const bf16_t*>(kpages), static_cast<const bf16_t*>(vpages), tiles, n_tiles, block_table,          \
+    auto kern = latent_attention_mfma_kernel<KS, CT>;                                                                        \
+    constexpr size_t lds = lat_lds_bytes<KS, CT>();                                                                          \
+    if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                               static_cast<int>(lds)) != hipSuccess)                                         \
+      return yk_fail("latent_attention_mfma: the group's buffers do not fit in LDS");                                        \
+    kern<<<grid, 512, lds, stream>>>(                                                                                        \
+        q_lat, static_cast<const bf16_t*>(kpages), static_cast<const bf16_t*>(vpages), tiles, block_table,                   \
         table_width, page_size, n_heads, scale_log2, n_splits, sink, out, ws_o, ws_ml);                                            \
     if (yk_check_launch("latent_attention_mfma") != 0) return -1;                                                            \
   }
@@ -754,7 +863,7 @@ extern "C" int yk_latent_attention_mfma(const float* q_lat, const void* kpages, 
   YK_CASE(2, 4)
 #undef YK_CASE
   if (n_splits > 1) {
-    latent_attention_merge_kernel<<<dim3(n_tiles, chunks, 16), 128, 0, stream>>>(ws_o, ws_ml, tiles, n_heads, kv_rank, n_splits, sink, out);
+    latent_attention_merge_kernel<<<dim3(n_tiles, chunks, kLatCols), 128, 0, stream>>>(ws_o, ws_ml, tiles, n_heads, kv_rank, n_splits, sink, out);
     return yk_check_launch("latent_attention_merge");
   }
   return 0;

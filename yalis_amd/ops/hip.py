@@ -11,6 +11,7 @@ product and everything else are the hand-written kernels.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -1725,11 +1726,22 @@ class HipOps:
         return self._ask("yk_latent_mfma_tile_tokens" if matrix_cores else "yk_latent_tile_tokens", n_heads)
 
     @staticmethod
-    def latent_attention_splits(n_tiles: int, n_heads: int, max_ctx: int) -> int:
-        """Into how many workgroups the matrix-core form divides the keys of a tile: none while the
-        tiles alone make some hundreds of waves; else as many as that takes, each with at least 128 keys."""
-        waves = n_tiles * -(-n_heads // 16)
-        return max(1, min(-(-512 // max(waves, 1)), max(1, -(-max_ctx // 32) // 4), 64))
+    @functools.lru_cache(maxsize=4096)
+    def latent_attention_splits(n_tiles: int, n_heads: int, max_ctx: int, n_tokens: int = 0, kv_rank: int = 512) -> int:
+        """Into how many workgroups the matrix-core form divides the keys of a tile: the power of two with the
+        smallest estimate of the longest tile's walk (0.5 us a group of 32 keys and 0.9 with a latent of 512, twice as
+        long where a compute unit has two workgroups to run) and, where the keys are divided, of the merge (5 us and the partial sums written
+        and read once).  Measured (us, 16 heads, rows of 576): eight decoded tokens behind 1,000 keys whole / in 4 / 8 /
+        16 51.5 / 24.0 / 19.0 / 17.6, behind 4,000 in 16 / 32 38 / 30; 64 behind 500 whole / in 2 / 4 / 8 35 / 29.5 /
+        29.6 / 41.8; 512 tokens behind 1,536 whole / in two 147 / 103; four prompts of 200 whole / in two 36 / 62."""
+        workgroups = n_tiles * -(-n_heads // 64)
+        groups = -(-max_ctx // 32)
+
+        def estimate(s: int) -> float:
+            walk = -(-groups // s) * (0.5 + 0.9 * kv_rank / 512) * max(1.0, workgroups * s / 256)
+            return walk if s == 1 else walk + 5.0 + max(n_tokens, n_tiles) * n_heads * s * kv_rank * 8 / 4e6
+
+        return min((s for s in (1, 2, 4, 8, 16, 32, 64) if s <= max(groups, 1)), key=estimate)
 
     def latent_attention(self, q_lat, pages, n_heads, kv_rank, rot_dim, scale, ctx, group, page_size, tiles=None, values=None,
                          splits: Optional[int] = None, sink=None) -> torch.Tensor:
@@ -1756,7 +1768,7 @@ class HipOps:
                     or values.dtype != pages.dtype or tuple(values.shape) != (pages.shape[0], 1, kv_rank, page_size):
                 raise KernelError("latent_attention: transposed pages are for the matrix-core form, with tiles cut for it")
             if splits is None:  # (given: tests and measurements force a number)
-                splits = self.latent_attention_splits(tiles.shape[0], n_heads, int(ctx.max_ctx))
+                splits = self.latent_attention_splits(tiles.shape[0], n_heads, int(ctx.max_ctx), n, kv_rank)
             floats = self.lib.yk_latent_mfma_workspace(tiles.shape[0], n_heads, kv_rank, splits)
             ws = self._ws(floats) if floats else None
             self._check(self.lib.yk_latent_attention_mfma(
