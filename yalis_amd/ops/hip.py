@@ -164,6 +164,12 @@ _SIGNATURES = {
          _c_int, _vp, _vp, _c_float, _vp, _c_int, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp],
         _c_int,
     ),
+    "yk_state_scan_chunks_floats": ([_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int], _c_size_t),
+    "yk_state_scan_chunks": (
+        [_vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_float, _c_float, _c_int, _vp, _c_int,
+         _c_int, _vp, _vp, _c_float, _vp, _c_int, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _c_size_t, _vp],
+        _c_int,
+    ),
     "yk_gated_head_norm": (
         [_vp, _vp, _c_int, _c_float, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp],
         _c_int,
@@ -1793,8 +1799,15 @@ class HipOps:
             x.data_ptr(), x.stride(0), _code(x.dtype), state.data_ptr(), a["seq_qstart"].data_ptr(), a["seq_qlen"].data_ptr(),
             a["state_slots"].data_ptr(), a["seq_qstart"].numel(), state.shape[1], channels, self._stream()))
 
+    # Steps whose spans meet chunk by chunk: one of 256 tokens at least (one span of 256, 16 heads of 128 x 128: 47 us against 62
+    # token by token, of 160: 42 against 41), and 128 tokens a request on average, since a request of one token costs a whole chunk (512 tokens
+    # with 16 requests of one: 186 against 170; 8 of 256: 108 against 151).
+    STATE_CHUNKS_MIN_SPAN, STATE_CHUNKS_MIN_AVERAGE = 256, 128
+    # scratch for what the chunks of a step's spans are worked into (15,000 tokens of 16 heads; beyond that heads are taken by turns)
+    STATE_CHUNKS_BYTES = 512 << 20
+
     def linear_state_scan(self, qkv, n_heads, n_kv, dim, vdim, state, ctx, q_scale=1.0, unit_eps=None, decay=None, beta=None,
-                          columns=None, skip=None, bonus=None):
+                          columns=None, skip=None, bonus=None, form: Optional[str] = None):
         """The recurrence S <- diag(a) S; u = v or beta (v - S^T k); S += k u^T; o = S^T q over each
         request's span, S [slots, heads, dim, vdim] float32 updated in place.  ``qkv`` [N, >= 2 * kv_heads *
         dim + heads * vdim]: columns [q | k | v].  ``unit_eps``: q and k are divided by sqrt(sum of squares +
@@ -1807,6 +1820,8 @@ class HipOps:
         decay.  ``columns`` = (q, k, v): where the kv heads' queries and keys and the heads' values start in a row
         (default 0, n_kv * dim, 2 * n_kv * dim).  ``skip`` (float32 [heads]): o += skip_h v.  ``bonus`` (float32
         [heads, dim], plain writes): o = (S + diag(bonus) k v^T)^T q of the memory before the token's decay and write.
+        Steps of long spans are taken by chunks of 64 tokens in matrix products where sizes and alignment allow
+        (``STATE_CHUNKS_MIN_SPAN``); all others are walked token by token.  ``form`` ("chunks", "walk") forces one of them (tests).
         Returns o float32 [N, heads * vdim]."""
         self._rows(qkv, "linear_state_scan input")
         n = qkv.shape[0]
@@ -1851,10 +1866,28 @@ class HipOps:
         a = ctx.arrays
         mode = {"head": 0, "channel": 1, "channel_softplus": 2, "channel_exp": 3, "fixed": 4}[kind]
         beta_f32 = beta is not None and beta[0].dtype == torch.float32
+        out = torch.empty((n, n_heads * vdim), dtype=torch.float32, device=qkv.device)
+        n_seqs, max_qlen, a_head = a["seq_qstart"].numel(), getattr(ctx, "max_qlen", 0), 0
+        aligned = qkv.stride(0) % 8 == 0 and q_col % 8 == 0 and k_col % 8 == 0 and qkv.data_ptr() % 16 == 0
+        long = max_qlen >= self.STATE_CHUNKS_MIN_SPAN and n >= self.STATE_CHUNKS_MIN_AVERAGE * n_seqs
+        if aligned and (form == "chunks" or (form is None and long)):
+            a_head = self.lib.yk_state_scan_chunks_floats(n, n_seqs, dim, vdim, mode, write_mode, int(bonus is not None), int(skip is not None))
+        if form == "chunks" and not a_head:
+            raise KernelError("linear_state_scan: this step cannot be taken chunk by chunk")
+        if a_head and (form == "chunks" or 4 * a_head <= self.STATE_CHUNKS_BYTES):
+            heads = max(1, min(n_heads, self.STATE_CHUNKS_BYTES // (4 * a_head)))
+            ws = torch.empty(heads * a_head, dtype=torch.float32, device=qkv.device)
+            self._check(self.lib.yk_state_scan_chunks(
+                qkv.data_ptr(), qkv.stride(0), _code(qkv.dtype), n_heads, n_kv, dim, vdim, state.data_ptr(), a["seq_qstart"].data_ptr(),
+                a["seq_qlen"].data_ptr(), a["state_slots"].data_ptr(), n_seqs, n, max_qlen, float(q_scale),
+                -1.0 if unit_eps is None else float(unit_eps), mode, src.data_ptr(), src.stride(0), col, p0.data_ptr(), _ptr(p1), tau,
+                beta[0].data_ptr() if beta_f32 else None, 0 if beta is None else beta[0].stride(0), 0 if beta is None else int(beta[1]),
+                out.data_ptr(), int(q_col), int(k_col), int(v_col), write_mode, _ptr(skip),
+                beta[0].data_ptr() if beta is not None and not beta_f32 else None, _ptr(bonus), ws.data_ptr(), ws.numel(), self._stream()))
+            return out
         # where tokens are many their decays per channel are made first, once for all the columns that read them
         many = mode not in (0, 4) and n > 4 * a["seq_qstart"].numel()
         decays = torch.empty((n, n_heads * dim), dtype=torch.float32, device=qkv.device) if many else None
-        out = torch.empty((n, n_heads * vdim), dtype=torch.float32, device=qkv.device)
         self._check(self.lib.yk_linear_state_scan(
             qkv.data_ptr(), qkv.stride(0), _code(qkv.dtype), n_heads, n_kv, dim, vdim, state.data_ptr(), a["seq_qstart"].data_ptr(),
             a["seq_qlen"].data_ptr(), a["state_slots"].data_ptr(), a["seq_qstart"].numel(), n, float(q_scale),
