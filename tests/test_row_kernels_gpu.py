@@ -1,0 +1,54 @@
+"""Norms and activations whose threads hold one or two pieces of a row, at rows that do not fill their threads."""
+import pytest
+import torch
+
+import kernel_refs as R
+from yalis_amd.ops.hip import HipOps
+
+pytestmark = pytest.mark.gpu
+_ops = {}
+
+
+def ops():
+    if "o" not in _ops:
+        _ops["o"] = HipOps("cuda:0")
+    return _ops["o"]
+
+
+def close(got, want, tol):
+    err = (got.double().cpu() - want.double()).abs().max().item() / want.double().abs().max().item()
+    assert err <= tol, err
+
+
+@pytest.mark.parametrize("n", [3, 1023, 1024])
+@pytest.mark.parametrize("width", [4, 260, 516, 1028, 2052, 4092, 4096])
+def test_norms_of_few_and_many_rows(n, width):
+    """Float32 rows: a row's sum of squares is added in up to width / 64 + 10 roundings of 2^-24, halved by the root: 4e-6 holds
+    for 4,096; both kernels write every column, and none of the next row's."""
+    o, g = ops(), torch.Generator().manual_seed(width + n)
+    res, br, other = (torch.randn(n, width, generator=g) for _ in range(3))
+    w, w2 = torch.rand(width, generator=g) + 0.5, torch.rand(width, generator=g) + 0.5
+    post, pre = (w, w2, 1e-5, True), (w2, None, 1e-6, False)
+    dev = lambda c: tuple(t.cuda() if torch.is_tensor(t) else t for t in c)
+    r_ref, r_dev = res.clone(), res.clone().cuda()
+    want = R.sandwich_norm(r_ref, br, post, 0.3, pre, None, torch.float32)
+    close(o.sandwich_norm(r_dev, br.cuda(), dev(post), 0.3, dev(pre), None, torch.float32), want, 4e-6)
+    close(r_dev, r_ref, 4e-6)
+    r_ref, r_dev = res.clone(), res.clone().cuda()
+    R.sum_norm(r_ref, [(br, w, 1e-5), (other, w2, 1e-5)], 0.5, None, 2.0, w, 1e-5, True, torch.bfloat16)
+    o.sum_norm(r_dev, [(br.cuda(), w.cuda(), 1e-5), (other.cuda(), w2.cuda(), 1e-5)], 0.5, None, 2.0, w.cuda(), 1e-5, True, torch.bfloat16)
+    close(r_dev, r_ref, 4e-6)
+
+
+@pytest.mark.parametrize("kind", ["relu2", "silu", "gelu_tanh"])
+@pytest.mark.parametrize("shape,shift", [((1, 4), 0), ((3, 1020), 0), ((3, 1021), 0), ((5, 1024), 1)])
+def test_activation_in_pieces(kind, shape, shift):
+    """Whole pieces, a count that is none and rows that are not aligned: within one rounding to bfloat16, NaN where the input is."""
+    o, g = ops(), torch.Generator().manual_seed(shape[1])
+    flat = torch.randn(shape[0] * shape[1] + shift, generator=g).to(torch.bfloat16)
+    if kind != "relu2":  # (whose maximum with 0 drops it)
+        flat[shift] = float("nan")
+    x = flat.cuda()[shift:].view(shape)
+    got, want = o.activation(x, kind, torch.bfloat16).cpu(), R.activation(flat[shift:].view(shape), kind, torch.bfloat16)
+    assert torch.equal(got.isnan(), want.isnan())
+    close(got.nan_to_num().float(), want.nan_to_num().float(), 2 ** -8)
