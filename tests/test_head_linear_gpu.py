@@ -1,0 +1,31 @@
+"""Per-head products of a handful of tokens by pairs of columns, against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+_ops = {}
+
+
+def ops():
+    if "o" not in _ops:
+        from yalis_amd.ops.hip import HipOps
+
+        _ops["o"] = HipOps("cuda:0")
+    return _ops["o"]
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 32, 33])
+@pytest.mark.parametrize("in_dim,out_dim", [(1, 2), (31, 62), (32, 64), (33, 66), (256, 130), (257, 64), (1000, 48), (40, 33), (1500, 20)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_head_products_by_pairs(dtype, in_dim, out_dim, n):
+    """Fewer elements than slices, one more and one less than a round of weights, columns that do not fill a tile, an odd number of
+    columns and heads too long for the pairs' workspace (both one column a thread).  A sum of in_dim products in float32, by slices: within 8
+    roundings (2^-24) of the sum of their sizes."""
+    o, h = ops(), 3
+    g = torch.Generator().manual_seed(in_dim + n)
+    x = torch.randn(n, h * in_dim, generator=g).to(dtype)
+    w = torch.randn(h, in_dim, out_dim, generator=g).to(dtype)
+    got = o.head_linear(x.cuda(), w.cuda(), h, in_dim, out_dim, torch.float32).cpu().double().view(n, h, out_dim)
+    xs, ws = x.double().view(n, h, in_dim).transpose(0, 1).contiguous(), w.double()
+    want, size = (torch.matmul(a, b).transpose(0, 1) for a, b in ((xs, ws), (xs.abs(), ws.abs())))
+    assert ((got - want).abs() <= 8 * 2.0 ** -24 * size).all()

@@ -21,7 +21,7 @@
 
 // --------------------------------------------------------------------------------- prepare
 template <typename T, typename TW>
-__global__ __launch_bounds__(128) void latent_prepare_kernel(
+__global__ __launch_bounds__(512) void latent_prepare_kernel(
     const T* __restrict__ proj, int proj_stride, int q_rank, const TW* __restrict__ q_norm, float eps, T* __restrict__ c_q,
     int kv_col, int kv_rank, int rot_dim, const TW* __restrict__ kv_norm, const int32_t* __restrict__ positions,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, int interleaved, T* __restrict__ pages,
@@ -29,17 +29,18 @@ __global__ __launch_bounds__(128) void latent_prepare_kernel(
   __shared__ float scratch[17];
   const size_t n = blockIdx.x;
   const T* row = proj + n * proj_stride;
-  float ss = 0.f;
-  for (int c = threadIdx.x; c < q_rank; c += blockDim.x) {
-    const float v = to_f32<T>(row[c]);
-    ss = fmaf(v, v, ss);
+  float ss = 0.f, inv;
+  if (blockIdx.y == 0) {
+    for (int c = threadIdx.x; c < q_rank; c += blockDim.x) {
+      const float v = to_f32<T>(row[c]);
+      ss = fmaf(v, v, ss);
+    }
+    inv = 1.f / sqrtf(block_sum(ss, scratch) / static_cast<float>(q_rank) + eps);
+    for (int c = threadIdx.x; c < q_rank; c += blockDim.x)
+      c_q[n * q_rank + c] = from_f32<T>(to_f32<T>(row[c]) * inv * to_f32<TW>(q_norm[c]));
+    return;
   }
-  float inv = 1.f / sqrtf(block_sum(ss, scratch) / static_cast<float>(q_rank) + eps);
-  for (int c = threadIdx.x; c < q_rank; c += blockDim.x)
-    c_q[n * q_rank + c] = from_f32<T>(to_f32<T>(row[c]) * inv * to_f32<TW>(q_norm[c]));
-  if (kv_rank == 0) return;
   const T* kv = row + kv_col;
-  ss = 0.f;
   for (int c = threadIdx.x; c < kv_rank; c += blockDim.x) {
     const float v = to_f32<T>(kv[c]);
     ss = fmaf(v, v, ss);
@@ -80,9 +81,12 @@ extern "C" int yk_latent_prepare(const void* proj, int proj_stride, int dtype, i
   YK_REQUIRE(kv_rank == 0 || rot_dim == 0 || (cos_t != nullptr && sin_t != nullptr && max_positions > 0),
              "latent_prepare: the rotated part needs its tables");
   if (n_tokens == 0) return 0;
+  // queries and cache rows in workgroups of their own, of as many threads as leave one or two rounds of a row to read where tokens are
+  // few (eight tokens of a width of 4,096: 13.0 -> 5.0 us)
+  const int threads = n_tokens < 256 ? 512 : 128;
 #define YK_CASE(D, T, WD, TW)                                                                                         \
   if (dtype == D && w_dtype == WD) {                                                                                  \
-    latent_prepare_kernel<T, TW><<<n_tokens, 128, 0, stream>>>(                                                       \
+    latent_prepare_kernel<T, TW><<<dim3(n_tokens, kv_rank > 0 ? 2 : 1), threads, 0, stream>>>(                                                       \
         static_cast<const T*>(proj), proj_stride, q_rank, static_cast<const TW*>(q_norm), eps, static_cast<T*>(c_q),  \
         kv_col, kv_rank, rot_dim, static_cast<const TW*>(kv_norm), positions, cos_t, sin_t, interleaved,              \
         static_cast<T*>(pages), static_cast<T*>(pages_t), page_size, slots);                                          \
@@ -98,13 +102,12 @@ extern "C" int yk_latent_prepare(const void* proj, int proj_stride, int dtype, i
 // ------------------------------------------------------------------------- per-head products
 constexpr int kHeadTokens = 8;   // tokens a workgroup multiplies by one head's matrix
 constexpr int kHeadOut = 64;     // output columns a workgroup makes
-// SLICES groups of 64 threads divide the input elements among them: four for a handful of tokens (more
-// waves on a product that is all latency), one for many (no meeting in LDS, every weight read once a tile)
+constexpr int kHeadSlices = 4;   // groups of 64 threads that divide the input elements among them
 
 // out[n, h, o] = sum_i x[n, h, i] w[h][i][o] for a tile of kHeadTokens tokens, one head and kHeadOut
 // columns; thread (slice, column) sums every fourth input element, the slices meet in LDS.  TX: the
 // input's and TG the gate's element type.
-template <typename TX, typename TW, typename TG, typename TO, int kHeadSlices>
+template <typename TX, typename TW, typename TG, typename TO>
 __global__ __launch_bounds__(kHeadOut * kHeadSlices) void head_linear_kernel(
     const TX* __restrict__ x, int x_stride, const TW* __restrict__ w, TO* __restrict__ out, int out_stride, int in_dim,
     int out_dim, int tail, const int32_t* __restrict__ positions, const float* __restrict__ cos_t,
@@ -170,6 +173,111 @@ __global__ __launch_bounds__(kHeadOut * kHeadSlices) void head_linear_kernel(
   }
 }
 
+// The same for an even out_dim and a handful of tokens, where the product is all latency: 32 slices of 32 threads, a thread two
+// columns; eight of its weights (of 4 or 8 bytes) are on their way at a time, the first before the input is staged; a token's inputs lie
+// side by side in LDS, so that an input element of all eight tokens is two reads for sixteen multiplications.  Eight tokens of 32 heads,
+// bfloat16: 512 -> 128 elements 42 -> 6.7 us in a replayed step, 128 -> 512 14 -> under 6 us against head_linear_kernel, whose loads wait for one
+// another; errors against float64 9.6e-8 and 7.3e-8 of the size in float32 (2.1e-7 and 1.1e-7), the waves' sums being added pairwise.
+constexpr int kPairSlices = 32, kPairBatch = 8;
+__device__ __forceinline__ float2 pair_of(uint32_t w) { return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u)); }
+__device__ __forceinline__ float2 pair_of(uint2 w) { return make_float2(__uint_as_float(w.x), __uint_as_float(w.y)); }
+template <typename T>
+struct PairBits;
+template <>
+struct PairBits<float> {
+  typedef uint2 type;
+};
+template <>
+struct PairBits<bf16_t> {
+  typedef uint32_t type;
+};
+
+template <typename TX, typename TW, typename TG, typename TO>
+__global__ __launch_bounds__(32 * kPairSlices) void head_linear_pair_kernel(
+    const TX* __restrict__ x, int x_stride, const TW* __restrict__ w, TO* __restrict__ out, int out_stride, int in_dim,
+    int out_dim, int tail, const int32_t* __restrict__ positions, const float* __restrict__ cos_t,
+    const float* __restrict__ sin_t, int interleaved, const TG* __restrict__ gate, int gate_stride, int gate_col,
+    int gate_elems, int n_tokens) {
+  static_assert(kHeadTokens == 8 && kHeadOut == 64, "thread (slice, pair) and two 16-byte reads a row");
+  extern __shared__ __attribute__((aligned(16))) float xs[];  // [in_dim + tail][8], then [16 waves][8][64]
+  const int n0 = blockIdx.x * kHeadTokens, h = blockIdx.y, o0 = blockIdx.z * kHeadOut;
+  const int count = min(kHeadTokens, n_tokens - n0), xw = in_dim + tail, ow = out_dim + tail;
+  float* part = xs + kHeadTokens * xw;
+  const int slice = threadIdx.x / 32, o = o0 + 2 * (threadIdx.x % 32);
+  typedef typename PairBits<TW>::type bits_t;
+  const TW* wh = w + static_cast<size_t>(h) * in_dim * out_dim + min(o, out_dim - 2);
+  bits_t wv[kPairBatch];
+  auto ask = [&](int i0) {
+#pragma unroll
+    for (int j = 0; j < kPairBatch; ++j)
+      wv[j] = *reinterpret_cast<const bits_t*>(wh + static_cast<size_t>(min(i0 + j * kPairSlices, in_dim - 1)) * out_dim);
+  };
+  ask(slice);
+  for (int i = threadIdx.x; i < kHeadTokens * xw; i += blockDim.x) {
+    const int t = i % kHeadTokens, c = i / kHeadTokens;
+    xs[i] = t < count ? to_f32<TX>(x[static_cast<size_t>(n0 + t) * x_stride + h * xw + c]) : 0.f;
+  }
+  __syncthreads();
+  float acc[kHeadTokens][2] = {};
+  for (int i0 = slice; i0 < in_dim; i0 += kPairBatch * kPairSlices) {
+#pragma unroll
+    for (int j = 0; j < kPairBatch; ++j) {
+      const int i = i0 + j * kPairSlices;
+      if (i >= in_dim) continue;
+      const float2 p = pair_of(wv[j]);
+      const float4 a = *reinterpret_cast<const float4*>(&xs[i * kHeadTokens]), b = *reinterpret_cast<const float4*>(&xs[i * kHeadTokens + 4]);
+      const float v[kHeadTokens] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int t = 0; t < kHeadTokens; ++t) {
+        acc[t][0] = fmaf(v[t], p.x, acc[t][0]);
+        acc[t][1] = fmaf(v[t], p.y, acc[t][1]);
+      }
+    }
+    if (i0 + kPairBatch * kPairSlices < in_dim) ask(i0 + kPairBatch * kPairSlices);
+  }
+  // a wave's two slices meet in registers, the waves in LDS
+#pragma unroll
+  for (int t = 0; t < kHeadTokens; ++t) {
+    float sum[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const auto half = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[t][e]), __float_as_uint(acc[t][e]), false, false);
+      sum[e] = __uint_as_float(half[0]) + __uint_as_float(half[1]);
+    }
+    if (threadIdx.x % 64 < 32)
+      *reinterpret_cast<float2*>(&part[(threadIdx.x / 64 * kHeadTokens + t) * kHeadOut + 2 * (threadIdx.x % 32)]) = make_float2(sum[0], sum[1]);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < count * kHeadOut; i += blockDim.x) {
+    const int t = i / kHeadOut, oc = i % kHeadOut;
+    if (o0 + oc >= out_dim) continue;
+    float q[kPairSlices / 2];
+#pragma unroll
+    for (int sl = 0; sl < kPairSlices / 2; ++sl) q[sl] = part[(sl * kHeadTokens + t) * kHeadOut + oc];
+#pragma unroll
+    for (int d = kPairSlices / 4; d > 0; d /= 2)
+#pragma unroll
+      for (int sl = 0; sl < d; ++sl) q[sl] += q[sl + d];
+    float v = q[0];
+    if (gate != nullptr)
+      v *= 1.f / (1.f + expf(-to_f32<TG>(gate[static_cast<size_t>(n0 + t) * gate_stride + gate_col + h * gate_elems +
+                                                  (gate_elems > 1 ? o0 + oc : 0)])));
+    out[static_cast<size_t>(n0 + t) * out_stride + h * ow + o0 + oc] = from_f32<TO>(v);
+  }
+  if (blockIdx.z != 0) return;
+  const int half = tail / 2;
+  for (int i = threadIdx.x; i < count * half; i += blockDim.x) {
+    const int t = i / half, j = i % half;
+    const int ia = interleaved ? 2 * j : j, ib = interleaved ? 2 * j + 1 : j + half;
+    const float a = xs[(in_dim + ia) * kHeadTokens + t], b = xs[(in_dim + ib) * kHeadTokens + t];
+    const size_t p = static_cast<size_t>(positions[n0 + t]);
+    const float c = cos_t[p * half + j], s = sin_t[p * half + j];
+    TO* dst = out + static_cast<size_t>(n0 + t) * out_stride + h * ow + out_dim;
+    dst[ia] = from_f32<TO>(rot_first(a, b, c, s));
+    dst[ib] = from_f32<TO>(rot_second(a, b, c, s));
+  }
+}
+
 // x, w, gate and out each float32 or bfloat16 (the gate in the output's dtype where the input is float32:
 // the way out of the latent; else in the input's)
 extern "C" int yk_head_linear(const void* x, int x_stride, int x_dtype, const void* w, int w_dtype, void* out, int out_dtype,
@@ -180,8 +288,11 @@ extern "C" int yk_head_linear(const void* x, int x_stride, int x_dtype, const vo
   YK_REQUIRE(gate == nullptr || gate_elems == 1 || gate_elems == out_dim, "head_linear: a gate per head or per output element");
   YK_REQUIRE(x_stride >= n_heads * (in_dim + tail), "head_linear: the input's rows are shorter than its heads");
   YK_REQUIRE(tail == 0 || (positions != nullptr && cos_t != nullptr && sin_t != nullptr), "head_linear: a turned tail needs positions and tables");
-  const int slices = 4;
-  const size_t lds = sizeof(float) * (static_cast<size_t>(kHeadTokens) * (in_dim + tail) + slices * kHeadTokens * kHeadOut);
+  const size_t lds = sizeof(float) * (static_cast<size_t>(kHeadTokens) * (in_dim + tail) + kHeadSlices * kHeadTokens * kHeadOut);
+  const size_t pair_lds = sizeof(float) * (static_cast<size_t>(kHeadTokens) * (in_dim + tail) + kPairSlices / 2 * kHeadTokens * kHeadOut);
+  // (many tokens of few elements are better off with the smaller workgroups: 512 tokens of 32 heads, float32, 128 -> 512 93 us against
+  // 114, 512 -> 128 99 against 63)
+  const bool pairs = (n_tokens <= 32 || in_dim >= 256) && out_dim % 2 == 0 && reinterpret_cast<uintptr_t>(w) % 8 == 0 && pair_lds <= 64 * 1024;
   YK_REQUIRE(lds <= 64 * 1024, "head_linear: heads of more than 1,700 input elements do not fit");
   if (n_tokens == 0) return 0;
   dim3 grid((n_tokens + kHeadTokens - 1) / kHeadTokens, n_heads, (out_dim + kHeadOut - 1) / kHeadOut);
@@ -189,13 +300,13 @@ extern "C" int yk_head_linear(const void* x, int x_stride, int x_dtype, const vo
   if (gate == nullptr) gate_dtype = out_dtype;
 #define YK_CASE(XD, TX, WD, TW, GD, TG, OD, TO)                                                                      \
   if (x_dtype == XD && w_dtype == WD && gate_dtype == GD && out_dtype == OD) {                                       \
-    if (slices == 1)                                                                                                 \
-      head_linear_kernel<TX, TW, TG, TO, 1><<<grid, kHeadOut, lds, stream>>>(                                        \
+    if (pairs)                                                                                                       \
+      head_linear_pair_kernel<TX, TW, TG, TO><<<grid, 32 * kPairSlices, pair_lds, stream>>>(                         \
           static_cast<const TX*>(x), x_stride, static_cast<const TW*>(w), static_cast<TO*>(out), out_stride, in_dim, \
           out_dim, tail, positions, cos_t, sin_t, interleaved, static_cast<const TG*>(gate), gate_stride, gate_col,  \
           gate_elems, n_tokens);                                                                                              \
     else                                                                                                             \
-      head_linear_kernel<TX, TW, TG, TO, 4><<<grid, kHeadOut * 4, lds, stream>>>(                                    \
+      head_linear_kernel<TX, TW, TG, TO><<<grid, kHeadOut * kHeadSlices, lds, stream>>>(                             \
           static_cast<const TX*>(x), x_stride, static_cast<const TW*>(w), static_cast<TO*>(out), out_stride, in_dim, \
           out_dim, tail, positions, cos_t, sin_t, interleaved, static_cast<const TG*>(gate), gate_stride, gate_col,  \
           gate_elems, n_tokens);                                                                                              \
