@@ -55,10 +55,10 @@ def reference(kind, t, columns, heads, kv, dim, vdim, spans, slots):
          "exp_bonus": lambda: torch.exp(-torch.exp(z + t["vec"].double())).view(n, heads, dim)}.get(
              kind, lambda: torch.exp(-rate * step)[:, :, None].expand(n, heads, dim))()
     beta = torch.sigmoid(t["scalars"][:, 1: 1 + heads].double())
-    out, states, i = torch.empty(n, heads, vdim, dtype=torch.float64), t["state"].double(), 0
+    out, states, first = torch.empty(n, heads, vdim, dtype=torch.float64), t["state"].double(), 0
     for slot, length in zip(slots, spans):
         S = states[slot]
-        for i in range(i, i + length):
+        for i in range(first, first + length):
             read = lambda row, m: (row[:, None] @ m)[:, 0]
             if kind == "exp_bonus":
                 w = k[i][:, :, None] * v[i][:, None]
@@ -69,7 +69,7 @@ def reference(kind, t, columns, heads, kv, dim, vdim, spans, slots):
             u = beta[i][:, None] * (v[i] - read(k[i], S)) if "delta" in kind else step[i][:, None] * v[i] if kind == "step_skip" else v[i]
             S = S + k[i][:, :, None] * u[:, None]
             out[i] = read(q[i], S) + (t["skip"].double()[:, None] * v[i] if kind == "step_skip" else 0)
-        states[slot], i = S, i + 1
+        states[slot], first = S, first + length
     return out.view(n, -1), states
 
 
@@ -135,3 +135,22 @@ def test_steps_that_are_taken_by_chunks():
             S = t["state"].cuda()
             got[form] = o.linear_state_scan(x, 2, 2, 64, 16, S, ctx, form=form, **kw)
         assert torch.equal(got[None], got[same]), (spans, off)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(2, 1, 64, 64), (3, 3, 128, 192), (2, 2, 256, 128)])
+@pytest.mark.parametrize("kind", list(KINDS))
+def test_scan_of_single_tokens(kind, heads, kv, dim, vdim, dtype):
+    """One token a request, and (as many tokens as requests, not one each) spans of none and two: within 16 roundings of the largest, as
+    above."""
+    o, slots = ops(), [4, 0, 2, 5]
+    for spans in ([1, 1, 1, 1], [1, 2, 0, 1]):
+        t, args, columns = inputs(kind, heads, kv, dim, vdim, dtype, spans)
+        t["state"] = torch.cat([t["state"], t["state"][:1]])
+        want, states = reference(kind, t, columns, heads, kv, dim, vdim, spans, slots)
+        S = t["state"].cuda()
+        y = o.linear_state_scan(t["qkv"].cuda(), heads, kv, dim, vdim, S, step_of(spans, slots), **args(lambda m: m.cuda()))
+        for m, ref in ((y, want), (S, states)):
+            err = (m.double().cpu() - ref).abs().max().item() / ref.abs().max().item()
+            assert err <= 1e-6, (spans, err)
+        assert torch.equal(S[[1, 3]].cpu(), t["state"][[1, 3]]), "slots outside the step stay as they are"

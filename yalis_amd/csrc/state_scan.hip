@@ -574,6 +574,121 @@ __global__ __launch_bounds__(256) void linear_state_scan_fast_kernel(const T* __
   }
 }
 
+// Steps of single tokens: all state traffic and no walk.  A workgroup takes 64 columns of a (request, head)'s S, thread (row group, four
+// columns) every sixteenth row of them 16 bytes at a time, so a wave reads rows in pieces of 256 bytes (a column a group of
+// lanes, as above, reads them in pieces of 16 to 64); all of S is asked for before the token's inputs are, and both sums over
+// the decayed S meet once, in registers and then over the four waves in LDS.  Longer spans stay right: a token after the other.
+// Eight requests, us in a replayed step: 8 heads of 256 x 512 gated 59 -> 12.9 (67 MB of states read and written), 32 of 128 x 128 with the
+// delta rule 17.4 -> 8.9, 16 with decays per channel 10.2 -> 7.9; 64 requests of 4 heads of 256 x 512 222 -> 41.
+__device__ __forceinline__ void token_load4(const float* p, float* v) {
+  const float4 x = *reinterpret_cast<const float4*>(p);
+  v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+}
+__device__ __forceinline__ void token_load4(const bf16_t* p, float* v) {
+  const uint2 w = *reinterpret_cast<const uint2*>(p);
+  v[0] = __uint_as_float(w.x << 16); v[1] = __uint_as_float(w.x & 0xffff0000u);
+  v[2] = __uint_as_float(w.y << 16); v[3] = __uint_as_float(w.y & 0xffff0000u);
+}
+
+template <typename T, int D, int KIND>
+__global__ __launch_bounds__(256) void linear_state_token_kernel(const T* __restrict__ qkv, float* __restrict__ state, float* __restrict__ out,
+                                                                 const T* __restrict__ beta_rows, ScanArgs g) {
+  constexpr bool CH = KIND & kScanChannel, DELTA = KIND & kScanDelta, FIRST = KIND & kScanReadFirst;
+  constexpr int ROWS = D / 16;
+  __shared__ __attribute__((aligned(16))) float ks[D], qs[D], as[CH ? D : 1], red[2][4][64], sums[4][4];
+  const int seq = blockIdx.x, h = blockIdx.y, kvh = h / (g.n_heads / g.n_kv), vdim = g.vdim;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, group = threadIdx.x / 16, col = 64 * blockIdx.z + 4 * (threadIdx.x % 16);
+  const int q0 = g.seq_qstart[seq], ql = g.seq_qlen[seq];
+  if (ql <= 0) return;
+  float* S_head = state + (static_cast<size_t>(g.state_slots[seq]) * g.n_heads + h) * D * vdim + col;
+  float S[ROWS][4];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) token_load4(S_head + static_cast<size_t>(group + 16 * r) * vdim, S[r]);
+  const float skip_h = g.skip != nullptr ? g.skip[h] : 0.f;
+  const float dec_rate = CH && g.decay_mode == 2 ? expf(g.decay_p0[h]) : 1.f;
+
+  for (int t = 0; t < ql; ++t) {
+    const size_t n = static_cast<size_t>(q0) + t;
+    const T* row = qkv + n * g.qkv_stride;
+    float v[4];
+    token_load4(row + g.v_col + h * vdim + col, v);
+    if (t > 0) __syncthreads();
+    float q = 0.f, k = 0.f, w = 0.f;
+    const int i = threadIdx.x;
+    if (i < D) {
+      q = to_f32<T>(row[g.q_col + kvh * D + i]);
+      k = to_f32<T>(row[g.k_col + kvh * D + i]);
+      w = FIRST ? q * g.bonus[h * D + i] * k : q * k;
+      qs[i] = q;
+      ks[i] = k;
+      if (CH) as[i] = channel_decay(g.decay[n * g.decay_stride + g.decay_col + h * D + i] + (g.decay_mode == 2 ? g.decay_p1 : g.decay_p0)[h * D + i], g.decay_mode,
+                                    g.tau, dec_rate);
+    }
+    const float wave_q = wave_sum(q * q), wave_k = wave_sum(k * k), wave_w = wave_sum(w);
+    if (lane == 0) sums[wave][0] = wave_q, sums[wave][1] = wave_k, sums[wave][2] = wave_w;
+    float a = 1.f, strength = 1.f;
+    if (!CH) {
+      const float step = g.decay_mode == 0 ? scan_softplus(g.decay[n * g.decay_stride + g.decay_col + h] + g.decay_p1[h]) : 1.f;
+      a = g.decay_mode == 4 ? g.decay_p0[h] : expf(-expf(g.decay_p0[h]) * step);
+      if (g.by_step) strength = step;
+    }
+    if (DELTA) {
+      const size_t at = n * g.beta_stride + g.beta_col + h;
+      strength = 1.f / (1.f + expf(-(beta_rows != nullptr ? to_f32<T>(beta_rows[at]) : g.beta[at])));
+    }
+    __syncthreads();
+    float mq = g.q_scale, mk = 1.f;
+    if (g.unit_eps >= 0.f) {
+      mq = g.q_scale / sqrtf((sums[0][0] + sums[1][0]) + (sums[2][0] + sums[3][0]) + g.unit_eps);
+      mk = 1.f / sqrtf((sums[0][1] + sums[1][1]) + (sums[2][1] + sums[3][1]) + g.unit_eps);
+    }
+    const float kq = ((sums[0][2] + sums[1][2]) + (sums[2][2] + sums[3][2])) * (mq * mk);
+    float pk[2][4] = {}, pq[2][4] = {};
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const float ar = CH ? as[group + 16 * r] : a, kr = ks[group + 16 * r], qr = qs[group + 16 * r];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (FIRST) pq[r % 2][e] = fmaf(S[r][e], qr, pq[r % 2][e]);
+        S[r][e] *= ar;
+        if (DELTA) pk[r % 2][e] = fmaf(S[r][e], kr, pk[r % 2][e]);
+        if (!FIRST) pq[r % 2][e] = fmaf(S[r][e], qr, pq[r % 2][e]);
+      }
+    }
+    float sk[4], sq[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sq[e] = column_lanes_sum(pq[0][e] + pq[1][e]);
+      sk[e] = DELTA ? column_lanes_sum(pk[0][e] + pk[1][e]) : 0.f;
+    }
+    if (lane < 16) {
+      *reinterpret_cast<float4*>(&red[0][wave][4 * lane]) = make_float4(sq[0], sq[1], sq[2], sq[3]);
+      if (DELTA) *reinterpret_cast<float4*>(&red[1][wave][4 * lane]) = make_float4(sk[0], sk[1], sk[2], sk[3]);
+    }
+    __syncthreads();
+    float u[4], o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int c = 4 * (lane % 16) + e;
+      u[e] = v[e];
+      if (DELTA) u[e] = strength * (v[e] - mk * ((red[1][0][c] + red[1][1][c]) + (red[1][2][c] + red[1][3][c])));
+      else if (!CH) u[e] *= strength;
+      o[e] = fmaf(u[e], kq, mq * ((red[0][0][c] + red[0][1][c]) + (red[0][2][c] + red[0][3][c])));
+      if (!CH && !DELTA) o[e] = fmaf(skip_h, v[e], o[e]);
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const float kr = ks[group + 16 * r] * mk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[r][e] = fmaf(kr, u[e], S[r][e]);
+    }
+    if (threadIdx.x < 16) *reinterpret_cast<float4*>(out + (n * g.n_heads + h) * vdim + col) = make_float4(o[0], o[1], o[2], o[3]);
+  }
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+    *reinterpret_cast<float4*>(S_head + static_cast<size_t>(group + 16 * r) * vdim) = make_float4(S[r][0], S[r][1], S[r][2], S[r][3]);
+}
+
 // decays per key channel, made once for all the columns that will read them: out[n][h * dim + i], four a thread
 __global__ __launch_bounds__(256) void channel_decay_kernel(const float* __restrict__ z, int stride, int col, const float* __restrict__ p0,
                                                             const float* __restrict__ p1, int mode, float tau, int dim, int channels,
@@ -642,6 +757,28 @@ extern "C" int yk_linear_state_scan(const void* qkv, int qkv_stride, int dtype, 
   const int kind = (per_channel ? kScanChannel : 0) + (write_mode == 1 ? kScanDelta : 0) + (bonus != nullptr ? kScanReadFirst : 0);
   const bool fast = dim % 8 == 0 && qkv_stride % 8 == 0 && q_col % 8 == 0 && k_col % 8 == 0 && al16(qkv) && chunk * dp <= 8192 && kind != kScanReadFirst &&
                     (skip == nullptr || kind == 0);
+  // one token a request: 64 columns a workgroup in 16-byte pieces (wider heads than 256 channels do not fit in registers)
+  if (n_tokens == n_seqs && (dim == 64 || dim == 128 || dim == 256) && vdim % 64 == 0 && qkv_stride % 8 == 0 && v_col % 8 == 0 && al16(qkv) &&
+      al16(state) && al16(out) && kind != kScanReadFirst && (skip == nullptr || kind == 0)) {
+    const ScanArgs g{seq_qstart, seq_qlen, state_slots, qkv_stride, n_heads, n_kv, dim, vdim, q_col, k_col, v_col, q_scale, unit_eps, decay_mode, 0, decay,
+                     decay_stride, decay_col, decay_p0, decay_p1, tau, beta, beta_stride, beta_col, write_mode == 2, skip, bonus, 1};
+    const dim3 token_grid(n_seqs, n_heads, vdim / 64);
+#define YK_TOKEN(T, D, KIND)                                                                                                    \
+  if (dim == D && kind == KIND) {                                                                                               \
+    linear_state_token_kernel<T, D, KIND><<<token_grid, 256, 0, stream>>>(static_cast<const T*>(qkv), state, out,               \
+                                                                          static_cast<const T*>(beta_rows), g);                 \
+    return yk_check_launch("linear_state_token");                                                                               \
+  }
+#define YK_TOKEN_KINDS(T, D) YK_TOKEN(T, D, 0) YK_TOKEN(T, D, 1) YK_TOKEN(T, D, 2) YK_TOKEN(T, D, 3) YK_TOKEN(T, D, 5)
+    if (dtype == YK_F32) {
+      YK_TOKEN_KINDS(float, 64) YK_TOKEN_KINDS(float, 128) YK_TOKEN_KINDS(float, 256)
+    }
+    if (dtype == YK_BF16) {
+      YK_TOKEN_KINDS(bf16_t, 64) YK_TOKEN_KINDS(bf16_t, 128) YK_TOKEN_KINDS(bf16_t, 256)
+    }
+#undef YK_TOKEN_KINDS
+#undef YK_TOKEN
+  }
   if (fast) {
     // many tokens: their decays per channel first, where the caller gave room for them
     const bool given = per_channel && decays != nullptr && decay_stride % 4 == 0 && decay_col % 4 == 0 && al16(decay) && al16(decays) &&
