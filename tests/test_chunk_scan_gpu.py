@@ -125,15 +125,17 @@ def test_what_is_not_finite_stays_behind_its_token(kind):
 def test_steps_that_are_taken_by_chunks():
     """Long spans by chunks; short ones, many short ones beside a long one, and rows that are not aligned as they are walked."""
     o = ops()
-    for spans, off, same in (([256], 0, "chunks"), ([255], 0, "walk"), ([256] + [1] * 2, 0, "walk"), ([256], 4, "walk")):
-        t, args, columns = inputs("delta", 2, 2, 64, 16, torch.bfloat16, spans)
+    for spans, off, same, kind, heads, dim, vdim in (
+            ([256], 0, "chunks", "delta", 2, 64, 16), ([255], 0, "walk", "delta", 2, 64, 16), ([256] + [1] * 2, 0, "walk", "delta", 2, 64, 16),
+            ([256], 4, "walk", "delta", 2, 64, 16), ([64, 64, 70], 0, "chunks", "channel", 8, 256, 1024), ([63, 64, 64], 0, "walk", "channel", 8, 256, 1024)):
+        t, args, columns = inputs(kind, heads, heads, dim, vdim, torch.bfloat16, spans)
         x = tf.pad(t["qkv"], (off, 8 - off)).cuda()
         kw = args(lambda m: m.cuda())
         kw["columns"] = tuple(c + off for c in columns)
         ctx, got = step_of(spans, list(range(len(spans)))), {}
         for form in (None, same):
             S = t["state"].cuda()
-            got[form] = o.linear_state_scan(x, 2, 2, 64, 16, S, ctx, form=form, **kw)
+            got[form] = o.linear_state_scan(x, heads, heads, dim, vdim, S, ctx, form=form, **kw)
         assert torch.equal(got[None], got[same]), (spans, off)
 
 

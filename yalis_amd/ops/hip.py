@@ -1803,6 +1803,9 @@ class HipOps:
     # token by token, of 160: 42 against 41), and 128 tokens a request on average, since a request of one token costs a whole chunk (512 tokens
     # with 16 requests of one: 186 against 170; 8 of 256: 108 against 151).
     STATE_CHUNKS_MIN_SPAN, STATE_CHUNKS_MIN_AVERAGE = 256, 128
+    # Heads of 256 key channels are walked at half the rate and meet earlier where there are columns (tokens * heads * vdim) to
+    # fill the chip: 4 heads of 256 x 512, 8 spans of 96 107 us against 200, of 128 110 against 272, 32 of 64 180 against 553, but one of 160 69 against 50.
+    STATE_CHUNKS_WIDE_SPAN, STATE_CHUNKS_WIDE_COLUMNS = 64, 1500000
     # scratch for what the chunks of a step's spans are worked into (15,000 tokens of 16 heads; beyond that heads are taken by turns)
     STATE_CHUNKS_BYTES = 512 << 20
 
@@ -1870,7 +1873,8 @@ class HipOps:
         n_seqs, max_qlen, a_head = a["seq_qstart"].numel(), getattr(ctx, "max_qlen", 0), 0
         aligned = qkv.stride(0) % 8 == 0 and q_col % 8 == 0 and k_col % 8 == 0 and qkv.data_ptr() % 16 == 0
         long = max_qlen >= self.STATE_CHUNKS_MIN_SPAN and n >= self.STATE_CHUNKS_MIN_AVERAGE * n_seqs
-        if aligned and (form == "chunks" or (form is None and long)):
+        long = long or (dim == 256 and n >= self.STATE_CHUNKS_WIDE_SPAN * n_seqs and n * n_heads * vdim >= self.STATE_CHUNKS_WIDE_COLUMNS)
+        if aligned and (form == "chunks" or (form is None and long and max_qlen > 1)):
             a_head = self.lib.yk_state_scan_chunks_floats(n, n_seqs, dim, vdim, mode, write_mode, int(bonus is not None), int(skip is not None))
         if form == "chunks" and not a_head:
             raise KernelError("linear_state_scan: this step cannot be taken chunk by chunk")
