@@ -145,7 +145,8 @@ template <int M0>
 __device__ __forceinline__ int at(int i, int m, int lane) {
   return ((i * M0 + m) * 64 + lane) * 4;
 }
-// chunk c of request seq: its place among the parts (no two requests share one)
+// chunk c of request seq: its place among the parts (requests' spans lie in the batch in their own order, as a step's arrays are built,
+// so no two share one)
 __device__ __forceinline__ size_t part_of(int seq, int q0, int c, int n_heads_here, int head_local) {
   return static_cast<size_t>(q0 / kTok + seq + c) * n_heads_here + head_local;
 }
