@@ -24,11 +24,12 @@
 // ahead, in the order and place where the products take it.  Eight waves that share the two read-outs, with all operands twice,
 // took 170 us where four take 120: their registers leave no room for the loads on their way.
 //
-// 2,048 tokens of one request in bfloat16, us with prepare and walk (token by token: yk_linear_state_scan): 16 heads of 128 x 128, delta
-// rule 158 = 39 + 120 (472), with decays per channel 183 = 69 + 119 (498); 4 of 256 x 512 gated 187 = 61 + 133 (500); 32 of 64 x 64
-// with a bonus 93 (397); 32 of 128 x 64 by step 131 (398).  Errors of the read-outs against float64, of their size: 1.1e-7, 1.1e-7,
-// 2.7e-7, 0.7e-7, 0.8e-7 (1.1e-7, 1.1e-7, 2.7e-7, 0.8e-7, 0.8e-7).
+// 2,048 tokens of one request in bfloat16, us (of which prepare; token by token: yk_linear_state_scan): 16 heads of 128 x 128, delta rule 158
+// (39; 465), with decays per channel 185 (69; 496); 4 of 256 x 512 gated 189 (61; 497); 32 of 64 x 64 with a bonus 96 (396); 32 of
+// 128 x 64 by step 132 (396).  Errors against float64, of their size, of the read-outs 1.1e-7, 1.1e-7, 2.5e-7, 0.7e-7, 0.8e-7 (walked
+// 1.1e-7, 1.1e-7, 2.6e-7, 0.9e-7, 0.9e-7) and of the kept memories 0.8e-7, 0.8e-7, 2.4e-7, 0.4e-7, 0.6e-7 (0.8e-7, 0.8e-7, 2.6e-7, 0.4e-7, 0.6e-7).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -603,7 +604,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
     ask_b(part0);
     ask_ke(part0);
   }
-  for (int c = 0; c < chunks; ++c) {
+  auto turn = [&](int c, auto last) {
     const float* next = part0 + min(c + 1, chunks - 1) * step;  // (the last chunk asks for itself once more, unread)
 #pragma unroll
     for (int m = 0; m < MT; ++m) s_lds[wave * MT + m][lane] = S[m];
@@ -637,11 +638,31 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
     f32x4_t u[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) u[m] = u_lds[m][lane];
+    if (!decltype(last)::value) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const f32x4_t sum = mma64(ke[m], u);
+      for (int m = 0; m < MT; ++m) {
+        const f32x4_t sum = mma64(ke[m], u);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) S[m][i] = fmaf(S[m][i], dec[m][i], sum[i]);
+        for (int i = 0; i < 4; ++i) S[m][i] = fmaf(S[m][i], dec[m][i], sum[i]);
+      }
+    } else {
+      // the memory that is kept: in float64, rounded once.  Its last tokens weigh the most and 64 products in float32 round them oftener than
+      // the walk does: time mixing 0.57e-7 -> 0.40e-7 of its size (walked 0.44e-7), delta rule 1.00e-7 -> 0.85e-7 (0.83e-7).  A product in
+      // float64 leaves row lg + 4 i in lane (r, lg), so the keys' rows are handed over in that order.
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        f64x4_t sum;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[i] = static_cast<double>(S[m][i]) * static_cast<double>(dec[m][i]);
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sum = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(__shfl(ke[m][x][e], 4 * (r % 4) + r / 4 + 16 * lg, 64)),
+                                                       static_cast<double>(u[x][e]), sum, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[m][i] = static_cast<float>(sum[i]);
+      }
     }
     ask_ke(next);
     o = lower(b, u, o);
@@ -651,7 +672,9 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
       const int t = c * kTok + 16 * wave + 4 * lg + i;
       if (t < ql) out[(static_cast<size_t>(q0 + t) * g.n_heads + h) * vdim + col0 + r] = o[i];
     }
-  }
+  };
+  for (int c = 0; c + 1 < chunks; ++c) turn(c, std::false_type{});
+  if (chunks > 0) turn(chunks - 1, std::true_type{});
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
