@@ -121,6 +121,20 @@ def test_kept_memories_are_as_exact_as_when_walked(kind, heads, dim, vdim):
     assert error["chunks"] <= 1.1 * error["walk"], error
 
 
+@pytest.mark.parametrize("kind", ["plain", "softplus_delta"])
+def test_spans_in_any_order(kind):
+    """Requests listed in another order than their spans lie in the rows: the same bits."""
+    o, spans, slots = ops(), [128, 128, 64, 1, 200, 65], [0, 1, 2, 3, 4, 5]
+    t, args, _ = inputs(kind, 2, 2, 64, 16, torch.bfloat16, spans)
+    got = []
+    for order in ([0, 1, 2, 3, 4, 5], [5, 4, 3, 2, 1, 0], [1, 0, 4, 2, 5, 3]):
+        ctx, S = step_of(spans, slots), t["state"].cuda()
+        ctx.arrays = {k: v[order].contiguous() for k, v in ctx.arrays.items()}
+        y = o.linear_state_scan(t["qkv"].cuda(), 2, 2, 64, 16, S, ctx, form="chunks", **args(lambda m: m.cuda()))
+        got.append((y, S))
+    assert all(torch.equal(y, got[0][0]) and torch.equal(S, got[0][1]) for y, S in got[1:])
+
+
 @pytest.mark.parametrize("kind", ["plain", "delta", "channel", "softplus_delta", "exp_bonus"])
 def test_what_is_not_finite_stays_behind_its_token(kind):
     """A value, a key and a query that are not finite, in the middle of a chunk's tile: what comes before them and the other

@@ -146,10 +146,10 @@ template <int M0>
 __device__ __forceinline__ int at(int i, int m, int lane) {
   return ((i * M0 + m) * 64 + lane) * 4;
 }
-// chunk c of request seq: its place among the parts (requests' spans lie in the batch in their own order, as a step's arrays are built,
-// so no two share one)
-__device__ __forceinline__ size_t part_of(int seq, int q0, int c, int n_heads_here, int head_local) {
-  return static_cast<size_t>(q0 / kTok + seq + c) * n_heads_here + head_local;
+// Chunk c of request seq: its place among the n_tokens / 64 + n_seqs parts.  First chunks by request, the others by the token they start
+// at: 64 tokens of the span lie before it, so no two of them start in the same 64 tokens, whatever the order of the spans in the batch.
+__device__ __forceinline__ size_t part_of(int seq, int n_seqs, int q0, int c, int n_heads_here, int head_local) {
+  return static_cast<size_t>(c == 0 ? seq : n_seqs + q0 / kTok + c - 1) * n_heads_here + head_local;
 }
 
 // ------------------------------------------------------------------------------------------- prepare
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
   if (c * kTok >= ql) return;
   const int n = min(kTok, ql - c * kTok);
   const size_t n0 = static_cast<size_t>(q0) + c * kTok;
-  float* part = g.ws + part_of(seq, q0, c, gridDim.y, hl) * P::SIZE;
+  float* part = g.ws + part_of(seq, gridDim.z, q0, c, gridDim.y, hl) * P::SIZE;
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), r = lane % 16, lg = lane / 16;
 
   // the tokens' scalars
@@ -556,8 +556,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
 
   f32x4_t q[M], k[DELTA ? M : 1], ke[MT][4], b[4], tm[DELTA ? 4 : 1], dec[MT];
   uint32_t raw_v[4];  // (as they lie there: a conversion where they are asked for would wait for them)
-  const float* part0 = g.ws + part_of(seq, q0, 0, gridDim.x, hl) * P::SIZE;
-  const size_t step = static_cast<size_t>(gridDim.x) * P::SIZE;
+  const float* part0 = g.ws + part_of(seq, gridDim.z, q0, 0, gridDim.x, hl) * P::SIZE;
   auto ask_qk = [&](const float* p) {
 #pragma unroll
     for (int m = 0; m < M; ++m) {
@@ -605,7 +604,8 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
     ask_ke(part0);
   }
   auto turn = [&](int c, auto last) {
-    const float* next = part0 + min(c + 1, chunks - 1) * step;  // (the last chunk asks for itself once more, unread)
+    // (the last chunk asks for itself once more, unread)
+    const float* next = g.ws + part_of(seq, gridDim.z, q0, decltype(last)::value ? c : c + 1, gridDim.x, hl) * P::SIZE;
 #pragma unroll
     for (int m = 0; m < MT; ++m) s_lds[wave * MT + m][lane] = S[m];
     __syncthreads();
