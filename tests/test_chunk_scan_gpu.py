@@ -135,6 +135,21 @@ def test_spans_in_any_order(kind):
     assert all(torch.equal(y, got[0][0]) and torch.equal(S, got[0][1]) for y, S in got[1:])
 
 
+@pytest.mark.parametrize("kind", ["plain", "softplus_delta"])
+def test_spans_of_no_tokens(kind):
+    """Requests without tokens, before, between and behind the others, one of them with another's slot: the memories and
+    read-outs are those of the step without them."""
+    o, spans, slots = ops(), [128, 70], [0, 1]
+    t, args, _ = inputs(kind, 2, 2, 64, 16, torch.bfloat16, spans)
+    got = []
+    for lengths, at in ((spans, slots), ([0, 128, 0, 70, 0], [2, 0, 1, 1, 0])):
+        S = t["state"].cuda()
+        y = o.linear_state_scan(t["qkv"].cuda(), 2, 2, 64, 16, S, step_of(lengths, at), form="chunks", **args(lambda m: m.cuda()))
+        got.append((y, S))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert torch.equal(got[1][1][2].cpu(), t["state"][2])
+
+
 @pytest.mark.parametrize("kind", ["plain", "delta", "channel", "softplus_delta", "exp_bonus"])
 def test_what_is_not_finite_stays_behind_its_token(kind):
     """A value, a key and a query that are not finite, in the middle of a chunk's tile: what comes before them and the other

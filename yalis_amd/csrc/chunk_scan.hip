@@ -543,6 +543,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
   __shared__ __attribute__((aligned(16))) f32x4_t s_lds[M][64], x_lds[4][64], u_lds[4][64];
   const int hl = blockIdx.x, h = g.head0 + hl, col0 = 16 * blockIdx.y, seq = blockIdx.z, vdim = g.vdim;
   const int q0 = g.seq_qstart[seq], ql = g.seq_qlen[seq], chunks = (ql + kTok - 1) / kTok;
+  if (ql <= 0) return;  // (a request without tokens leaves its memory alone: its slot may be another's by now)
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), r = lane % 16, lg = lane / 16;
   float* S_head = state + (static_cast<size_t>(g.state_slots[seq]) * g.n_heads + h) * D * vdim + col0 + r;
   f32x4_t S[MT];
@@ -596,13 +597,11 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
       if (m < wave) c = mma16(a[m], b[m], c);
     return wave == 0 ? triangle16(a[0], b[0], c) : wave == 1 ? triangle16(a[1], b[1], c) : wave == 2 ? triangle16(a[2], b[2], c) : triangle16(a[3], b[3], c);
   };
-  if (chunks > 0) {
-    ask_qk(part0);
-    ask_v(0);
-    ask_t(part0);
-    ask_b(part0);
-    ask_ke(part0);
-  }
+  ask_qk(part0);
+  ask_v(0);
+  ask_t(part0);
+  ask_b(part0);
+  ask_ke(part0);
   auto turn = [&](int c, auto last) {
     // (the last chunk asks for itself once more, unread)
     const float* next = g.ws + part_of(seq, gridDim.z, q0, decltype(last)::value ? c : c + 1, gridDim.x, hl) * P::SIZE;
@@ -674,7 +673,7 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
     }
   };
   for (int c = 0; c + 1 < chunks; ++c) turn(c, std::false_type{});
-  if (chunks > 0) turn(chunks - 1, std::true_type{});
+  turn(chunks - 1, std::true_type{});
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
