@@ -682,6 +682,28 @@ def test_attention_generic_many_tokens(ops, h, g, d, page, window, dtype):
         close(got, want, 1e-2, 2**-7)
 
 
+# one key alone in its block: the last of 65, or the first that a window of 68 shows behind 131; forms of eight waves and of one
+@pytest.mark.parametrize("h,g,n", [(4, 4, 2), (64, 16, 64), (63, 63, 66)])
+@pytest.mark.parametrize("last,window,low", [(64, 0, 64), (130, 68, 63), (130, 0, 3)])
+def test_attention_generic_where_a_block_scores_minus_infinity(ops, h, g, n, last, window, low):
+    """A key whose product with the query overflows to -inf has weight 0, also where it is all that its block shows."""
+    d, page, gen = 16, 16, torch.Generator().manual_seed(n)
+    keys, values = torch.randn((last + 1, g, d), generator=gen), torch.randn((last + 1, g, d), generator=gen)
+    keys[low] = -3e38
+    pages = -(-(last + 1) // page)
+    kc, vc = torch.zeros((pages, g, page, d)), torch.zeros((pages, g, d, page))
+    for pos in range(last + 1):
+        kc[pos // page, :, pos % page], vc[pos // page, :, :, pos % page] = keys[pos], values[pos]
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    ctx = types.SimpleNamespace(arrays={"positions": dev([last] * n), "token_seq": dev([0] * n), "block_table_g0": dev([list(range(pages))])}, max_ctx=last + 1)
+    q = torch.rand((n, h, d), generator=gen) + 0.5
+    got = ops.attention(q.view(n, -1).to(DEV), h, g, d, kc.to(DEV), vc.to(DEV), page, 0.25, window, ctx, 0, None)
+    first = max(0, last - window + 1) if window else 0
+    s = torch.einsum("nhd,khd->nhk", q.double(), keys[first:].double().repeat_interleave(h // g, 1)) * 0.25
+    want = torch.einsum("nhk,khd->nhd", s.softmax(-1), values[first:].double().repeat_interleave(h // g, 1))
+    close(got, want.reshape(n, -1), 2e-5, 1e-5)
+
+
 @pytest.mark.parametrize("h,g,d,page", [(4, 2, 16, 16), (4, 1, 32, 32), (6, 3, 48, 16), (5, 5, 80, 64), (2, 1, 256, 16)])
 @pytest.mark.parametrize("window", [0, 24])
 def test_attention_generic_f32(ops, h, g, d, page, window):

@@ -104,9 +104,11 @@ __global__ __launch_bounds__(64 * W) void attn_generic_kernel(
     float alpha[HQ];
 #pragma unroll
     for (int e = 0; e < HQ; ++e) {
-      const float m_new = fmaxf(m[e], wave_max(s[e]));  // finite: the block holds at least one visible key
-      const float p = valid ? expf(s[e] - m_new) : 0.f;
-      alpha[e] = expf(m[e] - m_new);  // 0 on the first block
+      const float m_new = fmaxf(m[e], wave_max(s[e]));
+      // (the visible keys of a wave's first block may all score -inf, where another block's do not)
+      const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+      const float p = valid ? expf(s[e] - m_safe) : 0.f;
+      alpha[e] = expf(m[e] - m_safe);  // 0 on the first block
       l[e] = l[e] * alpha[e] + wave_sum(p);
       m[e] = m_new;
       ps[wave][e][lane] = p;
