@@ -682,6 +682,24 @@ def test_attention_generic_many_tokens(ops, h, g, d, page, window, dtype):
         close(got, want, 1e-2, 2**-7)
 
 
+# pages whose slots are no multiple of four, and pages that do not start at a multiple of 16 bytes; few and many (token, head)s
+@pytest.mark.parametrize("h,g,d,page,shift", [(4, 2, 16, 6, 0), (6, 3, 48, 1, 0), (5, 5, 80, 18, 0), (48, 12, 16, 7, 0), (4, 1, 32, 32, 1), (48, 12, 16, 16, 3)])
+@pytest.mark.parametrize("window", [0, 3, 66])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_attention_generic_any_pages(ops, h, g, d, page, shift, window, dtype, monkeypatch):
+    def shifted(t):
+        room = torch.full((t.numel() + shift,), float("nan"), dtype=t.dtype, device=DEV)
+        room[shift:] = t.reshape(-1).to(DEV)
+        return room[shift:].view(t.shape)
+
+    monkeypatch.setitem(globals(), "device_cache", lambda ops, kc, vc: (shifted(kc), shifted(vc)))
+    got, want = _attention_case(ops, dtype, h, g, d, page, SPANS, window, 19, n_pages=400)
+    if dtype == torch.float32:
+        close(got, want, 2e-5, 1e-5)
+    else:
+        close(got, want, 1e-2, 2**-7)
+
+
 # one key alone in its block: the last of 65, or the first that a window of 68 shows behind 131; forms of eight waves and of one
 @pytest.mark.parametrize("h,g,n", [(4, 4, 2), (64, 16, 64), (63, 63, 66)])
 @pytest.mark.parametrize("last,window,low", [(64, 0, 64), (130, 68, 63), (130, 0, 3)])

@@ -28,11 +28,17 @@
 #include "common.h"
 
 // ---------------------------------------------------------------------------- generic
-// four elements of a row as float32 (rows of pages start at multiples of 16 elements)
-__device__ __forceinline__ float4 generic_load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 generic_load4(const bf16_t* p) {
-  const uint2 u = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u));
+// four consecutive elements as float32, in one load where they lie aligned
+template <bool WIDE, typename T>
+__device__ __forceinline__ float4 generic_load4(const T* p) {
+  if constexpr (!WIDE) {
+    return make_float4(to_f32<T>(p[0]), to_f32<T>(p[1]), to_f32<T>(p[2]), to_f32<T>(p[3]));
+  } else if constexpr (sizeof(T) == 4) {
+    return *reinterpret_cast<const float4*>(p);
+  } else {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u));
+  }
 }
 
 // A workgroup of W waves makes HQ heads of one token that share a key/value head; its waves take the
@@ -43,7 +49,9 @@ __device__ __forceinline__ float4 generic_load4(const bf16_t* p) {
 // for all heads that want it, and many waves.  32 heads of 64 elements over 8 kv heads, float32 (us a
 // layer; before: one wave a head with 4-byte loads): 2 tokens behind 200 and 311 keys 45 -> 12, 511 tokens
 // of two prompts 357 -> 74 (164 with one head a wave).
-template <typename T, int W, int HQ>
+// WIDE: pages of a multiple of four slots that start at multiples of 16 bytes.  Else (the engine makes no such pages) four consecutive keys
+// may lie in two pages, and every element is a load and every key has a place of its own.
+template <typename T, int W, int HQ, bool WIDE>
 __global__ __launch_bounds__(64 * W) void attn_generic_kernel(
     const T* __restrict__ q, int q_stride, T* __restrict__ out, const T* __restrict__ k_cache,
     const T* __restrict__ v_cache, const int32_t* __restrict__ positions,
@@ -53,7 +61,8 @@ __global__ __launch_bounds__(64 * W) void attn_generic_kernel(
   const size_t slab = static_cast<size_t>(page_size) * head_dim;
   __shared__ __attribute__((aligned(16))) float qs[HQ][256];
   __shared__ __attribute__((aligned(16))) float ps[W][HQ][64];
-  __shared__ int2 where[W][16];        // (page * n_kv + kv_head, slot) of every fourth key of a wave's block
+  constexpr int STEP = WIDE ? 4 : 1;
+  __shared__ int2 where[W][64 / STEP];  // (page * n_kv + kv_head, slot) of every fourth, or every, key of a wave's block
   __shared__ float merged[W][HQ][258];  // a wave's sums, maximum and sum of weights
   const int n = blockIdx.x, h0 = blockIdx.y * HQ, lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int qpk = n_heads / n_kv, g = h0 / qpk;
@@ -87,7 +96,7 @@ __global__ __launch_bounds__(64 * W) void attn_generic_kernel(
       float4 dot[HQ] = {};
 #pragma unroll 4
       for (int d = 0; d < head_dim; d += 4) {
-        const float4 k4 = generic_load4(kp + cache_k_offset(tiled, page_size, head_dim, off, d));
+        const float4 k4 = generic_load4<WIDE>(kp + cache_k_offset(tiled, page_size, head_dim, off, d));
 #pragma unroll
         for (int e = 0; e < HQ; ++e) {
           const float4 q4 = *reinterpret_cast<const float4*>(&qs[e][d]);
@@ -114,9 +123,9 @@ __global__ __launch_bounds__(64 * W) void attn_generic_kernel(
       ps[wave][e][lane] = p;
     }
     // four keys' place is that of any of them that is visible
-    const int first = min(max(t0 + lane / 4 * 4, lo), hi - 1);
+    const int first = min(max(t0 + lane / STEP * STEP, lo), hi - 1);
     const int from = __shfl(base, first - t0, 64), slot = __shfl(off, first - t0, 64);
-    if (lane % 4 == 0) where[wave][lane / 4] = make_int2(from, slot & ~3);
+    if (lane % STEP == 0) where[wave][lane / STEP] = make_int2(from, slot & ~(STEP - 1));
     __builtin_amdgcn_wave_barrier();
     const int j0 = max(0, lo - t0) / 4, j1 = (min(64, hi - t0) + 3) / 4;
 #pragma unroll
@@ -127,8 +136,13 @@ __global__ __launch_bounds__(64 * W) void attn_generic_kernel(
         for (int e = 0; e < HQ; ++e) acc[e][i] *= alpha[e];
 #pragma unroll 4
         for (int j = j0; j < j1; ++j) {
-          const int2 at = where[wave][j];
-          float4 v4 = generic_load4(v_cache + static_cast<size_t>(at.x) * slab + cache_v_offset(tiled, page_size, head_dim, at.y, d));
+          auto value = [&](int k) {
+            const int2 at = where[wave][k];
+            return v_cache + static_cast<size_t>(at.x) * slab + cache_v_offset(tiled, page_size, head_dim, at.y, d);
+          };
+          float4 v4;
+          if constexpr (WIDE) v4 = generic_load4<WIDE>(value(j));
+          else v4 = make_float4(to_f32<T>(*value(4 * j)), to_f32<T>(*value(4 * j + 1)), to_f32<T>(*value(4 * j + 2)), to_f32<T>(*value(4 * j + 3)));
           const int k0 = t0 + 4 * j;  // what lies in a page beside the visible keys (weight 0) is not to be read as a number
           v4.x = k0 >= lo && k0 < hi ? v4.x : 0.f;
           v4.y = k0 + 1 >= lo && k0 + 1 < hi ? v4.y : 0.f;
@@ -191,10 +205,12 @@ static void launch_generic(const T* q, int q_stride, T* out, const T* k_cache, c
     kernel<<<dim3(n_tokens, n_heads / heads), 64 * waves, 0, stream>>>(q, q_stride, out, k_cache, v_cache, positions, token_seq, block_table,
                                                                        table_width, page_size, head_dim, n_heads, n_kv, scale, window);
   };
-  if (static_cast<long long>(n_tokens) * n_heads < 4096) return with(attn_generic_kernel<T, 8, 1>, 8, 1);
-  if (qpk % 4 == 0) return with(attn_generic_kernel<T, 1, 4>, 1, 4);
-  if (qpk % 2 == 0) return with(attn_generic_kernel<T, 1, 2>, 1, 2);
-  with(attn_generic_kernel<T, 1, 1>, 1, 1);
+  if (page_size % 4 != 0 || (reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) % 16 != 0)
+    return with(attn_generic_kernel<T, 8, 1, false>, 8, 1);
+  if (static_cast<long long>(n_tokens) * n_heads < 4096) return with(attn_generic_kernel<T, 8, 1, true>, 8, 1);
+  if (qpk % 4 == 0) return with(attn_generic_kernel<T, 1, 4, true>, 1, 4);
+  if (qpk % 2 == 0) return with(attn_generic_kernel<T, 1, 2, true>, 1, 2);
+  with(attn_generic_kernel<T, 1, 1, true>, 1, 1);
 }
 
 extern "C" int yk_attn_generic(const void* q, int q_stride, void* out, const void* k_cache,
