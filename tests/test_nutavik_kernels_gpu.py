@@ -268,6 +268,31 @@ def test_matrix_core_form_at_every_border(heads, kv_rank, rot_dim, page, special
         assert (got[seen].view(len(seen), heads, kv_rank)[:, :, 0].cpu() > 20.0).all()
 
 
+@pytest.mark.parametrize("heads,kv_rank,rot_dim", [(2, 64, 32), (16, 256, 64), (24, 128, 32)])
+@pytest.mark.parametrize("at", [63, 66, 97])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_what_is_not_finite_stays_behind_its_token(heads, kv_rank, rot_dim, at, splits):
+    """A token whose latent is NaN, inside, at the end and at the start of a tile of several tokens: the tokens before it are what
+    they are without it, bit for bit, and those from it on are NaN."""
+    o, page, n, width = ops(), 32, 101, kv_rank + rot_dim
+    g = torch.Generator().manual_seed(at)
+    tile = o.latent_tile_tokens(heads, True)
+    dev, cpu, n_pages = context([(0, n)], page, tile_tokens=tile)
+    q, got = torch.randn(n, heads * width, generator=g) * 0.3, []
+    rows = torch.randn(n, width, generator=g) * 0.2
+    for value in (0.5, float("nan")):
+        rows[at, 3] = value
+        pages = torch.zeros(n_pages, 1, page, width)
+        bt = cpu.arrays["block_table_g0"]
+        for j in range(n):
+            pages[int(bt[0, j // page]), 0, j % page] = rows[j]
+        pages = pages.to(torch.bfloat16).cuda()
+        values = pages[..., :kv_rank].transpose(2, 3).contiguous()
+        got.append(o.latent_attention(q.cuda(), pages, heads, kv_rank, rot_dim, 0.7, dev, 0, page, tiles=dev.arrays[f"latent_tiles_{tile}"],
+                                      values=values, splits=splits))
+    assert torch.equal(got[0][:at], got[1][:at]) and got[1][at:].isnan().all() and not got[0].isnan().any()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("taps", [1, 2, 4, 5])
 def test_convolution_with_silu_and_its_state(dtype, taps):

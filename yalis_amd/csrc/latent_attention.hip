@@ -726,7 +726,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int ct = 0; ct < HALF; ++ct) acc[ct] = lat_f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  lat_u32x4_t kreg[KN], vreg[VN];
+  lat_u32x4_t kreg[KN], vreg[VN] = {};
   auto page_of = [&](int grp) { return static_cast<size_t>(bt[grp * 32 / page_size]); };
   // (a uniform base and a 32-bit offset in bytes: one register an address)
   auto fetch_k = [&](int grp) {
@@ -756,19 +756,40 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   };
   auto park_v = [&](int b, int grp) {
-    const int key_max = last - grp * 32;
+    const int key_max = last - grp * 32, seen_by_all = pos0 - grp * 32;
+    if (seen_by_all < 31) {
+      // Slots behind the last key hold whatever was there; and a later token's latents meet the weights 0 of the tile's earlier ones:
+      // what is not finite in them must not make NaN of these.  (The columns that see the token have its score from the page row.)
+      uint32_t full = 0;
+#pragma unroll
+      for (int i = 0; i < VN; ++i) {
+        const int key0 = threadIdx.x % 4 * 8;
+        LatFrag f;
+        f.u = vreg[i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (key0 + j > key_max) f.h[j] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) full |= (f.u[j] & 0x7f807f80u) + 0x00800080u;  // (an exponent of ones carries)
+        vreg[i] = f.u;
+      }
+      if (count > 1 && __any((full & 0x80008000u) != 0)) {
+#pragma unroll
+        for (int i = 0; i < VN; ++i) {
+          LatFrag f;
+          f.u = vreg[i];
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (threadIdx.x % 4 * 8 + j > seen_by_all && (f.h[j] & 0x7f80) == 0x7f80) f.h[j] = 0;
+          vreg[i] = f.u;
+        }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < VN; ++i) {
       const int e = threadIdx.x + 512 * i;
       if (VP % 512 == 0 || e < VP) {
-        LatFrag f;
-        f.u = vreg[i];
-        if (key_max < 31) {  // slots behind the last key hold whatever was there
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (e % 4 * 8 + j > key_max) f.h[j] = 0;
-        }
-        *reinterpret_cast<lat_u32x4_t*>(vbuf(b) + e / 4 * 32 + ((e % 4) ^ (e / 16 % 4)) * 8) = f.u;
+        *reinterpret_cast<lat_u32x4_t*>(vbuf(b) + e / 4 * 32 + ((e % 4) ^ (e / 16 % 4)) * 8) = vreg[i];
       }
     }
   };
