@@ -1734,18 +1734,22 @@ class HipOps:
     @staticmethod
     @functools.lru_cache(maxsize=4096)
     def latent_attention_splits(n_tiles: int, n_heads: int, max_ctx: int, n_tokens: int = 0, kv_rank: int = 512) -> int:
-        """Into how many workgroups the matrix-core form divides the keys of a tile: the power of two with the
-        smallest estimate of the longest tile's walk (0.5 us a group of 32 keys and 0.9 with a latent of 512, twice as
-        long where a compute unit has two workgroups to run) and, where the keys are divided, of the merge (5 us and the partial sums written
-        and read once).  Measured (us, 16 heads, rows of 576): eight decoded tokens behind 1,000 keys whole / in 4 / 8 /
-        16 51.5 / 24.0 / 19.0 / 17.6, behind 4,000 in 16 / 32 38 / 30; 64 behind 500 whole / in 2 / 4 / 8 35 / 29.5 /
-        29.6 / 41.8; 512 tokens behind 1,536 whole / in two 147 / 103; four prompts of 200 whole / in two 36 / 62."""
+        """Into how many workgroups the matrix-core form divides the keys of a tile: the power of two with the smallest estimate of the
+        longest tile's walk and of the merge, in us: 0.5 + 0.9 kv_rank / 512 a group of 32 keys, twice as long where a compute unit has two
+        workgroups to run; for the merge 5, 0.1 a part, and the partial sums written and read once.  Measured (us, whole / in 2 / 4 / 8 / 16 /
+        32, the choice in brackets): latent 512, 16 heads, eight decoded tokens behind 1,000 keys 50 / 33 / 23 / 18.4 / [18.3] / 18.9, 64 behind
+        500 34 / 29 / [29] / 41, 512 behind 1,536 140 / [94] / 114; latent 256, eight behind 4,000 120 / 68 / 40 / 26 / 20 / [19]; latent 128,
+        two behind 3,000 74 / 43 / 25 / 17 / 13 / [12.5] (in 64 14.7); latent 64, one behind 1,000 29 / 20 / 13 / 10 / [9.4] / 10.  A group takes 0.8,
+        0.75, 0.9 and 1.4 at latents of 64, 128, 256 and 512 in decoded tokens of up to 16 heads, but 1.0, 1.2, 1.75 and 2.8 where a prompt's
+        tiles fill all columns, which the estimate leaves out: with it 512 tokens of 8 heads from the start would be divided in four (latent
+        128 [23] / 20 / 17, 256 [33] / 28 / 24, 512 [50] / 43 / 39).  They stay whole because that other order of sums took a 456-token prompt
+        of a design whose experts are chosen by near scores past the error it is held to (0.52 against 0.5 of the logits at one position)."""
         workgroups = n_tiles * -(-n_heads // 64)
         groups = -(-max_ctx // 32)
 
         def estimate(s: int) -> float:
             walk = -(-groups // s) * (0.5 + 0.9 * kv_rank / 512) * max(1.0, workgroups * s / 256)
-            return walk if s == 1 else walk + 5.0 + max(n_tokens, n_tiles) * n_heads * s * kv_rank * 8 / 4e6
+            return walk if s == 1 else walk + 5.0 + 0.1 * s + max(n_tokens, n_tiles) * n_heads * s * kv_rank * 8 / 4e6
 
         return min((s for s in (1, 2, 4, 8, 16, 32, 64) if s <= max(groups, 1)), key=estimate)
 
