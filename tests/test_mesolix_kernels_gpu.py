@@ -127,7 +127,7 @@ def test_biased_attention_at_every_edge(dtype, head_dim, value_dim, heads, kv, s
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("heads,kv_rank,page", [(2, 64, 32), (5, 20, 16), (16, 512, 64), (3, 128, 32), (1, 130, 16), (20, 256, 32)])
+@pytest.mark.parametrize("heads,kv_rank,page", [(2, 64, 32), (5, 20, 16), (16, 512, 64), (3, 128, 32), (1, 130, 16), (20, 256, 32), (40, 64, 32), (64, 64, 32), (72, 64, 32)])
 @pytest.mark.parametrize("special", [0, 31, 32, 63, 64, 399, 400])
 def test_latent_rows_alone_with_sinks(dtype, heads, kv_rank, page, special):
     """Page rows that are the latent alone (no rotated part) and a sink per head, some so large that they take most

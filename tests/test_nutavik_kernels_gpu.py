@@ -101,17 +101,18 @@ def on_device(rot):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [24, 255, 256])
 @pytest.mark.parametrize("q_rank,kv_rank,rot_dim", [(12, 20, 6), (128, 64, 16), (96, 512, 64), (9, 5, 2)])
-def test_latent_prepare(dtype, q_rank, kv_rank, rot_dim):
+def test_latent_prepare(dtype, q_rank, kv_rank, rot_dim, n):
+    """Few tokens, and as many as the smaller workgroups take; values wider than a round of a workgroup."""
     o = ops()
     page = 16
-    dev, cpu, n_pages = context([(0, 21), (37, 1), (16, 2)], page)
-    n = 24
+    dev, cpu, n_pages = context([(0, n - 3), (37, 1), (16, 2)], page)
     g = torch.Generator().manual_seed(q_rank)
     kv_col = q_rank + (-q_rank % 8)
     proj = (torch.randn(n, kv_col + kv_rank + rot_dim + 3, generator=g) * 2).to(dtype)
     qn, kn = (torch.randn(q_rank, generator=g) * 0.3 + 1).to(dtype), (torch.randn(kv_rank, generator=g) * 0.3 + 1).to(dtype)
-    rot = rotation(rot_dim, 64)
+    rot = rotation(rot_dim, 256)
     pages_ref = torch.zeros(n_pages, 1, page, kv_rank + rot_dim, dtype=dtype)
     pages_dev = pages_ref.clone().cuda()
     values_dev = torch.zeros(n_pages, 1, kv_rank, page, dtype=dtype).cuda()
@@ -224,14 +225,15 @@ def test_head_linear_on_matrix_cores(heads, in_dim, out_dim, tail, n):
     assert (got.float().cpu() - exact.to(bf).float()).abs().max() <= 2.0 ** -7 * exact.abs().max()
 
 
-@pytest.mark.parametrize("heads,kv_rank,rot_dim,page", [(2, 64, 32, 32), (5, 128, 32, 64), (16, 512, 64, 64), (20, 256, 64, 32)])
+@pytest.mark.parametrize("heads,kv_rank,rot_dim,page", [(2, 64, 32, 32), (5, 128, 32, 64), (16, 512, 64, 64), (20, 256, 64, 32), (24, 64, 32, 32), (40, 64, 32, 64),
+                                                         (64, 64, 32, 32), (72, 64, 32, 32), (128, 128, 32, 64)])
 @pytest.mark.parametrize("special", [0, 31, 32, 63, 64, 399, 400])
 @pytest.mark.parametrize("splits", [1, 3, None])
 def test_matrix_core_form_at_every_border(heads, kv_rank, rot_dim, page, special, splits):
     """The same towering row for the matrix-core form (bfloat16 pages, the latent a second time in
     transposed pages): borders of its groups of 32 keys and of pages, tiles of several tokens where
-    heads are few and of one token's heads in chunks of 16 where they are many, the keys whole,
-    divided in three, and divided as the library decides; against float64 over the same rounded rows."""
+    heads are few (some of the tile's 64 columns idle where 64 is no multiple of them) and of one token's heads in chunks
+    of 64, the last of them ragged or full, where they are many, the keys whole, divided in three, and divided as the library decides; against float64 over the same rounded rows."""
     if kv_rank >= 256 and special not in (0, 63, 64, 400):
         pytest.skip("the largest sizes run a few of the borders")
     o = ops()
