@@ -3,7 +3,7 @@ import pytest
 import torch
 
 import kernel_refs as R
-from yalis_amd.ops.hip import HipOps
+from yalis_amd.ops.hip import HipOps, SplitSum
 
 pytestmark = pytest.mark.gpu
 _ops = {}
@@ -35,9 +35,10 @@ def test_norms_of_few_and_many_rows(n, width):
     close(o.sandwich_norm(r_dev, br.cuda(), dev(post), 0.3, dev(pre), None, torch.float32), want, 4e-6)
     close(r_dev, r_ref, 4e-6)
     r_ref, r_dev = res.clone(), res.clone().cuda()
-    R.sum_norm(r_ref, [(br, w, 1e-5), (other, w2, 1e-5)], 0.5, None, 2.0, w, 1e-5, True, torch.bfloat16)
-    o.sum_norm(r_dev, [(br.cuda(), w.cuda(), 1e-5), (other.cuda(), w2.cuda(), 1e-5)], 0.5, None, 2.0, w.cuda(), 1e-5, True, torch.bfloat16)
+    want = R.sum_norm(r_ref, [(br, w, 1e-5), (other, w2, 1e-5)], 0.5, None, 2.0, w, 1e-5, True, torch.bfloat16)
+    got = o.sum_norm(r_dev, [(br.cuda(), w.cuda(), 1e-5), (other.cuda(), w2.cuda(), 1e-5)], 0.5, None, 2.0, w.cuda(), 1e-5, True, torch.bfloat16)
     close(r_dev, r_ref, 4e-6)
+    close(got, want, 2 ** -8)  # (the rounded copy: a rounding to bfloat16 may fall to the other side)
 
 
 @pytest.mark.parametrize("kind", ["relu2", "silu", "gelu_tanh"])
@@ -52,3 +53,20 @@ def test_activation_in_pieces(kind, shape, shift):
     got, want = o.activation(x, kind, torch.bfloat16).cpu(), R.activation(flat[shift:].view(shape), kind, torch.bfloat16)
     assert torch.equal(got.isnan(), want.isnan())
     close(got.nan_to_num().float(), want.nan_to_num().float(), 2 ** -8)
+
+
+@pytest.mark.parametrize("kind", ["relu2", "silu", "gelu_tanh"])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("columns", [1020, 1021])
+@pytest.mark.parametrize("slices", [2, 8, 9, 10, 17])
+def test_activation_of_slices(slices, columns, out_dtype, kind):
+    """A product's slices, added eight at a time: one round, a full one, one and two more, two full ones, in whole pieces and in none; the
+    sum is rounded to the product's type first.  The slices are added in their order, so only the activation's own roundings remain."""
+    o, g = ops(), torch.Generator().manual_seed(slices)
+    parts = torch.randn(slices, 3, columns, generator=g)
+    total = parts[0]
+    for p in parts[1:]:
+        total = total + p
+    want = R.activation(total.to(out_dtype), kind, out_dtype)
+    got = o.activation(SplitSum(parts.cuda(), out_dtype), kind, out_dtype)
+    close(got, want, 2e-6 if out_dtype == torch.float32 else 2 ** -8)
