@@ -121,6 +121,28 @@ def test_kept_memories_are_as_exact_as_when_walked(kind, heads, dim, vdim):
     assert error["chunks"] <= 1.1 * error["walk"], error
 
 
+@pytest.mark.parametrize("kind", list(KINDS))
+def test_a_span_cut_across_forms(kind):
+    """A span whole, by chunks, against the same span cut so that its pieces take different forms: chunks and a single token, chunks and
+    a walk.  Every form makes the sums in an order of its own: the same numbers within 16 roundings of the largest, as above, twice."""
+    o, heads, dim, vdim, n = ops(), 2, 128, 64, 400
+    t, args, _ = inputs(kind, heads, heads, dim, vdim, torch.bfloat16, [n])
+    kw, got = args(lambda m: m.cuda()), []
+    for cut in (n, n - 1, 256):
+        S, rows = t["state"].cuda(), []
+        for first, last in ((0, cut), (cut, n)):
+            piece = {k: v for k, v in kw.items()}
+            for name in ("decay", "beta"):  # (tensors with a row a token)
+                if isinstance(piece[name], tuple):
+                    piece[name] = tuple(v[first:last] if torch.is_tensor(v) and v.shape[0] == n and v.dim() == 2 else v for v in piece[name])
+            if last > first:
+                rows.append(o.linear_state_scan(t["qkv"][first:last].cuda(), heads, heads, dim, vdim, S, step_of([last - first], [1]), **piece))
+        got.append((torch.cat(rows), S))
+    for y, S in got[1:]:
+        for a, b in ((y, got[0][0]), (S, got[0][1])):
+            assert (a - b).abs().max() <= 2e-6 * b.abs().max(), (a - b).abs().max() / b.abs().max()
+
+
 @pytest.mark.parametrize("kind", ["plain", "softplus_delta"])
 def test_spans_in_any_order(kind):
     """Requests listed in another order than their spans lie in the rows: the same bits."""

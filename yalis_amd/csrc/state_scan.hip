@@ -21,7 +21,8 @@
 //  fixed decay:        a constant of the model per head
 //   beta:               sigmoid(x[n, h])
 //   unit vectors:       q / sqrt(sum q^2 + eps), k likewise (with unit_eps >= 0), then q * q_scale
-// A span cut anywhere gives the same S bit for bit: every token's step is made alone.
+// A span cut into pieces that are both walked gives the same S bit for bit: every token's step is made alone.  Steps of single tokens
+// (linear_state_token_kernel) and chunks (chunk_scan.hip) add in orders of their own.
 //
 // Beside it: the read-out's norm and gate (each head's o divided by its root mean square, times a
 // weight shared by the heads, times silu or the sigmoid of a gate column), and the shift of a convolution's kept

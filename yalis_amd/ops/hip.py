@@ -797,7 +797,8 @@ class HipOps:
 
     def gemm_fma(self, x, w, out_dtype):
         """x [M, K] . w [N, K]^T with float32 arithmetic, for any types and sizes: on the float32 matrix cores where
-        an operand is float32 and rows can be read four elements at a time, else by multiply-adds."""
+        an operand is float32 and rows can be read four elements at a time, else by multiply-adds.  The order of a sum,
+        and so a row's last bits, depend on the number of rows."""
         m, k = x.shape
         n = w.shape[0]
         y = torch.empty((m, n), dtype=out_dtype, device=x.device)
@@ -1828,7 +1829,8 @@ class HipOps:
         (default 0, n_kv * dim, 2 * n_kv * dim).  ``skip`` (float32 [heads]): o += skip_h v.  ``bonus`` (float32
         [heads, dim], plain writes): o = (S + diag(bonus) k v^T)^T q of the memory before the token's decay and write.
         Steps of long spans are taken by chunks of 64 tokens in matrix products where sizes and alignment allow
-        (``STATE_CHUNKS_MIN_SPAN``); all others are walked token by token.  ``form`` ("chunks", "walk") forces one of them (tests).
+        (``STATE_CHUNKS_MIN_SPAN``: by all spans of the step), steps of single tokens by a form of theirs, all others are walked token by token;
+        the forms agree to rounding.  ``form`` ("chunks", "walk") forces one of them (tests).
         Returns o float32 [N, heads * vdim]."""
         self._rows(qkv, "linear_state_scan input")
         n = qkv.shape[0]
