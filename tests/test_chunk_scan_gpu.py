@@ -194,7 +194,8 @@ def test_steps_that_are_taken_by_chunks():
     o = ops()
     for spans, off, same, kind, heads, dim, vdim in (
             ([256], 0, "chunks", "delta", 2, 64, 16), ([255], 0, "walk", "delta", 2, 64, 16), ([256] + [1] * 2, 0, "walk", "delta", 2, 64, 16),
-            ([256], 4, "walk", "delta", 2, 64, 16), ([64, 64, 70], 0, "chunks", "channel", 8, 256, 1024), ([63, 64, 64], 0, "walk", "channel", 8, 256, 1024)):
+            ([256], 4, "walk", "delta", 2, 64, 16), ([64, 64, 70], 0, "chunks", "channel", 8, 256, 1024), ([63, 64, 64], 0, "walk", "channel", 8, 256, 1024),
+            ([100, 49], 0, "chunks", "channel", 4, 256, 1008), ([100, 48], 0, "walk", "channel", 4, 256, 1008)):
         t, args, columns = inputs(kind, heads, heads, dim, vdim, torch.bfloat16, spans)
         x = tf.pad(t["qkv"], (off, 8 - off)).cuda()
         kw = args(lambda m: m.cuda())

@@ -1808,9 +1808,12 @@ class HipOps:
     # token by token, of 160: 42 against 41), and 128 tokens a request on average, since a request of one token costs a whole chunk (512 tokens
     # with 16 requests of one: 186 against 170; 8 of 256: 108 against 151).
     STATE_CHUNKS_MIN_SPAN, STATE_CHUNKS_MIN_AVERAGE = 256, 128
-    # Heads of 256 key channels are walked at half the rate and meet earlier where there are columns (tokens * heads * vdim) to
-    # fill the chip: 4 heads of 256 x 512, 8 spans of 96 107 us against 200, of 128 110 against 272, 32 of 64 180 against 553, but one of 160 69 against 50.
-    STATE_CHUNKS_WIDE_SPAN, STATE_CHUNKS_WIDE_COLUMNS = 64, 1500000
+    # Heads of 256 key channels are walked at half the rate and meet earlier where there are columns (tokens * heads * vdim) to fill the
+    # chip.  Above the line every measured step gains, spans of one length or not (us walked / by chunks): 4 heads of 256 x 512, two of 160
+    # (0.66 M) 85 / 72, four of 96 (0.79 M) 104 / 87, 200 + 144 + four of 10 (0.79 M) 157 / 100, 255 + two of 20 (0.60 M) 127 / 79, eight of 64
+    # (1.05 M) 143 / 95; 8 heads, one of 160 (0.66 M) 86 / 69, two of 96 104 / 76; 2 heads of 256 x 256, 16 of 100 (0.82 M) 115 / 89.  Below
+    # it they part: one of 256 (0.52 M) 71 / 73, two of 128 (0.52 M) 72 / 67, one of 200 (0.41 M) 60 / 73, two of 96 (0.39 M) 56 / 67, one of 64 26 / 61.
+    STATE_CHUNKS_WIDE_SPAN, STATE_CHUNKS_WIDE_COLUMNS = 64, 600000
     # scratch for what the chunks of a step's spans are worked into (15,000 tokens of 16 heads; beyond that heads are taken by turns)
     STATE_CHUNKS_BYTES = 512 << 20
 
