@@ -143,6 +143,24 @@ def test_a_span_cut_across_forms(kind):
             assert (a - b).abs().max() <= 2e-6 * b.abs().max(), (a - b).abs().max() / b.abs().max()
 
 
+def test_a_step_without_room_for_scratch_is_walked(monkeypatch):
+    o, spans = ops(), [300]
+    t, args, _ = inputs("softplus_delta", 2, 2, 64, 16, torch.bfloat16, spans)
+    run = lambda S, form: o.linear_state_scan(t["qkv"].cuda(), 2, 2, 64, 16, S, step_of(spans, [0]), form=form, **args(lambda m: m.cuda()))
+    walked, S = t["state"].cuda(), t["state"].cuda()
+    want, empty = run(walked, "walk"), torch.empty
+
+    def full(*shape, **kw):
+        if len(shape) == 1 and isinstance(shape[0], int):
+            raise torch.OutOfMemoryError("no room")
+        return empty(*shape, **kw)
+
+    monkeypatch.setattr(torch, "empty", full)
+    assert torch.equal(run(S, None), want) and torch.equal(S, walked)
+    with pytest.raises(torch.OutOfMemoryError):
+        run(S, "chunks")
+
+
 @pytest.mark.parametrize("kind", ["plain", "softplus_delta"])
 def test_spans_in_any_order(kind):
     """Requests listed in another order than their spans lie in the rows: the same bits."""

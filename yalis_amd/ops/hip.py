@@ -1887,9 +1887,15 @@ class HipOps:
             a_head = self.lib.yk_state_scan_chunks_floats(n, n_seqs, dim, vdim, mode, write_mode, int(bonus is not None), int(skip is not None))
         if form == "chunks" and not a_head:
             raise KernelError("linear_state_scan: this step cannot be taken chunk by chunk")
+        ws = None
         if a_head and (form == "chunks" or 4 * a_head <= self.STATE_CHUNKS_BYTES):
             heads = max(1, min(n_heads, self.STATE_CHUNKS_BYTES // (4 * a_head)))
-            ws = torch.empty(heads * a_head, dtype=torch.float32, device=qkv.device)
+            try:
+                ws = torch.empty(heads * a_head, dtype=torch.float32, device=qkv.device)
+            except torch.OutOfMemoryError:  # the walk needs no such scratch
+                if form == "chunks":
+                    raise
+        if ws is not None:
             self._check(self.lib.yk_state_scan_chunks(
                 qkv.data_ptr(), qkv.stride(0), _code(qkv.dtype), n_heads, n_kv, dim, vdim, state.data_ptr(), a["seq_qstart"].data_ptr(),
                 a["seq_qlen"].data_ptr(), a["state_slots"].data_ptr(), n_seqs, n, max_qlen, float(q_scale),
