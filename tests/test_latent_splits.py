@@ -32,3 +32,14 @@ def test_keys_are_divided_as_measured(heads, latent, cached, new, requests, us):
 @pytest.mark.parametrize("keys", [1, 31, 32, 33, 64, 65])
 def test_a_part_has_keys(keys):
     assert HipOps.latent_attention_splits(1, 16, keys, 1, 512) <= -(-keys // 32)
+
+
+@pytest.mark.parametrize("heads", [1, 4, 16, 48, 64, 65, 128])
+@pytest.mark.parametrize("latent", [64, 128, 256, 512])
+def test_decode_steps_fit_the_scratch_that_captures_reserve(heads, latent):
+    """A captured step may not grow its scratch, and 1 << 24 floats are reserved: a division never makes 512 workgroups (beyond 256 it wins
+    nothing), each of which leaves 64 columns of the latent and two numbers."""
+    for requests in list(range(1, 260)) + [300, 511, 512, 1024]:
+        for keys in (256, 512, 1024, 4096, 16384, 131072, 1 << 20):
+            parts = HipOps.latent_attention_splits(requests, heads, keys, requests, latent)
+            assert parts == 1 or requests * -(-heads // 64) * parts * 64 * (latent + 2) <= 1 << 24
