@@ -16,6 +16,7 @@
 //     of heads (16 pairs at most, four to a wave), walks the keys in blocks staged once in LDS,
 //     a lane to a key for the scores and a lane to a latent column for the weighted sum.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -804,27 +805,32 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int j = 0; j < 4; ++j) s0[j] = key + j <= my_pos ? s0[j] * scale_log2 : -INFINITY;
     *reinterpret_cast<lat_f32x4_t*>(sbuf(b) + r * SROW + 16 * half + 4 * g) = s0;
   };
-  // (nothing in the walk is conditional: behind the last group it fetches, parks and scores that group again, unread)
+  // Nothing in the walk is conditional: before the last group it fetches and parks that group's rows once more, unread.  The last group is
+  // a turn of its own, which fetches, parks and scores nothing (as another turn of the walk it cost 0.5 to 1.7 us a call: one token behind
+  // ten keys, latent 64, 4.5 -> 3.7 us; eight, latent 512, 11.0 -> 9.5).
   const int g_end = g_hi - 1;
   if (g_lo < g_hi) {
     fetch_k(g_lo);
     fetch_v(g_lo);
     park_k(0);
     park_v(0, g_lo);
-    fetch_k(min(g_lo + 1, g_end));
+    if (g_lo < g_end) fetch_k(g_lo + 1);
     __syncthreads();
     if (wave_ok) scores(0, g_lo);
-    park_k(1);
+    if (g_lo < g_end) park_k(1);
   }
-  for (int grp = g_lo; grp < g_hi; ++grp) {
+  auto turn = [&](int grp, auto is_last) {
+    constexpr bool LAST = decltype(is_last)::value;
     const int b = (grp - g_lo) & 1;
-    fetch_k(min(grp + 2, g_end));
-    fetch_v(min(grp + 1, g_end));
+    if (!LAST) {
+      fetch_k(min(grp + 2, g_end));
+      fetch_v(grp + 1);
+    }
     // the rows of the next group, the latents and scores of this one are parked, and every wave is done with what is
     // written below: the rows and latents of this group's and the next one's buffers as they were two groups ago
     __syncthreads();
     if (wave_ok) {
-      scores(b ^ 1, grp + 1);
+      if (!LAST) scores(b ^ 1, grp + 1);
       // this lane: column r, keys 8 g .. 8 g + 7 of the group
       lat_f32x4_t s[2];
       s[0] = *reinterpret_cast<const lat_f32x4_t*>(sbuf(b) + r * SROW + 8 * g);
@@ -862,9 +868,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       lat_read_ahead<HALF>([&](int ct) { return *reinterpret_cast<const lat_u32x4_t*>(vcol + 16 * ct * 32); },
                            [&](int ct, const LatFrag& vf) { acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, acc[ct], 0, 0, 0); });
     }
-    park_k(b);
-    park_v(b ^ 1, min(grp + 1, g_end));
-  }
+    if (!LAST) {
+      park_k(b);
+      park_v(b ^ 1, grp + 1);
+    }
+  };
+  for (int grp = g_lo; grp < g_end; ++grp) turn(grp, std::false_type{});
+  if (g_lo < g_hi) turn(g_end, std::true_type{});
   if (!col_ok && !__any(col_ok)) return;  // (uniform: the sum below exchanges lanes)
   l = column_lanes_sum(l);
   if (!col_ok) return;
