@@ -5,19 +5,19 @@ from yalis_amd.ops.hip import HipOps
 
 # heads, latent, cached, new tokens, requests; us by parts (one MI355X, a latent's rows 32 or 64 longer)
 MEASURED = [
-    (16, 512, 0, 512, 1, {1: 50.9, 2: 48.8, 4: 68.3, 8: 111.0}),
-    (16, 512, 1536, 512, 1, {1: 140.4, 2: 93.7, 4: 113.7, 8: 158.2}),
-    (16, 512, 1000, 1, 8, {1: 50.4, 2: 33.3, 4: 23.1, 8: 18.4, 16: 18.3, 32: 18.9}),
-    (16, 512, 500, 1, 64, {1: 34.2, 2: 28.9, 4: 29.1, 8: 41.1, 16: 62.9}),
-    (32, 256, 1536, 512, 1, {1: 93.8, 2: 111.0, 4: 136.6, 8: 193.0}),
-    (16, 256, 4000, 1, 8, {1: 120.4, 2: 67.7, 4: 40.0, 8: 26.2, 16: 20.0, 32: 18.7}),
-    (16, 256, 0, 100, 8, {1: 19.0, 2: 38.8}),
-    (8, 128, 0, 2048, 1, {1: 70.2, 2: 63.2}),
-    (16, 128, 3000, 1, 2, {1: 73.5, 2: 42.5, 4: 25.3, 8: 16.7, 16: 12.9, 32: 12.5, 64: 14.7}),
-    (4, 64, 0, 512, 1, {1: 18.6, 2: 15.3, 4: 12.4, 8: 11.2, 16: 16.5, 32: 24.2}),
-    (16, 64, 0, 512, 1, {1: 19.0, 2: 20.4, 4: 23.8, 8: 32.7, 16: 49.5}),
-    (16, 64, 1000, 1, 1, {1: 28.8, 2: 19.6, 4: 13.2, 8: 10.1, 16: 9.4, 32: 10.3}),
-    (16, 64, 0, 33, 1, {1: 6.4, 2: 9.4, 4: 9.6, 8: 10.0}),
+    (16, 512, 0, 512, 1, {1: 49.7, 2: 46.9, 4: 68.0, 8: 111.0}),
+    (16, 512, 1536, 512, 1, {1: 139.2, 2: 92.6, 4: 113.9, 8: 157.1}),
+    (16, 512, 1000, 1, 8, {1: 49.1, 2: 32.1, 4: 21.9, 8: 18.2, 16: 15.7, 32: 17.3}),
+    (16, 512, 500, 1, 64, {1: 33.0, 2: 27.8, 4: 27.7, 8: 39.5, 16: 57.7}),
+    (32, 256, 1536, 512, 1, {1: 94.1, 2: 118.9, 4: 141.9, 8: 194.8}),
+    (16, 256, 4000, 1, 8, {1: 122.2, 2: 68.7, 4: 40.3, 8: 25.9, 16: 19.6, 32: 17.9}),
+    (16, 256, 0, 100, 8, {1: 17.9, 2: 37.7}),
+    (8, 128, 0, 2048, 1, {1: 70.0, 2: 69.6}),
+    (16, 128, 3000, 1, 2, {1: 79.3, 2: 44.9, 4: 26.4, 8: 16.8, 16: 12.7, 32: 11.9, 64: 14.3}),
+    (4, 64, 0, 512, 1, {1: 17.5, 2: 14.4, 4: 11.5, 8: 10.6, 16: 13.2, 32: 19.6}),
+    (16, 64, 0, 512, 1, {1: 17.9, 2: 19.4, 4: 20.4, 8: 27.4, 16: 38.9}),
+    (16, 64, 1000, 1, 1, {1: 24.1, 2: 16.9, 4: 11.5, 8: 9.1, 16: 8.5, 32: 9.2}),
+    (16, 64, 0, 33, 1, {1: 5.3, 2: 8.3, 4: 8.5, 8: 8.9}),
 ]
 
 

@@ -634,9 +634,11 @@ extern "C" int yk_latent_attention(const float* q_lat, const void* pages, int dt
 // and sum.  With n_splits > 1 the groups of keys are divided among gridDim.z workgroups, which leave
 // unnormalised sums, maxima and sums of weights for a merging kernel.
 // Bound by the LDS reads (a group of rows of 576 and latents of 512 is read four times over, 272 KiB).
-// Before (every wave walking the pages on its own, its loads not staged) / this, 16 heads, rows of 576
-// (us): a prompt of 2,048 tokens 580 / 195, 512 tokens behind 1,536 525 / 103, eight decoded tokens behind 100 keys 42 /
-// 15, behind 1,000 46 / 18, behind 4,000 63 / 30.
+// Before (every wave walking the pages on its own, its loads not staged) / this, 16 heads, rows of 576, shuffled pages
+// (us): a prompt of 2,048 tokens 757 / 217, 512 tokens behind 1,536 525 / 93, eight decoded tokens behind 100 keys 42 /
+// 14, behind 1,000 45 / 16, behind 4,000 63 / 29.  Two workgroups share a compute unit at latents of up to 128, whose registers and
+// LDS leave room for them (latent 128, a prompt of 2,048 tokens 108 -> 88 us against one; eight prompts of 100, 64 heads, 33 -> 28);
+// wider ones take all registers.
 constexpr int kLatCols = 64;  // columns of a workgroup
 typedef __bf16 lat_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float lat_f32x4_t __attribute__((ext_vector_type(4)));
@@ -675,7 +677,7 @@ constexpr size_t lat_lds_bytes() {  // two buffers each of rows, latents and sco
 }
 
 template <int KS, int CT>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_attention_mfma_kernel(
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, CT <= 8 ? 4 : 2))) void latent_attention_mfma_kernel(
     const float* __restrict__ q_lat, const bf16_t* __restrict__ kpages, const bf16_t* __restrict__ vpages,
     const int32_t* __restrict__ tiles, const int32_t* __restrict__ block_table, int table_width, int page_size,
     int n_heads, float scale_log2, int n_splits, const float* __restrict__ sink, float* __restrict__ out, float* __restrict__ ws_o,

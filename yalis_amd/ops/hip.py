@@ -1738,12 +1738,12 @@ class HipOps:
         """Into how many workgroups the matrix-core form divides the keys of a tile: the power of two with the smallest estimate of the
         longest tile's walk and of the merge, in us: 0.5 + 0.9 kv_rank / 512 a group of 32 keys, twice as long where a compute unit has two
         workgroups to run; for the merge 5, 0.1 a part, and the partial sums written and read once.  Measured (us, whole / in 2 / 4 / 8 / 16 /
-        32, the choice in brackets): latent 512, 16 heads, eight decoded tokens behind 1,000 keys 50 / 33 / 23 / 18.4 / [18.3] / 18.9, 64 behind
-        500 34 / 29 / [29] / 41, 512 behind 1,536 140 / [94] / 114; latent 256, eight behind 4,000 120 / 68 / 40 / 26 / 20 / [19]; latent 128,
-        two behind 3,000 74 / 43 / 25 / 17 / 13 / [12.5] (in 64 14.7); latent 64, one behind 1,000 29 / 20 / 13 / 10 / [9.4] / 10.  A group takes 0.8,
-        0.75, 0.9 and 1.4 at latents of 64, 128, 256 and 512 in decoded tokens of up to 16 heads, but 1.0, 1.2, 1.75 and 2.8 where a prompt's
+        32, the choice in brackets): latent 512, 16 heads, eight decoded tokens behind 1,000 keys 49 / 32 / 22 / 18.2 / [15.7] / 17.3, 64 behind
+        500 33 / 28 / [28] / 40, 512 behind 1,536 139 / [93] / 114; latent 256, eight behind 4,000 122 / 69 / 40 / 26 / 20 / [18]; latent 128,
+        two behind 3,000 79 / 45 / 26 / 17 / 13 / [12] (in 64 14.3); latent 64, one behind 1,000 24 / 17 / 12 / 9.1 / [8.5] / 9.2.  A group takes 0.7,
+        0.8, 0.9 and 1.4 at latents of 64, 128, 256 and 512 in decoded tokens of up to 16 heads, but 1.0, 1.2, 1.75 and 2.8 where a prompt's
         tiles fill all columns, which the estimate leaves out: with it 512 tokens of 8 heads from the start would be divided in four (latent
-        128 [23] / 20 / 17, 256 [33] / 28 / 24, 512 [50] / 43 / 39).  They stay whole because that other order of sums took a 456-token prompt
+        128 [23] / 20 / 16, 256 [32] / 27 / 23, 512 [49] / 42 / 38).  They stay whole because that other order of sums took a 456-token prompt
         of a design whose experts are chosen by near scores past the error it is held to (0.52 against 0.5 of the logits at one position)."""
         workgroups = n_tiles * -(-n_heads // 64)
         groups = -(-max_ctx // 32)
