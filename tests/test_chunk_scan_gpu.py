@@ -242,3 +242,18 @@ def test_scan_of_single_tokens(kind, heads, kv, dim, vdim, dtype):
             err = (m.double().cpu() - ref).abs().max().item() / ref.abs().max().item()
             assert err <= 1e-6, (spans, err)
         assert torch.equal(S[[1, 3]].cpu(), t["state"][[1, 3]]), "slots outside the step stay as they are"
+
+
+def test_chunks_need_the_longest_span():
+    """A step that does not say how long its longest span is cannot be cut into chunks: refused where the form is forced, else walked."""
+    o, spans = ops(), [300]
+    t, args, _ = inputs("softplus_delta", 2, 2, 64, 16, torch.bfloat16, spans)
+    ctx, got = step_of(spans, [0]), []
+    run = lambda S, form: o.linear_state_scan(t["qkv"].cuda(), 2, 2, 64, 16, S, ctx, form=form, **args(lambda m: m.cuda()))
+    S = t["state"].cuda()
+    want = run(S, "walk")
+    del ctx.max_qlen
+    walked = t["state"].cuda()
+    assert torch.equal(run(walked, None), want) and torch.equal(walked, S)
+    with pytest.raises(RuntimeError, match="chunk by chunk"):
+        run(t["state"].cuda(), "chunks")

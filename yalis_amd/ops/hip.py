@@ -1883,7 +1883,7 @@ class HipOps:
         aligned = qkv.stride(0) % 8 == 0 and q_col % 8 == 0 and k_col % 8 == 0 and qkv.data_ptr() % 16 == 0
         long = max_qlen >= self.STATE_CHUNKS_MIN_SPAN and n >= self.STATE_CHUNKS_MIN_AVERAGE * n_seqs
         long = long or (dim == 256 and n >= self.STATE_CHUNKS_WIDE_SPAN * n_seqs and n * n_heads * vdim >= self.STATE_CHUNKS_WIDE_COLUMNS)
-        if aligned and (form == "chunks" or (form is None and long and max_qlen > 1)):
+        if aligned and max_qlen > 0 and (form == "chunks" or (form is None and long and max_qlen > 1)):  # (0: a step that does not say)
             a_head = self.lib.yk_state_scan_chunks_floats(n, n_seqs, dim, vdim, mode, write_mode, int(bonus is not None), int(skip is not None))
         if form == "chunks" and not a_head:
             raise KernelError("linear_state_scan: this step cannot be taken chunk by chunk")
