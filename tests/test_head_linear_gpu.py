@@ -18,10 +18,22 @@ def ops():
 @pytest.mark.parametrize("in_dim,out_dim", [(1, 2), (31, 62), (32, 64), (33, 66), (256, 130), (257, 64), (1000, 48), (40, 33), (1500, 20)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_head_products_by_pairs(dtype, in_dim, out_dim, n):
-    """Fewer elements than slices, one more and one less than a round of weights, columns that do not fill a tile, an odd number of
+    """Few elements (one column a thread), as many as slices and one more, one more and one less than a round of weights, columns that do not fill a tile, an odd number of
     columns and heads too long for the pairs' workspace (both one column a thread).  A sum of in_dim products in float32, by slices: within 8
     roundings (2^-24) of the sum of their sizes."""
-    o, h = ops(), 3
+    check(3, n, in_dim, out_dim, dtype)
+
+
+@pytest.mark.parametrize("h,n", [(32, 8), (33, 8), (64, 8), (64, 16), (65, 16), (64, 9), (16, 32), (17, 32)])
+@pytest.mark.parametrize("in_dim", [31, 32, 33, 47, 48, 63, 64, 65, 95, 96, 127, 128, 129])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_where_pairs_end(dtype, in_dim, h, n):
+    """Both sides of the lines in input elements and in workgroups (a head's 512 columns are eight of them for every eight tokens)."""
+    check(h, n, in_dim, 512, dtype)
+
+
+def check(h, n, in_dim, out_dim, dtype):
+    o = ops()
     g = torch.Generator().manual_seed(in_dim + n)
     x = torch.randn(n, h * in_dim, generator=g).to(dtype)
     w = torch.randn(h, in_dim, out_dim, generator=g).to(dtype)

@@ -291,12 +291,18 @@ extern "C" int yk_head_linear(const void* x, int x_stride, int x_dtype, const vo
   YK_REQUIRE(tail == 0 || (positions != nullptr && cos_t != nullptr && sin_t != nullptr), "head_linear: a turned tail needs positions and tables");
   const size_t lds = sizeof(float) * (static_cast<size_t>(kHeadTokens) * (in_dim + tail) + kHeadSlices * kHeadTokens * kHeadOut);
   const size_t pair_lds = sizeof(float) * (static_cast<size_t>(kHeadTokens) * (in_dim + tail) + kPairSlices / 2 * kHeadTokens * kHeadOut);
-  // (many tokens of few elements are better off with the smaller workgroups: 512 tokens of 32 heads, float32, 128 -> 512 93 us against
-  // 114, 512 -> 128 99 against 63)
-  const bool pairs = (n_tokens <= 32 || in_dim >= 256) && out_dim % 2 == 0 && reinterpret_cast<uintptr_t>(w) % 8 == 0 && pair_lds <= 64 * 1024;
+  // Pairs win by how long a thread's chain of weights is, and lose by their larger workgroups, of which a compute unit runs one.  Up to 32
+  // tokens, time over head_linear_kernel's by workgroups (256 / 512 / 1,024 / 2,048): float32 weights, 32 input elements 1.15 / 1.35 / 1.75 /
+  // 2.1, 64 0.94 / 1.11 / 1.3 / 1.55, 96 0.81 / 0.96 / 1.2 / 1.3, 128 0.71 / 0.8 / 0.98 / 1.13, 192 0.58 / 0.65 / 0.85 / 0.97; bfloat16 ones are about
+  // as those of twice the elements (32 0.93 / 1.1 / 1.5 / 1.8, 64 0.73 / 0.87 / 1.13 / 1.35, 96 0.6 / 0.71 / 0.96 / 1.06, 128 0.51 / 0.63 / 0.75 / 0.87).  More tokens
+  // (float32): 512 of 32 heads, 128 -> 512 93 us against 114, 512 -> 128 99 against 63.
+  const dim3 grid((n_tokens + kHeadTokens - 1) / kHeadTokens, n_heads, (out_dim + kHeadOut - 1) / kHeadOut);
+  const long long workgroups = static_cast<long long>(grid.x) * grid.y * grid.z;
+  const int chain = w_dtype == YK_F32 ? in_dim : 2 * in_dim;
+  const bool few = n_tokens <= 32 && (chain >= 192 || workgroups <= (chain >= 128 ? 1024 : chain >= 96 ? 512 : chain >= 64 ? 256 : 0));
+  const bool pairs = (few || in_dim >= 256) && out_dim % 2 == 0 && reinterpret_cast<uintptr_t>(w) % 8 == 0 && pair_lds <= 64 * 1024;
   YK_REQUIRE(lds <= 64 * 1024, "head_linear: heads of more than 1,700 input elements do not fit");
   if (n_tokens == 0) return 0;
-  dim3 grid((n_tokens + kHeadTokens - 1) / kHeadTokens, n_heads, (out_dim + kHeadOut - 1) / kHeadOut);
   const int out_stride = n_heads * (out_dim + tail);
   if (gate == nullptr) gate_dtype = out_dtype;
 #define YK_CASE(XD, TX, WD, TW, GD, TG, OD, TO)                                                                      \
