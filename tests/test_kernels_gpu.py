@@ -1167,6 +1167,36 @@ def test_sample_divided_rows(ops, kind):
             assert got[i].item() == want, (kind, i, settings[i], draw, got[i].item(), want)
 
 
+@pytest.mark.parametrize("vocab", [8192, 8195, 16385, 128256, 131077])
+def test_sample_small_top_k(ops, vocab):
+    """Rows with a small top_k are settled among what stretches of the row hand on, with the word
+    that all rows are such or without it: the tokens of the whole-row path, at the largest top_k
+    that is settled so, one more, ties with the top_k-th, more ties than are handed on, and rows
+    with masked logits, at lengths whose rows start off 16 bytes."""
+    gen = torch.Generator().manual_seed(vocab)
+    rows = 9
+    logits = torch.randn((rows, vocab), generator=gen) * 2.5
+    logits[1] = logits[1].round()  # hundreds of equal logits
+    logits[2, ::2] = float("-inf")
+    logits[3, : vocab - 3] = float("-inf")  # fewer finite logits than top_k
+    logits[4] = 1.5  # all equal: more than are handed on
+    logits[5, 100:140] += 9.0
+    logits[6] -= 200.0
+    logits[7] = torch.sort(logits[7]).values  # a thread's largest logits lie side by side
+    dev = logits.to(DEV)
+    seeds = torch.arange(rows, dtype=torch.int32, device=DEV) + 3
+    for k, top_p, temperature in [(1, 1.0, 1.0), (50, 0.8, 0.7), (50, 1.0, 1.3), (128, 0.95, 1.0), (129, 0.95, 1.0), (5, 0.0, 1.0)]:
+        full = lambda v, dt: torch.full((rows,), v, dtype=dt, device=DEV)
+        t = full(temperature, torch.float32)
+        t[8] = 0.0
+        args = (dev, t, full(k, torch.int32), full(top_p, torch.float32), seeds, full(k, torch.int32))
+        want = ops.sample(*args, whole_row=True).tolist()
+        paths = full(-1, torch.int32)
+        assert ops.sample(*args, most_top_k=k, paths=paths).tolist() == want, (k, top_p)
+        assert paths[8].item() == 0 and paths[0].item() == 3
+        assert ops.sample(*args).tolist() == want, (k, top_p)
+
+
 def test_sample_rows_are_independent(ops):
     """Many rows with different settings in one launch give what each gives alone."""
     vocab = 50000

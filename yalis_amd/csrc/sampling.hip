@@ -39,6 +39,11 @@ __device__ __forceinline__ uint32_t order_key(float f) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// and back
+__device__ __forceinline__ float order_value(uint32_t key) {
+  return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key);
+}
+
 struct ArgMax {
   float v;
   int i;
@@ -305,6 +310,22 @@ __device__ int sample_whole_row(const float* __restrict__ row, int vocab, ArgMax
 // wave finds among them.  Masses are summed as integers (units of 2^-40 of the largest
 // token's), so that sums do not depend on their order and a sum over bins equals the sum
 // over their tokens.  A row whose candidates do not fit is left to the one-workgroup kernel.
+//
+// A row with a small top_k needs none of the bins: its kept tokens are among the top_k largest of
+// every stretch of the row.  The pass that looks for the largest logit holds its stretch in
+// registers and writes those tokens out, and one more workgroup a row finds the exact thresholds
+// among them and draws (sp_extent_kernel, sp_settle_kernel).  Where the caller says that all rows
+// are such rows or greedy, these two are all that is launched.  Bound by the launches and the chain
+// inside the second kernel.  128,256 logits a row, top_k 50, top_p 0.8, us a call:
+//   1 row 51 -> 29 (seven kernels -> two), 8 rows 52 -> 22 to 29 (small launches in a row / alone),
+//   64 rows 70 to 73 -> 38.  Rows under plain temperature or top_p alone pay for the shared first
+//   pass: 38.2 -> 38.8 at 8 rows, 56 -> 59 at 64.
+// Stretches of 16,384 rather than 8,192 logits: 35 against 43 at 64 rows, 29 against 28 at one.
+constexpr int SP_PART = 16384;        // logits a workgroup of sp_extent_kernel holds at most
+constexpr int SP_PART_KEEP = 512;     // tokens that such a stretch hands on at most
+constexpr int SP_SETTLE_K = 128;      // largest top_k that is settled that way
+constexpr int SP_SETTLE_TOKENS = 3072;  // and how many tokens its stretches may hand on, without ties
+constexpr int SP_KEPT_MAX = 1024;     // tokens at least as likely as the top_k-th, ties among them
 constexpr int SP_CHUNKS = 8;
 constexpr int SP_BINS = 1024;
 constexpr int SP_THREADS = 1024;
@@ -344,19 +365,37 @@ __device__ __forceinline__ void sp_chunk(int vocab, int chunk, int& lo, int& hi)
   hi = min(vocab, lo + per);
 }
 
-// The largest logit of a row and the scale of its bins, from the chunks' parts.
+// Stretches of a row, their length (starts stay 16-byte aligned) and the largest top_k that is
+// settled among what they hand on.
+__host__ __device__ __forceinline__ int sp_parts(int vocab) { return (vocab + SP_PART - 1) / SP_PART; }
+__device__ __forceinline__ void sp_part(int vocab, int part, int& lo, int& hi) {
+  const int n = sp_parts(vocab), per = ((vocab + n - 1) / n + 3) & ~3;
+  lo = min(vocab, part * per);
+  hi = min(vocab, lo + per);
+}
+__host__ __device__ __forceinline__ int sp_settle_limit(int vocab) {
+  const int fits = SP_SETTLE_TOKENS / sp_parts(vocab);
+  return fits < SP_SETTLE_K ? fits : SP_SETTLE_K;
+}
+
+// The largest logit of a row and the scale of its bins, from the stretches' parts.
 struct SampleExtent {
   ArgMax best;
   float top, bin_scale;
 };
 __device__ __forceinline__ SampleExtent sp_extent(const ArgMax* __restrict__ part_best,
-                                                  const float* __restrict__ part_low, float inv_t) {
+                                                  const float* __restrict__ part_low, int parts, float inv_t) {
   SampleExtent x;
   x.best = ArgMax{-INFINITY, 0x7fffffff};
   float low = INFINITY;
-  for (int c = 0; c < SP_CHUNKS; ++c) {
+  for (int c = threadIdx.x % 64; c < parts; c += 64) {
     x.best = better(x.best, part_best[c]);
     low = fminf(low, part_low[c]);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    x.best = better(x.best, ArgMax{__shfl_xor(x.best.v, o, 64), __shfl_xor(x.best.i, o, 64)});
+    low = fminf(low, __shfl_xor(low, o, 64));
   }
   x.top = x.best.v * inv_t;
   const float far = -sp_exponent(low, inv_t, x.top);  // the smallest finite logit's distance
@@ -371,7 +410,8 @@ __device__ __forceinline__ T sp_wave_sum(T v) {
   return v;
 }
 
-// Per row: temperature, top_k (0: off), top_p, seed, draw.
+// The token of a row, for every thread of the workgroup: temperature, top_k (0: off), top_p, seed,
+// draw.
 //
 // With top_k or top_p the tokens that can be kept are first narrowed down: passes over the
 // row count the keys at or above 15 thresholds at once (four bits of the threshold a pass)
@@ -379,36 +419,8 @@ __device__ __forceinline__ T sp_wave_sum(T v) {
 // number (k, or CAND_MAX itself for top_p alone); those are copied to LDS in index order
 // (each wave owns a stretch of the row, so the order does not depend on timing) and the
 // exact thresholds, the sums and the race are done there.
-__global__ __launch_bounds__(1024) void sample_kernel(
-    const float* __restrict__ logits, int32_t* __restrict__ out, int vocab,
-    const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
-    const float* __restrict__ top_p, const int32_t* __restrict__ seeds,
-    const int32_t* __restrict__ draws, int force_whole_row, const SamplePlan* __restrict__ plans,
-    const ArgMax* __restrict__ race_part, int32_t* __restrict__ paths_out) {
-  __shared__ SampleShared sh;
-  const int rowi = blockIdx.x;
-  if (plans) {
-    // the row was divided among workgroups: finish what they left, or do the whole row here
-    const SamplePlan& plan = plans[rowi];
-    if (paths_out && threadIdx.x == 0) paths_out[rowi] = plan.path;
-    if (plan.path == SP_DONE) return;
-    if (plan.path == SP_GREEDY) {
-      if (threadIdx.x == 0) out[rowi] = plan.best_i == 0x7fffffff ? 0 : plan.best_i;
-      return;
-    }
-    if (plan.path == SP_RACE) {
-      if (threadIdx.x == 0) {
-        ArgMax win{-INFINITY, 0x7fffffff};
-        for (int c = 0; c < SP_CHUNKS; ++c) win = better(win, race_part[rowi * SP_CHUNKS + c]);
-        out[rowi] = win.i == 0x7fffffff ? plan.best_i : win.i;
-      }
-      return;
-    }
-  }
-  const float* row = logits + static_cast<size_t>(rowi) * vocab;
-  const float temp = temperature[rowi];
-  const int k = top_k[rowi];
-  const float p_lim = top_p[rowi];
+__device__ __forceinline__ int sample_row(const float* __restrict__ row, int vocab, float temp, int k, float p_lim, int32_t seed,
+                                          int32_t draw, bool force_whole_row, SampleShared& sh) {
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, n_waves = blockDim.x / 64;
 
   // the largest logit and its index
@@ -416,13 +428,12 @@ __global__ __launch_bounds__(1024) void sample_kernel(
   for_each_logit(row, vocab, [&](float x, int i) { best = better(best, ArgMax{x, i}); });
   best = block_argmax(best, sh.ascratch);
   if (temp <= 0.f) {
-    if (threadIdx.x == 0) out[rowi] = best.i == 0x7fffffff ? 0 : best.i;
-    return;
+    return best.i == 0x7fffffff ? 0 : best.i;
   }
   const float inv_t = 1.f / temp;
   const float top = best.v * inv_t;
-  const uint64_t base = mix64((static_cast<uint64_t>(static_cast<uint32_t>(seeds[rowi])) << 32) |
-                              static_cast<uint32_t>(draws[rowi]));
+  const uint64_t base = mix64((static_cast<uint64_t>(static_cast<uint32_t>(seed)) << 32) |
+                              static_cast<uint32_t>(draw));
   const bool k_active = k > 0 && k < vocab;
   const bool p_active = p_lim < 1.f;
 
@@ -438,8 +449,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(
       win = better(win, ArgMax{expf(x * inv_t - top) / z / -logf(u), i});
     });
     win = block_argmax(win, sh.ascratch);
-    if (threadIdx.x == 0) out[rowi] = win.i == 0x7fffffff ? best.i : win.i;
-    return;
+    return win.i == 0x7fffffff ? best.i : win.i;
   }
 
   // ---- narrow down: the largest bound with count(key >= bound) >= want, four bits a pass
@@ -484,11 +494,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(
     bits_done += 4;
   }
   fits = fits && n_ge <= CAND_MAX;
-  if (!fits) {
-    const int tok = sample_whole_row(row, vocab, best, inv_t, k, p_lim, base, sh);
-    if (threadIdx.x == 0) out[rowi] = tok;
-    return;
-  }
+  if (!fits) return sample_whole_row(row, vocab, best, inv_t, k, p_lim, base, sh);
 
   // ---- copy the candidates (key >= bound) to LDS in index order: wave w owns the w-th stretch
   const int per_wave = (vocab + n_waves - 1) / n_waves;
@@ -552,11 +558,7 @@ __global__ __launch_bounds__(1024) void sample_kernel(
       float mass = 0.f;
       for (int j = threadIdx.x; j < n_cand; j += blockDim.x) mass += sh.e[j];
       mass = block_sum(mass, sh.fscratch);
-      if (!(mass > p_lim * z) && n_cand < vocab) {
-        const int tok = sample_whole_row(row, vocab, best, inv_t, k, p_lim, base, sh);
-        if (threadIdx.x == 0) out[rowi] = tok;
-        return;
-      }
+      if (!(mass > p_lim * z) && n_cand < vocab) return sample_whole_row(row, vocab, best, inv_t, k, p_lim, base, sh);
     }
     uint32_t t = 0u;
     for (int bit = 31; bit >= 0; --bit) {
@@ -588,45 +590,374 @@ __global__ __launch_bounds__(1024) void sample_kernel(
     }
   }
   win = block_argmax(win, sh.ascratch);
-  if (threadIdx.x == 0) out[rowi] = win.i == 0x7fffffff ? best.i : win.i;
+  return win.i == 0x7fffffff ? best.i : win.i;
 }
 
-// ---- 1: the largest and the smallest finite logit of each chunk
+__global__ __launch_bounds__(1024) void sample_kernel(
+    const float* __restrict__ logits, int32_t* __restrict__ out, int vocab,
+    const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+    const float* __restrict__ top_p, const int32_t* __restrict__ seeds,
+    const int32_t* __restrict__ draws, int force_whole_row, const SamplePlan* __restrict__ plans,
+    const ArgMax* __restrict__ race_part, int32_t* __restrict__ paths_out) {
+  __shared__ SampleShared sh;
+  const int rowi = blockIdx.x;
+  if (plans) {
+    // the row was divided among workgroups: finish what they left, or do the whole row here
+    const SamplePlan& plan = plans[rowi];
+    if (paths_out && threadIdx.x == 0) paths_out[rowi] = plan.path;
+    if (plan.path == SP_DONE || plan.path == SP_GREEDY) return;
+    if (plan.path == SP_RACE) {
+      if (threadIdx.x == 0) {
+        ArgMax win{-INFINITY, 0x7fffffff};
+        for (int c = 0; c < SP_CHUNKS; ++c) win = better(win, race_part[rowi * SP_CHUNKS + c]);
+        out[rowi] = win.i == 0x7fffffff ? plan.best_i : win.i;
+      }
+      return;
+    }
+  }
+  const int token = sample_row(logits + static_cast<size_t>(rowi) * vocab, vocab, temperature[rowi], top_k[rowi], top_p[rowi],
+                               seeds[rowi], draws[rowi], force_whole_row != 0, sh);
+  if (threadIdx.x == 0) out[rowi] = token;
+}
+
+// A bound that at least k of the workgroup's keys reach, and not many more: keys are put into
+// SP_BINS bins by their distance from the largest; the bin that holds the k-th is divided again
+// where it holds too many (logits of both signs: their keys lie far apart), at most four times.
+struct KeyBins {
+  uint32_t count[SP_BINS];
+  uint32_t wave[SP_BINS / 64];
+  uint32_t low, high;      // of the keys
+  uint32_t first, before;  // the bin that holds the k-th largest key, and how many lie in bins before it
+};
+struct KeyBound {
+  uint32_t key;           // the bound
+  uint32_t above, edge;   // keys above its bin, keys of its bin
+  uint32_t bin_high;      // the largest key that the bin can hold
+};
+__device__ __forceinline__ void sp_clear_bins(KeyBins& b) {
+  b.count[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) b.first = SP_BINS - 1, b.before = 0u;
+}
+__device__ __forceinline__ void sp_clear_range(KeyBins& b) {
+  sp_clear_bins(b);
+  if (threadIdx.x == 0) b.low = 0xffffffffu, b.high = 0u;
+}
+// after a barrier; another has to follow
+__device__ __forceinline__ void sp_key_range(KeyBins& b, uint32_t least, uint32_t most) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    least = min(least, static_cast<uint32_t>(__shfl_xor(least, o, 64)));
+    most = max(most, static_cast<uint32_t>(__shfl_xor(most, o, 64)));
+  }
+  if (threadIdx.x % 64 == 0) {
+    atomicMin(&b.low, least);
+    atomicMax(&b.high, most);
+  }
+}
+// each(f) calls f with the thread's keys, of which the workgroup of SP_BINS threads has at least k;
+// ends when at most k + slack keys reach the bound, or only equal ones are left to part
+template <typename Each>
+__device__ __forceinline__ KeyBound sp_find_bound(KeyBins& b, uint32_t k, uint32_t slack, Each each) {
+  static_assert(SP_BINS == 1 << 10 && SP_BINS == SP_THREADS);
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  KeyBound bound{0u, 0u, 0u, b.high};
+  int bits = max(0, 22 - __clz(static_cast<int>((b.high - b.low) | 1u)));  // of a key, that a bin spans
+  while (true) {
+    each([&](uint32_t key) {
+      const uint32_t bin = (bound.bin_high - key) >> bits;
+      if (key <= bound.bin_high && bin < SP_BINS) atomicAdd(&b.count[bin], 1u);
+    });
+    __syncthreads();
+    const uint32_t mine = b.count[threadIdx.x];
+    uint32_t to = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(to, o, 64);
+      if (lane >= o) to += y;
+    }
+    if (lane == 63) b.wave[wave] = to;
+    __syncthreads();
+    to += bound.above;
+#pragma unroll
+    for (int w = 0; w < SP_BINS / 64; ++w) to += w < wave ? b.wave[w] : 0u;
+    if (to >= k && to - mine < k) b.first = threadIdx.x, b.before = to - mine;
+    __syncthreads();
+    const uint32_t first = b.first;
+    bound.above = b.before;
+    bound.edge = b.count[first];
+    bound.bin_high -= first << bits;
+    const uint32_t span = (1u << bits) - 1u;
+    bound.key = bound.bin_high > span ? bound.bin_high - span : 0u;
+    if (bits == 0 || bound.above + bound.edge <= k + slack) return bound;
+    __syncthreads();
+    sp_clear_bins(b);
+    __syncthreads();
+    bits = max(0, bits - 10);
+  }
+}
+
+// ---- 1: the largest and the smallest finite logit of each stretch, and of a row with a small top_k
+// the stretch's tokens that can be among the row's top_k
+// The stretch is held in registers.  k threads whose largest logit reaches a bound hold k tokens that
+// do: the bound is sought over the threads' largest alone, and what reaches it is handed on in any order.
 __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __restrict__ logits, int vocab,
-                                                               ArgMax* __restrict__ part_best,
-                                                               float* __restrict__ part_low) {
+                                                               const float* __restrict__ temperature,
+                                                               const int32_t* __restrict__ top_k, ArgMax* __restrict__ part_best,
+                                                               float* __restrict__ part_low, uint32_t* __restrict__ top_key,
+                                                               int32_t* __restrict__ top_idx, int32_t* __restrict__ top_count) {
   __shared__ ArgMax ascratch[17];
   __shared__ float fscratch[17];
-  const int rowi = blockIdx.x, chunk = blockIdx.y;
-  const float* row = logits + static_cast<size_t>(rowi) * vocab;
+  __shared__ KeyBins bins;
+  __shared__ int handed;
+  constexpr int PER = SP_PART / SP_THREADS;
+  const int rowi = blockIdx.x, tid = threadIdx.x;
+  const int k = temperature[rowi] > 0.f ? top_k[rowi] : 0;
   int lo, hi;
-  sp_chunk(vocab, chunk, lo, hi);
+  sp_part(vocab, blockIdx.y, lo, hi);
+  const int n = hi - lo;
+  const float* from = logits + static_cast<size_t>(rowi) * vocab + lo;
+  // four consecutive logits a load where the row is 16-byte aligned, else one
+  const bool wide = reinterpret_cast<uintptr_t>(from) % 16 == 0;
+  auto place = [&](int j) { return wide ? 4 * (tid + j / 4 * SP_THREADS) + j % 4 : tid + j * SP_THREADS; };
+  float v[PER];
+#pragma unroll
+  for (int q = 0; q < PER / 4; ++q) {
+    const int at = place(4 * q);
+    if (wide && at + 3 < n) {
+      const float4 x = *reinterpret_cast<const float4*>(from + at);
+      v[4 * q] = x.x;
+      v[4 * q + 1] = x.y;
+      v[4 * q + 2] = x.z;
+      v[4 * q + 3] = x.w;
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[4 * q + c] = place(4 * q + c) < n ? from[place(4 * q + c)] : -INFINITY;
+    }
+  }
   ArgMax best{-INFINITY, 0x7fffffff};
   float neg_low = -INFINITY;
-  for_each_logit(row + lo, hi - lo, [&](float x, int i) {
-    best = better(best, ArgMax{x, lo + i});
-    if (x > -INFINITY) neg_low = fmaxf(neg_low, -x);
-  });
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    // (what stands for a place beyond the stretch never wins: it is -INFINITY, its index the larger)
+    best = better(best, ArgMax{v[j], lo + place(j)});
+    if (v[j] > -INFINITY) neg_low = fmaxf(neg_low, -v[j]);
+  }
+  sp_clear_range(bins);
+  if (tid == 0) handed = 0;
   best = block_argmax(best, ascratch);
+  if (best.v == -INFINITY && best.i >= hi) best.i = 0x7fffffff;
   neg_low = block_max(neg_low, fscratch);
+  const size_t part = static_cast<size_t>(rowi) * gridDim.y + blockIdx.y;
+  if (tid == 0) {
+    part_best[part] = best;
+    part_low[part] = -neg_low;
+  }
+  if (k < 1 || k > sp_settle_limit(vocab)) return;
+
+  uint32_t mine = 0;  // the thread's largest key; 0: it has none
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (place(j) < n) mine = max(mine, order_key(v[j]));
+  uint32_t bound = 1;
+  if (n > SP_PART_KEEP) {  // else all are handed on; there are more than SP_PART_KEEP / 4 >= k threads with logits
+    sp_key_range(bins, mine ? mine : 0xffffffffu, mine);
+    __syncthreads();
+    bound = sp_find_bound(bins, k, 32, [&](auto take) {
+      if (mine) take(mine);
+    }).key;
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const uint32_t key = order_key(v[j]);
+    if (place(j) < n && key >= bound) {
+      const int slot = atomicAdd(&handed, 1);
+      if (slot < SP_PART_KEEP) {
+        top_key[part * SP_PART_KEEP + slot] = key;
+        top_idx[part * SP_PART_KEEP + slot] = lo + place(j);
+      }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) top_count[part] = handed;
+}
+
+// ---- greedy rows, and rows with a small top_k from what their stretches handed on
+// The exact thresholds, sums and the race as in sp_choose_kernel (the same values: masses are sums of
+// integers).  A key's mass of all that are at least as large is summed by one thread a kept token,
+// since they are few.  Returns the row's token and which way it went, or SP_WHOLE_ROW.
+struct SettleShared {
+  uint32_t key[CAND_MAX];
+  int32_t idx[CAND_MAX];
+  uint32_t kept_key[SP_KEPT_MAX];
+  int32_t kept_idx[SP_KEPT_MAX];
+  sp_mass_t kept_mass[SP_KEPT_MAX];
+  ArgMax ascratch[17];
+  KeyBins bins;
+  uint32_t edge[SP_KEPT_MAX];  // the keys of the bin that holds the top_k-th
+  sp_mass_t mass_sum;
+  uint32_t p_found;
+  int taken, misfit, n_kept, n_edge;
+};
+struct Settled {
+  int path, token;
+};
+__device__ __forceinline__ bool sp_settles(float temp, int k, int vocab) {
+  return temp <= 0.f || (k >= 1 && k <= sp_settle_limit(vocab));
+}
+
+__device__ __forceinline__ Settled sp_settle(int rowi, int vocab, float temp, int k, float p_lim, int32_t seed, int32_t draw,
+                                             const ArgMax* __restrict__ part_best, const uint32_t* __restrict__ top_key,
+                                             const int32_t* __restrict__ top_idx, const int32_t* __restrict__ top_count,
+                                             SettleShared& st) {
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, n_waves = blockDim.x / 64;  // SP_BINS threads
+  const int parts = sp_parts(vocab);
+  const size_t first = static_cast<size_t>(rowi) * parts;
+  // a wave's first stretch: what it handed on is asked for before its number is known
+  uint32_t key0 = 0u;
+  int32_t idx0 = 0;
+  if (temp > 0.f && wave < parts) {
+    key0 = top_key[(first + wave) * SP_PART_KEEP + lane];
+    idx0 = top_idx[(first + wave) * SP_PART_KEEP + lane];
+  }
+  ArgMax best{-INFINITY, 0x7fffffff};
+  for (int c = tid; c < parts; c += blockDim.x) best = better(best, part_best[first + c]);
+  if (tid == 0) {
+    st.taken = st.misfit = st.n_kept = st.n_edge = 0;
+    st.mass_sum = 0ull;
+    st.p_found = 0u;
+  }
+  sp_clear_range(st.bins);
+  best = block_argmax(best, st.ascratch);
+  if (temp <= 0.f) return Settled{SP_GREEDY, best.i == 0x7fffffff ? 0 : best.i};
+  uint32_t least = 0xffffffffu, most = 0u;
+  for (int c = wave; c < parts; c += n_waves) {
+    const int count = top_count[first + c];
+    int at = 0;
+    if (lane == 0) {
+      at = atomicAdd(&st.taken, count);
+      if (count > SP_PART_KEEP) st.misfit = 1;
+    }
+    at = __shfl(at, 0, 64);
+    for (int j = lane; j < min(count, SP_PART_KEEP); j += 64) {
+      const bool asked = c == wave && j == lane;
+      const uint32_t key = asked ? key0 : top_key[(first + c) * SP_PART_KEEP + j];
+      const int32_t idx = asked ? idx0 : top_idx[(first + c) * SP_PART_KEEP + j];
+      if (at + j < CAND_MAX) {
+        st.key[at + j] = key;
+        st.idx[at + j] = idx;
+        least = min(least, key);
+        most = max(most, key);
+      }
+    }
+  }
+  sp_key_range(st.bins, least, most);
+  __syncthreads();
+  const int n = st.taken;
+  if (st.misfit || n > CAND_MAX || n < k) return Settled{SP_WHOLE_ROW, 0};
+  const KeyBound bound = sp_find_bound(st.bins, k, 64, [&](auto take) {
+    for (int j = tid; j < n; j += blockDim.x) take(st.key[j]);
+  });
+  const uint32_t reach = bound.above + bound.edge;
+  if (reach > SP_KEPT_MAX) return Settled{SP_WHOLE_ROW, 0};
+  if (reach > static_cast<uint32_t>(k)) {
+    for (int j = tid; j < n; j += blockDim.x) {
+      const uint32_t key = st.key[j];
+      if (key >= bound.key && key <= bound.bin_high) st.edge[atomicAdd(&st.n_edge, 1)] = key;
+    }
+    __syncthreads();
+  }
+  const int n_edge = st.n_edge;
+
+  const float inv_t = 1.f / temp, top = best.v * inv_t;
+  sp_mass_t m = 0ull;
+  for (int j = tid; j < n; j += blockDim.x) {
+    const uint32_t key = st.key[j];
+    if (key < bound.key) continue;
+    if (key <= bound.bin_high) {  // kept if fewer than top_k keys are larger
+      uint32_t larger = bound.above;
+      for (int i = 0; i < n_edge; ++i) larger += st.edge[i] > key ? 1u : 0u;
+      if (larger >= static_cast<uint32_t>(k)) continue;
+    }
+    const int slot = atomicAdd(&st.n_kept, 1);
+    st.kept_key[slot] = key;
+    st.kept_idx[slot] = st.idx[j];
+    const sp_mass_t mj = sp_mass(expf(sp_exponent(order_value(key), inv_t, top)));
+    st.kept_mass[slot] = mj;
+    m += mj;
+  }
+  m = sp_wave_sum(m);
+  if (lane == 0) atomicAdd(&st.mass_sum, m);
+  __syncthreads();
+  const int kept = st.n_kept;
+  const sp_mass_t total = st.mass_sum;
+  const float z = static_cast<float>(static_cast<double>(total) * (1.0 / SP_ONE));
+  uint32_t p_key = 0u;
+  const bool p_active = p_lim < 1.f;
+  if (p_active) {
+    // the largest key whose mass(key >= it) exceeds top_p of the kept mass
+    const double limit = static_cast<double>(p_lim) * static_cast<double>(total);
+    for (int j = tid; j < kept; j += blockDim.x) {
+      const uint32_t key = st.kept_key[j];
+      sp_mass_t at_least = 0ull;
+      for (int i = 0; i < kept; ++i) at_least += st.kept_key[i] >= key ? st.kept_mass[i] : 0ull;
+      if (static_cast<double>(at_least) > limit) atomicMax(&st.p_found, key);
+    }
+    __syncthreads();
+    p_key = st.p_found;
+  }
+  const uint64_t seed_base = mix64((static_cast<uint64_t>(static_cast<uint32_t>(seed)) << 32) |
+                                   static_cast<uint32_t>(draw));
+  ArgMax win{-INFINITY, 0x7fffffff};
+  for (int j = tid; j < kept; j += blockDim.x) {
+    const uint32_t key = st.kept_key[j];
+    const int i = st.kept_idx[j];
+    if (p_active && key <= p_key && i != best.i) continue;
+    const uint64_t zz = mix64(seed_base + static_cast<uint64_t>(i));
+    const float u = (static_cast<float>(zz >> 41) + 0.5f) * (1.f / 8388608.f);
+    win = better(win, ArgMax{expf(sp_exponent(order_value(key), inv_t, top)) / z / -logf(u), i});
+  }
+  win = block_argmax(win, st.ascratch);
+  return Settled{SP_DONE, win.i == 0x7fffffff ? best.i : win.i};
+}
+
+// ---- 2, where all rows are such rows
+constexpr int SP_SETTLE_THREADS = 1024;  // a wave a stretch at the usual vocabularies
+
+__global__ __launch_bounds__(SP_SETTLE_THREADS) void sp_settle_kernel(
+    const float* __restrict__ logits, int32_t* __restrict__ out, int vocab, const float* __restrict__ temperature,
+    const int32_t* __restrict__ top_k, const float* __restrict__ top_p, const int32_t* __restrict__ seeds,
+    const int32_t* __restrict__ draws, const ArgMax* __restrict__ part_best, const uint32_t* __restrict__ top_key,
+    const int32_t* __restrict__ top_idx, const int32_t* __restrict__ top_count, int32_t* __restrict__ paths_out) {
+  __shared__ union {
+    SettleShared settle;
+    SampleShared row;
+  } sh;
+  const int rowi = blockIdx.x, k = top_k[rowi];
+  const float temp = temperature[rowi], p_lim = top_p[rowi];
+  Settled s{SP_WHOLE_ROW, 0};
+  if (sp_settles(temp, k, vocab))
+    s = sp_settle(rowi, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key, top_idx, top_count, sh.settle);
+  if (s.path == SP_WHOLE_ROW) {
+    __syncthreads();
+    s.token = sample_row(logits + static_cast<size_t>(rowi) * vocab, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], false, sh.row);
+  }
   if (threadIdx.x == 0) {
-    part_best[rowi * SP_CHUNKS + chunk] = best;
-    part_low[rowi * SP_CHUNKS + chunk] = -neg_low;
+    out[rowi] = s.token;
+    if (paths_out) paths_out[rowi] = s.path;
   }
 }
 
 // ---- 2: count and mass of every bin, chunk by chunk
 __global__ __launch_bounds__(SP_THREADS) void sp_histogram_kernel(
-    const float* __restrict__ logits, int vocab, const float* __restrict__ temperature,
-    const ArgMax* __restrict__ part_best, const float* __restrict__ part_low,
-    uint32_t* __restrict__ hist_count, sp_mass_t* __restrict__ hist_mass) {
+    const float* __restrict__ logits, int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+    const ArgMax* __restrict__ part_best, const float* __restrict__ part_low, uint32_t* __restrict__ hist_count,
+    sp_mass_t* __restrict__ hist_mass) {
   __shared__ uint32_t count[SP_BINS];
   __shared__ sp_mass_t mass[SP_BINS];
-  const int rowi = blockIdx.x, chunk = blockIdx.y;
-  const float temp = temperature[rowi];
-  if (temp <= 0.f) return;
-  const float inv_t = 1.f / temp;
-  const SampleExtent ext = sp_extent(part_best + rowi * SP_CHUNKS, part_low + rowi * SP_CHUNKS, inv_t);
+  const int rowi = blockIdx.x, chunk = blockIdx.y, parts = sp_parts(vocab);
+  if (sp_settles(temperature[rowi], top_k[rowi], vocab)) return;
+  const float inv_t = 1.f / temperature[rowi];
+  const SampleExtent ext = sp_extent(part_best + static_cast<size_t>(rowi) * parts, part_low + static_cast<size_t>(rowi) * parts, parts, inv_t);
   for (int b = threadIdx.x; b < SP_BINS; b += blockDim.x) {
     count[b] = 0u;
     mass[b] = 0ull;
@@ -666,36 +997,43 @@ __device__ sp_mass_t sp_block_scan(sp_mass_t v, sp_mass_t* scratch) {
   return v + before;
 }
 
-// ---- 3: which bins hold the thresholds; one workgroup a row, one thread a bin
+// ---- 3: which bins hold the thresholds; one workgroup a row, one thread a bin (rows that need no
+// bins are settled here)
 __global__ __launch_bounds__(SP_BINS) void sp_plan_kernel(
     int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
-    const float* __restrict__ top_p, const ArgMax* __restrict__ part_best,
-    const float* __restrict__ part_low, const uint32_t* __restrict__ hist_count,
-    const sp_mass_t* __restrict__ hist_mass, SamplePlan* __restrict__ plans) {
+    const float* __restrict__ top_p, const int32_t* __restrict__ seeds, const int32_t* __restrict__ draws,
+    const ArgMax* __restrict__ part_best, const float* __restrict__ part_low, const uint32_t* __restrict__ hist_count,
+    const sp_mass_t* __restrict__ hist_mass, const uint32_t* __restrict__ top_key, const int32_t* __restrict__ top_idx,
+    const int32_t* __restrict__ top_count, SamplePlan* __restrict__ plans, int32_t* __restrict__ out) {
+  __shared__ SettleShared settle_shared;
   __shared__ sp_mass_t scan_scratch[17];
   __shared__ float fscratch[17];
   __shared__ sp_mass_t picked[3];
-  const int rowi = blockIdx.x, b = threadIdx.x;
-  const float temp = temperature[rowi];
+  const int rowi = blockIdx.x, b = threadIdx.x, parts = sp_parts(vocab);
+  const float temp = temperature[rowi], p_lim = top_p[rowi];
+  const int k = top_k[rowi];
+  if (sp_settles(temp, k, vocab)) {
+    const Settled s =
+        sp_settle(rowi, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key, top_idx, top_count, settle_shared);
+    if (b == 0) {
+      plans[rowi].path = s.path;
+      if (s.path != SP_WHOLE_ROW) out[rowi] = s.token;
+    }
+    return;
+  }
   SamplePlan plan;
-  plan.path = SP_GREEDY;
   plan.k_active = plan.p_active = 0;
   plan.bin_lo = plan.bin_hi = plan.n_cand = 0;
   plan.p_key = 0u;
   plan.z = 1.f;
   plan.mass_before = plan.mass_total = 0ull;
   for (int c = 0; c < SP_CHUNKS; ++c) plan.chunk_at[c] = 0;
-  plan.inv_t = temp > 0.f ? 1.f / temp : 1.f;
-  const SampleExtent ext = sp_extent(part_best + rowi * SP_CHUNKS, part_low + rowi * SP_CHUNKS, plan.inv_t);
+  plan.inv_t = 1.f / temp;
+  const SampleExtent ext =
+      sp_extent(part_best + static_cast<size_t>(rowi) * parts, part_low + static_cast<size_t>(rowi) * parts, parts, plan.inv_t);
   plan.best_i = ext.best.i;
   plan.best_v = ext.best.v;
   plan.bin_scale = ext.bin_scale;
-  if (temp <= 0.f) {
-    if (b == 0) plans[rowi] = plan;
-    return;
-  }
-  const int k = top_k[rowi];
-  const float p_lim = top_p[rowi];
   plan.k_active = k > 0 && k < vocab;
   plan.p_active = p_lim < 1.f;
 
@@ -960,10 +1298,14 @@ struct SampleWorkspace {
   uint32_t* cand_key;
   float* cand_e;
   int32_t* cand_idx;
+  uint32_t* top_key;
+  int32_t* top_idx;
+  int32_t* top_count;
   size_t bytes;
 };
 
-static SampleWorkspace sample_workspace(void* base, size_t n_rows) {
+static SampleWorkspace sample_workspace(void* base, size_t n_rows, int vocab) {
+  const size_t parts = n_rows * static_cast<size_t>(sp_parts(vocab));
   SampleWorkspace w;
   char* at = static_cast<char*>(base);
   auto take = [&](size_t bytes) {
@@ -974,12 +1316,16 @@ static SampleWorkspace sample_workspace(void* base, size_t n_rows) {
   w.hist_mass = reinterpret_cast<sp_mass_t*>(take(n_rows * SP_CHUNKS * SP_BINS * sizeof(sp_mass_t)));
   w.plans = reinterpret_cast<SamplePlan*>(take(n_rows * sizeof(SamplePlan)));
   w.hist_count = reinterpret_cast<uint32_t*>(take(n_rows * SP_CHUNKS * SP_BINS * sizeof(uint32_t)));
-  w.part_best = reinterpret_cast<ArgMax*>(take(n_rows * SP_CHUNKS * sizeof(ArgMax)));
+  w.part_best = reinterpret_cast<ArgMax*>(take(parts * sizeof(ArgMax)));
   w.race_part = reinterpret_cast<ArgMax*>(take(n_rows * SP_CHUNKS * sizeof(ArgMax)));
-  w.part_low = reinterpret_cast<float*>(take(n_rows * SP_CHUNKS * sizeof(float)));
+  w.part_low = reinterpret_cast<float*>(take(parts * sizeof(float)));
   w.cand_key = reinterpret_cast<uint32_t*>(take(n_rows * CAND_MAX * sizeof(uint32_t)));
   w.cand_e = reinterpret_cast<float*>(take(n_rows * CAND_MAX * sizeof(float)));
   w.cand_idx = reinterpret_cast<int32_t*>(take(n_rows * CAND_MAX * sizeof(int32_t)));
+  const size_t handed = sp_settle_limit(vocab) > 0 ? parts * SP_PART_KEEP : 0;
+  w.top_key = reinterpret_cast<uint32_t*>(take(handed * sizeof(uint32_t)));
+  w.top_idx = reinterpret_cast<int32_t*>(take(handed * sizeof(int32_t)));
+  w.top_count = reinterpret_cast<int32_t*>(take(parts * sizeof(int32_t)));
   w.bytes = static_cast<size_t>(at - static_cast<char*>(base));
   return w;
 }
@@ -988,36 +1334,44 @@ static SampleWorkspace sample_workspace(void* base, size_t n_rows) {
 // workgroups (0: this vocabulary is left to one workgroup a row, which needs none).
 extern "C" size_t yk_sample_workspace_bytes(int n_rows, int vocab) {
   if (n_rows <= 0 || vocab < SP_MIN_VOCAB) return 0;
-  return sample_workspace(nullptr, static_cast<size_t>(n_rows)).bytes;
+  return sample_workspace(nullptr, static_cast<size_t>(n_rows), vocab).bytes;
 }
 
 // workspace: yk_sample_workspace_bytes bytes, 256-byte aligned, or null (then, as with
-// force_whole_row, every row is one workgroup's work).  paths_out (may be null) receives, for
+// force_whole_row, every row is one workgroup's work).  most_top_k: the caller's word that every
+// row is greedy or has a top_k of 1 to most_top_k (0: no word); up to what two kernels settle, no
+// others are launched, and a row that they cannot settle after all is one workgroup's work.  paths_out (may be null) receives, for
 // rows that were divided, which way each went (SamplePath); other rows are left untouched.
 extern "C" int yk_sample(const float* logits, int32_t* out, int n_rows, int vocab,
                          const float* temperature, const int32_t* top_k, const float* top_p,
-                         const int32_t* seeds, const int32_t* draws, int force_whole_row,
+                         const int32_t* seeds, const int32_t* draws, int force_whole_row, int most_top_k,
                          void* workspace, size_t workspace_bytes, int32_t* paths_out,
                          hipStream_t stream) {
   YK_REQUIRE(n_rows >= 0 && vocab > 0, "sample: bad sizes");
   if (n_rows == 0) return 0;
   const size_t need = yk_sample_workspace_bytes(n_rows, vocab);
-  const bool divide = need > 0 && !force_whole_row && workspace && workspace_bytes >= need && n_rows <= 65535;
+  const bool divide = need > 0 && !force_whole_row && workspace && workspace_bytes >= need && n_rows <= 65535 && sp_parts(vocab) <= 65535;
   if (!divide) {
     sample_kernel<<<n_rows, 1024, 0, stream>>>(logits, out, vocab, temperature, top_k, top_p, seeds, draws,
                                                force_whole_row, nullptr, nullptr, nullptr);
     return yk_check_launch("sample");
   }
   YK_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 256 == 0, "sample: the workspace must be 256-byte aligned");
-  const SampleWorkspace w = sample_workspace(workspace, static_cast<size_t>(n_rows));
-  const dim3 chunks(n_rows, SP_CHUNKS);
-  sp_extent_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, w.part_best, w.part_low);
+  const SampleWorkspace w = sample_workspace(workspace, static_cast<size_t>(n_rows), vocab);
+  sp_extent_kernel<<<dim3(n_rows, sp_parts(vocab)), SP_THREADS, 0, stream>>>(logits, vocab, temperature, top_k, w.part_best,
+                                                                            w.part_low, w.top_key, w.top_idx, w.top_count);
   if (yk_check_launch("sample: extent")) return -1;
-  sp_histogram_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, temperature, w.part_best, w.part_low,
+  if (most_top_k > 0 && most_top_k <= sp_settle_limit(vocab)) {
+    sp_settle_kernel<<<n_rows, SP_SETTLE_THREADS, 0, stream>>>(logits, out, vocab, temperature, top_k, top_p, seeds, draws,
+                                                               w.part_best, w.top_key, w.top_idx, w.top_count, paths_out);
+    return yk_check_launch("sample: settle");
+  }
+  const dim3 chunks(n_rows, SP_CHUNKS);
+  sp_histogram_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, temperature, top_k, w.part_best, w.part_low,
                                                          w.hist_count, w.hist_mass);
   if (yk_check_launch("sample: histogram")) return -1;
-  sp_plan_kernel<<<n_rows, SP_BINS, 0, stream>>>(vocab, temperature, top_k, top_p, w.part_best, w.part_low,
-                                                 w.hist_count, w.hist_mass, w.plans);
+  sp_plan_kernel<<<n_rows, SP_BINS, 0, stream>>>(vocab, temperature, top_k, top_p, seeds, draws, w.part_best, w.part_low,
+                                                 w.hist_count, w.hist_mass, w.top_key, w.top_idx, w.top_count, w.plans, out);
   if (yk_check_launch("sample: plan")) return -1;
   sp_collect_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, w.plans, w.cand_key, w.cand_e, w.cand_idx);
   if (yk_check_launch("sample: collect")) return -1;

@@ -253,7 +253,7 @@ _LATER_SIGNATURES = {
     "sampling": {
         "yk_abi_version": ([], _c_int),
         "yk_argmax": ([_vp, _vp, _c_int, _c_int, _vp, _c_size_t, _vp], _c_int),
-        "yk_sample": ([_vp, _vp, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _vp, _c_size_t, _vp, _vp], _c_int),
+        "yk_sample": ([_vp, _vp, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int, _vp, _c_size_t, _vp, _vp], _c_int),
         "yk_sample_workspace_bytes": ([_c_int, _c_int], _c_size_t),
     },
     "probe": {
@@ -2322,13 +2322,15 @@ class HipOps:
                                   ws.data_ptr(), ws.numel(), self._stream()), lib)
         return out
 
-    def sample(self, logits, temperature, top_k, top_p, seeds, draws, whole_row: bool = False, paths=None) -> torch.Tensor:
+    def sample(self, logits, temperature, top_k, top_p, seeds, draws, whole_row: bool = False, paths=None, most_top_k: int = 0) -> torch.Tensor:
         """Per row: temperature (float32; 0 = greedy), top_k (int32; 0 = off), top_p
         (float32), seed and draw number (int32).  Returns int32 token ids.  Rows of a large
         vocabulary are divided among workgroups; ``whole_row`` forces one workgroup a row on
         the path that never narrows the row down to candidates (for tests), and ``paths``
         (int32, one per row) receives which way each divided row went: 0 greedy, 1 a race
-        over the row, 3 settled among candidates, 4 left to one workgroup after all."""
+        over the row, 3 settled among candidates, 4 left to one workgroup after all.
+        ``most_top_k``: the caller's word that every row is greedy or has a top_k of 1 to this
+        (0: no word), which saves the launches that only other rows need; the tokens are the same."""
         if logits.dtype != torch.float32 or not logits.is_contiguous() or logits.dim() != 2:
             raise KernelError("sample takes contiguous float32 logits [rows, vocab]")
         rows = logits.shape[0]
@@ -2345,7 +2347,7 @@ class HipOps:
         self._check(
             lib.yk_sample(
                 logits.data_ptr(), out.data_ptr(), rows, logits.shape[1], temperature.data_ptr(), top_k.data_ptr(),
-                top_p.data_ptr(), seeds.data_ptr(), draws.data_ptr(), int(bool(whole_row)),
+                top_p.data_ptr(), seeds.data_ptr(), draws.data_ptr(), int(bool(whole_row)), int(most_top_k),
                 _ptr(ws), 0 if ws is None else ws.numel() * 4, _ptr(paths), self._stream(),
             ),
             lib,

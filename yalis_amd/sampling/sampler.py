@@ -14,7 +14,7 @@ what else is in the batch or on whether it was preempted and recomputed.
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import List, Optional, Sequence
+from typing import List, NamedTuple, Optional, Sequence
 
 import torch
 
@@ -44,6 +44,18 @@ class SamplingParams:
         return self.temperature == 0.0
 
 
+class PreparedRows(NamedTuple):
+    """What sampling needs on the device, one entry a row, and the largest top_k if every row is
+    greedy or has one (0: some row has none)."""
+
+    temperature: torch.Tensor
+    top_k: torch.Tensor
+    top_p: torch.Tensor
+    seeds: torch.Tensor
+    draws: torch.Tensor
+    most_top_k: int
+
+
 class Sampler:
     def __init__(self, ops, device: str):
         self.ops = ops
@@ -58,8 +70,7 @@ class Sampler:
 
     def prepare(self, params: Sequence[SamplingParams], draws: Sequence[int]):
         """What ``sample_prepared`` needs on the device for these rows: None when every row is
-        greedy, else (temperature, top_k, top_p, seeds, draws) tensors.  Made once for a run
-        of steps over the same requests."""
+        greedy, else ``PreparedRows``.  Made once for a run of steps over the same requests."""
         if len(params) != len(draws):
             raise ValueError("one SamplingParams and one draw number per row of logits")
         if all(p.greedy for p in params):
@@ -68,7 +79,9 @@ class Sampler:
         ints = torch.tensor(
             [[p.top_k or 0 for p in params], [p.seed & 0x7FFFFFFF for p in params], list(draws)], dtype=torch.int32
         ).to(self.device)
-        return floats[0].contiguous(), ints[0].contiguous(), floats[1].contiguous(), ints[1].contiguous(), ints[2].contiguous()
+        limits = [p.top_k or 0 for p in params if not p.greedy]
+        return PreparedRows(floats[0].contiguous(), ints[0].contiguous(), floats[1].contiguous(), ints[1].contiguous(),
+                            ints[2].contiguous(), max(limits) if all(limits) else 0)
 
     @staticmethod
     def narrow(prepared, index: torch.Tensor):
@@ -76,14 +89,14 @@ class Sampler:
         prepared set, in that order."""
         if prepared is None:
             return None
-        return tuple(t.index_select(0, index) for t in prepared)
+        return PreparedRows(*(t.index_select(0, index) for t in prepared[:-1]), prepared.most_top_k)
 
     def sample_prepared(self, logits: torch.Tensor, prepared, step: int) -> torch.Tensor:
         """Token ids (int32, on the device) for rows prepared with ``prepare``; ``step`` is
         added to every row's draw number (the step within a run that shares one preparation)."""
         if prepared is None:
             return self.ops.argmax(logits)
-        temperature, top_k, top_p, seeds, draws = prepared
+        temperature, top_k, top_p, seeds, draws, most_top_k = prepared
         if logits.shape[0] != draws.numel():
             raise ValueError("one SamplingParams and one draw number per row of logits")
-        return self.ops.sample(logits, temperature, top_k, top_p, seeds, draws + step if step else draws)
+        return self.ops.sample(logits, temperature, top_k, top_p, seeds, draws + step if step else draws, most_top_k=most_top_k)
