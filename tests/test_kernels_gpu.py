@@ -157,6 +157,25 @@ def test_float32_matrix_core_products(ops, form, m, n, k, xd, wd, od):
     close(got, want, atol, 2.0**-23 if od == torch.float32 else 2.0**-8)
 
 
+# one to four rows: a wave's one or two rows of the weight, K around its pieces of 256 and its 8 (4) in flight
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+@pytest.mark.parametrize("n,k", [(1, 252), (5, 256), (9, 1028), (7, 2048), (6, 2052), (8191, 260), (8193, 1024), (8195, 1284)])
+@pytest.mark.parametrize("xd,wd,od", [
+    (torch.float32, torch.float32, torch.float32),
+    (torch.bfloat16, torch.float32, torch.bfloat16),
+    (torch.float32, torch.bfloat16, torch.float32),
+])
+def test_float32_products_of_up_to_four_rows(ops, m, n, k, xd, wd, od):
+    x = rnd((m, k + 12), xd, 43)[:, 4: 4 + k]
+    w = rnd((n, k + 4), wd, 44)[:, :k]
+    got = ops.gemm_fma(x, w, od)
+    want = x.double().cpu() @ w.double().cpu().T
+    # a lane's four chains of at most k / 256 + 1 additions and eight more: the running sum, of about sqrt(k), is rounded
+    # by 2^-24 of itself at each
+    atol = math.sqrt(k) * math.sqrt(k / 256 + 9) * 2.0**-24 * 8
+    close(got, want, atol, 2.0**-23 if od == torch.float32 else 2.0**-8)
+
+
 def test_gemm_fma_is_true_float32(ops):
     """Inputs that a reduced-precision matrix mode would truncate: 1 + 2^-12 has more
     mantissa bits than bfloat16 (8) or a 10-bit tensor-float mode keep, and every partial

@@ -129,6 +129,66 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_tile_kernel(const TX* __res
   }
 }
 
+// ------------------------------------------------------------------------- one to four rows, no tile
+// A wave makes R outputs for every row of x: its lanes read the weight's rows 1 KiB at a time (256
+// consecutive elements), eight loads in flight, and every lane sums its own products in four chains a
+// row (one of the four elements each) that meet at the end.  A row of the weight is one wave's, so that
+// a matrix of 2,000 rows still occupies every compute unit, which tiles of 16 rows do not.
+// Bound by the reading of the weight.
+template <typename TX, typename TW, typename TO, int MR, int R>
+__global__ __launch_bounds__(256) void gemm_f32_dot_kernel(const TX* __restrict__ x, const TW* __restrict__ w, TO* __restrict__ y,
+                                                           int N, int K, int ldx, int ldw, int ldy) {
+  constexpr int AHEAD = 8 / R;  // pieces of a row in flight
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int n0 = (blockIdx.x * 4 + wave) * R;
+  if (n0 >= N) return;
+  const TW* wp[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) wp[i] = w + static_cast<size_t>(min(n0 + i, N - 1)) * ldw + 4 * lane;
+  const TX* xp = x + 4 * lane;
+  f32x4_t acc[R][MR] = {};
+  auto add = [&](const f32x4_t (&a)[R], const f32x4_t (&b)[MR]) {
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int m = 0; m < MR; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][m][e] = fmaf(a[i][e], b[m][e], acc[i][m][e]);
+  };
+  int k0 = 0;
+  for (; k0 + 256 * AHEAD <= K; k0 += 256 * AHEAD) {
+    f32x4_t a[AHEAD][R];
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c)
+#pragma unroll
+      for (int i = 0; i < R; ++i) a[c][i] = stream4(wp[i] + k0 + 256 * c);
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c) {
+      f32x4_t b[MR];
+#pragma unroll
+      for (int m = 0; m < MR; ++m) b[m] = load4(xp + static_cast<size_t>(m) * ldx + k0 + 256 * c);
+      add(a[c], b);
+    }
+  }
+  for (; k0 < K; k0 += 256) {
+    const bool in = k0 + 4 * lane < K;  // K is a multiple of four
+    const f32x4_t none = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t a[R], b[MR];
+#pragma unroll
+    for (int i = 0; i < R; ++i) a[i] = in ? stream4(wp[i] + k0) : none;
+#pragma unroll
+    for (int m = 0; m < MR; ++m) b[m] = in ? load4(xp + static_cast<size_t>(m) * ldx + k0) : none;
+    add(a, b);
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+      const float v = wave_sum((acc[i][m][0] + acc[i][m][1]) + (acc[i][m][2] + acc[i][m][3]));
+      if (lane == 0 && n0 + i < N) y[static_cast<size_t>(m) * ldy + n0 + i] = from_f32<TO>(v);
+    }
+}
+
 // ------------------------------------------------------------------------------ few rows, one pass
 // A workgroup of W waves makes 16 outputs for up to 16 MT rows of x (blockIdx.y: which of them); its
 // waves walk K by turns, 64 elements each, and their sums meet in LDS at the end, wave by wave.  A
@@ -203,9 +263,24 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_rows_kernel(const TX* __restr
 //   N 2,048, K 8,192   64 rows 102 / 218 / 176 / 160   311 rows 266 / 218 / 176 / 162   511 rows 339 / 222 / 178 / 164   (1,488, 1,404, 1,423)
 //   N 16,384, K 2,048   32 rows 48 / 61 / 48 / 47   64 rows 90 / 61 / 50 / 47   511 rows 696 / 334 / 330 / 340   (351, 391, 932)
 //   N 6,144, K 4,096   48 rows 79 / 112 / 89 / 84   1,024 rows 1,032 / 481 / 462 / 486
-// One row of x: 27 us for N 16,384, K 2,048 (4.9 TB/s), 26 us for N 2,048, K 8,192 (2.6 TB/s: 128 workgroups), where the
-// kernel of gemm.hip takes 328 and 1,140.
+// Up to four rows no tile at all: a wave a row of the weight (two from DOT_PAIR_N rows on, which share the reads of x).
+// Measured (us, tiles of 16 rows / this), 1, 2, 3 and 4 rows of x:
+//   N 2,048, K 8,192   27.9 / 12.7   28.4 / 14.7   28.8 / 16.6   29.3 / 18.4 (128 tiles leave half of the compute units idle)
+//   N 3,072, K 2,048   9.5 / 6.2   9.8 / 7.4   10.1 / 8.2   10.1 / 9.2
+//   N 16,384, K 2,048   29.2 / 22.8   29.6 / 25.3   30.7 / 27.1   31.3 / 30.8
+//   N 128,256, K 2,048   197 / 153   200 / 162   205 / 186   210 / 217
+// Its sums are closer to 64 bits than the tiles' (0.9 to 1.3e-7 of the result, 1.2 to 1.5e-7).
+constexpr int DOT_ROWS = 4;
+constexpr int DOT_PAIR_N = 8192;
 static int g_force_form = 0;  // 0: the rule; 1: few rows; 2, 4: tiles with that many groups of waves
+
+template <typename TX, typename TW, typename TO, int MR>
+void launch_dot(const TX* x, const TW* w, TO* y, int N, int K, int ldx, int ldw, int ldy, hipStream_t stream) {
+  if (N < DOT_PAIR_N)
+    gemm_f32_dot_kernel<TX, TW, TO, MR, 1><<<(N + 3) / 4, 256, 0, stream>>>(x, w, y, N, K, ldx, ldw, ldy);
+  else
+    gemm_f32_dot_kernel<TX, TW, TO, MR, 2><<<(N + 7) / 8, 256, 0, stream>>>(x, w, y, N, K, ldx, ldw, ldy);
+}
 
 template <typename TX, typename TW, typename TO>
 int launch(const TX* x, const TW* w, TO* y, int M, int N, int K, int ldx, int ldw, int ldy, hipStream_t stream) {
@@ -216,6 +291,15 @@ int launch(const TX* x, const TW* w, TO* y, int M, int N, int K, int ldx, int ld
     gemm_f32_tile_kernel<TX, TW, TO, 4><<<tiles, 1024, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy);
   } else if (form == 2) {
     gemm_f32_tile_kernel<TX, TW, TO, 2><<<tiles, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy);
+  } else if (M <= DOT_ROWS && g_force_form != 1) {
+    if (M == 1)
+      launch_dot<TX, TW, TO, 1>(x, w, y, N, K, ldx, ldw, ldy, stream);
+    else if (M == 2)
+      launch_dot<TX, TW, TO, 2>(x, w, y, N, K, ldx, ldw, ldy, stream);
+    else if (M == 3)
+      launch_dot<TX, TW, TO, 3>(x, w, y, N, K, ldx, ldw, ldy, stream);
+    else
+      launch_dot<TX, TW, TO, 4>(x, w, y, N, K, ldx, ldw, ldy, stream);
   } else {
     const int cols = (N + 15) / 16;
     if (M <= 16 && cols <= 512 && K >= 1024)
@@ -239,9 +323,9 @@ int launch_out(const void* x, const void* w, void* y, int y_dtype, int M, int N,
 
 }  // namespace
 
-// For tests and measurements: which form a product takes (0: the library decides).
+// For tests and measurements: which form a product takes (0: the library decides; 1: tiles of 16 rows).
 extern "C" int yk_gemm_f32_force(int form) {
-  YK_REQUIRE(form == 0 || form == 1 || form == 2 || form == 4, "gemm_f32_force: 0 the rule, 1 few rows, 2 / 4 tiles with that many groups of waves");
+  YK_REQUIRE(form == 0 || form == 1 || form == 2 || form == 4, "gemm_f32_force: 0 the rule, 1 few rows in tiles of 16, 2 / 4 tiles with that many groups of waves");
   g_force_form = form;
   return 0;
 }
