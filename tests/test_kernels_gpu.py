@@ -176,6 +176,40 @@ def test_float32_products_of_up_to_four_rows(ops, m, n, k, xd, wd, od):
     close(got, want, atol, 2.0**-23 if od == torch.float32 else 2.0**-8)
 
 
+# columns around a tile of 16, K around a chunk of 256 and a round of the eight waves (2,048), fewer chunks than waves
+@pytest.mark.parametrize("m", [1, 7, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(16, 8), (48, 248), (32, 264), (64, 2048), (2064, 2056), (96, 4096), (16, 2304)])
+def test_products_with_their_own_end(ops, m, n, k):
+    """A few-row product with a bias or a gated pair in its launch: what the product and a kernel after it give,
+    and the 64-bit result."""
+    x = rnd((m, k + 16), torch.bfloat16, 45)[:, 8: 8 + k]  # rows of their own stride
+    w = rnd((n, k + 8), torch.bfloat16, 46, scale=k**-0.5)[:, :k]
+    bias = rnd((n,), torch.float32, 47)
+    bf = torch.bfloat16
+    exact = x.double() @ w.double().T
+    # float32 sums of k products of about k^-1/2: the running sum, of at most about 4, is rounded by 2^-24 of itself at each
+    # of k / 32 + 8 additions
+    atol = 4 * math.sqrt(k / 32 + 8) * 2.0**-24 * 8
+    close(ops.gemm_cols(x, w, torch.float32), exact.cpu(), atol, 1e-6)
+    close(ops.gemm_cols(x, w, bf), exact.cpu(), atol, 2.0**-8)
+    close(ops.gemm_cols(x, w, bf, bias=bias), (exact + bias.double()).cpu(), atol + 2.0**-8 * atol, 2.0**-8)
+    close(ops.gemm_cols(x, w, bf, bias=bias.to(bf)), (exact + bias.to(bf).double()).cpu(), atol, 2.0**-8)
+    prod = ops.gemm_cols(x, w, bf)  # rounded as the pairs take it
+    for pair in ("silu", "gelu_tanh", ("clamped_swish", 1.5, 1.7)):
+        assert torch.equal(ops.gemm_cols(x, w, bf, gated=pair), ops.gated_act(prod, pair, bf, group=8))
+
+
+def test_products_with_their_own_end_at_any_width(ops):
+    """Columns that are no multiple of 16, and entries that are not finite where nothing is stored."""
+    x = rnd((5, 264), torch.bfloat16, 48)
+    w = rnd((33, 264), torch.bfloat16, 49)
+    close(ops.gemm_cols(x, w, torch.float32), (x.double() @ w.double().T).cpu(), 16 * 2.0**-24 * 8 * 6, 1e-6)
+    with pytest.raises(Exception):
+        ops.gemm_cols(rnd((17, 264), torch.bfloat16, 48), w, torch.bfloat16)
+    with pytest.raises(Exception):
+        ops.gemm_cols(x, w, torch.bfloat16, gated="silu")
+
+
 def test_gemm_fma_is_true_float32(ops):
     """Inputs that a reduced-precision matrix mode would truncate: 1 + 2^-12 has more
     mantissa bits than bfloat16 (8) or a 10-bit tensor-float mode keep, and every partial

@@ -217,6 +217,10 @@ _SIGNATURES = {
         _c_int,
     ),
     "yk_gemm_tile_force": ([_c_int], _c_int),
+    "yk_gemm_cols": ([_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _c_int, _c_int, _c_int, _c_float,
+                      _c_float, _vp], _c_int),
+    "yk_gemm_cols_ok": ([_c_int, _c_int, _c_int, _c_int], _c_int),
+    "yk_gemm_cols_force": ([_c_int], _c_int),
     "yk_attn_generic": (
         [_vp, _c_int, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _vp],
         _c_int,
@@ -396,6 +400,7 @@ class HipOps:
         self._workspace: Optional[torch.Tensor] = None  # attention splits, argmax parts
         self._library_workspace: Optional[torch.Tensor] = None  # the vendor library's scratch
         self._gemm_workspace: Optional[torch.Tensor] = None  # K slices of products
+        self._skinny_forced = False
         # how often each workspace has been handed out: what lives in one (SplitSum,
         # SplitAttention) remembers the number and is refused once it has moved on
         self._ws_gen = 0
@@ -470,6 +475,7 @@ class HipOps:
         """For tests and measurements: force the few-row product's chunk length (128 / 256), waves a
         workgroup and number of K slices (0: the library decides); call without arguments to clear."""
         self._check(self.lib.yk_gemm_skinny_force(int(chunk), int(waves), int(slices)))
+        self._skinny_forced = bool(chunk or waves or slices)  # what is forced is also what runs
         self._answers = {k: v for k, v in self._answers.items() if k[0] not in ("yk_gemm_skinny_splits", "yk_gemm_skinny_from_attention_ok")}
 
     def wide_skinny_products(self, mode: int = 1) -> None:
@@ -658,6 +664,8 @@ class HipOps:
         """x [M, K] . w [N, K]^T (+ bias [N]) -> [M, N].  With ``partial_ok`` (and no bias) the
         result may come as a ``SplitSum`` for a consumer that adds the slices itself."""
         if bias is not None:
+            if isinstance(x, torch.Tensor) and self._takes_cols(x, w):
+                return self.gemm_cols(x, w, out_dtype, bias=bias)
             # the product in float32, the bias added there, one rounding (as a product that adds
             # the bias to its accumulators rounds: the reference's biased Linear)
             acc = self.linear(x, w, torch.float32, partial_ok=False)
@@ -693,6 +701,8 @@ class HipOps:
                 # vendor library, float32 accumulators stored as they are (the output head for
                 # more than 64 wanted rows: the few-row kernel would stream the table once per 64)
                 return self.gemm_library(x, w, torch.float32)
+            if self._takes_cols(x, w, slices_do=partial_ok or self._ask("yk_gemm_skinny_splits", m, n, k, 0) == 1):
+                return self.gemm_cols(x, w, out_dtype)
             return self.gemm_mfma_skinny(x, w, out_dtype, partial_ok)
         return self.gemm_fma(x, w, out_dtype)
 
@@ -880,6 +890,8 @@ class HipOps:
             and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0 and n % 16 == 0
             and self._ask("yk_gemm_skinny_splits", m, n, k, 1) == 1
         )
+        if not fused and group == self.GATE_UP_GROUP and out_dtype == bf and n % 16 == 0 and self._takes_cols(x, w_gate_up):
+            return self.gemm_cols(x, w_gate_up, bf, gated=activation)
         if not fused:
             return self.gated_act(self.linear(x, w_gate_up, out_dtype, partial_ok=True), activation, out_dtype, group=group)
         y = torch.empty((m, n // 2), dtype=bf, device=x.device)
@@ -889,6 +901,33 @@ class HipOps:
         )
         if rc < 0:
             self._check(rc)
+        return y
+
+    def force_cols(self, mode: int = 0) -> None:
+        """For tests and measurements: where ``gemm_cols`` runs (0 the rule, 1 nowhere, 2 wherever it can)."""
+        self._check(self.lib.yk_gemm_cols_force(int(mode)))
+        self._answers = {k: v for k, v in self._answers.items() if k[0] != "yk_gemm_cols_ok"}
+
+    def _takes_cols(self, x, w, slices_do: bool = False) -> bool:
+        """Whether a few-row product is ``gemm_cols``'s; ``slices_do``: no kernel of its own would have to follow the other form."""
+        m, k = x.shape
+        bf = torch.bfloat16
+        return (0 < m <= 16 and not self._skinny_forced and x.dtype == bf and w.dtype == bf and w.shape[1] == k and x.stride(1) == 1 and w.stride(1) == 1
+                and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and bool(self._ask("yk_gemm_cols_ok", m, w.shape[0], k, int(slices_do))))
+
+    def gemm_cols(self, x, w, out_dtype, bias=None, gated=None) -> torch.Tensor:
+        """x [M <= 16, K] . w [N, K]^T with the product's own end in the same launch: plus ``bias`` [N], or
+        ``gated`` pairs of groups of eight columns (see ``gated_kind``)."""
+        m, k = x.shape
+        n = w.shape[0]
+        kind, p0, p1 = (0, 0.0, 0.0) if gated is None else self.gated_kind(gated)
+        if bias is not None and (bias.numel() != n or not bias.is_contiguous()):
+            raise KernelError(f"linear: bias has {bias.numel()} elements, the product {n} columns")
+        y = torch.empty((m, n // 2 if gated is not None else n), dtype=out_dtype, device=x.device)
+        self._check(self.lib.yk_gemm_cols(
+            x.data_ptr(), w.data_ptr(), y.data_ptr(), _code(out_dtype), m, n, k, x.stride(0), w.stride(0), y.shape[1], _ptr(bias),
+            0 if bias is None else _code(bias.dtype), int(gated is not None), kind, p0, p1, self._stream()))
         return y
 
     def gemm_mfma_skinny(self, x, w, out_dtype, partial_ok: bool = False):
@@ -2321,6 +2360,8 @@ class HipOps:
         self._check(lib.yk_argmax(logits.data_ptr(), out.data_ptr(), logits.shape[0], logits.shape[1],
                                   ws.data_ptr(), ws.numel(), self._stream()), lib)
         return out
+
+    sample_takes_most_top_k = True
 
     def sample(self, logits, temperature, top_k, top_p, seeds, draws, whole_row: bool = False, paths=None, most_top_k: int = 0) -> torch.Tensor:
         """Per row: temperature (float32; 0 = greedy), top_k (int32; 0 = off), top_p

@@ -99,4 +99,5 @@ class Sampler:
         temperature, top_k, top_p, seeds, draws, most_top_k = prepared
         if logits.shape[0] != draws.numel():
             raise ValueError("one SamplingParams and one draw number per row of logits")
-        return self.ops.sample(logits, temperature, top_k, top_p, seeds, draws + step if step else draws, most_top_k=most_top_k)
+        word = {"most_top_k": most_top_k} if most_top_k and getattr(self.ops, "sample_takes_most_top_k", False) else {}
+        return self.ops.sample(logits, temperature, top_k, top_p, seeds, draws + step if step else draws, **word)
