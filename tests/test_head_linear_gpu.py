@@ -41,3 +41,30 @@ def check(h, n, in_dim, out_dim, dtype):
     xs, ws = x.double().view(n, h, in_dim).transpose(0, 1).contiguous(), w.double()
     want, size = (torch.matmul(a, b).transpose(0, 1) for a, b in ((xs, ws), (xs.abs(), ws.abs())))
     assert ((got - want).abs() <= 8 * 2.0 ** -24 * size).all()
+
+
+# 16 heads x 512 columns: 128 units of 16 tokens x 64 columns for every 16 tokens; one, two (from 1,792 units) and four (from 3,584) token
+# tiles a wave, with tokens around the end of a tile and of a wave's run
+@pytest.mark.parametrize("n", [33, 48, 208, 209, 225, 432, 433, 449, 577])
+@pytest.mark.parametrize("in_dim,out_dim", [(32, 512), (128, 496), (64, 528)])
+@pytest.mark.parametrize("first", [True, False])
+def test_head_products_of_many_tokens(first, in_dim, out_dim, n):
+    """bfloat16 in and float32 out, or float32 in (as two bfloat16 parts) and gated bfloat16 out."""
+    o = ops()
+    h = 16
+    g = torch.Generator().manual_seed(n + in_dim)
+    xd, od = (torch.bfloat16, torch.float32) if first else (torch.float32, torch.bfloat16)
+    x = torch.randn(n, h * in_dim, generator=g).to(xd)
+    w = torch.randn(h, in_dim, out_dim, generator=g).to(torch.bfloat16)
+    gate = None if first else torch.randn(n, 3 + h * out_dim, generator=g).to(torch.bfloat16)
+    w_t = w.transpose(1, 2).contiguous().cuda()
+    got = o.head_linear(x.cuda(), w.cuda(), h, in_dim, out_dim, od, w_t=w_t, gate=None if gate is None else gate.cuda(), gate_col=3,
+                        gate_elems=out_dim).cpu().double().view(n, h, out_dim)
+    xs, ws = x.double().view(n, h, in_dim).transpose(0, 1).contiguous(), w.double()
+    want, size = (torch.matmul(a, b).transpose(0, 1) for a, b in ((xs, ws), (xs.abs(), ws.abs())))
+    if gate is not None:
+        s = torch.sigmoid(gate[:, 3:].double()).view(n, h, out_dim)
+        want, size = want * s, size * s
+    # in_dim / 32 + 32 additions in float32; a float32 input's two parts leave out 2^-17 of it; the gate's own roundings; the output's rounding
+    tol = (in_dim / 32 + 32) * 2.0**-24 * size + (0 if first else 2.0**-17 * size + 2.0**-8 * want.abs() + 1e-6)
+    assert ((got - want).abs() <= tol).all()

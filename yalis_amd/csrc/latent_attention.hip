@@ -329,9 +329,17 @@ extern "C" int yk_head_linear(const void* x, int x_stride, int x_dtype, const vo
 }
 
 // The same products on the matrix cores, for many tokens: bfloat16 weights kept [heads][out][in] (a row of
-// the second operand is then 16 bytes of memory a lane), the input bfloat16 or float32 (as two bfloat16
-// parts, the rounded value and what the rounding left over, each with its own product).  A wave makes 16 tokens x 64 columns of one head: the first operand is 16 input rows x 32
-// elements, loaded as it lies there.  Four waves a workgroup take four token tiles.
+// the first operand is then 16 bytes of memory a lane), the input bfloat16 or float32 (as two bfloat16
+// parts, the rounded value and what the rounding left over, each with its own product).  A wave makes
+// 16 TT tokens x 64 columns of one head; the weight is the first operand, so that a lane ends with four
+// consecutive columns of one token, a store of 16 bytes.  The next step's operands are in flight while
+// the current ones are multiplied.  Four waves a workgroup take four runs of tokens.
+// Bound by the float32 side (its reading or writing) and the reads of the weights from the caches, which
+// every wave makes for its tokens: hence several token tiles a wave.  16 heads, us (one tile a wave,
+// nothing in flight, 4-byte stores: before / 1 / 2 / 4 tiles a wave):
+//   128 -> 512 in float32    100 tokens  5.6 / 5.0 / 5.7 / 5.5    512 14.7 / 14.2 / 11.0 / 9.5    2,048 45.8 / 43.4 / 32.6 / 27.1
+//   512 -> 128 from float32  100 tokens 15.8 / 13.1 / 16.3 / 15.1  512 20.3 / 14.1 / 17.9 / 26.3  2,048 47.1 / 46.6 / 33.8 / 28.3
+// (2,048 tokens: 83 MB, 17 us at what a copy reaches.  Twice the columns a wave: 30.1 and 27.7.)
 typedef __bf16 hl_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float hl_f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t hl_u32x4_t __attribute__((ext_vector_type(4)));
@@ -340,84 +348,115 @@ union HlFrag {
   hl_bf16x8_t v;
 };
 
+// eight consecutive elements of an input row as they lie there
 template <typename TX>
-__device__ __forceinline__ hl_u32x4_t hl_load8(const TX* p);
-template <>
-__device__ __forceinline__ hl_u32x4_t hl_load8<bf16_t>(const bf16_t* p) {
-  return *reinterpret_cast<const hl_u32x4_t*>(p);
+struct HlRaw {
+  hl_u32x4_t u[sizeof(TX) / 2];
+};
+template <typename TX>
+__device__ __forceinline__ HlRaw<TX> hl_raw8(const TX* p) {
+  HlRaw<TX> x;
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(TX) / 2; ++i) x.u[i] = reinterpret_cast<const hl_u32x4_t*>(p)[i];
+  return x;
 }
-template <>
-__device__ __forceinline__ hl_u32x4_t hl_load8<float>(const float* p) {
-  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-  return hl_u32x4_t{pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w)};
+__device__ __forceinline__ hl_u32x4_t hl_high8(const HlRaw<bf16_t>& x) { return x.u[0]; }
+__device__ __forceinline__ hl_u32x4_t hl_high8(const HlRaw<float>& x) {
+  hl_u32x4_t v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = pack_bf16x2(__uint_as_float(x.u[i / 2][2 * (i % 2)]), __uint_as_float(x.u[i / 2][2 * (i % 2) + 1]));
+  return v;
 }
 // what the rounding of eight floats to bfloat16 left over, itself rounded to bfloat16: a float32 input goes
 // through the matrix cores as the sum of the two, so the product sees it to 16 bits of fraction
-template <typename TX>
-__device__ __forceinline__ hl_u32x4_t hl_rest8(const TX* p, hl_u32x4_t hi);
-template <>
-__device__ __forceinline__ hl_u32x4_t hl_rest8<bf16_t>(const bf16_t*, hl_u32x4_t) {
-  return hl_u32x4_t{0u, 0u, 0u, 0u};
-}
+__device__ __forceinline__ hl_u32x4_t hl_rest8(const HlRaw<bf16_t>&, hl_u32x4_t) { return hl_u32x4_t{0u, 0u, 0u, 0u}; }
 __device__ __forceinline__ uint32_t hl_rest2(float x, float y, uint32_t hi) {
   return pack_bf16x2(x - __uint_as_float(hi << 16), y - __uint_as_float(hi & 0xffff0000u));
 }
-template <>
-__device__ __forceinline__ hl_u32x4_t hl_rest8<float>(const float* p, hl_u32x4_t hi) {
-  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-  return hl_u32x4_t{hl_rest2(a.x, a.y, hi[0]), hl_rest2(a.z, a.w, hi[1]), hl_rest2(b.x, b.y, hi[2]), hl_rest2(b.z, b.w, hi[3])};
+__device__ __forceinline__ hl_u32x4_t hl_rest8(const HlRaw<float>& x, hl_u32x4_t hi) {
+  hl_u32x4_t v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    v[i] = hl_rest2(__uint_as_float(x.u[i / 2][2 * (i % 2)]), __uint_as_float(x.u[i / 2][2 * (i % 2) + 1]), hi[i]);
+  return v;
+}
+__device__ __forceinline__ void hl_store4(float* p, float a, float b, float c, float d) { *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d); }
+__device__ __forceinline__ void hl_store4(bf16_t* p, float a, float b, float c, float d) {
+  *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(a, b), pack_bf16x2(c, d));
 }
 
-template <typename TX, typename TG, typename TO>
+template <typename TX, typename TG, typename TO, int TT>
 __global__ __launch_bounds__(256) void head_linear_mfma_kernel(
     const TX* __restrict__ x, int x_stride, const bf16_t* __restrict__ w_t, TO* __restrict__ out, int out_stride, int in_dim,
     int out_dim, int tail, const int32_t* __restrict__ positions, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, int interleaved, const TG* __restrict__ gate, int gate_stride, int gate_col,
     int gate_elems, int n_tokens) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  constexpr int NT = 4;
   const int r = lane % 16, g = lane / 16;
-  const int n0 = (blockIdx.x * 4 + wave) * 16, h = blockIdx.y, o0 = blockIdx.z * 64;
+  const int n0 = (blockIdx.x * 4 + wave) * (16 * TT), h = blockIdx.y, o0 = blockIdx.z * (16 * NT);
   if (n0 >= n_tokens) return;
   const int xw = in_dim + tail, ow = out_dim + tail;
-  const int tok = min(n0 + r, n_tokens - 1);  // (rows past the end repeat the last token and are not stored)
-  const TX* xp = x + static_cast<size_t>(tok) * x_stride + h * xw + 8 * g;
-  const bf16_t* wp = w_t + (static_cast<size_t>(h) * out_dim + o0 + r) * in_dim + 8 * g;
-  hl_f32x4_t acc[4];
+  const TX* xp[TT];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc[j] = hl_f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int n_tiles = min(4, (out_dim - o0) / 16);
+  for (int t = 0; t < TT; ++t)  // (rows past the end repeat the last token and are not stored)
+    xp[t] = x + static_cast<size_t>(min(n0 + 16 * t + r, n_tokens - 1)) * x_stride + h * xw + 8 * g;
+  const int n_tiles = min(NT, (out_dim - o0) / 16);
+  const bf16_t* wp[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)  // (tiles past the end repeat the last and are not stored)
+    wp[j] = w_t + (static_cast<size_t>(h) * out_dim + o0 + 16 * min(j, n_tiles - 1) + r) * in_dim + 8 * g;
+  hl_f32x4_t acc[TT][NT] = {};
+  HlRaw<TX> xr[TT];
+  HlFrag wr[NT];
+  auto ask = [&](int k0) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t) xr[t] = hl_raw8(xp[t] + k0);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wr[j].u = *reinterpret_cast<const hl_u32x4_t*>(wp[j] + k0);
+  };
+  ask(0);
   for (int k0 = 0; k0 < in_dim; k0 += 32) {
-    HlFrag a, a_rest;
-    a.u = hl_load8<TX>(xp + k0);
-    a_rest.u = hl_rest8<TX>(xp + k0, a.u);
+    HlFrag a[TT], rest[TT], b[NT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (j < n_tiles) {
-        HlFrag b;
-        b.u = *reinterpret_cast<const hl_u32x4_t*>(wp + static_cast<size_t>(16 * j) * in_dim + k0);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc[j], 0, 0, 0);
-        if (sizeof(TX) == 4) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_rest.v, b.v, acc[j], 0, 0, 0);
-      }
+    for (int t = 0; t < TT; ++t) {
+      a[t].u = hl_high8(xr[t]);
+      rest[t].u = hl_rest8(xr[t], a[t].u);
     }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) b[j] = wr[j];
+    ask(min(k0 + 32, in_dim - 32));  // (the last step asks for itself once more, unread)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j].v, a[t].v, acc[t][j], 0, 0, 0);
+        if (sizeof(TX) == 4) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j].v, rest[t].v, acc[t][j], 0, 0, 0);
+      }
   }
-  // acc[j][i]: token n0 + 4 g + i, column o0 + 16 j + r
+  // acc[t][j][i]: token n0 + 16 t + r, column o0 + 16 j + 4 g + i
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int n = n0 + 4 * g + i;
+  for (int t = 0; t < TT; ++t) {
+    const int n = n0 + 16 * t + r;
     if (n >= n_tokens) continue;
-    float gv = 1.f;
+    float gv[4] = {1.f, 1.f, 1.f, 1.f};
     const TG* grow = gate == nullptr ? nullptr : gate + static_cast<size_t>(n) * gate_stride + gate_col + h * gate_elems;
-    if (gate != nullptr && gate_elems == 1) gv = 1.f / (1.f + expf(-to_f32<TG>(grow[0])));
+    if (gate != nullptr && gate_elems == 1) gv[0] = gv[1] = gv[2] = gv[3] = 1.f / (1.f + expf(-to_f32<TG>(grow[0])));
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < NT; ++j)
       if (j < n_tiles) {
-        if (gate != nullptr && gate_elems > 1) gv = 1.f / (1.f + expf(-to_f32<TG>(grow[o0 + 16 * j + r])));
-        out[static_cast<size_t>(n) * out_stride + h * ow + o0 + 16 * j + r] = from_f32<TO>(acc[j][i] * gv);
+        const int o = o0 + 16 * j + 4 * g;
+        if (gate != nullptr && gate_elems > 1) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) gv[i] = 1.f / (1.f + expf(-to_f32<TG>(grow[o + i])));
+        }
+        hl_store4(out + static_cast<size_t>(n) * out_stride + h * ow + o, acc[t][j][0] * gv[0], acc[t][j][1] * gv[1], acc[t][j][2] * gv[2],
+                  acc[t][j][3] * gv[3]);
       }
   }
   if (blockIdx.z != 0 || tail == 0) return;
   const int half = tail / 2;
-  for (int i = lane; i < 16 * half; i += kWave) {
+  for (int i = lane; i < 16 * TT * half; i += kWave) {
     const int t = i / half, j = i % half, n = n0 + t;
     if (n >= n_tokens) break;
     const int ia = interleaved ? 2 * j : j, ib = interleaved ? 2 * j + 1 : j + half;
@@ -445,20 +484,29 @@ extern "C" int yk_head_linear_mfma(const void* x, int x_stride, int x_dtype, con
              "head_linear_mfma: the input's rows must be 16-byte aligned");
   YK_REQUIRE(tail == 0 || (positions != nullptr && cos_t != nullptr && sin_t != nullptr), "head_linear_mfma: a turned tail needs positions and tables");
   if (n_tokens == 0) return 0;
-  dim3 grid((n_tokens + 63) / 64, n_heads, (out_dim + 63) / 64);
   const int out_stride = n_heads * (out_dim + tail);
   if (gate == nullptr) gate_dtype = out_dtype;
-#define YK_CASE(XD, TX, GD, TG, OD, TO)                                                                                 \
-  if (x_dtype == XD && gate_dtype == GD && out_dtype == OD) {                                                           \
-    head_linear_mfma_kernel<TX, TG, TO><<<grid, 256, 0, stream>>>(                                                      \
+  YK_REQUIRE(reinterpret_cast<uintptr_t>(out) % 16 == 0, "head_linear_mfma: the output must be 16-byte aligned");
+  // as many token tiles a wave as still leave a wave for every SIMD (1,024)
+  const long long units = static_cast<long long>((n_tokens + 15) / 16) * n_heads * ((out_dim + 63) / 64);
+  const int tiles = units >= 3584 ? 4 : units >= 1792 ? 2 : 1;
+#define YK_TILES(TX, TG, TO, TT)                                                                                        \
+  if (tiles == TT) {                                                                                                    \
+    const dim3 grid((n_tokens + 64 * TT - 1) / (64 * TT), n_heads, (out_dim + 63) / 64);                                \
+    head_linear_mfma_kernel<TX, TG, TO, TT><<<grid, 256, 0, stream>>>(                                                  \
         static_cast<const TX*>(x), x_stride, static_cast<const bf16_t*>(w_t), static_cast<TO*>(out), out_stride, in_dim, \
         out_dim, tail, positions, cos_t, sin_t, interleaved, static_cast<const TG*>(gate), gate_stride, gate_col,       \
-        gate_elems, n_tokens);                                                                                                      \
+        gate_elems, n_tokens);                                                                                          \
     return yk_check_launch("head_linear_mfma");                                                                         \
+  }
+#define YK_CASE(XD, TX, GD, TG, OD, TO)                                                                                 \
+  if (x_dtype == XD && gate_dtype == GD && out_dtype == OD) {                                                           \
+    YK_TILES(TX, TG, TO, 1) YK_TILES(TX, TG, TO, 2) YK_TILES(TX, TG, TO, 4)                                             \
   }
   YK_CASE(YK_BF16, bf16_t, YK_F32, float, YK_F32, float)
   YK_CASE(YK_F32, float, YK_BF16, bf16_t, YK_BF16, bf16_t)
 #undef YK_CASE
+#undef YK_TILES
   return yk_fail("head_linear_mfma: unsupported dtype combination");
 }
 
