@@ -39,7 +39,9 @@ struct Finish {
 // lane holds w[lane % 16][8 (lane / 16) ..]); x comes from the caches straight into the B operand, since
 // no other wave of the workgroup wants the same piece.  Rows beyond N are read from the last row and
 // never stored, K beyond the end is read from valid places and meets zeros of x.  Workgroups start at
-// different chunks, so that they do not ask for addresses a whole number of rows apart at every moment.
+// different chunks, so that they do not ask for addresses a whole number of rows apart at every moment,
+// and those of one die (every eighth) at different ones too: 4,096 x 4,096 11.1 -> 8.3 us against starting
+// at the workgroup's number, 8,192 x 4,096 19.2 -> 15.5, 4,672 x 2,048 8.9 -> 8.4.
 // gated: the 16 rows are eight gate rows, then the eight up rows that belong to them.
 // Bound by the reading of the weight.
 template <typename TO>
@@ -56,7 +58,7 @@ __global__ __launch_bounds__(64 * W) void gemm_cols_kernel(const bf16_t* __restr
 #pragma unroll
   for (int j = 0; j < STEPS; ++j) wrow[j] = w + static_cast<size_t>(min(n0 + 2 * j + half, N - 1)) * ldw;
   const bf16_t* xrow = x + static_cast<size_t>(min(r, M - 1)) * ldx;
-  const int start = blockIdx.x % n_chunks;
+  const int start = (5 * blockIdx.x + blockIdx.x / 8) % n_chunks;
   auto chunk_at = [&](int i) {
     const int j = i + start;
     return (j >= n_chunks ? j - n_chunks : j) * KC;
