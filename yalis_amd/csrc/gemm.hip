@@ -261,19 +261,17 @@ __global__ __launch_bounds__(W * 64) void gemm_mfma_skinny_kernel(
   // few memory channels: where the rows are a multiple of 4 KiB apart, that is (measured at the 8B
   // shape, 8 rows: gate/up 40.2 -> 37.6 us; the decode step 3.60 -> 3.53 ms, that of the 70B shape
   // 25.9 -> 25.1; with rows 6 KiB apart, the 3B shape, it cost half a percent).  Of b alone, the
-  // workgroups of one die (every eighth) would share few starts: us, 8 and 64 rows of x, together / from
-  // b / from 5 b + b / 8: 16,384 x 4,096 26.6 / 23.3 / 22.8 and 33.5 / - / 28.1, 4,096 x 16,384 29.1 / 23.5 /
-  // 22.2 and 33.9 / - / 27.4, 12,352 x 4,096 20.6 / 19.7 / 19.3 and 27.2 / - / 23.2, 6,144 x 4,096 10.5 / 10.7 /
-  // 10.4 and 15.6 / - / 15.4.  With 33 rows of x and more a workgroup stages as many bytes of x as of the
-  // weight, which those at the same place share: there only in slices of 2,048 and more (slices of 1,792,
-  // the 8B shape's down-proj at 64 rows, 23.8 / - / 24.2).  (The unit does not depend on the chunk length, nor, with 33 rows of x and more,
-  // the start on the number of waves, so the order of the sums does not either.)
+  // workgroups of one die (every eighth) would share few starts: us, 8 rows of x, together / from b / from
+  // 5 b + b / 8: 16,384 x 4,096 26.6 / 23.3 / 22.8, 4,096 x 16,384 29.1 / 23.5 / 22.2, 12,352 x 4,096
+  // 20.6 / 19.7 / 19.3, 6,144 x 4,096 10.5 / 10.7 / 10.4.  With 33 rows of x and more a workgroup stages as
+  // many bytes of x as of the weight, which those at the same place share: not there (the 8B shape's
+  // decode step at 64 rows 5.34 -> 5.41 to 5.66 ms, also where only slices of 2,048 and more did it).  (The unit
+  // does not depend on the chunk length, so the order of the sums does not either.)
   const int n_chunks = (kb1 - kb0 + KC - 1) / KC;
   constexpr int PER_UNIT = SK_KC / KC;              // chunks in a unit of 256
   const int n_units = (kb1 - kb0 + SK_KC - 1) / SK_KC;
   const int slots = PER_UNIT * n_units;             // the last one may lie beyond the slice
-  const unsigned start_of = MT == 4 ? blockIdx.x / (8 / W) : blockIdx.x;
-  const int first_slot = ldw % 2048 == 0 && (MT < 4 || n_units >= 8) ? static_cast<int>((5 * start_of + start_of / 8) % n_units) * PER_UNIT : 0;
+  const int first_slot = MT < 4 && ldw % 2048 == 0 ? static_cast<int>((5 * blockIdx.x + blockIdx.x / 8) % n_units) * PER_UNIT : 0;
   const bool last_missing = slots > n_chunks;
   const int missing_at = slots - 1 - first_slot;    // where the last slot comes in this workgroup's order
   auto chunk_start = [&](int i) {
