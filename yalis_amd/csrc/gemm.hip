@@ -264,9 +264,9 @@ __global__ __launch_bounds__(W * 64) void gemm_mfma_skinny_kernel(
   // workgroups of one die (every eighth) would share few starts: us, 8 rows of x, together / from b / from
   // 5 b + b / 8: 16,384 x 4,096 26.6 / 23.3 / 22.8, 4,096 x 16,384 29.1 / 23.5 / 22.2, 12,352 x 4,096
   // 20.6 / 19.7 / 19.3, 6,144 x 4,096 10.5 / 10.7 / 10.4.  With 33 rows of x and more a workgroup stages as
-  // many bytes of x as of the weight, which those at the same place share: not there (the 8B shape's
-  // decode step at 64 rows 5.34 -> 5.41 to 5.66 ms, also where only slices of 2,048 and more did it).  (The unit
-  // does not depend on the chunk length, so the order of the sums does not either.)
+  // many bytes of x as of the weight, which those at the same place share: not there (64 short questions
+  // and eight tokens each, 12 layers of the 8B shape, 47.17 -> 47.39 ms).  (The unit does not depend on the
+  // chunk length, so the order of the sums does not either.)
   const int n_chunks = (kb1 - kb0 + KC - 1) / KC;
   constexpr int PER_UNIT = SK_KC / KC;              // chunks in a unit of 256
   const int n_units = (kb1 - kb0 + SK_KC - 1) / SK_KC;
