@@ -23,6 +23,7 @@ constexpr int KC = 256;      // K elements a wave takes at a time
 constexpr int ROW = KC + 8;  // an LDS row (16-byte reads of 16 neighbouring lanes meet no bank twice)
 constexpr int STEPS = KC / 32;
 constexpr int W = 8;         // waves a workgroup
+constexpr int CHAINS = 2;    // running sums a wave keeps of one output, which its products join by turns
 
 // what becomes of the sums
 struct Finish {
@@ -43,6 +44,10 @@ struct Finish {
 // and those of one die (every eighth) at different ones too: 4,096 x 4,096 11.1 -> 8.3 us against starting
 // at the workgroup's number, 8,192 x 4,096 19.2 -> 15.5, 4,672 x 2,048 8.9 -> 8.4.
 // gated: the 16 rows are eight gate rows, then the eight up rows that belong to them.
+// A wave's products join two running sums by turns: every addition rounds the sum it joins, and from a K of about
+// 5,000 on one sum a wave met more of them than the slices of the other form do.  Distance from 64 bits in parts of
+// 10^-7 of the result's norm (slices / one sum a wave / two): 1,024 x 5,632 1.41 / 1.62 / 1.22, 1,500 x 8,192
+// 1.46 / 1.92 / 1.40, 1,024 x 12,288 1.76 / 2.38 / 1.68, 2,048 x 2,048 1.32 / 1.02 / 0.86; the same time.
 // Bound by the reading of the weight.
 template <typename TO>
 __global__ __launch_bounds__(64 * W) void gemm_cols_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
@@ -54,9 +59,11 @@ __global__ __launch_bounds__(64 * W) void gemm_cols_kernel(const bf16_t* __restr
   const int r = lane % 16, g = lane / 16, half = lane / 32, l32 = lane % 32;
   const int n0 = blockIdx.x * 16;
   const int n_chunks = (K + KC - 1) / KC, k_last = K - 8;
-  const bf16_t* wrow[STEPS];
+  // the rows of a load as bytes from the workgroup's first (they leave registers for a second workgroup on the compute unit)
+  const bf16_t* w0 = w + static_cast<size_t>(n0) * ldw;
+  uint32_t wrow[STEPS];
 #pragma unroll
-  for (int j = 0; j < STEPS; ++j) wrow[j] = w + static_cast<size_t>(min(n0 + 2 * j + half, N - 1)) * ldw;
+  for (int j = 0; j < STEPS; ++j) wrow[j] = 2u * static_cast<uint32_t>(min(2 * j + half, N - 1 - n0)) * static_cast<uint32_t>(ldw);
   const bf16_t* xrow = x + static_cast<size_t>(min(r, M - 1)) * ldx;
   const int start = (5 * blockIdx.x + blockIdx.x / 8) % n_chunks;
   auto chunk_at = [&](int i) {
@@ -65,15 +72,16 @@ __global__ __launch_bounds__(64 * W) void gemm_cols_kernel(const bf16_t* __restr
   };
   u32x4_t wr[STEPS], xr[STEPS];
   auto fetch_w = [&](int kc) {
-    const int k = min(kc + 8 * l32, k_last);
+    const uint32_t k = 2u * static_cast<uint32_t>(min(kc + 8 * l32, k_last));
 #pragma unroll
-    for (int j = 0; j < STEPS; ++j) wr[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wrow[j] + k));
+    for (int j = 0; j < STEPS; ++j)
+      wr[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(w0) + (wrow[j] + k)));
   };
   auto fetch_x = [&](int kc) {
 #pragma unroll
     for (int u = 0; u < STEPS; ++u) xr[u] = *reinterpret_cast<const u32x4_t*>(xrow + min(kc + 32 * u + 8 * g, k_last));
   };
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[CHAINS] = {};
   if (wave < n_chunks) {
     fetch_w(chunk_at(wave));
     fetch_x(chunk_at(wave));
@@ -91,13 +99,13 @@ __global__ __launch_bounds__(64 * W) void gemm_cols_kernel(const bf16_t* __restr
     for (int u = 0; u < STEPS; ++u) {
       Frag8 b;
       b.u = whole || kc + 32 * u + 8 * g < K ? xr[u] : u32x4_t{0u, 0u, 0u, 0u};
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u].v, b.v, acc, 0, 0, 0);
+      acc[u % CHAINS] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u].v, b.v, acc[u % CHAINS], 0, 0, 0);
     }
     if (i + W < n_chunks) fetch_x(chunk_at(i + W));
   }
   // lane holds columns 4g .. 4g + 3 of row r of x
 #pragma unroll
-  for (int e = 0; e < 4; ++e) sums[wave][r][4 * g + e] = acc[e];
+  for (int e = 0; e < 4; ++e) sums[wave][r][4 * g + e] = acc[0][e] + acc[1][e];
   __syncthreads();
   auto total = [&](int m, int c) {
     float s = 0.f;
@@ -170,6 +178,7 @@ extern "C" int yk_gemm_cols(const void* x, const void* w, void* y, int y_dtype, 
                             const void* bias, int bias_dtype, int gated, int kind, float p0, float p1, hipStream_t stream) {
   YK_REQUIRE(M >= 0 && M <= 16 && N > 0 && K > 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0,
              "gemm_cols: up to 16 rows; K and the leading dimensions must be multiples of 8");
+  YK_REQUIRE(ldw < 1 << 27, "gemm_cols: a workgroup's rows of the weight must lie within 4 GiB");
   YK_REQUIRE(ldx >= K && ldw >= K && ldy >= (gated ? N / 2 : N), "gemm_cols: leading dimensions too small");
   YK_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0, "gemm_cols: operands must be 16-byte aligned");
   YK_REQUIRE(y_dtype == YK_BF16 || (y_dtype == YK_F32 && !gated), "gemm_cols: unsupported output dtype");

@@ -913,7 +913,7 @@ class HipOps:
         m, k = x.shape
         bf = torch.bfloat16
         return (0 < m <= 16 and not self._skinny_forced and x.dtype == bf and w.dtype == bf and w.shape[1] == k and x.stride(1) == 1 and w.stride(1) == 1
-                and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+                and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and w.stride(0) < 1 << 27 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
                 and bool(self._ask("yk_gemm_cols_ok", m, w.shape[0], k, int(slices_do))))
 
     def gemm_cols(self, x, w, out_dtype, bias=None, gated=None) -> torch.Tensor:
