@@ -1263,6 +1263,22 @@ def test_sample_small_top_k(ops, vocab):
         assert ops.sample(*args).tolist() == want, (k, top_p)
 
 
+def test_sample_temperature_that_is_no_number(ops):
+    """NaN is neither greedy nor a temperature: no probability is a number then, no token wins the race, and the most likely one stays
+    (with a small top_k too, whose rows otherwise take what their stretches hand on)."""
+    logits = torch.randn((3, 40000), generator=torch.Generator().manual_seed(5))
+    dev, want = logits.to(DEV), logits.argmax(-1).tolist()
+    full = lambda v, dt: torch.full((3,), v, dtype=dt, device=DEV)
+    t = full(0.7, torch.float32)
+    t[1] = float("nan")
+    for k, top_p in [(50, 1.0), (50, 0.8), (0, 1.0), (0, 0.8), (500, 0.9)]:
+        args = (dev, t, full(k, torch.int32), full(top_p, torch.float32), full(7, torch.int32), full(1, torch.int32))
+        alone = ops.sample(*args, whole_row=True).tolist()
+        for word in {0, min(k, 128)}:
+            got = ops.sample(*args, most_top_k=word).tolist()
+            assert got[1] == want[1] and got == alone, (k, top_p, word, got, want)
+
+
 def test_sample_rows_are_independent(ops):
     """Many rows with different settings in one launch give what each gives alone."""
     vocab = 50000

@@ -378,6 +378,13 @@ __host__ __device__ __forceinline__ int sp_settle_limit(int vocab) {
   return fits < SP_SETTLE_K ? fits : SP_SETTLE_K;
 }
 
+// Whether a row's stretches hand on what can be among its top_k, and whether a row is settled without bins: the one rule of
+// every kernel that writes or reads what is handed on.  (A temperature that is no number is neither greedy nor such a row.)
+__device__ __forceinline__ bool sp_hands_on(float temp, int k, int vocab) {
+  return temp > 0.f && k >= 1 && k <= sp_settle_limit(vocab);
+}
+__device__ __forceinline__ bool sp_settles(float temp, int k, int vocab) { return temp <= 0.f || sp_hands_on(temp, k, vocab); }
+
 // The largest logit of a row and the scale of its bins, from the stretches' parts.
 struct SampleExtent {
   ArgMax best;
@@ -711,7 +718,8 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
   __shared__ int handed;
   constexpr int PER = SP_PART / SP_THREADS;
   const int rowi = blockIdx.x, tid = threadIdx.x;
-  const int k = temperature[rowi] > 0.f ? top_k[rowi] : 0;
+  const int k = top_k[rowi];
+  const bool hands_on = sp_hands_on(temperature[rowi], k, vocab);
   int lo, hi;
   sp_part(vocab, blockIdx.y, lo, hi);
   const int n = hi - lo;
@@ -752,7 +760,7 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
     part_best[part] = best;
     part_low[part] = -neg_low;
   }
-  if (k < 1 || k > sp_settle_limit(vocab)) return;
+  if (!hands_on) return;
 
   uint32_t mine = 0;  // the thread's largest key; 0: it has none
 #pragma unroll
@@ -801,9 +809,6 @@ struct SettleShared {
 struct Settled {
   int path, token;
 };
-__device__ __forceinline__ bool sp_settles(float temp, int k, int vocab) {
-  return temp <= 0.f || (k >= 1 && k <= sp_settle_limit(vocab));
-}
 
 __device__ __forceinline__ Settled sp_settle(int rowi, int vocab, float temp, int k, float p_lim, int32_t seed, int32_t draw,
                                              const ArgMax* __restrict__ part_best, const uint32_t* __restrict__ top_key,
