@@ -1263,6 +1263,31 @@ def test_sample_small_top_k(ops, vocab):
         assert ops.sample(*args).tolist() == want, (k, top_p)
 
 
+def test_sample_small_top_k_of_masked_rows(ops):
+    """Logits of minus infinity have no mass and are not handed on: rows of which stretches are masked, or hold fewer finite logits than
+    top_k or than top_k threads, are settled as others are (path 3).  100,001 logits: seven stretches of about 14,300."""
+    vocab = 100001
+    gen = torch.Generator().manual_seed(3)
+    base = torch.randn((9, vocab), generator=gen) * 2.5
+    logits = torch.full_like(base, float("-inf"))
+    keep = [slice(vocab // 2, vocab), slice(20000, 20700), slice(50000, 50130), slice(99990, vocab), slice(7, 8), slice(0, vocab, 160), slice(0, vocab, 1000)]
+    for row, where in enumerate(keep):
+        logits[row, where] = base[row, where]
+    for q in range(4):  # about 60 threads with 16 logits each, more than a stretch hands on
+        logits[7, 4096 * q: 4096 * q + 240] = base[7, 4096 * q: 4096 * q + 240]
+    logits[8] = torch.sort(base[8]).values  # the largest side by side
+    dev, rows = logits.to(DEV), 9
+    seeds = torch.arange(rows, dtype=torch.int32, device=DEV) + 11
+    full = lambda v, dt: torch.full((rows,), v, dtype=dt, device=DEV)
+    for k, top_p, temperature in [(50, 0.8, 0.7), (50, 1.0, 1.3), (128, 0.95, 1.0), (1, 1.0, 1.0), (100, 0.0, 1.0)]:
+        args = (dev, full(temperature, torch.float32), full(k, torch.int32), full(top_p, torch.float32), seeds, full(k, torch.int32))
+        want = ops.sample(*args, whole_row=True).tolist()
+        for word in (k, 0):
+            paths = full(-1, torch.int32)
+            assert ops.sample(*args, most_top_k=word, paths=paths).tolist() == want, (k, top_p, word)
+            assert paths.tolist() == [3] * rows, (k, word, paths.tolist())
+
+
 def test_sample_temperature_that_is_no_number(ops):
     """NaN is neither greedy nor a temperature: no probability is a number then, no token wins the race, and the most likely one stays
     (with a small top_k too, whose rows otherwise take what their stretches hand on)."""

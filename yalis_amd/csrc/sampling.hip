@@ -707,6 +707,13 @@ __device__ __forceinline__ KeyBound sp_find_bound(KeyBins& b, uint32_t k, uint32
 // the stretch's tokens that can be among the row's top_k
 // The stretch is held in registers.  k threads whose largest logit reaches a bound hold k tokens that
 // do: the bound is sought over the threads' largest alone, and what reaches it is handed on in any order.
+// Where that is more than fits (large logits side by side, or fewer than k threads with a finite one),
+// the bound is sought once more over every token; then only ties are too many.  Tokens of minus
+// infinity have no mass and are not handed on: a stretch with fewer than k finite logits hands on
+// those (128,256 logits, 8 rows, top_k 50, the first half masked, us: seven kernels 63, a row of
+// which -inf was handed on and left to one workgroup 188, this 21, or 28 where the bins are launched too).
+constexpr uint32_t SP_NO_MASS = 0x007fffffu;  // order_key(-INFINITY)
+
 __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __restrict__ logits, int vocab,
                                                                const float* __restrict__ temperature,
                                                                const int32_t* __restrict__ top_k, ArgMax* __restrict__ part_best,
@@ -715,7 +722,7 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
   __shared__ ArgMax ascratch[17];
   __shared__ float fscratch[17];
   __shared__ KeyBins bins;
-  __shared__ int handed;
+  __shared__ int handed, holders;
   constexpr int PER = SP_PART / SP_THREADS;
   const int rowi = blockIdx.x, tid = threadIdx.x;
   const int k = top_k[rowi];
@@ -751,7 +758,7 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
     if (v[j] > -INFINITY) neg_low = fmaxf(neg_low, -v[j]);
   }
   sp_clear_range(bins);
-  if (tid == 0) handed = 0;
+  if (tid == 0) handed = holders = 0;
   best = block_argmax(best, ascratch);
   if (best.v == -INFINITY && best.i >= hi) best.i = 0x7fffffff;
   neg_low = block_max(neg_low, fscratch);
@@ -762,30 +769,53 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
   }
   if (!hands_on) return;
 
-  uint32_t mine = 0;  // the thread's largest key; 0: it has none
+  uint32_t mine = 0;  // the thread's largest key; 0: it has none (what stands for a place beyond the stretch has no mass either)
 #pragma unroll
-  for (int j = 0; j < PER; ++j)
-    if (place(j) < n) mine = max(mine, order_key(v[j]));
-  uint32_t bound = 1;
-  if (n > SP_PART_KEEP) {  // else all are handed on; there are more than SP_PART_KEEP / 4 >= k threads with logits
+  for (int j = 0; j < PER; ++j) mine = max(mine, order_key(v[j]));
+  if (mine <= SP_NO_MASS) mine = 0;
+  uint32_t bound = SP_NO_MASS + 1;  // (a bin may span keys below the smallest: never less than this)
+  if (n > SP_PART_KEEP) {  // else all are handed on
     sp_key_range(bins, mine ? mine : 0xffffffffu, mine);
+    const int in_wave = __popcll(__ballot(mine != 0));
+    if (tid % 64 == 0) atomicAdd(&holders, in_wave);
     __syncthreads();
-    bound = sp_find_bound(bins, k, 32, [&](auto take) {
-      if (mine) take(mine);
-    }).key;
+    if (holders >= k)
+      bound = max(bound, sp_find_bound(bins, k, 32, [&](auto take) {
+        if (mine) take(mine);
+      }).key);
   }
+  auto hand_on = [&] {
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const uint32_t key = order_key(v[j]);
-    if (place(j) < n && key >= bound) {
-      const int slot = atomicAdd(&handed, 1);
-      if (slot < SP_PART_KEEP) {
-        top_key[part * SP_PART_KEEP + slot] = key;
-        top_idx[part * SP_PART_KEEP + slot] = lo + place(j);
+    for (int j = 0; j < PER; ++j) {
+      const uint32_t key = order_key(v[j]);
+      if (key >= bound) {
+        const int slot = atomicAdd(&handed, 1);
+        if (slot < SP_PART_KEEP) {
+          top_key[part * SP_PART_KEEP + slot] = key;
+          top_idx[part * SP_PART_KEEP + slot] = lo + place(j);
+        }
       }
     }
-  }
+  };
+  hand_on();
   __syncthreads();
+  const int reach = handed;
+  if (reach > SP_PART_KEEP) {
+    __syncthreads();
+    sp_clear_bins(bins);
+    if (tid == 0) {
+      handed = 0;
+      bins.low = bound;
+    }
+    __syncthreads();
+    bound = max(bound, sp_find_bound(bins, k, SP_PART_KEEP - k, [&](auto take) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (order_key(v[j]) > SP_NO_MASS) take(order_key(v[j]));
+    }).key);
+    hand_on();
+    __syncthreads();
+  }
   if (tid == 0) top_count[part] = handed;
 }
 
@@ -858,13 +888,15 @@ __device__ __forceinline__ Settled sp_settle(int rowi, int vocab, float temp, in
   sp_key_range(st.bins, least, most);
   __syncthreads();
   const int n = st.taken;
-  if (st.misfit || n > CAND_MAX || n < k) return Settled{SP_WHOLE_ROW, 0};
-  const KeyBound bound = sp_find_bound(st.bins, k, 64, [&](auto take) {
+  if (st.misfit || n > CAND_MAX || n == 0) return Settled{SP_WHOLE_ROW, 0};
+  // (fewer than top_k: every stretch handed on all that it has, the rest of the row has no mass)
+  const uint32_t want = static_cast<uint32_t>(min(k, n));
+  const KeyBound bound = sp_find_bound(st.bins, want, 64, [&](auto take) {
     for (int j = tid; j < n; j += blockDim.x) take(st.key[j]);
   });
   const uint32_t reach = bound.above + bound.edge;
   if (reach > SP_KEPT_MAX) return Settled{SP_WHOLE_ROW, 0};
-  if (reach > static_cast<uint32_t>(k)) {
+  if (reach > want) {
     for (int j = tid; j < n; j += blockDim.x) {
       const uint32_t key = st.key[j];
       if (key >= bound.key && key <= bound.bin_high) st.edge[atomicAdd(&st.n_edge, 1)] = key;
@@ -881,7 +913,7 @@ __device__ __forceinline__ Settled sp_settle(int rowi, int vocab, float temp, in
     if (key <= bound.bin_high) {  // kept if fewer than top_k keys are larger
       uint32_t larger = bound.above;
       for (int i = 0; i < n_edge; ++i) larger += st.edge[i] > key ? 1u : 0u;
-      if (larger >= static_cast<uint32_t>(k)) continue;
+      if (larger >= want) continue;
     }
     const int slot = atomicAdd(&st.n_kept, 1);
     st.kept_key[slot] = key;
