@@ -1288,6 +1288,52 @@ def test_sample_small_top_k_of_masked_rows(ops):
             assert paths.tolist() == [3] * rows, (k, word, paths.tolist())
 
 
+def test_sample_small_top_k_with_ties(ops):
+    """Ties with the top_k-th that a stretch may not hand on, that are no list any more (1,024) or do not fit (4,096) are settled in the
+    same sums of integers, from the row itself; more than that is one workgroup's work (path 4)."""
+    vocab = 100001
+    gen = torch.Generator().manual_seed(4)
+    logits = torch.randn((8, vocab), generator=gen) * 2.5
+    logits[0, 3000:3600] = 20.0  # more than a stretch hands on
+    logits[1, 3000:4024] = 20.0  # as many as the list holds, and one more
+    logits[2, 3000:4025] = 20.0
+    logits[3, 10000:14000] = 20.0
+    logits[3, 50000:50040] = 21.0  # with some above them
+    logits[4, ::25] = 20.0  # 4,001 over all stretches, none with more than it may hand on
+    logits[5, ::20] = 20.0  # 5,001
+    logits[6] = 1.5
+    logits[7, 3000:3600] = 9.0
+    logits[7, 60000:60049] += 30.0  # the 50th is tied
+    dev, rows = logits.to(DEV), 8
+    seeds = torch.arange(rows, dtype=torch.int32, device=DEV) + 5
+    full = lambda v, dt: torch.full((rows,), v, dtype=dt, device=DEV)
+    for k, top_p, temperature in [(50, 0.8, 0.7), (50, 1.0, 2.0), (128, 0.3, 1.0), (1, 1.0, 1.0), (30, 0.0, 1.0)]:
+        args = (dev, full(temperature, torch.float32), full(k, torch.int32), full(top_p, torch.float32), seeds, full(k, torch.int32))
+        want = ops.sample(*args, whole_row=True).tolist()
+        for word in (k, 0):
+            paths = full(-1, torch.int32)
+            assert ops.sample(*args, most_top_k=word, paths=paths).tolist() == want, (k, top_p, word)
+            settled = paths.tolist()
+            assert settled[:3] == [3] * 3 and settled[4:] == [3, 4, 4, 3] and settled[3] == 3, (k, word, settled)
+
+
+@pytest.mark.parametrize("vocab,k", [(300000, 128), (300000, 50), (400003, 122), (400003, 123), (1000003, 49)])
+def test_sample_small_top_k_of_many_stretches(ops, vocab, k):
+    """More stretches than waves (19, 25, 62): a wave gathers several, and the largest top_k that is settled is 3,072 / stretches."""
+    gen = torch.Generator().manual_seed(k)
+    logits = torch.randn((3, vocab), generator=gen) * 2.5
+    logits[1] = (logits[1] * 4).round() / 4  # ties in every stretch
+    logits[2] = torch.sort(logits[2]).values
+    dev = logits.to(DEV)
+    full = lambda v, dt: torch.full((3,), v, dtype=dt, device=DEV)
+    args = (dev, full(0.9, torch.float32), full(k, torch.int32), full(0.9, torch.float32), full(8, torch.int32), full(2, torch.int32))
+    want = ops.sample(*args, whole_row=True).tolist()
+    for word in (k, 0):
+        paths = full(-1, torch.int32)
+        assert ops.sample(*args, most_top_k=word, paths=paths).tolist() == want, word
+        assert paths.tolist() == [3, 3, 3]
+
+
 def test_sample_temperature_that_is_no_number(ops):
     """NaN is neither greedy nor a temperature: no probability is a number then, no token wins the race, and the most likely one stays
     (with a small top_k too, whose rows otherwise take what their stretches hand on)."""

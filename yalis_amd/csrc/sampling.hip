@@ -324,8 +324,10 @@ __device__ int sample_whole_row(const float* __restrict__ row, int vocab, ArgMax
 constexpr int SP_PART = 16384;        // logits a workgroup of sp_extent_kernel holds at most
 constexpr int SP_PART_KEEP = 512;     // tokens that such a stretch hands on at most
 constexpr int SP_SETTLE_K = 128;      // largest top_k that is settled that way
-constexpr int SP_SETTLE_TOKENS = 3072;  // and how many tokens its stretches may hand on, without ties
-constexpr int SP_KEPT_MAX = 1024;     // tokens at least as likely as the top_k-th, ties among them
+// top_k times the stretches at most: of the CAND_MAX tokens that fit, the rest is for what a stretch hands on beyond its top_k (up
+// to 32 threads' largest and what lies beside them; a row for which that is not enough is asked itself)
+constexpr int SP_SETTLE_TOKENS = 3072;
+constexpr int SP_KEPT_MAX = 1024;     // tokens that are kept in a list
 constexpr int SP_CHUNKS = 8;
 constexpr int SP_BINS = 1024;
 constexpr int SP_THREADS = 1024;
@@ -822,7 +824,13 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
 // ---- greedy rows, and rows with a small top_k from what their stretches handed on
 // The exact thresholds, sums and the race as in sp_choose_kernel (the same values: masses are sums of
 // integers).  A key's mass of all that are at least as large is summed by one thread a kept token,
-// since they are few.  Returns the row's token and which way it went, or SP_WHOLE_ROW.
+// since they are few; ties with the top_k-th, which can be many, share one key and one mass and need no
+// list.  Where a stretch has more tokens than it may hand on, or all stretches together more than fit
+// (ties again, or very many stretches), what was handed on still gives a bound that top_k tokens reach,
+// and the row itself is asked for what reaches it (8 rows of 128,256 logits, top_k 50, 2,000 of them equal,
+// us: seven kernels 49, left to one workgroup with float32 masses 184, this 40, or 47 where the bins are launched too).
+// Returns the row's token and which way it went, or SP_WHOLE_ROW (more than CAND_MAX tokens reach
+// the bound, or none has a mass).
 struct SettleShared {
   uint32_t key[CAND_MAX];
   int32_t idx[CAND_MAX];
@@ -833,17 +841,17 @@ struct SettleShared {
   KeyBins bins;
   uint32_t edge[SP_KEPT_MAX];  // the keys of the bin that holds the top_k-th
   sp_mass_t mass_sum;
-  uint32_t p_found;
-  int taken, misfit, n_kept, n_edge;
+  uint32_t p_found, floor;
+  int taken, more, n_kept, n_edge;
 };
 struct Settled {
   int path, token;
 };
 
-__device__ __forceinline__ Settled sp_settle(int rowi, int vocab, float temp, int k, float p_lim, int32_t seed, int32_t draw,
-                                             const ArgMax* __restrict__ part_best, const uint32_t* __restrict__ top_key,
-                                             const int32_t* __restrict__ top_idx, const int32_t* __restrict__ top_count,
-                                             SettleShared& st) {
+__device__ __forceinline__ Settled sp_settle(const float* __restrict__ row, int rowi, int vocab, float temp, int k, float p_lim,
+                                             int32_t seed, int32_t draw, const ArgMax* __restrict__ part_best,
+                                             const uint32_t* __restrict__ top_key, const int32_t* __restrict__ top_idx,
+                                             const int32_t* __restrict__ top_count, SettleShared& st) {
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, n_waves = blockDim.x / 64;  // SP_BINS threads
   const int parts = sp_parts(vocab);
   const size_t first = static_cast<size_t>(rowi) * parts;
@@ -857,46 +865,77 @@ __device__ __forceinline__ Settled sp_settle(int rowi, int vocab, float temp, in
   ArgMax best{-INFINITY, 0x7fffffff};
   for (int c = tid; c < parts; c += blockDim.x) best = better(best, part_best[first + c]);
   if (tid == 0) {
-    st.taken = st.misfit = st.n_kept = st.n_edge = 0;
+    st.taken = st.more = st.n_kept = st.n_edge = 0;
     st.mass_sum = 0ull;
     st.p_found = 0u;
+    st.floor = SP_NO_MASS + 1;
   }
   sp_clear_range(st.bins);
   best = block_argmax(best, st.ascratch);
   if (temp <= 0.f) return Settled{SP_GREEDY, best.i == 0x7fffffff ? 0 : best.i};
   uint32_t least = 0xffffffffu, most = 0u;
+  auto keep = [&](int slot, uint32_t key, int32_t idx) {
+    if (slot >= CAND_MAX) return;
+    st.key[slot] = key;
+    st.idx[slot] = idx;
+    least = min(least, key);
+    most = max(most, key);
+  };
   for (int c = wave; c < parts; c += n_waves) {
-    const int count = top_count[first + c];
+    const int reached = top_count[first + c], count = min(reached, SP_PART_KEEP);
     int at = 0;
     if (lane == 0) {
       at = atomicAdd(&st.taken, count);
-      if (count > SP_PART_KEEP) st.misfit = 1;
+      if (reached > count) st.more = 1;
     }
     at = __shfl(at, 0, 64);
-    for (int j = lane; j < min(count, SP_PART_KEEP); j += 64) {
+    for (int j = lane; j < count; j += 64) {
       const bool asked = c == wave && j == lane;
-      const uint32_t key = asked ? key0 : top_key[(first + c) * SP_PART_KEEP + j];
-      const int32_t idx = asked ? idx0 : top_idx[(first + c) * SP_PART_KEEP + j];
-      if (at + j < CAND_MAX) {
-        st.key[at + j] = key;
-        st.idx[at + j] = idx;
-        least = min(least, key);
-        most = max(most, key);
-      }
+      keep(at + j, asked ? key0 : top_key[(first + c) * SP_PART_KEEP + j], asked ? idx0 : top_idx[(first + c) * SP_PART_KEEP + j]);
     }
   }
-  sp_key_range(st.bins, least, most);
-  __syncthreads();
-  const int n = st.taken;
-  if (st.misfit || n > CAND_MAX || n == 0) return Settled{SP_WHOLE_ROW, 0};
-  // (fewer than top_k: every stretch handed on all that it has, the rest of the row has no mass)
-  const uint32_t want = static_cast<uint32_t>(min(k, n));
-  const KeyBound bound = sp_find_bound(st.bins, want, 64, [&](auto take) {
-    for (int j = tid; j < n; j += blockDim.x) take(st.key[j]);
-  });
+  KeyBound bound;
+  uint32_t want;
+  int n;
+  for (bool from_row = false;; from_row = true) {
+    sp_key_range(st.bins, least, most);
+    __syncthreads();
+    n = min(st.taken, CAND_MAX);
+    const bool more = !from_row && (st.more || st.taken > CAND_MAX);  // more than were handed on, or fit
+    if (n == 0 || (from_row && st.taken > CAND_MAX)) return Settled{SP_WHOLE_ROW, 0};
+    // (fewer than top_k: every stretch handed on all that it has, the rest of the row has no mass)
+    want = static_cast<uint32_t>(min(k, n));
+    bound = sp_find_bound(st.bins, want, 64, [&](auto take) {
+      for (int j = tid; j < n; j += blockDim.x) take(st.key[j]);
+    });
+    if (!more) break;
+    // top_k tokens of the row reach this bound, and the smallest that a stretch with top_k of them handed on: what can be kept
+    // reaches the largest of these, and is taken from the row itself
+    for (int c = wave; c < parts; c += n_waves) {
+      const int count = min(top_count[first + c], SP_PART_KEEP);
+      if (count < k) continue;
+      uint32_t smallest = 0xffffffffu;
+      for (int j = lane; j < count; j += 64) smallest = min(smallest, top_key[(first + c) * SP_PART_KEEP + j]);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) smallest = min(smallest, static_cast<uint32_t>(__shfl_xor(smallest, o, 64)));
+      if (lane == 0) atomicMax(&st.floor, smallest);
+    }
+    __syncthreads();
+    const uint32_t floor = max(st.floor, bound.key);
+    if (tid == 0) st.taken = 0;
+    sp_clear_range(st.bins);
+    __syncthreads();
+    least = 0xffffffffu;
+    most = 0u;
+    for_each_logit(row, vocab, [&](float x, int i) {
+      const uint32_t key = order_key(x);
+      if (key >= floor) keep(atomicAdd(&st.taken, 1), key, i);
+    });
+  }
   const uint32_t reach = bound.above + bound.edge;
-  if (reach > SP_KEPT_MAX) return Settled{SP_WHOLE_ROW, 0};
-  if (reach > want) {
+  // ties with the top_k-th, too many for a list: the bin is then one key
+  const bool ties = reach > SP_KEPT_MAX;
+  if (!ties && reach > want) {
     for (int j = tid; j < n; j += blockDim.x) {
       const uint32_t key = st.key[j];
       if (key >= bound.key && key <= bound.bin_high) st.edge[atomicAdd(&st.n_edge, 1)] = key;
@@ -910,17 +949,18 @@ __device__ __forceinline__ Settled sp_settle(int rowi, int vocab, float temp, in
   for (int j = tid; j < n; j += blockDim.x) {
     const uint32_t key = st.key[j];
     if (key < bound.key) continue;
-    if (key <= bound.bin_high) {  // kept if fewer than top_k keys are larger
+    if (!ties && key <= bound.bin_high) {  // kept if fewer than top_k keys are larger
       uint32_t larger = bound.above;
       for (int i = 0; i < n_edge; ++i) larger += st.edge[i] > key ? 1u : 0u;
       if (larger >= want) continue;
     }
+    const sp_mass_t mj = sp_mass(expf(sp_exponent(order_value(key), inv_t, top)));
+    m += mj;
+    if (ties && key == bound.key) continue;
     const int slot = atomicAdd(&st.n_kept, 1);
     st.kept_key[slot] = key;
     st.kept_idx[slot] = st.idx[j];
-    const sp_mass_t mj = sp_mass(expf(sp_exponent(order_value(key), inv_t, top)));
     st.kept_mass[slot] = mj;
-    m += mj;
   }
   m = sp_wave_sum(m);
   if (lane == 0) atomicAdd(&st.mass_sum, m);
@@ -939,20 +979,23 @@ __device__ __forceinline__ Settled sp_settle(int rowi, int vocab, float temp, in
       for (int i = 0; i < kept; ++i) at_least += st.kept_key[i] >= key ? st.kept_mass[i] : 0ull;
       if (static_cast<double>(at_least) > limit) atomicMax(&st.p_found, key);
     }
+    if (ties && tid == 0 && static_cast<double>(total) > limit) atomicMax(&st.p_found, bound.key);
     __syncthreads();
     p_key = st.p_found;
   }
   const uint64_t seed_base = mix64((static_cast<uint64_t>(static_cast<uint32_t>(seed)) << 32) |
                                    static_cast<uint32_t>(draw));
   ArgMax win{-INFINITY, 0x7fffffff};
-  for (int j = tid; j < kept; j += blockDim.x) {
-    const uint32_t key = st.kept_key[j];
-    const int i = st.kept_idx[j];
-    if (p_active && key <= p_key && i != best.i) continue;
+  auto race = [&](uint32_t key, int i) {
+    if (p_active && key <= p_key && i != best.i) return;
     const uint64_t zz = mix64(seed_base + static_cast<uint64_t>(i));
     const float u = (static_cast<float>(zz >> 41) + 0.5f) * (1.f / 8388608.f);
     win = better(win, ArgMax{expf(sp_exponent(order_value(key), inv_t, top)) / z / -logf(u), i});
-  }
+  };
+  for (int j = tid; j < kept; j += blockDim.x) race(st.kept_key[j], st.kept_idx[j]);
+  if (ties)
+    for (int j = tid; j < n; j += blockDim.x)
+      if (st.key[j] == bound.key) race(bound.key, st.idx[j]);
   win = block_argmax(win, st.ascratch);
   return Settled{SP_DONE, win.i == 0x7fffffff ? best.i : win.i};
 }
@@ -973,7 +1016,7 @@ __global__ __launch_bounds__(SP_SETTLE_THREADS) void sp_settle_kernel(
   const float temp = temperature[rowi], p_lim = top_p[rowi];
   Settled s{SP_WHOLE_ROW, 0};
   if (sp_settles(temp, k, vocab))
-    s = sp_settle(rowi, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key, top_idx, top_count, sh.settle);
+    s = sp_settle(logits + static_cast<size_t>(rowi) * vocab, rowi, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key, top_idx, top_count, sh.settle);
   if (s.path == SP_WHOLE_ROW) {
     __syncthreads();
     s.token = sample_row(logits + static_cast<size_t>(rowi) * vocab, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], false, sh.row);
@@ -1037,7 +1080,7 @@ __device__ sp_mass_t sp_block_scan(sp_mass_t v, sp_mass_t* scratch) {
 // ---- 3: which bins hold the thresholds; one workgroup a row, one thread a bin (rows that need no
 // bins are settled here)
 __global__ __launch_bounds__(SP_BINS) void sp_plan_kernel(
-    int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+    const float* __restrict__ logits, int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
     const float* __restrict__ top_p, const int32_t* __restrict__ seeds, const int32_t* __restrict__ draws,
     const ArgMax* __restrict__ part_best, const float* __restrict__ part_low, const uint32_t* __restrict__ hist_count,
     const sp_mass_t* __restrict__ hist_mass, const uint32_t* __restrict__ top_key, const int32_t* __restrict__ top_idx,
@@ -1051,7 +1094,8 @@ __global__ __launch_bounds__(SP_BINS) void sp_plan_kernel(
   const int k = top_k[rowi];
   if (sp_settles(temp, k, vocab)) {
     const Settled s =
-        sp_settle(rowi, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key, top_idx, top_count, settle_shared);
+        sp_settle(logits + static_cast<size_t>(rowi) * vocab, rowi, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key,
+                  top_idx, top_count, settle_shared);
     if (b == 0) {
       plans[rowi].path = s.path;
       if (s.path != SP_WHOLE_ROW) out[rowi] = s.token;
@@ -1407,7 +1451,7 @@ extern "C" int yk_sample(const float* logits, int32_t* out, int n_rows, int voca
   sp_histogram_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, temperature, top_k, w.part_best, w.part_low,
                                                          w.hist_count, w.hist_mass);
   if (yk_check_launch("sample: histogram")) return -1;
-  sp_plan_kernel<<<n_rows, SP_BINS, 0, stream>>>(vocab, temperature, top_k, top_p, seeds, draws, w.part_best, w.part_low,
+  sp_plan_kernel<<<n_rows, SP_BINS, 0, stream>>>(logits, vocab, temperature, top_k, top_p, seeds, draws, w.part_best, w.part_low,
                                                  w.hist_count, w.hist_mass, w.top_key, w.top_idx, w.top_count, w.plans, out);
   if (yk_check_launch("sample: plan")) return -1;
   sp_collect_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, w.plans, w.cand_key, w.cand_e, w.cand_idx);
