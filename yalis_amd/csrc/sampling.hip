@@ -316,11 +316,11 @@ __device__ int sample_whole_row(const float* __restrict__ row, int vocab, ArgMax
 // registers and writes those tokens out, and one more workgroup a row finds the exact thresholds
 // among them and draws (sp_extent_kernel, sp_settle_kernel).  Where the caller says that all rows
 // are such rows or greedy, these two are all that is launched.  Bound by the launches and the chain
-// inside the second kernel.  128,256 logits a row, top_k 50, top_p 0.8, us a call:
-//   1 row 51 -> 29 (seven kernels -> two), 8 rows 52 -> 22 to 29 (small launches in a row / alone),
-//   64 rows 70 to 73 -> 38.  Rows under plain temperature or top_p alone pay for the shared first
-//   pass: 38.2 -> 38.8 at 8 rows, 56 -> 59 at 64.
-// Stretches of 16,384 rather than 8,192 logits: 35 against 43 at 64 rows, 29 against 28 at one.
+// inside the second kernel.  128,256 logits a row, top_k 50, top_p 0.8, us in a replayed graph, seven
+// kernels that all divide every row into bins / seven / two: 1 row 51 / 28 / 20, 8 rows 51 / 28 / 20,
+// 64 rows 68 / 37 / 28.  Rows under plain temperature or top_p alone share the first pass and neither gain
+// nor lose: 37.1 / 36.2 and 48.4 / 47.6 at 8 rows, 53.1 / 53.6 and 70.9 / 71.7 at 64.
+// Stretches of 16,384 rather than 8,192 logits: when they were chosen 35 against 43 at 64 rows, 29 against 28 at one.
 constexpr int SP_PART = 16384;        // logits a workgroup of sp_extent_kernel holds at most
 constexpr int SP_PART_KEEP = 512;     // tokens that such a stretch hands on at most
 constexpr int SP_SETTLE_K = 128;      // largest top_k that is settled that way
@@ -368,24 +368,27 @@ __device__ __forceinline__ void sp_chunk(int vocab, int chunk, int& lo, int& hi)
 }
 
 // Stretches of a row, their length (starts stay 16-byte aligned) and the largest top_k that is
-// settled among what they hand on.
-__host__ __device__ __forceinline__ int sp_parts(int vocab) { return (vocab + SP_PART - 1) / SP_PART; }
-__device__ __forceinline__ void sp_part(int vocab, int part, int& lo, int& hi) {
-  const int n = sp_parts(vocab), per = ((vocab + n - 1) / n + 3) & ~3;
-  lo = min(vocab, part * per);
-  hi = min(vocab, lo + per);
-}
-__host__ __device__ __forceinline__ int sp_settle_limit(int vocab) {
-  const int fits = SP_SETTLE_TOKENS / sp_parts(vocab);
-  return fits < SP_SETTLE_K ? fits : SP_SETTLE_K;
+// settled among what they hand on.  Made on the host, so that four kernels in a row do not start
+// with divisions.  A row has at least eight places for its stretches' parts, the rest of them hold
+// nothing: eight at known addresses are one load (64 rows of 128,256 logits, histogram and plan, us:
+// 13.0 + 5.9 as against 14.0 + 6.4 where the places were as many as the stretches).
+constexpr int SP_SLOTS = 8;
+struct Stretches {
+  int n, slots, per, most_top_k;
+};
+static Stretches sp_stretches(int vocab) {
+  Stretches s;
+  s.n = vocab / SP_PART + (vocab % SP_PART ? 1 : 0);
+  s.slots = std::max(s.n, SP_SLOTS);
+  s.per = (vocab / s.n + (vocab % s.n ? 1 : 0) + 3) & ~3;
+  s.most_top_k = std::min(SP_SETTLE_K, SP_SETTLE_TOKENS / s.n);
+  return s;
 }
 
 // Whether a row's stretches hand on what can be among its top_k, and whether a row is settled without bins: the one rule of
 // every kernel that writes or reads what is handed on.  (A temperature that is no number is neither greedy nor such a row.)
-__device__ __forceinline__ bool sp_hands_on(float temp, int k, int vocab) {
-  return temp > 0.f && k >= 1 && k <= sp_settle_limit(vocab);
-}
-__device__ __forceinline__ bool sp_settles(float temp, int k, int vocab) { return temp <= 0.f || sp_hands_on(temp, k, vocab); }
+__device__ __forceinline__ bool sp_hands_on(float temp, int k, Stretches s) { return temp > 0.f && k >= 1 && k <= s.most_top_k; }
+__device__ __forceinline__ bool sp_settles(float temp, int k, Stretches s) { return temp <= 0.f || sp_hands_on(temp, k, s); }
 
 // The largest logit of a row and the scale of its bins, from the stretches' parts.
 struct SampleExtent {
@@ -393,18 +396,26 @@ struct SampleExtent {
   float top, bin_scale;
 };
 __device__ __forceinline__ SampleExtent sp_extent(const ArgMax* __restrict__ part_best,
-                                                  const float* __restrict__ part_low, int parts, float inv_t) {
+                                                  const float* __restrict__ part_low, int slots, float inv_t) {
   SampleExtent x;
   x.best = ArgMax{-INFINITY, 0x7fffffff};
   float low = INFINITY;
-  for (int c = threadIdx.x % 64; c < parts; c += 64) {
-    x.best = better(x.best, part_best[c]);
-    low = fminf(low, part_low[c]);
-  }
+  if (slots == SP_SLOTS) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    x.best = better(x.best, ArgMax{__shfl_xor(x.best.v, o, 64), __shfl_xor(x.best.i, o, 64)});
-    low = fminf(low, __shfl_xor(low, o, 64));
+    for (int c = 0; c < SP_SLOTS; ++c) {
+      x.best = better(x.best, part_best[c]);
+      low = fminf(low, part_low[c]);
+    }
+  } else {
+    for (int c = threadIdx.x % 64; c < slots; c += 64) {
+      x.best = better(x.best, part_best[c]);
+      low = fminf(low, part_low[c]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      x.best = better(x.best, ArgMax{__shfl_xor(x.best.v, o, 64), __shfl_xor(x.best.i, o, 64)});
+      low = fminf(low, __shfl_xor(low, o, 64));
+    }
   }
   x.top = x.best.v * inv_t;
   const float far = -sp_exponent(low, inv_t, x.top);  // the smallest finite logit's distance
@@ -716,7 +727,7 @@ __device__ __forceinline__ KeyBound sp_find_bound(KeyBins& b, uint32_t k, uint32
 // which -inf was handed on and left to one workgroup 188, this 21, or 28 where the bins are launched too).
 constexpr uint32_t SP_NO_MASS = 0x007fffffu;  // order_key(-INFINITY)
 
-__global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __restrict__ logits, int vocab,
+__global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __restrict__ logits, int vocab, Stretches stretches,
                                                                const float* __restrict__ temperature,
                                                                const int32_t* __restrict__ top_k, ArgMax* __restrict__ part_best,
                                                                float* __restrict__ part_low, uint32_t* __restrict__ top_key,
@@ -727,10 +738,7 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
   __shared__ int handed, holders;
   constexpr int PER = SP_PART / SP_THREADS;
   const int rowi = blockIdx.x, tid = threadIdx.x;
-  const int k = top_k[rowi];
-  const bool hands_on = sp_hands_on(temperature[rowi], k, vocab);
-  int lo, hi;
-  sp_part(vocab, blockIdx.y, lo, hi);
+  const int lo = min(vocab, static_cast<int>(blockIdx.y) * stretches.per), hi = min(vocab, lo + stretches.per);
   const int n = hi - lo;
   const float* from = logits + static_cast<size_t>(rowi) * vocab + lo;
   // four consecutive logits a load where the row is 16-byte aligned, else one
@@ -751,30 +759,43 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
       for (int c = 0; c < 4; ++c) v[4 * q + c] = place(4 * q + c) < n ? from[place(4 * q + c)] : -INFINITY;
     }
   }
-  ArgMax best{-INFINITY, 0x7fffffff};
-  float neg_low = -INFINITY;
+  // the largest and the smallest first, which are an instruction each, then where the largest is; NaN is neither.  (What stands
+  // for a place beyond the stretch never wins: it is -INFINITY, its index the larger.)
+  float most = -INFINITY, low = INFINITY;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    // (what stands for a place beyond the stretch never wins: it is -INFINITY, its index the larger)
-    best = better(best, ArgMax{v[j], lo + place(j)});
-    if (v[j] > -INFINITY) neg_low = fmaxf(neg_low, -v[j]);
+    most = fmaxf(most, v[j]);
+    low = fminf(low, v[j]);
   }
+  if (__any(low == -INFINITY)) {  // the smallest finite one
+    low = INFINITY;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) low = fminf(low, v[j] > -INFINITY ? v[j] : INFINITY);
+  }
+  ArgMax best{most, 0x7fffffff};
+#pragma unroll
+  for (int j = PER - 1; j >= 0; --j) best.i = v[j] == most ? j : best.i;
+  if (best.i < PER) best.i = lo + (wide ? 4 * (tid + best.i / 4 * SP_THREADS) + best.i % 4 : tid + best.i * SP_THREADS);
+  float neg_low = -low;
   sp_clear_range(bins);
   if (tid == 0) handed = holders = 0;
   best = block_argmax(best, ascratch);
   if (best.v == -INFINITY && best.i >= hi) best.i = 0x7fffffff;
   neg_low = block_max(neg_low, fscratch);
   const size_t part = static_cast<size_t>(rowi) * gridDim.y + blockIdx.y;
+  const size_t slot0 = static_cast<size_t>(rowi) * stretches.slots;
   if (tid == 0) {
-    part_best[part] = best;
-    part_low[part] = -neg_low;
+    part_best[slot0 + blockIdx.y] = best;
+    part_low[slot0 + blockIdx.y] = -neg_low;
   }
-  if (!hands_on) return;
+  if (blockIdx.y == 0 && tid >= stretches.n && tid < stretches.slots && tid < SP_SLOTS) {
+    part_best[slot0 + tid] = ArgMax{-INFINITY, 0x7fffffff};
+    part_low[slot0 + tid] = INFINITY;
+  }
+  const int k = top_k[rowi];
+  if (!sp_hands_on(temperature[rowi], k, stretches)) return;
 
-  uint32_t mine = 0;  // the thread's largest key; 0: it has none (what stands for a place beyond the stretch has no mass either)
-#pragma unroll
-  for (int j = 0; j < PER; ++j) mine = max(mine, order_key(v[j]));
-  if (mine <= SP_NO_MASS) mine = 0;
+  const uint32_t mine = most > -INFINITY ? order_key(most) : 0u;  // the thread's largest key; 0: it has none with a mass
   uint32_t bound = SP_NO_MASS + 1;  // (a bin may span keys below the smallest: never less than this)
   if (n > SP_PART_KEEP) {  // else all are handed on
     sp_key_range(bins, mine ? mine : 0xffffffffu, mine);
@@ -848,12 +869,12 @@ struct Settled {
   int path, token;
 };
 
-__device__ __forceinline__ Settled sp_settle(const float* __restrict__ row, int rowi, int vocab, float temp, int k, float p_lim,
+__device__ __forceinline__ Settled sp_settle(const float* __restrict__ row, int rowi, int vocab, Stretches stretches, float temp, int k, float p_lim,
                                              int32_t seed, int32_t draw, const ArgMax* __restrict__ part_best,
                                              const uint32_t* __restrict__ top_key, const int32_t* __restrict__ top_idx,
                                              const int32_t* __restrict__ top_count, SettleShared& st) {
   const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, n_waves = blockDim.x / 64;  // SP_BINS threads
-  const int parts = sp_parts(vocab);
+  const int parts = stretches.n;
   const size_t first = static_cast<size_t>(rowi) * parts;
   // a wave's first stretch: what it handed on is asked for before its number is known
   uint32_t key0 = 0u;
@@ -863,7 +884,7 @@ __device__ __forceinline__ Settled sp_settle(const float* __restrict__ row, int 
     idx0 = top_idx[(first + wave) * SP_PART_KEEP + lane];
   }
   ArgMax best{-INFINITY, 0x7fffffff};
-  for (int c = tid; c < parts; c += blockDim.x) best = better(best, part_best[first + c]);
+  for (int c = tid; c < parts; c += blockDim.x) best = better(best, part_best[static_cast<size_t>(rowi) * stretches.slots + c]);
   if (tid == 0) {
     st.taken = st.more = st.n_kept = st.n_edge = 0;
     st.mass_sum = 0ull;
@@ -1004,9 +1025,9 @@ __device__ __forceinline__ Settled sp_settle(const float* __restrict__ row, int 
 constexpr int SP_SETTLE_THREADS = 1024;  // a wave a stretch at the usual vocabularies
 
 __global__ __launch_bounds__(SP_SETTLE_THREADS) void sp_settle_kernel(
-    const float* __restrict__ logits, int32_t* __restrict__ out, int vocab, const float* __restrict__ temperature,
-    const int32_t* __restrict__ top_k, const float* __restrict__ top_p, const int32_t* __restrict__ seeds,
-    const int32_t* __restrict__ draws, const ArgMax* __restrict__ part_best, const uint32_t* __restrict__ top_key,
+    const float* __restrict__ logits, int32_t* __restrict__ out, int vocab, Stretches stretches,
+    const float* __restrict__ temperature, const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
+    const int32_t* __restrict__ seeds, const int32_t* __restrict__ draws, const ArgMax* __restrict__ part_best, const uint32_t* __restrict__ top_key,
     const int32_t* __restrict__ top_idx, const int32_t* __restrict__ top_count, int32_t* __restrict__ paths_out) {
   __shared__ union {
     SettleShared settle;
@@ -1015,8 +1036,8 @@ __global__ __launch_bounds__(SP_SETTLE_THREADS) void sp_settle_kernel(
   const int rowi = blockIdx.x, k = top_k[rowi];
   const float temp = temperature[rowi], p_lim = top_p[rowi];
   Settled s{SP_WHOLE_ROW, 0};
-  if (sp_settles(temp, k, vocab))
-    s = sp_settle(logits + static_cast<size_t>(rowi) * vocab, rowi, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key, top_idx, top_count, sh.settle);
+  if (sp_settles(temp, k, stretches))
+    s = sp_settle(logits + static_cast<size_t>(rowi) * vocab, rowi, vocab, stretches, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key, top_idx, top_count, sh.settle);
   if (s.path == SP_WHOLE_ROW) {
     __syncthreads();
     s.token = sample_row(logits + static_cast<size_t>(rowi) * vocab, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], false, sh.row);
@@ -1029,15 +1050,17 @@ __global__ __launch_bounds__(SP_SETTLE_THREADS) void sp_settle_kernel(
 
 // ---- 2: count and mass of every bin, chunk by chunk
 __global__ __launch_bounds__(SP_THREADS) void sp_histogram_kernel(
-    const float* __restrict__ logits, int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
-    const ArgMax* __restrict__ part_best, const float* __restrict__ part_low, uint32_t* __restrict__ hist_count,
+    const float* __restrict__ logits, int vocab, Stretches stretches, const float* __restrict__ temperature,
+    const int32_t* __restrict__ top_k, const ArgMax* __restrict__ part_best, const float* __restrict__ part_low,
+    uint32_t* __restrict__ hist_count,
     sp_mass_t* __restrict__ hist_mass) {
   __shared__ uint32_t count[SP_BINS];
   __shared__ sp_mass_t mass[SP_BINS];
-  const int rowi = blockIdx.x, chunk = blockIdx.y, parts = sp_parts(vocab);
-  if (sp_settles(temperature[rowi], top_k[rowi], vocab)) return;
+  const int rowi = blockIdx.x, chunk = blockIdx.y;
+  if (sp_settles(temperature[rowi], top_k[rowi], stretches)) return;
   const float inv_t = 1.f / temperature[rowi];
-  const SampleExtent ext = sp_extent(part_best + static_cast<size_t>(rowi) * parts, part_low + static_cast<size_t>(rowi) * parts, parts, inv_t);
+  const size_t slot0 = static_cast<size_t>(rowi) * stretches.slots;
+  const SampleExtent ext = sp_extent(part_best + slot0, part_low + slot0, stretches.slots, inv_t);
   for (int b = threadIdx.x; b < SP_BINS; b += blockDim.x) {
     count[b] = 0u;
     mass[b] = 0ull;
@@ -1080,22 +1103,22 @@ __device__ sp_mass_t sp_block_scan(sp_mass_t v, sp_mass_t* scratch) {
 // ---- 3: which bins hold the thresholds; one workgroup a row, one thread a bin (rows that need no
 // bins are settled here)
 __global__ __launch_bounds__(SP_BINS) void sp_plan_kernel(
-    const float* __restrict__ logits, int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
-    const float* __restrict__ top_p, const int32_t* __restrict__ seeds, const int32_t* __restrict__ draws,
-    const ArgMax* __restrict__ part_best, const float* __restrict__ part_low, const uint32_t* __restrict__ hist_count,
+    const float* __restrict__ logits, int vocab, Stretches stretches, const float* __restrict__ temperature,
+    const int32_t* __restrict__ top_k, const float* __restrict__ top_p, const int32_t* __restrict__ seeds,
+    const int32_t* __restrict__ draws, const ArgMax* __restrict__ part_best, const float* __restrict__ part_low, const uint32_t* __restrict__ hist_count,
     const sp_mass_t* __restrict__ hist_mass, const uint32_t* __restrict__ top_key, const int32_t* __restrict__ top_idx,
     const int32_t* __restrict__ top_count, SamplePlan* __restrict__ plans, int32_t* __restrict__ out) {
   __shared__ SettleShared settle_shared;
   __shared__ sp_mass_t scan_scratch[17];
   __shared__ float fscratch[17];
   __shared__ sp_mass_t picked[3];
-  const int rowi = blockIdx.x, b = threadIdx.x, parts = sp_parts(vocab);
+  const int rowi = blockIdx.x, b = threadIdx.x;
   const float temp = temperature[rowi], p_lim = top_p[rowi];
   const int k = top_k[rowi];
-  if (sp_settles(temp, k, vocab)) {
+  if (sp_settles(temp, k, stretches)) {
     const Settled s =
-        sp_settle(logits + static_cast<size_t>(rowi) * vocab, rowi, vocab, temp, k, p_lim, seeds[rowi], draws[rowi], part_best, top_key,
-                  top_idx, top_count, settle_shared);
+        sp_settle(logits + static_cast<size_t>(rowi) * vocab, rowi, vocab, stretches, temp, k, p_lim, seeds[rowi], draws[rowi], part_best,
+                  top_key, top_idx, top_count, settle_shared);
     if (b == 0) {
       plans[rowi].path = s.path;
       if (s.path != SP_WHOLE_ROW) out[rowi] = s.token;
@@ -1110,8 +1133,8 @@ __global__ __launch_bounds__(SP_BINS) void sp_plan_kernel(
   plan.mass_before = plan.mass_total = 0ull;
   for (int c = 0; c < SP_CHUNKS; ++c) plan.chunk_at[c] = 0;
   plan.inv_t = 1.f / temp;
-  const SampleExtent ext =
-      sp_extent(part_best + static_cast<size_t>(rowi) * parts, part_low + static_cast<size_t>(rowi) * parts, parts, plan.inv_t);
+  const size_t slot0 = static_cast<size_t>(rowi) * stretches.slots;
+  const SampleExtent ext = sp_extent(part_best + slot0, part_low + slot0, stretches.slots, plan.inv_t);
   plan.best_i = ext.best.i;
   plan.best_v = ext.best.v;
   plan.bin_scale = ext.bin_scale;
@@ -1386,7 +1409,8 @@ struct SampleWorkspace {
 };
 
 static SampleWorkspace sample_workspace(void* base, size_t n_rows, int vocab) {
-  const size_t parts = n_rows * static_cast<size_t>(sp_parts(vocab));
+  const Stretches stretches = sp_stretches(vocab);
+  const size_t parts = n_rows * static_cast<size_t>(stretches.n);
   SampleWorkspace w;
   char* at = static_cast<char*>(base);
   auto take = [&](size_t bytes) {
@@ -1397,13 +1421,13 @@ static SampleWorkspace sample_workspace(void* base, size_t n_rows, int vocab) {
   w.hist_mass = reinterpret_cast<sp_mass_t*>(take(n_rows * SP_CHUNKS * SP_BINS * sizeof(sp_mass_t)));
   w.plans = reinterpret_cast<SamplePlan*>(take(n_rows * sizeof(SamplePlan)));
   w.hist_count = reinterpret_cast<uint32_t*>(take(n_rows * SP_CHUNKS * SP_BINS * sizeof(uint32_t)));
-  w.part_best = reinterpret_cast<ArgMax*>(take(parts * sizeof(ArgMax)));
+  w.part_best = reinterpret_cast<ArgMax*>(take(n_rows * stretches.slots * sizeof(ArgMax)));
   w.race_part = reinterpret_cast<ArgMax*>(take(n_rows * SP_CHUNKS * sizeof(ArgMax)));
-  w.part_low = reinterpret_cast<float*>(take(parts * sizeof(float)));
+  w.part_low = reinterpret_cast<float*>(take(n_rows * stretches.slots * sizeof(float)));
   w.cand_key = reinterpret_cast<uint32_t*>(take(n_rows * CAND_MAX * sizeof(uint32_t)));
   w.cand_e = reinterpret_cast<float*>(take(n_rows * CAND_MAX * sizeof(float)));
   w.cand_idx = reinterpret_cast<int32_t*>(take(n_rows * CAND_MAX * sizeof(int32_t)));
-  const size_t handed = sp_settle_limit(vocab) > 0 ? parts * SP_PART_KEEP : 0;
+  const size_t handed = stretches.most_top_k > 0 ? parts * SP_PART_KEEP : 0;
   w.top_key = reinterpret_cast<uint32_t*>(take(handed * sizeof(uint32_t)));
   w.top_idx = reinterpret_cast<int32_t*>(take(handed * sizeof(int32_t)));
   w.top_count = reinterpret_cast<int32_t*>(take(parts * sizeof(int32_t)));
@@ -1431,7 +1455,8 @@ extern "C" int yk_sample(const float* logits, int32_t* out, int n_rows, int voca
   YK_REQUIRE(n_rows >= 0 && vocab > 0, "sample: bad sizes");
   if (n_rows == 0) return 0;
   const size_t need = yk_sample_workspace_bytes(n_rows, vocab);
-  const bool divide = need > 0 && !force_whole_row && workspace && workspace_bytes >= need && n_rows <= 65535 && sp_parts(vocab) <= 65535;
+  const Stretches stretches = sp_stretches(vocab);
+  const bool divide = need > 0 && !force_whole_row && workspace && workspace_bytes >= need && n_rows <= 65535 && stretches.n <= 65535;
   if (!divide) {
     sample_kernel<<<n_rows, 1024, 0, stream>>>(logits, out, vocab, temperature, top_k, top_p, seeds, draws,
                                                force_whole_row, nullptr, nullptr, nullptr);
@@ -1439,19 +1464,19 @@ extern "C" int yk_sample(const float* logits, int32_t* out, int n_rows, int voca
   }
   YK_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 256 == 0, "sample: the workspace must be 256-byte aligned");
   const SampleWorkspace w = sample_workspace(workspace, static_cast<size_t>(n_rows), vocab);
-  sp_extent_kernel<<<dim3(n_rows, sp_parts(vocab)), SP_THREADS, 0, stream>>>(logits, vocab, temperature, top_k, w.part_best,
-                                                                            w.part_low, w.top_key, w.top_idx, w.top_count);
+  sp_extent_kernel<<<dim3(n_rows, stretches.n), SP_THREADS, 0, stream>>>(logits, vocab, stretches, temperature, top_k, w.part_best,
+                                                                         w.part_low, w.top_key, w.top_idx, w.top_count);
   if (yk_check_launch("sample: extent")) return -1;
-  if (most_top_k > 0 && most_top_k <= sp_settle_limit(vocab)) {
-    sp_settle_kernel<<<n_rows, SP_SETTLE_THREADS, 0, stream>>>(logits, out, vocab, temperature, top_k, top_p, seeds, draws,
+  if (most_top_k > 0 && most_top_k <= stretches.most_top_k) {
+    sp_settle_kernel<<<n_rows, SP_SETTLE_THREADS, 0, stream>>>(logits, out, vocab, stretches, temperature, top_k, top_p, seeds, draws,
                                                                w.part_best, w.top_key, w.top_idx, w.top_count, paths_out);
     return yk_check_launch("sample: settle");
   }
   const dim3 chunks(n_rows, SP_CHUNKS);
-  sp_histogram_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, temperature, top_k, w.part_best, w.part_low,
+  sp_histogram_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, stretches, temperature, top_k, w.part_best, w.part_low,
                                                          w.hist_count, w.hist_mass);
   if (yk_check_launch("sample: histogram")) return -1;
-  sp_plan_kernel<<<n_rows, SP_BINS, 0, stream>>>(logits, vocab, temperature, top_k, top_p, seeds, draws, w.part_best, w.part_low,
+  sp_plan_kernel<<<n_rows, SP_BINS, 0, stream>>>(logits, vocab, stretches, temperature, top_k, top_p, seeds, draws, w.part_best, w.part_low,
                                                  w.hist_count, w.hist_mass, w.top_key, w.top_idx, w.top_count, w.plans, out);
   if (yk_check_launch("sample: plan")) return -1;
   sp_collect_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, w.plans, w.cand_key, w.cand_e, w.cand_idx);
