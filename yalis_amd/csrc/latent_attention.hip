@@ -340,6 +340,8 @@ extern "C" int yk_head_linear(const void* x, int x_stride, int x_dtype, const vo
 //   128 -> 512 in float32    100 tokens  5.6 / 5.0 / 5.7 / 5.5    512 14.7 / 14.2 / 11.0 / 9.5    2,048 45.8 / 43.4 / 32.6 / 27.1
 //   512 -> 128 from float32  100 tokens 15.8 / 13.1 / 16.3 / 15.1  512 20.3 / 14.1 / 17.9 / 26.3  2,048 47.1 / 46.6 / 33.8 / 28.3
 // (2,048 tokens: 83 MB, 17 us at what a copy reaches.  Twice the columns a wave: 30.1 and 27.7.)
+// With a turned tail of 64 behind each head, which the head's workgroups share, 128 -> 512 (us, one tile / several, the tail
+// left to the first workgroup / several, shared): 512 tokens 17.9 / 22.7 / 10.4, 1,000 27.7 / 30.2 / 16.6, 2,048 45.9 / 35.6 / 28.2.
 typedef __bf16 hl_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float hl_f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t hl_u32x4_t __attribute__((ext_vector_type(4)));
@@ -454,11 +456,12 @@ __global__ __launch_bounds__(256) void head_linear_mfma_kernel(
                   acc[t][j][3] * gv[3]);
       }
   }
-  if (blockIdx.z != 0 || tail == 0) return;
-  const int half = tail / 2;
-  for (int i = lane; i < 16 * TT * half; i += kWave) {
+  if (tail == 0) return;
+  // the wave's tokens' tails are shared among the head's workgroups, which would otherwise end while the first still turns them
+  const int half = tail / 2, pairs = min(16 * TT, n_tokens - n0) * half;
+#pragma unroll 4
+  for (int i = static_cast<int>(blockIdx.z) * kWave + lane; i < pairs; i += static_cast<int>(gridDim.z) * kWave) {
     const int t = i / half, j = i % half, n = n0 + t;
-    if (n >= n_tokens) break;
     const int ia = interleaved ? 2 * j : j, ib = interleaved ? 2 * j + 1 : j + half;
     const TX* src = x + static_cast<size_t>(n) * x_stride + h * xw + in_dim;
     const float a = to_f32<TX>(src[ia]), b = to_f32<TX>(src[ib]);
@@ -487,9 +490,14 @@ extern "C" int yk_head_linear_mfma(const void* x, int x_stride, int x_dtype, con
   const int out_stride = n_heads * (out_dim + tail);
   if (gate == nullptr) gate_dtype = out_dtype;
   YK_REQUIRE(reinterpret_cast<uintptr_t>(out) % 16 == 0, "head_linear_mfma: the output must be 16-byte aligned");
-  // as many token tiles a wave as still leave a wave for every SIMD (1,024)
+  // as many token tiles a wave as still leave 896 waves (of the 1,024 that a wave for every SIMD would be); four only
+  // where a wave's walk over the input is long enough to share what it read: us with a turned tail, one / two / four
+  // tiles, 24 heads 96 -> 128 at 1,500 tokens 12.1 / 11.8 / 13.4, 32 heads 64 -> 128 14.0 / 12.4 / 13.8, 16 heads
+  // 128 -> 512 at 1,000 26.6 / 19.4 / 16.6.  (At both lines more tiles are faster: 1,792 units, 32 heads 512 -> 128, 25.1 / 18.6 / 27.1,
+  // 3,584 units, 16 heads 128 -> 512, 14.7 / 11.9 / 9.9; and already some way below them: 1,408 units 24.8 / 18.3, 2,816 units
+  // 36.1 / 32.9 / 27.6.)
   const long long units = static_cast<long long>((n_tokens + 15) / 16) * n_heads * ((out_dim + 63) / 64);
-  const int tiles = units >= 3584 ? 4 : units >= 1792 ? 2 : 1;
+  const int tiles = units >= 3584 && in_dim >= 128 ? 4 : units >= 1792 ? 2 : 1;
 #define YK_TILES(TX, TG, TO, TT)                                                                                        \
   if (tiles == TT) {                                                                                                    \
     const dim3 grid((n_tokens + 64 * TT - 1) / (64 * TT), n_heads, (out_dim + 63) / 64);                                \
