@@ -159,7 +159,8 @@ def test_float32_matrix_core_products(ops, form, m, n, k, xd, wd, od):
 
 # one to four rows: a wave's one or two rows of the weight, K around its pieces of 256 and its 8 (4) in flight
 @pytest.mark.parametrize("m", [1, 2, 3, 4])
-@pytest.mark.parametrize("n,k", [(1, 252), (5, 256), (9, 1028), (7, 2048), (6, 2052), (8191, 260), (8193, 1024), (8195, 1284)])
+@pytest.mark.parametrize("n,k", [(1, 252), (5, 256), (9, 1028), (7, 2048), (6, 2052), (8191, 260), (8193, 1024), (8195, 1284),
+                                 (3, 512), (5, 1800), (4095, 3844), (4097, 776), (4098, 1540)])
 @pytest.mark.parametrize("xd,wd,od", [
     (torch.float32, torch.float32, torch.float32),
     (torch.bfloat16, torch.float32, torch.bfloat16),
@@ -221,6 +222,22 @@ def test_products_with_their_own_end_at_any_width(ops):
         ops.gemm_cols(rnd((17, 264), torch.bfloat16, 48), w, torch.bfloat16)
     with pytest.raises(Exception):
         ops.gemm_cols(x, w, torch.bfloat16, gated="silu")
+
+
+@pytest.mark.parametrize("m,n,k,xd,wd,tiles", [(m, n, k, *[torch.float32 if c == "f" else torch.bfloat16 for c in types], tiles) for m, n, k, types, tiles in [
+    (1, 700, 252, "fb", False), (2, 700, 252, "ff", False), (2, 700, 252, "bf", True), (2, 700, 256, "bf", False), (3, 700, 252, "ff", True),
+    (3, 700, 256, "ff", False), (3, 700, 508, "fb", True), (3, 700, 512, "fb", False), (4, 700, 508, "ff", True),
+    (4, 700, 512, "fb", False), (4, 65536, 2048, "ff", True), (4, 65536, 2044, "ff", False), (4, 65535, 2048, "ff", False), (4, 65536, 2048, "bf", False),
+    (5, 700, 2048, "ff", True)]])
+def test_float32_products_of_few_rows_take_the_form_that_was_faster(ops, m, n, k, xd, wd, tiles):
+    """Both sides of every line between tiles of 16 rows and a wave a row of the weight, whose sums run in different orders."""
+    x, w = rnd((m, k), xd, 7), rnd((n, k), wd, 8)
+    got = ops.gemm_fma(x, w, torch.float32)
+    ops.force_float32_form(1)
+    try:
+        assert torch.equal(got, ops.gemm_fma(x, w, torch.float32)) == tiles
+    finally:
+        ops.force_float32_form()
 
 
 def test_gemm_fma_is_true_float32(ops):

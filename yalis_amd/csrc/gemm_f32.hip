@@ -7,6 +7,8 @@
 // a sum of K terms carries the rounding of about sqrt(K / 16) + 4 additions instead of sqrt(K).
 #include <algorithm>
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -156,19 +158,46 @@ __global__ __launch_bounds__(256) void gemm_f32_dot_kernel(const TX* __restrict_
         for (int e = 0; e < 4; ++e) acc[i][m][e] = fmaf(a[i][e], b[m][e], acc[i][m][e]);
   };
   int k0 = 0;
-  for (; k0 + 256 * AHEAD <= K; k0 += 256 * AHEAD) {
-    f32x4_t a[AHEAD][R];
+  // What is left of a row is asked for by four and two pieces at once too, or a wave waits for each (2 rows, bfloat16 x,
+  // N 4,096, K 1,536 8.4 -> 6.7 us, 4 rows, N 2,048 9.2 -> 5.4); and with three rows (float32 weights) and four, whose sums
+  // take long enough, x beside the weight (4 rows, bfloat16 x, 4,096 x 4,096 18.1 -> 15.1; with fewer that only costs registers).
+  constexpr bool X_AHEAD = MR == 4 || (MR == 3 && sizeof(TW) == 4);
+  auto pieces = [&](auto count) {
+    constexpr int P = decltype(count)::value;
+    f32x4_t a[P][R], b[P][MR];
 #pragma unroll
-    for (int c = 0; c < AHEAD; ++c)
+    for (int c = 0; c < P; ++c)
 #pragma unroll
       for (int i = 0; i < R; ++i) a[c][i] = stream4(wp[i] + k0 + 256 * c);
 #pragma unroll
-    for (int c = 0; c < AHEAD; ++c) {
-      f32x4_t b[MR];
+    for (int c = 0; c < P; ++c)
 #pragma unroll
-      for (int m = 0; m < MR; ++m) b[m] = load4(xp + static_cast<size_t>(m) * ldx + k0 + 256 * c);
-      add(a[c], b);
+      for (int m = 0; m < MR; ++m) b[c][m] = load4(xp + static_cast<size_t>(m) * ldx + k0 + 256 * c);
+#pragma unroll
+    for (int c = 0; c < P; ++c) add(a[c], b[c]);
+    k0 += 256 * P;
+  };
+  if constexpr (X_AHEAD) {
+    while (k0 + 256 * AHEAD <= K) pieces(std::integral_constant<int, AHEAD>());
+  } else {
+    for (; k0 + 256 * AHEAD <= K; k0 += 256 * AHEAD) {
+      f32x4_t a[AHEAD][R];
+#pragma unroll
+      for (int c = 0; c < AHEAD; ++c)
+#pragma unroll
+        for (int i = 0; i < R; ++i) a[c][i] = stream4(wp[i] + k0 + 256 * c);
+#pragma unroll
+      for (int c = 0; c < AHEAD; ++c) {
+        f32x4_t b[MR];
+#pragma unroll
+        for (int m = 0; m < MR; ++m) b[m] = load4(xp + static_cast<size_t>(m) * ldx + k0 + 256 * c);
+        add(a[c], b);
+      }
     }
+  }
+  if constexpr (MR > 1) {
+    if (AHEAD > 4 && k0 + 1024 <= K) pieces(std::integral_constant<int, 4>());
+    if (k0 + 512 <= K) pieces(std::integral_constant<int, 2>());
   }
   for (; k0 < K; k0 += 256) {
     const bool in = k0 + 4 * lane < K;  // K is a multiple of four
@@ -263,20 +292,32 @@ __global__ __launch_bounds__(64 * W) void gemm_f32_rows_kernel(const TX* __restr
 //   N 2,048, K 8,192   64 rows 102 / 218 / 176 / 160   311 rows 266 / 218 / 176 / 162   511 rows 339 / 222 / 178 / 164   (1,488, 1,404, 1,423)
 //   N 16,384, K 2,048   32 rows 48 / 61 / 48 / 47   64 rows 90 / 61 / 50 / 47   511 rows 696 / 334 / 330 / 340   (351, 391, 932)
 //   N 6,144, K 4,096   48 rows 79 / 112 / 89 / 84   1,024 rows 1,032 / 481 / 462 / 486
-// Up to four rows no tile at all: a wave a row of the weight (two from DOT_PAIR_N rows on, which share the reads of x).
+// Up to four rows no tile at all: a wave a row of the weight, or two rows, which share the reads of x: from 8,192 rows of the
+// weight on, with three rows of x (float32 weights) and four from 4,096 (4 rows, N 8,191, K 4,096, one / two rows a wave 37 / 30 us).
 // Measured (us, tiles of 16 rows / this), 1, 2, 3 and 4 rows of x:
-//   N 2,048, K 8,192   27.9 / 12.7   28.4 / 14.7   28.8 / 16.6   29.3 / 18.4 (128 tiles leave half of the compute units idle)
-//   N 3,072, K 2,048   9.5 / 6.2   9.8 / 7.4   10.1 / 8.2   10.1 / 9.2
-//   N 16,384, K 2,048   29.2 / 22.8   29.6 / 25.3   30.7 / 27.1   31.3 / 30.8
-//   N 128,256, K 2,048   197 / 153   200 / 162   205 / 186   210 / 217
+//   N 2,048, K 8,192   25.9 / 12.2   27.1 / 14.0   27.8 / 14.9   28.2 / 17.0 (128 tiles leave half of the compute units idle)
+//   N 3,072, K 2,048   8.5 / 5.9   8.6 / 6.8   8.8 / 7.5   8.9 / 8.4
+//   N 16,384, K 2,048   28.4 / 22.5   28.6 / 25.4   29.2 / 26.8   29.6 / 29.6
+//   N 128,256, K 2,048   186 / 149   190 / 157   198 / 181   204 / 211
+//   N 128,256, K 2,048, bfloat16 weights   170 / 85   174 / 104   180 / 122   183 / 140
+// Not where the tiles are faster (the same way round, over N 64 to 128,256 and K 128 to 14,336):
+//   four float32 rows against a float32 table: 65,536 x 4,096 209 / 217, 128,256 x 2,048 above (32,768 x 3,072 88 / 85);
+//   rows too short for the loads of several pieces to overlap (bfloat16 x, N 65,536): 2 rows, K 128 10.3 / 12.2, 3 rows, K 256
+//   14.9 / 20.3, (K 512 26.7 / 22.5); both float32, 3 rows, K 128 11.7 / 13.5, (K 256 16.8 / 15.5).
 // Its sums are closer to 64 bits than the tiles' (0.9 to 1.3e-7 of the result, 1.2 to 1.5e-7).
-constexpr int DOT_ROWS = 4;
-constexpr int DOT_PAIR_N = 8192;
+template <typename TX, typename TW>
+bool takes_dot(int M, int N, int K) {
+  constexpr bool both_float32 = sizeof(TX) == 4 && sizeof(TW) == 4;
+  if (M == 1) return true;
+  if (M == 2) return both_float32 || K >= 256;
+  if (M == 3) return K >= (both_float32 ? 256 : 512);
+  return M == 4 && K >= 512 && !(both_float32 && N >= 65536 && K >= 2048);
+}
 static int g_force_form = 0;  // 0: the rule; 1: few rows; 2, 4: tiles with that many groups of waves
 
 template <typename TX, typename TW, typename TO, int MR>
 void launch_dot(const TX* x, const TW* w, TO* y, int N, int K, int ldx, int ldw, int ldy, hipStream_t stream) {
-  if (N < DOT_PAIR_N)
+  if (N < (MR == 4 || (MR == 3 && sizeof(TW) == 4) ? 4096 : 8192))
     gemm_f32_dot_kernel<TX, TW, TO, MR, 1><<<(N + 3) / 4, 256, 0, stream>>>(x, w, y, N, K, ldx, ldw, ldy);
   else
     gemm_f32_dot_kernel<TX, TW, TO, MR, 2><<<(N + 7) / 8, 256, 0, stream>>>(x, w, y, N, K, ldx, ldw, ldy);
@@ -291,7 +332,7 @@ int launch(const TX* x, const TW* w, TO* y, int M, int N, int K, int ldx, int ld
     gemm_f32_tile_kernel<TX, TW, TO, 4><<<tiles, 1024, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy);
   } else if (form == 2) {
     gemm_f32_tile_kernel<TX, TW, TO, 2><<<tiles, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy);
-  } else if (M <= DOT_ROWS && g_force_form != 1) {
+  } else if (g_force_form != 1 && takes_dot<TX, TW>(M, N, K)) {
     if (M == 1)
       launch_dot<TX, TW, TO, 1>(x, w, y, N, K, ldx, ldw, ldy, stream);
     else if (M == 2)
