@@ -213,6 +213,48 @@ def test_products_with_their_own_end_are_no_further_from_64_bits(ops, n, k):
     assert far[1] <= 1.02 * far[0], far
 
 
+# both sides of every line of yk_gemm_cols_ok: rows of x, rows of w, elements, K
+@pytest.mark.parametrize("m,n,k,whole,handed_on", [
+    (1, 1024, 512, True, True), (8, 1024, 2048, True, True), (8, 1023, 2048, False, False), (9, 1024, 2048, True, False), (17, 1024, 2048, False, False),
+    (8, 1040, 6248, True, True), (8, 1040, 6256, True, False), (16, 1040, 12496, True, False), (16, 1040, 12504, False, False),
+    (8, 6352, 2048, True, False), (9, 6352, 2048, False, False), (9, 6344, 2048, True, False), (8, 6320, 2056, True, False), (8, 6336, 2056, False, False),
+    (8, 17576, 2048, True, False), (8, 17584, 2048, False, False),
+])
+def test_where_products_have_their_own_end(ops, m, n, k, whole, handed_on):
+    """Which of the two forms a product takes, told by the order of its sums, and the same value as the other up to that."""
+    x, w = rnd((m, k), torch.bfloat16, 51), rnd((n, k), torch.bfloat16, 52, scale=k**-0.5)
+    f32 = torch.float32
+    own, slices = (ops.gemm_cols(x, w, f32) if m <= 16 else None), ops.gemm_mfma_skinny(x, w, f32)
+    exact = x.double() @ w.double().T
+    # float32 sums of products of about k^-1/2, at most about 4: rounded by 2^-24 of that at each of up to k / 32 + 16 additions
+    atol = 4 * math.sqrt(k / 32 + 16) * 2.0**-24 * 8
+    close(slices, exact.cpu(), atol, 1e-6)
+    if own is not None:
+        close(own, slices.cpu(), 2 * atol, 2e-6)
+        assert not torch.equal(own, slices)
+    got, part = ops.linear(x, w, f32), ops.linear(x, w, f32, partial_ok=True)
+    assert torch.equal(got, own if whole else slices)
+    if handed_on:
+        assert torch.equal(part, own)
+    elif isinstance(part, torch.Tensor):  # one slice
+        assert torch.equal(part, slices)
+    else:
+        close(part.reduce(), slices.cpu(), atol, 1e-6)  # (torch adds the slices in an order of its own)
+    bias = rnd((n,), f32, 53)
+    close(ops.linear(x, w, f32, bias=bias), (exact + bias.double()).cpu(), 2 * atol, 1e-6)
+    if whole and handed_on and n % 16 == 0:
+        # one form whatever becomes of the product
+        assert torch.equal(ops.linear(x, w, f32, bias=bias), got + bias)
+        bf = torch.bfloat16
+        for act in ("silu", ("clamped_swish", 1.5, 1.7)):
+            assert torch.equal(ops.gate_up_act(x, w, 8, act, bf), ops.gated_act(ops.linear(x, w, bf), act, bf, group=8))
+    ops.force_cols(1)
+    try:
+        assert torch.equal(ops.linear(x, w, f32), slices)
+    finally:
+        ops.force_cols()
+
+
 def test_products_with_their_own_end_at_any_width(ops):
     """Columns that are no multiple of 16, and entries that are not finite where nothing is stored."""
     x = rnd((5, 264), torch.bfloat16, 48)

@@ -174,7 +174,8 @@ __device__ __forceinline__ float gated_pair(float g, float u, int kind, float p0
 
 // The sum of a product's K slices (or an accumulator) stands for the product's output: with
 // `round_sum` it is rounded to bfloat16 as that output would have been, so that what follows
-// does not depend on whether the product came reduced (bfloat16), as slices, or fused.
+// rounds at the same places whether the product came reduced (bfloat16), as slices, or fused
+// (and has the same bits where the same kernel made the sums).
 __device__ __forceinline__ float as_output(float v, int round_sum) {
   return round_sum ? to_f32<bf16_t>(from_f32<bf16_t>(v)) : v;
 }

@@ -287,9 +287,11 @@ class SplitSum:
     the first axis is the result.  The kernels that consume a projection (norm, rotary +
     append, gated activation) add the slices themselves, which saves a pass over memory
     of its own.  ``out_dtype`` is the dtype the product was asked for: the consumers round
-    the sum to it, so that a value does not depend on whether its product came reduced or
-    as slices.  It lives in the library's workspace: consume it before the next product
-    is launched.  One that the library made carries the workspace's generation number, and
+    the sum to it, so that the slices' sum stands for the same value as the product that
+    ``reduce`` or the library's own reduction makes of them.  (A product asked for without
+    ``partial_ok`` may be ``gemm_cols``'s, whose sums run in another order: the same up to
+    rounding.  ``linear`` says where.)  It lives in the library's workspace: consume it
+    before the next product is launched.  One that the library made carries the workspace's generation number, and
     the library refuses (``StaleWorkspace``) to consume it once a later product has taken
     the workspace."""
 
@@ -662,7 +664,14 @@ class HipOps:
     # --------------------------------------------------------------------- linear
     def linear(self, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, partial_ok: bool = False, bias=None):
         """x [M, K] . w [N, K]^T (+ bias [N]) -> [M, N].  With ``partial_ok`` (and no bias) the
-        result may come as a ``SplitSum`` for a consumer that adds the slices itself."""
+        result may come as a ``SplitSum`` for a consumer that adds the slices itself.
+
+        bfloat16 products of up to 16 rows run in one of two forms whose sums run in different orders (``gemm_cols`` and
+        K slices).  Which of them may depend on what is asked for: where slices need a kernel of their own to add them, more
+        sizes are ``gemm_cols``'s (``yk_gemm_cols_ok``).  A product has the same bits whole, as slices, with a bias added
+        afterwards or in ``gate_up_act`` where it is ``gemm_cols``'s even as slices (up to 8 rows, 6.5 M elements of w, 1,024
+        rows of w or more) and where it is never (fewer rows of w, more than 16 of x, large matrices); between these only
+        up to rounding."""
         if bias is not None:
             if isinstance(x, torch.Tensor) and self._takes_cols(x, w):
                 return self.gemm_cols(x, w, out_dtype, bias=bias)
@@ -884,13 +893,18 @@ class HipOps:
         m, k = x.shape
         n = w_gate_up.shape[0]
         bf = torch.bfloat16
+        pairs = group == self.GATE_UP_GROUP and out_dtype == bf and n % 16 == 0
+        # a matrix small enough that ``linear`` multiplies by it in this form whatever becomes of the product: here too, so
+        # that the fused pairs are those of the product
+        if pairs and self._takes_cols(x, w_gate_up, slices_do=True):
+            return self.gemm_cols(x, w_gate_up, bf, gated=activation)
         fused = (
             act > 0 and group == self.GATE_UP_GROUP and 0 < m <= SKINNY_MAX_ROWS and x.dtype == bf and w_gate_up.dtype == bf and out_dtype == bf
             and w_gate_up.shape[1] == k and k % 8 == 0 and x.stride(0) % 8 == 0 and w_gate_up.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0 and n % 16 == 0
             and self._ask("yk_gemm_skinny_splits", m, n, k, 1) == 1
         )
-        if not fused and group == self.GATE_UP_GROUP and out_dtype == bf and n % 16 == 0 and self._takes_cols(x, w_gate_up):
+        if not fused and pairs and self._takes_cols(x, w_gate_up):
             return self.gemm_cols(x, w_gate_up, bf, gated=activation)
         if not fused:
             return self.gated_act(self.linear(x, w_gate_up, out_dtype, partial_ok=True), activation, out_dtype, group=group)
