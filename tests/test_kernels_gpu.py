@@ -218,7 +218,8 @@ def test_products_with_their_own_end_are_no_further_from_64_bits(ops, n, k):
     (1, 1024, 512, True, True), (8, 1024, 2048, True, True), (8, 1023, 2048, False, False), (9, 1024, 2048, True, False), (17, 1024, 2048, False, False),
     (8, 1040, 6248, True, True), (8, 1040, 6256, True, False), (16, 1040, 12496, True, False), (16, 1040, 12504, False, False),
     (8, 6352, 2048, True, False), (9, 6352, 2048, False, False), (9, 6344, 2048, True, False), (8, 6320, 2056, True, False), (8, 6336, 2056, False, False),
-    (8, 17576, 2048, True, False), (8, 17584, 2048, False, False),
+    (8, 17576, 2048, True, False), (8, 17584, 2048, False, False), (8, 1024, 256, True, True), (8, 1024, 248, False, False), (8, 8192, 512, True, True),
+    (8, 8208, 512, False, False), (8, 14336, 896, True, False), (8, 14352, 896, False, False), (16, 10752, 896, True, False), (16, 10768, 896, False, False),
 ])
 def test_where_products_have_their_own_end(ops, m, n, k, whole, handed_on):
     """Which of the two forms a product takes, told by the order of its sums, and the same value as the other up to that."""

@@ -135,31 +135,46 @@ static int g_mode = 0;
 
 // Whether a product of these sizes goes this way; slices_do: the other form would need no kernel of its own
 // after it (its consumer adds the slices, or there is one slice only).
-// Measured in replayed graphs (us, slices and the kernel that adds them / this, 8 and 16 rows of x):
-//   plain  4,672 x 2,048   10.2 / 7.8   10.4 / 9.5      2,048 x 2,048    7.9 / 4.9    8.3 / 5.6
-//          3,072 x 4,096   10.7 / 9.2   11.4 / 11.0     2,176 x 4,096   10.6 / 8.0   11.0 / 9.7
-//            512 x   512    4.8 / 2.9    5.2 / 3.1      8,320 x 2,048   10.5 / 10.5  11.3 / 12.8
-//          5,120 x 3,072   10.5 / 10.7  11.2 / 12.5     8,192 x 4,096   15.5 / 18.6  15.8 / 22.1
-//   gated 11,264 x 2,048   12.7 / 12.1  13.5 / 14.5    16,384 x 2,048   17.5 / 15.9  18.3 / 18.5
-//          4,096 x 2,048    8.8 / 6.3    9.4 / 7.0     22,016 x 4,096   33.8 / 42.2  34.9 / 50.8
+// Measured in replayed graphs (us, slices and the kernel that adds them (without it) / this, at 1, 8 and 16 rows of x):
+//   plain  1,024 x 1,024    6.8 (4.7) / 3.3    6.9 (4.8) / 3.5    7.3 (5.2) / 3.9
+//          2,048 x 2,048    7.4 (5.0) / 4.4    7.8 (5.2) / 4.8    8.4 (5.5) / 5.5
+//          3,072 x 2,048    7.8 (5.3) / 4.7    8.2 (5.4) / 5.1    8.7 (5.8) / 6.0
+//          4,672 x 2,048    9.9 (6.9) / 6.6    9.5 (7.0) / 7.5   10.1 (7.5) / 8.9
+//          2,048 x 5,632   10.5 (7.1) / 7.8   11.2 (7.3) / 9.1   11.9 (7.8) / 10.9
+//          3,072 x 4,096   10.1 (6.3) / 7.1   10.5 (6.6) / 7.7   11.2 (7.1) / 9.1
+//          6,144 x 2,048    9.3 (6.4) / 7.0    9.5 (6.6) / 7.6   10.3 (7.1) / 9.2
+//          4,096 x 4,096   11.4 (7.7) / 8.0   11.5 (7.4) / 8.4   12.1 (7.8) / 10.1
+//          2,048 x 8,192   12.8 (7.6) / 9.4   13.9 (7.7) / 11.2  14.4 (7.9) / 13.8
+//          8,320 x 2,048   10.8 (8.4) / 8.9   10.6 (8.2) / 10.0  11.4 (8.7) / 12.2
+//         16,384 x 2,048   15.3 (13.1) / 13.6 14.8 (12.3) / 13.5 15.5 (12.6) / 16.4
+//          8,192 x 4,096   17.4 (14.8) / 13.7 17.4 (14.5) / 14.3 18.0 (14.9) / 17.7
+//         12,352 x 4,096   21.1 (18.9) / 20.7 21.1 (18.9) / 23.7 22.0 (19.4) / 30.2
+//   gated  4,096 x 2,048    8.4 / 5.5    8.9 / 5.8    9.5 / 6.6     11,264 x 2,048  12.7 / 11.0  12.7 / 11.5  13.4 / 13.5
+//         16,384 x 2,048   15.3 / 14.1  15.8 / 15.2  15.5 / 16.6    22,016 x 4,096  33.4 / 33.0  34.1 / 37.2  33.8 / 45.7
 // A workgroup of 16 columns reads x once for them, four times as often a column as the other form, and
 // ends with a barrier and a few sums: both count the more, the more workgroups a compute unit runs one
 // after another, and the first with the rows of x.  So: matrices of up to 13 M elements, and with up to
-// 8 rows of x those of up to 36 M whose K is one round of the eight waves.  (Four or sixteen waves a
-// workgroup: 4,672 x 2,048 8.0 and 8.7, 16,384 x 2,048 16.1 and 19.1, 4,096 x 2,048 6.6 and 6.3.)
+// 8 rows of x those of up to 36 M whose K is one round of the eight waves.  (These two lines were drawn when a die's
+// workgroups still started at few places, which cost the larger matrices most; since then this form is also faster some way
+// beyond them, as the table shows.  Four or sixteen waves a workgroup, then too: 4,672 x 2,048 8.0 and 8.7, 16,384 x 2,048
+// 16.1 and 19.1, 4,096 x 2,048 6.6 and 6.3.)
+// A K of a few chunks leaves waves without any, and from 8,192 columns on a second round of workgroups waits for the first
+// (two a compute unit): not below 256, and beyond 8,192 columns only up to 16 for every element of K, 12 with more than 8 rows
+// (8 and 16 rows, 8,192 x 512 5.3 / 4.3, 5.8 / 4.6; 12,288 x 512 5.5 / 5.7, 6.1 / 6.6; 25,344 x 256 4.8 / 8.2; 12,288 x 768 7.1 / 7.1,
+// 7.8 / 8.0; 16,384 x 768 7.5 / 7.9; 16,384 x 1,024 9.8 / 9.3; 27,000 x 1,024 11.3 / 14.6).
 // Where slices would do, this form still saves what starting a second round of workgroups and adding the
 // slices cost, in small matrices: a decode step of the 1B shape (qkv 3,072 x 2,048, o-proj 2,048 x 2,048)
 // went from 0.84 to 0.80 ms with up to 6.5 M elements; with up to 13 M the delta-rule design's step at eight
 // rows (down-proj 2,048 x 5,632) lost what it had gained (12.65 -> 12.82 ms for 16 steps and their prompts).
-// Only up to eight rows: at 16 the two are even (2,048 x 2,048 5.6 / 5.4), and a product that takes attention's
+// Only up to eight rows: at 16 the two are even, and a product that takes attention's
 // unmerged splits (which this form does not) has the bits of the one that takes them merged there.
-// Narrow products, of fewer than 1,024 columns, would gain too (256 x 2,048 7.2 / 4.4) and stay where they are:
+// Narrow products, of fewer than 1,024 columns, would gain too (256 x 2,048 7.2 / 4.0) and stay where they are:
 // there a product has the same bits whether it comes as slices or reduced, which programs that compare the two
 // may count on; here its sums run in another order.
 extern "C" int yk_gemm_cols_ok(int M, int N, int K, int slices_do) {
   if (M < 1 || M > 16 || K < 8 || K % 8 || N < 1) return 0;
   if (g_mode) return g_mode == 2;
-  if (N < 1024) return 0;
+  if (N < 1024 || K < KC || (N > 8192 && N > (M <= 8 ? 16LL : 12LL) * K)) return 0;
   const long long elements = static_cast<long long>(N) * K;
   if (slices_do) return M <= 8 && elements <= 6500000;
   return elements <= 13000000 || (M <= 8 && K <= W * KC && elements <= 36000000);
