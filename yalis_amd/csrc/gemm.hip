@@ -256,22 +256,26 @@ __global__ __launch_bounds__(W * 64) void gemm_mfma_skinny_kernel(
   }
 
   // The workgroups of a launch do not all start at the same place of their slices: workgroup b
-  // starts 5 b + b / 8 units of 256 into its slice and wraps round.  Row blocks started together would
+  // starts b units of 256 into its slice, or 5 b + b / 8, and wraps round.  Row blocks started together would
   // otherwise ask for addresses a whole number of rows apart at every moment, which crowd onto
   // few memory channels: where the rows are a multiple of 4 KiB apart, that is (measured at the 8B
   // shape, 8 rows: gate/up 40.2 -> 37.6 us; the decode step 3.60 -> 3.53 ms, that of the 70B shape
   // 25.9 -> 25.1; with rows 6 KiB apart, the 3B shape, it cost half a percent).  Of b alone, the
-  // workgroups of one die (every eighth) would share few starts: us, 8 rows of x, together / from b / from
-  // 5 b + b / 8: 16,384 x 4,096 26.6 / 23.3 / 22.8, 4,096 x 16,384 29.1 / 23.5 / 22.2, 12,352 x 4,096
-  // 20.6 / 19.7 / 19.3, 6,144 x 4,096 10.5 / 10.7 / 10.4.  With 33 rows of x and more a workgroup stages as
-  // many bytes of x as of the weight, which those at the same place share: not there (64 short questions
-  // and eight tokens each, 12 layers of the 8B shape, 47.17 -> 47.39 ms).  (The unit does not depend on the
+  // workgroups of one die (every eighth) share few starts where the units are an even number; where they are odd, b already
+  // takes a die through all of them.  us, 8 rows of x, from b / from 5 b + b / 8: 16 units 28,672 x 8,192 gated
+  // 158 / 149, 8 units 16,384 x 4,096 24.1 / 23.6, 4,096 x 16,384 24.0 / 22.9, 12,352 x 4,096 19.9 / 19.5, 2 units 6,144 x 4,096
+  // 10.8 / 10.5; 7 units 4,096 x 14,336 20.9 / 21.4, 5 units 4,096 x 10,240 15.7 / 15.9; at 17 and 32 rows 16,384 x 4,096
+  // 25.6 / 24.5 and 26.1 / 26.0, 4,096 x 16,384 25.2 / 24.0 and 26.3 / 25.4, 4,096 x 14,336 21.6 / 22.2 and 21.8 / 22.2.  With
+  // 33 rows of x and more a workgroup stages as many bytes of x as of the weight, which those at the same place
+  // share: not there (64 short questions and eight tokens each, 12 layers of the 8B shape, 47.17 -> 47.39 ms, though
+  // the products alone gained: 16,384 x 4,096 33.5 -> 28.1).  (The unit does not depend on the
   // chunk length, so the order of the sums does not either.)
   const int n_chunks = (kb1 - kb0 + KC - 1) / KC;
   constexpr int PER_UNIT = SK_KC / KC;              // chunks in a unit of 256
   const int n_units = (kb1 - kb0 + SK_KC - 1) / SK_KC;
   const int slots = PER_UNIT * n_units;             // the last one may lie beyond the slice
-  const int first_slot = MT < 4 && ldw % 2048 == 0 ? static_cast<int>((5 * blockIdx.x + blockIdx.x / 8) % n_units) * PER_UNIT : 0;
+  const unsigned start = n_units % 2 ? blockIdx.x : 5 * blockIdx.x + blockIdx.x / 8;
+  const int first_slot = MT < 4 && ldw % 2048 == 0 ? static_cast<int>(start % n_units) * PER_UNIT : 0;
   const bool last_missing = slots > n_chunks;
   const int missing_at = slots - 1 - first_slot;    // where the last slot comes in this workgroup's order
   auto chunk_start = [&](int i) {
