@@ -256,32 +256,36 @@ def test_where_products_have_their_own_end(ops, m, n, k, whole, handed_on):
         ops.force_cols()
 
 
+def test_biased_products_refuse_what_others_refuse(ops):
+    """Inputs and weights that are no rows end in the library's own error, with a bias and without one."""
+    from yalis_amd.ops.hip import KernelError
+
+    x, w, bias = rnd((4, 64), torch.bfloat16, 55), rnd((1024, 64), torch.bfloat16, 56), rnd((1024,), torch.bfloat16, 57)
+    for b in (None, bias):
+        for bad_x, bad_w in ((x[None], w), (x[0], w), (x, w[None]), (x, w[0]), (x[:, ::2], w[:, ::2]), (x[:, :32], w)):
+            with pytest.raises(KernelError):
+                ops.linear(bad_x, bad_w, torch.bfloat16, bias=b)
+        with pytest.raises(KernelError):
+            ops.linear(x, w, torch.bfloat16, bias=bias[:-1])
+
+
 def test_products_with_their_own_end_at_any_width(ops):
-    """Columns that are no multiple of 16, and entries that are not finite where nothing is stored."""
-    x = rnd((5, 264), torch.bfloat16, 48)
-    w = rnd((33, 264), torch.bfloat16, 49)
-    close(ops.gemm_cols(x, w, torch.float32), (x.double() @ w.double().T).cpu(), 16 * 2.0**-24 * 8 * 6, 1e-6)
+    """Columns that are no multiple of 16, K that is no multiple of a chunk, and entries that are not finite in what lies around the
+    operands: behind the K columns, before them and behind the last row."""
+    for m, n, k in ((5, 33, 264), (16, 1, 8), (1, 47, 520), (9, 17, 2304)):
+        xs, ws = rnd((m + 4, k + 24), torch.bfloat16, 48), rnd((n + 20, k + 24), torch.bfloat16, 49)
+        for t, rows in ((xs, m), (ws, n)):
+            t[:, :8] = float("nan")
+            t[:, 8 + k:] = float("inf")
+            t[rows:] = float("nan")
+        x, w = xs[:m, 8: 8 + k], ws[:n, 8: 8 + k]
+        got = ops.gemm_cols(x, w, torch.float32)
+        # the running sum, of about sqrt(k), is rounded by 2^-24 of itself at each of k / 32 + 16 additions
+        close(got, (x.double() @ w.double().T).cpu(), math.sqrt(k) * math.sqrt(k / 32 + 16) * 2.0**-24 * 8, 1e-6)
     with pytest.raises(Exception):
-        ops.gemm_cols(rnd((17, 264), torch.bfloat16, 48), w, torch.bfloat16)
+        ops.gemm_cols(rnd((17, 264), torch.bfloat16, 48), rnd((33, 264), torch.bfloat16, 49), torch.bfloat16)
     with pytest.raises(Exception):
-        ops.gemm_cols(x, w, torch.bfloat16, gated="silu")
-
-
-@pytest.mark.parametrize("m,n,k,xd,wd,tiles", [(m, n, k, *[torch.float32 if c == "f" else torch.bfloat16 for c in types], tiles) for m, n, k, types, tiles in [
-    (1, 700, 252, "fb", False), (2, 700, 252, "ff", False), (2, 700, 252, "bf", True), (2, 700, 256, "bf", False), (3, 700, 252, "ff", True),
-    (3, 700, 256, "ff", False), (3, 700, 508, "fb", True), (3, 700, 512, "fb", False), (4, 700, 508, "ff", True),
-    (4, 700, 512, "fb", False), (4, 65536, 2048, "ff", True), (4, 65536, 2044, "ff", False), (4, 65535, 2048, "ff", False), (4, 65536, 2048, "bf", False),
-    (5, 700, 2048, "ff", True)]])
-def test_float32_products_of_few_rows_take_the_form_that_was_faster(ops, m, n, k, xd, wd, tiles):
-    """Both sides of every line between tiles of 16 rows and a wave a row of the weight, whose sums run in different orders."""
-    x, w = rnd((m, k), xd, 7), rnd((n, k), wd, 8)
-    got = ops.gemm_fma(x, w, torch.float32)
-    ops.force_float32_form(1)
-    try:
-        assert torch.equal(got, ops.gemm_fma(x, w, torch.float32)) == tiles
-    finally:
-        ops.force_float32_form()
-
+        ops.gemm_cols(rnd((5, 264), torch.bfloat16, 48), rnd((33, 264), torch.bfloat16, 49), torch.bfloat16, gated="silu")
 
 def test_gemm_fma_is_true_float32(ops):
     """Inputs that a reduced-precision matrix mode would truncate: 1 + 2^-12 has more

@@ -673,8 +673,11 @@ class HipOps:
         rows of w or more) and where it is never (fewer rows of w, more than 16 of x, large matrices); between these only
         up to rounding."""
         if bias is not None:
-            if isinstance(x, torch.Tensor) and self._takes_cols(x, w):
-                return self.gemm_cols(x, w, out_dtype, bias=bias)
+            if isinstance(x, torch.Tensor):
+                self._rows(x, "linear input")
+                self._rows(w, "linear weight")
+                if self._takes_cols(x, w):
+                    return self.gemm_cols(x, w, out_dtype, bias=bias)
             # the product in float32, the bias added there, one rounding (as a product that adds
             # the bias to its accumulators rounds: the reference's biased Linear)
             acc = self.linear(x, w, torch.float32, partial_ok=False)
