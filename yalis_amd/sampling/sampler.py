@@ -14,7 +14,7 @@ what else is in the batch or on whether it was preempted and recomputed.
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import List, NamedTuple, Optional, Sequence
+from typing import List, Optional, Sequence
 
 import torch
 
@@ -44,16 +44,16 @@ class SamplingParams:
         return self.temperature == 0.0
 
 
-class PreparedRows(NamedTuple):
-    """What sampling needs on the device, one entry a row, and the largest top_k if every row is
-    greedy or has one (0: some row has none)."""
+class PreparedRows(tuple):
+    """What sampling needs on the device, one entry a row: (temperature, top_k, top_p, seeds, draws).  ``most_top_k``: the largest
+    top_k if every row is greedy or has one (0: some row has none)."""
 
-    temperature: torch.Tensor
-    top_k: torch.Tensor
-    top_p: torch.Tensor
-    seeds: torch.Tensor
-    draws: torch.Tensor
     most_top_k: int
+
+    def __new__(cls, tensors, most_top_k: int = 0):
+        rows = super().__new__(cls, tensors)
+        rows.most_top_k = most_top_k
+        return rows
 
 
 class Sampler:
@@ -80,8 +80,8 @@ class Sampler:
             [[p.top_k or 0 for p in params], [p.seed & 0x7FFFFFFF for p in params], list(draws)], dtype=torch.int32
         ).to(self.device)
         limits = [p.top_k or 0 for p in params if not p.greedy]
-        return PreparedRows(floats[0].contiguous(), ints[0].contiguous(), floats[1].contiguous(), ints[1].contiguous(),
-                            ints[2].contiguous(), max(limits) if all(limits) else 0)
+        tensors = floats[0].contiguous(), ints[0].contiguous(), floats[1].contiguous(), ints[1].contiguous(), ints[2].contiguous()
+        return PreparedRows(tensors, max(limits) if all(limits) else 0)
 
     @staticmethod
     def narrow(prepared, index: torch.Tensor):
@@ -89,14 +89,15 @@ class Sampler:
         prepared set, in that order."""
         if prepared is None:
             return None
-        return PreparedRows(*(t.index_select(0, index) for t in prepared[:-1]), prepared.most_top_k)
+        return PreparedRows((t.index_select(0, index) for t in prepared), getattr(prepared, "most_top_k", 0))
 
     def sample_prepared(self, logits: torch.Tensor, prepared, step: int) -> torch.Tensor:
-        """Token ids (int32, on the device) for rows prepared with ``prepare``; ``step`` is
-        added to every row's draw number (the step within a run that shares one preparation)."""
+        """Token ids (int32, on the device) for rows prepared with ``prepare`` (or a plain tuple of
+        the five tensors); ``step`` is added to every row's draw number (the step within a run that shares one preparation)."""
         if prepared is None:
             return self.ops.argmax(logits)
-        temperature, top_k, top_p, seeds, draws, most_top_k = prepared
+        temperature, top_k, top_p, seeds, draws = prepared
+        most_top_k = getattr(prepared, "most_top_k", 0)
         if logits.shape[0] != draws.numel():
             raise ValueError("one SamplingParams and one draw number per row of logits")
         word = {"most_top_k": most_top_k} if most_top_k and getattr(self.ops, "sample_takes_most_top_k", False) else {}
