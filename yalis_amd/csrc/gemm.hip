@@ -264,7 +264,9 @@ __global__ __launch_bounds__(W * 64) void gemm_mfma_skinny_kernel(
   // workgroups of one die (every eighth) share few starts where the units are an even number; where they are odd, b already
   // takes a die through all of them.  us, 8 rows of x, from b / from 5 b + b / 8: 16 units 28,672 x 8,192 gated
   // 158 / 149, 8 units 16,384 x 4,096 24.1 / 23.6, 4,096 x 16,384 24.0 / 22.9, 12,352 x 4,096 19.9 / 19.5, 2 units 6,144 x 4,096
-  // 10.8 / 10.5; 7 units 4,096 x 14,336 20.9 / 21.4, 5 units 4,096 x 10,240 15.7 / 15.9; at 17 and 32 rows 16,384 x 4,096
+  // 10.8 / 10.5, 4 units 16,384 x 2,048 15.0 / 13.3, 4,096 x 8,192 13.2 / 12.8; 7 units 4,096 x 14,336 20.9 / 21.4, 5 units
+  // 4,096 x 10,240 15.7 / 15.9, 11 units 10,240 x 8,192 28.7 / 29.3.  Four slices of four units (rows of 8 KiB) are the exception:
+  // 8,192 x 4,096 12.9 / 14.4, 11,264 x 4,096 17.5 / 18.9, 7,168 x 4,096 12.1 / 12.4.  At 17 and 32 rows 16,384 x 4,096
   // 25.6 / 24.5 and 26.1 / 26.0, 4,096 x 16,384 25.2 / 24.0 and 26.3 / 25.4, 4,096 x 14,336 21.6 / 22.2 and 21.8 / 22.2.  With
   // 33 rows of x and more a workgroup stages as many bytes of x as of the weight, which those at the same place
   // share: not there (64 short questions and eight tokens each, 12 layers of the 8B shape, 47.17 -> 47.39 ms, though
@@ -274,7 +276,9 @@ __global__ __launch_bounds__(W * 64) void gemm_mfma_skinny_kernel(
   constexpr int PER_UNIT = SK_KC / KC;              // chunks in a unit of 256
   const int n_units = (kb1 - kb0 + SK_KC - 1) / SK_KC;
   const int slots = PER_UNIT * n_units;             // the last one may lie beyond the slice
-  const unsigned start = n_units % 2 ? blockIdx.x : 5 * blockIdx.x + blockIdx.x / 8;
+  const int block_units = (k_block + SK_KC - 1) / SK_KC;  // (of every slice but the last)
+  const bool spread = block_units % 2 == 0 && !(block_units == 4 && gridDim.z == 4);
+  const unsigned start = spread ? 5 * blockIdx.x + blockIdx.x / 8 : blockIdx.x;
   const int first_slot = MT < 4 && ldw % 2048 == 0 ? static_cast<int>(start % n_units) * PER_UNIT : 0;
   const bool last_missing = slots > n_chunks;
   const int missing_at = slots - 1 - first_slot;    // where the last slot comes in this workgroup's order
