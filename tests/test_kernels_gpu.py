@@ -216,10 +216,12 @@ def test_products_with_their_own_end_are_no_further_from_64_bits(ops, n, k):
 # both sides of every line of yk_gemm_cols_ok: rows of x, rows of w, elements, K
 @pytest.mark.parametrize("m,n,k,whole,handed_on", [
     (1, 1024, 512, True, True), (8, 1024, 2048, True, True), (8, 1023, 2048, False, False), (9, 1024, 2048, True, False), (17, 1024, 2048, False, False),
-    (8, 1040, 6248, True, True), (8, 1040, 6256, True, False), (16, 1040, 12496, True, False), (16, 1040, 12504, False, False),
+    (8, 3168, 2048, True, True), (8, 3184, 2048, True, False), (8, 1536, 2304, True, True), (8, 1536, 2312, True, False), (8, 1024, 256, True, True),
+    (8, 1024, 248, False, False), (8, 8192, 512, True, True), (8, 8208, 512, False, False), (8, 8208, 768, True, True), (8, 12304, 520, False, False),
     (8, 6352, 2048, True, False), (9, 6352, 2048, False, False), (9, 6344, 2048, True, False), (8, 6320, 2056, True, False), (8, 6336, 2056, False, False),
-    (8, 17576, 2048, True, False), (8, 17584, 2048, False, False), (8, 1024, 256, True, True), (8, 1024, 248, False, False), (8, 8192, 512, True, True),
-    (8, 8208, 512, False, False), (8, 14336, 896, True, False), (8, 14352, 896, False, False), (16, 10752, 896, True, False), (16, 10768, 896, False, False),
+    (8, 17576, 2048, True, False), (8, 17584, 2048, False, False), (8, 16384, 1024, True, False), (8, 16400, 1024, False, False),
+    (8, 1040, 8192, True, False), (8, 1040, 8200, False, False), (4, 1040, 8200, True, False), (12, 1040, 6152, True, False), (13, 1040, 6152, False, False),
+    (16, 2112, 6144, True, False), (16, 2120, 6144, False, False),
 ])
 def test_where_products_have_their_own_end(ops, m, n, k, whole, handed_on):
     """Which of the two forms a product takes, told by the order of its sums, and the same value as the other up to that."""
@@ -249,6 +251,7 @@ def test_where_products_have_their_own_end(ops, m, n, k, whole, handed_on):
         bf = torch.bfloat16
         for act in ("silu", ("clamped_swish", 1.5, 1.7)):
             assert torch.equal(ops.gate_up_act(x, w, 8, act, bf), ops.gated_act(ops.linear(x, w, bf), act, bf, group=8))
+    assert ops.lib.yk_gemm_cols_ok(8, 16384, 256, 0) and not ops.lib.yk_gemm_cols_ok(8, 16400, 256, 0)  # (one slice, and a kernel after it)
     ops.force_cols(1)
     try:
         assert torch.equal(ops.linear(x, w, f32), slices)

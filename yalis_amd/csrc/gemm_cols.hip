@@ -158,26 +158,32 @@ static int g_mode = 0;
 // workgroups still started at few places, which cost the larger matrices most; since then this form is also faster some way
 // beyond them, as the table shows.  Four or sixteen waves a workgroup, then too: 4,672 x 2,048 8.0 and 8.7, 16,384 x 2,048
 // 16.1 and 19.1, 4,096 x 2,048 6.6 and 6.3.)
-// A K of a few chunks leaves waves without any, and from 8,192 columns on a second round of workgroups waits for the first
-// (two a compute unit): not below 256, and beyond 8,192 columns only up to 16 for every element of K, 12 with more than 8 rows
-// (8 and 16 rows, 8,192 x 512 5.3 / 4.3, 5.8 / 4.6; 12,288 x 512 5.5 / 5.7, 6.1 / 6.6; 25,344 x 256 4.8 / 8.2; 12,288 x 768 7.1 / 7.1,
-// 7.8 / 8.0; 16,384 x 768 7.5 / 7.9; 16,384 x 1,024 9.8 / 9.3; 27,000 x 1,024 11.3 / 14.6).
+// Nor where K and columns are far apart: few columns are few workgroups, whose walk over a long K is not divided any further
+// (1,024 x 8,192 at 9 and 16 rows 12.5 / 10.8 and 12.6 / 13.3, 1,024 x 11,008 at 4, 8 and 16 12.7 / 11.4, 13.2 / 13.9 and 13.8 / 17.4); a short K leaves
+// waves without a chunk, and from 8,192 columns on a second round of workgroups waits for the first, two a compute unit (with a
+// bias 16,384 x 256 6.1 / 5.2, 22,016 x 256 7.0 / 7.2 at 8 rows; 16,384 x 1,024 9.8 / 9.3, 22,016 x 1,024 11.7 / 12.4).
 // Where slices would do, this form still saves what starting a second round of workgroups and adding the
 // slices cost, in small matrices: a decode step of the 1B shape (qkv 3,072 x 2,048, o-proj 2,048 x 2,048)
 // went from 0.84 to 0.80 ms with up to 6.5 M elements; with up to 13 M the delta-rule design's step at eight
 // rows (down-proj 2,048 x 5,632) lost what it had gained (12.65 -> 12.82 ms for 16 steps and their prompts).
 // Only up to eight rows: at 16 the two are even, and a product that takes attention's
 // unmerged splits (which this form does not) has the bits of the one that takes them merged there.
+// The lines for K and columns are narrower here (8 rows, with the norm that follows, slices / this: 1,024 x 4,096 8.2 / 9.4,
+// 1,536 x 3,072 8.6 / 8.9, 1,024 x 5,632 9.4 / 11.2; one slice: 8,192 x 512 5.3 / 4.3, 12,288 x 512 5.5 / 5.7, 25,344 x 256 4.8 / 8.2,
+// 8,208 x 768 6.7 / 5.7).
 // Narrow products, of fewer than 1,024 columns, would gain too (256 x 2,048 7.2 / 4.0) and stay where they are:
 // there a product has the same bits whether it comes as slices or reduced, which programs that compare the two
 // may count on; here its sums run in another order.
 extern "C" int yk_gemm_cols_ok(int M, int N, int K, int slices_do) {
   if (M < 1 || M > 16 || K < 8 || K % 8 || N < 1) return 0;
   if (g_mode) return g_mode == 2;
-  if (N < 1024 || K < KC || (N > 8192 && N > (M <= 8 ? 16LL : 12LL) * K)) return 0;
+  if (N < 1024) return 0;
   const long long elements = static_cast<long long>(N) * K;
-  if (slices_do) return M <= 8 && elements <= 6500000;
-  return elements <= 13000000 || (M <= 8 && K <= W * KC && elements <= 36000000);
+  if (slices_do)
+    return M <= 8 && elements <= 6500000 && K >= KC && (K <= W * KC || 2LL * K <= 3LL * N) && (N <= 8192 || N <= 16LL * K);
+  if (M > 4 && K > (M <= 12 ? 8192 : 6144)) return 0;
+  if (elements <= 13000000) return N <= 64LL * K;
+  return M <= 8 && elements <= 36000000 && K <= W * KC && N <= 16LL * K;
 }
 
 // For tests and measurements: 0 the rule, 1 never, 2 wherever it can.

@@ -669,9 +669,9 @@ class HipOps:
         bfloat16 products of up to 16 rows run in one of two forms whose sums run in different orders (``gemm_cols`` and
         K slices).  Which of them may depend on what is asked for: where slices need a kernel of their own to add them, more
         sizes are ``gemm_cols``'s (``yk_gemm_cols_ok``).  A product has the same bits whole, as slices, with a bias added
-        afterwards or in ``gate_up_act`` where it is ``gemm_cols``'s even as slices (up to 8 rows, 6.5 M elements of w, 1,024
-        rows of w or more) and where it is never (fewer rows of w, more than 16 of x, large matrices); between these only
-        up to rounding."""
+        afterwards or in ``gate_up_act`` where it is ``gemm_cols``'s even as slices (most products of up to 8 rows, 6.5 M elements
+        of w and 1,024 rows of w or more) and where it is never (fewer rows of w, more than 16 of x, large matrices); between
+        these only up to rounding."""
         if bias is not None:
             if isinstance(x, torch.Tensor):
                 self._rows(x, "linear input")
