@@ -312,14 +312,13 @@ __device__ int sample_whole_row(const float* __restrict__ row, int vocab, ArgMax
 // over their tokens.  A row whose candidates do not fit is left to the one-workgroup kernel.
 //
 // A row with a small top_k needs none of the bins: its kept tokens are among the top_k largest of
-// every stretch of the row.  The pass that looks for the largest logit holds its stretch in
-// registers and writes those tokens out, and one more workgroup a row finds the exact thresholds
-// among them and draws (sp_extent_kernel, sp_settle_kernel).  Where the caller says that all rows
-// are such rows or greedy, these two are all that is launched.  Bound by the launches and the chain
-// inside the second kernel.  128,256 logits a row, top_k 50, top_p 0.8, us in a replayed graph, seven
-// kernels that all divide every row into bins / seven / two: 1 row 51 / 28 / 20, 8 rows 51 / 28 / 20,
-// 64 rows 68 / 37 / 28.  Rows under plain temperature or top_p alone share the first pass and neither gain
-// nor lose: 37.1 / 36.2 and 48.4 / 47.6 at 8 rows, 53.1 / 53.6 and 70.9 / 71.7 at 64.
+// every stretch of the row.  Where the caller says that all rows are such rows or greedy, one kernel
+// holds the stretches in registers and writes those tokens out, and one more workgroup a row finds
+// the exact thresholds among them and draws (sp_top_kernel, sp_settle_kernel).  Bound by the launches
+// and the chain inside the second kernel.  128,256 logits a row, top_k 50, top_p 0.8, us in a
+// replayed graph, by bins / this: 1 row 51 / 20, 8 rows 51 / 20, 64 rows 68 / 28.  (Where only some rows
+// are such rows the bins are needed anyway, and settling those rows beside them made the chain of the
+// others longer: 64 rows of which half have a top_k of up to 50, 99 / 110.)
 // Stretches of 16,384 rather than 8,192 logits: when they were chosen 35 against 43 at 64 rows, 29 against 28 at one.
 constexpr int SP_PART = 16384;        // logits a workgroup of sp_extent_kernel holds at most
 constexpr int SP_PART_KEEP = 512;     // tokens that such a stretch hands on at most
@@ -367,19 +366,14 @@ __device__ __forceinline__ void sp_chunk(int vocab, int chunk, int& lo, int& hi)
   hi = min(vocab, lo + per);
 }
 
-// Stretches of a row, their length (starts stay 16-byte aligned) and the largest top_k that is
-// settled among what they hand on.  Made on the host, so that four kernels in a row do not start
-// with divisions.  A row has at least eight places for its stretches' parts, the rest of them hold
-// nothing: eight at known addresses are one load (64 rows of 128,256 logits, histogram and plan, us:
-// 13.0 + 5.9 as against 14.0 + 6.4 where the places were as many as the stretches).
-constexpr int SP_SLOTS = 8;
+// Stretches of a row, their length (starts stay 16-byte aligned) and the largest top_k that is settled
+// among what they hand on.  Made on the host, so that kernels do not start with divisions.
 struct Stretches {
-  int n, slots, per, most_top_k;
+  int n, per, most_top_k;
 };
 static Stretches sp_stretches(int vocab) {
   Stretches s;
   s.n = vocab / SP_PART + (vocab % SP_PART ? 1 : 0);
-  s.slots = std::max(s.n, SP_SLOTS);
   s.per = (vocab / s.n + (vocab % s.n ? 1 : 0) + 3) & ~3;
   s.most_top_k = std::min(SP_SETTLE_K, SP_SETTLE_TOKENS / s.n);
   return s;
@@ -390,32 +384,19 @@ static Stretches sp_stretches(int vocab) {
 __device__ __forceinline__ bool sp_hands_on(float temp, int k, Stretches s) { return temp > 0.f && k >= 1 && k <= s.most_top_k; }
 __device__ __forceinline__ bool sp_settles(float temp, int k, Stretches s) { return temp <= 0.f || sp_hands_on(temp, k, s); }
 
-// The largest logit of a row and the scale of its bins, from the stretches' parts.
+// The largest logit of a row and the scale of its bins, from the chunks' parts.
 struct SampleExtent {
   ArgMax best;
   float top, bin_scale;
 };
 __device__ __forceinline__ SampleExtent sp_extent(const ArgMax* __restrict__ part_best,
-                                                  const float* __restrict__ part_low, int slots, float inv_t) {
+                                                  const float* __restrict__ part_low, float inv_t) {
   SampleExtent x;
   x.best = ArgMax{-INFINITY, 0x7fffffff};
   float low = INFINITY;
-  if (slots == SP_SLOTS) {
-#pragma unroll
-    for (int c = 0; c < SP_SLOTS; ++c) {
-      x.best = better(x.best, part_best[c]);
-      low = fminf(low, part_low[c]);
-    }
-  } else {
-    for (int c = threadIdx.x % 64; c < slots; c += 64) {
-      x.best = better(x.best, part_best[c]);
-      low = fminf(low, part_low[c]);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      x.best = better(x.best, ArgMax{__shfl_xor(x.best.v, o, 64), __shfl_xor(x.best.i, o, 64)});
-      low = fminf(low, __shfl_xor(low, o, 64));
-    }
+  for (int c = 0; c < SP_CHUNKS; ++c) {
+    x.best = better(x.best, part_best[c]);
+    low = fminf(low, part_low[c]);
   }
   x.top = x.best.v * inv_t;
   const float far = -sp_exponent(low, inv_t, x.top);  // the smallest finite logit's distance
@@ -625,7 +606,11 @@ __global__ __launch_bounds__(1024) void sample_kernel(
     // the row was divided among workgroups: finish what they left, or do the whole row here
     const SamplePlan& plan = plans[rowi];
     if (paths_out && threadIdx.x == 0) paths_out[rowi] = plan.path;
-    if (plan.path == SP_DONE || plan.path == SP_GREEDY) return;
+    if (plan.path == SP_DONE) return;
+    if (plan.path == SP_GREEDY) {
+      if (threadIdx.x == 0) out[rowi] = plan.best_i == 0x7fffffff ? 0 : plan.best_i;
+      return;
+    }
     if (plan.path == SP_RACE) {
       if (threadIdx.x == 0) {
         ArgMax win{-INFINITY, 0x7fffffff};
@@ -716,24 +701,23 @@ __device__ __forceinline__ KeyBound sp_find_bound(KeyBins& b, uint32_t k, uint32
   }
 }
 
-// ---- 1: the largest and the smallest finite logit of each stretch, and of a row with a small top_k
-// the stretch's tokens that can be among the row's top_k
+// ---- all rows greedy or with a small top_k, 1: the largest logit of each stretch, and of a row with a
+// top_k the stretch's tokens that can be among the row's
 // The stretch is held in registers.  k threads whose largest logit reaches a bound hold k tokens that
 // do: the bound is sought over the threads' largest alone, and what reaches it is handed on in any order.
 // Where that is more than fits (large logits side by side, or fewer than k threads with a finite one),
 // the bound is sought once more over every token; then only ties are too many.  Tokens of minus
 // infinity have no mass and are not handed on: a stretch with fewer than k finite logits hands on
 // those (128,256 logits, 8 rows, top_k 50, the first half masked, us: seven kernels 63, a row of
-// which -inf was handed on and left to one workgroup 188, this 21, or 28 where the bins are launched too).
+// which -inf was handed on and left to one workgroup 188, this 21).
 constexpr uint32_t SP_NO_MASS = 0x007fffffu;  // order_key(-INFINITY)
 
-__global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __restrict__ logits, int vocab, Stretches stretches,
-                                                               const float* __restrict__ temperature,
-                                                               const int32_t* __restrict__ top_k, ArgMax* __restrict__ part_best,
-                                                               float* __restrict__ part_low, uint32_t* __restrict__ top_key,
-                                                               int32_t* __restrict__ top_idx, int32_t* __restrict__ top_count) {
+__global__ __launch_bounds__(SP_THREADS) void sp_top_kernel(const float* __restrict__ logits, int vocab, Stretches stretches,
+                                                            const float* __restrict__ temperature,
+                                                            const int32_t* __restrict__ top_k, ArgMax* __restrict__ part_best,
+                                                            uint32_t* __restrict__ top_key, int32_t* __restrict__ top_idx,
+                                                            int32_t* __restrict__ top_count) {
   __shared__ ArgMax ascratch[17];
-  __shared__ float fscratch[17];
   __shared__ KeyBins bins;
   __shared__ int handed, holders;
   constexpr int PER = SP_PART / SP_THREADS;
@@ -759,39 +743,21 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
       for (int c = 0; c < 4; ++c) v[4 * q + c] = place(4 * q + c) < n ? from[place(4 * q + c)] : -INFINITY;
     }
   }
-  // the largest and the smallest first, which are an instruction each, then where the largest is; NaN is neither.  (What stands
-  // for a place beyond the stretch never wins: it is -INFINITY, its index the larger.)
-  float most = -INFINITY, low = INFINITY;
+  // the largest first, which is an instruction a logit, then where it is; NaN is not the largest.  (What stands for a place
+  // beyond the stretch never wins: it is -INFINITY, its index the larger.)
+  float most = -INFINITY;
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    most = fmaxf(most, v[j]);
-    low = fminf(low, v[j]);
-  }
-  if (__any(low == -INFINITY)) {  // the smallest finite one
-    low = INFINITY;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) low = fminf(low, v[j] > -INFINITY ? v[j] : INFINITY);
-  }
+  for (int j = 0; j < PER; ++j) most = fmaxf(most, v[j]);
   ArgMax best{most, 0x7fffffff};
 #pragma unroll
   for (int j = PER - 1; j >= 0; --j) best.i = v[j] == most ? j : best.i;
   if (best.i < PER) best.i = lo + (wide ? 4 * (tid + best.i / 4 * SP_THREADS) + best.i % 4 : tid + best.i * SP_THREADS);
-  float neg_low = -low;
   sp_clear_range(bins);
   if (tid == 0) handed = holders = 0;
   best = block_argmax(best, ascratch);
   if (best.v == -INFINITY && best.i >= hi) best.i = 0x7fffffff;
-  neg_low = block_max(neg_low, fscratch);
-  const size_t part = static_cast<size_t>(rowi) * gridDim.y + blockIdx.y;
-  const size_t slot0 = static_cast<size_t>(rowi) * stretches.slots;
-  if (tid == 0) {
-    part_best[slot0 + blockIdx.y] = best;
-    part_low[slot0 + blockIdx.y] = -neg_low;
-  }
-  if (blockIdx.y == 0 && tid >= stretches.n && tid < stretches.slots && tid < SP_SLOTS) {
-    part_best[slot0 + tid] = ArgMax{-INFINITY, 0x7fffffff};
-    part_low[slot0 + tid] = INFINITY;
-  }
+  const size_t part = static_cast<size_t>(rowi) * stretches.n + blockIdx.y;
+  if (tid == 0) part_best[part] = best;
   const int k = top_k[rowi];
   if (!sp_hands_on(temperature[rowi], k, stretches)) return;
 
@@ -842,14 +808,14 @@ __global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __re
   if (tid == 0) top_count[part] = handed;
 }
 
-// ---- greedy rows, and rows with a small top_k from what their stretches handed on
+// ---- 2: greedy rows, and rows with a top_k from what their stretches handed on
 // The exact thresholds, sums and the race as in sp_choose_kernel (the same values: masses are sums of
 // integers).  A key's mass of all that are at least as large is summed by one thread a kept token,
 // since they are few; ties with the top_k-th, which can be many, share one key and one mass and need no
 // list.  Where a stretch has more tokens than it may hand on, or all stretches together more than fit
 // (ties again, or very many stretches), what was handed on still gives a bound that top_k tokens reach,
 // and the row itself is asked for what reaches it (8 rows of 128,256 logits, top_k 50, 2,000 of them equal,
-// us: seven kernels 49, left to one workgroup with float32 masses 184, this 40, or 47 where the bins are launched too).
+// us: seven kernels 49, left to one workgroup with float32 masses 184, this 40).
 // Returns the row's token and which way it went, or SP_WHOLE_ROW (more than CAND_MAX tokens reach
 // the bound, or none has a mass).
 struct SettleShared {
@@ -884,7 +850,7 @@ __device__ __forceinline__ Settled sp_settle(const float* __restrict__ row, int 
     idx0 = top_idx[(first + wave) * SP_PART_KEEP + lane];
   }
   ArgMax best{-INFINITY, 0x7fffffff};
-  for (int c = tid; c < parts; c += blockDim.x) best = better(best, part_best[static_cast<size_t>(rowi) * stretches.slots + c]);
+  for (int c = tid; c < parts; c += blockDim.x) best = better(best, part_best[first + c]);
   if (tid == 0) {
     st.taken = st.more = st.n_kept = st.n_edge = 0;
     st.mass_sum = 0ull;
@@ -1021,7 +987,6 @@ __device__ __forceinline__ Settled sp_settle(const float* __restrict__ row, int 
   return Settled{SP_DONE, win.i == 0x7fffffff ? best.i : win.i};
 }
 
-// ---- 2, where all rows are such rows
 constexpr int SP_SETTLE_THREADS = 1024;  // a wave a stretch at the usual vocabularies
 
 __global__ __launch_bounds__(SP_SETTLE_THREADS) void sp_settle_kernel(
@@ -1048,19 +1013,42 @@ __global__ __launch_bounds__(SP_SETTLE_THREADS) void sp_settle_kernel(
   }
 }
 
+// ---- other batches, 1: the largest and the smallest finite logit of each chunk
+__global__ __launch_bounds__(SP_THREADS) void sp_extent_kernel(const float* __restrict__ logits, int vocab,
+                                                               ArgMax* __restrict__ part_best,
+                                                               float* __restrict__ part_low) {
+  __shared__ ArgMax ascratch[17];
+  __shared__ float fscratch[17];
+  const int rowi = blockIdx.x, chunk = blockIdx.y;
+  const float* row = logits + static_cast<size_t>(rowi) * vocab;
+  int lo, hi;
+  sp_chunk(vocab, chunk, lo, hi);
+  ArgMax best{-INFINITY, 0x7fffffff};
+  float neg_low = -INFINITY;
+  for_each_logit(row + lo, hi - lo, [&](float x, int i) {
+    best = better(best, ArgMax{x, lo + i});
+    if (x > -INFINITY) neg_low = fmaxf(neg_low, -x);
+  });
+  best = block_argmax(best, ascratch);
+  neg_low = block_max(neg_low, fscratch);
+  if (threadIdx.x == 0) {
+    part_best[rowi * SP_CHUNKS + chunk] = best;
+    part_low[rowi * SP_CHUNKS + chunk] = -neg_low;
+  }
+}
+
 // ---- 2: count and mass of every bin, chunk by chunk
 __global__ __launch_bounds__(SP_THREADS) void sp_histogram_kernel(
-    const float* __restrict__ logits, int vocab, Stretches stretches, const float* __restrict__ temperature,
-    const int32_t* __restrict__ top_k, const ArgMax* __restrict__ part_best, const float* __restrict__ part_low,
-    uint32_t* __restrict__ hist_count,
-    sp_mass_t* __restrict__ hist_mass) {
+    const float* __restrict__ logits, int vocab, const float* __restrict__ temperature,
+    const ArgMax* __restrict__ part_best, const float* __restrict__ part_low,
+    uint32_t* __restrict__ hist_count, sp_mass_t* __restrict__ hist_mass) {
   __shared__ uint32_t count[SP_BINS];
   __shared__ sp_mass_t mass[SP_BINS];
   const int rowi = blockIdx.x, chunk = blockIdx.y;
-  if (sp_settles(temperature[rowi], top_k[rowi], stretches)) return;
-  const float inv_t = 1.f / temperature[rowi];
-  const size_t slot0 = static_cast<size_t>(rowi) * stretches.slots;
-  const SampleExtent ext = sp_extent(part_best + slot0, part_low + slot0, stretches.slots, inv_t);
+  const float temp = temperature[rowi];
+  if (temp <= 0.f) return;
+  const float inv_t = 1.f / temp;
+  const SampleExtent ext = sp_extent(part_best + rowi * SP_CHUNKS, part_low + rowi * SP_CHUNKS, inv_t);
   for (int b = threadIdx.x; b < SP_BINS; b += blockDim.x) {
     count[b] = 0u;
     mass[b] = 0ull;
@@ -1100,44 +1088,36 @@ __device__ sp_mass_t sp_block_scan(sp_mass_t v, sp_mass_t* scratch) {
   return v + before;
 }
 
-// ---- 3: which bins hold the thresholds; one workgroup a row, one thread a bin (rows that need no
-// bins are settled here)
+// ---- 3: which bins hold the thresholds; one workgroup a row, one thread a bin
 __global__ __launch_bounds__(SP_BINS) void sp_plan_kernel(
-    const float* __restrict__ logits, int vocab, Stretches stretches, const float* __restrict__ temperature,
-    const int32_t* __restrict__ top_k, const float* __restrict__ top_p, const int32_t* __restrict__ seeds,
-    const int32_t* __restrict__ draws, const ArgMax* __restrict__ part_best, const float* __restrict__ part_low, const uint32_t* __restrict__ hist_count,
-    const sp_mass_t* __restrict__ hist_mass, const uint32_t* __restrict__ top_key, const int32_t* __restrict__ top_idx,
-    const int32_t* __restrict__ top_count, SamplePlan* __restrict__ plans, int32_t* __restrict__ out) {
-  __shared__ SettleShared settle_shared;
+    int vocab, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+    const float* __restrict__ top_p, const ArgMax* __restrict__ part_best,
+    const float* __restrict__ part_low, const uint32_t* __restrict__ hist_count,
+    const sp_mass_t* __restrict__ hist_mass, SamplePlan* __restrict__ plans) {
   __shared__ sp_mass_t scan_scratch[17];
   __shared__ float fscratch[17];
   __shared__ sp_mass_t picked[3];
   const int rowi = blockIdx.x, b = threadIdx.x;
-  const float temp = temperature[rowi], p_lim = top_p[rowi];
-  const int k = top_k[rowi];
-  if (sp_settles(temp, k, stretches)) {
-    const Settled s =
-        sp_settle(logits + static_cast<size_t>(rowi) * vocab, rowi, vocab, stretches, temp, k, p_lim, seeds[rowi], draws[rowi], part_best,
-                  top_key, top_idx, top_count, settle_shared);
-    if (b == 0) {
-      plans[rowi].path = s.path;
-      if (s.path != SP_WHOLE_ROW) out[rowi] = s.token;
-    }
-    return;
-  }
+  const float temp = temperature[rowi];
   SamplePlan plan;
+  plan.path = SP_GREEDY;
   plan.k_active = plan.p_active = 0;
   plan.bin_lo = plan.bin_hi = plan.n_cand = 0;
   plan.p_key = 0u;
   plan.z = 1.f;
   plan.mass_before = plan.mass_total = 0ull;
   for (int c = 0; c < SP_CHUNKS; ++c) plan.chunk_at[c] = 0;
-  plan.inv_t = 1.f / temp;
-  const size_t slot0 = static_cast<size_t>(rowi) * stretches.slots;
-  const SampleExtent ext = sp_extent(part_best + slot0, part_low + slot0, stretches.slots, plan.inv_t);
+  plan.inv_t = temp <= 0.f ? 1.f : 1.f / temp;  // (a temperature that is no number stays one)
+  const SampleExtent ext = sp_extent(part_best + rowi * SP_CHUNKS, part_low + rowi * SP_CHUNKS, plan.inv_t);
   plan.best_i = ext.best.i;
   plan.best_v = ext.best.v;
   plan.bin_scale = ext.bin_scale;
+  if (temp <= 0.f) {
+    if (b == 0) plans[rowi] = plan;
+    return;
+  }
+  const int k = top_k[rowi];
+  const float p_lim = top_p[rowi];
   plan.k_active = k > 0 && k < vocab;
   plan.p_active = p_lim < 1.f;
 
@@ -1421,9 +1401,9 @@ static SampleWorkspace sample_workspace(void* base, size_t n_rows, int vocab) {
   w.hist_mass = reinterpret_cast<sp_mass_t*>(take(n_rows * SP_CHUNKS * SP_BINS * sizeof(sp_mass_t)));
   w.plans = reinterpret_cast<SamplePlan*>(take(n_rows * sizeof(SamplePlan)));
   w.hist_count = reinterpret_cast<uint32_t*>(take(n_rows * SP_CHUNKS * SP_BINS * sizeof(uint32_t)));
-  w.part_best = reinterpret_cast<ArgMax*>(take(n_rows * stretches.slots * sizeof(ArgMax)));
+  w.part_best = reinterpret_cast<ArgMax*>(take(std::max(parts, n_rows * SP_CHUNKS) * sizeof(ArgMax)));
   w.race_part = reinterpret_cast<ArgMax*>(take(n_rows * SP_CHUNKS * sizeof(ArgMax)));
-  w.part_low = reinterpret_cast<float*>(take(n_rows * stretches.slots * sizeof(float)));
+  w.part_low = reinterpret_cast<float*>(take(n_rows * SP_CHUNKS * sizeof(float)));
   w.cand_key = reinterpret_cast<uint32_t*>(take(n_rows * CAND_MAX * sizeof(uint32_t)));
   w.cand_e = reinterpret_cast<float*>(take(n_rows * CAND_MAX * sizeof(float)));
   w.cand_idx = reinterpret_cast<int32_t*>(take(n_rows * CAND_MAX * sizeof(int32_t)));
@@ -1464,20 +1444,22 @@ extern "C" int yk_sample(const float* logits, int32_t* out, int n_rows, int voca
   }
   YK_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 256 == 0, "sample: the workspace must be 256-byte aligned");
   const SampleWorkspace w = sample_workspace(workspace, static_cast<size_t>(n_rows), vocab);
-  sp_extent_kernel<<<dim3(n_rows, stretches.n), SP_THREADS, 0, stream>>>(logits, vocab, stretches, temperature, top_k, w.part_best,
-                                                                         w.part_low, w.top_key, w.top_idx, w.top_count);
-  if (yk_check_launch("sample: extent")) return -1;
   if (most_top_k > 0 && most_top_k <= stretches.most_top_k) {
+    sp_top_kernel<<<dim3(n_rows, stretches.n), SP_THREADS, 0, stream>>>(logits, vocab, stretches, temperature, top_k, w.part_best,
+                                                                        w.top_key, w.top_idx, w.top_count);
+    if (yk_check_launch("sample: top")) return -1;
     sp_settle_kernel<<<n_rows, SP_SETTLE_THREADS, 0, stream>>>(logits, out, vocab, stretches, temperature, top_k, top_p, seeds, draws,
                                                                w.part_best, w.top_key, w.top_idx, w.top_count, paths_out);
     return yk_check_launch("sample: settle");
   }
   const dim3 chunks(n_rows, SP_CHUNKS);
-  sp_histogram_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, stretches, temperature, top_k, w.part_best, w.part_low,
+  sp_extent_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, w.part_best, w.part_low);
+  if (yk_check_launch("sample: extent")) return -1;
+  sp_histogram_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, temperature, w.part_best, w.part_low,
                                                          w.hist_count, w.hist_mass);
   if (yk_check_launch("sample: histogram")) return -1;
-  sp_plan_kernel<<<n_rows, SP_BINS, 0, stream>>>(logits, vocab, stretches, temperature, top_k, top_p, seeds, draws, w.part_best, w.part_low,
-                                                 w.hist_count, w.hist_mass, w.top_key, w.top_idx, w.top_count, w.plans, out);
+  sp_plan_kernel<<<n_rows, SP_BINS, 0, stream>>>(vocab, temperature, top_k, top_p, w.part_best, w.part_low,
+                                                 w.hist_count, w.hist_mass, w.plans);
   if (yk_check_launch("sample: plan")) return -1;
   sp_collect_kernel<<<chunks, SP_THREADS, 0, stream>>>(logits, vocab, w.plans, w.cand_key, w.cand_e, w.cand_idx);
   if (yk_check_launch("sample: collect")) return -1;
