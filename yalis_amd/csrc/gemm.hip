@@ -190,12 +190,20 @@ struct AttnSplits {
   const int32_t* token_col;
   int n_splits, n_heads, n_kv, head_dim, hpt, chunks;
 };
+// Where the workgroups of a few-row product start in their slices of K (gemm_mfma_skinny_kernel says why): all at the same place,
+// workgroup b at unit b, or at 5 b + b / 8.  Told by the host, so that the first loads do not wait for the decision.
+enum SkinnyStarts { SK_START_SAME = 0, SK_START_TURNS = 1, SK_START_SPREAD = 2 };
+static int skinny_starts(int mt, int ldw, int k_block, int splits) {
+  if (mt >= 4 || ldw % 2048) return SK_START_SAME;
+  const int units = (k_block + SK_KC - 1) / SK_KC;  // of every slice but the last
+  return units % 2 || (units == 4 && splits == 4) ? SK_START_TURNS : SK_START_SPREAD;
+}
 constexpr int SK_SPLITS_MAX_K_BLOCK = 1024;  // a workgroup's whole slice of x then fits beside the weights
 
 template <int MT, int W, typename TO, int GATED, bool FROM_SPLITS, int KC, int DEPTH = 1>
 __global__ __launch_bounds__(W * 64) void gemm_mfma_skinny_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, float* __restrict__ part,
-    TO* __restrict__ y, int M, int N, int K, int ldx, int ldw, int ldy, int k_block, AttnSplits xa, int xg_rows = 0,
+    TO* __restrict__ y, int M, int N, int K, int ldx, int ldw, int ldy, int k_block, int starts, AttnSplits xa, int xg_rows = 0,
     size_t xg_stride = 0) {
   static_assert(!FROM_SPLITS || (MT == 1 && GATED == 0), "unmerged attention feeds plain products of up to 16 rows");
   extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
@@ -276,10 +284,8 @@ __global__ __launch_bounds__(W * 64) void gemm_mfma_skinny_kernel(
   constexpr int PER_UNIT = SK_KC / KC;              // chunks in a unit of 256
   const int n_units = (kb1 - kb0 + SK_KC - 1) / SK_KC;
   const int slots = PER_UNIT * n_units;             // the last one may lie beyond the slice
-  const int block_units = (k_block + SK_KC - 1) / SK_KC;  // (of every slice but the last)
-  const bool spread = block_units % 2 == 0 && !(block_units == 4 && gridDim.z == 4);
-  const unsigned start = spread ? 5 * blockIdx.x + blockIdx.x / 8 : blockIdx.x;
-  const int first_slot = MT < 4 && ldw % 2048 == 0 ? static_cast<int>(start % n_units) * PER_UNIT : 0;
+  const unsigned start = starts == SK_START_SPREAD ? 5 * blockIdx.x + blockIdx.x / 8 : blockIdx.x;
+  const int first_slot = starts != SK_START_SAME ? static_cast<int>(start % n_units) * PER_UNIT : 0;
   const bool last_missing = slots > n_chunks;
   const int missing_at = slots - 1 - first_slot;    // where the last slot comes in this workgroup's order
   auto chunk_start = [&](int i) {
@@ -715,7 +721,8 @@ static int launch_skinny(const bf16_t* x, const bf16_t* w, float* part, TO* y, i
         return yk_fail("gemm_mfma_skinny: cannot raise the LDS limit");
       raised = true;
     }
-    gemm_mfma_skinny_kernel<1, 4, TO, 0, true, SK_KC><<<grid, dim3(256), lds, stream>>>(nullptr, w, part, y, M, N, K, 0, ldw, ldy, k_block, *from_splits);
+    gemm_mfma_skinny_kernel<1, 4, TO, 0, true, SK_KC><<<grid, dim3(256), lds, stream>>>(nullptr, w, part, y, M, N, K, 0, ldw, ldy, k_block,
+                                                                                   skinny_starts(mt, ldw, k_block, splits), *from_splits);
     return yk_check_launch("gemm_mfma_skinny (from attention splits)");
   }
   dim3 grid((N + 16 * waves - 1) / (16 * waves), (M + 16 * mt - 1) / (16 * mt), splits);
@@ -783,7 +790,8 @@ static int launch_skinny(const bf16_t* x, const bf16_t* w, float* part, TO* y, i
         return yk_fail("gemm_mfma_skinny: cannot raise the LDS limit");                                 \
       raised = true;                                                                                    \
     }                                                                                                   \
-    gemm_mfma_skinny_kernel<MT_, W_, TO, G_, false, KC_, D_><<<grid, block, lds, stream>>>(x, w, part, y, M, N, K, ldx, ldw, ldy, k_block, AttnSplits{}, xg_rows, xg_stride); \
+    gemm_mfma_skinny_kernel<MT_, W_, TO, G_, false, KC_, D_><<<grid, block, lds, stream>>>(x, w, part, y, M, N, K, ldx, ldw, ldy, k_block, \
+                                                                                          skinny_starts(mt, ldw, k_block, splits), AttnSplits{}, xg_rows, xg_stride); \
     return yk_check_launch("gemm_mfma_skinny");                                                         \
   }
   SK_GO_KC(4, 8, 0, 128, 2)
