@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void gemm_f32_dot_kernel(const TX* __restrict_
   };
   int k0 = 0;
   // What is left of a row is asked for by four and two pieces at once too, or a wave waits for each (2 rows, bfloat16 x,
-  // N 4,096, K 1,536 8.4 -> 6.7 us, 4 rows, N 2,048 9.2 -> 5.4); and with three rows (float32 weights) and four, whose sums
+  // N 4,096, K 1,536 8.4 -> 6.7 us, 4 rows, N 2,048 9.2 -> 5.4; two float32 rows are faster than tiles without that); and with three rows (float32 weights) and four, whose sums
   // take long enough, x beside the weight (4 rows, bfloat16 x, 4,096 x 4,096 18.1 -> 15.1; with fewer that only costs registers).
   constexpr bool X_AHEAD = MR == 4 || (MR == 3 && sizeof(TW) == 4);
   auto pieces = [&](auto count) {
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256) void gemm_f32_dot_kernel(const TX* __restrict_
       }
     }
   }
-  if constexpr (MR > 1) {
+  if constexpr (MR > 2 || (MR == 2 && sizeof(TX) + sizeof(TW) < 8)) {
     if (AHEAD > 4 && k0 + 1024 <= K) pieces(std::integral_constant<int, 4>());
     if (k0 + 512 <= K) pieces(std::integral_constant<int, 2>());
   }
