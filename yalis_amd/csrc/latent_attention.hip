@@ -341,7 +341,8 @@ extern "C" int yk_head_linear(const void* x, int x_stride, int x_dtype, const vo
 //   512 -> 128 from float32  100 tokens 15.8 / 13.1 / 16.3 / 15.1  512 20.3 / 14.1 / 17.9 / 26.3  2,048 47.1 / 46.6 / 33.8 / 28.3
 // (2,048 tokens: 83 MB, 17 us at what a copy reaches.  Twice the columns a wave: 30.1 and 27.7.)
 // With a turned tail of 64 behind each head, which the head's workgroups share, 128 -> 512 (us, one tile / several, the tail
-// left to the first workgroup / several, shared): 512 tokens 17.9 / 22.7 / 10.4, 1,000 27.7 / 30.2 / 16.6, 2,048 45.9 / 35.6 / 28.2.
+// left to the first workgroup / several, shared): 512 tokens 17.9 / 22.7 / 10.4, 1,000 27.7 / 30.2 / 16.6, 2,048 45.9 / 35.6 / 28.2
+// (within a prompt, its inputs from memory, 46.8 -> 39.7).
 typedef __bf16 hl_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float hl_f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t hl_u32x4_t __attribute__((ext_vector_type(4)));
