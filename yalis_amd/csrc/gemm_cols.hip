@@ -41,8 +41,8 @@ struct Finish {
 // no other wave of the workgroup wants the same piece.  Rows beyond N are read from the last row and
 // never stored, K beyond the end is read from valid places and meets zeros of x.  Workgroups start at
 // different chunks, so that they do not ask for addresses a whole number of rows apart at every moment,
-// and those of one die (every eighth) at different ones too: 4,096 x 4,096 11.1 -> 8.3 us against starting
-// at the workgroup's number, 8,192 x 4,096 19.2 -> 15.5, 4,672 x 2,048 8.9 -> 8.4.
+// and those of one die (every eighth) at different ones too: against starting at the workgroup's number, when
+// this was chosen, 4,096 x 4,096 11.1 -> 8.3 us, 8,192 x 4,096 19.2 -> 15.5, 4,672 x 2,048 8.9 -> 8.4.
 // gated: the 16 rows are eight gate rows, then the eight up rows that belong to them.
 // A wave's products join two running sums by turns: every addition rounds the sum it joins, and from a K of about
 // 5,000 on one sum a wave met more of them than the slices of the other form do.  Distance from 64 bits in parts of
