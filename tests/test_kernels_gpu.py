@@ -450,6 +450,87 @@ def test_gemm_mfma_skinny_wide_form(ops, forced, chunk, waves):
         ops.wide_skinny_products(1)
 
 
+def _held(rows, cols, ld, seed):
+    """Small whole numbers in bfloat16 rows ``ld`` apart, NaN in the gaps and behind the last row: products are exact, and a read too far shows."""
+    g = torch.Generator().manual_seed(seed)
+    buf = torch.full((rows + 3, ld), float("nan"), dtype=torch.bfloat16)
+    buf[:rows, :cols] = torch.randint(-4, 5, (rows, cols), generator=g).to(torch.bfloat16)
+    return buf.to(DEV)[:rows, :cols]
+
+
+@pytest.mark.parametrize("form,least_k,sub", [(0, 192, 64), (1, 192, 64), (2, 256, 64), (3, 384, 128), (4, 256, 64)])
+def test_gemm_block_forms(ops, form, least_k, sub):
+    """Every form of the product in large tiles, bit for bit (sums of small whole numbers are exact in float32): tiles that hang over on
+    either side, more tiles than a grid has workgroups, the shortest K, K cut into slices of which the last is shorter, rows with gaps."""
+    from yalis_amd.ops.hip import KernelError, SplitSum
+
+    for m, n, k in [(1, 8, least_k), (65, 200, least_k + sub), (255, 264, 2 * least_k), (300, 1032, 3 * least_k + sub), (129, 24, 1024), (700, 40008, least_k)]:
+        x, w = _held(m, k, k + 8, 1), _held(n, k, k + 64, 2)
+        want = x.float().cpu() @ w.float().cpu().T
+        for slices in (1, 2, 3):
+            per = -(-(k // sub) // slices)
+            if k // sub - (slices - 1) * per <= least_k // sub - 1:
+                with pytest.raises(KernelError, match="too short"):
+                    ops.gemm_block(x, w, torch.bfloat16, form * 256 + slices)
+                continue
+            if slices == 1:
+                assert torch.equal(ops.gemm_block(x, w, torch.float32, form * 256 + 1).cpu(), want), (m, n, k)
+                assert torch.equal(ops.gemm_block(x, w, torch.bfloat16, form * 256 + 1).cpu(), want.to(torch.bfloat16)), (m, n, k)
+            else:
+                y = ops.gemm_block(x, w, torch.bfloat16, form * 256 + slices)
+                assert isinstance(y, SplitSum) and y.n_splits == slices and y.out_dtype == torch.bfloat16
+                assert torch.equal(y.tensor.sum(0).cpu(), want), (m, n, k, slices)
+    with pytest.raises(KernelError, match="too short"):
+        ops.gemm_block(_held(65, 64, 64, 1), _held(64, 64, 64, 2), torch.bfloat16, form * 256 + 1)
+
+
+@pytest.mark.parametrize("form", [0, 2, 3, 4])
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh", ("clamped_swish", 7.0, 1.702)])
+def test_gemm_block_gated(ops, form, activation):
+    """Gated pairs in the product's end: the pairs of its own rounded product (one unit of bfloat16 apart at most, where the float32 values
+    of the two activations straddle a rounding), gates of every sign and size, infinities and NaN as they come."""
+    for m, n, k in [(1, 16, 512), (130, 528, 512), (300, 1040, 640)]:
+        x, w = rnd((m, k), torch.bfloat16, 3), rnd((n, k), torch.bfloat16, 4, 0.3)
+        x[0, 0], x[m // 2, 3] = float("inf"), float("nan")
+        if m > 1:
+            x[m - 1] *= 1000.0
+        gu = ops.gemm_block(x, w, torch.bfloat16, form * 256 + 1)
+        want = ops.gated_act(gu, activation, torch.bfloat16, group=8).float()
+        got = ops.gemm_block(x, w, torch.bfloat16, form * 256 + 1, gated=activation).float()
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        both_inf = torch.isinf(want) & (got == want)
+        off = (got - want).abs()[~(torch.isnan(want) | both_inf)]
+        assert bool((off <= 2**-7 * want.abs()[~(torch.isnan(want) | both_inf)] + 1e-37).all())
+
+
+def test_gemm_block_is_what_linear_takes(ops):
+    """Where ``linear`` and ``gate_up_act`` take the product in large tiles by themselves, and that they agree with the kernels for other sizes."""
+    from yalis_amd.ops.hip import SplitSum
+
+    x, w = rnd((999, 1024), torch.bfloat16, 5), rnd((3072, 1024), torch.bfloat16, 6, 0.05)
+    want = x.double().cpu() @ w.double().cpu().T
+    assert ops._block_plan(x, w, False) >= 0
+    close(ops.linear(x, w, torch.bfloat16), want, 2e-2, 2**-7)
+    close(ops.linear(x, w, torch.float32), want, 2e-5 * 32, 1e-5)
+    bias = rnd((3072,), torch.bfloat16, 7)
+    close(ops.linear(x, w, torch.bfloat16, bias=bias), want + bias.double().cpu(), 2e-2, 2**-7)
+    xl, wl = rnd((300, 4096), torch.bfloat16, 8), rnd((1024, 4096), torch.bfloat16, 9, 0.05)
+    y = ops.linear(xl, wl, torch.bfloat16, partial_ok=True)
+    assert isinstance(y, SplitSum)
+    close(y.reduce(), xl.double().cpu() @ wl.double().cpu().T, 2e-2, 2**-7)
+    packed, group = ops.pack_gate_up(rnd((2048, 1024), torch.bfloat16, 10, 0.05), rnd((2048, 1024), torch.bfloat16, 11, 0.05))
+    assert ops._block_plan(x, packed, False, gated=True) >= 0
+    got = ops.gate_up_act(x, packed, group, "silu", torch.bfloat16)
+    ops.force_block_plan(-2)
+    try:
+        assert ops._block_plan(x, packed, False, gated=True) < 0
+        close(got, ops.gate_up_act(x, packed, group, "silu", torch.bfloat16).double().cpu(), 2e-2, 2**-6)
+    finally:
+        ops.force_block_plan()
+    for m, n, k in [(64, 3072, 1024), (999, 3072, 1000), (999, 3073, 1024), (999, 3072, 64)]:  # too few rows, K no multiple of 64, odd columns, K too short
+        assert ops._block_plan(torch.empty(m, k, device=DEV), torch.empty(n, k, device=DEV), True) < 0
+
+
 def test_gemm_tile(ops):
     """The product in tiles of 128 x 128 for some dozens to a few hundred rows: sizes that are no
     multiples of the tile or of the step of 64 along K, one-hot operands, K cut into 1 to 8 slices

@@ -1,0 +1,392 @@
+// Products of many rows: y = x . w^T, bfloat16 operands, float32 accumulation, in large tiles; K cut into slices where tiles are few, and
+// gate/up products with their activation in the end.  The reference leaves these to its vendor library (yalis/external/model.py:449, 462-466,
+// 717-722); so does this engine where the library is faster (plan()).
+//
+// What bounds it.  With every compute unit at work the card's power: the clock falls to 1.4 to 1.9 GHz, so what counts is what a product
+// costs beside the matrix instructions.  v_mfma_f32_16x16x32_bf16 reads and writes fewer registers for the same products than 32x32x16 (8,192 x
+// 28,672 x 4,096: 1,325 us where 32x32x16 takes 1,450), tiles of 256 x 256 fetch least, and workgroups of one die take tiles that share rows
+// (L2 answers 4 of 5 reads).  Dies that start at different places of K spread their reads over the memory channels (1,325 -> 1,286).
+// Loads go to LDS without registers between (a form with them, 128 x 128, ended at 0.4 to 0.77 PFLOP/s: 1,024 clocks of writes a
+// step), and stand one by one between the matrix instructions: all at once behind the barrier the same product takes 5 to 7 % longer.
+// One operand has a step more under way than the other, which is what LDS holds (2,048 x 6,144 x 4,096 as 192 x 256: 87 -> 77 us).
+// With few tiles the memory's latency: slices along K put more under way.
+// Measured in replayed graphs, weights from memory, with the norm that follows where slices are handed on (us, the library and the
+// kernels for fewer rows before / this): 999 x 3,072 x 2,048 21.4 / 17.8, 797 x 4,096 x 4,096 39 / 33, 2,048 x 2,048 x 2,048 22 / 19, 2,048 x 1,360 x 2,048
+// 20 / 16; slices: 150 x 3,072 x 8,192 29 / 23, 512 x 2,048 x 8,192 39 / 32, 999 x 4,096 x 14,336 151 / 114; gate/up with its activation: 256 x 16,384 x 3,072 45 /
+// 35, 999 x 16,384 x 2,048 67 / 58, 3,985 x 16,384 x 3,072 321 / 299, 8,192 x 28,672 x 4,096 1,374 / 1,313.  Over 1,084 products of 66 to 6,000 rows
+// the 276 that changed kernel take 1.14 times less.
+#include <algorithm>
+
+#include "common.h"
+
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// Lane i's 16 bytes at `at` + `lane_off` + `off` (nothing beyond `bytes`) to place i of the KiB of LDS at `to`.
+__device__ __forceinline__ void load_to_lds(const void* at, int bytes, void* to, int lane_off, int off) {
+#ifdef __HIP_DEVICE_COMPILE__  // the builtin takes 16 bytes for the device alone
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(at), 0, bytes, 0x00027000), (lds_void_t*)to, 16,
+                                           lane_off, off, 0, 0);
+#endif
+}
+
+// Until no more than VM loads and stores and LGKM LDS reads of this wave are under way (the builtin: the compiler then adds no waits of its
+// own for those reads).
+template <int VM, int LGKM>
+__device__ __forceinline__ void wait_for() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 7 << 4 | LGKM << 8);
+}
+
+enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GATED = 2 };
+
+// x * sigmoid(slope * x), within two units of float32's last place: exp(y) as 2^(y log2 e) with the product's rounding carried along.
+__device__ __forceinline__ float swish(float x, float slope) {
+  const float y = fminf(fmaxf(-slope * x, -90.f), 90.f), t = y * 1.44269504f;
+  const float low = fmaf(y, 1.92596303e-8f, fmaf(y, 1.44269504f, -t));
+  const float e = __builtin_amdgcn_exp2f(t);
+  return x * __builtin_amdgcn_rcpf(1.f + fmaf(e, low * 0.693147181f, e));
+}
+__device__ __forceinline__ float gated(float g, float u, int kind, float p0, float p1) {
+  if (kind == 0) return swish(g, 1.f) * u;
+  if (kind == 1) return gated_pair(g, u, 1, p0, p1);
+  return swish(fminf(g, p0), p1) * (fminf(fmaxf(u, -p0), p0) + 1.f);
+}
+
+// A workgroup of WN x WM waves makes BN columns (rows of w) x BM rows of y over `per` steps of 64 along K.
+//
+// LDS: a step's rows of w, then of x, 128 bytes each, STAGES steps in flight.  buffer_load ... lds writes lane i's 16 bytes to
+// place i of a KiB, so what is swapped is the address each lane reads from: piece c of row p lies at place c ^ (p / 2 % 8), with which
+// the operand reads (16 rows x 64 bytes a wave) meet every bank once.  Row p of w's part holds row 32 (p / 32) + 8 (p / 4 % 4) +
+// 4 (p / 16 % 2) + p % 4 of the tile: two products of 16 x 16 then leave eight consecutive columns of a row in a lane.
+template <int BN, int BM, int WN, int WM, int SUB, int AHEAD, bool X_FIRST, int OUT>
+__global__ __launch_bounds__(64 * WN * WM, 1) void gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                     void* __restrict__ yv, int M, int N, int K, int ldx, int ldw, int ldy,
+                                                                     int slices, int kind, float p0, float p1) {
+  constexpr int NW = WN * WM, BK = 64 * SUB, FN = BN / WN / 16, FM = BM / WM / 16, WS = BN * 128, XS = BM * 128, WB = WS * SUB, XB = XS * SUB;
+  constexpr int LW = BN / 8 / NW, LX = BM / 8 / NW, L = LW + LX, Q = FN * FM, R = FN + FM;
+  // of one operand AHEAD steps lie in LDS, of the other, which is loaded half a step later, one more
+  constexpr int SW = AHEAD + X_FIRST, SX = AHEAD + !X_FIRST, LF = X_FIRST ? LX : LW, LT = X_FIRST ? LW : LX;
+  static_assert(BN % (8 * NW) == 0 && BM % (8 * NW) == 0 && (NW == 4 || NW == 8) && FN % 2 == 0 && (OUT != OUT_GATED || FN % 4 == 0), "tiles");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[SW * WB + SX * XB];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  // The dies take turns with workgroups; each die gets a run of tiles, which its workgroups walk side by side; eight tiles of rows to a
+  // band of tiles.
+  const int tn = (N + BN - 1) / BN, tm = (M + BM - 1) / BM, flat = tn * tm, total = flat * slices, die = blockIdx.x % 8;
+  const int mine = total / 8 + (die < total % 8), run0 = die * (total / 8) + min(die, total % 8);
+  const int all = K / BK, per = (all + slices - 1) / slices;
+  struct Tile {
+    int m0, n0, slice, steps;
+  };
+  auto tile_of = [&](int at) {
+    int t = run0 + at;
+    const int slice = t / flat;
+    t -= slice * flat;
+    constexpr int BAND = 8;
+    const int first = t / (BAND * tn) * BAND, high = min(BAND, tm - first), r = t - first * tn;
+    return Tile{(first + r % high) * BM, r / high * BN, slice, min(per, all - slice * per)};
+  };
+  // a tile's rows of an operand: where they begin and how many bytes they reach over, behind which nothing is read (rows beyond N or M)
+  struct Rows {
+    const bf16_t* at;
+    int bytes;
+  };
+  auto w_of = [&](const Tile& t) {
+    return Rows{w + static_cast<size_t>(t.n0) * ldw + t.slice * per * BK, ((min(BN, N - t.n0) - 1) * ldw + t.steps * BK) * 2};
+  };
+  auto x_of = [&](const Tile& t) {
+    return Rows{x + static_cast<size_t>(t.m0) * ldx + t.slice * per * BK, ((min(BM, M - t.m0) - 1) * ldx + t.steps * BK) * 2};
+  };
+  const int piece = 8 * ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4)));
+  const int wrow = 32 * (wave / 4) + 8 * (2 * (wave & 1) + (lane >> 5)) + 4 * (wave / 2 % 2) + ((lane >> 3) & 3);
+  const int wvo = (wrow * ldw + piece) * 2, xvo = ((8 * wave + (lane >> 3)) * ldx + piece) * 2;
+  const int wstep = 8 * NW * ldw * 2, xstep = 8 * NW * ldx * 2;
+  // What is loaded runs AHEAD steps before what is multiplied, into the workgroup's next tile, and past its last one into nothing (a
+  // buffer of no bytes): every tile has more steps than that.  Every die starts at a place of its own along K.
+  const int stride = gridDim.x / 8 + (die < static_cast<int>(gridDim.x % 8));
+  int at_tile = blockIdx.x / 8;
+  if (at_tile >= mine) return;
+  Tile t = tile_of(at_tile);
+  Rows wr = w_of(t), xr = x_of(t);
+  constexpr int STEP = BK * 2;
+  int wk = die * t.steps / 8 * STEP, xk = wk, around = t.steps * STEP;
+  auto load_w = [&](int buf, int sub, int l) {
+    load_to_lds(wr.at, wr.bytes, lds + buf + sub * WS + (l * NW + wave) * 1024, wvo, l * wstep + sub * 128 + wk);
+  };
+  auto load_x = [&](int buf, int sub, int l) {
+    load_to_lds(xr.at, xr.bytes, lds + SW * WB + buf + sub * XS + (l * NW + wave) * 1024, xvo, l * xstep + sub * 128 + xk);
+  };
+  auto onward = [&](int& k) { k = k + STEP == around ? 0 : k + STEP; };
+  const int wn = wave % WN, wm = wave / WN, row = lane % 16, quarter = lane / 16;
+  const int at = row * 128 + ((quarter ^ (row >> 1)) * 16);
+  const unsigned char* const wl = lds + wn * FN * 2048;
+  const unsigned char* const xl = lds + SW * WB + wm * FM * 2048;
+  f32x4_t acc[FN][FM] = {};
+  bf16x8_t a[2][FN], b[2][FM];
+  auto read_one = [&](int wat, int xat, int sub, int to, int f) {
+    if (f < FN)
+      a[to][f] = *reinterpret_cast<const bf16x8_t*>(wl + sub * WS + f * 2048 + wat);
+    else
+      b[to][f - FN] = *reinterpret_cast<const bf16x8_t*>(xl + sub * XS + (f - FN) * 2048 + xat);
+  };
+  // 32 along K: the products from operands p % 2, and spread evenly between them the reads of the next 32's operands, loads, and what
+  // `beside` says (one wave a SIMD issues an instruction every four clocks, a product takes sixteen: what stands together leaves the
+  // matrix cores idle)
+  auto part = [&](int p, int wat, int xat, int to, auto beside) {
+    const int use = p % 2, sub = (p + 1) / 2 % SUB, n = p == 2 * SUB - 1 ? LF * SUB : LT * SUB, parts = p == 2 * SUB - 1 ? 1 : 2 * SUB - 1, c = p == 2 * SUB - 1 ? 0 : p;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int i = q / FM, j = i % 2 ? FM - 1 - q % FM : q % FM;  // neighbours share an operand
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[use][i], b[use][j], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int f = (q * R + Q - 1) / Q; f < ((q + 1) * R + Q - 1) / Q; ++f) read_one(wat, xat, sub, use ^ 1, f);
+#pragma unroll
+      for (int l = (c * Q + q) * n / (parts * Q); l < (c * Q + q + 1) * n / (parts * Q); ++l) {
+        if ((p == 2 * SUB - 1) == X_FIRST)
+          load_x(to, l / LX, l % LX);
+        else
+          load_w(to, l / LW, l % LW);
+      }
+      beside(q);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto meet = [] {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) {
+#pragma unroll
+    for (int sub = 0; sub < SUB; ++sub) {
+#pragma unroll
+      for (int l = 0; l < LX; ++l) load_x(s * XB, sub, l);
+#pragma unroll
+      for (int l = 0; l < LW; ++l) load_w(s * WB, sub, l);
+    }
+    onward(wk);
+    onward(xk);
+  }
+  wait_for<(AHEAD - 1) * L * SUB, 15>();
+  meet();
+#pragma unroll
+  for (int f = 0; f < R; ++f) read_one(at, at, 0, 0, f);
+  int wcur = 0, xcur = 0;
+  int late = AHEAD * (X_FIRST ? WB : XB);  // the buffer that the last step left of the operand loaded later
+  int wat = at, xat = at;
+  for (;;) {
+    at_tile += stride;
+    const bool more = at_tile < mine;
+    const Tile next = tile_of(more ? at_tile : 0);
+    Rows wnext = w_of(next), xnext = x_of(next);
+    if (!more) wnext.bytes = xnext.bytes = 0;
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+      for (int j = 0; j < FM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    int s = t.steps - AHEAD;
+    for (bool last = false;; last = true) {
+      do {
+        int wnxt = 0, xnxt = 0;
+#pragma unroll
+        for (int p = 0; p < 2 * SUB - 1; ++p)
+          part(p, wat ^ (p % 2 ? 0 : 64), xat ^ (p % 2 ? 0 : 64), late, [&](int q) {
+            if (p == 0 && q == 1) wnxt = wcur + WB == SW * WB ? 0 : wcur + WB;
+            if (p == 0 && q == 2) xnxt = xcur + XB == SX * XB ? 0 : xcur + XB;
+            if (p == 0 && q == 1) asm volatile("" : "+s"(wnxt));
+            if (p == 0 && q == 2) asm volatile("" : "+s"(xnxt));
+          });
+        onward(X_FIRST ? wk : xk);
+        // the next step has landed, and every wave holds the last operands of this one, whose buffers are loaded into from here on
+        wait_for<((AHEAD - 2) * L + LT) * SUB, 0>();
+        meet();
+        wat = wnxt + at;
+        xat = xnxt + at;
+        part(2 * SUB - 1, wat, xat, X_FIRST ? xcur : wcur, [](int) {});
+        onward(X_FIRST ? xk : wk);
+        late = X_FIRST ? wcur : xcur;
+        wcur = wnxt;
+        xcur = xnxt;
+      } while (--s > 0);
+      if (last) break;
+      wr = wnext;
+      xr = xnext;
+      around = next.steps * STEP;
+      wk = xk = die * next.steps / 8 * STEP;
+      s = AHEAD;
+    }
+  // lane l holds columns 8 (l / 16) .. + 3 of 32 in one product's registers and the four after them in the next one's
+  const int m = t.m0 + wm * FM * 16 + row, nw = t.n0 + wn * FN * 16;
+#pragma unroll
+  for (int j = 0; j < FM; ++j) {
+    const int mj = m + 16 * j;
+    if constexpr (OUT == OUT_GATED) {
+      bf16_t* const y = static_cast<bf16_t*>(yv) + static_cast<size_t>(mj) * ldy;
+#pragma unroll
+      for (int i = 0; i < FN; i += 4) {
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          // eight columns of gate lie in even rows of 16 lanes, their eight of up in the odd row after
+          const auto s2 = __builtin_amdgcn_permlane16_swap(__float_as_uint(as_output(acc[i + e / 4][j][e % 4], 1)),
+                                                           __float_as_uint(as_output(acc[i + 2 + e / 4][j][e % 4], 1)), false, false);
+          o[e] = gated(__uint_as_float(s2[0]), __uint_as_float(s2[1]), kind, p0, p1);
+        }
+        const int n = nw + 16 * i + 32 * (quarter & 1) + 16 * (quarter >> 1);  // of the packed matrix
+        if (mj < M && n < N)
+          *reinterpret_cast<u32x4_t*>(y + n / 2) = u32x4_t{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7])};
+      }
+    } else if constexpr (OUT == OUT_BF16) {
+      bf16_t* const y = static_cast<bf16_t*>(yv) + static_cast<size_t>(mj) * ldy;
+#pragma unroll
+      for (int i = 0; i < FN; i += 2) {
+        const int n = nw + 16 * i + 8 * quarter;
+        const f32x4_t u = acc[i][j], v = acc[i + 1][j];
+        if (mj < M && n < N)
+          *reinterpret_cast<u32x4_t*>(y + n) = u32x4_t{pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      }
+    } else {
+      float* const y = static_cast<float*>(yv) + (static_cast<size_t>(t.slice) * M + mj) * ldy;
+#pragma unroll
+      for (int i = 0; i < FN; i += 2) {
+        f32x4_t u, v;  // columns 4 (l / 16) .. + 3 of the 32, and those 16 further: a row's 64 bytes in one store
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const auto s2 = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i][j][e]), __float_as_uint(acc[i + 1][j][e]), false, false);
+          const auto s4 = __builtin_amdgcn_permlane32_swap(s2[0], s2[1], false, false);
+          u[e] = __uint_as_float(s4[0]);
+          v[e] = __uint_as_float(s4[1]);
+        }
+        const int n = nw + 16 * i + 4 * quarter;
+        if (mj < M && n < N) *reinterpret_cast<f32x4_t*>(y + n) = u;
+        if (mj < M && n + 16 < N) *reinterpret_cast<f32x4_t*>(y + n + 16) = v;
+      }
+    }
+  }
+    if (!more) break;
+    t = next;
+  }
+  wait_for<0, 15>();  // no load may still be on its way into LDS
+}
+
+// Columns and rows of a tile, workgroups a compute unit holds, 64s of K a step, steps under way; and what a product takes, in us: `once`, and
+// for every time the compute units are filled `each` and, per 64 of K, `step` (`full` more where every compute unit is at work), and
+// `out` a million bytes written.  Least squares over some 7,000 products timed back to back (72 to 8,192 rows, 512 to 28,672 columns, K 768 to
+// 16,384, one to four slices; 7 to 15 % off on average), only to choose among the forms.
+struct Form {
+  int bn, bm, fit, sub, ahead;
+  float once, each, step, full, out;
+};
+constexpr Form FORMS[] = {{256, 256, 1, 1, 2, 6.9f, 2.4f, 0.97f, 0.21f, 0.15f},
+                          {192, 256, 1, 1, 2, 6.1f, -0.4f, 1.03f, 0.05f, 0.21f},
+                          {256, 128, 1, 1, 3, 7.0f, -1.7f, 0.72f, 0.02f, 0.25f},
+                          {128, 128, 1, 2, 2, 5.7f, -2.4f, 0.45f, 0.01f, 0.38f},
+                          {128, 64, 2, 1, 3, 3.9f, -2.2f, 0.34f, 0.31f, 0.44f}};
+constexpr int N_FORMS = sizeof(FORMS) / sizeof(FORMS[0]);
+constexpr int UNITS = 256;  // compute units
+
+bool fits(const Form& f, int K, int slices) {
+  const int steps = K / (64 * f.sub);
+  return K % (64 * f.sub) == 0 && steps - (slices - 1) * ((steps + slices - 1) / slices) > f.ahead;
+}
+
+// The form and the slices of K for a product (form * 256 + slices), or -1 where the vendor library, or the kernels for fewer rows, do better.
+int plan(int M, int N, int K, bool partial, bool gated) {
+  if (M <= 64 || K % 64 || N % (gated ? 16 : 8)) return -1;
+  int best = -1, best_slices = 1, best_rounds = 1;
+  float least = 1e30f;
+  for (int i = 0; i < N_FORMS; ++i) {
+    const Form& f = FORMS[i];
+    if (gated && i == 1) continue;
+    for (int slices = 1; slices <= (partial ? 4 : 1); slices *= 2) {
+      if (!fits(f, K, slices)) continue;
+      const long long tiles = static_cast<long long>((N + f.bn - 1) / f.bn) * ((M + f.bm - 1) / f.bm) * slices;
+      const int room = UNITS * f.fit, rounds = static_cast<int>((tiles + room - 1) / room);
+      const float steps = static_cast<float>((K / 64 + slices - 1) / slices), fill = static_cast<float>(tiles) / room / rounds;
+      const float megabytes = static_cast<float>(M) * N * (slices > 1 ? 4 * slices : 2) * 1e-6f;
+      // (the consumer of slices reads them all, where it would read bfloat16)
+      const float us = f.once + rounds * (f.each + steps * (f.step + f.full * fill)) + megabytes * f.out +
+                       (slices > 1 ? static_cast<float>(M) * N * (4 * slices - 2) / 4.5e6f : 0.f);
+      if (us < least) least = us, best = i, best_slices = slices, best_rounds = rounds;
+    }
+  }
+  if (best < 0) return -1;
+  const Form& f = FORMS[best];
+  // the part of the compute units' time that goes into y and not into tiles that hang over or units without one
+  const float used = static_cast<float>(M) * N * best_slices / (static_cast<float>(best_rounds) * UNITS * f.fit * f.bn * f.bm);
+  bool ours;
+  if (gated)
+    ours = N >= 2048 && (M <= 128 || used >= (M <= 256 ? 0.6f : M <= 720 ? 0.76f : 0.65f));
+  else if (best_slices > 1)
+    ours = N <= 5120 && M <= 1100 && best != 1 && (K >= 3072 || (M <= 128 ? K <= 1024 : M <= 256 && N <= 2560)) && (N >= 1024 || M <= 512);
+  else
+    ours = (best_rounds == 1 && ((best == 2 && used >= 0.8f) || (best == 3 && used >= 0.7f))) || (N % 128 && N <= 8192 && M > 720);
+  return ours ? best * 256 + best_slices : -1;
+}
+
+template <int OUT>
+int launch(int form, const bf16_t* x, const bf16_t* w, void* y, int M, int N, int K, int ldx, int ldw, int ldy, int slices, int kind, float p0,
+           float p1, hipStream_t stream) {
+  const Form f = FORMS[form];
+  const int total = ((N + f.bn - 1) / f.bn) * ((M + f.bm - 1) / f.bm) * slices;
+  const int room = UNITS * f.fit, rounds = (total + room - 1) / room, grid = std::min(room, ((total + rounds - 1) / rounds + 7) / 8 * 8);
+  switch (form) {
+    case 0:
+      if constexpr (OUT != OUT_GATED)
+        gemm_block_kernel<256, 256, 2, 2, 1, 2, true, OUT><<<grid, 256, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1);
+      else
+        gemm_block_kernel<256, 256, 2, 4, 1, 2, true, OUT><<<grid, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1);
+      break;
+    case 1:
+      if constexpr (OUT != OUT_GATED) gemm_block_kernel<192, 256, 2, 4, 1, 2, true, OUT><<<grid, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1);
+      break;
+    case 2: gemm_block_kernel<256, 128, 2, 4, 1, 3, false, OUT><<<grid, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1); break;
+    case 3: gemm_block_kernel<128, 128, 2, 4, 2, 2, true, OUT><<<grid, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1); break;
+    default: gemm_block_kernel<128, 64, 2, 2, 1, 3, false, OUT><<<grid, 256, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1); break;
+  }
+  return yk_check_launch("gemm_block");
+}
+
+int g_force_block = -1;
+
+}  // namespace
+
+// The form and slices for a product as form * 256 + slices, -1: not this kernel's.  `partial`: slices may be handed on.
+extern "C" int yk_gemm_block_plan(int M, int N, int K, int partial, int gated) {
+  if (g_force_block != -1) return std::max(g_force_block, -1);
+  return plan(M, N, K, partial != 0, gated != 0);
+}
+
+// For tests and measurements: the plan of every product (form * 256 + slices; -1: the rule; -2: nothing is this kernel's).
+extern "C" int yk_gemm_block_force(int plan) {
+  YK_REQUIRE(plan >= -2 && (plan < 0 || (plan / 256 < N_FORMS && plan % 256 >= 1)), "gemm_block_force: form * 256 + slices, or -1");
+  g_force_block = plan;
+  return 0;
+}
+
+// y [M, N] = x [M, K] . w [N, K]^T, bfloat16 operands, in the form and slices of `plan`.  out: 0 bfloat16, 1 float32 (`slices` > 1: the unreduced
+// slices [slices, M, N] one behind the other, ldy = N), 2 gated pairs of groups of eight columns, bfloat16 [M, N / 2] (kind, p0, p1: common.h).
+extern "C" int yk_gemm_block(const void* x, const void* w, void* y, int out, int M, int N, int K, int ldx, int ldw, int ldy, int plan, int kind,
+                             float p0, float p1, hipStream_t stream) {
+  const int form = plan / 256, slices = plan % 256;
+  YK_REQUIRE(M > 0 && N > 0 && K > 0 && K % 64 == 0 && N % 8 == 0, "gemm_block: K is a multiple of 64, N of 8");
+  YK_REQUIRE(out >= 0 && out <= 2 && plan >= 0 && form < N_FORMS, "gemm_block: unknown output or form");
+  YK_REQUIRE(!(out == OUT_GATED && (N % 16 || form == 1)), "gemm_block: gated pairs are groups of eight columns, and form 1 has none");
+  YK_REQUIRE(out != OUT_GATED || (kind >= 0 && kind < YK_GATED_KINDS), "gemm_block: unknown activation");
+  YK_REQUIRE(slices >= 1 && (slices == 1 || (out == OUT_F32 && ldy == N)), "gemm_block: slices are float32, one behind the other");
+  YK_REQUIRE(fits(FORMS[form], K, slices), "gemm_block: a slice of K is too short");
+  YK_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0 && ldx < 1 << 21 && ldw < 1 << 21, "gemm_block: rows of x and w");
+  YK_REQUIRE(ldy >= (out == OUT_GATED ? N / 2 : N) && ldy % 8 == 0, "gemm_block: rows of y");
+  YK_REQUIRE(static_cast<long long>((N + 63) / 64) * ((M + 63) / 64) * slices < 1 << 30, "gemm_block: too many tiles");
+  YK_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0,
+             "gemm_block: operands must be 16-byte aligned");
+  const auto* xb = static_cast<const bf16_t*>(x);
+  const auto* wb = static_cast<const bf16_t*>(w);
+  if (out == OUT_BF16) return launch<OUT_BF16>(form, xb, wb, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1, stream);
+  if (out == OUT_F32) return launch<OUT_F32>(form, xb, wb, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1, stream);
+  return launch<OUT_GATED>(form, xb, wb, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1, stream);
+}

@@ -35,6 +35,9 @@ class StaleWorkspace(KernelError):
     been handed to a later launch."""
 
 
+_OUT_CODES = {torch.bfloat16: 0, torch.float32: 1}  # what gemm_block writes
+
+
 def _code(dtype: torch.dtype) -> int:
     if dtype == torch.float32:
         return _F32
@@ -207,6 +210,12 @@ _SIGNATURES = {
         [_vp, _vp, _vp, _c_int, _vp, _c_size_t, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp],
         _c_int,
     ),
+    "yk_gemm_block": (
+        [_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _vp],
+        _c_int,
+    ),
+    "yk_gemm_block_plan": ([_c_int, _c_int, _c_int, _c_int, _c_int], _c_int),
+    "yk_gemm_block_force": ([_c_int], _c_int),
     "yk_gemm_tile": (
         [_vp, _vp, _vp, _c_int, _vp, _c_size_t, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp],
         _c_int,
@@ -266,7 +275,7 @@ _LATER_SIGNATURES = {
         "yk_probe_mfma_bf16": ([_c_int, _c_int, _vp, _vp], _c_int),
     },
 }
-_ABI = 25
+_ABI = 26
 
 # Rows of x up to which the hand-written matrix-core kernel runs a bfloat16 product;
 # above it the vendor library does.
@@ -470,6 +479,9 @@ class HipOps:
             for n, k in products:
                 if k >= 8 and k % 8 == 0:
                     need = max(need, self._ask("yk_gemm_skinny_splits", rows, n, k, 0) * rows * n)
+        else:
+            for n, k in products:
+                need = max(need, max(self._ask("yk_gemm_block_plan", rows, n, k, 1, 0), 0) % 256 * rows * n)
         self._ws(1 << 24)
         self._gemm_ws(need)
 
@@ -705,8 +717,13 @@ class HipOps:
         bf = torch.bfloat16
         aligned = k % 8 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
         if x.dtype == bf and w.dtype == bf and aligned:
-            if out_dtype == bf and self.long_matrix_tiles(m, n, k):
+            slices_do = partial_ok and out_dtype == bf
+            if out_dtype == bf and self.long_matrix_tiles(m, n, k, slices_do):
                 return self.gemm_tile(x, w, bf, partial_ok)
+            if m > SKINNY_MAX_ROWS and out_dtype in (bf, torch.float32):
+                plan = self._block_plan(x, w, slices_do)
+                if plan >= 0:
+                    return self.gemm_block(x, w, out_dtype, plan)
             if m > SKINNY_MAX_ROWS and out_dtype == bf and not self.few_library_tiles(m, n):
                 return self.gemm_library(x, w, bf)  # vendor library, bfloat16 in and out
             if m > SKINNY_MAX_ROWS and out_dtype == torch.float32:
@@ -719,7 +736,7 @@ class HipOps:
         return self.gemm_fma(x, w, out_dtype)
 
     @staticmethod
-    def long_matrix_tiles(m: int, n: int, k: int) -> bool:
+    def long_matrix_tiles(m: int, n: int, k: int, slices_do: bool = False) -> bool:
         """Whether a product of 65 to 256 rows is ``gemm_tile``'s: where the matrix is at least twice
         as long as it is wide (a down projection), so that tiles of 128 x 128 cut along K occupy
         the GPU and the slices are long.  Measured in replayed graphs (us, vendor library's first
@@ -729,7 +746,7 @@ class HipOps:
         128 200 / 167 / 110, at 256 314 / - / 200; 1B (2,048 x 8,192) at 192 22.9 / 19.7 / 18.2.  On
         squarer matrices the three are within a tenth of each other up to 128 rows, and from 384
         rows on the library wins everywhere."""
-        return SKINNY_MAX_ROWS < m <= 256 and k >= 2 * n and k >= 4096
+        return SKINNY_MAX_ROWS < m <= (128 if slices_do and k < 4 * n else 256) and k >= 2 * n and k >= 4096
 
     @staticmethod
     def few_library_tiles(m: int, n: int) -> bool:
@@ -785,6 +802,35 @@ class HipOps:
             x.data_ptr(), w.data_ptr(), y.data_ptr(), _code(out_dtype), m, n, k, x.stride(0), w.stride(0), n,
             self._library_workspace.data_ptr(), self._library_workspace.numel(), None, self._stream()))
         return y
+
+    def _block_plan(self, x, w, partial_ok: bool, gated: bool = False) -> int:
+        """The form and slices in which a product of many rows of bfloat16 is ``gemm_block``'s, or -1."""
+        if x.stride(0) >= 1 << 21 or w.stride(0) >= 1 << 21:
+            return -1
+        return self._ask("yk_gemm_block_plan", x.shape[0], w.shape[0], x.shape[1], int(partial_ok), int(gated))
+
+    def gemm_block(self, x, w, out_dtype, plan: int, gated=None):
+        """x [M, K] . w [N, K]^T in large tiles (bfloat16 operands with 16-byte aligned rows, K a multiple of 64) in the form and
+        slices of ``plan`` (form * 256 + slices): a tensor, or with slices a ``SplitSum``; ``gated``: pairs of groups of eight columns
+        (see ``gated_kind``)."""
+        m, k = x.shape
+        n = w.shape[0]
+        kind, p0, p1 = (0, 0.0, 0.0) if gated is None else self.gated_kind(gated)
+        slices = plan % 256
+        if slices > 1:
+            y, out = self._gemm_ws(slices * m * n), 1
+        else:
+            y = torch.empty((m, n // 2 if gated is not None else n), dtype=out_dtype, device=x.device)
+            out = 2 if gated is not None else _OUT_CODES[out_dtype]
+        self._check(self.lib.yk_gemm_block(
+            x.data_ptr(), w.data_ptr(), y.data_ptr(), out, m, n, k, x.stride(0), w.stride(0), n // 2 if gated is not None else n, plan, kind, p0, p1,
+            self._stream()))
+        return SplitSum(y[: slices * m * n].view(slices, m, n), out_dtype, self, self._gemm_gen) if slices > 1 else y
+
+    def force_block_plan(self, plan: int = -1) -> None:
+        """For tests and measurements: the plan of every product that ``gemm_block`` may take (form * 256 + slices; -1 the rule, -2 none)."""
+        self._check(self.lib.yk_gemm_block_force(int(plan)))
+        self._answers = {k: v for k, v in self._answers.items() if k[0] != "yk_gemm_block_plan"}
 
     def gemm_tile(self, x, w, out_dtype, partial_ok: bool = False):
         """x [M, K] . w [N, K]^T in tiles of 128 x 128 on the matrix cores (bfloat16 operands with
@@ -887,7 +933,8 @@ class HipOps:
     def gate_up_act(self, x: torch.Tensor, w_gate_up: torch.Tensor, group: int, activation: str, out_dtype: torch.dtype) -> torch.Tensor:
         """act(x . gate^T) * (x . up^T) -> [M, intermediate], ``w_gate_up`` and ``group`` as
         ``pack_gate_up`` gave them.  Few rows of bfloat16 whose product is not split over K
-        run as one kernel; otherwise the product, then the activation kernel."""
+        run as one kernel; so do many rows where ``gemm_block`` takes the product (the pairs of its own sums: those of ``linear`` and
+        ``gated_act`` up to rounding); otherwise the product, then the activation kernel."""
         act = {"silu": 1, "gelu_tanh": 2}.get(activation if isinstance(activation, str) else None)
         if act is None:
             self.gated_kind(activation)  # raises for an unknown one
@@ -909,6 +956,11 @@ class HipOps:
         )
         if not fused and pairs and self._takes_cols(x, w_gate_up):
             return self.gemm_cols(x, w_gate_up, bf, gated=activation)
+        if (pairs and m > SKINNY_MAX_ROWS and x.dtype == bf and w_gate_up.dtype == bf and w_gate_up.shape[1] == k and w_gate_up.stride(1) == 1
+                and x.stride(0) % 8 == 0 and w_gate_up.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0):
+            plan = self._block_plan(x, w_gate_up, False, gated=True)
+            if plan >= 0:
+                return self.gemm_block(x, w_gate_up, bf, plan, gated=activation)
         if not fused:
             return self.gated_act(self.linear(x, w_gate_up, out_dtype, partial_ok=True), activation, out_dtype, group=group)
         y = torch.empty((m, n // 2), dtype=bf, device=x.device)
