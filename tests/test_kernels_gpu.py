@@ -157,6 +157,57 @@ def test_float32_matrix_core_products(ops, form, m, n, k, xd, wd, od):
     close(got, want, atol, 2.0**-23 if od == torch.float32 else 2.0**-8)
 
 
+# rows around tiles of 64, columns around waves' 32 and tiles of 128, K around steps of 32 and sums of 128, slices with a short last one and
+# fewer made than asked for (5 of 6 pieces); 130 x 8 x 90,000: rows in three passes
+@pytest.mark.parametrize("m,n,k,slices", [(33, 1, 4, 1), (64, 128, 36, 1), (65, 129, 128, 1), (1, 31, 132, 1), (129, 132, 132, 2), (63, 64, 640, 5),
+                                          (127, 33, 1028, 1), (200, 260, 768, 5), (514, 260, 2048, 16), (130, 8, 90000, 1)])
+def test_gemm_split(ops, m, n, k, slices):
+    x = rnd((m, k + 8), torch.float32, 45)[:, 4: 4 + k]
+    w = rnd((n, k + 4), torch.float32, 46)[:, :k]
+    got = ops.gemm_split(x, w, slices)
+    want = x.double().cpu() @ w.double().cpu().T
+    # the running sum, of about sqrt(k), is rounded by 2^-24 of itself at each of k / 128 additions and some 16 of sums of 128 products and of
+    # slices; what else is lost is 2^-7 of that
+    close(got, want, math.sqrt(k) * math.sqrt(k / 128 + 16) * 2.0**-24 * 8, 2.0**-23)
+
+
+@pytest.mark.parametrize("slices", [1, 2])
+def test_gemm_split_of_numbers_at_the_limits(ops, slices):
+    x, w = rnd((40, 256), torch.float32, 47), rnd((12, 256), torch.float32, 48)
+    x[1] *= 1e-38  # subnormal numbers among them, and products that are
+    x[2] = x[2].abs() * 1e36  # the products of this row
+    w[1] = w[1].abs() * 1e30  # and this one grow beyond float32, and one another's signs hide none
+    w[2] *= 1e-30
+    x[3, 200], x[4, 9], w[3, 130] = math.inf, math.nan, -math.inf
+    x[5] = 0
+    got = ops.gemm_split(x, w, slices).cpu()
+    want = x.double().cpu() @ w.double().cpu().T
+    assert bool((got.isnan() == want.isnan()).all())
+    big = want.abs() > 3.4028235e38
+    assert bool((got.isinf() == big).all()) and bool((got[big].sign().double() == want[big].sign()).all())
+    rest = ~(big | want.isnan())
+    # 256 products, each at most the largest of its row and column, and sums below float32's smallest normal number to its last place
+    scale = x.double().cpu().abs().nan_to_num(0, 0, 0).amax(1)[:, None] * w.double().cpu().abs().nan_to_num(0, 0, 0).amax(1)[None]
+    bound = 16 * math.sqrt(256 / 128 + 16) * 2.0**-24 * 8 * scale + 2.0**-149 * 4
+    assert bool(((got.double() - want).abs() <= bound)[rest].all())
+
+
+def test_gemm_split_is_what_float32_products_of_many_rows_are(ops):
+    for m, n, k, taken in [(33, 3072, 2048, True), (511, 2048, 8192, True), (64, 512, 512, False), (32, 3072, 2048, False)]:
+        x, w = rnd((m, k), torch.float32, 49), rnd((n, k), torch.float32, 50)
+        slices = ops._ask("yk_gemm_split_plan", m, n, k)
+        assert bool(slices) == taken
+        if taken:
+            assert torch.equal(ops.gemm_fma(x, w, torch.float32), ops.gemm_split(x, w, slices))
+    from yalis_amd.ops.hip import KernelError
+
+    x, w = rnd((64, 256), torch.float32, 51), rnd((6, 256), torch.float32, 52)
+    with pytest.raises(KernelError):
+        ops.gemm_split(x, w, 2)  # rows of six columns are not for slices
+    with pytest.raises(KernelError):
+        ops.gemm_split(x, w, 3)
+
+
 # one to four rows: a wave's one or two rows of the weight, K around its pieces of 256 and its 8 (4) in flight
 @pytest.mark.parametrize("m", [1, 2, 3, 4])
 @pytest.mark.parametrize("n,k", [(1, 252), (5, 256), (9, 1028), (7, 2048), (6, 2052), (8191, 260), (8193, 1024), (8195, 1284),

@@ -1,7 +1,8 @@
 // Products y[M, N] = x[M, K] . w[N, K]^T with float32 arithmetic on the matrix cores
 // (v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32: float32 inputs, products and sums, no
 // narrower mode), for operands whose rows can be read four elements at a time.  gemm_fma in
-// gemm.hip takes what these do not: K or strides that are no multiple of four, unaligned rows.
+// gemm.hip takes what these do not: K or strides that are no multiple of four, unaligned rows.  Of more than 32 rows, all float32,
+// most are made by gemm_split.hip instead (its rule has both sides' times).
 //
 // As there, every 16 products along K are summed on their own and then added to the running sum:
 // a sum of K terms carries the rounding of about sqrt(K / 16) + 4 additions instead of sqrt(K).

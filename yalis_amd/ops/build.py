@@ -28,7 +28,7 @@ HOST_SOURCES = ["cache_manager.cpp"]
 # "kernels" only (so that is all a trace replay compiles), choosing tokens "sampling", the
 # benchmark's machine probes "probe".  Every library carries runtime.hip (its error slot).
 KERNEL_LIBS = {
-    "kernels": ["runtime.hip", "elementwise.hip", "gemm.hip", "gemm_f32.hip", "gemm_tile.hip", "gemm_cols.hip", "gemm_block.hip", "attention.hip", "library_gemm.hip",
+    "kernels": ["runtime.hip", "elementwise.hip", "gemm.hip", "gemm_f32.hip", "gemm_tile.hip", "gemm_cols.hip", "gemm_block.hip", "gemm_split.hip", "attention.hip", "library_gemm.hip",
                 "branch.hip", "attention_masked.hip", "recurrent.hip", "moe.hip", "sandwich_norm.hip", "latent_attention.hip",
                 "state_scan.hip", "chunk_scan.hip", "time_mix.hip", "streams.hip", "decay_scan.hip"],
     "sampling": ["runtime.hip", "sampling.hip"],

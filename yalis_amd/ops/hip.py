@@ -216,6 +216,12 @@ _SIGNATURES = {
     ),
     "yk_gemm_block_plan": ([_c_int, _c_int, _c_int, _c_int, _c_int], _c_int),
     "yk_gemm_block_force": ([_c_int], _c_int),
+    "yk_gemm_split": (
+        [_vp, _vp, _vp, _vp, ctypes.c_int64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp],
+        _c_int,
+    ),
+    "yk_gemm_split_plan": ([_c_int, _c_int, _c_int], _c_int),
+    "yk_gemm_split_floats": ([_c_int, _c_int, _c_int, _c_int], ctypes.c_int64),
     "yk_gemm_tile": (
         [_vp, _vp, _vp, _c_int, _vp, _c_size_t, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp],
         _c_int,
@@ -275,7 +281,7 @@ _LATER_SIGNATURES = {
         "yk_probe_mfma_bf16": ([_c_int, _c_int, _vp, _vp], _c_int),
     },
 }
-_ABI = 26
+_ABI = 27
 
 # Rows of x up to which the hand-written matrix-core kernel runs a bfloat16 product;
 # above it the vendor library does.
@@ -412,6 +418,7 @@ class HipOps:
         self._library_workspace: Optional[torch.Tensor] = None  # the vendor library's scratch
         self._gemm_workspace: Optional[torch.Tensor] = None  # K slices of products
         self._skinny_forced = False
+        self._float32_form = 0
         # how often each workspace has been handed out: what lives in one (SplitSum,
         # SplitAttention) remembers the number and is refused once it has moved on
         self._ws_gen = 0
@@ -862,13 +869,20 @@ class HipOps:
         """For tests and measurements: the form of float32 products (1: few rows; 2 and 4: tiles with that many
         groups of waves; 0: the library decides)."""
         self._check(self.lib.yk_gemm_f32_force(int(form)))
+        self._float32_form = int(form)
 
     def gemm_fma(self, x, w, out_dtype):
-        """x [M, K] . w [N, K]^T with float32 arithmetic, for any types and sizes: on the float32 matrix cores where
-        an operand is float32 and rows can be read four elements at a time, else by multiply-adds.  The order of a sum,
-        and so a row's last bits, depend on the number of rows."""
+        """x [M, K] . w [N, K]^T with float32 arithmetic, for any types and sizes: where an operand is float32 and rows can be
+        read four elements at a time on the matrix cores (of more than 32 rows, all float32, as ``gemm_split``), else by
+        multiply-adds.  The order of a sum, and so a row's last bits, depend on the number of rows."""
         m, k = x.shape
         n = w.shape[0]
+        f32 = torch.float32
+        if (m > 32 and k % 4 == 0 and x.dtype == f32 and w.dtype == f32 and out_dtype == f32 and not self._float32_form
+                and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and w.stride(0) <= 1 << 21 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+            slices = self._ask("yk_gemm_split_plan", m, n, k)
+            if slices:
+                return self.gemm_split(x, w, slices)
         y = torch.empty((m, n), dtype=out_dtype, device=x.device)
         self._check(
             self.lib.yk_gemm_fma(
@@ -876,6 +890,18 @@ class HipOps:
                 m, n, k, x.stride(0), w.stride(0), n, self._stream(),
             )
         )
+        return y
+
+    def gemm_split(self, x, w, slices: int = 1) -> torch.Tensor:
+        """x [M, K] . w [N, K]^T, all float32, as products of the operands' parts of 16 bits, which lose nothing of them: the
+        sums' error is no larger than that of float32 products.  K in ``slices`` slices."""
+        m, k = x.shape
+        n = w.shape[0]
+        y = torch.empty((m, n), dtype=torch.float32, device=x.device)
+        # of the call's own: other products' unreduced slices may wait in the shared scratch
+        ws = torch.empty(self._ask("yk_gemm_split_floats", m, n, k, slices), dtype=torch.float32, device=x.device)
+        self._check(self.lib.yk_gemm_split(x.data_ptr(), w.data_ptr(), y.data_ptr(), ws.data_ptr(), ws.numel(), m, n, k, x.stride(0),
+                                           w.stride(0), n, slices, self._stream()))
         return y
 
     # ---------------------------------------------------------- gate/up + activation
