@@ -19,14 +19,16 @@
 // lower triangle of 64 x 64 is cut into blocks n x n below the diagonal, n = 32, 16, 8, 4, 2, 1, and in a block the
 // rows' vectors carry the decays from the block's first token on, the columns' those up to the token before it.
 //
-// Bound by the walk, whose chunks come one after the other along the span: 4,100 clocks of matrix products (128 channels, delta
-// rule; 1.7 us) in about 3.7 us, the rest being its three meetings through LDS.  Everything it reads is asked for most of a chunk
-// ahead, in the order and place where the products take it.  Eight waves that share the two read-outs, with all operands twice,
-// took 170 us where four take 120: their registers leave no room for the loads on their way.
+// Bound by the walk, whose chunks come one after the other along the span: 3,700 clocks of matrix products a SIMD (128 channels, delta
+// rule; 1.5 us) in 2.9 us, the rest being three meetings through LDS and what waits between them.  Four waves carry S on and four make
+// the read-outs beside them: 2,048 tokens, 4 heads of 256 x 512 135 -> 95 us, 16 of 128 x 128 by the delta rule 123 -> 94, where the same four
+// waves did both in turn; 8 requests of 400 tokens 137 -> 103 and 120 -> 94.  What that rests on: the loads of the next chunk are asked
+// for between the products, a few at a time as their registers come free (all together they hold a wave's products up: 119 and 102 us),
+// with one scalar base a chunk; asking two chunks ahead is no faster (132, 110: it is the loads' issue that costs, not their time).
 //
-// 2,048 tokens of one request in bfloat16, us (of which prepare; token by token: yk_linear_state_scan): 16 heads of 128 x 128, delta rule 158
-// (39; 465), with decays per channel 185 (69; 496); 4 of 256 x 512 gated 189 (61; 497); 32 of 64 x 64 with a bonus 96 (396); 32 of
-// 128 x 64 by step 132 (396).  Errors against float64, of their size, of the read-outs 1.1e-7, 1.1e-7, 2.5e-7, 0.7e-7, 0.8e-7 (walked
+// 2,048 tokens of one request in bfloat16, us (of which prepare; token by token: yk_linear_state_scan): 16 heads of 128 x 128, delta rule 135
+// (41; 465), with decays per channel 164 (69; 496); 4 of 256 x 512 gated 156 (61; 497); 32 of 64 x 64 with a bonus 84 (396); 32 of
+// 128 x 64 by step 112 (396).  Errors against float64, of their size, of the read-outs 1.1e-7, 1.1e-7, 2.5e-7, 0.7e-7, 0.8e-7 (walked
 // 1.1e-7, 1.1e-7, 2.6e-7, 0.9e-7, 0.9e-7) and of the kept memories 0.8e-7, 0.8e-7, 2.4e-7, 0.4e-7, 0.6e-7 (0.8e-7, 0.8e-7, 2.6e-7, 0.4e-7, 0.6e-7).
 #include <algorithm>
 #include <type_traits>
@@ -83,6 +85,26 @@ __device__ __forceinline__ f32x4_t triangle16(f32x4_t a, f32x4_t b, f32x4_t c) {
         if (4 * kk + e <= 4 * lg + i && !(fabsf(y) < INFINITY)) c[i] = fmaf(x, y, c[i]);
       }
     }
+  return c;
+}
+
+// c + row ROW of tiles, up to the diagonal's, times a column of them (the tiles' products side by side, added in their order)
+template <int ROW>
+__device__ __forceinline__ f32x4_t lower_row(const f32x4_t* a, const f32x4_t* b, f32x4_t c) {
+  const float sum = fabsf(b[ROW][0]) + fabsf(b[ROW][1]) + fabsf(b[ROW][2]) + fabsf(b[ROW][3]);
+  if (__any(!(sum < INFINITY))) {
+#pragma unroll
+    for (int m = 0; m < ROW; ++m) c = mma16(a[m], b[m], c);
+    return triangle16(a[ROW], b[ROW], c);
+  }
+  f32x4_t s[ROW + 1];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int m = 0; m <= ROW; ++m)
+      s[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][i], b[m][i], i == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : s[m], 0, 0, 0);
+#pragma unroll
+  for (int m = 0; m <= ROW; ++m) c = c + s[m];
   return c;
 }
 
@@ -531,20 +553,79 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
 }
 
 // ---------------------------------------------------------------------------------------------- walk
-// A workgroup of four waves a (head, 16 columns of S, request).  A wave owns a quarter of the rows of S, as the products
-// that update it leave them (lane (r, g): rows 4g .. 4g + 3 of a tile of 16, column r), which is also how the other
-// products take S, v and u as their second operand; through LDS every wave gets all of them.  For the read-outs a wave
-// owns 16 tokens.
+// A workgroup of eight waves a (head, 16 columns of S, request).  Four of them carry S on: a wave owns a quarter of its rows, as the
+// products that update it leave them (lane (r, g): rows 4g .. 4g + 3 of a tile of 16, column r), which is also how the other products take
+// S, v and u as their second operand; through LDS every wave gets all of them.  The other four make the read-outs, 16 tokens each, of S
+// and u in LDS while the first are at the update (a wave of each kind a SIMD; the waves with the most tiles up to the diagonal of T and of
+// B are not neighbours).
 template <typename T, int D, int KIND>
-__global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict__ qkv, float* __restrict__ state, float* __restrict__ out, ChunkArgs g) {
+__global__ __launch_bounds__(512, 2) void chunk_walk_kernel(const T* __restrict__ qkv, float* __restrict__ state, float* __restrict__ out, ChunkArgs g) {
   constexpr bool DELTA = KIND & kDelta;
   constexpr int M = D / 16, MT = D / 64;
   using P = Part<D, KIND>;
-  __shared__ __attribute__((aligned(16))) f32x4_t s_lds[M][64], x_lds[4][64], u_lds[4][64];
+  // (two of what a chunk's read-outs may still read while the next chunk's is written)
+  __shared__ __attribute__((aligned(16))) f32x4_t s_lds[2][M][64], x_lds[DELTA ? 4 : 1][64], u_lds[2][4][64];
   const int hl = blockIdx.x, h = g.head0 + hl, col0 = 16 * blockIdx.y, seq = blockIdx.z, vdim = g.vdim;
   const int q0 = g.seq_qstart[seq], ql = g.seq_qlen[seq], chunks = (ql + kTok - 1) / kTok;
   if (ql <= 0) return;  // (a request without tokens leaves its memory alone: its slot may be another's by now)
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), r = lane % 16, lg = lane / 16;
+  // (the last chunk asks for itself once more, unread)
+  auto part = [&](int c) {
+    return __builtin_amdgcn_make_buffer_rsrc(g.ws + part_of(seq, gridDim.z, q0, min(c, chunks - 1), gridDim.x, hl) * P::SIZE, 0, P::SIZE * 4, 0x00027000);
+  };
+  // (a scalar base and place: addresses of their own would take the registers that the loads on their way need)
+  using Source = __amdgpu_buffer_rsrc_t;
+  auto piece = [](Source p, int lane_bytes, int at) {
+    return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(p, lane_bytes, 4 * at, 0));
+  };
+  auto lower = [&](int row, const f32x4_t* a, const f32x4_t* b, f32x4_t c) {
+    return row == 0 ? lower_row<0>(a, b, c) : row == 1 ? lower_row<1>(a, b, c) : row == 2 ? lower_row<2>(a, b, c) : lower_row<3>(a, b, c);
+  };
+
+  if (wave >= 4) {
+    const int tile = 7 - wave;
+    f32x4_t q[M], b[4];
+    auto ask_q = [&](Source p, int m) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) q[m + x] = piece(p, 16 * lane, P::Q + at<M>(tile, m + x, 0));
+    };
+    auto ask_b = [&](Source p) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) b[m] = piece(p, 16 * lane, P::B + at<4>(tile, m, 0));
+    };
+#pragma unroll
+    for (int m = 0; m < M; m += 4) ask_q(part(0), m);
+    ask_b(part(0));
+    for (int c = 0; c < chunks; ++c) {
+      const Source next = part(c + 1);
+      __syncthreads();  // S is in LDS (and u, where it is v)
+      f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int m = 0; m < M; m += 4) {
+        if (DELTA && m == M / 2) __syncthreads();  // (the writers': v - K' S is in LDS)
+        f32x4_t s4[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) s4[x] = s_lds[c % 2][m + x][lane];
+        o += mma64(&q[m], s4);
+        ask_q(next, m);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (DELTA && M == 4) __syncthreads();
+      if (DELTA) __syncthreads();  // u is in LDS
+      f32x4_t u[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) u[m] = u_lds[c % 2][m][lane];
+      o = lower(tile, b, u, o);
+      ask_b(next);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = c * kTok + 16 * tile + 4 * lg + i;
+        if (t < ql) out[(static_cast<size_t>(q0 + t) * g.n_heads + h) * vdim + col0 + r] = o[i];
+      }
+    }
+    return;
+  }
+
   float* S_head = state + (static_cast<size_t>(g.state_slots[seq]) * g.n_heads + h) * D * vdim + col0 + r;
   f32x4_t S[MT];
 #pragma unroll
@@ -555,15 +636,11 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
   // (waited for here: a load from before the loop that may still be on its way inside it makes every turn wait for its own)
   __builtin_amdgcn_s_waitcnt(0);
 
-  f32x4_t q[M], k[DELTA ? M : 1], ke[MT][4], b[4], tm[DELTA ? 4 : 1], dec[MT];
+  f32x4_t k[DELTA ? M : 1], ke[MT][4], tm[DELTA ? 4 : 1], dec[MT];
   uint32_t raw_v[4];  // (as they lie there: a conversion where they are asked for would wait for them)
-  const float* part0 = g.ws + part_of(seq, gridDim.z, q0, 0, gridDim.x, hl) * P::SIZE;
-  auto ask_qk = [&](const float* p) {
+  auto ask_k = [&](Source p, int m) {
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      if (DELTA) k[m] = *reinterpret_cast<const f32x4_t*>(p + P::K + at<M>(wave, m, lane));
-      q[m] = *reinterpret_cast<const f32x4_t*>(p + P::Q + at<M>(wave, m, lane));
-    }
+    for (int x = 0; x < 4; ++x) k[m + x] = piece(p, 16 * lane, P::K + at<M>(wave, m + x, 0));
   };
   auto ask_v = [&](int c) {
 #pragma unroll
@@ -572,77 +649,72 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
       raw_v[i] = raw_bits(qkv[static_cast<size_t>(q0 + min(t, ql - 1)) * g.qkv_stride + g.v_col + h * vdim + col0 + r]);
     }
   };
-  auto ask_t = [&](const float* p) {
+  auto ask_t = [&](Source p) {
     if (DELTA) {
 #pragma unroll
-      for (int m = 0; m < 4; ++m) tm[m] = *reinterpret_cast<const f32x4_t*>(p + P::T + at<4>(wave, m, lane));
+      for (int m = 0; m < 4; ++m) tm[m] = piece(p, 16 * lane, P::T + at<4>(wave, m, 0));
     }
   };
-  auto ask_b = [&](const float* p) {
+  auto ask_ke = [&](Source p, int m) {
+    dec[m] = piece(p, 16 * lg, P::DEC + 16 * (wave * MT + m));
 #pragma unroll
-    for (int m = 0; m < 4; ++m) b[m] = *reinterpret_cast<const f32x4_t*>(p + P::B + at<4>(wave, m, lane));
+    for (int x = 0; x < 4; ++x) ke[m][x] = piece(p, 16 * lane, P::KE + at<4>(wave * MT + m, x, 0));
   };
-  auto ask_ke = [&](const float* p) {
+  if (DELTA) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      dec[m] = *reinterpret_cast<const f32x4_t*>(p + P::DEC + 16 * (wave * MT + m) + 4 * lg);
-#pragma unroll
-      for (int x = 0; x < 4; ++x) ke[m][x] = *reinterpret_cast<const f32x4_t*>(p + P::KE + at<4>(wave * MT + m, x, lane));
-    }
-  };
-  // the tiles up to the diagonal of this wave's row of tiles
-  auto lower = [&](const f32x4_t* a, const f32x4_t* b, f32x4_t c) {
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-      if (m < wave) c = mma16(a[m], b[m], c);
-    return wave == 0 ? triangle16(a[0], b[0], c) : wave == 1 ? triangle16(a[1], b[1], c) : wave == 2 ? triangle16(a[2], b[2], c) : triangle16(a[3], b[3], c);
-  };
-  ask_qk(part0);
+    for (int m = 0; m < M; m += 4) ask_k(part(0), m);
+  }
   ask_v(0);
-  ask_t(part0);
-  ask_b(part0);
-  ask_ke(part0);
+  ask_t(part(0));
+#pragma unroll
+  for (int m = 0; m < MT; ++m) ask_ke(part(0), m);
   auto turn = [&](int c, auto last) {
-    // (the last chunk asks for itself once more, unread)
-    const float* next = g.ws + part_of(seq, gridDim.z, q0, decltype(last)::value ? c : c + 1, gridDim.x, hl) * P::SIZE;
+    const Source next = part(c + 1);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) s_lds[wave * MT + m][lane] = S[m];
-    __syncthreads();
-    f32x4_t o = {0.f, 0.f, 0.f, 0.f}, p = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int m = 0; m < M; m += 4) {
-      f32x4_t s4[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) s4[x] = s_lds[m + x][lane];
-      if (DELTA) p += mma64(&k[m], s4);
-      o += mma64(&q[m], s4);
-    }
-    ask_qk(next);
+    for (int m = 0; m < MT; ++m) s_lds[c % 2][wave * MT + m][lane] = S[m];
     f32x4_t v;
+    auto take_v = [&] {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = c * kTok + 16 * wave + 4 * lg + i < ql ? from_raw<T>(raw_v[i]) : 0.f;
-    ask_v(min(c + 1, chunks - 1));
+      for (int i = 0; i < 4; ++i) v[i] = c * kTok + 16 * wave + 4 * lg + i < ql ? from_raw<T>(raw_v[i]) : 0.f;
+      ask_v(min(c + 1, chunks - 1));
+    };
+    if (!DELTA) {
+      take_v();
+      u_lds[c % 2][wave][lane] = v;
+    }
+    __syncthreads();
     if (DELTA) {
+      f32x4_t p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int m = 0; m < M; m += 4) {
+        f32x4_t s4[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) s4[x] = s_lds[c % 2][m + x][lane];
+        p += mma64(&k[m], s4);
+        ask_k(next, m);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      take_v();
       x_lds[wave][lane] = v - p;
       __syncthreads();
       f32x4_t x4[4];
 #pragma unroll
       for (int m = 0; m < 4; ++m) x4[m] = x_lds[m][lane];
-      u_lds[wave][lane] = lower(tm, x4, f32x4_t{0.f, 0.f, 0.f, 0.f});
+      u_lds[c % 2][wave][lane] = lower(wave, tm, x4, f32x4_t{0.f, 0.f, 0.f, 0.f});
       ask_t(next);
-    } else {
-      u_lds[wave][lane] = v;
+      __syncthreads();
     }
-    __syncthreads();
     f32x4_t u[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) u[m] = u_lds[m][lane];
+    for (int m = 0; m < 4; ++m) u[m] = u_lds[c % 2][m][lane];
     if (!decltype(last)::value) {
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         const f32x4_t sum = mma64(ke[m], u);
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[m][i] = fmaf(S[m][i], dec[m][i], sum[i]);
+        ask_ke(next, m);
+        __builtin_amdgcn_sched_barrier(0);
       }
     } else {
       // the memory that is kept: in float64, rounded once.  Its last tokens weigh the most and 64 products in float32 round them oftener than
@@ -662,14 +734,6 @@ __global__ __launch_bounds__(256, 1) void chunk_walk_kernel(const T* __restrict_
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[m][i] = static_cast<float>(sum[i]);
       }
-    }
-    ask_ke(next);
-    o = lower(b, u, o);
-    ask_b(next);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = c * kTok + 16 * wave + 4 * lg + i;
-      if (t < ql) out[(static_cast<size_t>(q0 + t) * g.n_heads + h) * vdim + col0 + r] = o[i];
     }
   };
   for (int c = 0; c + 1 < chunks; ++c) turn(c, std::false_type{});
@@ -691,7 +755,7 @@ int launch(const T* qkv, const T* beta_rows, float* state, float* out, ChunkArgs
     const int here = std::min(heads, g.n_heads - g.head0);
     chunk_prepare_kernel<T, D, KIND><<<dim3((max_qlen + kTok - 1) / kTok, here, n_seqs), 256 * prepare_groups(D), 0, stream>>>(qkv, beta_rows, g);
     if (yk_check_launch("chunk_prepare")) return -1;
-    chunk_walk_kernel<T, D, KIND><<<dim3(here, g.vdim / 16, n_seqs), 256, 0, stream>>>(qkv, state, out, g);
+    chunk_walk_kernel<T, D, KIND><<<dim3(here, g.vdim / 16, n_seqs), 512, 0, stream>>>(qkv, state, out, g);
     if (yk_check_launch("chunk_walk")) return -1;
   }
   return 0;
