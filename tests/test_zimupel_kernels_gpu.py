@@ -320,6 +320,20 @@ def test_gated_head_norm_forms(dtype, heads, vdim, gate_act, gate_first):
             close(got, want, dtype, "read-out", f32=1e-5, bf16=8e-3)
 
 
+# parts around the sizes where more threads or more pieces a thread take one; a number of parts that leaves a workgroup half empty
+@pytest.mark.parametrize("vdim", [4, 60, 64, 68, 128, 132, 256, 260, 512, 516, 1024, 1028])
+@pytest.mark.parametrize("n,heads", [(1, 1), (7, 5)])
+def test_gated_head_norm_of_parts_of_any_size(n, heads, vdim):
+    o = ops()
+    g = torch.Generator().manual_seed(vdim)
+    x, gate, w = (torch.randn(*s, generator=g) for s in ((n, heads * vdim), (n, heads * vdim), (vdim,)))
+    y = x.double().view(n, heads, vdim)
+    want = (y / torch.sqrt((y * y).mean(-1, keepdim=True) + 1e-4) * w.double() * (gate.double() * torch.sigmoid(gate.double())).view(n, heads, vdim)).reshape(n, -1)
+    got = o.gated_head_norm(x.cuda(), w.cuda(), 1e-4, gate.cuda(), 0, heads, vdim, torch.float32)
+    # a sum of at most 1,028 squares in float32, its root, a quotient and three products, each rounded once: 16 roundings cover them
+    assert bool(((got.double().cpu() - want).abs() <= 16 * 2.0**-24 * want.abs() + 1e-37).all())
+
+
 # ------------------------------------------------------------------------------------------------------- the router
 @pytest.mark.parametrize("n,experts,top,padded,groups", [(1, 2, 1, 16, None), (37, 12, 4, 16, (2, 1)), (200, 8, 8, 8, (4, 4)), (64, 40, 3, 48, (10, 4)),
                                                          (9, 130, 6, 144, (13, 2)), (50, 6, 2, 16, (6, 3)), (5, 256, 8, 256, (8, 4)), (33, 9, 5, 16, None)])

@@ -944,8 +944,11 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* __res
     out[item * vdim + c] = from_f32<TO>(row[c] * inv * weight(c) * head_gate_act(to_f32<TG>(g[c]), gate_act));
 }
 
-// The same in pieces of four elements, a thread holding up to four of them: everything is asked for before the sum.  A wave a
-// part (four parts a workgroup) or, for parts of more than 1,024 elements, a workgroup a part.
+// The same in pieces of four elements, a thread holding P of them: everything is asked for before the sum.  LANES threads a part: as few
+// as hold it in one piece each up to a wave, which holds up to 1,024 elements in four, beyond it a workgroup.  Bound by memory where the
+// parts are many (bfloat16 gates and results, us, with its launch): 3,241 tokens of 16 parts of 128 12.9, where a wave a part with four pieces
+// a thread, three of them empty, took 46 for the gates' exponentials of nothing; 2,048 tokens of 32 parts of 64 7.8 (53), 16 of 128 8.4
+// (28), 8 of 256 8.0 (15.8), 4 of 512 8.1 (10.1), 2 of 1,024 8.1 (8.2).
 template <typename T>
 __device__ __forceinline__ float4 hn_load4(const T* p);
 template <>
@@ -958,17 +961,24 @@ __device__ __forceinline__ float4 hn_load4<bf16_t>(const bf16_t* p) {
 __device__ __forceinline__ void hn_store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void hn_store4(bf16_t* p, float4 v) { *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)); }
 
-template <typename TW, typename TG, typename TO, bool WAVE>
+template <int LANES>
+__device__ __forceinline__ float hn_sum(float v, float* scratch) {
+  if (LANES > kWave) return block_sum(v, scratch);
+  if (LANES == kWave) return wave_sum(v);
+  if (LANES == 16) return row_sum(v);
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return row_sum(__uint_as_float(rows[0]) + __uint_as_float(rows[1]));
+}
+
+template <typename TW, typename TG, typename TO, int LANES, int P>
 __global__ __launch_bounds__(256) void gated_head_norm_vec_kernel(const float* __restrict__ o, const TW* __restrict__ w, float eps,
                                                                   const TG* __restrict__ gate, int gate_stride, int gate_col, int n_heads,
                                                                   int vdim, TO* __restrict__ out, size_t total, int w_stride, int gate_first,
                                                                   int gate_act) {
   __shared__ float scratch[17];
-  constexpr int T = WAVE ? kWave : 256, P = 4;
-  const size_t wanted = WAVE ? blockIdx.x * static_cast<size_t>(4) + threadIdx.x / kWave : blockIdx.x;
-  if (WAVE && wanted >= total) return;  // (a whole wave)
-  const size_t item = wanted;
-  const int t = threadIdx.x % T;
+  const size_t wanted = blockIdx.x * static_cast<size_t>(256 / LANES) + threadIdx.x / LANES;
+  const size_t item = min(wanted, total - 1);  // (threads past the end repeat the last part and store nothing)
+  const int t = threadIdx.x % LANES;
   const size_t n = item / n_heads;
   const int h = static_cast<int>(item % n_heads);
   const float* row = o + item * vdim;
@@ -977,7 +987,7 @@ __global__ __launch_bounds__(256) void gated_head_norm_vec_kernel(const float* _
   float ss = 0.f;
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const int c = 4 * (t + p * T);
+    const int c = 4 * (t + p * LANES);
     v[p] = a[p] = make_float4(0.f, 0.f, 0.f, 0.f);
     m[p] = make_float4(1.f, 1.f, 1.f, 1.f);
     if (c < vdim) {
@@ -992,12 +1002,12 @@ __global__ __launch_bounds__(256) void gated_head_norm_vec_kernel(const float* _
     if (gate_first) v[p] = make_float4(v[p].x * a[p].x, v[p].y * a[p].y, v[p].z * a[p].z, v[p].w * a[p].w);
     ss = fmaf(v[p].x, v[p].x, fmaf(v[p].y, v[p].y, fmaf(v[p].z, v[p].z, fmaf(v[p].w, v[p].w, ss))));
   }
-  ss = WAVE ? wave_sum(ss) : block_sum(ss, scratch);
+  ss = hn_sum<LANES>(ss, scratch);
   const float inv = 1.f / sqrtf(ss / static_cast<float>(vdim) + eps);
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const int c = 4 * (t + p * T);
-    if (c < vdim) {
+    const int c = 4 * (t + p * LANES);
+    if (c < vdim && wanted < total) {
       float4 y = make_float4(v[p].x * inv * m[p].x, v[p].y * inv * m[p].y, v[p].z * inv * m[p].z, v[p].w * inv * m[p].w);
       if (!gate_first) y.x *= a[p].x, y.y *= a[p].y, y.z *= a[p].z, y.w *= a[p].w;
       hn_store4(out + item * vdim + c, y);
@@ -1017,16 +1027,18 @@ extern "C" int yk_gated_head_norm(const float* o, const void* w, int w_dtype, fl
   const int w_stride = w_per_part ? vdim : 0;
   auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool vec = vdim % 4 == 0 && vdim <= 4096 && gate_stride % 4 == 0 && gate_col % 4 == 0 && al16(o) && al16(w) && al16(gate) && al16(out);
+#define YK_VEC(TW, TG, TO, LANES, P)                                                                                  \
+  gated_head_norm_vec_kernel<TW, TG, TO, LANES, P><<<static_cast<unsigned>((total + 256 / LANES - 1) / (256 / LANES)), 256, 0, stream>>>( \
+      o, static_cast<const TW*>(w), eps, static_cast<const TG*>(gate), gate_stride, gate_col, n_heads, vdim,          \
+      static_cast<TO*>(out), total, w_stride, gate_first, gate_act)
 #define YK_CASE(WD, TW, GD, TG, OD, TO)                                                                               \
   if (w_dtype == WD && gate_dtype == GD && out_dtype == OD) {                                                         \
-    if (vec && vdim > 1024)                                                                                           \
-      gated_head_norm_vec_kernel<TW, TG, TO, false><<<static_cast<unsigned>(total), 256, 0, stream>>>(                \
-          o, static_cast<const TW*>(w), eps, static_cast<const TG*>(gate), gate_stride, gate_col, n_heads, vdim,      \
-          static_cast<TO*>(out), total, w_stride, gate_first, gate_act);                                              \
-    else if (vec)                                                                                                     \
-      gated_head_norm_vec_kernel<TW, TG, TO, true><<<grid, 256, 0, stream>>>(                                         \
-          o, static_cast<const TW*>(w), eps, static_cast<const TG*>(gate), gate_stride, gate_col, n_heads, vdim,      \
-          static_cast<TO*>(out), total, w_stride, gate_first, gate_act);                                              \
+    if (vec && vdim > 1024) YK_VEC(TW, TG, TO, 256, 4);                                                               \
+    else if (vec && vdim > 512) YK_VEC(TW, TG, TO, 64, 4);                                                            \
+    else if (vec && vdim > 256) YK_VEC(TW, TG, TO, 64, 2);                                                            \
+    else if (vec && vdim > 128) YK_VEC(TW, TG, TO, 64, 1);                                                            \
+    else if (vec && vdim > 64) YK_VEC(TW, TG, TO, 32, 1);                                                             \
+    else if (vec) YK_VEC(TW, TG, TO, 16, 1);                                                                          \
     else                                                                                                              \
     gated_head_norm_kernel<TW, TG, TO><<<grid, 256, 0, stream>>>(o, static_cast<const TW*>(w), eps,                   \
                                                                  static_cast<const TG*>(gate), gate_stride, gate_col, \
