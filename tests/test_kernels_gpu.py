@@ -947,6 +947,35 @@ def test_attention_generic_many_tokens(ops, h, g, d, page, window, dtype):
         close(got, want, 1e-2, 2**-7)
 
 
+# head sizes 64 and 128 in float32: tiles of 16 columns of 16, 8, 4, 2 and 1 heads, which tokens of several requests share; pages of a few slots
+@pytest.mark.parametrize("h,g,d,page", [(48, 3, 64, 16), (40, 5, 128, 4), (48, 12, 64, 64), (72, 2, 128, 20), (40, 20, 64, 8), (45, 15, 128, 32)])
+@pytest.mark.parametrize("window", [0, 3, 66])
+def test_attention_float32_tiles(ops, h, g, d, page, window):
+    got, want = _attention_case(ops, torch.float32, h, g, d, page, SPANS, window, 20, n_pages=160)
+    close(got, want, 2e-5, 1e-5)
+
+
+@pytest.mark.parametrize("window", [0, 9])
+def test_attention_float32_tiles_keep_later_values_from_earlier_tokens(ops, window):
+    n, h, g, d, page, gen = 70, 64, 16, 64, 16, torch.Generator().manual_seed(21)
+    q, keys, values = (torch.randn(s, generator=gen) for s in ((n, h, d), (n, g, d), (n, g, d)))
+    values[10, :, 5], values[30, :, 7], values[69, 2] = math.inf, math.nan, -math.inf
+    pages = -(-n // page)
+    kc, vc = torch.zeros((pages, g, page, d)), torch.zeros((pages, g, d, page))
+    for pos in range(n):
+        kc[pos // page, :, pos % page], vc[pos // page, :, :, pos % page] = keys[pos], values[pos]
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    ctx = types.SimpleNamespace(arrays={"positions": dev(list(range(n))), "token_seq": dev([0] * n), "block_table_g0": dev([list(range(pages))])}, max_ctx=n)
+    got = ops.attention(q.view(n, -1).to(DEV), h, g, d, kc.to(DEV), vc.to(DEV), page, 0.125, window, ctx, 0, None).cpu().view(n, h, d)
+    for t in range(n):
+        first = max(0, t - window + 1) if window else 0
+        k, v = (x[first: t + 1].double().repeat_interleave(h // g, 1) for x in (keys, values))
+        want = torch.einsum("hk,khd->hd", (torch.einsum("hd,khd->hk", q[t].double(), k) * 0.125).softmax(-1), v)
+        assert bool((got[t].isfinite() == want.isfinite()).all()), t
+        at = want.isfinite()
+        close(got[t][at], want[at], 2e-5, 1e-5)
+
+
 # pages whose slots are no multiple of four, and pages that do not start at a multiple of 16 bytes; few and many (token, head)s
 @pytest.mark.parametrize("h,g,d,page,shift", [(4, 2, 16, 6, 0), (6, 3, 48, 1, 0), (5, 5, 80, 18, 0), (48, 12, 16, 7, 0), (4, 1, 32, 32, 1), (48, 12, 16, 16, 3)])
 @pytest.mark.parametrize("window", [0, 3, 66])

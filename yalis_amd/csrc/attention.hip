@@ -194,8 +194,156 @@ __global__ __launch_bounds__(64 * W) void attn_generic_kernel(
   }
 }
 
-// Where the (token, head)s alone fill the GPU several times over, a wave makes up to four heads that
-// share their keys; else (decoded tokens, short portions) eight waves share a head's keys.
+// The same in float32 for many tokens, on the matrix cores (v_mfma_f32_16x16x4_f32; head sizes 64 and 128, pages and rows in aligned
+// pieces of 16 bytes): 16 columns, some heads that share a key/value head of neighbouring tokens, to a workgroup whose W waves take blocks of
+// 16 keys by turns and merge at the end.  Lane (r, g) holds elements 16 j + 4 g .. + 3 of key r and of column r's query, then keys
+// 4 g .. + 3 of element 16 t + r: the scores leave the first product as the second takes them, nothing passes LDS.  Tokens of several requests
+// in one workgroup are walked a request at a time, the others' columns masked.  The sums of a block's 16 products join the running sums at once.
+// Bound by the latency of the loads.  32 heads of 64 over 8 kv heads, us (as a wave a token and four heads): 511 tokens of two prompts 22
+// (69), 2,048 of one 296 (1,283), 128 behind 1,000 35 (143), 128 requests of one token behind 300 47 (48); of 128, two prompts of 300 47 (148).
+// Error against 64 bits 1.3e-7, 2.0e-7 and 1.7e-7 of the first, the third and the fourth's size (1.7e-7, 6.1e-7, 3.4e-7).
+template <int DT, int W>
+__global__ __launch_bounds__(64 * W) void attn_f32_tile_kernel(const float* __restrict__ q, int q_stride, float* __restrict__ out,
+                                                               const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+                                                               const int32_t* __restrict__ positions, const int32_t* __restrict__ token_seq,
+                                                               const int32_t* __restrict__ block_table, int table_width, int page_size,
+                                                               int n_tokens, int n_heads, int n_kv, int hpt, float scale, int window) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  constexpr int D = 16 * DT;
+  __shared__ f4 part_o[W][DT][64];
+  __shared__ float part_m[W][16], part_l[W][16];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), r = lane % 16, g = lane / 16;
+  const bool tiled = cache_is_tiled(YK_F32, D, page_size);
+  const size_t slab = static_cast<size_t>(page_size) * D;
+  const int tpt = 16 / hpt, first = blockIdx.x * tpt, here = min(tpt, n_tokens - first), h0 = blockIdx.y * hpt, kv = h0 / (n_heads / n_kv);
+  const int tt = r / hpt, n = first + min(tt, here - 1), head = h0 + r % hpt;
+  const int pos = positions[n], my_lo = window > 0 ? max(0, pos - window + 1) : 0;
+  f4 qf[DT], acc[DT];
+#pragma unroll
+  for (int j = 0; j < DT; ++j) {
+    qf[j] = *reinterpret_cast<const f4*>(q + static_cast<size_t>(n) * q_stride + static_cast<size_t>(head) * D + 16 * j + 4 * g);
+    acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+  }
+  float m = -INFINITY, l = 0.f;
+  for (int t0 = 0; t0 < here;) {
+    // the tokens from t0 on that are of its request, and the keys they see
+    const int seq = token_seq[first + t0];
+    int t1 = t0, hi = 0, lo = INT_MAX;
+    for (; t1 < here && token_seq[first + t1] == seq; ++t1) {
+      const int p = positions[first + t1];
+      hi = max(hi, p + 1);
+      lo = min(lo, window > 0 ? max(0, p - window + 1) : 0);
+    }
+    const bool mine = tt >= t0 && tt < t1;
+    t0 = t1;
+    const int32_t* bt = block_table + static_cast<size_t>(seq) * table_width;
+    for (int key0 = (lo / 16 + wave) * 16; key0 < hi; key0 += 16 * W) {
+      f4 k4[DT], v4[DT];
+      {
+        const int key = min(max(key0 + r, lo), hi - 1);
+        const float* kp = k_cache + (static_cast<size_t>(bt[key / page_size]) * n_kv + kv) * slab;
+#pragma unroll
+        for (int j = 0; j < DT; ++j) k4[j] = *reinterpret_cast<const f4*>(kp + cache_k_offset(tiled, page_size, D, key % page_size, 16 * j + 4 * g));
+      }
+      const int keys = key0 + 4 * g;  // (four consecutive slots of one page)
+      {
+        const int key = min(max(keys, lo), hi - 1) & ~3;
+        const float* vp = v_cache + (static_cast<size_t>(bt[key / page_size]) * n_kv + kv) * slab;
+#pragma unroll
+        for (int j = 0; j < DT; ++j) v4[j] = *reinterpret_cast<const f4*>(vp + cache_v_offset(tiled, page_size, D, key % page_size, 16 * j + r));
+      }
+      f4 s4[4];
+#pragma unroll
+      for (int j = 0; j < DT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          s4[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[j][i], qf[j][i], j == 0 ? f4{0.f, 0.f, 0.f, 0.f} : s4[i], 0, 0, 0);
+      f4 s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+      bool seen[4], all = true;
+      float top = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        seen[i] = mine && keys + i <= pos && keys + i >= my_lo;
+        all = all && seen[i];
+        s[i] = seen[i] ? s[i] * scale : -INFINITY;
+        top = fmaxf(top, s[i]);
+      }
+      const float m_new = fmaxf(m, column_lanes_max(top));
+      const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = m == m_new ? 1.f : expf(m - m_safe);
+      m = m_new;
+      f4 p;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = seen[i] ? expf(s[i] - m_safe) : 0.f;
+      l = fmaf(l, alpha, (p[0] + p[1]) + (p[2] + p[3]));
+      bool finite = true;
+      if (!__all(all)) {  // what lies in a page beside the keys is not to be read as a number
+#pragma unroll
+        for (int j = 0; j < DT; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v4[j][i] = keys + i >= lo && keys + i < hi ? v4[j][i] : 0.f;
+            finite = finite && fabsf(v4[j][i]) < INFINITY;
+          }
+      }
+      if (__all(finite)) {
+#pragma unroll
+        for (int j = 0; j < DT; ++j) {
+          f4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[j][i], p[i], sum, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[j][i] = fmaf(acc[j][i], alpha, sum[i]);
+        }
+      } else {
+        // a key that some column does not see has what is no number: it is kept from that column, which its weight of zero would not do
+#pragma unroll
+        for (int j = 0; j < DT; ++j) {
+          acc[j] *= alpha;
+#pragma unroll 1
+          for (int from = 0; from < 4; ++from)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float weight = __shfl(p[e], 16 * from + r, 64);
+              const bool sees = __shfl(static_cast<int>(seen[e]), 16 * from + r, 64) != 0;
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const float v = __shfl(v4[j][e], 16 * from + 4 * g + i, 64);
+                if (sees) acc[j][i] = fmaf(weight, v, acc[j][i]);
+              }
+            }
+        }
+      }
+    }
+  }
+  l = column_lanes_sum(l);
+  if (g == 0) {
+    part_m[wave][r] = m;
+    part_l[wave][r] = l;
+  }
+#pragma unroll
+  for (int j = 0; j < DT; ++j) part_o[wave][j][lane] = acc[j];
+  __syncthreads();
+  float top = -INFINITY, sum = 0.f, weight[W];
+#pragma unroll
+  for (int w = 0; w < W; ++w) top = fmaxf(top, part_m[w][r]);
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    weight[w] = expf(part_m[w][r] - top);
+    sum = fmaf(weight[w], part_l[w][r], sum);
+  }
+  const float inv = 1.f / sum;
+#pragma unroll
+  for (int j = wave; j < DT; j += W) {
+    f4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; ++w) o += weight[w] * part_o[w][j][lane];
+    if (tt < here) *reinterpret_cast<f4*>(out + (static_cast<size_t>(n) * n_heads + head) * D + 16 * j + 4 * g) = o * inv;
+  }
+}
+
+// Where the (token, head)s alone fill the GPU several times over, tiles of 16 columns (float32, sizes above) or a wave up to four heads
+// that share their keys; else (decoded tokens, short portions) eight waves share a head's keys.
 template <typename T>
 static void launch_generic(const T* q, int q_stride, T* out, const T* k_cache, const T* v_cache, const int32_t* positions,
                            const int32_t* token_seq, const int32_t* block_table, int table_width, int n_tokens, int page_size, int head_dim,
@@ -208,6 +356,18 @@ static void launch_generic(const T* q, int q_stride, T* out, const T* k_cache, c
   if (page_size % 4 != 0 || (reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) % 16 != 0)
     return with(attn_generic_kernel<T, 8, 1, false>, 8, 1);
   if (static_cast<long long>(n_tokens) * n_heads < 4096) return with(attn_generic_kernel<T, 8, 1, true>, 8, 1);
+  if constexpr (sizeof(T) == 4) {
+    if ((head_dim == 64 || head_dim == 128) && q_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(out)) % 16 == 0) {
+      int hpt = 16;
+      while (qpk % hpt != 0) hpt /= 2;
+      const dim3 grid((n_tokens + 16 / hpt - 1) / (16 / hpt), n_heads / hpt);
+      auto tiles = [&](auto kernel) {
+        kernel<<<grid, 256, 0, stream>>>(q, q_stride, out, k_cache, v_cache, positions, token_seq, block_table, table_width, page_size, n_tokens,
+                                         n_heads, n_kv, hpt, scale, window);
+      };
+      return head_dim == 64 ? tiles(attn_f32_tile_kernel<4, 4>) : tiles(attn_f32_tile_kernel<8, 4>);
+    }
+  }
   if (qpk % 4 == 0) return with(attn_generic_kernel<T, 1, 4, true>, 1, 4);
   if (qpk % 2 == 0) return with(attn_generic_kernel<T, 1, 2, true>, 1, 2);
   with(attn_generic_kernel<T, 1, 1, true>, 1, 1);
