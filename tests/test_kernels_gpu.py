@@ -554,6 +554,26 @@ def test_gemm_block_gated(ops, form, activation):
         assert bool((off <= 2**-7 * want.abs()[~(torch.isnan(want) | both_inf)] + 1e-37).all())
 
 
+# every form, rows and columns around its tiles
+@pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("kind", ["silu", "gelu_tanh", "relu2"])
+@pytest.mark.parametrize("m,n,k", [(129, 264, 640), (300, 8, 384), (257, 520, 384)])
+def test_linear_act_is_the_product_and_its_activation(ops, form, kind, m, n, k):
+    x, w = rnd((m, k), torch.bfloat16, 61), rnd((n, k), torch.bfloat16, 62) * 0.1
+    plan = form * 256 + 1
+    want = ops.activation(ops.gemm_block(x, w, torch.bfloat16, plan), kind, torch.bfloat16)
+    ops.force_block_plan(plan)
+    try:
+        got = ops.linear_act(x, w, kind, torch.bfloat16)
+    finally:
+        ops.force_block_plan()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    # few rows, float32 and a view that starts off 16 bytes: the product, then the activation
+    for a, b in ((x[:40], w), (x.float(), w.float()), (x[:, 4:], w[:, 4:])):
+        old = ops.activation(ops.linear(a, b, a.dtype, partial_ok=True), kind, a.dtype)
+        assert torch.equal(ops.linear_act(a, b, kind, a.dtype), old)
+
+
 def test_gemm_block_is_what_linear_takes(ops):
     """Where ``linear`` and ``gate_up_act`` take the product in large tiles by themselves, and that they agree with the kernels for other sizes."""
     from yalis_amd.ops.hip import SplitSum

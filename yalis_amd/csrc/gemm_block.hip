@@ -42,7 +42,7 @@ __device__ __forceinline__ void wait_for() {
   __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 7 << 4 | LGKM << 8);
 }
 
-enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GATED = 2 };
+enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GATED = 2, OUT_ACT = 3 };
 
 // x * sigmoid(slope * x), within two units of float32's last place: exp(y) as 2^(y log2 e) with the product's rounding carried along.
 __device__ __forceinline__ float swish(float x, float slope) {
@@ -240,12 +240,16 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void gemm_block_kernel(const bf16_
         if (mj < M && n < N)
           *reinterpret_cast<u32x4_t*>(y + n / 2) = u32x4_t{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]), pack_bf16x2(o[4], o[5]), pack_bf16x2(o[6], o[7])};
       }
-    } else if constexpr (OUT == OUT_BF16) {
+    } else if constexpr (OUT == OUT_BF16 || OUT == OUT_ACT) {
       bf16_t* const y = static_cast<bf16_t*>(yv) + static_cast<size_t>(mj) * ldy;
 #pragma unroll
       for (int i = 0; i < FN; i += 2) {
         const int n = nw + 16 * i + 8 * quarter;
-        const f32x4_t u = acc[i][j], v = acc[i + 1][j];
+        f32x4_t u = acc[i][j], v = acc[i + 1][j];
+        if constexpr (OUT == OUT_ACT) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) u[e] = act_plain(as_output(u[e], 1), kind), v[e] = act_plain(as_output(v[e], 1), kind);
+        }
         if (mj < M && n < N)
           *reinterpret_cast<u32x4_t*>(y + n) = u32x4_t{pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]), pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
       }
@@ -295,8 +299,8 @@ bool fits(const Form& f, int K, int slices) {
 }
 
 // The form and the slices of K for a product (form * 256 + slices), or -1 where the vendor library, or the kernels for fewer rows, do better.
-int plan(int M, int N, int K, bool partial, bool gated) {
-  if (M <= 64 || K % 64 || N % (gated ? 16 : 8)) return -1;
+int plan(int M, int N, int K, bool partial, bool gated, bool act) {
+  if (M <= (act ? 128 : 64) || K % 64 || N % (gated ? 16 : 8)) return -1;
   int best = -1, best_slices = 1, best_rounds = 1;
   float least = 1e30f;
   for (int i = 0; i < N_FORMS; ++i) {
@@ -319,7 +323,13 @@ int plan(int M, int N, int K, bool partial, bool gated) {
   // the part of the compute units' time that goes into y and not into tiles that hang over or units without one
   const float used = static_cast<float>(M) * N * best_slices / (static_cast<float>(best_rounds) * UNITS * f.fit * f.bn * f.bm);
   bool ours;
-  if (gated)
+  // With a pass over the product saved, library (or slices) and pass / here, us: 8,192 x 2,048, 129 rows 22.5 / 13.4, 512 24.6 / 21.2, 2,048
+  // 67.8 / 58.0, 4,096 126 / 111; 2,048 x 1,024 16.3 / 8.8, 22.2 / 9.2, 19.2 / 12.7, 27.7 / 22.8; 16,384 x 4,096 35.2 / 31.1, 63.0 / 58.3,
+  // 209 / 195, 415 / 399 (of 84 products one lost: 800 x 11,008 x 4,096 68.2 / 70.4).  Not where K is long and tiles are few, which slices
+  // help: 3,072 x 8,192 20.2 / 34.1, 33.6 / 36.4.
+  if (act)
+    ours = N >= 2048 && K <= N;
+  else if (gated)
     ours = N >= 2048 && (M <= 128 || used >= (M <= 256 ? 0.6f : M <= 720 ? 0.76f : 0.65f));
   else if (best_slices > 1)
     ours = N <= 5120 && M <= 1100 && best != 1 && (K >= 3072 || (M <= 128 ? K <= 1024 : M <= 256 && N <= 2560)) && (N >= 1024 || M <= 512);
@@ -336,7 +346,7 @@ int launch(int form, const bf16_t* x, const bf16_t* w, void* y, int M, int N, in
   const int room = UNITS * f.fit, rounds = (total + room - 1) / room, grid = std::min(room, ((total + rounds - 1) / rounds + 7) / 8 * 8);
   switch (form) {
     case 0:
-      if constexpr (OUT != OUT_GATED)
+      if constexpr (OUT != OUT_GATED && OUT != OUT_ACT)  // (whose ends need the registers of four waves more)
         gemm_block_kernel<256, 256, 2, 2, 1, 2, true, OUT><<<grid, 256, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1);
       else
         gemm_block_kernel<256, 256, 2, 4, 1, 2, true, OUT><<<grid, 512, 0, stream>>>(x, w, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1);
@@ -356,9 +366,10 @@ int g_force_block = -1;
 }  // namespace
 
 // The form and slices for a product as form * 256 + slices, -1: not this kernel's.  `partial`: slices may be handed on.
+// gated: 1 pairs, 2 an activation of every element.
 extern "C" int yk_gemm_block_plan(int M, int N, int K, int partial, int gated) {
   if (g_force_block != -1) return std::max(g_force_block, -1);
-  return plan(M, N, K, partial != 0, gated != 0);
+  return plan(M, N, K, partial != 0, gated == 1, gated == 2);
 }
 
 // For tests and measurements: the plan of every product (form * 256 + slices; -1: the rule; -2: nothing is this kernel's).
@@ -369,14 +380,16 @@ extern "C" int yk_gemm_block_force(int plan) {
 }
 
 // y [M, N] = x [M, K] . w [N, K]^T, bfloat16 operands, in the form and slices of `plan`.  out: 0 bfloat16, 1 float32 (`slices` > 1: the unreduced
-// slices [slices, M, N] one behind the other, ldy = N), 2 gated pairs of groups of eight columns, bfloat16 [M, N / 2] (kind, p0, p1: common.h).
+// slices [slices, M, N] one behind the other, ldy = N), 2 gated pairs of groups of eight columns, bfloat16 [M, N / 2] (kind, p0, p1: common.h), 3
+// bfloat16 with the activation `kind` (act_plain) of the rounded product.
 extern "C" int yk_gemm_block(const void* x, const void* w, void* y, int out, int M, int N, int K, int ldx, int ldw, int ldy, int plan, int kind,
                              float p0, float p1, hipStream_t stream) {
   const int form = plan / 256, slices = plan % 256;
   YK_REQUIRE(M > 0 && N > 0 && K > 0 && K % 64 == 0 && N % 8 == 0, "gemm_block: K is a multiple of 64, N of 8");
-  YK_REQUIRE(out >= 0 && out <= 2 && plan >= 0 && form < N_FORMS, "gemm_block: unknown output or form");
+  YK_REQUIRE(out >= 0 && out <= 3 && plan >= 0 && form < N_FORMS, "gemm_block: unknown output or form");
   YK_REQUIRE(!(out == OUT_GATED && (N % 16 || form == 1)), "gemm_block: gated pairs are groups of eight columns, and form 1 has none");
   YK_REQUIRE(out != OUT_GATED || (kind >= 0 && kind < YK_GATED_KINDS), "gemm_block: unknown activation");
+  YK_REQUIRE(out != OUT_ACT || (kind >= 0 && kind <= 2), "gemm_block: unknown activation");
   YK_REQUIRE(slices >= 1 && (slices == 1 || (out == OUT_F32 && ldy == N)), "gemm_block: slices are float32, one behind the other");
   YK_REQUIRE(fits(FORMS[form], K, slices), "gemm_block: a slice of K is too short");
   YK_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0 && ldx < 1 << 21 && ldw < 1 << 21, "gemm_block: rows of x and w");
@@ -387,6 +400,7 @@ extern "C" int yk_gemm_block(const void* x, const void* w, void* y, int out, int
   const auto* xb = static_cast<const bf16_t*>(x);
   const auto* wb = static_cast<const bf16_t*>(w);
   if (out == OUT_BF16) return launch<OUT_BF16>(form, xb, wb, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1, stream);
+  if (out == OUT_ACT) return launch<OUT_ACT>(form, xb, wb, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1, stream);
   if (out == OUT_F32) return launch<OUT_F32>(form, xb, wb, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1, stream);
   return launch<OUT_GATED>(form, xb, wb, y, M, N, K, ldx, ldw, ldy, slices, kind, p0, p1, stream);
 }

@@ -810,25 +810,26 @@ class HipOps:
             self._library_workspace.data_ptr(), self._library_workspace.numel(), None, self._stream()))
         return y
 
-    def _block_plan(self, x, w, partial_ok: bool, gated: bool = False) -> int:
-        """The form and slices in which a product of many rows of bfloat16 is ``gemm_block``'s, or -1."""
+    def _block_plan(self, x, w, partial_ok: bool, gated: int = 0) -> int:
+        """The form and slices in which a product of many rows of bfloat16 is ``gemm_block``'s, or -1; ``gated``: with its pairs (1) or an
+        activation of every element (2) made on the way."""
         if x.stride(0) >= 1 << 21 or w.stride(0) >= 1 << 21:
             return -1
         return self._ask("yk_gemm_block_plan", x.shape[0], w.shape[0], x.shape[1], int(partial_ok), int(gated))
 
-    def gemm_block(self, x, w, out_dtype, plan: int, gated=None):
+    def gemm_block(self, x, w, out_dtype, plan: int, gated=None, act=None):
         """x [M, K] . w [N, K]^T in large tiles (bfloat16 operands with 16-byte aligned rows, K a multiple of 64) in the form and
         slices of ``plan`` (form * 256 + slices): a tensor, or with slices a ``SplitSum``; ``gated``: pairs of groups of eight columns
         (see ``gated_kind``)."""
         m, k = x.shape
         n = w.shape[0]
-        kind, p0, p1 = (0, 0.0, 0.0) if gated is None else self.gated_kind(gated)
+        kind, p0, p1 = (0 if act is None else self.ACTIVATION_KINDS[act], 0.0, 0.0) if gated is None else self.gated_kind(gated)
         slices = plan % 256
         if slices > 1:
             y, out = self._gemm_ws(slices * m * n), 1
         else:
             y = torch.empty((m, n // 2 if gated is not None else n), dtype=out_dtype, device=x.device)
-            out = 2 if gated is not None else _OUT_CODES[out_dtype]
+            out = 2 if gated is not None else 3 if act is not None else _OUT_CODES[out_dtype]
         self._check(self.lib.yk_gemm_block(
             x.data_ptr(), w.data_ptr(), y.data_ptr(), out, m, n, k, x.stride(0), w.stride(0), n // 2 if gated is not None else n, plan, kind, p0, p1,
             self._stream()))
@@ -984,7 +985,7 @@ class HipOps:
             return self.gemm_cols(x, w_gate_up, bf, gated=activation)
         if (pairs and m > SKINNY_MAX_ROWS and x.dtype == bf and w_gate_up.dtype == bf and w_gate_up.shape[1] == k and w_gate_up.stride(1) == 1
                 and x.stride(0) % 8 == 0 and w_gate_up.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0):
-            plan = self._block_plan(x, w_gate_up, False, gated=True)
+            plan = self._block_plan(x, w_gate_up, False, gated=1)
             if plan >= 0:
                 return self.gemm_block(x, w_gate_up, bf, plan, gated=activation)
         if not fused:
@@ -1712,6 +1713,18 @@ class HipOps:
         self._check(self.lib.yk_activation(src.data_ptr(), _code(src.dtype), n_splits, round_sum, self.ACTIVATION_KINDS[kind],
                                            out.data_ptr(), _code(out_dtype), out.numel(), self._stream()))
         return out
+
+    def linear_act(self, x, w, kind: str, out_dtype: torch.dtype) -> torch.Tensor:
+        """act(x . w^T) of the product rounded to ``out_dtype``: many rows of bfloat16 in one kernel where ``gemm_block`` takes the product, else
+        ``linear`` and ``activation``."""
+        bf = torch.bfloat16
+        if (kind in self.ACTIVATION_KINDS and isinstance(x, torch.Tensor) and x.dim() == 2 and w.dim() == 2 and x.shape[0] > SKINNY_MAX_ROWS
+                and x.dtype == bf and w.dtype == bf and out_dtype == bf and w.shape[1] == x.shape[1] and x.stride(1) == 1 and w.stride(1) == 1
+                and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
+            plan = self._block_plan(x, w, False, gated=2)
+            if plan >= 0 and plan % 256 == 1:
+                return self.gemm_block(x, w, bf, plan, act=kind)
+        return self.activation(self.linear(x, w, out_dtype, partial_ok=True), kind, out_dtype)
 
     def scale_rows(self, x: torch.Tensor, s: float, softcap: float = 0.0) -> torch.Tensor:
         """x (contiguous float32) *= s, in place; with ``softcap`` c, x = c tanh(s x / c)."""
