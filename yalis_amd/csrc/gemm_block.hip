@@ -329,8 +329,13 @@ int plan(int M, int N, int K, bool partial, bool gated, bool act) {
   // help: 3,072 x 8,192 20.2 / 34.1, 33.6 / 36.4.
   if (act)
     ours = N >= 2048 && K <= N;
+  // Not where the library's product of the same tiles of 256 x 256 gains more than its pass for the pairs costs: long and wide matrices (us, library
+  // and pass / here: 28,672 x 4,096, 1,300 rows 275 / 289, 2,048 378 / 396, 57,344 x 8,192 1,032 / 1,091, 1,316 / 1,382; from 2,560 rows on
+  // 581 / 574, 982 / 871; 24,576 x 4,096 304.5 / 303.9 at 2,048), and a third time round for few tiles where its own fit (24,576 x 4,096, 1,536 rows
+  // 258 / 266, 12,288 x 2,048, 3,000 rows 146 / 151).
   else if (gated)
-    ours = N >= 2048 && (M <= 128 || used >= (M <= 256 ? 0.6f : M <= 720 ? 0.76f : 0.65f));
+    ours = N >= 2048 && !(best == 0 && N > 24576 && K >= 4096 && M <= 2560) &&
+           (M <= 128 || used >= (M <= 256 ? 0.6f : M <= 720 ? 0.76f : best == 0 && best_rounds == 3 && N % 1024 == 0 ? 0.77f : 0.65f));
   else if (best_slices > 1)
     ours = N <= 5120 && M <= 1100 && best != 1 && (K >= 3072 || (M <= 128 ? K <= 1024 : M <= 256 && N <= 2560)) && (N >= 1024 || M <= 512);
   else
