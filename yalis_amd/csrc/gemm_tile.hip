@@ -5,7 +5,7 @@
 // layer (512 rows x 3,072 columns: 24 to 48 tiles for 256 compute units), which this kernel
 // answers with tiles of 128 x 128 cut along K as well (the unreduced K slices go to the same
 // consumers that add the few-row product's slices).  What it wins, and so what it is used for
-// (HipOps.mid_rows_product): 65 to 256 rows against matrices at least twice as long as wide,
+// (HipOps.long_matrix_tiles; gemm_block.hip has the larger tiles): 65 to 256 rows against matrices at least twice as long as wide,
 // the down projections (us at 128 rows, vendor library's first candidate / few-row kernel / this:
 // 8B shape 57.9 / 35.4 / 27.0, 3B 32.9 / 19.6 / 17.7, 70B 200 / 167 / 110).  From 384 rows on, and
 // for gate/up at any number of rows, the library is faster (8B shape at 512 rows, library / this:

@@ -1,4 +1,4 @@
-// Products of many rows: y = x . w^T in the vendor library (hipBLASLt), called directly.
+// Products of many rows: y = x . w^T in the vendor library (hipBLASLt), called directly (those that gemm_block.hip does not take).
 // The reference hands the same products to its vendor library (yalis/external/model.py:449,
 // 462-466, 717-722).  What this file adds to a plain library call: the descriptors and the
 // chosen algorithm of every shape are kept, so that a call costs the host a few microseconds

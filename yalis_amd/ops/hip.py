@@ -690,7 +690,8 @@ class HipOps:
         sizes are ``gemm_cols``'s (``yk_gemm_cols_ok``).  A product has the same bits whole, as slices, with a bias added
         afterwards or in ``gate_up_act`` where it is ``gemm_cols``'s even as slices (most products of up to 8 rows, 6.5 M elements
         of w and 1,024 rows of w or more) and where it is never (fewer rows of w, more than 16 of x, large matrices); between
-        these only up to rounding."""
+        these only up to rounding.  More than 64 rows of bfloat16 are ``gemm_block``'s, ``gemm_tile``'s or the vendor library's by size
+        and by whether slices will do; float32 is ``gemm_fma``'s."""
         if bias is not None:
             if isinstance(x, torch.Tensor):
                 self._rows(x, "linear input")
@@ -752,7 +753,8 @@ class HipOps:
         (3,072 x 8,192) at 128 32.9 / 19.6 / 17.7, at 192 45.3 / 27.5 / 28.5; 70B (8,192 x 28,672) at
         128 200 / 167 / 110, at 256 314 / - / 200; 1B (2,048 x 8,192) at 192 22.9 / 19.7 / 18.2.  On
         squarer matrices the three are within a tenth of each other up to 128 rows, and from 384
-        rows on the library wins everywhere."""
+        rows on the library wins everywhere.  Where the consumer adds slices (``slices_do``) ``gemm_block`` in slices is faster from 129
+        rows on unless K is four times N or more."""
         return SKINNY_MAX_ROWS < m <= (128 if slices_do and k < 4 * n else 256) and k >= 2 * n and k >= 4096
 
     @staticmethod
@@ -764,7 +766,7 @@ class HipOps:
         128 rows: o-proj 13.8 / 15.3, down-proj 38.7 / 52.1, but qkv 23.7 / 16.6 and gate/up
         96 / 58; at 160 rows o-proj 20.2 / 16.4, down-proj 65.6 / 58.7.  3B shapes at 128 rows:
         o-proj 10.9 / 11.4, down-proj 20.6 / 22.9, qkv 13.7 / 13.2.  So: up to 128 rows and up to
-        4,096 columns."""
+        4,096 columns (of what ``gemm_block`` does not take)."""
         return m <= 128 and -(-n // 256) <= 16
 
     def _linear_from_attention(self, x: "SplitAttention", w: torch.Tensor, out_dtype, partial_ok: bool):
