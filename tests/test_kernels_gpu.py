@@ -554,6 +554,31 @@ def test_gemm_block_gated(ops, form, activation):
         assert bool((off <= 2**-7 * want.abs()[~(torch.isnan(want) | both_inf)] + 1e-37).all())
 
 
+@pytest.mark.parametrize("form", [0, 2, 3, 4])
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"] + [("clamped_swish", 7.0, s) for s in (-1.702, 0.0, 1.0, 1.25, 1.5, 1.6, 1.7, 1.702, 2.0)])
+def test_gemm_block_gated_of_every_gate(ops, form, activation):
+    """Every finite bfloat16 as a gate, and twice it (infinities among these): row i of x holds one 1 or 2 that picks element i of w's rows."""
+    bits = torch.arange(1 << 16).view(128, 512)
+    bits[(bits & 0x7F80) == 0x7F80] = 0  # (0 times what is no finite number would be no number in every row)
+    gate = torch.zeros((512, 512), dtype=torch.bfloat16)
+    gate[:, :128] = bits.to(torch.int16).view(torch.bfloat16).T
+    up = torch.zeros_like(gate)
+    up[:, :128] = torch.tensor([1.5, -3.0, 0.75, -1.0]).repeat(128)[:, None]
+    x = torch.zeros((256, 512), dtype=torch.bfloat16)
+    x[torch.arange(256), torch.arange(256) % 128] = torch.tensor([1.0, 2.0]).repeat_interleave(128).to(torch.bfloat16)
+    w, group = ops.pack_gate_up(gate.to(DEV), up.to(DEV))
+    gu = ops.gemm_block(x.to(DEV), w, torch.bfloat16, form * 256 + 1)
+    seen, normal = gu.cpu().view(256, 64, 2, 8)[:128, :, 0].reshape(128, 512), gate[:, :128].T.abs() >= 2.0**-126  # (others may come as zeros)
+    assert torch.equal(seen[normal], gate[:, :128].T[normal])
+    want = ops.gated_act(gu, activation, torch.bfloat16, group=group).float()
+    got = ops.gemm_block(x.to(DEV), w, torch.bfloat16, form * 256 + 1, gated=activation).float()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(torch.signbit(got) | got.isnan(), torch.signbit(want) | want.isnan())
+    # a unit of bfloat16 where the float32 values straddle a rounding, at its smallest numbers one of 2^-133
+    off = (got - want).abs()[torch.isfinite(want)]
+    assert bool((off <= 2**-7 * want.abs()[torch.isfinite(want)] + 2.0**-133).all())
+
+
 # every form, rows and columns around its tiles
 @pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
 @pytest.mark.parametrize("kind", ["silu", "gelu_tanh", "relu2"])

@@ -44,12 +44,17 @@ __device__ __forceinline__ void wait_for() {
 
 enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GATED = 2, OUT_ACT = 3 };
 
-// x * sigmoid(slope * x), within two units of float32's last place: exp(y) as 2^(y log2 e) with the product's rounding carried along.
+// x * sigmoid(slope * x), within about three units of float32's last place: exp(y) as 2^(y log2 e) with the product's rounding carried
+// along, unless the power is infinite (or y no number), which has no rest: the result is then zero (or no number), as a division's would be.
+// A quarter of the divisor, so that its reciprocal is no subnormal number, which the instruction gives as zero.
 __device__ __forceinline__ float swish(float x, float slope) {
-  const float y = fminf(fmaxf(-slope * x, -90.f), 90.f), t = y * 1.44269504f;
+  float y = -slope * x;
+  y = y < -90.f ? -90.f : y;
+  const float t = y * 1.44269504f;
   const float low = fmaf(y, 1.92596303e-8f, fmaf(y, 1.44269504f, -t));
   const float e = __builtin_amdgcn_exp2f(t);
-  return x * __builtin_amdgcn_rcpf(1.f + fmaf(e, low * 0.693147181f, e));
+  const float power = t < 128.f ? fmaf(e, low * 0.693147181f, e) : e;
+  return 0.25f * x * __builtin_amdgcn_rcpf(fmaf(0.25f, power, 0.25f));
 }
 __device__ __forceinline__ float gated(float g, float u, int kind, float p0, float p1) {
   if (kind == 0) return swish(g, 1.f) * u;
