@@ -327,7 +327,7 @@ def breakdown(runner, shape: Shape, gen, batch: int, prompt_len: int, prefill_le
     from yalis_amd.engine.step import StepEntry
 
     ops = runner.rt.ops
-    kinds = {"linear": "products", "gate_up_act": "products", "gemm_mfma_skinny": None, "gemm_fma": None,
+    kinds = {"linear": "products", "gate_up_act": "products", "linear_act": "products", "gemm_mfma_skinny": None, "gemm_fma": None,
              "attention": "attention", "rope_append": "attention", "add_rmsnorm": "norms", "gather_add_rmsnorm": "norms",
              "gated_act": "activation", "embed": "other", "argmax": "other"}
     spans, depth, head_rows = [], [0], shape.vocab
@@ -511,7 +511,7 @@ def _op_costs(ops, hb):
     def moved(a, kw, out):
         return 0.0, float(nbytes(*a, *kw.values()) + (nbytes(out) if hasattr(out, "numel") else 0))
 
-    return {"linear": linear, "gate_up_act": linear, "moe_experts": moe, "attention_masked": attention_masked, "attention": attention,
+    return {"linear": linear, "gate_up_act": linear, "linear_act": linear, "moe_experts": moe, "attention_masked": attention_masked, "attention": attention,
             "rglru": rglru, "norm_add": moved, "add_rmsnorm": moved, "gather_add_rmsnorm": moved, "qkv_prepare": moved,
             "rope_append": moved, "causal_conv": moved, "gated_act": moved, "round_rows": moved, "embed": embed,
             "sandwich_norm": moved, "activation": moved, "latent_prepare": moved, "head_linear": head_linear,
