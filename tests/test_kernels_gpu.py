@@ -192,6 +192,30 @@ def test_gemm_split_of_numbers_at_the_limits(ops, slices):
     assert bool(((got.double() - want).abs() <= bound)[rest].all())
 
 
+# sums that are finite, but not when their operands are scaled: all of them, and those of one column; a short last piece of K
+@pytest.mark.parametrize("k,slices", [(4096, 1), (4100, 1), (8192, 3), (2060, 1), (20, 1)])
+def test_gemm_split_of_large_sums(ops, k, slices):
+    x, w = rnd((70, k), torch.float32, 53), rnd((140, k), torch.float32, 54)
+    for all_large in (True, False):
+        a, b = x.clone(), w.clone()
+        (a if all_large else b[7])[:] *= 2.0**90
+        (b[7] if all_large else a[5])[:] *= 2.0**20
+        want = a.double().cpu() @ b.double().cpu().T
+        # in units of what a sum is large: 16 products are added one by one, the lanes' K / 1,024 sums of them (a lane's), and the lanes' in 6
+        # steps, every addition rounded by at most 2^-24 of what it gives (on average half of that): in all of less than a sum's
+        # size times sqrt(8 + K / 2,048 + 6) / 2; and the matrix cores' sums as above
+        size = a.double().cpu().norm(dim=1)[:, None] * b.double().cpu().norm(dim=1)[None] / math.sqrt(k)
+        off = ((ops.gemm_split(a, b, slices).double().cpu() - want) / size).square().mean().sqrt()
+        assert off <= 1.5 * math.sqrt(14 + k / 2048) / 2 * 2.0**-24, off
+        if k >= 2048:  # and it is what the float32 instructions give, or better
+            ops.force_float32_form(4)
+            try:
+                other = ((ops.gemm_fma(a, b, torch.float32).double().cpu() - want) / size).square().mean().sqrt()
+            finally:
+                ops.force_float32_form()
+            assert off <= 1.1 * other, (off, other)
+
+
 def test_gemm_split_is_what_float32_products_of_many_rows_are(ops):
     for m, n, k, taken in [(33, 3072, 2048, True), (511, 2048, 8192, True), (64, 512, 512, False), (32, 3072, 2048, False)]:
         x, w = rnd((m, k), torch.float32, 49), rnd((n, k), torch.float32, 50)

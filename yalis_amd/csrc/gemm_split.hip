@@ -10,7 +10,8 @@
 //
 // us, before (float32 instructions) / now: 511 x 16,384 x 2,048 314 / 209 (164 TFLOP/s), 511 x 3,072 x 2,048 78 / 52, 511 x 2,048 x 2,048
 // 42.6 / 36.7, 511 x 2,048 x 8,192 160 / 115, 2,000 x 6,144 x 4,096 915 / 547 (184), 200 x 16,384 x 2,048 160 / 94, 64 x 2,048 x 8,192
-// 101 / 29, 33 x 3,072 x 2,048 28 / 17.
+// 101 / 29, 33 x 3,072 x 2,048 28 / 17.  With one row of x that makes infinities, NaN or sums beyond 2^80 (below): 511 x 16,384 x 2,048 317, 511 x
+// 2,048 x 8,192 183, 200 x 3,072 x 2,048 59 (34 without); with all of them so 10.0, 5.0 and 1.5 ms, by a lane for each element 30, 15 and 3.8.
 // What bounds it: the largest is held by the matrix cores (50% busy) and the vector instructions that take w apart (30%) at 2.0 GHz, which
 // is what power leaves; LDS reads are 25%.  Splitting both operands in the kernel through LDS took 200 to 250 us there and 66 to 94 on 511 x
 // 3,072 x 2,048.
@@ -208,6 +209,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(const bf16_t* __rest
   }
   __builtin_amdgcn_s_waitcnt(0);  // no load may still be on its way into LDS
   // lane l holds columns 4 (l / 16) .. + 3 of row l % 16
+  uint32_t again = 0;  // bit 16 i + 4 j + e
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -218,15 +220,7 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(const bf16_t* __rest
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         o[e] = (acc[i][j][e] + rest[i][j][e]) * (1.f / SCALE) * (1.f / SCALE);
-        if (!(fabsf(o[e]) <= 3.402823466e38f) && n + e < N) {
-          // An infinity has no rest, and neither has a number that is one when scaled or rounded: what such operands give is made of them
-          // as they are.
-          float v = 0.f;
-          const float* const xm = x + static_cast<size_t>(mi) * ldx;
-          const float* const wv = w + static_cast<size_t>(n + e) * ldw;
-          for (int k = s0 * 32; k < min(K, (s0 + steps) * 32); ++k) v = fmaf(xm[k], wv[k], v);
-          o[e] = v;
-        }
+        if (!(fabsf(o[e]) <= 3.402823466e38f) && n + e < N) again |= 1u << (16 * i + 4 * j + e);
       }
       float* const to = y + static_cast<size_t>(mi) * ldy + n;
       if (vector && n + 3 < N) {
@@ -237,6 +231,33 @@ __global__ __launch_bounds__(256, 2) void gemm_split_kernel(const bf16_t* __rest
           if (n + e < N) to[e] = o[e];
       }
     }
+  // An infinity has no rest, and neither has a number that is one when scaled or rounded: what such operands give is made of them as they
+  // are, an element at a time by the whole wave: sums of 16 products, added up along K by each lane and then over the lanes.
+  const int k0 = s0 * 32, k1 = min(K, k0 + steps * 32);
+  for (uint64_t lanes = __ballot(again != 0); lanes != 0; lanes = __ballot(again != 0)) {
+    const int from = __builtin_ctzll(lanes);
+    const int which = __builtin_ctz(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(again), from)));
+    const int mi = m0 + which / 4 % 4 * 16 + from % 16, n = n0 + wave * 32 + which / 16 * 16 + from / 16 * 4 + which % 4;
+    const float* const xm = x + static_cast<size_t>(mi) * ldx;
+    const float* const wv = w + static_cast<size_t>(n) * ldw;
+    float v = 0.f;
+    for (int k = k0 + 16 * lane; k < k1; k += 16 * 64) {
+      float sum = 0.f;
+#pragma unroll
+      for (int p = 0; p < 16; p += 4) {
+        if (k + p >= k1) break;  // (K is a multiple of four)
+        const f32x4_t a4 = *reinterpret_cast<const f32x4_t*>(xm + k + p), b4 = *reinterpret_cast<const f32x4_t*>(wv + k + p);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum = fmaf(a4[e], b4[e], sum);
+      }
+      v += sum;
+    }
+    v = wave_sum(v);
+    if (lane == from) {
+      y[static_cast<size_t>(mi) * ldy + n] = v;
+      again &= again - 1;
+    }
+  }
 }
 
 // y [M, N] of slices [slices][M][N], added in order; four elements a thread (count = M N of a multiple of four, y rows N apart)
