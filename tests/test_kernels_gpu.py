@@ -1024,6 +1024,17 @@ def test_attention_float32_tiles(ops, h, g, d, page, window):
     close(got, want, 2e-5, 1e-5)
 
 
+# a tile's requests shared out among workgroups (many requests of few tokens, one of them behind many keys): 16, 8 and 4 shares, tiles that hang over
+@pytest.mark.parametrize("h,g,d,page", [(45, 15, 128, 32), (40, 20, 64, 8), (48, 12, 64, 64), (45, 15, 64, 20)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_attention_float32_tiles_of_many_requests(ops, h, g, d, page, window):
+    spans = [(260 + i if i % 9 == 0 else 7 * i % 40, 1 + (i % 5 == 4)) for i in range(90)]
+    n = sum(new for _, new in spans)
+    assert ops._ask("yk_attn_f32_form", n, h, g, len(spans), 1, max(a + b for a, b in spans), 0) == 2
+    got, want = _attention_case(ops, torch.float32, h, g, d, page, spans, window, 22, n_pages=900)
+    close(got, want, 2e-5, 1e-5)
+
+
 @pytest.mark.parametrize("window", [0, 9])
 def test_attention_float32_tiles_keep_later_values_from_earlier_tokens(ops, window):
     n, h, g, d, page, gen = 70, 64, 16, 64, 16, torch.Generator().manual_seed(21)

@@ -1,0 +1,21 @@
+"""Which kernel takes a call: the rules of the kernel library that need no GPU to be asked."""
+import pytest
+
+from yalis_amd.ops.build import load_kernels
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return load_kernels()
+
+
+# tokens, heads, kv heads, requests, tokens of the longest span, keys, window
+@pytest.mark.parametrize("step,form", [
+    ((128, 32, 32, 128, 1, 20, 0), 0), ((128, 32, 32, 128, 1, 256, 0), 0), ((128, 32, 8, 128, 1, 2000, 64), 0),  # few keys: a wave a token
+    ((200, 32, 8, 100, 2, 2, 0), 1),  # (two tokens of four heads fill half a tile)
+    ((128, 32, 32, 128, 1, 300, 0), 2), ((128, 32, 8, 128, 1, 2000, 0), 2), ((231, 32, 32, 32, 200, 301, 0), 2), ((180, 32, 16, 60, 3, 203, 0), 2),
+    ((352, 32, 32, 352, 1, 300, 0), 1), ((128, 32, 4, 128, 1, 2000, 0), 1), ((500, 32, 32, 100, 5, 5, 0), 1),
+    ((2000, 32, 32, 1, 2000, 2000, 0), 1), ((8320, 32, 8, 64, 130, 130, 0), 1), ((1, 4096, 4096, 1, 1, 300, 0), 1),
+])
+def test_float32_attention_of_several_requests(lib, step, form):
+    assert lib.yk_attn_f32_form(*step) == form

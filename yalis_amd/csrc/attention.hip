@@ -198,11 +198,12 @@ __global__ __launch_bounds__(64 * W) void attn_generic_kernel(
 // pieces of 16 bytes): 16 columns, some heads that share a key/value head of neighbouring tokens, to a workgroup whose W waves take blocks of
 // 16 keys by turns and merge at the end.  Lane (r, g) holds elements 16 j + 4 g .. + 3 of key r and of column r's query, then keys
 // 4 g .. + 3 of element 16 t + r: the scores leave the first product as the second takes them, nothing passes LDS.  Tokens of several requests
-// in one workgroup are walked a request at a time, the others' columns masked.  The sums of a block's 16 products join the running sums at once.
+// in one workgroup are walked a request at a time, the others' columns masked; SHARED: the gridDim.z workgroups of a tile take every
+// gridDim.z-th of its requests.  The sums of a block's 16 products join the running sums at once.
 // Bound by the latency of the loads.  32 heads of 64 over 8 kv heads, us (as a wave a token and four heads): 511 tokens of two prompts 22
-// (69), 2,048 of one 296 (1,283), 128 behind 1,000 35 (143), 128 requests of one token behind 300 47 (48); of 128, two prompts of 300 47 (148).
+// (69), 2,048 of one 296 (1,283), 128 behind 1,000 35 (143), 128 requests of one token behind 300 37 (48; shared); of 128, two prompts of 300 47 (148).
 // Error against 64 bits 1.3e-7, 2.0e-7 and 1.7e-7 of the first, the third and the fourth's size (1.7e-7, 6.1e-7, 3.4e-7).
-template <int DT, int W>
+template <int DT, int W, bool SHARED>
 __global__ __launch_bounds__(64 * W) void attn_f32_tile_kernel(const float* __restrict__ q, int q_stride, float* __restrict__ out,
                                                                const float* __restrict__ k_cache, const float* __restrict__ v_cache,
                                                                const int32_t* __restrict__ positions, const int32_t* __restrict__ token_seq,
@@ -215,7 +216,15 @@ __global__ __launch_bounds__(64 * W) void attn_f32_tile_kernel(const float* __re
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), r = lane % 16, g = lane / 16;
   const bool tiled = cache_is_tiled(YK_F32, D, page_size);
   const size_t slab = static_cast<size_t>(page_size) * D;
-  const int tpt = 16 / hpt, first = blockIdx.x * tpt, here = min(tpt, n_tokens - first), h0 = blockIdx.y * hpt, kv = h0 / (n_heads / n_kv);
+  // (the dies take workgroups by turns: the shares of one tile are not all to be one die's)
+  const int shares = SHARED ? gridDim.z : 1, share = blockIdx.z, tile = SHARED ? (blockIdx.x + share) % gridDim.x : blockIdx.x;
+  const int tpt = 16 / hpt, first = tile * tpt, here = min(tpt, n_tokens - first), h0 = blockIdx.y * hpt, kv = h0 / (n_heads / n_kv);
+  uint64_t begins = 0;  // bit t: token t begins a run of tokens of one request
+  if constexpr (SHARED) {
+    const int of = token_seq[first + min(lane, here - 1)], before = __shfl(of, max(lane - 1, 0), 64);
+    begins = __ballot(lane < here && (lane == 0 || of != before));
+    if (__popcll(begins) <= share) return;
+  }
   const int tt = r / hpt, n = first + min(tt, here - 1), head = h0 + r % hpt;
   const int pos = positions[n], my_lo = window > 0 ? max(0, pos - window + 1) : 0;
   f4 qf[DT], acc[DT];
@@ -225,17 +234,25 @@ __global__ __launch_bounds__(64 * W) void attn_f32_tile_kernel(const float* __re
     acc[j] = f4{0.f, 0.f, 0.f, 0.f};
   }
   float m = -INFINITY, l = 0.f;
-  for (int t0 = 0; t0 < here;) {
-    // the tokens from t0 on that are of its request, and the keys they see
+  bool taken = !SHARED && tt < here;
+  for (int run = 0, t0, t1 = 0; t1 < here; ++run) {
+    // the tokens from t0 up to t1 are of one request; the keys they see
+    t0 = t1;
+    if constexpr (SHARED) {
+      begins &= begins - 1;
+      t1 = begins != 0 ? __builtin_ctzll(begins) : here;
+      if (run % shares != share) continue;
+    }
     const int seq = token_seq[first + t0];
-    int t1 = t0, hi = 0, lo = INT_MAX;
-    for (; t1 < here && token_seq[first + t1] == seq; ++t1) {
-      const int p = positions[first + t1];
+    int hi = 0, lo = INT_MAX, t = t0;
+    for (; SHARED ? t < t1 : t < here && token_seq[first + t] == seq; ++t) {
+      const int p = positions[first + t];
       hi = max(hi, p + 1);
       lo = min(lo, window > 0 ? max(0, p - window + 1) : 0);
     }
+    t1 = t;
     const bool mine = tt >= t0 && tt < t1;
-    t0 = t1;
+    if constexpr (SHARED) taken = taken || mine;
     const int32_t* bt = block_table + static_cast<size_t>(seq) * table_width;
     for (int key0 = (lo / 16 + wave) * 16; key0 < hi; key0 += 16 * W) {
       f4 k4[DT], v4[DT];
@@ -338,16 +355,45 @@ __global__ __launch_bounds__(64 * W) void attn_f32_tile_kernel(const float* __re
     f4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < W; ++w) o += weight[w] * part_o[w][j][lane];
-    if (tt < here) *reinterpret_cast<f4*>(out + (static_cast<size_t>(n) * n_heads + head) * D + 16 * j + 4 * g) = o * inv;
+    if (taken) *reinterpret_cast<f4*>(out + (static_cast<size_t>(n) * n_heads + head) * D + 16 * j + 4 * g) = o * inv;
   }
 }
 
-// Where the (token, head)s alone fill the GPU several times over, tiles of 16 columns (float32, sizes above) or a wave up to four heads
-// that share their keys; else (decoded tokens, short portions) eight waves share a head's keys.
+// How many (token, head)s of float32 with head sizes 64 and 128 go: 0 a wave a token, 1 in tiles, 2 in tiles whose requests are shared out
+// among workgroups.  A tile's 16 columns are `hpt` heads of neighbouring tokens, of which a request's tokens fill some; it walks one request
+// after the other.  Tiles as they are where a request fills half of one, and where they alone fill the GPU: from there on the shares' columns
+// without a token cost what they save.  Else the tile's requests go to workgroups of their own, unless keys are few, where a wave a
+// token has the least to start and to merge.  us, a wave a token / tiles / shared (head size 64, 32 heads over 32 and over 8 kv heads): 128 requests
+// of one token behind 20 16 / 37 / 36 and 8.2 / 9.6 / 10, behind 300 163 / 244 / 143 and 48 / 47 / 37, behind 2,000 1,067 / 1,519 / 780 and 397 / 385 /
+// 262; 352 behind 20 30 / 49 / 87 and 13 / 16 / 23, behind 300 467 / 359 / 380 and 123 / 92 / 99; 31 behind 300 and a prompt of 200 83 / 202 / 48 and 47 /
+// 46 / 24; 60 requests of 3 tokens behind 200 119 / 65 / 48 and 43 / 24 / 18; 100 prompts of 5 27 / 25 / 35 and 12 / 11 / 14, 64 of 130 1,215 / 195 /
+// 346 and 370 / 168 / 197.  Over 461 such steps the rule takes 0.60 of the first form's time (the worst 1.28: 200 prompts of 2 tokens, 9.6 / 12.3) and
+// 0.83 of that of tiles alone.
+static int f32_form(int n_tokens, int n_heads, int hpt, int n_seqs, int longest, int max_ctx, int window) {
+  const int tpt = 16 / hpt, workgroups = (n_tokens + tpt - 1) / tpt * (n_heads / hpt), reach = window > 0 ? std::min(window, max_ctx) : max_ctx;
+  const int rest = n_seqs > 1 ? (n_tokens - longest) / (n_seqs - 1) : n_tokens;  // a request's tokens, the longest span apart
+  if (hpt * rest >= 8) return 1;
+  if (reach <= 64) return hpt * rest <= 4 ? 0 : 1;
+  if (longest > 1) return 2;
+  return workgroups >= 512 ? 1 : reach <= 256 ? 0 : 2;  // (256: what a captured step of few keys is launched for)
+}
+static int f32_heads_per_tile(int qpk) {
+  int hpt = 16;
+  while (qpk % hpt != 0) hpt /= 2;
+  return hpt;
+}
+// For tests: the form of a step of so many (token, head)s.
+extern "C" int yk_attn_f32_form(int n_tokens, int n_heads, int n_kv, int n_seqs, int longest, int max_ctx, int window) {
+  YK_REQUIRE(n_kv > 0 && n_heads % n_kv == 0, "attention: the head count must be a multiple of the kv head count");
+  return f32_form(n_tokens, n_heads, f32_heads_per_tile(n_heads / n_kv), n_seqs, longest, max_ctx, window);
+}
+
+// Where the (token, head)s alone fill the GPU several times over, tiles (float32, above) or a wave up to four heads that share their keys;
+// else (decoded tokens, short portions) eight waves share a head's keys.
 template <typename T>
 static void launch_generic(const T* q, int q_stride, T* out, const T* k_cache, const T* v_cache, const int32_t* positions,
                            const int32_t* token_seq, const int32_t* block_table, int table_width, int n_tokens, int page_size, int head_dim,
-                           int n_heads, int n_kv, float scale, int window, hipStream_t stream) {
+                           int n_heads, int n_kv, float scale, int window, int n_seqs, int longest, int max_ctx, hipStream_t stream) {
   const int qpk = n_heads / n_kv;
   auto with = [&](auto kernel, int waves, int heads) {
     kernel<<<dim3(n_tokens, n_heads / heads), 64 * waves, 0, stream>>>(q, q_stride, out, k_cache, v_cache, positions, token_seq, block_table,
@@ -358,14 +404,13 @@ static void launch_generic(const T* q, int q_stride, T* out, const T* k_cache, c
   if (static_cast<long long>(n_tokens) * n_heads < 4096) return with(attn_generic_kernel<T, 8, 1, true>, 8, 1);
   if constexpr (sizeof(T) == 4) {
     if ((head_dim == 64 || head_dim == 128) && q_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(out)) % 16 == 0) {
-      int hpt = 16;
-      while (qpk % hpt != 0) hpt /= 2;
-      const dim3 grid((n_tokens + 16 / hpt - 1) / (16 / hpt), n_heads / hpt);
+      const int hpt = f32_heads_per_tile(qpk), tpt = 16 / hpt, form = f32_form(n_tokens, n_heads, hpt, n_seqs, longest, max_ctx, window);
       auto tiles = [&](auto kernel) {
-        kernel<<<grid, 256, 0, stream>>>(q, q_stride, out, k_cache, v_cache, positions, token_seq, block_table, table_width, page_size, n_tokens,
-                                         n_heads, n_kv, hpt, scale, window);
+        kernel<<<dim3((n_tokens + tpt - 1) / tpt, n_heads / hpt, form == 2 ? tpt : 1), 256, 0, stream>>>(
+            q, q_stride, out, k_cache, v_cache, positions, token_seq, block_table, table_width, page_size, n_tokens, n_heads, n_kv, hpt, scale, window);
       };
-      return head_dim == 64 ? tiles(attn_f32_tile_kernel<4, 4>) : tiles(attn_f32_tile_kernel<8, 4>);
+      if (form == 2) return head_dim == 64 ? tiles(attn_f32_tile_kernel<4, 4, true>) : tiles(attn_f32_tile_kernel<8, 4, true>);
+      if (form == 1) return head_dim == 64 ? tiles(attn_f32_tile_kernel<4, 4, false>) : tiles(attn_f32_tile_kernel<8, 4, false>);
     }
   }
   if (qpk % 4 == 0) return with(attn_generic_kernel<T, 1, 4, true>, 1, 4);
@@ -377,7 +422,7 @@ extern "C" int yk_attn_generic(const void* q, int q_stride, void* out, const voi
                                const void* v_cache, int dtype, const int32_t* positions,
                                const int32_t* token_seq, const int32_t* block_table,
                                int table_width, int n_tokens, int page_size, int head_dim,
-                               int n_heads, int n_kv, float scale, int window,
+                               int n_heads, int n_kv, float scale, int window, int n_seqs, int longest, int max_ctx,
                                hipStream_t stream) {
   YK_REQUIRE(n_tokens >= 0 && n_heads > 0 && n_kv > 0, "attention: bad sizes");
   YK_REQUIRE(n_heads % n_kv == 0, "attention: the head count must be a multiple of the kv head count");
@@ -390,11 +435,11 @@ extern "C" int yk_attn_generic(const void* q, int q_stride, void* out, const voi
   if (dtype == YK_F32)
     launch_generic(static_cast<const float*>(q), q_stride, static_cast<float*>(out), static_cast<const float*>(k_cache),
                    static_cast<const float*>(v_cache), positions, token_seq, block_table, table_width, n_tokens, page_size, head_dim, n_heads,
-                   n_kv, scale, window, stream);
+                   n_kv, scale, window, n_seqs, longest, max_ctx, stream);
   else if (dtype == YK_BF16)
     launch_generic(static_cast<const bf16_t*>(q), q_stride, static_cast<bf16_t*>(out), static_cast<const bf16_t*>(k_cache),
                    static_cast<const bf16_t*>(v_cache), positions, token_seq, block_table, table_width, n_tokens, page_size, head_dim, n_heads,
-                   n_kv, scale, window, stream);
+                   n_kv, scale, window, n_seqs, longest, max_ctx, stream);
   else
     return yk_fail("attention: unsupported dtype");
   return yk_check_launch("attn_generic");

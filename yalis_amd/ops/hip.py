@@ -237,9 +237,11 @@ _SIGNATURES = {
     "yk_gemm_cols_ok": ([_c_int, _c_int, _c_int, _c_int], _c_int),
     "yk_gemm_cols_force": ([_c_int], _c_int),
     "yk_attn_generic": (
-        [_vp, _c_int, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _vp],
+        [_vp, _c_int, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int, _c_int,
+         _vp],
         _c_int,
     ),
+    "yk_attn_f32_form": ([_c_int] * 7, _c_int),
     "yk_attn_mfma_supported": ([_c_int], _c_int),
     "yk_attn_heads_per_tile": ([_c_int, _c_int], _c_int),
     "yk_attn_long_tile_tokens": ([_c_int, _c_int, _c_int], _c_int),
@@ -281,7 +283,7 @@ _LATER_SIGNATURES = {
         "yk_probe_mfma_bf16": ([_c_int, _c_int, _vp, _vp], _c_int),
     },
 }
-_ABI = 27
+_ABI = 28
 
 # Rows of x up to which the hand-written matrix-core kernel runs a bfloat16 product;
 # above it the vendor library does.
@@ -1244,7 +1246,7 @@ class HipOps:
                     qkv.data_ptr(), qkv.stride(0), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                     _code(qkv.dtype), ctx.arrays["positions"].data_ptr(), ctx.arrays["token_seq"].data_ptr(),
                     bt.data_ptr(), bt.shape[1], n, page_size, head_dim, n_heads, n_kv, float(scale), int(window),
-                    self._stream(),
+                    bt.shape[0], getattr(ctx, "max_qlen", 1), ctx.max_ctx, self._stream(),
                 )
             )
         return out
