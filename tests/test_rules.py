@@ -19,3 +19,13 @@ def lib():
 ])
 def test_float32_attention_of_several_requests(lib, step, form):
     assert lib.yk_attn_f32_form(*step) == form
+
+
+def test_what_is_taken_whole_is_not_refused_where_slices_would_do(lib):
+    for n in (512, 1360, 2048, 3072, 4096, 5120, 6144, 8192, 28672):
+        for k in (1024, 2048, 4096, 8192, 14336):
+            for m in range(65, 2101, 13):
+                whole, either = lib.yk_gemm_block_plan(m, n, k, 0, 0), lib.yk_gemm_block_plan(m, n, k, 1, 0)
+                assert either >= 0 or whole < 0, (m, n, k)
+                assert whole < 0 or whole % 256 == 1
+                assert either < 0 or either % 256 > 1 or either == whole

@@ -303,15 +303,17 @@ bool fits(const Form& f, int K, int slices) {
   return K % (64 * f.sub) == 0 && steps - (slices - 1) * ((steps + slices - 1) / slices) > f.ahead;
 }
 
-// The form and the slices of K for a product (form * 256 + slices), or -1 where the vendor library, or the kernels for fewer rows, do better.
-int plan(int M, int N, int K, bool partial, bool gated, bool act) {
-  if (M <= (act ? 128 : 64) || K % 64 || N % (gated ? 16 : 8)) return -1;
-  int best = -1, best_slices = 1, best_rounds = 1;
-  float least = 1e30f;
+struct Choice {
+  int form = -1, slices = 1, rounds = 1;
+  float us = 1e30f;
+};
+// The cheapest form with `from` to `to` slices of K.
+Choice cheapest(int M, int N, int K, bool gated, int from, int to) {
+  Choice best;
   for (int i = 0; i < N_FORMS; ++i) {
     const Form& f = FORMS[i];
     if (gated && i == 1) continue;
-    for (int slices = 1; slices <= (partial ? 4 : 1); slices *= 2) {
+    for (int slices = from; slices <= to; slices *= 2) {
       if (!fits(f, K, slices)) continue;
       const long long tiles = static_cast<long long>((N + f.bn - 1) / f.bn) * ((M + f.bm - 1) / f.bm) * slices;
       const int room = UNITS * f.fit, rounds = static_cast<int>((tiles + room - 1) / room);
@@ -320,13 +322,29 @@ int plan(int M, int N, int K, bool partial, bool gated, bool act) {
       // (the consumer of slices reads them all, where it would read bfloat16)
       const float us = f.once + rounds * (f.each + steps * (f.step + f.full * fill)) + megabytes * f.out +
                        (slices > 1 ? static_cast<float>(M) * N * (4 * slices - 2) / 4.5e6f : 0.f);
-      if (us < least) least = us, best = i, best_slices = slices, best_rounds = rounds;
+      if (us < best.us) best = {i, slices, rounds, us};
     }
   }
-  if (best < 0) return -1;
-  const Form& f = FORMS[best];
+  return best;
+}
+
+// The form and the slices of K for a product (form * 256 + slices), or -1 where the vendor library, or the kernels for fewer rows, do better.
+int plan(int M, int N, int K, bool partial, bool gated, bool act) {
+  if (M <= (act ? 128 : 64) || K % 64 || N % (gated ? 16 : 8)) return -1;
+  const Choice whole = cheapest(M, N, K, gated, 1, 1);
+  if (partial) {
+    // Up to 1,100 rows: beyond, whole tiles fill the compute units (us, library / whole / two slices: 1,110 x 3,072 x 8,192 82 / 76 / 72, but 1,300 89 /
+    // - / 112; 1,110 x 4,096 x 8,192 102 / - / 122, 4,096 x 4,096 62 / - / 75).
+    const Choice cut = cheapest(M, N, K, gated, 2, 4);
+    if (cut.form != 1 && cut.us < whole.us && N <= 5120 && M <= 1100 && (K >= 3072 || (M <= 128 ? K <= 1024 : M <= 256 && N <= 2560)) &&
+        (N >= 1024 || M <= 512))
+      return cut.form * 256 + cut.slices;
+  }
+  if (whole.form < 0) return -1;
+  const Form& f = FORMS[whole.form];
+  const int best = whole.form, best_rounds = whole.rounds;
   // the part of the compute units' time that goes into y and not into tiles that hang over or units without one
-  const float used = static_cast<float>(M) * N * best_slices / (static_cast<float>(best_rounds) * UNITS * f.fit * f.bn * f.bm);
+  const float used = static_cast<float>(M) * N / (static_cast<float>(best_rounds) * UNITS * f.fit * f.bn * f.bm);
   bool ours;
   // With a pass over the product saved, library (or slices) and pass / here, us: 8,192 x 2,048, 129 rows 22.5 / 13.4, 512 24.6 / 21.2, 2,048
   // 67.8 / 58.0, 4,096 126 / 111; 2,048 x 1,024 16.3 / 8.8, 22.2 / 9.2, 19.2 / 12.7, 27.7 / 22.8; 16,384 x 4,096 35.2 / 31.1, 63.0 / 58.3,
@@ -341,11 +359,14 @@ int plan(int M, int N, int K, bool partial, bool gated, bool act) {
   else if (gated)
     ours = N >= 2048 && !(best == 0 && N > 24576 && K >= 4096 && M <= 2560) &&
            (M <= 128 || used >= (M <= 256 ? 0.6f : M <= 720 ? 0.76f : best == 0 && best_rounds == 3 && N % 1024 == 0 ? 0.77f : 0.65f));
-  else if (best_slices > 1)
-    ours = N <= 5120 && M <= 1100 && best != 1 && (K >= 3072 || (M <= 128 ? K <= 1024 : M <= 256 && N <= 2560)) && (N >= 1024 || M <= 512);
+  // Whole tiles where one time round is nearly full, and widths of no whole number of the library's tiles, of a long K only where half of the time is
+  // y's (us, library / here: 1,360 x 2,048, 1,055 rows 21 / 20; 1,360 x 8,192, 1,154 rows, .37 of the time 50 / 62, 1,877, .61, 69 / 62; 1,360 x 5,120, 1,418 rows,
+  // .46, 41 / 48).  Tiles of 128 x 128 wait for memory the longer K is (1,148 x 2,560 x 14,336, .70 109 / 126, 1,343 rows, .82, 132 / 120; 439 x
+  // 8,192 x 14,336, .86, 150 / 130).  The same whether slices would do or not: 1,649 x 4,096 x 8,192 125 / 120, 1,187 x 3,072 x 11,008 106 / 98.
   else
-    ours = (best_rounds == 1 && ((best == 2 && used >= 0.8f) || (best == 3 && used >= 0.7f))) || (N % 128 && N <= 8192 && M > 720);
-  return ours ? best * 256 + best_slices : -1;
+    ours = (best_rounds == 1 && ((best == 2 && used >= 0.8f) || (best == 3 && used >= (K >= 8192 && M > 256 ? 0.75f : 0.7f)))) ||
+           (N % 128 && N <= 8192 && M > 720 && (K <= 2048 || used >= 0.5f));
+  return ours ? best * 256 + 1 : -1;
 }
 
 template <int OUT>
