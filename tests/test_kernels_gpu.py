@@ -651,6 +651,17 @@ def test_gemm_block_is_what_linear_takes(ops):
         assert ops._block_plan(torch.empty(m, k, device=DEV), torch.empty(n, k, device=DEV), True) < 0
 
 
+# long matrices of 129 to 256 rows: cut along K by one kernel or the other, never the library's
+@pytest.mark.parametrize("m,n,k,block", [(129, 8192, 28672, True), (256, 8192, 28672, True), (192, 6144, 16384 - 32, False), (256, 2048, 8192, False), (192, 3072, 8192, True)])
+def test_linear_of_long_matrices(ops, m, n, k, block):
+    x, w = rnd((m, k), torch.bfloat16, 12), rnd((n, k), torch.bfloat16, 13, 0.05)
+    y = ops.linear(x, w, torch.bfloat16, partial_ok=True)
+    assert y.n_splits > 1
+    got = y.tensor.clone()
+    other = ops.gemm_block(x, w, torch.bfloat16, ops._block_plan(x, w, True)) if block else ops.gemm_tile(x, w, torch.bfloat16, True)
+    assert torch.equal(got, other.tensor)
+
+
 def test_gemm_tile(ops):
     """The product in tiles of 128 x 128 for some dozens to a few hundred rows: sizes that are no
     multiples of the tile or of the step of 64 along K, one-hot operands, K cut into 1 to 8 slices

@@ -2,6 +2,7 @@
 import pytest
 
 from yalis_amd.ops.build import load_kernels
+from yalis_amd.ops.hip import HipOps
 
 
 @pytest.fixture(scope="module")
@@ -29,3 +30,13 @@ def test_what_is_taken_whole_is_not_refused_where_slices_would_do(lib):
                 assert either >= 0 or whole < 0, (m, n, k)
                 assert whole < 0 or whole % 256 == 1
                 assert either < 0 or either % 256 > 1 or either == whole
+
+
+@pytest.mark.parametrize("m", [129, 160, 192, 224, 256])
+@pytest.mark.parametrize("n,k", [(8192, 28672), (8192, 22016), (7168, 20480), (6144, 16384), (5120, 13824), (4096, 14336), (3072, 8192)])
+def test_long_matrices_are_cut_along_k(lib, m, n, k):
+    plan = lib.yk_gemm_block_plan(m, n, k, 1, 0)
+    assert plan >= 0 and plan % 256 > 1
+    assert HipOps.long_matrix_tiles(m, n, k) and not HipOps.long_matrix_tiles(m, n, k, True)
+    assert lib.yk_gemm_block_plan(m, n, k - 32, 1, 0) < 0  # then they are gemm_tile's
+    assert HipOps.long_matrix_tiles(128, n, k, True) and not HipOps.long_matrix_tiles(257, n, k)

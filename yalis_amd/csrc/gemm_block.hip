@@ -334,10 +334,12 @@ int plan(int M, int N, int K, bool partial, bool gated, bool act) {
   const Choice whole = cheapest(M, N, K, gated, 1, 1);
   if (partial) {
     // Up to 1,100 rows: beyond, whole tiles fill the compute units (us, library / whole / two slices: 1,110 x 3,072 x 8,192 82 / 76 / 72, but 1,300 89 /
-    // - / 112; 1,110 x 4,096 x 8,192 102 / - / 122, 4,096 x 4,096 62 / - / 75).
+    // - / 112; 1,110 x 4,096 x 8,192 102 / - / 122, 4,096 x 4,096 62 / - / 75).  Up to 5,120 columns, and up to 8,192 where K is twice as long, which
+    // the library has no tiles for (library / gemm_tile / here: 8,192 x 28,672, 129 rows 308 / 197 / 137, 256 323 / 204 / 162; 7,168 x 20,480, 256 rows
+    // 240 / 139 / 112; 6,144 x 16,384, 129 rows 151 / 102 / 67).
     const Choice cut = cheapest(M, N, K, gated, 2, 4);
-    if (cut.form != 1 && cut.us < whole.us && N <= 5120 && M <= 1100 && (K >= 3072 || (M <= 128 ? K <= 1024 : M <= 256 && N <= 2560)) &&
-        (N >= 1024 || M <= 512))
+    if (cut.form != 1 && cut.us < whole.us && M <= 1100 && (N >= 1024 || M <= 512) &&
+        (N <= 5120 ? K >= 3072 || (M <= 128 ? K <= 1024 : M <= 256 && N <= 2560) : N <= 8192 && K >= 2 * N && M > 128 && M <= 256))
       return cut.form * 256 + cut.slices;
   }
   if (whole.form < 0) return -1;

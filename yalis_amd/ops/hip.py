@@ -728,12 +728,11 @@ class HipOps:
         aligned = k % 8 == 0 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
         if x.dtype == bf and w.dtype == bf and aligned:
             slices_do = partial_ok and out_dtype == bf
-            if out_dtype == bf and self.long_matrix_tiles(m, n, k, slices_do):
+            plan = self._block_plan(x, w, slices_do) if m > SKINNY_MAX_ROWS and out_dtype in (bf, torch.float32) else -1
+            if out_dtype == bf and self.long_matrix_tiles(m, n, k, plan >= 0 and plan % 256 > 1):
                 return self.gemm_tile(x, w, bf, partial_ok)
-            if m > SKINNY_MAX_ROWS and out_dtype in (bf, torch.float32):
-                plan = self._block_plan(x, w, slices_do)
-                if plan >= 0:
-                    return self.gemm_block(x, w, out_dtype, plan)
+            if plan >= 0:
+                return self.gemm_block(x, w, out_dtype, plan)
             if m > SKINNY_MAX_ROWS and out_dtype == bf and not self.few_library_tiles(m, n):
                 return self.gemm_library(x, w, bf)  # vendor library, bfloat16 in and out
             if m > SKINNY_MAX_ROWS and out_dtype == torch.float32:
@@ -746,7 +745,7 @@ class HipOps:
         return self.gemm_fma(x, w, out_dtype)
 
     @staticmethod
-    def long_matrix_tiles(m: int, n: int, k: int, slices_do: bool = False) -> bool:
+    def long_matrix_tiles(m: int, n: int, k: int, block_slices: bool = False) -> bool:
         """Whether a product of 65 to 256 rows is ``gemm_tile``'s: where the matrix is at least twice
         as long as it is wide (a down projection), so that tiles of 128 x 128 cut along K occupy
         the GPU and the slices are long.  Measured in replayed graphs (us, vendor library's first
@@ -755,9 +754,10 @@ class HipOps:
         (3,072 x 8,192) at 128 32.9 / 19.6 / 17.7, at 192 45.3 / 27.5 / 28.5; 70B (8,192 x 28,672) at
         128 200 / 167 / 110, at 256 314 / - / 200; 1B (2,048 x 8,192) at 192 22.9 / 19.7 / 18.2.  On
         squarer matrices the three are within a tenth of each other up to 128 rows, and from 384
-        rows on the library wins everywhere.  Where the consumer adds slices (``slices_do``) ``gemm_block`` in slices is faster from 129
-        rows on unless K is four times N or more."""
-        return SKINNY_MAX_ROWS < m <= (128 if slices_do and k < 4 * n else 256) and k >= 2 * n and k >= 4096
+        rows on the library wins everywhere.  Where ``gemm_block`` takes the product in slices (``block_slices``) it is faster from 129
+        rows on unless K is four times N or more (at 192 rows, tiles / ``gemm_block``, with the norm that adds the slices: 70B 198 / 150, 8B 59 / 46,
+        3B 36 / 28)."""
+        return SKINNY_MAX_ROWS < m <= (128 if block_slices and k < 4 * n else 256) and k >= 2 * n and k >= 4096
 
     @staticmethod
     def few_library_tiles(m: int, n: int) -> bool:
