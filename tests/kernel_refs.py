@@ -889,6 +889,7 @@ RefOps.grouped_linear = staticmethod(grouped_linear)
 RefOps.low_rank = staticmethod(low_rank)
 RefOps.sandwich_norm = staticmethod(sandwich_norm)
 RefOps.activation = staticmethod(activation)
+RefOps.linear_act = staticmethod(lambda x, w, kind, out_dtype: activation(linear(x, w, out_dtype), kind, out_dtype))
 RefOps.scale_rows = staticmethod(scale_rows)
 RefOps.latent_prepare = staticmethod(latent_prepare)
 RefOps.head_linear = staticmethod(head_linear)

@@ -120,8 +120,5 @@ class DenseMLP(FeedForward):
 
     def forward(self, h: torch.Tensor, ctx) -> torch.Tensor:
         ops = self.rt.ops
-        if hasattr(ops, "linear_act"):  # (a set of plain operations need not have it)
-            a = ops.linear_act(h, self.w_up, self.activation, self.rt.act_dtype)
-        else:
-            a = ops.activation(ops.linear(h, self.w_up, self.rt.act_dtype, partial_ok=True), self.activation, self.rt.act_dtype)
+        a = ops.linear_act(h, self.w_up, self.activation, self.rt.act_dtype)
         return ops.linear(a, self.w_down, self.rt.act_dtype, partial_ok=True)
