@@ -578,6 +578,19 @@ def test_gemm_block_gated(ops, form, activation):
         assert bool((off <= 2**-7 * want.abs()[~(torch.isnan(want) | both_inf)] + 1e-37).all())
 
 
+@pytest.mark.parametrize("plan", [2 * 256 + 2, 256 + 1])
+def test_gate_up_act_where_the_forced_plan_has_no_pairs(ops, plan):
+    x = rnd((130, 1024), torch.bfloat16, 14)
+    w, group = ops.pack_gate_up(rnd((256, 1024), torch.bfloat16, 15, 0.05), rnd((256, 1024), torch.bfloat16, 16, 0.05))
+    want = ops.gated_act(ops.linear(x, w, torch.bfloat16), "silu", torch.bfloat16, group=group)
+    ops.force_block_plan(plan)
+    try:
+        got = ops.gate_up_act(x, w, group, "silu", torch.bfloat16)
+    finally:
+        ops.force_block_plan()
+    close(got, want.double().cpu(), 2e-2, 2**-6)
+
+
 @pytest.mark.parametrize("form", [0, 2, 3, 4])
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh"] + [("clamped_swish", 7.0, s) for s in (-1.702, 0.0, 1.0, 1.25, 1.5, 1.6, 1.7, 1.702, 2.0)])
 def test_gemm_block_gated_of_every_gate(ops, form, activation):

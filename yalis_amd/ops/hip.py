@@ -990,7 +990,7 @@ class HipOps:
         if (pairs and m > SKINNY_MAX_ROWS and x.dtype == bf and w_gate_up.dtype == bf and w_gate_up.shape[1] == k and w_gate_up.stride(1) == 1
                 and x.stride(0) % 8 == 0 and w_gate_up.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0):
             plan = self._block_plan(x, w_gate_up, False, gated=1)
-            if plan >= 0:
+            if plan >= 0 and plan % 256 == 1 and plan // 256 != 1:  # (a forced plan may be slices, or the form without pairs)
                 return self.gemm_block(x, w_gate_up, bf, plan, gated=activation)
         if not fused:
             return self.gated_act(self.linear(x, w_gate_up, out_dtype, partial_ok=True), activation, out_dtype, group=group)
