@@ -145,6 +145,15 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 __device__ __forceinline__ float wave_max(float v) { return row_max(column_lanes_max(v)); }
 
+// Lane i's 16 bytes at `at` + `lane_off` + `off` (zeros beyond `bytes`, against which both offsets count) to place i of the KiB of LDS at `to`.
+__device__ __forceinline__ void load_to_lds(const void* at, int bytes, void* to, int lane_off, int off) {
+#ifdef __HIP_DEVICE_COMPILE__  // the builtin takes 16 bytes for the device alone
+  typedef __attribute__((address_space(3))) void lds_void_t;
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(at), 0, bytes, 0x00027000), (lds_void_t*)to, 16,
+                                           lane_off, off, 0, 0);
+#endif
+}
+
 // Gated activations: 0 = silu, 1 = gelu (tanh form); float32.
 __device__ __forceinline__ float act_silu(float z) { return z / (1.f + expf(-z)); }
 __device__ __forceinline__ float act_gelu_tanh(float z) {

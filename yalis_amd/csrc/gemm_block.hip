@@ -24,15 +24,6 @@ namespace {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-// Lane i's 16 bytes at `at` + `lane_off` + `off` (zeros beyond `bytes`, against which both offsets count) to place i of the KiB of LDS at `to`.
-__device__ __forceinline__ void load_to_lds(const void* at, int bytes, void* to, int lane_off, int off) {
-#ifdef __HIP_DEVICE_COMPILE__  // the builtin takes 16 bytes for the device alone
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(at), 0, bytes, 0x00027000), (lds_void_t*)to, 16,
-                                           lane_off, off, 0, 0);
-#endif
-}
 
 // Until no more than VM loads and stores and LGKM LDS reads of this wave are under way (the builtin: the compiler then adds no waits of its
 // own for those reads).

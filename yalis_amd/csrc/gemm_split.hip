@@ -27,7 +27,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void_t;
 
 // Operands are taken 2^24 times as large, so that the parts of the smallest float32 are no subnormal numbers, which the bfloat16 products
 // take for zeros; what grows beyond float32 on the way is made again without (below).
@@ -65,14 +64,6 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
   *reinterpret_cast<u32x4_t*>(parts + at) = u32x4_t{h[0], h[1], h[2], h[3]};
   *reinterpret_cast<u32x4_t*>(parts + plane + at) = u32x4_t{mid[0], mid[1], mid[2], mid[3]};
   *reinterpret_cast<u32x4_t*>(parts + 2 * plane + at) = u32x4_t{l[0], l[1], l[2], l[3]};
-}
-
-// Lane i's 16 bytes at `at` + `lane_off` + `off` (zeros beyond `bytes`, against which both offsets count) to place i of the KiB of LDS at `to`.
-__device__ __forceinline__ void load_to_lds(const void* at, int bytes, void* to, int lane_off, int off) {
-#ifdef __HIP_DEVICE_COMPILE__  // the builtin takes 16 bytes for the device alone
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(at), 0, bytes, 0x00027000), (lds_void_t*)to, 16,
-                                           lane_off, off, 0, 0);
-#endif
 }
 
 // f(0) .. f(N - 1), each number a constant
