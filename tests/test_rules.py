@@ -40,3 +40,16 @@ def test_long_matrices_are_cut_along_k(lib, m, n, k):
     assert HipOps.long_matrix_tiles(m, n, k) and not HipOps.long_matrix_tiles(m, n, k, True)
     assert lib.yk_gemm_block_plan(m, n, k - 32, 1, 0) < 0  # then they are gemm_tile's
     assert HipOps.long_matrix_tiles(128, n, k, True) and not HipOps.long_matrix_tiles(257, n, k)
+
+
+# rows, columns, K of a product with pairs (1) or an activation (2): faster without its pass in the product, and sizes beside them that are not
+@pytest.mark.parametrize("m,n,k,kind", [(107, 2048, 8192, 1), (105, 2048, 4096, 1), (98, 3584, 28672, 1), (128, 4096, 2048, 1), (106, 14336, 8192, 1), (2366, 8192, 4096, 1),
+                                        (2962, 4096, 5120, 1), (207, 8192, 5120, 2), (251, 7168, 5120, 2), (1300, 8192, 4096, 2)])
+def test_long_products_that_leave_units_idle_keep_their_pass(lib, m, n, k, kind):
+    assert lib.yk_gemm_block_plan(m, n, k, 0, kind) < 0
+
+
+@pytest.mark.parametrize("m,n,k,kind", [(107, 2048, 768, 1), (103, 16384, 2048, 1), (999, 16384, 2048, 1), (1005, 8192, 4096, 1), (3985, 16384, 3072, 1), (512, 16384, 3072, 1),
+                                        (8192, 28672, 4096, 1), (129, 2048, 1024, 2), (512, 8192, 2048, 2), (4096, 16384, 4096, 2)])
+def test_products_that_gain_by_their_pass_have_it(lib, m, n, k, kind):
+    assert lib.yk_gemm_block_plan(m, n, k, 0, kind) >= 0

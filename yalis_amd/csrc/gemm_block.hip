@@ -319,6 +319,37 @@ Choice cheapest(int M, int N, int K, bool gated, int from, int to) {
   return best;
 }
 
+int rounds_of(int M, int N, int bn, int bm) {
+  return static_cast<int>((static_cast<long long>((N + bn - 1) / bn) * ((M + bm - 1) / bm) + UNITS - 1) / UNITS);
+}
+// The part of the compute units' rounds that has a tile.
+float filled(const Choice& c, int M, int N) {
+  const Form& f = FORMS[c.form];
+  return static_cast<float>((N + f.bn - 1) / f.bn) * ((M + f.bm - 1) / f.bm) * c.slices / (c.rounds * UNITS * f.fit);
+}
+
+// Whether a product with a pass over it saved is faster here than the product in slices or in the library and the pass.  What is saved grows with
+// y, what is lost with K: the fused product cannot be cut, so that few tiles leave compute units idle for all of K, and the library's
+// product alone is up to 6 % ahead.  Short K always pays (few rows' slices lie closer: 768, else 1,024).  Beyond, small tiles only where they fill
+// half of the units (128 x 128) or a fifth and K is up to 2,048 (128 x 64); large ones where their rounds are full enough for their K.  us, without
+// / with the pairs here: 105 rows, 2,048 x 4,096 19 / 21, 107 rows, 2,048 x 8,192 24 / 42, 103 rows, 16,384 x 2,048 24 / 21; in tiles of 128 x 128 106
+// rows, 14,336 x 8,192 64 / 72; of 256 x 128 in three rounds 2,366 rows, 8,192 x 4,096 146 / 160, in one 1,005 rows 72 / 63.  Of 9,288 products with
+// pairs (65 to 4,096 rows, 1,024 to 32,768 columns, K 512 to 28,672) that a rule of the used part alone took 2,338 were more than 6 % slower than without;
+// this one takes 5,883, of which 162 are, in 0.82 of the time.  Of 4,870 with an activation it was 635, and is 45 of 3,488, in 0.83.
+bool pass_pays(const Choice& c, int M, int N, int K, bool act) {
+  if (K <= (act ? 1024 : 768)) return true;
+  const Form& f = FORMS[c.form];
+  const float fill = filled(c, M, N);
+  if (c.form == 4) return K <= 2048 && c.rounds == 1 && fill >= 0.2f;
+  if (c.form == 3) return c.rounds == 1 ? fill > (act && K > 4096 ? 0.6f : 0.5f) : c.rounds > 3 && K <= 2048;
+  // (the library's tiles of 256 x 192 in no more rounds than ours of 256 x 256: a quarter less of everything)
+  if (c.form == 0 && std::min(rounds_of(M, N, 256, 192), rounds_of(M, N, 192, 256)) <= c.rounds) return false;
+  if (K <= 2048) return true;
+  if (c.form == 2) return c.rounds <= 2 ? fill >= (act ? 0.8f : K <= 4096 ? 0.f : 0.75f) : c.rounds > 3 && fill >= 0.9f;
+  if (c.form == 1) return c.rounds > 2 || (K < 4096 && static_cast<float>(M) * N / (c.rounds * UNITS * f.bn * f.bm) >= 0.8f);
+  return c.rounds > 1 || (K <= 4096 && fill >= 0.8f);
+}
+
 // The form and the slices of K for a product (form * 256 + slices), or -1 where the vendor library, or the kernels for fewer rows, do better.
 int plan(int M, int N, int K, bool partial, bool gated, bool act) {
   if (M <= (act ? 128 : 64) || K % 64 || N % (gated ? 16 : 8)) return -1;
@@ -339,19 +370,17 @@ int plan(int M, int N, int K, bool partial, bool gated, bool act) {
   // the part of the compute units' time that goes into y and not into tiles that hang over or units without one
   const float used = static_cast<float>(M) * N / (static_cast<float>(best_rounds) * UNITS * f.fit * f.bn * f.bm);
   bool ours;
-  // With a pass over the product saved, library (or slices) and pass / here, us: 8,192 x 2,048, 129 rows 22.5 / 13.4, 512 24.6 / 21.2, 2,048
-  // 67.8 / 58.0, 4,096 126 / 111; 2,048 x 1,024 16.3 / 8.8, 22.2 / 9.2, 19.2 / 12.7, 27.7 / 22.8; 16,384 x 4,096 35.2 / 31.1, 63.0 / 58.3,
-  // 209 / 195, 415 / 399 (of 84 products one lost: 800 x 11,008 x 4,096 68.2 / 70.4).  Not where K is long and tiles are few, which slices
-  // help: 3,072 x 8,192 20.2 / 34.1, 33.6 / 36.4.
+  // With an activation of every element in the product's end, library (or slices) and pass / here, us: 8,192 x 2,048, 129 rows 22.5 / 13.4, 512
+  // 24.6 / 21.2, 2,048 67.8 / 58.0, 4,096 126 / 111; 2,048 x 1,024 16.3 / 8.8, 22.2 / 9.2, 19.2 / 12.7, 27.7 / 22.8; 16,384 x 4,096 35.2 / 31.1,
+  // 63.0 / 58.3, 209 / 195, 415 / 399.
   if (act)
-    ours = N >= 2048 && K <= N;
-  // Not where the library's product of the same tiles of 256 x 256 gains more than its pass for the pairs costs: long and wide matrices (us, library
+    ours = N >= 2048 && K <= N && (used >= 0.66f || best != 0 || K <= 2048) && pass_pays(whole, M, N, K, true);
+  // Pairs: not where the library's product of the same tiles of 256 x 256 gains more than its pass for the pairs costs: long and wide matrices (us, library
   // and pass / here: 28,672 x 4,096, 1,300 rows 275 / 289, 2,048 378 / 396, 57,344 x 8,192 1,032 / 1,091, 1,316 / 1,382; from 2,560 rows on
-  // 581 / 574, 982 / 871; 24,576 x 4,096 304.5 / 303.9 at 2,048), and a third time round for few tiles where its own fit (24,576 x 4,096, 1,536 rows
-  // 258 / 266, 12,288 x 2,048, 3,000 rows 146 / 151).
+  // 581 / 574, 982 / 871; 24,576 x 4,096 304.5 / 303.9 at 2,048; of fewer rows 512 102 / 103, 900 184 / 189, 57,344 x 8,192 397 / 391, 784 / 719).
   else if (gated)
-    ours = N >= 2048 && !(best == 0 && N > 24576 && K >= 4096 && M <= 2560) &&
-           (M <= 128 || used >= (M <= 256 ? 0.6f : M <= 720 ? 0.76f : best == 0 && best_rounds == 3 && N % 1024 == 0 ? 0.77f : 0.65f));
+    ours = N >= 2048 && !(best == 0 && N > 24576 && K >= 4096 && M <= 2560) && pass_pays(whole, M, N, K, false) &&
+           (M <= 128 || used >= (M <= 256 ? 0.6f : M <= 720 ? 0.76f : 0.65f));
   // Whole tiles where one time round is nearly full, and widths of no whole number of the library's tiles, of a long K only where half of the time is
   // y's (us, library / here: 1,360 x 2,048, 1,055 rows 21 / 20; 1,360 x 8,192, 1,154 rows, .37 of the time 50 / 62, 1,877, .61, 69 / 62; 1,360 x 5,120, 1,418 rows,
   // .46, 41 / 48).  Tiles of 128 x 128 wait for memory the longer K is (1,148 x 2,560 x 14,336, .70 109 / 126, 1,343 rows, .82, 132 / 120; 439 x
