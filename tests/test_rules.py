@@ -53,3 +53,10 @@ def test_long_products_that_leave_units_idle_keep_their_pass(lib, m, n, k, kind)
                                         (8192, 28672, 4096, 1), (129, 2048, 1024, 2), (512, 8192, 2048, 2), (4096, 16384, 4096, 2)])
 def test_products_that_gain_by_their_pass_have_it(lib, m, n, k, kind):
     assert lib.yk_gemm_block_plan(m, n, k, 0, kind) >= 0
+
+
+# rows, columns, K of products that were slower in large tiles, whole or in slices, than by the kernels and the library beside them
+@pytest.mark.parametrize("m,n,k", [(103, 1024, 3072), (110, 512, 3072), (103, 2560, 1024), (122, 3072, 1024), (536, 3584, 5120), (660, 1536, 3072),
+                                   (3195, 1360, 8192), (893, 8192, 28672), (1844, 4096, 28672), (373, 8192, 6144), (364, 8192, 5120)])
+def test_products_that_are_not_for_large_tiles(lib, m, n, k):
+    assert lib.yk_gemm_block_plan(m, n, k, 1, 0) < 0 and lib.yk_gemm_block_plan(m, n, k, 0, 0) < 0

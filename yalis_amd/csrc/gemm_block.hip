@@ -359,9 +359,13 @@ int plan(int M, int N, int K, bool partial, bool gated, bool act) {
     // - / 112; 1,110 x 4,096 x 8,192 102 / - / 122, 4,096 x 4,096 62 / - / 75).  Up to 5,120 columns, and up to 8,192 where K is twice as long, which
     // the library has no tiles for (library / gemm_tile / here: 8,192 x 28,672, 129 rows 308 / 197 / 137, 256 323 / 204 / 162; 7,168 x 20,480, 256 rows
     // 240 / 139 / 112; 6,144 x 16,384, 129 rows 151 / 102 / 67).
+    // Up to 128 rows the few-row kernel's slices are as fast unless K is short or long (its / here: 103 rows, 512 x 768 9.7 / 6.9, 1,024 x 3,072 11.0 / 13.3, 2,560 x
+    // 1,024 11.0 / 11.9); tiles of 128 x 64 that fill more than half of the units only where K is long (536 rows, 3,584 x 5,120 44 / 52, 660 rows, 1,536 x
+    // 3,072 23 / 25).
     const Choice cut = cheapest(M, N, K, gated, 2, 4);
-    if (cut.form != 1 && cut.us < whole.us && M <= 1100 && (N >= 1024 || M <= 512) &&
-        (N <= 5120 ? K >= 3072 || (M <= 128 ? K <= 1024 : M <= 256 && N <= 2560) : N <= 8192 && K >= 2 * N && M > 128 && M <= 256))
+    if (cut.form != 1 && cut.us < whole.us && M <= 1100 && (N >= 1024 || M <= 512) && !(cut.form == 4 && filled(cut, M, N) > 0.5f && K < 8192) &&
+        (N <= 5120 ? K >= (M <= 128 && N < 1280 ? 4096 : 3072) || (M <= 128 ? K <= (N <= 1536 ? 1024 : 768) : M <= 256 && N <= 2560 && (N > 640 || K >= 1024))
+                   : N <= 8192 && K >= 2 * N && M > 128 && M <= 256))
       return cut.form * 256 + cut.slices;
   }
   if (whole.form < 0) return -1;
@@ -381,13 +385,14 @@ int plan(int M, int N, int K, bool partial, bool gated, bool act) {
   else if (gated)
     ours = N >= 2048 && !(best == 0 && N > 24576 && K >= 4096 && M <= 2560) && pass_pays(whole, M, N, K, false) &&
            (M <= 128 || used >= (M <= 256 ? 0.6f : M <= 720 ? 0.76f : 0.65f));
-  // Whole tiles where one time round is nearly full, and widths of no whole number of the library's tiles, of a long K only where half of the time is
-  // y's (us, library / here: 1,360 x 2,048, 1,055 rows 21 / 20; 1,360 x 8,192, 1,154 rows, .37 of the time 50 / 62, 1,877, .61, 69 / 62; 1,360 x 5,120, 1,418 rows,
-  // .46, 41 / 48).  Tiles of 128 x 128 wait for memory the longer K is (1,148 x 2,560 x 14,336, .70 109 / 126, 1,343 rows, .82, 132 / 120; 439 x
-  // 8,192 x 14,336, .86, 150 / 130).  The same whether slices would do or not: 1,649 x 4,096 x 8,192 125 / 120, 1,187 x 3,072 x 11,008 106 / 98.
+  // Whole tiles where one time round is nearly full, and widths of no whole number of the library's tiles, of a long K only in the smaller tiles and where half
+  // of the time is y's (us, library / here: 1,360 x 2,048, 1,055 rows 21 / 20; 1,360 x 8,192, 1,154 rows, .37 of the time 50 / 62, 1,877, .61, 69 / 62; 1,360 x
+  // 5,120, 1,418 rows, .46, 41 / 48; in tiles of 256 x 128 3,195 rows, 1,360 x 8,192 77 / 85).  Tiles of 128 x 128 wait for memory the longer K is (1,148 x 2,560 x
+  // 14,336, .70 109 / 126, 1,343 rows, .82, 132 / 120; 439 x 8,192 x 14,336, .86, 150 / 130; 373 x 8,192 x 6,144, .73 52 / 58), and those of 256 x 128 beyond
+  // 16,384 (893 x 8,192 x 28,672 358 / 406).  The same whether slices would do or not: 1,649 x 4,096 x 8,192 125 / 120, 1,187 x 3,072 x 11,008 106 / 98.
   else
-    ours = (best_rounds == 1 && ((best == 2 && used >= 0.8f) || (best == 3 && used >= (K >= 8192 && M > 256 ? 0.75f : 0.7f)))) ||
-           (N % 128 && N <= 8192 && M > 720 && (K <= 2048 || used >= 0.5f));
+    ours = (best_rounds == 1 && ((best == 2 && used >= 0.8f && K <= 16384) || (best == 3 && used >= (K > 4096 ? 0.75f : 0.7f)))) ||
+           (N % 128 && N <= 8192 && M > 720 && (K <= 2048 || (used >= 0.5f && best != 2)));
   return ours ? best * 256 + 1 : -1;
 }
 
