@@ -60,3 +60,10 @@ def test_products_that_gain_by_their_pass_have_it(lib, m, n, k, kind):
                                    (3195, 1360, 8192), (893, 8192, 28672), (1844, 4096, 28672), (373, 8192, 6144), (364, 8192, 5120)])
 def test_products_that_are_not_for_large_tiles(lib, m, n, k):
     assert lib.yk_gemm_block_plan(m, n, k, 1, 0) < 0 and lib.yk_gemm_block_plan(m, n, k, 0, 0) < 0
+
+
+# rows beyond those that are taken apart at a time walk along K again, which pays where columns are many
+@pytest.mark.parametrize("m,n,k,taken", [(1681, 916, 7264, False), (5677, 632, 6592, False), (2247, 848, 15788, False), (1472, 916, 7264, True), (2009, 7724, 5428, True),
+                                         (2000, 6144, 4096, True), (8192, 2048, 8192, True)])
+def test_float32_products_of_several_passes(lib, m, n, k, taken):
+    assert (lib.yk_gemm_split_plan(m, n, k) > 0) == taken

@@ -267,9 +267,12 @@ int padded(int K) { return (K + 127) / 128 * 128; }
 // The rule: what a product takes here and in gemm_f32, us, fitted to what 104 products of 33 to 2,000 rows, 64 to 16,384 columns and K of
 // 4 to 8,192 took (nowhere 2% slower than gemm_f32 there; the largest gain left is 2,000 x 128 x 2,048, 34 where 25 us would do).  Here: the split of x; the compute
 // units work through their workgroups' steps in turn, however many are resident, and w comes at 4 TB/s; slices are written, and read by a
-// kernel of their own.  There: few tiles of 64 x 64 run as tiles of 16 rows, in the time of one walk along K, more in rounds of 256.
+// kernel of their own; rows beyond a pass walk along K again, which takes a tenth less than the passes apart (us, there / here: 5,677 x 632 x 6,592, four
+// passes, 501 / 677, 1,681 x 916 x 7,264, two, 288 / 324, 2,009 x 7,724 x 5,428 1,702 / 1,105; 63 of 120 such products are taken, the slowest in 1.02 times
+// its time there).  There: few tiles of 64 x 64 run as tiles of 16 rows, in the time of one walk along K, more in rounds of 256.
 double split_us(int M, int N, int K, int slices) {
-  const int kp = padded(K), per = (kp / 128 + slices - 1) / slices * 4;
+  const int kp = padded(K), per = (kp / 128 + slices - 1) / slices * 4, rows = pass_rows(kp);
+  if (M > rows) return .9 * (M / rows * split_us(rows, N, K, slices) + (M % rows ? split_us(M % rows, N, K, slices) : 0.));
   const double rounds = std::ceil(static_cast<double>((N + BN - 1) / BN) * ((M + BM - 1) / BM) * ((kp / 32 + per - 1) / per) / 256.);
   return 8. + std::max((rounds > 1. ? .7 : .75) * per * rounds, 1e-6 * N * K) + 1.5e-6 * M * kp + (slices > 1 ? 4. + 2e-6 * slices * M * N : 0.);
 }
