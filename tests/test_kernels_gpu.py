@@ -563,7 +563,8 @@ def test_gemm_block_forms(ops, form, least_k, sub):
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh", ("clamped_swish", 7.0, 1.702)])
 def test_gemm_block_gated(ops, form, activation):
     """Gated pairs in the product's end: the pairs of its own rounded product (one unit of bfloat16 apart at most, where the float32 values
-    of the two activations straddle a rounding), gates of every sign and size, infinities and NaN as they come."""
+    of the two activations straddle a rounding), for random gates, small and a thousand times as large, infinities and NaN as they come (every
+    gate there is: below)."""
     for m, n, k in [(1, 16, 512), (130, 528, 512), (300, 1040, 640)]:
         x, w = rnd((m, k), torch.bfloat16, 3), rnd((n, k), torch.bfloat16, 4, 0.3)
         x[0, 0], x[m // 2, 3] = float("inf"), float("nan")
