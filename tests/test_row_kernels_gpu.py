@@ -70,3 +70,43 @@ def test_activation_of_slices(slices, columns, out_dtype, kind):
     want = R.activation(total.to(out_dtype), kind, out_dtype)
     got = o.activation(SplitSum(parts.cuda(), out_dtype), kind, out_dtype)
     close(got, want, 2e-6 if out_dtype == torch.float32 else 2 ** -8)
+
+
+def in_order(t, dtype):
+    """The slices added one after another in float32 and rounded as a product of ``dtype`` would be."""
+    total = torch.zeros_like(t[0])
+    for one in t:
+        total = total + one
+    return total.to(dtype).float()
+
+
+def same(got, want):
+    return torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+CONSUMERS = {
+    "add_rmsnorm": lambda o, res, d, w, rows: o.add_rmsnorm(res, d, w, 1e-5, True, torch.bfloat16),
+    "gather_add_rmsnorm": lambda o, res, d, w, rows: o.gather_add_rmsnorm(res, d, rows, w, 1e-5, False, torch.float32),
+    "rmsnorm": lambda o, res, d, w, rows: o.rmsnorm(d, w, 1e-5, False, torch.bfloat16),
+}
+
+
+@pytest.mark.parametrize("consumer", CONSUMERS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,width", [(3, 4), (3, 516), (2, 4096), (2, 6148), (1025, 520)])  # one piece of a row a thread, two and four
+def test_any_number_of_slices(consumer, dtype, n, width):
+    """Slices go through registers in groups that depend on their number: the same bits as of the sum itself at every number,
+    infinities and NaN of single slices included."""
+    o, g = ops(), torch.Generator(device="cuda").manual_seed(width + n)
+    call = CONSUMERS[consumer]
+    w = torch.rand(width, device="cuda", generator=g) + 0.5
+    rows = torch.tensor([n - 1, 0, n // 2], dtype=torch.int32, device="cuda")
+    for slices in (2, 3, 4, 5, 8, 9, 12, 13, 16, 17, 20, 24, 25, 33):
+        t = torch.randn(slices, n, width, device="cuda", generator=g)
+        t[slices - 1, n - 1, width - 1] = float("inf") if slices % 2 else float("nan")
+        t[:, 0, 0] = -0.0
+        res = torch.randn(n, width, device="cuda", generator=g)
+        res2, whole = res.clone(), in_order(t, dtype)
+        got = call(o, res, SplitSum(t, dtype), w, rows)
+        want = call(o, res2, whole, w, rows)
+        assert same(got, want) and same(res, res2), slices

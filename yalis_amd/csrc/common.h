@@ -117,6 +117,79 @@ __host__ __device__ inline size_t cache_v_offset(bool tiled, int page_size, int 
   return static_cast<size_t>(slot / 64) * 64 * head_dim + piece * 8 + j % 8;
 }
 
+// Four neighbouring values as float32, and back.
+template <typename T>
+__device__ __forceinline__ float4 four_at(const T* p);
+template <>
+__device__ __forceinline__ float4 four_at<float>(const float* p) {
+  return *reinterpret_cast<const float4*>(p);
+}
+template <>
+__device__ __forceinline__ float4 four_at<bf16_t>(const bf16_t* p) {
+  const uint2 raw = *reinterpret_cast<const uint2*>(p);
+  return make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u), __uint_as_float(raw.y << 16),
+                     __uint_as_float(raw.y & 0xffff0000u));
+}
+template <typename T>
+__device__ __forceinline__ void put_four(T* p, float4 v);
+template <>
+__device__ __forceinline__ void put_four<float>(float* p, float4 v) {
+  *reinterpret_cast<float4*>(p) = v;
+}
+template <>
+__device__ __forceinline__ void put_four<bf16_t>(bf16_t* p, float4 v) {
+  *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
+}
+
+// `left` slices of IT pieces of four values, `stride` elements from one slice to the next, added to s in the slices' order.  SL of
+// them (at most) are asked for before the first is used, and nothing that is asked for hangs on a condition: a kernel of a few
+// microseconds lasts as long as the waits for memory it makes one after another, and the compiler moves a load to the condition
+// that its value alone is used under, and waits there.  So slices beyond the last are read from the last and masked to +0 with a
+// number that the compiler cannot take for a condition (a sum that began with +0 is never -0, and +0 leaves it as it is).
+template <int SL, int IT, typename T>
+__device__ __forceinline__ void add_slices(const T* const (&p)[IT], int left, size_t stride, float4 (&s)[IT]) {
+  float4 d[SL][IT];
+  size_t at = 0;
+#pragma unroll
+  for (int j = 0; j < SL; ++j) {
+#pragma unroll
+    for (int k = 0; k < IT; ++k) d[j][k] = four_at<T>(p[k] + at);
+    at += j + 1 < left ? stride : 0;
+  }
+#pragma unroll
+  for (int j = 0; j < SL; ++j) {
+    const uint32_t keep = __builtin_amdgcn_readfirstlane((j - left) >> 31);
+    auto kept = [&](float v) { return __uint_as_float(__float_as_uint(v) & keep); };
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      s[k].x += kept(d[j][k].x);
+      s[k].y += kept(d[j][k].y);
+      s[k].z += kept(d[j][k].z);
+      s[k].w += kept(d[j][k].w);
+    }
+  }
+}
+// The sum over n >= 1 slices of IT pieces of four values: one slice is one load, and of more up to 16 (8 with two pieces, 4 with more)
+// are in flight at a time.
+template <int IT, typename T>
+__device__ __forceinline__ void sum_slices(const T* (&p)[IT], int n, size_t stride, float4 (&s)[IT]) {
+  if (sizeof(T) == 2 || n == 1) {  // (slices are float32)
+#pragma unroll
+    for (int k = 0; k < IT; ++k) s[k] = four_at<T>(p[k]);
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < IT; ++k) s[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  constexpr int MOST = IT == 1 ? 16 : IT == 2 ? 8 : 4;
+  for (; n > MOST / 2; n -= MOST) {
+    add_slices<MOST, IT, T>(p, n, stride, s);
+#pragma unroll
+    for (int k = 0; k < IT; ++k) p[k] += MOST * stride;
+  }
+  if (n > MOST / 4) add_slices<MOST / 2, IT, T>(p, n, stride, s);
+  else if (n > 0) add_slices<MOST / 4, IT, T>(p, n, stride, s);
+}
+
 // Sums and maxima over a wave's 64 lanes, all of them active, in every lane: partners 32, 16, 8, 4, 2 and 1 lanes away, as moves between
 // registers (half-waves and rows of 16 swapped, rows rotated, quads permuted).  The same additions as with six shuffles, which go
 // through the LDS pipe and wait for it one after the other (a row's norm of one decode step: eight slices to add, 4.7 -> 4.0 us).
@@ -250,6 +323,15 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   v = wave_sum(v);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, nwaves = blockDim.x / kWave;
   __syncthreads();  // scratch may still be read from an earlier call
+  if (lane == 0) scratch[wave] = v;
+  __syncthreads();
+  return row_sum(lane % 16 < nwaves ? scratch[lane % 16] : 0.f);
+}
+
+// The same with the number of waves given, for a scratch that nothing has used yet: one barrier less, and no load of the block's size.
+__device__ __forceinline__ float block_sum_first(float v, float* scratch, int nwaves) {
+  v = wave_sum(v);
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
   return row_sum(lane % 16 < nwaves ? scratch[lane % 16] : 0.f);

@@ -187,37 +187,6 @@ extern "C" int yk_embed_pairs(const int32_t* ids, const void* table, int table_d
   return yk_fail("embed_pairs: unsupported table dtype");
 }
 
-// ---------------------------------------------------------------- four-wide accessors
-template <typename T>
-__device__ __forceinline__ float4 load4(const T* p);
-template <>
-__device__ __forceinline__ float4 load4<float>(const float* p) {
-  return *reinterpret_cast<const float4*>(p);
-}
-template <>
-__device__ __forceinline__ float4 load4<bf16_t>(const bf16_t* p) {
-  const uint2 raw = *reinterpret_cast<const uint2*>(p);
-  float4 v;
-  v.x = __uint_as_float(raw.x << 16);
-  v.y = __uint_as_float(raw.x & 0xffff0000u);
-  v.z = __uint_as_float(raw.y << 16);
-  v.w = __uint_as_float(raw.y & 0xffff0000u);
-  return v;
-}
-template <typename T>
-__device__ __forceinline__ void store4(T* p, float4 v);
-template <>
-__device__ __forceinline__ void store4<float>(float* p, float4 v) {
-  *reinterpret_cast<float4*>(p) = v;
-}
-template <>
-__device__ __forceinline__ void store4<bf16_t>(bf16_t* p, float4 v) {
-  uint2 raw;
-  raw.x = pack_bf16x2(v.x, v.y);
-  raw.y = pack_bf16x2(v.z, v.w);
-  *reinterpret_cast<uint2*>(p) = raw;
-}
-
 // (as_output, in common.h: the sum of a product's K slices is rounded as the product's
 // output would have been)
 
@@ -279,60 +248,44 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ residual, const TD* __res
   }
 }
 
-// Fast form: width a multiple of 4 and at most 4 * NORM_IT * blockDim; the row stays in
-// registers, every load of a thread is issued before the first use.  NORM_IT (four-wide
-// pieces per thread) is chosen by the launcher as small as the width allows.
+// Fast form: width a multiple of 4 and at most 4 * NORM_IT * blockDim; the row stays in registers.  NORM_IT (four-wide pieces per
+// thread) is chosen by the launcher as small as the width allows.  Bound by the launch and two trips to memory and back (the arguments
+// come with the launch; everything a row needs is asked for at once; the store): what decides is that no load waits for another.
+// FRESH (the row starts here: from a table, or there is no residual) is known when compiled, pieces beyond the row are read from
+// its end, and what is seldom used (`rows`, the table, add_row) is looked at where nothing else is in flight.  Behind a product of 32 MB of weights, us, with the loads under
+// conditions (the compiler waited for the residual, then the weight, then the slices, then the second slice again) / now:
+// one row of 2,048 2.58 / 1.90, with 8 slices 3.33 / 2.60, 16 4.35 / 3.24; eight rows 2.85 / 1.88, 3.61 / 2.63, 4.71 / 3.26; eight rows of 4,096 3.65 / 2.39, with 8 slices
+// 4.32 / 3.48.
+// `how` (one word, so that the arguments every row needs fit what comes with the launch): the bits below.
 constexpr int NORM_IT_MAX = 8;
-template <typename TD, typename TW, typename TO, int NORM_IT>
+constexpr uint32_t NORM_ROUND = 1u << 16, NORM_UNIT = 1u << 17, NORM_ROW = 1u << 18;  // bits 0-15: slices (0: no delta); 19-23: waves
+template <typename TD, typename TW, typename TO, int NORM_IT, bool FRESH>
 __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(
-    float* __restrict__ residual, const TD* __restrict__ delta, int n_splits, size_t split_stride,
-    int round_sum, const int32_t* __restrict__ rows, const TW* __restrict__ weight, TO* __restrict__ out,
-    int width, float eps, int unit_offset, const int32_t* __restrict__ table_ids, int table_rows,
-    const float* __restrict__ add_row) {
-  __shared__ float scratch[17];
+    float* __restrict__ residual, const TD* __restrict__ delta, const TW* __restrict__ weight, TO* __restrict__ out, int width,
+    uint32_t how, uint32_t split_stride, float eps, const int32_t* __restrict__ rows, const int32_t* __restrict__ table_ids,
+    int table_rows, const float* __restrict__ add_row) {
+  __shared__ float scratch[16];
+  const int n_splits = how & 0xffffu, waves = (how >> 19) & 31, round_sum = (how & NORM_ROUND) != 0;
   const int r = blockIdx.x;
-  const size_t src = rows ? static_cast<size_t>(rows[r]) : static_cast<size_t>(r);
-  float* res = residual ? residual + src * width : nullptr;
-  const bool fresh = table_ids != nullptr || res == nullptr;  // nothing is read from a residual
-  const TD* del = delta ? delta + (table_ids ? table_row(table_ids, src, table_rows) : src) * width : nullptr;
-  float4 v[NORM_IT], w[NORM_IT], ds[NORM_IT];
-  float ss = 0.f;
+  size_t src = r, from = r;
+  if (rows) src = from = rows[r];
+  if (FRESH && table_ids) from = table_row(table_ids, src, table_rows);
+  float* res = residual + src * width;
+  const TD* del = delta + from * width;
+  float4 v[NORM_IT], w[NORM_IT];
+  int at[NORM_IT];
 #pragma unroll
   for (int it = 0; it < NORM_IT; ++it) {
-    const int c = (threadIdx.x + it * blockDim.x) * 4;
-    if (c < width) {
-      v[it] = fresh ? make_float4(0.f, 0.f, 0.f, 0.f) : load4<float>(res + c);
-      w[it] = load4<TW>(weight + c);
-    }
+    at[it] = min((static_cast<int>(threadIdx.x) + it * 64 * waves) * 4, width - 4);
+    v[it] = FRESH ? make_float4(0.f, 0.f, 0.f, 0.f) : four_at<float>(res + at[it]);
+    w[it] = four_at<TW>(weight + at[it]);
   }
-  if (del) {
-    // SL slices at a time (eight where a thread has one piece of the row: a product's eight
-    // slices then cost one wait for memory, not two), all loads issued before the first
-    // sum; a slice index beyond the last is clamped and its value dropped, so that the
-    // loads carry no condition
-    constexpr int SL = NORM_IT == 1 ? 8 : 4;
+  if (FRESH || n_splits > 0) {
+    const TD* p[NORM_IT];
+    float4 ds[NORM_IT];
 #pragma unroll
-    for (int it = 0; it < NORM_IT; ++it) ds[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s0 = 0; s0 < n_splits; s0 += SL) {
-#pragma unroll
-      for (int it = 0; it < NORM_IT; ++it) {
-        const int c = (threadIdx.x + it * blockDim.x) * 4;
-        if (c < width) {
-          float4 d[SL];
-#pragma unroll
-          for (int j = 0; j < SL; ++j) d[j] = load4<TD>(del + static_cast<size_t>(min(s0 + j, n_splits - 1)) * split_stride + c);
-#pragma unroll
-          for (int j = 0; j < SL; ++j) {
-            if (s0 + j < n_splits) {
-              ds[it].x += d[j].x;
-              ds[it].y += d[j].y;
-              ds[it].z += d[j].z;
-              ds[it].w += d[j].w;
-            }
-          }
-        }
-      }
-    }
+    for (int it = 0; it < NORM_IT; ++it) p[it] = del + at[it];
+    sum_slices<NORM_IT, TD>(p, n_splits, split_stride, ds);
 #pragma unroll
     for (int it = 0; it < NORM_IT; ++it) {
       v[it].x += as_output(ds[it].x, round_sum);
@@ -341,36 +294,37 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(
       v[it].w += as_output(ds[it].w, round_sum);
     }
   }
+  if (how & NORM_ROW) {  // one vector for every row (the launcher allows it only where the residual is written back)
 #pragma unroll
-  for (int it = 0; it < NORM_IT; ++it) {
-    const int c = (threadIdx.x + it * blockDim.x) * 4;
-    if (c < width) {
-      if (add_row) {  // one vector for every row (the launcher allows it only where the residual is written back)
-        const float4 a = load4<float>(add_row + c);
-        v[it].x += a.x;
-        v[it].y += a.y;
-        v[it].z += a.z;
-        v[it].w += a.w;
-      }
-      if ((del || add_row) && !rows && res) store4<float>(res + c, v[it]);
-      ss += v[it].x * v[it].x + v[it].y * v[it].y + v[it].z * v[it].z + v[it].w * v[it].w;
+    for (int it = 0; it < NORM_IT; ++it) {
+      const float4 a = four_at<float>(add_row + at[it]);
+      v[it].x += a.x;
+      v[it].y += a.y;
+      v[it].z += a.z;
+      v[it].w += a.w;
     }
   }
-  ss = block_sum(ss, scratch);
+  const bool back = residual && !rows && (n_splits > 0 || (how & NORM_ROW));
+  float ss = 0.f;
+#pragma unroll
+  for (int it = 0; it < NORM_IT; ++it) {
+    const bool in = (static_cast<int>(threadIdx.x) + it * 64 * waves) * 4 < width;
+    if (back && in) put_four<float>(res + at[it], v[it]);
+    // (as multiply-adds written out: every form of the kernel rounds alike)
+    ss += in ? fmaf(v[it].w, v[it].w, fmaf(v[it].z, v[it].z, fmaf(v[it].y, v[it].y, v[it].x * v[it].x))) : 0.f;
+  }
+  ss = block_sum_first(ss, scratch, waves);
   const float inv = rsqrtf(ss / static_cast<float>(width) + eps);
-  const float off = unit_offset ? 1.f : 0.f;
+  const float off = how & NORM_UNIT ? 1.f : 0.f;
   TO* o = out + static_cast<size_t>(r) * width;
 #pragma unroll
   for (int it = 0; it < NORM_IT; ++it) {
-    const int c = (threadIdx.x + it * blockDim.x) * 4;
-    if (c < width) {
-      float4 y;
-      y.x = v[it].x * inv * (w[it].x + off);
-      y.y = v[it].y * inv * (w[it].y + off);
-      y.z = v[it].z * inv * (w[it].z + off);
-      y.w = v[it].w * inv * (w[it].w + off);
-      store4<TO>(o + c, y);
-    }
+    float4 y;
+    y.x = v[it].x * inv * (w[it].x + off);
+    y.y = v[it].y * inv * (w[it].y + off);
+    y.z = v[it].z * inv * (w[it].z + off);
+    y.w = v[it].w * inv * (w[it].w + off);
+    if ((static_cast<int>(threadIdx.x) + it * 64 * waves) * 4 < width) put_four<TO>(o + at[it], y);
   }
 }
 
@@ -382,7 +336,7 @@ static int launch_add_rmsnorm(float* residual, const void* delta, int n_splits, 
   const bool aligned = width % 4 == 0 && reinterpret_cast<uintptr_t>(residual) % 16 == 0 && reinterpret_cast<uintptr_t>(add_row) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(delta) % 16 == 0 && reinterpret_cast<uintptr_t>(weight) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(out) % 16 == 0 && split_stride % 4 == 0;
-  if (aligned && width <= 4 * NORM_IT_MAX * 512) {
+  if (aligned && width <= 4 * NORM_IT_MAX * 512 && n_splits < 1 << 16 && split_stride < size_t{1} << 32) {
     // one four-wide chunk per thread where the row allows (faster than two at 8 rows), at most
     // 1,024 threads; with rows enough to fill the GPU several times over, two chunks per thread:
     // twice the rows are in flight on a compute unit and a row's sum meets half the waves
@@ -390,14 +344,21 @@ static int launch_add_rmsnorm(float* residual, const void* delta, int n_splits, 
     int threads = ((n_rows >= 1024 ? width / 8 : width / 4) + 63) / 64 * 64;
     threads = std::max(64, std::min(threads, 1024));
     const int pieces = (width / 4 + threads - 1) / threads;
-#define YK_NORM(IT)                                                                           \
-    add_rmsnorm_vec_kernel<TD, TW, TO, IT><<<n_rows, threads, 0, stream>>>(                   \
-        residual, static_cast<const TD*>(delta), n_splits, split_stride, round_sum, rows,     \
-        static_cast<const TW*>(weight), static_cast<TO*>(out), width, eps, unit_offset, table_ids, table_rows, add_row)
-    if (pieces <= 1) YK_NORM(1);
-    else if (pieces <= 2) YK_NORM(2);
-    else if (pieces <= 4) YK_NORM(4);
-    else YK_NORM(8);
+    const uint32_t how = (delta ? static_cast<uint32_t>(n_splits) : 0u) | (round_sum ? NORM_ROUND : 0u) | (unit_offset ? NORM_UNIT : 0u) |
+                         (add_row ? NORM_ROW : 0u) | static_cast<uint32_t>(threads / 64) << 19;
+    const bool fresh = table_ids || !residual;
+#define YK_NORM(IT, FRESH)                                                                                                         \
+    add_rmsnorm_vec_kernel<TD, TW, TO, IT, FRESH><<<n_rows, threads, 0, stream>>>(                                                 \
+        residual, static_cast<const TD*>(delta), static_cast<const TW*>(weight), static_cast<TO*>(out), width, how,                \
+        static_cast<uint32_t>(split_stride), eps, rows, table_ids, table_rows, add_row)
+#define YK_NORM_IT(IT)             \
+    if (fresh) YK_NORM(IT, true);  \
+    else YK_NORM(IT, false)
+    if (pieces <= 1) YK_NORM_IT(1);
+    else if (pieces <= 2) YK_NORM_IT(2);
+    else if (pieces <= 4) YK_NORM_IT(4);
+    else YK_NORM_IT(8);
+#undef YK_NORM_IT
 #undef YK_NORM
   } else {
     add_rmsnorm_kernel<TD, TW, TO><<<n_rows, width >= 2048 ? 512 : 256, 0, stream>>>(
@@ -743,11 +704,11 @@ __global__ void gated_act_vec_kernel(const TS* __restrict__ gu, int n_splits, si
   const int j = static_cast<int>(v % per_row) * 4;
   const TS* p = gu + n * 2 * inter + gate_col(j, inter, group);  // four columns of one group (group % 4 == 0)
   const size_t up = up_offset(inter, group);
-  float4 g = load4<TS>(p), u = load4<TS>(p + up);
+  float4 g = four_at<TS>(p), u = four_at<TS>(p + up);
   for (int s0 = 1; s0 < n_splits; s0 += 2) {  // two slices in flight
     const int s1 = min(s0 + 1, n_splits - 1);
-    const float4 g2 = load4<TS>(p + s0 * split_stride), u2 = load4<TS>(p + s0 * split_stride + up);
-    const float4 g3 = load4<TS>(p + s1 * split_stride), u3 = load4<TS>(p + s1 * split_stride + up);
+    const float4 g2 = four_at<TS>(p + s0 * split_stride), u2 = four_at<TS>(p + s0 * split_stride + up);
+    const float4 g3 = four_at<TS>(p + s1 * split_stride), u3 = four_at<TS>(p + s1 * split_stride + up);
     g.x += g2.x; g.y += g2.y; g.z += g2.z; g.w += g2.w;
     u.x += u2.x; u.y += u2.y; u.z += u2.z; u.w += u2.w;
     if (s0 + 1 < n_splits) {
@@ -760,7 +721,7 @@ __global__ void gated_act_vec_kernel(const TS* __restrict__ gu, int n_splits, si
   y.y = gated_pair(as_output(g.y, round_sum), as_output(u.y, round_sum), act, p0, p1);
   y.z = gated_pair(as_output(g.z, round_sum), as_output(u.z, round_sum), act, p0, p1);
   y.w = gated_pair(as_output(g.w, round_sum), as_output(u.w, round_sum), act, p0, p1);
-  store4<TO>(out + n * inter + j, y);
+  put_four<TO>(out + n * inter + j, y);
 }
 
 // bfloat16 in and out, one slice, eight outputs per thread with 16-byte accesses (in the
