@@ -72,6 +72,22 @@ def test_activation_of_slices(slices, columns, out_dtype, kind):
     close(got, want, 2e-6 if out_dtype == torch.float32 else 2 ** -8)
 
 
+@pytest.mark.parametrize("n,width", [(3, 516), (2, 6148), (1030, 2052), (2, 10240)])  # one piece a thread, two, two of many rows, four
+@pytest.mark.parametrize("top", [1, 2, 3, 8, 9])
+def test_norm_add_of_expert_rows(n, width, top):
+    """A branch and a token's expert rows together, more of either than are asked for at once: float32 sums in the reference's order, up to the
+    rounding of the row's sum of squares (4e-6 as above)."""
+    o, g = ops(), torch.Generator().manual_seed(width + top)
+    res, src, e = torch.randn(n, width, generator=g), torch.randn(n, width, generator=g), torch.randn(n * top, width, generator=g)
+    w = torch.rand(width, generator=g) + 0.5
+    for branch in (src, None):
+        r_ref, r_dev = res.clone(), res.clone().cuda()
+        want = R.norm_add(r_ref, branch, w, 1e-5, True, torch.bfloat16, e, 0.3)
+        got = o.norm_add(r_dev, None if branch is None else branch.cuda(), w.cuda(), 1e-5, True, torch.bfloat16, e.cuda(), 0.3)
+        close(r_dev, r_ref, 4e-6)
+        close(got.float(), want.float(), 2 ** -8)
+
+
 def in_order(t, dtype):
     """The slices added one after another in float32 and rounded as a product of ``dtype`` would be."""
     total = torch.zeros_like(t[0])
@@ -88,6 +104,13 @@ CONSUMERS = {
     "add_rmsnorm": lambda o, res, d, w, rows: o.add_rmsnorm(res, d, w, 1e-5, True, torch.bfloat16),
     "gather_add_rmsnorm": lambda o, res, d, w, rows: o.gather_add_rmsnorm(res, d, rows, w, 1e-5, False, torch.float32),
     "rmsnorm": lambda o, res, d, w, rows: o.rmsnorm(d, w, 1e-5, False, torch.bfloat16),
+    "norm_add": lambda o, res, d, w, rows: o.norm_add(res, d, w, 1e-5, True, torch.bfloat16),
+    "sum_norm": lambda o, res, d, w, rows: o.sum_norm(res, [(d, w, 1e-5)], 0.5, w, 2.0, w, 1e-5, False, torch.bfloat16),
+    "sum_norm second": lambda o, res, d, w, rows: o.sum_norm(res, [(res * 0.5, None, 1e-5), (d, w, 1e-5)], 0.5, None, 2.0, w, 1e-5, True, torch.bfloat16),
+    "sandwich_norm": lambda o, res, d, w, rows: o.sandwich_norm(res, d, (w, w, 1e-5, True), 0.5, (w, None, 1e-5, False), None, torch.float32),
+    "sandwich_norm rows": lambda o, res, d, w, rows: o.sandwich_norm(res, d, None, 1.0, (w, w, 1e-5, True), rows, torch.bfloat16),
+    "activation": lambda o, res, d, w, rows: o.activation(d, "relu2", torch.float32),
+    "gated_act": lambda o, res, d, w, rows: o.gated_act(d, "silu", torch.float32) if d.shape[1] % 8 == 0 else torch.zeros(1),
 }
 
 

@@ -16,27 +16,12 @@
 //
 // Beside it: the other arrangement, the stream itself normed after a branch has joined it (yk_sum_norm).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
-// Four consecutive elements of a row of T as floats (16-byte aligned rows of a multiple of four).
-template <typename T>
-__device__ __forceinline__ float4 na_load4(const T* p);
-template <>
-__device__ __forceinline__ float4 na_load4<float>(const float* p) {
-  return *reinterpret_cast<const float4*>(p);
-}
-template <>
-__device__ __forceinline__ float4 na_load4<bf16_t>(const bf16_t* p) {
-  const uint2 w = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
-                     __uint_as_float(w.y & 0xffff0000u));
-}
-
-// VEC: four columns a thread with 16-byte accesses, and the slices (or a token's expert rows) of a
-// column asked for eight at a time before any is added: with one element a thread and one load
-// behind the other, eight rows of 2,048 took 17 us of waiting.  The sums keep the order of the slices.
-template <typename TS, typename TW, typename TO, bool VEC>
+// General form: any width, a column a thread, the row parked in LDS.
+template <typename TS, typename TW, typename TO>
 __global__ __launch_bounds__(256) void norm_add_kernel(
     float* __restrict__ residual, const TS* __restrict__ src, int n_splits, size_t split_stride, int round_sum,
     const float* __restrict__ pairs, int top, float pair_weight, const TW* __restrict__ w, int unit_offset,
@@ -45,79 +30,94 @@ __global__ __launch_bounds__(256) void norm_add_kernel(
   float* scratch = row + width;
   const size_t n = blockIdx.x;
   float ss = 0.f;
-  if (VEC) {
-    for (int c = 4 * threadIdx.x; c < width; c += 4 * blockDim.x) {
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (src != nullptr) {
-        for (int s0 = 0; s0 < n_splits; s0 += 8) {
-          float4 t[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (s0 + j < n_splits) t[j] = na_load4<TS>(src + (s0 + j) * split_stride + n * width + c);
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (s0 + j < n_splits) {
-              v.x += t[j].x; v.y += t[j].y; v.z += t[j].z; v.w += t[j].w;
-            }
-        }
-        v.x = as_output(v.x, round_sum); v.y = as_output(v.y, round_sum);
-        v.z = as_output(v.z, round_sum); v.w = as_output(v.w, round_sum);
-      }
-      if (pairs != nullptr) {
-        float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int k0 = 0; k0 < top; k0 += 8) {
-          float4 t[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (k0 + j < top) t[j] = *reinterpret_cast<const float4*>(pairs + (n * top + k0 + j) * width + c);
-#pragma unroll
-          for (int j = 0; j < 8; ++j)
-            if (k0 + j < top) {
-              e.x += t[j].x; e.y += t[j].y; e.z += t[j].z; e.w += t[j].w;
-            }
-        }
-        v.x = fmaf(pair_weight, e.x, v.x); v.y = fmaf(pair_weight, e.y, v.y);
-        v.z = fmaf(pair_weight, e.z, v.z); v.w = fmaf(pair_weight, e.w, v.w);
-      }
-      *reinterpret_cast<float4*>(row + c) = v;
-      ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+  for (int c = threadIdx.x; c < width; c += blockDim.x) {
+    float v = 0.f;
+    if (src != nullptr) {
+      for (int s = 0; s < n_splits; ++s) v += to_f32<TS>(src[s * split_stride + n * width + c]);
+      v = as_output(v, round_sum);
     }
-  } else {
-    for (int c = threadIdx.x; c < width; c += blockDim.x) {
-      float v = 0.f;
-      if (src != nullptr) {
-        for (int s = 0; s < n_splits; ++s) v += to_f32<TS>(src[s * split_stride + n * width + c]);
-        v = as_output(v, round_sum);
-      }
-      if (pairs != nullptr) {
-        float e = 0.f;
-        for (int k = 0; k < top; ++k) e += pairs[(n * top + k) * width + c];
-        v = fmaf(pair_weight, e, v);
-      }
-      row[c] = v;
-      ss = fmaf(v, v, ss);
+    if (pairs != nullptr) {
+      float e = 0.f;
+      for (int k = 0; k < top; ++k) e += pairs[(n * top + k) * width + c];
+      v = fmaf(pair_weight, e, v);
     }
+    row[c] = v;
+    ss = fmaf(v, v, ss);
   }
   const float total = block_sum(ss, scratch);
   const float inv = 1.f / sqrtf(total / static_cast<float>(width) + eps);
-  if (VEC) {
-    for (int c = 4 * threadIdx.x; c < width; c += 4 * blockDim.x) {
-      const float4 wv = na_load4<TW>(w + c), b = *reinterpret_cast<const float4*>(row + c);
-      const float off = unit_offset ? 1.f : 0.f;
-      float4 r = *reinterpret_cast<const float4*>(residual + n * width + c);
-      r.x += b.x * inv * (wv.x + off); r.y += b.y * inv * (wv.y + off);
-      r.z += b.z * inv * (wv.z + off); r.w += b.w * inv * (wv.w + off);
-      *reinterpret_cast<float4*>(residual + n * width + c) = r;
-      if (out != nullptr)
-        *reinterpret_cast<uint2*>(out + n * width + c) = make_uint2(pack_bf16x2(r.x, r.y), pack_bf16x2(r.z, r.w));
-    }
-    return;
-  }
   for (int c = threadIdx.x; c < width; c += blockDim.x) {
     const float wv = to_f32<TW>(w[c]) + (unit_offset ? 1.f : 0.f);
     const float r = residual[n * width + c] + row[c] * inv * wv;
     residual[n * width + c] = r;
     if (out != nullptr) out[n * width + c] = from_f32<TO>(r);
+  }
+}
+
+// Fast form: P pieces of four columns a thread, in registers throughout; the branch's slices, the token's expert rows, the residual and
+// the weight are all asked for before any is used (ask_slices in common.h says why that takes care).  Bound by the launch and one trip
+// to memory and back each way.  Behind copies of 16 MB and of its input in a replayed graph, four rows of 2,048 in bfloat16 alone / with two expert
+// rows, us: with 256 threads whose loads waited one for another 3.6 / 4.6, now 2.0 / 2.3.
+constexpr uint32_t ROW_ROUND = 1u << 16, ROW_UNIT = 1u << 17;  // `how`: bits 0-15 slices; 19-23 waves
+template <typename TS, typename TW, int P>
+__global__ __launch_bounds__(1024) void norm_add_vec_kernel(float* __restrict__ residual, const TS* __restrict__ src,
+                                                            const float* __restrict__ pairs, const TW* __restrict__ w,
+                                                            bf16_t* __restrict__ out, int width, uint32_t how, int top,
+                                                            uint32_t split_stride, float pair_weight, float eps) {
+  __shared__ float scratch[16];
+  constexpr int G = P == 1 ? 8 : 4, GS = sizeof(TS) == 2 ? 1 : G;  // expert rows and slices asked for at once
+  const int n_splits = how & 0xffffu, waves = (how >> 19) & 31, round_sum = (how & ROW_ROUND) != 0;
+  const size_t n = blockIdx.x;
+  float4 rs[P];
+  typename Four<TW>::raw wr[P];
+  uint32_t at[P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) at[k] = min(4 * (static_cast<int>(threadIdx.x) + 64 * waves * k), width - 4);
+  const TS* p = src + n * width;
+  const float* q = pairs + n * top * width;
+  typename Four<TS>::raw d[GS][P];
+  float4 e[G][P];
+  if (src != nullptr) ask_slices<GS, P, TS>(p, at, n_splits, split_stride, d);
+  if (pairs != nullptr) ask_slices<G, P, float>(q, at, top, width, e);
+#pragma unroll
+  for (int k = 0; k < P; ++k) {
+    rs[k] = four_at<float>(residual + n * width + at[k]);
+    wr[k] = Four<TW>::at(w + at[k]);
+  }
+  float4 v[P], es[P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) v[k] = es[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (src != nullptr) {
+    join_slices<GS, P, TS>(d, n_splits, v);
+    join_rest<GS, P, TS>(p, at, n_splits, split_stride, v);
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+      v[k] = make_float4(as_output(v[k].x, round_sum), as_output(v[k].y, round_sum), as_output(v[k].z, round_sum), as_output(v[k].w, round_sum));
+  }
+  if (pairs != nullptr) {
+    join_slices<G, P, float>(e, top, es);
+    join_rest<G, P, float>(q, at, top, width, es);
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+      v[k] = make_float4(fmaf(pair_weight, es[k].x, v[k].x), fmaf(pair_weight, es[k].y, v[k].y), fmaf(pair_weight, es[k].z, v[k].z),
+                         fmaf(pair_weight, es[k].w, v[k].w));
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < P; ++k) {
+    const bool in = 4 * (static_cast<int>(threadIdx.x) + 64 * waves * k) < width;
+    ss = in ? fmaf(v[k].x, v[k].x, fmaf(v[k].y, v[k].y, fmaf(v[k].z, v[k].z, fmaf(v[k].w, v[k].w, ss)))) : ss;
+  }
+  const float total = block_sum_first(ss, scratch, waves);
+  const float inv = 1.f / sqrtf(total / static_cast<float>(width) + eps), off = how & ROW_UNIT ? 1.f : 0.f;
+#pragma unroll
+  for (int k = 0; k < P; ++k) {
+    const float4 wv = Four<TW>::wide(wr[k]);
+    const float4 r = make_float4(fmaf(v[k].x * inv, wv.x + off, rs[k].x), fmaf(v[k].y * inv, wv.y + off, rs[k].y),
+                                 fmaf(v[k].z * inv, wv.z + off, rs[k].z), fmaf(v[k].w * inv, wv.w + off, rs[k].w));
+    if (4 * (static_cast<int>(threadIdx.x) + 64 * waves * k) >= width) continue;
+    put_four<float>(residual + n * width + at[k], r);
+    if (out != nullptr) put_four<bf16_t>(out + n * width + at[k], r);
   }
 }
 
@@ -151,15 +151,23 @@ extern "C" int yk_norm_add(float* residual, const void* src, int src_dtype, int 
   const size_t stride = static_cast<size_t>(n_rows) * width;
   const size_t lds = (static_cast<size_t>(width) + 17) * sizeof(float);
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const bool vec = width % 4 == 0 && al(residual) && al(src) && al(pairs) && al(w) && al(out);
+  const bool vec = width % 4 == 0 && al(residual) && al(src) && al(pairs) && al(w) && al(out) && n_splits < 1 << 16 && stride < size_t{1} << 32;
+  // a piece a thread where rows are few, two where they fill the chip (as add_rmsnorm), never more than 1,024 threads
+  const int threads = std::max(64, std::min(1024, ((n_rows >= 1024 ? width / 8 : width / 4) + 63) / 64 * 64));
+  const int pieces = (width / 4 + threads - 1) / threads;
+  const uint32_t how = static_cast<uint32_t>(n_splits & 0xffff) | (round_sum ? ROW_ROUND : 0u) | (unit_offset ? ROW_UNIT : 0u) |
+                       static_cast<uint32_t>(threads / 64) << 19;
+#define YK_VEC(TS, TW, P)                                                                                    \
+  norm_add_vec_kernel<TS, TW, P><<<n_rows, threads, 0, stream>>>(                                            \
+      residual, static_cast<const TS*>(src), pairs, static_cast<const TW*>(w), static_cast<bf16_t*>(out), width, how, top, \
+      static_cast<uint32_t>(stride), pair_weight, eps)
 #define YK_CASE(SD, TS, WD, TW)                                                                            \
   if ((src == nullptr || src_dtype == SD) && w_dtype == WD) {                                                \
-    if (vec)                                                                                                 \
-      norm_add_kernel<TS, TW, bf16_t, true><<<n_rows, 256, lds, stream>>>(                                   \
-          residual, static_cast<const TS*>(src), n_splits, stride, round_sum, pairs, top, pair_weight,       \
-          static_cast<const TW*>(w), unit_offset, eps, static_cast<bf16_t*>(out), width);                    \
+    if (vec && pieces <= 1) YK_VEC(TS, TW, 1);                                                               \
+    else if (vec && pieces <= 2) YK_VEC(TS, TW, 2);                                                          \
+    else if (vec) YK_VEC(TS, TW, 4);                                                                         \
     else                                                                                                     \
-      norm_add_kernel<TS, TW, bf16_t, false><<<n_rows, 256, lds, stream>>>(                                  \
+      norm_add_kernel<TS, TW, bf16_t><<<n_rows, 256, lds, stream>>>(                                         \
           residual, static_cast<const TS*>(src), n_splits, stride, round_sum, pairs, top, pair_weight,       \
           static_cast<const TW*>(w), unit_offset, eps, static_cast<bf16_t*>(out), width);                    \
     return yk_check_launch("norm_add");                                                                      \
@@ -169,6 +177,7 @@ extern "C" int yk_norm_add(float* residual, const void* src, int src_dtype, int 
   YK_CASE(YK_BF16, bf16_t, YK_F32, float)
   YK_CASE(YK_BF16, bf16_t, YK_BF16, bf16_t)
 #undef YK_CASE
+#undef YK_VEC
   return yk_fail("norm_add: unsupported dtype combination");
 }
 
@@ -201,28 +210,6 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float* scratch) {
   b = row_sum(lane % 16 < n_waves ? scratch[16 + lane % 16] : 0.f);
 }
 
-__device__ __forceinline__ float4 sum_term4(const SumTerm& t, size_t at, size_t stride) {
-  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (t.bf16) {
-    v = na_load4<bf16_t>(static_cast<const bf16_t*>(t.src) + at);
-  } else {
-    const float* p = static_cast<const float*>(t.src) + at;
-    for (int s0 = 0; s0 < t.n_splits; s0 += 8) {
-      float4 x[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (s0 + j < t.n_splits) x[j] = *reinterpret_cast<const float4*>(p + (s0 + j) * stride);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (s0 + j < t.n_splits) {
-          v.x += x[j].x; v.y += x[j].y; v.z += x[j].z; v.w += x[j].w;
-        }
-    }
-    v = make_float4(as_output(v.x, t.round_sum), as_output(v.y, t.round_sum), as_output(v.z, t.round_sum), as_output(v.w, t.round_sum));
-  }
-  return v;
-}
-
 __device__ __forceinline__ float sum_term1(const SumTerm& t, size_t at, size_t stride) {
   if (t.bf16) return to_f32<bf16_t>(static_cast<const bf16_t*>(t.src)[at]);
   float v = 0.f;
@@ -234,64 +221,113 @@ __device__ __forceinline__ float dot4(float4 v) { return fmaf(v.x, v.x, fmaf(v.y
 __device__ __forceinline__ float4 mul4(float4 a, float4 b) { return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w); }
 __device__ __forceinline__ float4 scaled4(float4 a, float s) { return make_float4(a.x * s, a.y * s, a.z * s, a.w * s); }
 
-// P: pieces of 4 columns x blockDim.x a thread holds
-template <typename TW, int P>
-__global__ __launch_bounds__(1024) void sum_norm_vec_kernel(float* __restrict__ residual, SumTerm ta, SumTerm tb, int has_b,
-                                                           size_t stride, float branch_scale, const TW* __restrict__ cw,
-                                                           float residual_scale, const TW* __restrict__ w, int unit_offset,
-                                                           float eps, bf16_t* __restrict__ out, int width) {
-  __shared__ float scratch[34];
+// P: pieces of 4 columns a thread holds; A16: the first term is bfloat16 rows; B: 0 no second term, 1 float32 rows or slices, 2 bfloat16
+// rows.  What a row needs is asked for before any of it is used.  Behind copies of 16 MB and of its input, eight rows of 2,048, one bfloat16 term / one of
+// eight slices / two bfloat16 terms with their own norms, us: with loads that waited one for another 2.3 / 3.3 / 3.9, now 2.2 / 3.1 / 3.1.
+// `how`: bits 0-7 and 8-15 the terms' slices; 19-23 waves; and the bits below
+constexpr uint32_t SUM_ROUND_A = 1u << 16, SUM_ROUND_B = 1u << 17, SUM_UNIT = 1u << 18, SUM_AW = 1u << 24, SUM_BW = 1u << 25, SUM_CW = 1u << 26;
+template <typename TW, bool A16, int B, int P>
+__global__ __launch_bounds__(1024) void sum_norm_vec_kernel(float* __restrict__ residual, const void* __restrict__ a_src,
+                                                            const void* __restrict__ b_src, const TW* __restrict__ w,
+                                                            bf16_t* __restrict__ out, int width, uint32_t how, uint32_t stride,
+                                                            float residual_scale, const TW* __restrict__ aw, const TW* __restrict__ bw,
+                                                            const TW* __restrict__ cw, float branch_scale, float eps, float a_eps,
+                                                            float b_eps) {
+  using TA = std::conditional_t<A16, bf16_t, float>;
+  using TB = std::conditional_t<B == 2, bf16_t, float>;
+  constexpr int GA = A16 ? 1 : P == 1 ? 8 : 4, GB = B != 1 ? 1 : P == 1 ? 8 : 4;  // slices asked for at once
+  __shared__ float scratch[3][16];
+  const int na = how & 0xff, nb = (how >> 8) & 0xff, waves = (how >> 19) & 31;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const size_t n = blockIdx.x;
-  const float4 one = make_float4(1.f, 1.f, 1.f, 1.f), zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  float4 a[P], b[P], rs[P], wn[P], wc[P], wa[P], wb[P];
-  float sa = 0.f, sb = 0.f;
+  uint32_t at[P];
+  float4 rs[P];
+  typename Four<TW>::raw wn[P], wc[P], wa[P], wb[P];
+  const TA* pa = static_cast<const TA*>(a_src) + n * width;
+  const TB* pb = static_cast<const TB*>(b_src) + n * width;
+  typename Four<TA>::raw da[GA][P];
+  typename Four<TB>::raw db[GB][P];
+#pragma unroll
+  for (int k = 0; k < P; ++k) at[k] = min(4 * (static_cast<int>(threadIdx.x) + 64 * waves * k), width - 4);
+  ask_slices<GA, P, TA>(pa, at, na, stride, da);
+  if (B) ask_slices<GB, P, TB>(pb, at, nb, stride, db);
 #pragma unroll
   for (int k = 0; k < P; ++k) {
-    const int c = 4 * (threadIdx.x + blockDim.x * k);
-    a[k] = b[k] = rs[k] = wn[k] = zero;
-    wc[k] = wa[k] = wb[k] = one;
-    if (c >= width) continue;
-    const size_t at = n * width + c;
-    rs[k] = *reinterpret_cast<const float4*>(residual + at);
-    wn[k] = na_load4<TW>(w + c);
-    if (cw != nullptr) wc[k] = na_load4<TW>(cw + c);
-    if (ta.w != nullptr) wa[k] = na_load4<TW>(static_cast<const TW*>(ta.w) + c);
-    if (has_b && tb.w != nullptr) wb[k] = na_load4<TW>(static_cast<const TW*>(tb.w) + c);
-    a[k] = sum_term4(ta, at, stride);
-    if (has_b) b[k] = sum_term4(tb, at, stride);
+    rs[k] = four_at<float>(residual + n * width + at[k]);
+    wn[k] = Four<TW>::at(w + at[k]);
+    wc[k] = wa[k] = wb[k] = Four<TW>::all(1.f);
   }
+  arguments_now(aw, bw, cw);
+  if (how & SUM_AW) {
 #pragma unroll
-  for (int k = 0; k < P; ++k) sa += dot4(a[k]), sb += dot4(b[k]);
+    for (int k = 0; k < P; ++k) wa[k] = Four<TW>::at(aw + at[k]);
+  }
+  if (B && (how & SUM_BW)) {
+#pragma unroll
+    for (int k = 0; k < P; ++k) wb[k] = Four<TW>::at(bw + at[k]);
+  }
+  if (how & SUM_CW) {
+#pragma unroll
+    for (int k = 0; k < P; ++k) wc[k] = Four<TW>::at(cw + at[k]);
+  }
+  float4 a[P], b[P];
+  auto term = [&](auto& d, auto p, int slices, int round_sum, float4 (&s)[P], auto type, auto group) {
+    using T = decltype(type);
+    constexpr int G = decltype(group)::value;
+#pragma unroll
+    for (int k = 0; k < P; ++k) s[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    join_slices<G, P, T>(d, slices, s);
+    join_rest<G, P, T>(p, at, slices, stride, s);
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int k = 0; k < P; ++k)
+        s[k] = make_float4(as_output(s[k].x, round_sum), as_output(s[k].y, round_sum), as_output(s[k].z, round_sum), as_output(s[k].w, round_sum));
+    }
+  };
+  term(da, pa, na, (how & SUM_ROUND_A) != 0, a, TA{}, std::integral_constant<int, GA>{});
+  if (B) term(db, pb, nb, (how & SUM_ROUND_B) != 0, b, TB{}, std::integral_constant<int, GB>{});
   float ia = 1.f, ib = 1.f;
-  if (ta.w != nullptr || (has_b && tb.w != nullptr)) {
-    block_sum2(sa, sb, scratch);
-    if (ta.w != nullptr) ia = 1.f / sqrtf(sa / static_cast<float>(width) + ta.eps);
-    if (has_b && tb.w != nullptr) ib = 1.f / sqrtf(sb / static_cast<float>(width) + tb.eps);
+  if (how & (SUM_AW | SUM_BW)) {
+    float sa = 0.f, sb = 0.f;
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+      const bool in = 4 * (static_cast<int>(threadIdx.x) + 64 * waves * k) < width;
+      sa += in ? dot4(a[k]) : 0.f;
+      if (B) sb += in ? dot4(b[k]) : 0.f;
+    }
+    sa = wave_sum(sa);
+    if (B) sb = wave_sum(sb);
+    if (lane == 0) scratch[0][wave] = sa, scratch[1][wave] = sb;
+    __syncthreads();
+    sa = row_sum(lane % 16 < waves ? scratch[0][lane % 16] : 0.f);
+    sb = row_sum(lane % 16 < waves ? scratch[1][lane % 16] : 0.f);
+    if (how & SUM_AW) ia = 1.f / sqrtf(sa / static_cast<float>(width) + a_eps);
+    if (B && (how & SUM_BW)) ib = 1.f / sqrtf(sb / static_cast<float>(width) + b_eps);
   }
-  float ss = 0.f, none = 0.f;
+  float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < P; ++k) {
-    float4 v = scaled4(mul4(a[k], wa[k]), ia);
-    if (has_b) {
-      const float4 u = mul4(b[k], wb[k]);
+    float4 v = scaled4(mul4(a[k], Four<TW>::wide(wa[k])), ia);
+    if (B) {
+      const float4 u = mul4(b[k], Four<TW>::wide(wb[k]));
       v = make_float4(fmaf(u.x, ib, v.x), fmaf(u.y, ib, v.y), fmaf(u.z, ib, v.z), fmaf(u.w, ib, v.w));
     }
-    v = mul4(scaled4(v, branch_scale), wc[k]);
+    v = mul4(scaled4(v, branch_scale), Four<TW>::wide(wc[k]));
     rs[k] = make_float4(fmaf(residual_scale, rs[k].x, v.x), fmaf(residual_scale, rs[k].y, v.y), fmaf(residual_scale, rs[k].z, v.z),
                         fmaf(residual_scale, rs[k].w, v.w));
-    if (4 * (threadIdx.x + static_cast<int>(blockDim.x) * k) < width) ss += dot4(rs[k]);
+    ss += 4 * (static_cast<int>(threadIdx.x) + 64 * waves * k) < width ? dot4(rs[k]) : 0.f;
   }
-  block_sum2(ss, none, scratch);
+  ss = block_sum_first(ss, scratch[2], waves);
   const float inv = 1.f / sqrtf(ss / static_cast<float>(width) + eps);
-  const float off = unit_offset ? 1.f : 0.f;
+  const float off = how & SUM_UNIT ? 1.f : 0.f;
 #pragma unroll
   for (int k = 0; k < P; ++k) {
-    const int c = 4 * (threadIdx.x + blockDim.x * k);
-    if (c >= width) continue;
-    const float4 r = make_float4(rs[k].x * inv * (wn[k].x + off), rs[k].y * inv * (wn[k].y + off), rs[k].z * inv * (wn[k].z + off),
-                                 rs[k].w * inv * (wn[k].w + off));
-    *reinterpret_cast<float4*>(residual + n * width + c) = r;
-    if (out != nullptr) *reinterpret_cast<uint2*>(out + n * width + c) = make_uint2(pack_bf16x2(r.x, r.y), pack_bf16x2(r.z, r.w));
+    const float4 wv = Four<TW>::wide(wn[k]);
+    const float4 r = make_float4(rs[k].x * inv * (wv.x + off), rs[k].y * inv * (wv.y + off), rs[k].z * inv * (wv.z + off),
+                                 rs[k].w * inv * (wv.w + off));
+    if (4 * (static_cast<int>(threadIdx.x) + 64 * waves * k) >= width) continue;
+    put_four<float>(residual + n * width + at[k], r);
+    if (out != nullptr) put_four<bf16_t>(out + n * width + at[k], r);
   }
 }
 
@@ -355,24 +391,41 @@ extern "C" int yk_sum_norm(float* residual, const void* a_src, int a_dtype, int 
   const int has_b = b_src != nullptr;
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool vec = width % 4 == 0 && width <= 4096 && al(residual) && al(a_src) && al(b_src) && al(a_w) && al(b_w) && al(channel_w) &&
-                   al(w) && al(out);
+                   al(w) && al(out) && a_splits <= 255 && b_splits <= 255 && stride < size_t{1} << 32;
   // a piece a thread for few rows, two where rows fill the chip (eight rows of 2,048: 6.2 -> 4.2 us with twice the threads)
-#define YK_ARGS(TW)                                                                                                        \
-  residual, ta, tb, has_b, stride, branch_scale, static_cast<const TW*>(channel_w), residual_scale, static_cast<const TW*>(w), \
-      unit_offset, eps, static_cast<bf16_t*>(out), width
+  const int pieces = n_rows < 1024 ? 1 : 2, threads = (width / 4 + 64 * pieces - 1) / (64 * pieces) * 64;
+  const uint32_t how = static_cast<uint32_t>(a_splits & 0xff) | static_cast<uint32_t>(b_splits & 0xff) << 8 | (a_round ? SUM_ROUND_A : 0u) |
+                       (b_round ? SUM_ROUND_B : 0u) | (unit_offset ? SUM_UNIT : 0u) | static_cast<uint32_t>(threads / 64) << 19 |
+                       (a_w ? SUM_AW : 0u) | (has_b && b_w ? SUM_BW : 0u) | (channel_w ? SUM_CW : 0u);
+#define YK_VEC(TW, A16, B, P)                                                                                              \
+  sum_norm_vec_kernel<TW, A16, B, P><<<n_rows, threads, 0, stream>>>(                                                      \
+      residual, a_src, b_src, static_cast<const TW*>(w), static_cast<bf16_t*>(out), width, how, static_cast<uint32_t>(stride), residual_scale, \
+      static_cast<const TW*>(a_w), static_cast<const TW*>(b_w), static_cast<const TW*>(channel_w), branch_scale, eps, a_eps, b_eps)
+#define YK_VEC_P(TW, A16, B)              \
+  if (pieces == 1) YK_VEC(TW, A16, B, 1); \
+  else YK_VEC(TW, A16, B, 2)
+#define YK_VEC_B(TW, A16)                 \
+  if (!has_b) { YK_VEC_P(TW, A16, 0); }   \
+  else if (tb.bf16) { YK_VEC_P(TW, A16, 2); } \
+  else { YK_VEC_P(TW, A16, 1); }
 #define YK_CASE(WD, TW)                                                                                                    \
   if (w_dtype == WD) {                                                                                                     \
-    if (vec && n_rows < 1024)                                                                                              \
-      sum_norm_vec_kernel<TW, 1><<<n_rows, (width / 4 + 63) / 64 * 64, 0, stream>>>(YK_ARGS(TW));                          \
-    else if (vec)                                                                                                          \
-      sum_norm_vec_kernel<TW, 2><<<n_rows, (width / 4 + 127) / 128 * 64, 0, stream>>>(YK_ARGS(TW));                        \
-    else                                                                                                                   \
-      sum_norm_kernel<TW><<<n_rows, 256, ((has_b ? 2 : 1) * static_cast<size_t>(width) + 34) * sizeof(float), stream>>>(YK_ARGS(TW)); \
+    if (vec && ta.bf16) {                                                                                                  \
+      YK_VEC_B(TW, true)                                                                                                   \
+    } else if (vec) {                                                                                                      \
+      YK_VEC_B(TW, false)                                                                                                  \
+    } else {                                                                                                               \
+      sum_norm_kernel<TW><<<n_rows, 256, ((has_b ? 2 : 1) * static_cast<size_t>(width) + 34) * sizeof(float), stream>>>(   \
+          residual, ta, tb, has_b, stride, branch_scale, static_cast<const TW*>(channel_w), residual_scale,                \
+          static_cast<const TW*>(w), unit_offset, eps, static_cast<bf16_t*>(out), width);                                  \
+    }                                                                                                                      \
     return yk_check_launch("sum_norm");                                                                                    \
   }
   YK_CASE(YK_F32, float)
   YK_CASE(YK_BF16, bf16_t)
 #undef YK_CASE
-#undef YK_ARGS
+#undef YK_VEC_B
+#undef YK_VEC_P
+#undef YK_VEC
   return yk_fail("sum_norm: unsupported weight dtype");
 }

@@ -117,77 +117,110 @@ __host__ __device__ inline size_t cache_v_offset(bool tiled, int page_size, int 
   return static_cast<size_t>(slot / 64) * 64 * head_dim + piece * 8 + j % 8;
 }
 
-// Four neighbouring values as float32, and back.
+// Four neighbouring values: as they lie in memory, as float32, and back.  A load under a condition (a weight that may be absent) is kept
+// as it lies until the condition's end: widened under it, it would be waited for there.
 template <typename T>
-__device__ __forceinline__ float4 four_at(const T* p);
+struct Four;
 template <>
-__device__ __forceinline__ float4 four_at<float>(const float* p) {
-  return *reinterpret_cast<const float4*>(p);
-}
+struct Four<float> {
+  typedef float4 raw;
+  static __device__ __forceinline__ raw at(const float* p) { return *reinterpret_cast<const float4*>(p); }
+  static __device__ __forceinline__ raw all(float v) { return make_float4(v, v, v, v); }
+  static __device__ __forceinline__ float4 wide(raw r) { return r; }
+  static __device__ __forceinline__ void put(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
+};
 template <>
-__device__ __forceinline__ float4 four_at<bf16_t>(const bf16_t* p) {
-  const uint2 raw = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u), __uint_as_float(raw.y << 16),
-                     __uint_as_float(raw.y & 0xffff0000u));
+struct Four<bf16_t> {
+  typedef uint2 raw;
+  static __device__ __forceinline__ raw at(const bf16_t* p) { return *reinterpret_cast<const uint2*>(p); }
+  static __device__ __forceinline__ raw all(float v) { return make_uint2(pack_bf16x2(v, v), pack_bf16x2(v, v)); }
+  static __device__ __forceinline__ float4 wide(raw r) {
+    return make_float4(__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xffff0000u), __uint_as_float(r.y << 16),
+                       __uint_as_float(r.y & 0xffff0000u));
+  }
+  static __device__ __forceinline__ void put(bf16_t* p, float4 v) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
+  }
+};
+template <typename T>
+__device__ __forceinline__ float4 four_at(const T* p) {
+  return Four<T>::wide(Four<T>::at(p));
 }
 template <typename T>
-__device__ __forceinline__ void put_four(T* p, float4 v);
-template <>
-__device__ __forceinline__ void put_four<float>(float* p, float4 v) {
-  *reinterpret_cast<float4*>(p) = v;
-}
-template <>
-__device__ __forceinline__ void put_four<bf16_t>(bf16_t* p, float4 v) {
-  *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
+__device__ __forceinline__ void put_four(T* p, float4 v) {
+  Four<T>::put(p, v);
 }
 
-// `left` slices of IT pieces of four values, `stride` elements from one slice to the next, added to s in the slices' order.  SL of
-// them (at most) are asked for before the first is used, and nothing that is asked for hangs on a condition: a kernel of a few
-// microseconds lasts as long as the waits for memory it makes one after another, and the compiler moves a load to the condition
-// that its value alone is used under, and waits there.  So slices beyond the last are read from the last and masked to +0 with a
-// number that the compiler cannot take for a condition (a sum that began with +0 is never -0, and +0 leaves it as it is).
-template <int SL, int IT, typename T>
-__device__ __forceinline__ void add_slices(const T* const (&p)[IT], int left, size_t stride, float4 (&s)[IT]) {
-  float4 d[SL][IT];
-  size_t at = 0;
+// `left` slices of IT pieces of four values (`at` elements from p, which is the same in every lane), `stride` elements from one slice to the next, added to s in the slices' order.  SL of
+// them (at most) are asked for before the first is used: a kernel of a few microseconds lasts as long as the waits for memory it makes
+// one after another, and the compiler moves a load to the condition that its value alone is used under, and waits there.  So they are
+// asked for in groups (one, two, four, eight: few slices ask for few), inside a group unconditionally; what lies beyond the last
+// slice is read from the last and masked to +0 with a number that the compiler cannot take for a condition (a sum that began
+// with +0 is never -0, and +0 leaves it as it is).  ask_slices and join_slices are the two halves, for kernels that have more to ask for in
+// between.
+template <int SL, int IT, typename T, int FROM = 0, int TO = 1>
+__device__ __forceinline__ void ask_slices(const T* p, const uint32_t (&at)[IT], int left, size_t stride, typename Four<T>::raw (&d)[SL][IT]) {
 #pragma unroll
-  for (int j = 0; j < SL; ++j) {
+  for (int j = FROM; j < TO; ++j) {
 #pragma unroll
-    for (int k = 0; k < IT; ++k) d[j][k] = four_at<T>(p[k] + at);
-    at += j + 1 < left ? stride : 0;
+    for (int k = 0; k < IT; ++k) d[j][k] = Four<T>::at(p + at[k]);
+    p += j + 1 < left ? stride : 0;
   }
+  if constexpr (TO < SL) {
+    if (left > TO) ask_slices<SL, IT, T, TO, 2 * TO>(p, at, left, stride, d);
+  }
+}
+template <int SL, int IT, typename T, int FROM = 0, int TO = 1>
+__device__ __forceinline__ void join_slices(const typename Four<T>::raw (&d)[SL][IT], int left, float4 (&s)[IT]) {
 #pragma unroll
-  for (int j = 0; j < SL; ++j) {
+  for (int j = FROM; j < TO; ++j) {
     const uint32_t keep = __builtin_amdgcn_readfirstlane((j - left) >> 31);
     auto kept = [&](float v) { return __uint_as_float(__float_as_uint(v) & keep); };
 #pragma unroll
     for (int k = 0; k < IT; ++k) {
-      s[k].x += kept(d[j][k].x);
-      s[k].y += kept(d[j][k].y);
-      s[k].z += kept(d[j][k].z);
-      s[k].w += kept(d[j][k].w);
+      const float4 v = Four<T>::wide(d[j][k]);
+      s[k].x += kept(v.x);
+      s[k].y += kept(v.y);
+      s[k].z += kept(v.z);
+      s[k].w += kept(v.w);
+    }
+  }
+  if constexpr (TO < SL) {
+    if (left > TO) join_slices<SL, IT, T, TO, 2 * TO>(d, left, s);
+  }
+}
+// The rest of the slices after the first SL have joined, SL at a time.
+template <int SL, int IT, typename T>
+__device__ __forceinline__ void join_rest(const T* p, const uint32_t (&at)[IT], int left, size_t stride, float4 (&s)[IT]) {
+  if constexpr (sizeof(T) == 4) {  // (slices are float32)
+    for (left -= SL; left > 0; left -= SL) {
+      typename Four<T>::raw d[SL][IT];
+      p += SL * stride;
+      ask_slices<SL, IT, T>(p, at, left, stride, d);
+      join_slices<SL, IT, T>(d, left, s);
     }
   }
 }
-// The sum over n >= 1 slices of IT pieces of four values: one slice is one load, and of more up to 16 (8 with two pieces, 4 with more)
-// are in flight at a time.
+// slices in flight at a time for IT pieces a thread: what the registers hold
+template <typename T, int IT>
+constexpr int slices_at_once = sizeof(T) == 2 ? 1 : IT == 1 ? 16 : IT == 2 ? 8 : 4;
+// The sum over n >= 1 slices of IT pieces of four values, `at` elements from p.
 template <int IT, typename T>
-__device__ __forceinline__ void sum_slices(const T* (&p)[IT], int n, size_t stride, float4 (&s)[IT]) {
-  if (sizeof(T) == 2 || n == 1) {  // (slices are float32)
-#pragma unroll
-    for (int k = 0; k < IT; ++k) s[k] = four_at<T>(p[k]);
-    return;
-  }
+__device__ __forceinline__ void sum_slices(const T* p, const uint32_t (&at)[IT], int n, size_t stride, float4 (&s)[IT]) {
+  constexpr int SL = slices_at_once<T, IT>;
 #pragma unroll
   for (int k = 0; k < IT; ++k) s[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-  constexpr int MOST = IT == 1 ? 16 : IT == 2 ? 8 : 4;
-  for (; n > MOST / 2; n -= MOST) {
-    add_slices<MOST, IT, T>(p, n, stride, s);
-#pragma unroll
-    for (int k = 0; k < IT; ++k) p[k] += MOST * stride;
-  }
-  if (n > MOST / 4) add_slices<MOST / 2, IT, T>(p, n, stride, s);
-  else if (n > 0) add_slices<MOST / 4, IT, T>(p, n, stride, s);
+  do {
+    typename Four<T>::raw d[SL][IT];
+    ask_slices<SL, IT, T>(p, at, n, stride, d);
+    join_slices<SL, IT, T>(d, n, s);
+    p += SL * stride;
+    n -= SL;
+  } while (sizeof(T) == 4 && n > 0);  // (slices are float32)
+}
+// Arguments that did not come with the launch, asked for here and not where they are first used, one wait after the other.
+__device__ __forceinline__ void arguments_now(const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr) {
+  asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d));
 }
 
 // Sums and maxima over a wave's 64 lanes, all of them active, in every lane: partners 32, 16, 8, 4, 2 and 1 lanes away, as moves between

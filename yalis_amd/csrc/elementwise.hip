@@ -273,7 +273,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(
   float* res = residual + src * width;
   const TD* del = delta + from * width;
   float4 v[NORM_IT], w[NORM_IT];
-  int at[NORM_IT];
+  uint32_t at[NORM_IT];
 #pragma unroll
   for (int it = 0; it < NORM_IT; ++it) {
     at[it] = min((static_cast<int>(threadIdx.x) + it * 64 * waves) * 4, width - 4);
@@ -281,11 +281,8 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(
     w[it] = four_at<TW>(weight + at[it]);
   }
   if (FRESH || n_splits > 0) {
-    const TD* p[NORM_IT];
     float4 ds[NORM_IT];
-#pragma unroll
-    for (int it = 0; it < NORM_IT; ++it) p[it] = del + at[it];
-    sum_slices<NORM_IT, TD>(p, n_splits, split_stride, ds);
+    sum_slices<NORM_IT, TD>(del, at, n_splits, split_stride, ds);
 #pragma unroll
     for (int it = 0; it < NORM_IT; ++it) {
       v[it].x += as_output(ds[it].x, round_sum);
@@ -669,8 +666,9 @@ extern "C" int yk_rope_append(const void* src, int src_dtype, int n_splits, int 
 // of gu are [gate | up] (group 0) or alternate in groups: `group` gate columns, then the
 // `group` up columns that belong to them, and so on (the layout the fused product uses).
 // With n_splits > 1, gu holds unreduced float32 K slices [n_splits][rows][2 * inter].
-__device__ __forceinline__ size_t gate_col(size_t j, int inter, int group) {
-  return group ? (j / group) * 2 * group + j % group : j;
+template <typename I>
+__device__ __forceinline__ I gate_col(I j, int inter, int group) {
+  return group ? (j / static_cast<I>(group)) * 2 * group + j % static_cast<I>(group) : j;
 }
 __device__ __forceinline__ size_t up_offset(int inter, int group) { return group ? group : inter; }
 
@@ -693,35 +691,24 @@ __global__ void gated_act_kernel(const TS* __restrict__ gu, int n_splits, size_t
   }
 }
 
-// four outputs per thread, no loop (inter a multiple of 4)
+// four outputs per thread, no loop (inter a multiple of 4); a workgroup stays in one row, and up to eight slices of both halves are asked
+// for at once
 template <typename TS, typename TO>
-__global__ void gated_act_vec_kernel(const TS* __restrict__ gu, int n_splits, size_t split_stride, int round_sum,
-                                     TO* __restrict__ out, int inter, size_t total_vec, int act, int group, float p0, float p1) {
-  const size_t v = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
-  if (v >= total_vec) return;
-  const int per_row = inter / 4;
-  const size_t n = v / per_row;
-  const int j = static_cast<int>(v % per_row) * 4;
-  const TS* p = gu + n * 2 * inter + gate_col(j, inter, group);  // four columns of one group (group % 4 == 0)
-  const size_t up = up_offset(inter, group);
-  float4 g = four_at<TS>(p), u = four_at<TS>(p + up);
-  for (int s0 = 1; s0 < n_splits; s0 += 2) {  // two slices in flight
-    const int s1 = min(s0 + 1, n_splits - 1);
-    const float4 g2 = four_at<TS>(p + s0 * split_stride), u2 = four_at<TS>(p + s0 * split_stride + up);
-    const float4 g3 = four_at<TS>(p + s1 * split_stride), u3 = four_at<TS>(p + s1 * split_stride + up);
-    g.x += g2.x; g.y += g2.y; g.z += g2.z; g.w += g2.w;
-    u.x += u2.x; u.y += u2.y; u.z += u2.z; u.w += u2.w;
-    if (s0 + 1 < n_splits) {
-      g.x += g3.x; g.y += g3.y; g.z += g3.z; g.w += g3.w;
-      u.x += u3.x; u.y += u3.y; u.z += u3.z; u.w += u3.w;
-    }
-  }
+__global__ __launch_bounds__(256) void gated_act_vec_kernel(const TS* __restrict__ gu, TO* __restrict__ out, int n_splits, size_t split_stride,
+                                                            int inter, uint32_t wgs_per_row, int group, int act, int round_sum, float p0,
+                                                            float p1) {
+  const uint32_t n = blockIdx.x / wgs_per_row, first = 1024 * (blockIdx.x % wgs_per_row);
+  const uint32_t j = min(first + 4 * threadIdx.x, static_cast<uint32_t>(inter) - 4);
+  const uint32_t gate = static_cast<uint32_t>(gate_col(j, inter, group));  // four columns of one group (group % 4 == 0)
+  const uint32_t at[2] = {gate, gate + static_cast<uint32_t>(up_offset(inter, group))};
+  float4 v[2];
+  sum_slices<2, TS>(gu + static_cast<size_t>(n) * 2 * inter, at, n_splits, split_stride, v);
   float4 y;
-  y.x = gated_pair(as_output(g.x, round_sum), as_output(u.x, round_sum), act, p0, p1);
-  y.y = gated_pair(as_output(g.y, round_sum), as_output(u.y, round_sum), act, p0, p1);
-  y.z = gated_pair(as_output(g.z, round_sum), as_output(u.z, round_sum), act, p0, p1);
-  y.w = gated_pair(as_output(g.w, round_sum), as_output(u.w, round_sum), act, p0, p1);
-  put_four<TO>(out + n * inter + j, y);
+  y.x = gated_pair(as_output(v[0].x, round_sum), as_output(v[1].x, round_sum), act, p0, p1);
+  y.y = gated_pair(as_output(v[0].y, round_sum), as_output(v[1].y, round_sum), act, p0, p1);
+  y.z = gated_pair(as_output(v[0].z, round_sum), as_output(v[1].z, round_sum), act, p0, p1);
+  y.w = gated_pair(as_output(v[0].w, round_sum), as_output(v[1].w, round_sum), act, p0, p1);
+  if (first + 4 * threadIdx.x < inter) put_four<TO>(out + static_cast<size_t>(n) * inter + j, y);
 }
 
 // bfloat16 in and out, one slice, eight outputs per thread with 16-byte accesses (in the
@@ -759,10 +746,10 @@ static int launch_gated_act(const void* gu, int n_splits, int round_sum, void* o
     gated_act_bf16x8_kernel<<<static_cast<unsigned>((total_vec + 255) / 256), 256, 0, stream>>>(
         static_cast<const bf16_t*>(gu), static_cast<bf16_t*>(out), inter, total_vec, act, group, p0, p1);
   } else if (aligned) {
-    const size_t total_vec = static_cast<size_t>(n_rows) * (inter / 4);
-    YK_REQUIRE((total_vec + 255) / 256 < (1ull << 31), "gated_act: too large for one launch");
-    gated_act_vec_kernel<TS, TO><<<static_cast<unsigned>((total_vec + 255) / 256), 256, 0, stream>>>(
-        static_cast<const TS*>(gu), n_splits, stride, round_sum, static_cast<TO*>(out), inter, total_vec, act, group, p0, p1);
+    const size_t wgs = (inter / 4 + 255) / 256;
+    YK_REQUIRE(n_rows * wgs < (1ull << 31), "gated_act: too large for one launch");
+    gated_act_vec_kernel<TS, TO><<<static_cast<unsigned>(n_rows * wgs), 256, 0, stream>>>(
+        static_cast<const TS*>(gu), static_cast<TO*>(out), n_splits, stride, inter, static_cast<uint32_t>(wgs), group, act, round_sum, p0, p1);
   } else {
     const size_t total = static_cast<size_t>(n_rows) * inter;
     const int grid = static_cast<int>(std::min<size_t>((total + 255) / 256, 65535));

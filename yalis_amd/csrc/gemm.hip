@@ -621,6 +621,17 @@ __global__ void reduce_splits_kernel(const float* __restrict__ part, TO* __restr
   }
 }
 
+// the same, four columns a thread with its slices asked for at once (N and ldy multiples of 4, y aligned)
+template <typename TO>
+__global__ __launch_bounds__(256) void reduce_splits_vec_kernel(const float* __restrict__ part, TO* __restrict__ y, uint32_t pieces, uint32_t per_row,
+                                                                int ldy, int splits) {
+  const uint32_t first = blockIdx.x * 256, i = min(first + threadIdx.x, pieces - 1);
+  const uint32_t at[1] = {4 * (i - first)};
+  float4 v[1];
+  sum_slices<1, float>(part + 4 * static_cast<size_t>(first), at, splits, 4 * static_cast<size_t>(pieces), v);
+  if (first + threadIdx.x < pieces) put_four<TO>(y + static_cast<size_t>(i / per_row) * ldy + 4 * (i % per_row), v[0]);
+}
+
 static int skinny_mt(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
 
 // How the skinny kernel cuts the work for these sizes: waves per workgroup (each wave owns
@@ -824,6 +835,15 @@ static int skinny_product(const bf16_t* xp, const AttnSplits* from_splits, const
   if (keep_splits) return splits;
   const size_t total = static_cast<size_t>(M) * N;
   const int rb = 256;
+  // (16 rows of 3,072 in eight slices, with their product of K 8,192: 15.1 us by elements, 13.6 by pieces of four)
+  if (N % 4 == 0 && ldy % 4 == 0 && total / 4 < (1ull << 31) && reinterpret_cast<uintptr_t>(y) % 16 == 0 && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
+    const uint32_t pieces = static_cast<uint32_t>(total / 4), wgs = (pieces + 255) / 256;
+    if (y_dtype == YK_F32)
+      reduce_splits_vec_kernel<float><<<wgs, rb, 0, stream>>>(workspace, static_cast<float*>(y), pieces, N / 4, ldy, splits);
+    else
+      reduce_splits_vec_kernel<bf16_t><<<wgs, rb, 0, stream>>>(workspace, static_cast<bf16_t*>(y), pieces, N / 4, ldy, splits);
+    return yk_check_launch("reduce_splits");
+  }
   const int rg = static_cast<int>(std::min<size_t>((total + rb - 1) / rb, 65535));
   if (y_dtype == YK_F32)
     reduce_splits_kernel<float><<<rg, rb, 0, stream>>>(workspace, static_cast<float*>(y), M, N, ldy, splits);

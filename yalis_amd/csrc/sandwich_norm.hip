@@ -86,50 +86,26 @@ __global__ __launch_bounds__(256) void sandwich_norm_kernel(
   }
 }
 
-// The same for rows of up to 4,096 elements in 16-byte pieces, a thread holding P of them in
-// registers: everything a thread reads (the branch's slices, the residual, both norms' weights and
-// biases) is asked for before the first reduction, one round trip to memory instead of six.
-template <typename T>
-__device__ __forceinline__ float4 sn_load4(const T* p);
-template <>
-__device__ __forceinline__ float4 sn_load4<float>(const float* p) {
-  return *reinterpret_cast<const float4*>(p);
-}
-template <>
-__device__ __forceinline__ float4 sn_load4<bf16_t>(const bf16_t* p) {
-  const uint2 w = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
-                     __uint_as_float(w.y & 0xffff0000u));
-}
-template <typename T>
-__device__ __forceinline__ void sn_store4(T* p, float4 v);
-template <>
-__device__ __forceinline__ void sn_store4<float>(float* p, float4 v) {
-  *reinterpret_cast<float4*>(p) = v;
-}
-template <>
-__device__ __forceinline__ void sn_store4<bf16_t>(bf16_t* p, float4 v) {
-  *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
-}
-
+// The same for rows of up to 4,096 elements in pieces of four, a thread holding P of them in registers: everything a thread reads (the
+// branch's slices, the residual, both norms' weights and biases) is asked for before any of it is used, and every reduction has a scratch
+// of its own and one barrier.  Behind copies of 16 MB and of its input, eight rows of 4,096 as eight slices / in bfloat16, a centred
+// norm after and a plain one before, us: with loads that waited one for another 5.5 / 4.7, now 5.0 / 4.1.
 template <int P>
-__device__ __forceinline__ NormStats piece_stats(const float4* v, const bool* has, int width, int center, float eps, float* scratch) {
+__device__ __forceinline__ NormStats piece_stats(const float4* v, const bool* in, int width, bool center, float eps, float (*scratch)[16], int waves) {
   float mean = 0.f;
   if (center) {
     float s = 0.f;
 #pragma unroll
-    for (int k = 0; k < P; ++k)
-      if (has[k]) s += (v[k].x + v[k].y) + (v[k].z + v[k].w);
-    mean = block_sum(s, scratch) / static_cast<float>(width);
+    for (int k = 0; k < P; ++k) s += in[k] ? (v[k].x + v[k].y) + (v[k].z + v[k].w) : 0.f;
+    mean = block_sum_first(s, scratch[0], waves) / static_cast<float>(width);
   }
   float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < P; ++k)
-    if (has[k]) {
-      const float a = v[k].x - mean, b = v[k].y - mean, c = v[k].z - mean, d = v[k].w - mean;
-      ss = fmaf(a, a, fmaf(b, b, fmaf(c, c, fmaf(d, d, ss))));
-    }
-  return {mean, 1.f / sqrtf(block_sum(ss, scratch) / static_cast<float>(width) + eps)};
+  for (int k = 0; k < P; ++k) {
+    const float a = v[k].x - mean, b = v[k].y - mean, c = v[k].z - mean, d = v[k].w - mean;
+    ss = in[k] ? fmaf(a, a, fmaf(b, b, fmaf(c, c, fmaf(d, d, ss)))) : ss;
+  }
+  return {mean, 1.f / sqrtf(block_sum_first(ss, scratch[1], waves) / static_cast<float>(width) + eps)};
 }
 
 __device__ __forceinline__ float4 piece_norm(float4 v, NormStats st, float4 w, float4 b) {
@@ -137,73 +113,89 @@ __device__ __forceinline__ float4 piece_norm(float4 v, NormStats st, float4 w, f
                      fmaf((v.z - st.mean) * st.inv, w.z, b.z), fmaf((v.w - st.mean) * st.inv, w.w, b.w));
 }
 
+// `how`: bits 0-15 slices; 19-23 waves; and these
+constexpr uint32_t SN_ROUND = 1u << 16, SN_CENTER_A = 1u << 17, SN_CENTER_B = 1u << 18, SN_ROWS = 1u << 24, SN_BIAS_A = 1u << 25,
+                   SN_BIAS_B = 1u << 26;
 template <typename TS, typename TW, typename TO, int P>
-__global__ __launch_bounds__(1024) void sandwich_norm_vec_kernel(
-    float* __restrict__ residual, const TS* __restrict__ src, int n_splits, size_t split_stride, int round_sum,
-    const TW* __restrict__ wa, const TW* __restrict__ ba, float eps_a, int center_a, int has_post, float scale,
-    const TW* __restrict__ wb, const TW* __restrict__ bb, float eps_b, int center_b, int has_pre,
-    const int32_t* __restrict__ rows, TO* __restrict__ out, int width) {
-  __shared__ float scratch[17];
+__global__ __launch_bounds__(1024) void sandwich_norm_vec_kernel(float* __restrict__ residual, const TS* __restrict__ src,
+                                                                 const TW* __restrict__ wa, const TW* __restrict__ wb,
+                                                                 TO* __restrict__ out, int width, uint32_t how, uint32_t split_stride,
+                                                                 float scale, const TW* __restrict__ ba, const TW* __restrict__ bb,
+                                                                 const int32_t* __restrict__ rows, float eps_a, float eps_b) {
+  constexpr int SL = sizeof(TS) == 2 ? 1 : P == 1 ? 8 : 4;  // slices asked for at once
+  __shared__ float scratch[4][16];
+  const int n_splits = how & 0xffffu, waves = (how >> 19) & 31, round_sum = (how & SN_ROUND) != 0;
   const size_t n = blockIdx.x;
-  const size_t r = rows != nullptr ? static_cast<size_t>(rows[n]) : n;
+  size_t r = n;
+  if (how & SN_ROWS) r = rows[n];
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  float4 br[P], rs[P], fwa[P], fba[P], fwb[P], fbb[P];
-  bool has[P];
+  float4 br[P], rs[P];
+  typename Four<TW>::raw wra[P], bra[P], wrb[P], brb[P];
+  typename Four<TS>::raw d[SL][P];
+  uint32_t at[P];
+  bool in[P];
 #pragma unroll
   for (int k = 0; k < P; ++k) {
-    const int c = 4 * (threadIdx.x + blockDim.x * k);
-    has[k] = c < width;
-    br[k] = rs[k] = fba[k] = fbb[k] = zero;
-    fwa[k] = fwb[k] = zero;
-    if (!has[k]) continue;
-    if (src != nullptr) {
-      for (int s0 = 0; s0 < n_splits; s0 += 8) {
-        float4 t[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (s0 + j < n_splits) t[j] = sn_load4<TS>(src + (s0 + j) * split_stride + r * width + c);
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (s0 + j < n_splits) {
-            br[k].x += t[j].x; br[k].y += t[j].y; br[k].z += t[j].z; br[k].w += t[j].w;
-          }
-      }
-      br[k] = make_float4(as_output(br[k].x, round_sum), as_output(br[k].y, round_sum), as_output(br[k].z, round_sum),
-                          as_output(br[k].w, round_sum));
-    }
-    if (residual != nullptr) rs[k] = *reinterpret_cast<const float4*>(residual + r * width + c);
-    if (has_post) {
-      fwa[k] = sn_load4<TW>(wa + c);
-      if (ba != nullptr) fba[k] = sn_load4<TW>(ba + c);
-    }
-    if (has_pre) {
-      fwb[k] = sn_load4<TW>(wb + c);
-      if (bb != nullptr) fbb[k] = sn_load4<TW>(bb + c);
-    }
+    const int c = 4 * (static_cast<int>(threadIdx.x) + 64 * waves * k);
+    in[k] = c < width;
+    at[k] = min(c, width - 4);
+    rs[k] = br[k] = zero;
+    wra[k] = bra[k] = wrb[k] = brb[k] = Four<TW>::all(0.f);
   }
-  if (src != nullptr && has_post) {
-    const NormStats st = piece_stats<P>(br, has, width, center_a, eps_a, scratch);
-#pragma unroll
-    for (int k = 0; k < P; ++k) br[k] = piece_norm(br[k], st, fwa[k], fba[k]);
-  }
+  const TS* p = src + r * width;
+  if (src != nullptr) ask_slices<SL, P, TS>(p, at, n_splits, split_stride, d);
   if (residual != nullptr) {
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
-      if (src != nullptr) {
+    for (int k = 0; k < P; ++k) rs[k] = four_at<float>(residual + r * width + at[k]);
+  }
+  if (wa != nullptr) {
+#pragma unroll
+    for (int k = 0; k < P; ++k) wra[k] = Four<TW>::at(wa + at[k]);
+  }
+  if (wb != nullptr) {
+#pragma unroll
+    for (int k = 0; k < P; ++k) wrb[k] = Four<TW>::at(wb + at[k]);
+  }
+  arguments_now(ba, bb);
+  if (how & SN_BIAS_A) {
+#pragma unroll
+    for (int k = 0; k < P; ++k) bra[k] = Four<TW>::at(ba + at[k]);
+  }
+  if (how & SN_BIAS_B) {
+#pragma unroll
+    for (int k = 0; k < P; ++k) brb[k] = Four<TW>::at(bb + at[k]);
+  }
+  if (src != nullptr) {
+    join_slices<SL, P, TS>(d, n_splits, br);
+    join_rest<SL, P, TS>(p, at, n_splits, split_stride, br);
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+      br[k] = make_float4(as_output(br[k].x, round_sum), as_output(br[k].y, round_sum), as_output(br[k].z, round_sum),
+                          as_output(br[k].w, round_sum));
+    if (wa != nullptr) {
+      const NormStats st = piece_stats<P>(br, in, width, how & SN_CENTER_A, eps_a, scratch, waves);
+#pragma unroll
+      for (int k = 0; k < P; ++k) br[k] = piece_norm(br[k], st, Four<TW>::wide(wra[k]), Four<TW>::wide(bra[k]));
+    }
+  }
+  if (residual != nullptr) {
+    if (src != nullptr) {
+#pragma unroll
+      for (int k = 0; k < P; ++k) {
         rs[k] = make_float4(fmaf(scale, br[k].x, rs[k].x), fmaf(scale, br[k].y, rs[k].y), fmaf(scale, br[k].z, rs[k].z),
                             fmaf(scale, br[k].w, rs[k].w));
-        if (rows == nullptr && has[k]) *reinterpret_cast<float4*>(residual + r * width + 4 * (threadIdx.x + blockDim.x * k)) = rs[k];
+        if (!(how & SN_ROWS) && in[k]) put_four<float>(residual + r * width + at[k], rs[k]);
       }
     }
   } else {
 #pragma unroll
     for (int k = 0; k < P; ++k) rs[k] = br[k];
   }
-  if (!has_pre) return;
-  const NormStats st = piece_stats<P>(rs, has, width, center_b, eps_b, scratch);
+  if (wb == nullptr) return;
+  const NormStats st = piece_stats<P>(rs, in, width, how & SN_CENTER_B, eps_b, scratch + 2, waves);
 #pragma unroll
   for (int k = 0; k < P; ++k)
-    if (has[k]) sn_store4<TO>(out + n * width + 4 * (threadIdx.x + blockDim.x * k), piece_norm(rs[k], st, fwb[k], fbb[k]));
+    if (in[k]) put_four<TO>(out + n * width + at[k], piece_norm(rs[k], st, Four<TW>::wide(wrb[k]), Four<TW>::wide(brb[k])));
 }
 
 // src_rows: rows of residual and of every slice of src (the stride between slices); n_rows: rows of out.
@@ -222,16 +214,18 @@ extern "C" int yk_sandwich_norm(float* residual, const void* src, int src_dtype,
   const size_t lds = (static_cast<size_t>(width) + 17) * sizeof(float);
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool vec = width % 4 == 0 && width <= 4096 && al(residual) && al(src) && al(wa) && al(ba) && al(wb) &&
-                   al(bb) && al(out);
+                   al(bb) && al(out) && n_splits < 1 << 16 && stride < size_t{1} << 32;
   // a piece a thread for few rows, two where rows fill the chip: eight rows of 4,096 11.1 -> 6.2 us, 2,048 rows of 2,048 24 -> 15 us
   // against 256 threads with up to four pieces each (whose slices were then added one round trip after the other)
   const int pieces = n_rows >= 1024 ? 2 : 1;
   const int threads = (width / 4 + 64 * pieces - 1) / (64 * pieces) * 64;
+  const uint32_t how = static_cast<uint32_t>(n_splits & 0xffff) | (round_sum ? SN_ROUND : 0u) | (center_a ? SN_CENTER_A : 0u) |
+                       (center_b ? SN_CENTER_B : 0u) | static_cast<uint32_t>(threads / 64) << 19 | (rows ? SN_ROWS : 0u) |
+                       (wa && ba ? SN_BIAS_A : 0u) | (wb && bb ? SN_BIAS_B : 0u);
 #define YK_VEC(TS, TW, TO, P)                                                                                     \
   sandwich_norm_vec_kernel<TS, TW, TO, P><<<n_rows, threads, 0, stream>>>(                                        \
-      residual, static_cast<const TS*>(src), n_splits, stride, round_sum, static_cast<const TW*>(wa),             \
-      static_cast<const TW*>(ba), eps_a, center_a, wa != nullptr, scale, static_cast<const TW*>(wb),              \
-      static_cast<const TW*>(bb), eps_b, center_b, wb != nullptr, rows, static_cast<TO*>(out), width)
+      residual, static_cast<const TS*>(src), static_cast<const TW*>(wa), static_cast<const TW*>(wb), static_cast<TO*>(out), width, how, \
+      static_cast<uint32_t>(stride), scale, static_cast<const TW*>(ba), static_cast<const TW*>(bb), rows, eps_a, eps_b)
 #define YK_CASE(SD, TS, WD, TW, OD, TO)                                                                           \
   if ((src == nullptr || src_dtype == SD) && w_dtype == WD && (out == nullptr || out_dtype == OD)) {              \
     if (vec && pieces == 1) YK_VEC(TS, TW, TO, 1);                                                                \
@@ -275,24 +269,17 @@ __global__ void activation_kernel(const TS* __restrict__ src, int n_splits, size
   }
 }
 
-// The same, four elements at a time and eight slices asked for at once (2,048 rows of 8,192: 39 -> 18 us).
+// The same, four elements a thread and all its slices (up to 16) asked for at once (2,048 rows of 8,192: 39 -> 18 us).
 template <typename TS, typename TO>
 __global__ __launch_bounds__(256) void activation_vec_kernel(const TS* __restrict__ src, int n_splits, size_t split_stride, int round_sum, int kind,
                                                              TO* __restrict__ out, size_t pieces) {
-  for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < pieces; i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    float4 v = sn_load4<TS>(src + 4 * i);
-    for (int s0 = 1; s0 < n_splits; s0 += 8) {
-      float4 t[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (s0 + j < n_splits) t[j] = sn_load4<TS>(src + (s0 + j) * split_stride + 4 * i);
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (s0 + j < n_splits) v.x += t[j].x, v.y += t[j].y, v.z += t[j].z, v.w += t[j].w;
-    }
-    sn_store4<TO>(out + 4 * i, make_float4(act_plain(as_output(v.x, round_sum), kind), act_plain(as_output(v.y, round_sum), kind),
-                                           act_plain(as_output(v.z, round_sum), kind), act_plain(as_output(v.w, round_sum), kind)));
-  }
+  const size_t first = blockIdx.x * static_cast<size_t>(256);
+  const uint32_t at[1] = {4 * static_cast<uint32_t>(min(static_cast<size_t>(threadIdx.x), pieces - 1 - first))};
+  float4 v[1];
+  sum_slices<1, TS>(src + 4 * first, at, n_splits, split_stride, v);
+  if (first + threadIdx.x < pieces)
+    put_four<TO>(out + 4 * first + at[0], make_float4(act_plain(as_output(v[0].x, round_sum), kind), act_plain(as_output(v[0].y, round_sum), kind),
+                                                      act_plain(as_output(v[0].z, round_sum), kind), act_plain(as_output(v[0].w, round_sum), kind)));
 }
 
 extern "C" int yk_activation(const void* src, int src_dtype, int n_splits, int round_sum, int kind, void* out, int out_dtype,
