@@ -133,3 +133,52 @@ def test_any_number_of_slices(consumer, dtype, n, width):
         got = call(o, res, SplitSum(t, dtype), w, rows)
         want = call(o, res2, whole, w, rows)
         assert same(got, want) and same(res, res2), slices
+
+
+@pytest.mark.parametrize("h,g,d", [(8, 2, 128), (12, 4, 64), (20, 4, 64), (36, 2, 128)])  # 4, 3, 5 and 18 heads that share keys
+@pytest.mark.parametrize("page", [48, 64, 192])
+def test_decode_attention_with_slices_and_splits(h, g, d, page):
+    """Single tokens behind contexts at the edges of half blocks, blocks and pages (sizes that are no powers of two among them), the slots
+    behind them NaN: any number of slices of the projection gives the bits of its sum, and any number of splits, up to more
+    than are merged at once, agrees with the plain reference within bfloat16's rounding of probabilities and values (2e-2, 2^-6 as elsewhere)."""
+    import math
+    import types
+
+    o, gen = ops(), torch.Generator().manual_seed(page + h)
+    cached = [0, 31, 32, 47, 48, 63, 64, 95, 96, 191, 192, 1000]
+    n, width = len(cached), -(-1001 // page)
+    pages = n * width
+    kc, vc = torch.full((pages, g, page, d), float("nan")), torch.full((pages, g, d, page), float("nan"))
+    table = torch.randperm(pages, generator=gen).int().view(n, width)
+    for r, c in enumerate(cached):
+        for p in range(c):
+            kc[table[r, p // page], :, p % page] = torch.randn(g, d, generator=gen)
+            vc[table[r, p // page], :, :, p % page] = torch.randn(g, d, generator=gen)
+    kc, vc = kc.bfloat16(), vc.bfloat16()
+    tiles = torch.tensor([[r, r, 1, c] for r, c in enumerate(cached)], dtype=torch.int32)
+    arrays = {"block_table_g0": table, "positions": torch.tensor(cached, dtype=torch.int32), "token_seq": torch.arange(n, dtype=torch.int32)}
+    ctx = types.SimpleNamespace(arrays={k: v.cuda() for k, v in arrays.items()}, max_ctx=1001, max_qlen=1)
+    angle = torch.rand(1001, d // 2, generator=gen) * 6
+    cos, sin = angle.cos(), angle.sin()
+    from test_kernels_gpu import device_cache
+    from yalis_amd.ops.hip import RopeInLaunch
+
+    rope = RopeInLaunch(cos.cuda(), sin.cuda(), d, False, True)
+    slots = torch.tensor([int(table[r, c // page]) * page + c % page for r, c in enumerate(cached)], dtype=torch.int32)
+    for slices in (1, 2, 4, 7, 8, 9, 17):
+        parts = torch.randn(slices, n, (h + 2 * g) * d, generator=gen) / math.sqrt(slices)
+        rows = in_order(parts, torch.bfloat16)
+        want = None
+        for splits in (1, 2, 3, 7, 8, 9, 12):
+            results = []
+            for given in (SplitSum(parts.cuda(), torch.bfloat16), rows.bfloat16().cuda()):
+                kd, vd = device_cache(o, kc.clone(), vc.clone())
+                results.append(o.attention(given, h, g, d, kd, vd, page, d ** -0.5, 0, ctx, 0, tiles.cuda(), rope=rope, plan=(4, splits)).float())
+            assert torch.equal(*results), (slices, splits)
+            if want is None:
+                q, kr, vr = rows.clone(), kc.float(), vc.float()
+                R.rope_append(q, h, g, d, arrays["positions"], cos, sin, d, False, kr, vr, slots, page)
+                want = R.attention(q[:, : h * d].bfloat16().float(), h, g, d, kr.bfloat16().float(), vr.bfloat16().float(), page, d ** -0.5, 0,
+                                   types.SimpleNamespace(arrays=arrays), 0, None)
+            err = (results[0].cpu() - want).abs()
+            assert bool((err <= 2e-2 + 2 ** -6 * want.abs()).all()), (slices, splits, err.max().item())

@@ -522,8 +522,8 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // the keys of the next are in flight while the block's scores are worked on.
 //
 // A workgroup has W waves that share the columns and divide the workgroup's key blocks
-// among themselves; at the end waves 1.. hand their running maximum, sum and output to
-// wave 0 through LDS (every lane to the same lane), and wave 0 merges and stores.  Across
+// among themselves; at the end every wave leaves its running maximum, sum and output in LDS
+// and merges (every lane from the same lane) and stores a part of the head.  Across
 // workgroups (blockIdx.z) the keys are split further when the launch needs more waves;
 // those partial results go through the workspace to the combine kernel.
 //
@@ -538,7 +538,8 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // (bfloat16, or the unreduced float32 K slices of the product): every workgroup sums the
 // slices of its heads, rotates them by the token's angle and parks them in LDS in bfloat16,
 // with the arithmetic and roundings of rope_append_kernel, so the bits are those of the
-// two-kernel path.  The token's own key and value are not in the pages yet: the one workgroup
+// two-kernel path (a thread takes two neighbouring pairs where whole heads turn in pairs (i, i + D/2), else
+// pair by pair).  The token's own key and value are not in the pages yet: the one workgroup
 // (per kv head and split) whose share of the keys holds the token's position makes them too,
 // puts them into its operand registers in place of what the pages gave, and (chunk 0 only)
 // stores them in the pages for later steps.  Nobody reads that slot of the pages as a number
@@ -554,6 +555,7 @@ struct RopeSrc {
   const float* sin_t;
   int rotary_dim, interleaved, max_positions;
   int append;           // 1: src holds the token's key and value heads too; they go to the pages
+  int by_fours;         // 1: whole heads turn in pairs (i, i + D/2), and rows, tables and strides allow loads of two elements
 };
 
 // Up to eight slices of one element, all asked for before any is used (a slice index beyond
@@ -584,12 +586,69 @@ __device__ __forceinline__ float rope_src_add8(float acc, const float (&d)[8], i
   return acc;
 }
 
+// Two neighbouring elements of the row at `src` (the same in every lane), `at` elements from its start: up to eight slices asked for, in
+// groups as ask_slices does it, and added in their order.
+template <int SRC, int FROM = 0, int TO = 1>
+__device__ __forceinline__ void rope_ask2(const void* src, uint32_t at, int left, size_t split_stride, float2 (&d)[8]) {
+  if constexpr (SRC == 1) {
+    d[0].x = __uint_as_float(*reinterpret_cast<const uint32_t*>(static_cast<const bf16_t*>(src) + at));  // (as it lies; rope_join2 widens)
+  } else {
+    const float* p = static_cast<const float*>(src);
+#pragma unroll
+    for (int j = FROM; j < TO; ++j) {
+      d[j] = *reinterpret_cast<const float2*>(p + at);
+      p += j + 1 < left ? split_stride : 0;
+    }
+    if constexpr (TO < 8) {
+      if (left > TO) rope_ask2<SRC, TO, 2 * TO>(p, at, left, split_stride, d);
+    }
+  }
+}
+template <int SRC, int FROM = 0, int TO = 1>
+__device__ __forceinline__ void rope_join2(const float2 (&d)[8], int left, float2& s) {
+  if constexpr (SRC == 1) {
+    s.x = __uint_as_float(__float_as_uint(d[0].x) << 16);
+    s.y = __uint_as_float(__float_as_uint(d[0].x) & 0xffff0000u);
+  } else {
+#pragma unroll
+    for (int j = FROM; j < TO; ++j) {
+      const uint32_t keep = __builtin_amdgcn_readfirstlane((j - left) >> 31);
+      s.x += __uint_as_float(__float_as_uint(d[j].x) & keep);
+      s.y += __uint_as_float(__float_as_uint(d[j].y) & keep);
+    }
+    if constexpr (TO < 8) {
+      if (left > TO) rope_join2<SRC, TO, 2 * TO>(d, left, s);
+    }
+  }
+}
+
+// A short launch is bound by its waves' longest chain: launch, tile, page, keys (three trips to memory), then a block's products, softmax and
+// merge, at five to eight cycles an instruction.  So: nothing divides, the rows to rotate are on their way before the keys are asked for and are
+// rotated while these come, no load hangs on a condition (the compiler, which cannot count loads that may not have been made, waited for the
+// keys before it rotated), masks are limits a half block and words a lane, and all waves merge.  Behind copies of 16 MB and of the rows, us, before / now:
+// one request of 48 keys, 32 heads of 64 6.7 / 4.4, of 1,000 keys (with its merge) 9.8 / 7.5; eight of 1,040 keys, 32 heads of 128, eight slices 15.7 /
+// 14.9 (34 MB of keys and values: 5.7 at 6 TB/s); four of 700 keys, 16 heads of 128, squashed scores 16.6 / 9.1; 64 of 200 keys 19.3 / 17.1.
+// What the host works out once a launch, so that no wave divides: one wave issues an instruction about every five cycles (eight where
+// it hangs on the one before), and a short launch lasts as long as its waves' longest chain of them.
+struct AttnShape {
+  int heads_per_kv, hpt, chunks;
+  uint32_t hpt_inverse;     // ceil(256 / hpt): (r * hpt_inverse) >> 8 = r / hpt for r < 16
+  uint32_t splits_inverse;  // inverse_of(n_splits), for n_splits > 1
+  uint32_t page_inverse;    // inverse_of(page_size)
+};
+// x / n for x from 0 and n from 2 up: by ceil(2^32 / n) the quotient is less than x / 2^32 too large before it is cut, so at most one
+static uint32_t inverse_of(int n) { return static_cast<uint32_t>(((1ull << 32) + n - 1) / n); }
+__device__ __forceinline__ int divide_by(int x, int n, uint32_t inverse) {
+  const uint32_t q = __umulhi(static_cast<uint32_t>(x), inverse);
+  return static_cast<int>(q - (q * static_cast<uint32_t>(n) > static_cast<uint32_t>(x) ? 1u : 0u));
+}
+
 template <int D, int W, bool TILED, int SRC, bool EXT = false>
 __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
-    const bf16_t* __restrict__ q, int q_stride, bf16_t* __restrict__ out,
+    const int32_t* __restrict__ tiles, const int32_t* __restrict__ block_table,
     const bf16_t* k_cache, const bf16_t* v_cache,  // (written too, with ROPE: the token's own slot)
-    const int32_t* __restrict__ tiles, const int32_t* __restrict__ block_table, int table_width,
-    int page_size, int n_heads, int n_kv, int hpt, int chunks, float scale_log2, int window,
+    const bf16_t* __restrict__ q, bf16_t* __restrict__ out, int table_width, int page_size, int q_stride,
+    int n_heads, int n_kv, AttnShape shape, float scale_log2, int window,
     int n_splits, float* __restrict__ ws_o, float* __restrict__ ws_ml, RopeSrc rs, int keep_first_arg = 0,
     float cap_over_scale = 0.f, float scale_over_cap_2log2e = 0.f, const float* __restrict__ dist_bias = nullptr,
     int bias_rows = 0, float inv_scale = 0.f, const float* __restrict__ sink = nullptr, int chunked_arg = 0, MapArgs maps = MapArgs{}) {
@@ -603,11 +662,15 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
   const int t = blockIdx.x;
   const int seq = tiles[4 * t], tok0 = tiles[4 * t + 1], pos0 = tiles[4 * t + 3];
   const int ntok = ROPE ? 1 : tiles[4 * t + 2];
-  const int g = blockIdx.y / chunks, chunk = blockIdx.y % chunks;
-  const int qpk = n_heads / n_kv;
+  // the arguments that do not come with the launch are asked for with the tile's row, not each where it is first used
+  asm volatile("" ::"s"(n_heads), "s"(n_kv), "s"(shape.heads_per_kv), "s"(shape.hpt), "s"(shape.chunks), "s"(shape.splits_inverse),
+               "s"(shape.page_inverse), "s"(scale_log2), "s"(window), "s"(n_splits), "s"(ws_o), "s"(ws_ml));
+  const int hpt = shape.hpt, qpk = shape.heads_per_kv;
+  int g = blockIdx.y, chunk = 0;
+  if (shape.chunks > 1) g = blockIdx.y / shape.chunks, chunk = blockIdx.y % shape.chunks;
   const int h_base = g * qpk + chunk * hpt;
   const int heads_here = min(hpt, qpk - chunk * hpt);
-  const int tt = r / hpt, hh = r % hpt;
+  const int tt = ROPE ? 0 : (r * shape.hpt_inverse) >> 8, hh = r - tt * hpt;
   const bool col_ok = tt < ntok && hh < heads_here;
   const int pos_c = pos0 + tt;
   const int lo_c = first_visible(pos_c, window, chunked);
@@ -618,13 +681,13 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
   const int n_first = EXT ? ext_first_blocks(keep_first, window, lo) : 0;
 #define ATT_BLK(VB) (EXT ? ext_block((VB), win_lo, n_first) : (VB))
   const int kb_lo = win_lo - n_first, kb_hi = (hi + 63) / 64;
-  const int per_split = (kb_hi - kb_lo + n_splits - 1) / n_splits;
+  const int share = kb_hi - kb_lo + n_splits - 1;
+  const int per_split = n_splits == 1 ? share : divide_by(share, n_splits, shape.splits_inverse);
   const int wg_lo = kb_lo + blockIdx.z * per_split;
   const int wg_hi = min(kb_hi, wg_lo + per_split);
   // the waves divide the workgroup's keys in halves of a block (32 keys: one group of the two
   // score products), so that the longest share is at most half a block above the mean; a half
-  // beyond the last key is nobody's.  A half that is not the wave's own is not loaded: its keys
-  // and values stand as zeros in the products and its scores are masked.
+  // beyond the last key is nobody's.  A half that is not the wave's own has its scores masked and its values zeroed.
   const int h_lo = wg_lo * 2, h_hi = min(wg_hi * 2, (hi + 31) / 32);
   const int per_wave = (max(0, h_hi - h_lo) + W - 1) / W;
   const int my_hlo = h_lo + wave * per_wave;
@@ -632,8 +695,13 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
   const int my_lo = my_hlo / 2;
   const int my_hi = my_hlo < my_hhi ? (my_hhi + 1) / 2 : my_lo;
   auto mine = [&](int kb, int u) { return 2 * kb + u >= my_hlo && 2 * kb + u < my_hhi; };
+  // the half that is read in its place, so that no load hangs on a condition: its own, or else the other one again
+  auto half_of = [&](int kb, int u) { return mine(kb, u) ? u : 1 - u; };
   const int32_t* bt = block_table + static_cast<size_t>(seq) * table_width;
-  const int last_page_col = min(table_width - 1, (hi - 1) / page_size);
+  // a key's page in the table, and its place there
+  auto page_col = [&](int key) { return divide_by(key, page_size, shape.page_inverse); };
+  auto key_in_page = [&](int key) { return key - page_col(key) * page_size; };
+  const int last_page_col = min(table_width - 1, page_col(hi - 1));
 
   const u32x4_t zero4 = {0u, 0u, 0u, 0u};
   float m = -INFINITY, l = 0.f;
@@ -644,7 +712,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
   // the key this lane's score rows stand for, relative to the block: [group][product]
   const int krow = 8 * (r / 4) + r % 4;
   // a page that exists for any key: keys beyond the request read the last allocated page
-  auto page_of = [&](int key) { return max(0, bt[min(key / page_size, last_page_col)]); };
+  auto page_of = [&](int key) { return max(0, bt[min(page_col(key), last_page_col)]); };
 
   AFrag8 kf[2][2][KS];
 #define ATT_LOAD_K(KB) ATT_LOAD_K_AT(KB, page_of(ATT_BLK(KB) * 64))
@@ -654,29 +722,20 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
   if (TILED) {                                                                                     \
     const int key0 = ATT_BLK(KB) * 64;                                                             \
     const bf16_t* kp = k_cache + (static_cast<size_t>(PAGE0) * n_kv + g) * page_size * D +         \
-                       static_cast<size_t>(key0 % page_size) * D + 8 * lane;                       \
+                       static_cast<size_t>(key_in_page(key0)) * D + 8 * lane;                      \
     _Pragma("unroll") for (int u = 0; u < 2; ++u) {                                                \
-      if (mine((KB), u)) {                                                                         \
-        _Pragma("unroll") for (int sb = 0; sb < 2; ++sb)                                           \
-        _Pragma("unroll") for (int ks = 0; ks < KS; ++ks)                                          \
-            kf[u][sb][ks].u = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(kp + ((u * 2 + sb) * KS + ks) * 512)); \
-      } else {                                                                                     \
-        _Pragma("unroll") for (int sb = 0; sb < 2; ++sb)                                           \
-        _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) kf[u][sb][ks].u = zero4;                 \
-      }                                                                                            \
+      const bf16_t* ku = kp + half_of((KB), u) * (2 * KS * 512);                                   \
+      _Pragma("unroll") for (int sb = 0; sb < 2; ++sb)                                             \
+      _Pragma("unroll") for (int ks = 0; ks < KS; ++ks)                                            \
+          kf[u][sb][ks].u = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(ku + (sb * KS + ks) * 512)); \
     }                                                                                              \
   } else {                                                                                         \
     _Pragma("unroll") for (int u = 0; u < 2; ++u) {                                                \
-      if (mine((KB), u)) {                                                                         \
-        _Pragma("unroll") for (int sb = 0; sb < 2; ++sb) {                                         \
-          const int key = ATT_BLK(KB) * 64 + 32 * u + krow + 4 * sb;                              \
-          const bf16_t* kp = k_cache + ((static_cast<size_t>(page_of(key)) * n_kv + g) * page_size + key % page_size) * D + 8 * gq; \
-          _Pragma("unroll") for (int ks = 0; ks < KS; ++ks)                                       \
-              kf[u][sb][ks].u = *reinterpret_cast<const u32x4_t*>(kp + 32 * ks);                  \
-        }                                                                                          \
-      } else {                                                                                     \
-        _Pragma("unroll") for (int sb = 0; sb < 2; ++sb)                                           \
-        _Pragma("unroll") for (int ks = 0; ks < KS; ++ks) kf[u][sb][ks].u = zero4;                 \
+      _Pragma("unroll") for (int sb = 0; sb < 2; ++sb) {                                           \
+        const int key = ATT_BLK(KB) * 64 + 32 * half_of((KB), u) + krow + 4 * sb;                  \
+        const bf16_t* kp = k_cache + ((static_cast<size_t>(page_of(key)) * n_kv + g) * page_size + key_in_page(key)) * D + 8 * gq; \
+        _Pragma("unroll") for (int ks = 0; ks < KS; ++ks)                                          \
+            kf[u][sb][ks].u = *reinterpret_cast<const u32x4_t*>(kp + 32 * ks);                     \
       }                                                                                            \
     }                                                                                              \
   }                                                                                                \
@@ -689,25 +748,18 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
   if (TILED) {                                                                                     \
     const int key0 = ATT_BLK(KB) * 64;                                                             \
     const bf16_t* vp = v_cache + (static_cast<size_t>(PAGE0) * n_kv + g) * D * page_size +         \
-                       static_cast<size_t>(key0 % page_size) * D + 8 * lane;                       \
+                       static_cast<size_t>(key_in_page(key0)) * D + 8 * lane;                      \
     _Pragma("unroll") for (int u = 0; u < 2; ++u) {                                                \
-      if (mine((KB), u)) {                                                                         \
-        _Pragma("unroll") for (int dt = 0; dt < DT; ++dt)                                          \
-            vf[u][dt].u = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(vp + (u * DT + dt) * 512)); \
-      } else {                                                                                     \
-        _Pragma("unroll") for (int dt = 0; dt < DT; ++dt) vf[u][dt].u = zero4;                     \
-      }                                                                                            \
+      const bf16_t* vu = vp + half_of((KB), u) * (DT * 512);                                       \
+      _Pragma("unroll") for (int dt = 0; dt < DT; ++dt)                                            \
+          vf[u][dt].u = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(vu + dt * 512)); \
     }                                                                                              \
   } else {                                                                                         \
     _Pragma("unroll") for (int u = 0; u < 2; ++u) {                                                \
-      if (mine((KB), u)) {                                                                         \
-        const int key = ATT_BLK(KB) * 64 + 32 * u + 8 * gq;                                        \
-        const bf16_t* vp = v_cache + (static_cast<size_t>(page_of(key)) * n_kv + g) * D * page_size + key % page_size; \
-        _Pragma("unroll") for (int dt = 0; dt < DT; ++dt)                                          \
-            vf[u][dt].u = *reinterpret_cast<const u32x4_t*>(vp + static_cast<size_t>(16 * dt + r) * page_size); \
-      } else {                                                                                     \
-        _Pragma("unroll") for (int dt = 0; dt < DT; ++dt) vf[u][dt].u = zero4;                     \
-      }                                                                                            \
+      const int key = ATT_BLK(KB) * 64 + 32 * half_of((KB), u) + 8 * gq;                           \
+      const bf16_t* vp = v_cache + (static_cast<size_t>(page_of(key)) * n_kv + g) * D * page_size + key_in_page(key); \
+      _Pragma("unroll") for (int dt = 0; dt < DT; ++dt)                                            \
+          vf[u][dt].u = *reinterpret_cast<const u32x4_t*>(vp + static_cast<size_t>(16 * dt + r) * page_size); \
     }                                                                                              \
   }                                                                                                \
   }
@@ -747,8 +799,9 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
     const int src_splits = SRC == 2 ? rs.n_splits : 1;
     const size_t src_split_stride = rs.split_stride;
     // the page of the first block is asked for first: the keys' addresses wait for it, and a
-    // wait for an older load leaves the younger ones in flight
-    const int first_page = my_lo < my_hi ? page_of(ATT_BLK(my_lo) * 64) : 0;
+    // wait for an older load leaves the younger ones in flight.  (A wave without keys asks for some block's all the same.)
+    const int first_kb = min(my_lo, kb_hi - 1);
+    const int first_entry = bt[min(page_col(max(0, ATT_BLK(first_kb)) * 64), last_page_col)];
     // one round; LOAD_K: the first block's keys are asked for while the round's rows are on
     // their way (the first round is straight-line code: its loads are all issued before the
     // first of them is waited for; rows of more than eight slices finish in a loop)
@@ -809,18 +862,60 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
           dst[j][ib[j]] = f32_to_bf16(rot[j] ? rot_second(a, b, c[j], sv[j]) : b);
         }
     };
-    round(0, [&]() {
-      if (my_lo < my_hi) {
-        ATT_LOAD_K_AT(my_lo, first_page)
-        ATT_LOAD_V_AT(my_lo, first_page)
-      }
-    });
-    for (int first = 2 * T; first < items; first += 2 * T) round(first, []() {});
+    auto load_first = [&]() {
+      const int first_page = max(0, first_entry);
+      ATT_LOAD_K_AT(first_kb, first_page)
+      ATT_LOAD_V_AT(first_kb, first_page)
+    };
+    if (rs.by_fours) {
+      // whole heads turning in pairs (i, i + D/2): a thread takes elements i, i + 1 and their partners, D / 4 threads a head
+      const int fours = (heads_here + (makes_kv ? 2 : 0)) * (D / 4);
+      const void* from = SRC == 1 ? static_cast<const void*>(static_cast<const bf16_t*>(rs.src) + row) : static_cast<const void*>(static_cast<const float*>(rs.src) + row);
+      auto turn = [&](int first, auto load_k) {
+        const int item = min(first + static_cast<int>(threadIdx.x), fours - 1);
+        const int hq = item / (D / 4), i = 2 * (item % (D / 4));
+        const bool is_k = hq == heads_here, is_v = hq > heads_here;
+        const uint32_t at_a = (is_v ? n_heads + n_kv + g : is_k ? n_heads + g : h_base + hq) * D + i;
+        const float2 c = *reinterpret_cast<const float2*>(cs + i), sv = *reinterpret_cast<const float2*>(sn + i);
+        float2 da[8], db[8], a = make_float2(0.f, 0.f), b = make_float2(0.f, 0.f);
+        rope_ask2<SRC>(from, at_a, src_splits, src_split_stride, da);
+        rope_ask2<SRC>(from, at_a + D / 2, src_splits, src_split_stride, db);
+        load_k();
+        rope_join2<SRC>(da, src_splits, a);
+        rope_join2<SRC>(db, src_splits, b);
+        if constexpr (SRC == 2) {
+          for (int s0 = 8; s0 < src_splits; s0 += 8) {
+            const float* rest = static_cast<const float*>(from) + s0 * src_split_stride;
+            rope_ask2<SRC>(rest, at_a, src_splits - s0, src_split_stride, da);
+            rope_ask2<SRC>(rest, at_a + D / 2, src_splits - s0, src_split_stride, db);
+            rope_join2<SRC>(da, src_splits - s0, a);
+            rope_join2<SRC>(db, src_splits - s0, b);
+          }
+        }
+        a = make_float2(as_output(a.x, rs.round_sum), as_output(a.y, rs.round_sum));
+        b = make_float2(as_output(b.x, rs.round_sum), as_output(b.y, rs.round_sum));
+        uint32_t lo2 = pack_bf16x2(rot_first(a.x, b.x, c.x, sv.x), rot_first(a.y, b.y, c.y, sv.y));
+        uint32_t hi2 = pack_bf16x2(rot_second(a.x, b.x, c.x, sv.x), rot_second(a.y, b.y, c.y, sv.y));
+        lo2 = is_v ? pack_bf16x2(a.x, a.y) : lo2;
+        hi2 = is_v ? pack_bf16x2(b.x, b.y) : hi2;
+        asm volatile("" : "+v"(lo2), "+v"(hi2));  // (made here, their loads before the keys': not moved under the condition below)
+        bf16_t* dst = hq >= heads_here ? kv_s[hq - heads_here] : q_s[hq];
+        if (first + static_cast<int>(threadIdx.x) < fours) {
+          *reinterpret_cast<uint32_t*>(dst + i) = lo2;
+          *reinterpret_cast<uint32_t*>(dst + D / 2 + i) = hi2;
+        }
+      };
+      turn(0, load_first);
+      for (int first = T; first < fours; first += T) turn(first, []() {});
+    } else {
+      round(0, load_first);
+      for (int first = 2 * T; first < items; first += 2 * T) round(first, []() {});
+    }
     __syncthreads();
     if (makes_kv && chunk == 0) {
       // into the pages, for the steps that follow
-      const int slot = pos0 % page_size;
-      const size_t slab = (static_cast<size_t>(max(0, bt[min(pos0 / page_size, table_width - 1)])) * n_kv + g) * page_size * D;
+      const int slot = key_in_page(pos0);
+      const size_t slab = (static_cast<size_t>(max(0, bt[min(page_col(pos0), table_width - 1)])) * n_kv + g) * page_size * D;
       for (int d = threadIdx.x; d < D; d += 64 * W) {
         const_cast<bf16_t*>(k_cache)[slab + cache_k_offset(TILED, page_size, D, slot, d)] = kv_s[0][d];
         const_cast<bf16_t*>(v_cache)[slab + cache_v_offset(TILED, page_size, D, slot, d)] = kv_s[1][d];
@@ -861,6 +956,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
         for (int ks = 0; ks < KS; ++ks)
           s[u][sb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u][sb][ks].v, qf[ks].v, s[u][sb], 0, 0, 0);
       }
+    __builtin_amdgcn_sched_barrier(0);
     if (kb + 1 < my_hi) {
       ATT_LOAD_K(kb + 1)
       ATT_PUT_NEW_K(kb + 1)
@@ -889,13 +985,23 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
           for (int i = 0; i < 4; ++i)
             s[u][sb][i] = fmaf(ext_bias(bcol, pos_c - (akb * 64 + 32 * u + 8 * gq + 4 * sb + i), bias_rows, n_heads), inv_scale, s[u][sb][i]);
     }
+    if (!whole && window == 0) {
+      // no lower bound: the last of the lane's keys in each half that its column sees, -1 for none
+      const int at = akb * 64 + 8 * gq;
+      const int last[2] = {col_ok && mine0 ? pos_c - at : -1, col_ok && mine1 ? pos_c - at - 32 : -1};
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int sb = 0; sb < 2; ++sb)
+        for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (!whole) {
+          for (int i = 0; i < 4; ++i) s[u][sb][i] = 4 * sb + i <= last[u] ? s[u][sb][i] : -INFINITY;
+    } else if (!whole) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
             const int key = akb * 64 + 32 * u + 8 * gq + 4 * sb + i;
             // (a lower bound per key; written as `key >= lo_c || key < keep_first` this kernel let the key
             // just below the window through in one of its four rows, which the test with one towering key shows)
@@ -903,8 +1009,13 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
             const bool ok = col_ok && key <= pos_c && key >= lo_k && (u == 0 ? mine0 : mine1);
             if (!ok) s[u][sb][i] = -INFINITY;
           }
-          tmax = fmaxf(tmax, s[u][sb][i]);
-        }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[u][sb][i]);
     tmax = column_lanes_max(tmax);
     // the maximum was taken over the raw scores (the scale is positive); the scale joins the
     // subtraction of the maximum in one fused multiply-add
@@ -935,15 +1046,19 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
     }
     // values of keys that do not exist yet, or that lie below the window (their pages may have
     // been given back), may be anything: zero them (the last and the first block only)
-    if (akb * 64 + 64 > hi || akb * 64 < lo) {
+    // (in the last block and in one that is half another wave's, whole above the window, with a mask of four words for the lane's eight keys)
+    const bool by_words = akb * 64 >= lo && (akb * 64 + 64 > hi || !(mine0 && mine1));
+    if (akb * 64 < lo) {
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const int key = akb * 64 + 32 * u + 8 * gq;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int e = 0; e < 8; ++e) {
+          const bool out_of = !(u == 0 ? mine0 : mine1) || key + e >= hi || (key + e < lo && key + e >= keep_first);
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (key + e >= hi || (key + e < lo && key + e >= keep_first)) vf[u][dt].h[e] = 0;
+          for (int dt = 0; dt < DT; ++dt)
+            if (out_of) vf[u][dt].h[e] = 0;
+        }
       }
     }
     if (ROPE && makes_kv && kb == kb_new && gq == new_gq) {
@@ -962,6 +1077,22 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
           }
         }
     }
+    if (by_words) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int n = (u == 0 ? mine0 : mine1) ? hi - (akb * 64 + 32 * u + 8 * gq) : 0;  // keys of the eight that count
+        u32x4_t keep;
+#pragma unroll
+        for (int wd = 0; wd < 4; ++wd) keep[wd] = n >= 2 * wd + 2 ? 0xffffffffu : n == 2 * wd + 1 ? 0x0000ffffu : 0u;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          AFrag8 v;
+          v.u = vf[u][dt].u & keep;
+          acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v.v, pf[u].v, acc[dt], 0, 0, 0);
+        }
+      }
+      continue;
+    }
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -975,34 +1106,47 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
 #undef ATT_PUT_NEW_K
   l = column_lanes_sum(l);
 
+  // Across the waves: every wave leaves its sums in LDS and merges a W-th of the head (with two maps, whose norm needs the whole head, wave
+  // 0 all of it): what is merged is DO tiles from dt0 on.
+  constexpr int DO = EXT || W == 1 ? DT : DT / W;
+  int dt0 = 0, dts = DT;
+  f32x4_t res[DO];
   if (W > 1) {
-    constexpr int WP = W > 1 ? W - 1 : 1;
-    __shared__ f32x4_t part_o[WP][DT][64];
-    __shared__ float part_m[WP][64], part_l[WP][64];
-    if (wave > 0) {
+    __shared__ f32x4_t part_o[W][DT][64];
+    __shared__ float part_m[W][64], part_l[W][64];
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) part_o[wave - 1][dt][lane] = acc[dt];
-      part_m[wave - 1][lane] = m;
-      part_l[wave - 1][lane] = l;
-    }
+    for (int dt = 0; dt < DT; ++dt) part_o[wave][dt][lane] = acc[dt];
+    part_m[wave][lane] = m;
+    part_l[wave][lane] = l;
     __syncthreads();
-    if (wave > 0) return;
-    float m_all = m;
+    if (!(EXT && maps.on)) dt0 = wave * (DT / W), dts = DT / W;
+    else if (wave > 0) return;
+    float pm[W], pl[W];
 #pragma unroll
-    for (int w = 0; w < W - 1; ++w) m_all = fmaxf(m_all, part_m[w][lane]);
+    for (int w = 0; w < W; ++w) pm[w] = part_m[w][lane], pl[w] = part_l[w][lane];
+#pragma unroll
+    for (int dt = 0; dt < DO; ++dt)
+      if (!EXT || dt < dts) res[dt] = part_o[0][dt0 + dt][lane];
+    float m_all = pm[0];
+#pragma unroll
+    for (int w = 1; w < W; ++w) m_all = fmaxf(m_all, pm[w]);
     const float m_safe = m_all == -INFINITY ? 0.f : m_all;
-    const float a0 = fast_exp2(m - m_safe);
-    l *= a0;
+    const float a0 = fast_exp2(pm[0] - m_safe);
+    l = pl[0] * a0;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] *= a0;
+    for (int dt = 0; dt < DO; ++dt) res[dt] *= a0;
 #pragma unroll
-    for (int w = 0; w < W - 1; ++w) {
-      const float aw = fast_exp2(part_m[w][lane] - m_safe);
-      l += aw * part_l[w][lane];
+    for (int w = 1; w < W; ++w) {
+      const float aw = fast_exp2(pm[w] - m_safe);
+      l += aw * pl[w];
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) acc[dt] += aw * part_o[w][dt][lane];
+      for (int dt = 0; dt < DO; ++dt)
+        if (!EXT || dt < dts) res[dt] += aw * part_o[w][dt0 + dt][lane];
     }
     m = m_all;
+  } else {
+#pragma unroll
+    for (int dt = 0; dt < DO; ++dt) res[dt] = acc[dt];
   }
 
   if (EXT && maps.on && n_splits == 1) {
@@ -1010,21 +1154,21 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
     const float inv = 1.f / l;
     float ss = 0.f;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < DO; ++dt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float a = acc[dt][i] * inv;
-        acc[dt][i] = fmaf(-maps.lambda, other_map(a), a);
-        ss = fmaf(acc[dt][i], acc[dt][i], ss);
+        const float a = res[dt][i] * inv;
+        res[dt][i] = fmaf(-maps.lambda, other_map(a), a);
+        ss = fmaf(res[dt][i], res[dt][i], ss);
       }
     const float to_unit = maps.gain / sqrtf(column_lanes_sum(ss) / static_cast<float>(D) + maps.eps);
     if (col_ok && hh % 2 == 0) {
       bf16_t* op = out + (static_cast<size_t>(tok0 + tt) * (n_heads / 2) + (h_base + hh) / 2) * D + 4 * gq;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
+      for (int dt = 0; dt < DO; ++dt) {
         u32x2_t w;
-        w[0] = pack_bf16x2(acc[dt][0] * to_unit, acc[dt][1] * to_unit);
-        w[1] = pack_bf16x2(acc[dt][2] * to_unit, acc[dt][3] * to_unit);
+        w[0] = pack_bf16x2(res[dt][0] * to_unit, res[dt][1] * to_unit);
+        w[1] = pack_bf16x2(res[dt][2] * to_unit, res[dt][3] * to_unit);
         *reinterpret_cast<u32x2_t*>(op + 16 * dt) = w;
       }
     }
@@ -1033,22 +1177,23 @@ __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
       // (m and l are in powers of two: the sink's share is 2^(sink log2(e) - m))
       if (EXT && sink != nullptr) l += fast_exp2(fmaf(sink[h_base + hh], 1.4426950408889634f, -m));
       const float inv = 1.f / l;
-      bf16_t* op = out + (static_cast<size_t>(tok0 + tt) * n_heads + h_base + hh) * D + 4 * gq;
+      bf16_t* op = out + (static_cast<size_t>(tok0 + tt) * n_heads + h_base + hh) * D + 16 * dt0 + 4 * gq;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
+      for (int dt = 0; dt < DO; ++dt) {
         u32x2_t w;
-        w[0] = pack_bf16x2(acc[dt][0] * inv, acc[dt][1] * inv);
-        w[1] = pack_bf16x2(acc[dt][2] * inv, acc[dt][3] * inv);
-        *reinterpret_cast<u32x2_t*>(op + 16 * dt) = w;
+        w[0] = pack_bf16x2(res[dt][0] * inv, res[dt][1] * inv);
+        w[1] = pack_bf16x2(res[dt][2] * inv, res[dt][3] * inv);
+        if (!EXT || dt < dts) *reinterpret_cast<u32x2_t*>(op + 16 * dt) = w;
       }
     }
   } else {
     // partial result of this split: unnormalised output, running maximum and sum
-    const size_t widx = (static_cast<size_t>(t) * gridDim.y + blockIdx.y) * n_splits + blockIdx.z;
-    float* wo = ws_o + (widx * 16 + r) * D + 4 * gq;
+    const size_t widx = (static_cast<size_t>(t) * (n_kv * shape.chunks) + blockIdx.y) * n_splits + blockIdx.z;
+    float* wo = ws_o + (widx * 16 + r) * D + 16 * dt0 + 4 * gq;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4_t*>(wo + 16 * dt) = acc[dt];
-    if (gq == 0) {
+    for (int dt = 0; dt < DO; ++dt)
+      if (!EXT || dt < dts) *reinterpret_cast<f32x4_t*>(wo + 16 * dt) = res[dt];
+    if (gq == 0 && dt0 == 0) {
       ws_ml[(widx * 16 + r) * 2] = m;
       ws_ml[(widx * 16 + r) * 2 + 1] = l;
     }
@@ -1430,32 +1575,53 @@ __global__ __launch_bounds__(256, CT == 1 ? 3 : 2) void attn_mfma_prefill_kernel
 // A thread owns four consecutive output elements of one column.
 // blockIdx.x names a group of 16 columns: a tile of the short-span kernel (parts == 1), or one
 // wave's share of a long tile (parts == 4: group x is wave x % 4 of tile x / 4).
+static uint32_t combine_shape(int hpt, int parts, int qpk) {
+  return static_cast<uint32_t>(hpt) | static_cast<uint32_t>(parts) << 5 | static_cast<uint32_t>(qpk) << 9;
+}
+// Bound by the launch and the trips to memory: a workgroup's first 256 pieces are asked for while the tile's row is still on its
+// way (the columns of a group are all there, whether they stand for anything or not).  One trip in place of three: the tile, then the maxima, then the outputs.
 template <int D>
 __global__ __launch_bounds__(256) void attn_combine_kernel(
-    bf16_t* __restrict__ out, const int32_t* __restrict__ tiles, int n_heads, int n_kv, int hpt,
-    int chunks, int n_splits, const float* __restrict__ ws_o, const float* __restrict__ ws_ml, int parts,
-    const float* __restrict__ sink) {
-  const int t = blockIdx.x / parts, part = blockIdx.x % parts;
+    bf16_t* __restrict__ out, const int32_t* __restrict__ tiles, const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+    const float* __restrict__ sink, int n_splits, int n_heads, int groups_y, uint32_t shape) {
+  // (`shape` and groups_y = gridDim.y: all arguments come with the launch)
+  const int hpt = shape & 31, parts = (shape >> 5) & 15, qpk = shape >> 9;
+  int t = blockIdx.x, part = 0, g = blockIdx.y, chunk = 0;
+  if (parts > 1) t = blockIdx.x / parts, part = blockIdx.x % parts;
+  if (qpk > hpt) {
+    const int chunks = (qpk + hpt - 1) / hpt;
+    g = blockIdx.y / chunks, chunk = blockIdx.y % chunks;
+  }
   const int tpt_ = 16 / hpt;
-  const int tok0 = tiles[4 * t + 1] + part * tpt_, ntok = tiles[4 * t + 2] - part * tpt_;
-  const int g = blockIdx.y / chunks, chunk = blockIdx.y % chunks;
-  const int qpk = n_heads / n_kv;
+  const int32_t* tile = tiles + 4 * t;
   const int h_base = g * qpk + chunk * hpt;
   const int heads_here = min(hpt, qpk - chunk * hpt);
-  const size_t w0 = (static_cast<size_t>(blockIdx.x) * gridDim.y + blockIdx.y) * n_splits;
-  for (int e = threadIdx.x; e < 16 * (D / 4); e += blockDim.x) {
+  const size_t w0 = (static_cast<size_t>(blockIdx.x) * groups_y + blockIdx.y) * n_splits;
+  // (a group of 16 columns holds tpt_ tokens; with a head count that does not divide 16 the
+  // columns left over stand for nothing, not for the next part's first token)
+  const bool all_heads = heads_here == hpt;  // (then the c-th column that may stand for something is column c)
+  auto merge = [&](int e) {
     const int c = e / (D / 4), d = (e % (D / 4)) * 4;
-    const int tt = c / hpt, hh = c % hpt;
-    // (a group of 16 columns holds tpt_ tokens; with a head count that does not divide 16 the
-    // columns left over stand for nothing, not for the next part's first token)
-    if (tt >= min(ntok, tpt_) || hh >= heads_here) continue;
+    float sink_raw = 0.f;
+    if (sink != nullptr) sink_raw = sink[h_base + c % heads_here];
+    int col = c;
+    if (!all_heads) col = min(c / heads_here, tpt_ - 1) * hpt + c % heads_here;
     float merged[4];
-    attn_merge_splits(ws_o, ws_ml, w0 * 16 + c, n_splits, D, d, merged,
-                      sink != nullptr ? sink[h_base + hh] * 1.4426950408889634f : -INFINITY);
-    u32x2_t o;
-    o[0] = pack_bf16x2(merged[0], merged[1]);
-    o[1] = pack_bf16x2(merged[2], merged[3]);
-    *reinterpret_cast<u32x2_t*>(out + (static_cast<size_t>(tok0 + tt) * n_heads + h_base + hh) * D + d) = o;
+    attn_merge_splits(ws_o, ws_ml, w0 * 16 + col, n_splits, D, d, merged, sink != nullptr ? sink_raw * 1.4426950408889634f : -INFINITY);
+    return u32x2_t{pack_bf16x2(merged[0], merged[1]), pack_bf16x2(merged[2], merged[3])};
+  };
+  const int tok0 = tile[1] + part * tpt_, ntok = tile[2] - part * tpt_;
+  u32x2_t o = merge(threadIdx.x);
+  asm volatile("" ::"v"(o));  // (made here: not moved to the condition below, which waits for the tile)
+  const int pieces = min(ntok, tpt_) * heads_here * (D / 4);
+  auto put = [&](int e) {
+    const int c = e / (D / 4), tt = c / heads_here, hh = c % heads_here;
+    *reinterpret_cast<u32x2_t*>(out + (static_cast<size_t>(tok0 + tt) * n_heads + h_base + hh) * D + (e % (D / 4)) * 4) = o;
+  };
+  if (static_cast<int>(threadIdx.x) < pieces) put(threadIdx.x);
+  for (int e = threadIdx.x + 256; e < pieces; e += 256) {
+    o = merge(e);
+    put(e);
   }
 }
 
@@ -1596,9 +1762,9 @@ extern "C" int yk_attn_mfma_prefill(const void* q, int q_stride, void* out, cons
     else if (maps == 2)
       attn_combine_maps_kernel<128><<<cgrid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, n_heads, n_kv, hpt, chunks, n_splits, ws_o, ws_ml, 4 * col_tiles, map_args);
     else if (head_dim == 64)
-      attn_combine_kernel<64><<<cgrid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, n_heads, n_kv, hpt, chunks, n_splits, ws_o, ws_ml, 4 * col_tiles, sink);
+      attn_combine_kernel<64><<<cgrid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, ws_o, ws_ml, sink, n_splits, n_heads, n_kv * chunks, combine_shape(hpt, 4 * col_tiles, n_heads / n_kv));
     else
-      attn_combine_kernel<128><<<cgrid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, n_heads, n_kv, hpt, chunks, n_splits, ws_o, ws_ml, 4 * col_tiles, sink);
+      attn_combine_kernel<128><<<cgrid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, ws_o, ws_ml, sink, n_splits, n_heads, n_kv * chunks, combine_shape(hpt, 4 * col_tiles, n_heads / n_kv));
     return yk_check_launch("attn_combine");
   }
   return 0;
@@ -1649,10 +1815,12 @@ static int launch_attn_mfma(const void* q, int q_stride, void* out, const void* 
   dim3 grid(n_tiles, n_kv * chunks, n_splits), block(64 * n_waves);
   const bool tiled = cache_is_tiled(YK_BF16, head_dim, page_size);
   const RopeSrc rs = rope ? *rope : RopeSrc{};
+  const AttnShape shape{n_heads / n_kv, hpt, chunks, static_cast<uint32_t>((256 + hpt - 1) / hpt),
+                        n_splits > 1 ? inverse_of(n_splits) : 0u, inverse_of(page_size)};
 #define YK_ARGS                                                                                    \
-      static_cast<const bf16_t*>(q), q_stride, static_cast<bf16_t*>(out),                          \
-      static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), tiles, block_table, \
-      table_width, page_size, n_heads, n_kv, hpt, chunks, scale_log2, window, n_splits, ws_o, ws_ml, rs
+      tiles, block_table, static_cast<const bf16_t*>(k_cache), static_cast<const bf16_t*>(v_cache), \
+      static_cast<const bf16_t*>(q), static_cast<bf16_t*>(out), table_width, page_size, q_stride,  \
+      n_heads, n_kv, shape, scale_log2, window, n_splits, ws_o, ws_ml, rs
 #define YK_LAUNCH_R(DD, RR)                                                                        \
   if (tiled) {                                                                                     \
     if (n_waves == 1) attn_mfma_kernel<DD, 1, true, RR><<<grid, block, 0, stream>>>(YK_ARGS);      \
@@ -1679,7 +1847,7 @@ static int launch_attn_mfma(const void* q, int q_stride, void* out, const void* 
     if (yk_check_launch("attn_combine")) return -1;                                                \
   } else if (n_splits > 1 && !leave_splits) {                                                      \
     attn_combine_kernel<DD><<<dim3(n_tiles, n_kv * chunks), 256, 0, stream>>>(                     \
-        static_cast<bf16_t*>(out), tiles, n_heads, n_kv, hpt, chunks, n_splits, ws_o, ws_ml, 1, sink); \
+        static_cast<bf16_t*>(out), tiles, ws_o, ws_ml, sink, n_splits, n_heads, n_kv * chunks, combine_shape(hpt, 1, n_heads / n_kv)); \
     if (yk_check_launch("attn_combine")) return -1;                                                \
   }
   if (head_dim == 64) {
@@ -1744,6 +1912,9 @@ extern "C" int yk_attn_mfma_rope(const void* src, int src_dtype, int n_src_split
   rs.interleaved = interleaved;
   rs.max_positions = rotary_dim ? max_positions : 1;
   rs.append = append != 0;
+  const uintptr_t two = src_dtype == YK_F32 ? 8 : 4;
+  rs.by_fours = rotary_dim == head_dim && !interleaved && src_stride % 2 == 0 && reinterpret_cast<uintptr_t>(src) % two == 0 &&
+                reinterpret_cast<uintptr_t>(cos_t) % 8 == 0 && reinterpret_cast<uintptr_t>(sin_t) % 8 == 0;
   return launch_attn_mfma(nullptr, 0, out, k_cache, v_cache, tiles, n_tiles, block_table, table_width, page_size,
                           head_dim, n_heads, n_kv, scale, window, n_waves, n_splits, workspace, workspace_floats,
                           leave_splits, &rs, src_dtype == YK_F32, stream);
@@ -1766,8 +1937,8 @@ extern "C" int yk_attn_combine(void* out, const int32_t* tiles, int n_tiles, int
   const float* ws_ml = workspace + (need / (head_dim + 2)) * head_dim;
   const dim3 grid(n_tiles, n_kv * chunks);
   if (head_dim == 64)
-    attn_combine_kernel<64><<<grid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, n_heads, n_kv, hpt, chunks, n_splits, ws_o, ws_ml, 1, nullptr);
+    attn_combine_kernel<64><<<grid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, ws_o, ws_ml, nullptr, n_splits, n_heads, n_kv * chunks, combine_shape(hpt, 1, n_heads / n_kv));
   else
-    attn_combine_kernel<128><<<grid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, n_heads, n_kv, hpt, chunks, n_splits, ws_o, ws_ml, 1, nullptr);
+    attn_combine_kernel<128><<<grid, 256, 0, stream>>>(static_cast<bf16_t*>(out), tiles, ws_o, ws_ml, nullptr, n_splits, n_heads, n_kv * chunks, combine_shape(hpt, 1, n_heads / n_kv));
   return yk_check_launch("attn_combine");
 }

@@ -325,24 +325,77 @@ __host__ __device__ inline int attn_heads_per_tile(int n_heads, int n_kv) {
 // exp2(m_s - max m), in the order of s.  `col0` is the column's index in split 0
 // (group * 16 + column); split s lies 16 columns further each.  `sink_log2` (-inf: none): a term 2^sink_log2 that joins
 // the sum of weights once, with no output of its own.
+// Up to MERGE_AT_ONCE splits are all asked for before any is used (in groups, as ask_slices does it: what lies beyond the last is read
+// from the last and masked to zero).
+constexpr int MERGE_AT_ONCE = 8;
+template <int FROM = 0, int TO = 1>
+__device__ __forceinline__ void merge_ask(const float* o, const float* ml, int n_splits, size_t o_stride, float2 (&w)[MERGE_AT_ONCE],
+                                          float4 (&v)[MERGE_AT_ONCE]) {
+#pragma unroll
+  for (int j = FROM; j < TO; ++j) {
+    w[j] = *reinterpret_cast<const float2*>(ml);
+    v[j] = *reinterpret_cast<const float4*>(o);
+    ml += j + 1 < n_splits ? 32 : 0;
+    o += j + 1 < n_splits ? o_stride : 0;
+  }
+  if constexpr (TO < MERGE_AT_ONCE) {
+    if (n_splits > TO) merge_ask<TO, 2 * TO>(o, ml, n_splits, o_stride, w, v);
+  }
+}
+template <int FROM = 0, int TO = 1>
+__device__ __forceinline__ float merge_max(int n_splits, const float2 (&w)[MERGE_AT_ONCE], float m_max) {
+#pragma unroll
+  for (int j = FROM; j < TO; ++j) m_max = fmaxf(m_max, w[j].x);
+  if constexpr (TO < MERGE_AT_ONCE) {
+    if (n_splits > TO) return merge_max<TO, 2 * TO>(n_splits, w, m_max);
+  }
+  return m_max;
+}
+template <int FROM = 0, int TO = 1>
+__device__ __forceinline__ void merge_join(int n_splits, const float2 (&w)[MERGE_AT_ONCE], const float4 (&v)[MERGE_AT_ONCE], float m_max,
+                                           float (&num)[4], float& den) {
+#pragma unroll
+  for (int j = FROM; j < TO; ++j) {
+    const uint32_t keep = __builtin_amdgcn_readfirstlane((j - n_splits) >> 31);
+    auto kept = [&](float x) { return __uint_as_float(__float_as_uint(x) & keep); };
+    const float e = exp2f(w[j].x - m_max);
+    num[0] += e * kept(v[j].x);
+    num[1] += e * kept(v[j].y);
+    num[2] += e * kept(v[j].z);
+    num[3] += e * kept(v[j].w);
+    den += e * kept(w[j].y);
+  }
+  if constexpr (TO < MERGE_AT_ONCE) {
+    if (n_splits > TO) merge_join<TO, 2 * TO>(n_splits, w, v, m_max, num, den);
+  }
+}
 __device__ __forceinline__ void attn_merge_splits(const float* __restrict__ o, const float* __restrict__ ml,
                                                   size_t col0, int n_splits, int head_dim, int d,
                                                   float out[4], float sink_log2 = -INFINITY) {
   const float* mlc = ml + col0 * 2;
+  const float* oc = o + col0 * head_dim + d;
   float m_max = sink_log2;
-#pragma unroll 4
-  for (int s = 0; s < n_splits; ++s) m_max = fmaxf(m_max, mlc[static_cast<size_t>(s) * 32]);
   float num[4] = {0.f, 0.f, 0.f, 0.f};
   float den = 0.f;
+  if (n_splits <= MERGE_AT_ONCE) {
+    float2 w[MERGE_AT_ONCE];
+    float4 v[MERGE_AT_ONCE];
+    merge_ask(oc, mlc, n_splits, static_cast<size_t>(16) * head_dim, w, v);
+    m_max = merge_max(n_splits, w, m_max);
+    merge_join(n_splits, w, v, m_max, num, den);
+  } else {
 #pragma unroll 4
-  for (int s = 0; s < n_splits; ++s) {
-    const float w = exp2f(mlc[static_cast<size_t>(s) * 32] - m_max);
-    const float4 v = *reinterpret_cast<const float4*>(o + (col0 + static_cast<size_t>(s) * 16) * head_dim + d);
-    num[0] += w * v.x;
-    num[1] += w * v.y;
-    num[2] += w * v.z;
-    num[3] += w * v.w;
-    den += w * mlc[static_cast<size_t>(s) * 32 + 1];
+    for (int s = 0; s < n_splits; ++s) m_max = fmaxf(m_max, mlc[static_cast<size_t>(s) * 32]);
+#pragma unroll 4
+    for (int s = 0; s < n_splits; ++s) {
+      const float w = exp2f(mlc[static_cast<size_t>(s) * 32] - m_max);
+      const float4 v = *reinterpret_cast<const float4*>(oc + static_cast<size_t>(s) * 16 * head_dim);
+      num[0] += w * v.x;
+      num[1] += w * v.y;
+      num[2] += w * v.z;
+      num[3] += w * v.w;
+      den += w * mlc[static_cast<size_t>(s) * 32 + 1];
+    }
   }
   if (sink_log2 != -INFINITY) den += exp2f(sink_log2 - m_max);
   const float inv = 1.f / den;
