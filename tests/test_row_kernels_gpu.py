@@ -1,4 +1,6 @@
 """Norms and activations whose threads hold one or two pieces of a row, at rows that do not fill their threads."""
+import math
+
 import pytest
 import torch
 
@@ -141,7 +143,6 @@ def test_decode_attention_with_slices_and_splits(h, g, d, page):
     """Single tokens behind contexts at the edges of half blocks, blocks and pages (sizes that are no powers of two among them), the slots
     behind them NaN: any number of slices of the projection gives the bits of its sum, and any number of splits, up to more
     than are merged at once, agrees with the plain reference within bfloat16's rounding of probabilities and values (2e-2, 2^-6 as elsewhere)."""
-    import math
     import types
 
     o, gen = ops(), torch.Generator().manual_seed(page + h)
@@ -182,3 +183,23 @@ def test_decode_attention_with_slices_and_splits(h, g, d, page):
                                    types.SimpleNamespace(arrays=arrays), 0, None)
             err = (results[0].cpu() - want).abs()
             assert bool((err <= 2e-2 + 2 ** -6 * want.abs()).all()), (slices, splits, err.max().item())
+
+
+# rows that fill a load of x and do not; K at a chunk, beyond one round of the waves, with remainders; 16 waves and eight; a last group of columns that is none
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(40, 8), (40, 256), (33, 2056), (48, 2304), (16, 6144), (40, 6400), (4112, 2312)])
+def test_few_rows_in_one_workgroup_by_rows_of_x(m, n, k):
+    """Each row of x against a row of ones but for one place far along K: a step that met another row's or another step's x would show."""
+    o, g = ops(), torch.Generator().manual_seed(m + k)
+    x, w = torch.randn(m, k, generator=g).bfloat16(), torch.randn(n, k, generator=g).bfloat16()
+    wide = torch.full((m, k + 8), float("nan"), dtype=torch.bfloat16)  # rows further apart than they are long
+    wide[:, :k] = x
+    want = x.double() @ w.double().T
+    got = o.gemm_cols(wide.cuda()[:, :k], w.cuda(), torch.float32)
+    # float32 sums of k products of about 1: each addition rounds by 2^-24 of a sum of up to 4 sqrt(k)
+    assert (got.cpu().double() - want).abs().max() <= 4 * math.sqrt(k) * 2.0 ** -24 * math.sqrt(k / 32 + 16) * 4
+    one = torch.zeros(m, k, dtype=torch.bfloat16)
+    for r in range(m):
+        one[r, (r * 37 + k // 2) % k] = 1.0
+    got = o.gemm_cols(one.cuda(), w.cuda(), torch.bfloat16).cpu()
+    assert torch.equal(got, torch.stack([w[:, (r * 37 + k // 2) % k] for r in range(m)]))

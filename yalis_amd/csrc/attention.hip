@@ -636,13 +636,6 @@ struct AttnShape {
   uint32_t splits_inverse;  // inverse_of(n_splits), for n_splits > 1
   uint32_t page_inverse;    // inverse_of(page_size)
 };
-// x / n for x from 0 and n from 2 up: by ceil(2^32 / n) the quotient is less than x / 2^32 too large before it is cut, so at most one
-static uint32_t inverse_of(int n) { return static_cast<uint32_t>(((1ull << 32) + n - 1) / n); }
-__device__ __forceinline__ int divide_by(int x, int n, uint32_t inverse) {
-  const uint32_t q = __umulhi(static_cast<uint32_t>(x), inverse);
-  return static_cast<int>(q - (q * static_cast<uint32_t>(n) > static_cast<uint32_t>(x) ? 1u : 0u));
-}
-
 template <int D, int W, bool TILED, int SRC, bool EXT = false>
 __global__ __launch_bounds__(64 * W, 2) void attn_mfma_kernel(
     const int32_t* __restrict__ tiles, const int32_t* __restrict__ block_table,

@@ -260,6 +260,13 @@ __device__ __forceinline__ void load_to_lds(const void* at, int bytes, void* to,
 #endif
 }
 
+// x / n for x from 0 and n from 2 up: by ceil(2^32 / n) the quotient is less than x / 2^32 too large before it is cut, so at most one
+inline uint32_t inverse_of(int n) { return static_cast<uint32_t>(((1ull << 32) + n - 1) / n); }
+__device__ __forceinline__ int divide_by(int x, int n, uint32_t inverse) {
+  const uint32_t q = __umulhi(static_cast<uint32_t>(x), inverse);
+  return static_cast<int>(q - (q * static_cast<uint32_t>(n) > static_cast<uint32_t>(x) ? 1u : 0u));
+}
+
 // Gated activations: 0 = silu, 1 = gelu (tanh form); float32.
 __device__ __forceinline__ float act_silu(float z) { return z / (1.f + expf(-z)); }
 __device__ __forceinline__ float act_gelu_tanh(float z) {

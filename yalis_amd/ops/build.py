@@ -50,12 +50,13 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-# Flags of one library alone.  "kernels": the first 14 words of a kernel's arguments come in scalar registers with the launch, in
-# place of a load that every wave waits for before it asks for anything else.  An empty kernel of a replayed graph takes 1.65 us
-# with it and 1.57 without, one whose first loads hang on its arguments 0.1 to 0.4 us less (8 MiB read by 256 workgroups 3.7 ->
-# 3.4, a norm of eight rows 2.85 -> 2.60; a decode step of the expert design's 1,400 kernels 11.9 -> 11.5 ms).  "sampling" goes
-# without: its two kernels are long, and took 20.4 -> 20.5 us.
-LIB_FLAGS = {"kernels": ["-mllvm", "-amdgpu-kernarg-preload-count=16"]}
+# Kernel arguments that come in scalar registers with the launch (the first 14 words), in place of a load that every wave waits for
+# before it asks for anything else.  An empty kernel of a replayed graph takes 1.65 us with it and 1.57 without, one whose first loads hang on
+# its arguments 0.1 to 0.4 us less (8 MiB read by 256 workgroups 3.7 -> 3.4, a norm of eight rows 2.85 -> 2.60; a decode step of the
+# expert design's 1,400 kernels 11.9 -> 11.5 ms).  Not the sources whose kernels ask for more before they begin: the few-row
+# product in slices takes 8.8 us without and 9.2 with it (one row, 2,048 x 8,192), choosing a token 20.4 and 20.5.
+PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
+NO_PRELOAD = {"gemm.hip", "sampling.hip", "probe.hip", "runtime.hip"}
 
 _lock = threading.Lock()
 _loaded: Dict[str, ctypes.CDLL] = {}
@@ -163,8 +164,7 @@ def build_host(force: bool = False) -> str:
 def build_kernels(name: str = "kernels", force: bool = False) -> str:
     """One library of HIP kernels for gfx950: one object per source, compiled side by side."""
     sources = KERNEL_LIBS[name]
-    flags = HIPCC_FLAGS + LIB_FLAGS.get(name, [])
-    digest = _digest(sources, flags + LINK_LIBS.get(name, []))
+    digest = _digest(sources, HIPCC_FLAGS + PRELOAD + sorted(NO_PRELOAD) + LINK_LIBS.get(name, []))
     bdir = build_dir()
     lib = os.path.join(bdir, f"libyalis_{name}.so")
     if not force and _is_current(lib, digest):
@@ -176,7 +176,7 @@ def build_kernels(name: str = "kernels", force: bool = False) -> str:
 
     def one(src: str, obj: str) -> None:
         try:
-            _run([hipcc, *flags, "-c", os.path.join(CSRC, src), "-o", obj], src)
+            _run([hipcc, *HIPCC_FLAGS, *([] if src in NO_PRELOAD else PRELOAD), "-c", os.path.join(CSRC, src), "-o", obj], src)
             _say(f"compiled {src}")
         except BaseException as e:  # noqa: BLE001 - reported below
             errors.append(e)
