@@ -203,3 +203,35 @@ def test_few_rows_in_one_workgroup_by_rows_of_x(m, n, k):
         one[r, (r * 37 + k // 2) % k] = 1.0
     got = o.gemm_cols(one.cuda(), w.cuda(), torch.bfloat16).cpu()
     assert torch.equal(got, torch.stack([w[:, (r * 37 + k // 2) % k] for r in range(m)]))
+
+
+@pytest.mark.parametrize("n,top,experts", [(1, 1, 2), (1, 4, 4), (4, 2, 16), (5, 3, 7), (16, 4, 32), (33, 1, 2), (64, 1, 2), (21, 3, 3)])
+@pytest.mark.parametrize("hidden,ff", [(32, 32), (96, 64), (160, 288), (1056, 1024), (2048, 96)])  # fewer steps of 32 than waves, than are asked for ahead, more
+def test_experts_of_few_pairs(n, top, experts, hidden, ff):
+    """Pairs that find their own tiles: the plain arithmetic (bfloat16 rounds y: 2e-2 as for every path), each token's rows the bits that it
+    has alone, whatever its neighbours choose (more than 16 of one expert among them), and a token of NaN changes no other's rows."""
+    o, g = ops(), torch.Generator().manual_seed(n + hidden + experts)
+    x = torch.randn(n, hidden, generator=g).bfloat16()
+    ids = torch.randint(-2, 55, (n,), generator=g, dtype=torch.int32)  # (ids out of the table's range read its ends)
+    table = torch.rand(50, experts, generator=g).argsort(-1)[:, :top].to(torch.int32).contiguous()
+    wgu = (torch.randn(experts, 2, ff, hidden, generator=g) / hidden ** 0.5).bfloat16()
+    wd = (torch.randn(experts, hidden, ff, generator=g) / ff ** 0.5).bfloat16()
+    act = ("clamped_swish", 1.5, 1.702)
+    dev = [t.cuda() for t in (x, ids, table, wgu, wd)]
+    got = o.moe_experts(*dev, act).cpu()
+    want = R.moe_experts(x, ids.clamp(0, 49), table, wgu, wd, act)
+    assert (got - want).abs().max() <= 2e-2 * max(1.0, float(want.abs().max()))
+    for t in {0, n // 2, n - 1}:
+        alone = o.moe_experts(dev[0][t: t + 1], dev[1][t: t + 1], *dev[2:], act).cpu()
+        assert torch.equal(alone, got[t * top: (t + 1) * top])
+    # a choice per token, with a row of x per token and per pair, without a gate
+    choice = table[ids.clamp(0, 49).long()].contiguous().cuda()
+    assert torch.equal(o.moe_experts(dev[0], None, choice, dev[3], dev[4], act, input_per_token=True).cpu(), got)
+    assert torch.equal(o.moe_experts(dev[0].repeat_interleave(top, 0), None, choice, dev[3], dev[4], act).cpu(), got)
+    up = wgu[:, :1].contiguous()
+    close(o.moe_experts(dev[0], dev[1], dev[2], up.cuda(), dev[4], "relu2").cpu(), R.moe_experts(x, ids.clamp(0, 49), table, up, wd, "relu2"), 2e-2)
+    if n > 1:
+        bad = dev[0].clone()
+        bad[0] = float("nan")
+        got2 = o.moe_experts(bad, *dev[1:], act).cpu()
+        assert torch.equal(got2[top:], got[top:])  # (its own rows: the pair's clamps drop a NaN)

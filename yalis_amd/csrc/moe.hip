@@ -664,3 +664,207 @@ extern "C" int yk_moe_down(const void* y, int dtype, const void* w, int w_dtype,
 #undef YK_CASE
   return yk_fail("moe_down: unsupported dtype combination");
 }
+
+// ------------------------------------------------------------------ products of few pairs
+// The decode steps' form.  Bound by the reading of the experts' weights; before, by the kernel that sorted the pairs (4 us of one
+// workgroup), by two steps of loads in flight and by a tile's workgroups all on one die (so that they share rows of x, which are few here).  Both products, us, sorted
+// first / now: one token of two experts of 1,024 in width 2,048 (25 MB) 22.2 / 10.6, four tokens (6 experts) 28.0 / 19.7, 16 (15 experts) 47.5 / 44.9; in width
+// 4,096, four tokens of four experts (12) 78.7 / 56.7, 16 (28) 151.6 / 142.8.
+// Up to 64 pairs route themselves: every wave of both products looks its pairs' experts up, one a lane, and finds its own tile in
+// them, so that no kernel has to sort them first.  Tile t (of as many as there are pairs) is the expert of pair t and that pair's place
+// among the expert's pairs if it is the first of 16 of them; other tiles are nobody's.  Rows of y lie in the order of the pairs.
+struct FewPairs {
+  const int32_t *token_ids, *table;  // as moe_route takes them
+  int vocab, top, n_pairs;
+  uint32_t top_inverse;  // inverse_of(top), for top > 1
+};
+__device__ __forceinline__ int pair_token(const FewPairs& p, int pair) { return p.top > 1 ? divide_by(pair, p.top, p.top_inverse) : pair; }
+// whether tile t is somebody's; then its expert, its pairs' count and the pair of the lane's row lane % 16 (rows beyond them repeat the last)
+__device__ __forceinline__ bool few_pairs_tile(const FewPairs& p, int t, int& e, int& count, int& pair) {
+  const int lane = threadIdx.x % 64, i = min(lane, p.n_pairs - 1), token = pair_token(p, i);
+  int id = token;
+  if (p.token_ids != nullptr) id = p.token_ids[token];
+  id = id < 0 ? 0 : (id >= p.vocab ? p.vocab - 1 : id);
+  const int mine = p.table[static_cast<size_t>(id) * p.top + (i - token * p.top)];
+  e = __builtin_amdgcn_readlane(mine, t);
+  const bool with = lane < p.n_pairs && mine == e;
+  const unsigned long long all = __ballot(with);
+  const int before = __popcll(all & ((1ull << t) - 1));
+  if (before % 16) return false;
+  count = min(16, static_cast<int>(__popcll(all)) - before);
+  // the pair of every rank: a pair's lane leaves its number with the lane of its rank (the others with the last lane, which has no rank then)
+  const int rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(all >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(all), 0));
+  const int by_rank = __builtin_amdgcn_ds_permute(4 * (with ? rank : 63), lane);
+  pair = __builtin_amdgcn_ds_bpermute(4 * (before + min(lane % 16, count - 1)), by_rank);
+  return true;
+}
+
+// acc[n] += 16 rows of w[n] . 16 rows of x over n_steps steps of 32 along K, DEPTH of them asked for ahead: a unit that runs one
+// such workgroup has as many bytes in flight as its waves ask for, and two steps are 32 KiB of them.
+template <int NW, int DEPTH>
+__device__ __forceinline__ void few_pairs_product(const bf16_t* const (&w)[NW], const bf16_t* x, int n_steps, f32x4_t (&acc)[NW]) {
+  MoeFrag a[DEPTH][NW], b[DEPTH];
+  auto ask = [&](int slot, int step) {
+#pragma unroll
+    for (int n = 0; n < NW; ++n) a[slot][n].u = *reinterpret_cast<const u32x4_t*>(w[n] + 32 * step);
+    b[slot].u = *reinterpret_cast<const u32x4_t*>(x + 32 * step);
+  };
+  auto multiply = [&](int slot) {
+#pragma unroll
+    for (int n = 0; n < NW; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[slot][n].v, b[slot].v, acc[n], 0, 0, 0);
+  };
+  if (n_steps < DEPTH) {
+    for (int s = 0; s < n_steps; ++s) {
+      ask(0, s);
+      multiply(0);
+    }
+    return;
+  }
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) ask(d, d);
+  int s = 0;
+  for (; s + 2 * DEPTH <= n_steps; s += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      multiply(d);
+      ask(d, s + DEPTH + d);
+    }
+  }
+  const int rest = n_steps - s - DEPTH;  // fewer than DEPTH, beyond those that are on their way
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    multiply(d);
+    if (d < rest) ask(d, s + DEPTH + d);
+  }
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d)
+    if (d < rest) multiply(d);
+}
+
+// Tile after tile, a tile's groups on all dies: its expert's weights are all that is read, and a die's own path to memory is an eighth of it.
+__device__ __forceinline__ void few_pairs_place(int n_groups, uint32_t groups_inverse, int& tile, int& group) {
+  tile = n_groups > 1 ? divide_by(blockIdx.x, n_groups, groups_inverse) : blockIdx.x;
+  group = blockIdx.x - tile * n_groups;
+}
+
+// The two products for them, with the operands, the division of K among a workgroup's four waves and the order of the sums of the
+// kernels above (KS): the same bits.  The waves leave their sums in LDS and finish a share each: an activation is some 70
+// instructions, which one wave alone would run through eight times a lane.
+template <int FT, int WAVES, int DEPTH, bool GATED>
+__global__ __launch_bounds__(64 * WAVES) void moe_gate_up_few_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
+                                                              const int32_t* __restrict__ token_ids, const int32_t* __restrict__ table, int n_pairs,
+                                                              int n_groups, uint32_t groups_inverse, int top, int vocab, uint32_t top_inverse,
+                                                              int x_stride, int x_per_token, int hidden, int ff, int kind, float p0, float p1) {
+  const FewPairs pairs{token_ids, table, vocab, top, n_pairs, top_inverse};
+  int t, group;
+  few_pairs_place(n_groups, groups_inverse, t, group);
+  if (t >= n_pairs) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
+  int e, count, pair;
+  if (!few_pairs_tile(pairs, t, e, count, pair)) return;
+  const int f0 = group * 16 * FT;
+  const int k_share = ((hidden / 32 + WAVES - 1) / WAVES) * 32, k_begin = wave * k_share, n_steps = max(0, min(hidden - k_begin, k_share)) / 32;
+  constexpr int NW = (GATED ? 2 : 1) * FT;
+  const bf16_t* rows[NW];
+#pragma unroll
+  for (int f = 0; f < FT; ++f) {
+    const int row = min(f0 + 16 * f + r, ff - 1);  // (tiles beyond the width repeat its last row and are not stored)
+    rows[f] = w + (static_cast<size_t>(e) * (GATED ? 2 : 1) * ff + row) * hidden + 8 * g + k_begin;
+    if (GATED) rows[FT + f] = rows[f] + static_cast<size_t>(ff) * hidden;
+  }
+  f32x4_t acc[NW] = {};
+  few_pairs_product<NW, DEPTH>(rows, x + static_cast<size_t>(x_per_token ? pair_token(pairs, pair) : pair) * x_stride + 8 * g + k_begin, n_steps, acc);
+  __shared__ f32x4_t part[WAVES][NW][64];
+#pragma unroll
+  for (int n = 0; n < NW; ++n) part[wave][n][lane] = acc[n];
+  __syncthreads();
+  // output o of the workgroup's 256 FT: element o % 4 of lane o / 4 of a tile
+  for (int o = threadIdx.x; o < 256 * FT; o += 64 * WAVES) {
+    const int f = o / 256, i = o % 4, l = o / 4 % 64;
+    auto total = [&](int n) {
+      float v = 0.f;
+#pragma unroll
+      for (int w2 = 0; w2 < WAVES; ++w2) v += reinterpret_cast<const float*>(&part[w2][n][l])[i];
+      return v;
+    };
+    const int row = f0 + 16 * f + 4 * (l / 16) + i, its_pair = __builtin_amdgcn_ds_bpermute(4 * (l % 16), pair);  // (lane l % 16 holds its row's)
+    if (row >= ff || l % 16 >= count) continue;
+    const float v = total(f);
+    y[static_cast<size_t>(its_pair) * ff + row] = f32_to_bf16(GATED ? gated_pair(v, total(FT + f), kind, p0, p1) : act_plain(v, kind));
+  }
+}
+
+template <int FT, int WAVES, int DEPTH>
+__global__ __launch_bounds__(64 * WAVES) void moe_down_few_kernel(const bf16_t* __restrict__ y, const bf16_t* __restrict__ w, float* __restrict__ out,
+                                                           const int32_t* __restrict__ token_ids, const int32_t* __restrict__ table, int n_pairs,
+                                                           int n_groups, uint32_t groups_inverse, int top, int vocab, uint32_t top_inverse, int hidden,
+                                                           int ff) {
+  const FewPairs pairs{token_ids, table, vocab, top, n_pairs, top_inverse};
+  int t, group;
+  few_pairs_place(n_groups, groups_inverse, t, group);
+  if (t >= n_pairs) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
+  int e, count, pair;
+  if (!few_pairs_tile(pairs, t, e, count, pair)) return;
+  const int h0 = group * 16 * FT;
+  const int k_share = ((ff / 32 + WAVES - 1) / WAVES) * 32, k_begin = wave * k_share, n_steps = max(0, min(ff - k_begin, k_share)) / 32;
+  const bf16_t* rows[FT];
+#pragma unroll
+  for (int f = 0; f < FT; ++f) rows[f] = w + (static_cast<size_t>(e) * hidden + min(h0 + 16 * f + r, hidden - 1)) * ff + 8 * g + k_begin;
+  f32x4_t acc[FT] = {};
+  few_pairs_product<FT, DEPTH>(rows, y + static_cast<size_t>(pair) * ff + 8 * g + k_begin, n_steps, acc);
+  __shared__ f32x4_t part[WAVES][FT][64];
+#pragma unroll
+  for (int f = 0; f < FT; ++f) part[wave][f][lane] = acc[f];
+  __syncthreads();
+  for (int o = threadIdx.x; o < 256 * FT; o += 64 * WAVES) {
+    const int f = o / 256, i = o % 4, l = o / 4 % 64;
+    float v = 0.f;
+#pragma unroll
+    for (int w2 = 0; w2 < WAVES; ++w2) v += reinterpret_cast<const float*>(&part[w2][f][l])[i];
+    const int row = h0 + 16 * f + 4 * (l / 16) + i, its_pair = __builtin_amdgcn_ds_bpermute(4 * (l % 16), pair);
+    if (row < hidden && l % 16 < count) out[static_cast<size_t>(its_pair) * hidden + row] = v;
+  }
+}
+
+// Whether the products of so many pairs route themselves.
+extern "C" int yk_moe_few_pairs_ok(int n_pairs, int hidden, int ff, int x_stride) {
+  return n_pairs >= 1 && n_pairs <= 64 && yk_moe_mfma_ok(hidden, ff, x_stride) ? 1 : 0;
+}
+
+// Both products of up to 64 pairs, bfloat16 throughout but the float32 rows that come out.  token_ids, table, vocab, top: as moe_route; x has a
+// row per token (x_per_token) or per pair; y [n_pairs, ff] scratch.
+extern "C" int yk_moe_few_pairs(const int32_t* token_ids, const int32_t* table, int vocab, int top, int n_pairs, const void* x, int x_stride,
+                                int x_per_token, const void* w_gate_up, const void* w_down, int hidden, int ff, int gated, int kind, float p0,
+                                float p1, void* y, float* rows, hipStream_t stream) {
+  YK_REQUIRE(vocab >= 1 && top >= 1 && hidden > 0 && ff > 0 && x_stride >= hidden, "moe_few_pairs: bad sizes");
+  YK_REQUIRE(kind >= 0 && kind < (gated ? YK_GATED_KINDS : YK_PLAIN_KINDS), "moe_few_pairs: unknown activation");
+  YK_REQUIRE(yk_moe_few_pairs_ok(n_pairs, hidden, ff, x_stride), "moe_few_pairs: up to 64 pairs, sizes in multiples of 32");
+  YK_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(w_down) && aligned16(y) && aligned16(rows), "moe_few_pairs: operands must be 16-byte aligned");
+  const uint32_t top_inverse = top > 1 ? inverse_of(top) : 0u;
+  const bf16_t *xb = static_cast<const bf16_t*>(x), *wg = static_cast<const bf16_t*>(w_gate_up), *wd = static_cast<const bf16_t*>(w_down);
+  bf16_t* yb = static_cast<bf16_t*>(y);
+  YK_REQUIRE(static_cast<long long>(n_pairs) * ((std::max(ff, hidden) + 15) / 16) <= 0x7fffffffLL, "moe_few_pairs: too many tiles for one launch");
+#define YK_GU(GF, GW, GD, GATED)                                                                                                        \
+  {                                                                                                                                     \
+    const int groups = (ff + 16 * GF - 1) / (16 * GF);                                                                                  \
+    moe_gate_up_few_kernel<GF, GW, GD, GATED><<<static_cast<unsigned>(n_pairs * groups), 64 * GW, 0, stream>>>(                          \
+        xb, wg, yb, token_ids, table, n_pairs, groups, groups > 1 ? inverse_of(groups) : 0u, top, vocab, top_inverse, x_stride, x_per_token, \
+        hidden, ff, kind, p0, p1);                                                                                                      \
+  }
+#define YK_DN(DF, DW, DD)                                                                                                               \
+  {                                                                                                                                     \
+    const int groups = (hidden + 16 * DF - 1) / (16 * DF);                                                                              \
+    moe_down_few_kernel<DF, DW, DD><<<static_cast<unsigned>(n_pairs * groups), 64 * DW, 0, stream>>>(                                    \
+        yb, wd, rows, token_ids, table, n_pairs, groups, groups > 1 ? inverse_of(groups) : 0u, top, vocab, top_inverse, hidden, ff);    \
+  }
+  // One tile of 16 features a workgroup and eight steps ahead (us of both products, 16 experts of 1,024 in width 2,048, pairs of four tokens with 6
+  // distinct experts / 16 experts' pairs of 4,096 with 12: two tiles of gate rows 20.3 / 64.7, sixteen steps 19.7 / 65.2, eight waves 22.7 / 60.6, this 19.7 / 56.8).
+  if (gated) YK_GU(1, 4, 8, true)
+  else YK_GU(1, 4, 8, false)
+  if (yk_check_launch("moe_few_pairs (gate/up)")) return -1;
+  YK_DN(1, 4, 8)
+#undef YK_DN
+#undef YK_GU
+  return yk_check_launch("moe_few_pairs (down)");
+}

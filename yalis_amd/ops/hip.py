@@ -195,6 +195,11 @@ _SIGNATURES = {
          _c_float, _vp, _c_int, _vp],
         _c_int,
     ),
+    "yk_moe_few_pairs_ok": ([_c_int, _c_int, _c_int, _c_int], _c_int),
+    "yk_moe_few_pairs": (
+        [_vp, _vp, _c_int, _c_int, _c_int, _vp, _c_int, _c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _vp, _vp, _vp],
+        _c_int,
+    ),
     "yk_moe_down": ([_vp, _c_int, _vp, _c_int, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _vp], _c_int),
     "yk_gemm_fma": (
         [_vp, _c_int, _vp, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp],
@@ -2344,6 +2349,18 @@ class HipOps:
             return rows
         # tiles of 128 or 64 pairs where an expert has that many on average, else of 16
         tile_rows = 128 if pairs >= 96 * experts else (64 if pairs >= 48 * experts else 16)
+        bf = torch.bfloat16
+        if (tile_rows == 16 and x.dtype == bf and w_gate_up.dtype == bf and w_down.dtype == bf and self._ask("yk_moe_few_pairs_ok", pairs, hidden, ff, x.stride(0))
+                and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0 and w_down.data_ptr() % 16 == 0):
+            # few pairs route themselves: no kernel before the products
+            y = torch.empty((pairs, ff), dtype=bf, device=dev)
+            self._check(
+                self.lib.yk_moe_few_pairs(
+                    _ptr(token_ids), table.data_ptr(), vocab, top, pairs, x.data_ptr(), x.stride(0), int(x_top > 1), w_gate_up.data_ptr(),
+                    w_down.data_ptr(), hidden, ff, int(gated), kind, p0, p1, y.data_ptr(), rows.data_ptr(), self._stream(),
+                )
+            )
+            return rows
         max_tiles = self.lib.yk_moe_max_tiles(pairs, experts, tile_rows)
         ints = torch.empty(2 * pairs + 3 * max_tiles + 1, dtype=torch.int32, device=dev)
         order, slot_expert = ints[:pairs], ints[pairs: 2 * pairs]
@@ -2352,7 +2369,6 @@ class HipOps:
             self.lib.yk_moe_route(_ptr(token_ids), table.data_ptr(), vocab, top, experts, n, tile_rows, order.data_ptr(),
                                   slot_expert.data_ptr(), tiles.data_ptr(), n_tiles.data_ptr(), self._stream())
         )
-        bf = torch.bfloat16
         if (tile_rows == 128 and x.dtype == bf and w_gate_up.dtype == bf and w_down.dtype == bf and hidden % 8 == 0 and ff % 8 == 0
                 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0):
             # many pairs an expert: both products as tiles of 128 x 128 through LDS (the grouped form of
