@@ -26,9 +26,9 @@
 // for between the products, a few at a time as their registers come free (all together they hold a wave's products up: 119 and 102 us),
 // with one scalar base a chunk; asking two chunks ahead is no faster (132, 110: it is the loads' issue that costs, not their time).
 //
-// 2,048 tokens of one request in bfloat16, us (of which prepare; token by token: yk_linear_state_scan): 16 heads of 128 x 128, delta rule 135
-// (41; 465), with decays per channel 164 (69; 496); 4 of 256 x 512 gated 156 (61; 497); 32 of 64 x 64 with a bonus 84 (396); 32 of
-// 128 x 64 by step 112 (396).  Errors against float64, of their size, of the read-outs 1.1e-7, 1.1e-7, 2.5e-7, 0.7e-7, 0.8e-7 (walked
+// 2,048 tokens of one request in bfloat16, us (of which prepare; token by token: yk_linear_state_scan): 16 heads of 128 x 128, delta rule 120
+// (33; 465), with decays per channel 131 (496); 4 of 256 x 512 gated 121 (33; 497); 32 of 64 x 64 with a bonus 66 (396); 32 of
+// 128 x 64 by step 97 (396).  Errors against float64, of their size, of the read-outs 1.1e-7, 1.1e-7, 2.5e-7, 0.7e-7, 0.8e-7 (walked
 // 1.1e-7, 1.1e-7, 2.6e-7, 0.9e-7, 0.9e-7) and of the kept memories 0.8e-7, 0.8e-7, 2.4e-7, 0.4e-7, 0.6e-7 (0.8e-7, 0.8e-7, 2.6e-7, 0.4e-7, 0.6e-7).
 #include <algorithm>
 #include <type_traits>
@@ -121,11 +121,10 @@ __device__ __forceinline__ void load8(const bf16_t* p, float* out) {
   out[6] = __uint_as_float(w.w << 16); out[7] = __uint_as_float(w.w & 0xffff0000u);
 }
 
-__device__ __forceinline__ float softplus(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 // a decay per key channel from its biased logit: kinds 1, 2 and 3 of yk_linear_state_scan
 __device__ __forceinline__ float decay_of(float x, int mode, float tau, float rate) {
-  if (mode == 1) return expf(-softplus(-x) / tau);
-  if (mode == 2) return expf(-rate * softplus(x));
+  if (mode == 1) return expf(-softplus_f32(-x) / tau);
+  if (mode == 2) return expf(-rate * softplus_f32(x));
   return expf(-expf(x));
 }
 
@@ -176,10 +175,14 @@ __device__ __forceinline__ size_t part_of(int seq, int n_seqs, int q0, int c, in
 
 // ------------------------------------------------------------------------------------------- prepare
 constexpr int prepare_groups(int dim) { return dim > 128 ? 2 : 1; }
-// A workgroup a (chunk, request, head); with 256 key channels two groups of waves divide them (57 us against 98 where one took them in
-// turn, at 2,048 tokens of 4 heads).  64 key channels at a time: thread (channel, quarter) holds its channel of 16 tokens in registers
+// A workgroup a (chunk, request, head); with 256 key channels two groups of waves divide them.  64 key channels at a time: thread (channel, quarter) holds its channel of 16 tokens in registers
 // and makes the running products of decays there, doubling the blocks; the vectors of a block size go to LDS and meet on the
 // matrix cores, where a wave owns the diagonal tile of 16 x 16 of its quarter.
+// Bound by the issue of instructions (a wave of 128 channels with the delta rule some 7,000, two waves a SIMD) and the matrix cores' float64
+// (60 of 84 us in sum): hence two block sizes a product within 16 tokens, the diagonal without one, no meeting there, loads all asked
+// for at once, A's and B's triangles from opposite ends, and the logarithm of softplus_f32.  8 requests of 111 to 700 tokens, us: 16 heads of
+// 128 x 128, delta rule with decays per channel 138 -> 84; 32 of 64 x 64 with a bonus 80 -> 49; one of 2,048 tokens: 4 of 256 x 512 gated
+// 61 -> 33, 16 of 128 x 128 by the delta rule 40 -> 33.
 template <typename T, int D, int KIND>
 __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kernel(const T* __restrict__ qkv, const T* __restrict__ beta_rows, ChunkArgs g) {
   constexpr bool CH = KIND & kChannel, DELTA = KIND & kDelta, FIRST = KIND & kReadFirst;
@@ -188,7 +191,8 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
   using P = Part<D, KIND>;
   __shared__ __attribute__((aligned(16))) float ks_all[G][kTok * kRow], qs_all[G][kTok * kRow];  // later A and B
   __shared__ float dm[CH ? 1 : kTok * (kTok + 1)];                                               // a_(j+1) .. a_t where there is one decay a head
-  __shared__ float mul_k[kTok], mul_q[kTok], a_s[kTok], b_s[kTok], total_all[G][4][64];
+  __shared__ __attribute__((aligned(16))) float mul_k[kTok], mul_q[kTok];
+  __shared__ float a_s[kTok], b_s[kTok], total_all[G][4][64];
   const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / 256), tid = threadIdx.x % 256;
   float *ks = ks_all[group], *qs = qs_all[group];
   float(*total)[64] = total_all[group];
@@ -208,7 +212,7 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
       const size_t at = n0 + t;
       float step = 1.f;
       if (!CH) {
-        step = softplus(g.decay[at * g.decay_stride + g.decay_col + h] + g.decay_p1[h]);
+        step = softplus_f32(g.decay[at * g.decay_stride + g.decay_col + h] + g.decay_p1[h]);
         a = expf(-expf(g.decay_p0[h]) * step);
       }
       if (DELTA) b = 1.f / (1.f + expf(-(beta_rows != nullptr ? to_f32<T>(beta_rows[at * g.beta_stride + g.beta_col + h]) : g.beta[at * g.beta_stride + g.beta_col + h])));
@@ -257,25 +261,61 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
   const float dec_rate = CH && g.decay_mode == 2 ? expf(g.decay_p0[h]) : 1.f;
   const float* dec_bias = g.decay_mode == 2 ? g.decay_p1 : g.decay_p0;
 
-  f32x4_t diag_a = {}, diag_b = {}, mid = {}, far_a = {}, far_b = {};  // with decays per channel: tiles of A and B
-  f32x4_t low_a[4] = {}, low_b[4] = {};                                // without: the tiles (wave, 0 .. wave)
+  // with decays per channel: tiles of A and B (near: blocks of 1 and 2, of 4 and 8 within the wave's own diagonal tile), B's diagonal
+  f32x4_t near_a[2] = {}, near_b[2] = {}, mid = {}, far_a = {}, far_b = {};
+  float diag = 0.f;
+  f32x4_t low_a[4] = {}, low_b[4] = {};  // without: the tiles (wave, 0 .. wave) of B and, as many for all waves together, (3 - wave, 0 .. 3 - wave) of A
+  // a wave's own rows of LDS, which no other reads before the next meeting: written before this, read behind it
+  auto own_rows = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
 
   for (int cb = 64 * group; cb < D; cb += 64 * G) {
     float k[16], q[16];
     const int ch = cb + lane, tok0 = 16 * wave;
+    // All of them asked for before the first is used: each under its own condition t < n, as the compiler leaves a load whose value is
+    // wanted on one side only, was a wait for each (32 one after the other, two thirds of the kernel's time).
+    // Rows by steps from one base (sixteen bases of each kept from one turn to the next went to and from a vector register).
+    uint32_t kr[16], qr[16];
+    float z[CH ? 16 : 1], bias = 0.f;
+    {
+      const int first = min(tok0, n - 1);
+      const T *k_row = qkv + (n0 + first) * g.qkv_stride + kvh * D + g.k_col + cb, *q_row = k_row + (g.q_col - g.k_col);
+      const float* z_row = CH ? g.decay + (n0 + first) * g.decay_stride + g.decay_col + h * D + cb : nullptr;
+      int left = n - 1 - first;
+      asm volatile("" : "+s"(k_row), "+s"(q_row), "+s"(z_row), "+s"(left));
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        kr[x] = raw_bits(k_row[lane]);
+        qr[x] = raw_bits(q_row[lane]);
+        if (CH) z[x] = z_row[lane];
+        const int step = x < left ? g.qkv_stride : 0;
+        k_row += step;
+        q_row += step;
+        if (CH) z_row += x < left ? g.decay_stride : 0;
+      }
+    }
+    if (CH) bias = dec_bias[h * D + ch];
+    f32x4_t km[4], qm[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      km[x] = *reinterpret_cast<const f32x4_t*>(&mul_k[tok0 + 4 * x]);
+      qm[x] = *reinterpret_cast<const f32x4_t*>(&mul_q[tok0 + 4 * x]);
+    }
 #pragma unroll
     for (int x = 0; x < 16; ++x) {
-      const int t = tok0 + x;
-      const T* row = qkv + (n0 + min(t, n - 1)) * g.qkv_stride + kvh * D + ch;
-      const float kv = to_f32<T>(row[g.k_col]), qv = to_f32<T>(row[g.q_col]);
-      k[x] = t < n ? kv * mul_k[t] : 0.f;
-      q[x] = t < n ? qv * mul_q[t] : 0.f;
+      k[x] = from_raw<T>(kr[x]) * km[x / 4][x % 4];
+      q[x] = from_raw<T>(qr[x]) * qm[x / 4][x % 4];
+      asm volatile("" : "+v"(k[x]), "+v"(q[x]));
     }
-    float z[CH ? 16 : 1], bias = 0.f;
-    if (CH) {
-      bias = dec_bias[h * D + ch];
+    if (tok0 + 16 > n) {
 #pragma unroll
-      for (int x = 0; x < 16; ++x) z[x] = g.decay[(n0 + min(tok0 + x, n - 1)) * g.decay_stride + g.decay_col + h * D + ch];
+      for (int x = 0; x < 16; ++x) {
+        k[x] = tok0 + x < n ? k[x] : 0.f;
+        q[x] = tok0 + x < n ? q[x] : 0.f;
+      }
     }
     // operands of a tile product: rows of LDS, 16 bytes at 16 m + 4 lg
     auto tile = [&](const float* rows, const float* cols, int i, int j, f32x4_t acc) {
@@ -287,9 +327,7 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
     };
     // Q' and K' of these channels, from qs and ks: a wave's own 16 tokens
     auto write_rows = [&](int first) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      own_rows();
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const int row = (tok0 + r) * kRow + 16 * m + 4 * lg;
@@ -319,39 +357,100 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
       float a[16], pre[16], suf[16];
 #pragma unroll
       for (int x = 0; x < 16; ++x) qs[(tok0 + x) * kRow + lane] = z[x];  // (only this thread reads them)
+      auto decays = [&](int mode) {
 #pragma unroll 4
-      for (int x = 0; x < 16; ++x) {
-        float* at = qs + (tok0 + x) * kRow + lane;
-        *at = decay_of(*at + bias, g.decay_mode, g.tau, dec_rate);
-      }
+        for (int x = 0; x < 16; ++x) {
+          float* at = qs + (tok0 + x) * kRow + lane;
+          *at = decay_of(*at + bias, mode, g.tau, dec_rate);
+        }
+      };
+      if (g.decay_mode == 1) decays(1);
+      else if (g.decay_mode == 2) decays(2);
+      else decays(3);
 #pragma unroll
-      for (int x = 0; x < 16; ++x) a[x] = tok0 + x < n ? qs[(tok0 + x) * kRow + lane] : 1.f;  // (this thread's own writes)
-      __syncthreads();
-      // the diagonal itself
+      for (int x = 0; x < 16; ++x) a[x] = qs[(tok0 + x) * kRow + lane];  // (this thread's own writes)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) asm volatile("" : "+v"(a[x]));
+      if (tok0 + 16 > n) {
+#pragma unroll
+        for (int x = 0; x < 16; ++x) a[x] = tok0 + x < n ? a[x] : 1.f;
+      }
+      // the diagonal itself: lane (token, quarter of 16 channels)
 #pragma unroll
       for (int x = 0; x < 16; ++x) {
         qs[(tok0 + x) * kRow + lane] = q[x];
         ks[(tok0 + x) * kRow + lane] = FIRST ? k[x] * g.bonus[h * D + ch] : k[x];
       }
-      __syncthreads();
+      own_rows();
       {
-        const f32x4_t s = tile64(qs, ks, wave, wave, f32x4_t{0.f, 0.f, 0.f, 0.f});
+        double sum = 0.;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (4 * lg + i == r) diag_b[i] += s[i];
+        for (int m = 0; m < 4; ++m) {
+          const int row = (tok0 + r) * kRow + 16 * m + 4 * lg;
+          const f32x4_t x = *reinterpret_cast<const f32x4_t*>(&qs[row]), y = *reinterpret_cast<const f32x4_t*>(&ks[row]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum = fma(static_cast<double>(x[e]), static_cast<double>(y[e]), sum);
+        }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        diag += static_cast<float>(sum);
       }
 #pragma unroll
       for (int x = 0; x < 16; ++x) {
         pre[x] = FIRST ? 1.f : a[x];
         suf[x] = 1.f;
       }
-      float whole = 1.f;
+      auto twice = [&](int w) {  // blocks twice as long
 #pragma unroll
-      for (int level = 0; level < 6; ++level) {
-        const int w = 1 << level;  // block size
-        __syncthreads();           // the vectors before have been read
-        if (level == 4) total[wave][lane] = FIRST ? pre[15] * a[15] : pre[15];
-        if (level == 5) {
+        for (int x = 0; x < 16; ++x)
+          if ((x / w) % 2 == 1) {
+            const int last = x / (2 * w) * (2 * w) + w - 1;  // of the first half; its whole product
+            pre[x] *= FIRST ? pre[last] * a[last] : pre[last];
+          }
+#pragma unroll
+        for (int x = 0; x < 16; ++x)
+          if ((x / w) % 2 == 0) {
+            const int second = x / (2 * w) * (2 * w) + w;  // the second half's whole product
+            suf[x] *= a[second] * (w > 1 ? suf[second] : 1.f);
+          }
+      };
+      // within 16 tokens, where at each size eight are rows and eight columns: two sizes a product, and nobody to meet
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        float rows[16];  // of A
+        own_rows();
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int w = 1 << (2 * half + s);
+#pragma unroll
+          for (int x = 0; x < 16; ++x) {
+            const int place = 8 * s + x / (2 * w) * w + x % w;
+            if ((x / w) % 2 == 1) {
+              qs[(tok0 + place) * kRow + lane] = q[x] * pre[x];
+              rows[place] = DELTA ? k[x] * pre[x] : 0.f;
+            } else {
+              ks[(tok0 + place) * kRow + lane] = k[x] * suf[x];
+            }
+          }
+          twice(w);
+        }
+        own_rows();
+        near_b[half] = tile64(qs, ks, wave, wave, near_b[half]);
+        if (DELTA) {
+          own_rows();
+#pragma unroll
+          for (int x = 0; x < 16; ++x) qs[(tok0 + x) * kRow + lane] = rows[x];
+          own_rows();
+          near_a[half] += tile(qs, ks, wave, wave, f32x4_t{0.f, 0.f, 0.f, 0.f});
+        }
+      }
+      own_rows();
+#pragma unroll
+      for (int w = 16; w <= 32; w *= 2) {
+        if (w == 16) {
+          total[wave][lane] = FIRST ? pre[15] * a[15] : pre[15];
+        } else {
+          __syncthreads();  // the vectors before have been read
           if (wave == 0) {
             const float m = total[1][lane];
 #pragma unroll
@@ -362,40 +461,18 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
             for (int x = 0; x < 16; ++x) pre[x] *= m;
           }
         }
+        if ((wave / (w / 16)) % 2 == 1) {
 #pragma unroll
-        for (int x = 0; x < 16; ++x) {
-          const bool row = w >= 16 ? (wave / (w / 16)) % 2 == 1 : (x / w) % 2 == 1;
-          if (!row || DELTA) ks[(tok0 + x) * kRow + lane] = k[x] * (row ? pre[x] : suf[x]);
-          if (row) qs[(tok0 + x) * kRow + lane] = q[x] * pre[x];
+          for (int x = 0; x < 16; ++x) {
+            if (DELTA) ks[(tok0 + x) * kRow + lane] = k[x] * pre[x];
+            qs[(tok0 + x) * kRow + lane] = q[x] * pre[x];
+          }
+        } else {
+#pragma unroll
+          for (int x = 0; x < 16; ++x) ks[(tok0 + x) * kRow + lane] = k[x] * suf[x];
         }
         __syncthreads();
-        if (w < 16) {
-          const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-          const f32x4_t sb = tile64(qs, ks, wave, wave, zero);
-          const f32x4_t sa = DELTA ? tile(ks, ks, wave, wave, zero) : zero;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int t = 4 * lg + i;
-            const bool here = (t / w) % 2 == 1 && r / w == t / w - 1;
-            diag_b[i] += here ? sb[i] : 0.f;
-            if (DELTA) diag_a[i] += here ? sa[i] : 0.f;
-          }
-          // blocks twice as long
-#pragma unroll
-          for (int x = 0; x < 16; ++x) {
-            const int start = x / (2 * w) * (2 * w);
-            const bool second = (x / w) % 2 == 1;
-            if (second) {
-              const int last = start + w - 1;  // of the first half; its whole product
-              pre[x] *= FIRST ? pre[last] * a[last] : pre[last];
-            }
-          }
-#pragma unroll
-          for (int x = 0; x < 16; ++x) {
-            const int start = x / (2 * w) * (2 * w);
-            if ((x / w) % 2 == 0) suf[x] *= a[start + w] * (w > 1 ? suf[start + w] : 1.f);  // the second half's whole product
-          }
-        } else if (w == 16) {
+        if (w == 16) {
           // tiles (1, 0) and (3, 2): of A by waves 0 and 1, of B by waves 2 and 3
           const int i = wave % 2 * 2 + 1;
           if (wave >= 2) mid = tile64(qs, ks, i, i - 1, mid);
@@ -408,7 +485,7 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
       }
       // the chunk's own products: undo nothing, the quarters' wholes join what a quarter's tokens have
       const float t0 = total[0][lane], t1 = total[1][lane], t2 = total[2][lane], t3 = total[3][lane];
-      whole = ((t0 * t1) * t2) * t3;
+      const float whole = ((t0 * t1) * t2) * t3;
       const float before = wave == 0 ? 1.f : wave == 1 ? t0 : t0 * t1;              // (wave 3's pre holds t2 already)
       const float after = wave == 3 ? 1.f : wave == 2 ? t3 : wave == 1 ? t2 * t3 : t2 * t3;  // (wave 0's suf holds t1 already)
       __syncthreads();
@@ -425,7 +502,7 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
       }
       if (wave == 0) part[P::DEC + ch] = whole;
     } else {
-      if (cb >= 64 * G) __syncthreads();
+      own_rows();
 #pragma unroll
       for (int x = 0; x < 16; ++x) {
         qs[(tok0 + x) * kRow + lane] = q[x];
@@ -434,10 +511,10 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (j <= wave) {
-          low_b[j] = tile64(qs, ks, wave, j, low_b[j]);
-          if (DELTA) low_a[j] = tile(ks, ks, wave, j, low_a[j]);
-        }
+        if (j <= wave) low_b[j] = tile64(qs, ks, wave, j, low_b[j]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (DELTA && j <= 3 - wave) low_a[j] = tile(ks, ks, 3 - wave, j, low_a[j]);
       __syncthreads();
 #pragma unroll
       for (int x = 0; x < 16; ++x) {
@@ -468,8 +545,19 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
     }
   };
   if (CH) {
-    put(qs, wave, wave, diag_b, true);
-    if (DELTA) put(ks, wave, wave, diag_a, false);
+    const int tok16 = 16 * wave;
+    if (lg == 0) qs[(tok16 + r) * kRow + tok16 + r] = diag;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {  // place 4 lg + e of the rows, r of the columns (see above)
+        const int size = 2 * half + (r >= 8), w = 1 << size, row = (4 * lg + e) % 8, col = r % 8;
+        const int at = (tok16 + (row >> size << (size + 1)) + w + row % w) * kRow + tok16 + (col >> size << (size + 1)) + col % w;
+        if ((4 * lg + e >= 8) == (r >= 8) && row >> size == col >> size) {
+          qs[at] = near_b[half][e];
+          if (DELTA) ks[at] = near_a[half][e];
+        }
+      }
     const int i = wave % 2 * 2 + 1;
     if (wave >= 2) put(qs, i, i - 1, mid, true);
     else if (DELTA) put(ks, i, i - 1, mid, false);
@@ -486,10 +574,18 @@ __global__ __launch_bounds__(256 * prepare_groups(D), 2) void chunk_prepare_kern
           const float d = at <= t ? dm[t * (kTok + 1) + at] : 0.f;
           low_b[j][e] *= DELTA ? d : d * b_s[at];
           if (at == t && group == 0) low_b[j][e] += skip;
-          low_a[j][e] *= d;
         }
         put(qs, wave, j, low_b[j], true);
-        if (DELTA) put(ks, wave, j, low_a[j], false);
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (DELTA && j <= 3 - wave) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int t = 16 * (3 - wave) + 4 * lg + e, at = 16 * j + r;
+          low_a[j][e] *= at <= t ? dm[t * (kTok + 1) + at] : 0.f;
+        }
+        put(ks, 3 - wave, j, low_a[j], false);
       }
   }
   __syncthreads();

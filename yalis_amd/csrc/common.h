@@ -47,6 +47,16 @@ __device__ __forceinline__ float column_lanes_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// max(x, 0) + log1p(u), u = e^-|x|.  log1p(u) is 2 atanh(u / (2 + u)): the quotient with its remainder, the series' tail fitted over
+// its range (to 1e-10 of the sum).  Against 64 bits, four million normal x of deviation 4: largest error 1.17e-7 of the result as with
+// log1pf, mean 2.54e-8 (2.55e-8), in some 35 instructions where that took 120, one after the other.
+__device__ __forceinline__ float softplus_f32(float x) {
+  const float u = expf(-fabsf(x)), w = 2.f + u, left = u - (w - 2.f), inverse = __builtin_amdgcn_rcpf(w);
+  const float q = u * inverse, z = q * q, rest = fmaf(-q, left, fmaf(-q, w, u)) * inverse;
+  const float tail = fmaf(z, fmaf(z, fmaf(z, fmaf(z, 0.121287405f, 0.107200928f), 0.143078059f), 0.199994653f), 0.333333373f);
+  return fmaf(2.f, q + fmaf(q * z, tail, rest), fmaxf(x, 0.f));
+}
+
 // two floats to two bfloat16 (round to nearest even; NaN stays NaN) in one word: gfx950
 // converts in hardware (v_cvt_pk_bf16_f32), one instruction where the shifts and adds of a
 // conversion by hand take six (measured: 2 us of a 41 us product that converted its staged rows)

@@ -173,7 +173,6 @@ extern "C" int yk_causal_conv(const void* x, int x_stride, int dtype, const void
 // --------------------------------------------------------------------------------- gates
 constexpr int kGateTokens = 16;  // tokens a workgroup takes through one block's two matrices
 
-__device__ __forceinline__ float softplus_f32(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 
 // Weights come transposed, [block][in][out], so that the threads of a workgroup (one per output
 // channel of the block) read consecutive addresses at every step of the sum.

@@ -34,12 +34,11 @@
 constexpr int kScanRowsMax = 16;  // rows of S a lane holds at the most (template R: 8 or 16): sub * R .. sub * R + R - 1 of its column
 constexpr int kScanTokens = 32;  // tokens staged at a time (fewer where LDS would not hold them)
 
-__device__ __forceinline__ float scan_softplus(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 
 // a decay per key channel from its biased logit x: kinds 1, 2 and 3 of yk_linear_state_scan
 __device__ __forceinline__ float channel_decay(float x, int mode, float tau, float rate) {
-  if (mode == 1) return expf(-scan_softplus(-x) / tau);
-  if (mode == 2) return expf(-rate * scan_softplus(x));
+  if (mode == 1) return expf(-softplus_f32(-x) / tau);
+  if (mode == 2) return expf(-rate * softplus_f32(x));
   return expf(-expf(x));
 }
 
@@ -191,7 +190,7 @@ __global__ __launch_bounds__(256) void linear_state_scan_kernel(
     }
     for (int t = threadIdx.x; t < nt; t += blockDim.x) {
       const size_t n = static_cast<size_t>(q0 + t0 + t);
-      const float step = decay_mode == 0 ? scan_softplus(decay[n * decay_stride + decay_col + h] + decay_p1[h]) : 1.f;
+      const float step = decay_mode == 0 ? softplus_f32(decay[n * decay_stride + decay_col + h] + decay_p1[h]) : 1.f;
       if (decay_mode == 0) as[t] = expf(-expf(decay_p0[h]) * step);
       if (decay_mode == 4) as[t] = decay_p0[h];
       float b = write_mode == 2 ? step : 1.f;
@@ -461,7 +460,7 @@ __global__ __launch_bounds__(256) void linear_state_scan_fast_kernel(const T* __
         if (i < nt * COLS) vs[i] = to_f32<T>(vv[j]);
       }
       if (threadIdx.x < nt) {
-        const float step = CH || g.decay_mode != 0 ? 1.f : scan_softplus(s_dec + g.decay_p1[h]);
+        const float step = CH || g.decay_mode != 0 ? 1.f : softplus_f32(s_dec + g.decay_p1[h]);
         if (!CH) sc[4 * threadIdx.x] = g.decay_mode == 4 ? g.decay_p0[h] : expf(-expf(g.decay_p0[h]) * step);
         sc[4 * threadIdx.x + 1] = DELTA ? 1.f / (1.f + expf(-s_beta)) : (g.by_step ? step : 1.f);
       }
@@ -629,7 +628,7 @@ __global__ __launch_bounds__(256) void linear_state_token_kernel(const T* __rest
     if (lane == 0) sums[wave][0] = wave_q, sums[wave][1] = wave_k, sums[wave][2] = wave_w;
     float a = 1.f, strength = 1.f;
     if (!CH) {
-      const float step = g.decay_mode == 0 ? scan_softplus(g.decay[n * g.decay_stride + g.decay_col + h] + g.decay_p1[h]) : 1.f;
+      const float step = g.decay_mode == 0 ? softplus_f32(g.decay[n * g.decay_stride + g.decay_col + h] + g.decay_p1[h]) : 1.f;
       a = g.decay_mode == 4 ? g.decay_p0[h] : expf(-expf(g.decay_p0[h]) * step);
       if (g.by_step) strength = step;
     }
