@@ -235,3 +235,61 @@ def test_experts_of_few_pairs(n, top, experts, hidden, ff):
         bad[0] = float("nan")
         got2 = o.moe_experts(bad, *dev[1:], act).cpu()
         assert torch.equal(got2[top:], got[top:])  # (its own rows: the pair's clamps drop a NaN)
+
+
+def _spans(spans, slots):
+    from types import SimpleNamespace
+
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    starts = [sum(spans[:i]) for i in range(len(spans))]
+    return SimpleNamespace(max_qlen=max(spans), arrays={"seq_qstart": dev(starts), "seq_qlen": dev(spans), "state_slots": dev(slots),
+                                                        "token_seq": dev([i for i, s in enumerate(spans) for _ in range(s)])})
+
+
+@pytest.mark.parametrize("dtype,w_dtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("spans", [[1], [1] * 9, [1] * 64, [2, 1, 5, 3], [1] * 65])
+@pytest.mark.parametrize("channels,bias,act", [(8, True, None), (128, False, "silu"), (136, True, "silu"), (1160, True, None)])
+def test_convolution_of_few_tokens(dtype, w_dtype, spans, channels, bias, act):
+    """Two channels a thread against the sum in float64 (rounded once: 2^-8 of the largest in bfloat16, four products in float32), the state moved."""
+    o, g = ops(), torch.Generator().manual_seed(channels + len(spans))
+    n, slots = sum(spans), [len(spans) - i for i in range(len(spans))]
+    x, w = torch.randn(n, channels + 8, generator=g).to(dtype)[:, :channels], torch.randn(channels, 4, generator=g).to(w_dtype)
+    b = torch.randn(channels, generator=g).to(w_dtype) if bias else None
+    state = torch.randn(len(spans) + 1, 3, channels, generator=g).to(dtype)
+    want, kept, first = [], state.clone(), 0
+    for slot, s in zip(slots, spans):
+        rows = torch.cat([state[slot], x[first: first + s]])
+        want += [sum(w[:, j].double() * rows[t + j].double() for j in range(4)) + (b.double() if bias else 0) for t in range(s)]
+        kept[slot], first = rows[-3:], first + s
+    want = torch.stack(want)
+    want = torch.nn.functional.silu(want) if act else want
+    st = state.cuda()
+    wide = torch.zeros(n, channels + 8, dtype=dtype, device="cuda")
+    wide[:, :channels] = x.cuda()
+    got = o.causal_conv(wide[:, :channels], w.cuda(), b.cuda() if bias else None, st, _spans(spans, slots), act=act, move_state=True)
+    close(got, want, 2.0 ** -8 if dtype == torch.bfloat16 else 1e-6)
+    assert torch.equal(st.cpu(), kept)
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 8, 9, 16, 17, 64])
+@pytest.mark.parametrize("blocks,size", [(3, 32), (2, 160), (1, 256), (2, 288)])  # fewer steps of 32 than are asked for ahead, all, more
+def test_gated_recurrence_of_few_tokens(n, blocks, size):
+    """Single tokens against float64 from the same bfloat16 numbers: the products are summed in float32 (size roundings of 2^-24), the
+    states then within 2e-5, the outputs rounded to bfloat16; the kept inputs exactly."""
+    o, g, c = ops(), torch.Generator().manual_seed(n + size), blocks * size
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    u, y, x, ba, bi, lam = r(n, c), r(n, c), r(n, c), r(c), r(c), r(c)
+    wa, wi = ((torch.randn(blocks, size, size, generator=g) / size ** 0.5).bfloat16() for _ in range(2))
+    S, kept = torch.randn(n + 1, c, generator=g), r(n + 1, 3, c)
+    slots = list(range(n, 0, -1))
+    product = lambda m, b: torch.einsum("nbk,bok->nbo", u.double().view(n, blocks, size), m.double()).reshape(n, c) + b.double()
+    log_a = -8.0 * torch.nn.functional.softplus(lam.double()) * torch.sigmoid(product(wa, ba))
+    want_S, want_kept = S.double(), kept.clone()
+    want_S[slots] = torch.exp(log_a) * S.double()[slots] + torch.sqrt(-torch.expm1(2 * log_a)) * torch.sigmoid(product(wi, bi)) * u.double()
+    want_kept[slots] = torch.cat([kept[slots][:, 1:], x[:, None]], 1)
+    Sd, kd = S.cuda(), kept.cuda()
+    t = lambda m: m.transpose(1, 2).contiguous().cuda()
+    got = o.rglru(u.cuda(), y.cuda(), x.cuda(), t(wa), ba.cuda(), t(wi), bi.cuda(), lam.cuda(), 8.0, Sd, kd, 4, _spans([1] * n, slots), wa=wa.cuda(), wi=wi.cuda())
+    close(Sd, want_S, 2e-5)
+    close(got, want_S[slots] * torch.nn.functional.gelu(y.double(), approximate="tanh"), 2.0 ** -8)
+    assert torch.equal(kd.cpu(), want_kept)

@@ -128,6 +128,70 @@ __global__ __launch_bounds__(256) void causal_conv_vec_kernel(const T* __restric
   }
 }
 
+// The same for few tokens and four taps: a thread takes two channels of one token, whose weights are one piece (float32: two) and whose
+// activations are two and not eight one after the other; everything is asked for before the first use, where a load under a condition of
+// its own was a wait of its own.  What a pushed token leaves in the state are the rows that it has read.  One token each of eight
+// requests, us in a replayed step: 2,560 to 8,192 channels 3.2 -> 2.4, with a bias 3.6 -> 2.4.
+template <typename T>
+__device__ __forceinline__ void conv_two(const T* p, uint32_t* raw) {
+  if constexpr (sizeof(T) == 2) {
+    raw[0] = *reinterpret_cast<const uint32_t*>(p);
+  } else {
+    const uint2 x = *reinterpret_cast<const uint2*>(p);
+    raw[0] = x.x, raw[1] = x.y;
+  }
+}
+template <typename T>
+__device__ __forceinline__ float conv_of(const uint32_t* raw, int e) {
+  if constexpr (sizeof(T) == 2) return __uint_as_float(e % 2 ? raw[e / 2] & 0xffff0000u : raw[e / 2] << 16);
+  return __uint_as_float(raw[e]);
+}
+
+template <typename T, typename TW>
+__global__ __launch_bounds__(64) void causal_conv_few_kernel(const T* __restrict__ x, int x_stride, const TW* __restrict__ w,
+                                                             const TW* __restrict__ bias, T* state, const int32_t* __restrict__ token_seq,
+                                                             const int32_t* __restrict__ seq_qstart, const int32_t* __restrict__ state_slots,
+                                                             T* __restrict__ out, int channels, int act, int push) {
+  constexpr int R = sizeof(T) / 2, RW = sizeof(TW) / 2;  // 32-bit pieces of two elements
+  const int n = blockIdx.y, c = 2 * (blockIdx.x * 64 + threadIdx.x), at = min(c, channels - 2);
+  const int seq = token_seq[n];
+  uint32_t wr[4 * RW], br[RW] = {}, v[4][R];
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    const uint4 p = reinterpret_cast<const uint4*>(w + static_cast<size_t>(at) * 4)[i];
+    wr[4 * i] = p.x, wr[4 * i + 1] = p.y, wr[4 * i + 2] = p.z, wr[4 * i + 3] = p.w;
+  }
+  if (bias != nullptr) conv_two<TW>(bias + at, br);
+  const int t = n - seq_qstart[seq];  // the token's place in its span
+  T* hist = state + static_cast<size_t>(state_slots[seq]) * 3 * channels + at;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int back = 3 - j;  // (see causal_conv_vec_kernel)
+    conv_two<T>(t >= back ? x + static_cast<size_t>(n - back) * x_stride + at : hist + static_cast<size_t>(3 + t - back) * channels, v[j]);
+  }
+  float acc[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    acc[e] = conv_of<TW>(br, e);  // (zero bits where there is no bias)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[e] = fmaf(conv_of<TW>(wr, 4 * e + j), conv_of<T>(v[j], e), acc[e]);
+    if (act == 1) acc[e] = act_silu(acc[e]);
+  }
+  if (c >= channels) return;
+  T* o = out + static_cast<size_t>(n) * channels + c;
+  if constexpr (sizeof(T) == 2) {
+    *reinterpret_cast<uint32_t*>(o) = pack_bf16x2(acc[0], acc[1]);
+  } else {
+    *reinterpret_cast<float2*>(o) = make_float2(acc[0], acc[1]);
+  }
+  if (push) {  // (spans of one token: the rows read are the state's three and the input)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int i = 0; i < R; ++i) reinterpret_cast<uint32_t*>(hist + static_cast<size_t>(j) * channels)[i] = v[j + 1][i];
+  }
+}
+
 // act: 0 none, 1 silu on the convolution's output.  push != 0 (steps whose spans are single tokens only): the state takes
 // in the token's input in the same pass.
 extern "C" int yk_causal_conv(const void* x, int x_stride, int dtype, const void* w, const void* bias, int w_dtype,
@@ -148,7 +212,14 @@ extern "C" int yk_causal_conv(const void* x, int x_stride, int dtype, const void
   // (few tokens: one each, in workgroups of a wave)
   const int threads = n_tokens <= 64 ? 64 : 256, each = n_tokens <= 64 ? 1 : kConvTokens;
   const dim3 vgrid((channels / piece + threads - 1) / threads, (n_tokens + each - 1) / each);
+  const bool few = vec && taps == 4 && n_tokens <= 64 && al16(w) && reinterpret_cast<uintptr_t>(bias) % 8 == 0;
 #define YK_CASE(D, T, WD, TW)                                                                                   \
+  if (dtype == D && w_dtype == WD && few) {                                                                      \
+    causal_conv_few_kernel<T, TW><<<dim3((channels / 2 + 63) / 64, n_tokens), 64, 0, stream>>>(                  \
+        static_cast<const T*>(x), x_stride, static_cast<const TW*>(w), static_cast<const TW*>(bias), static_cast<T*>(state), token_seq, \
+        seq_qstart, state_slots, static_cast<T*>(out), channels, act, push);                                     \
+    return yk_check_launch("causal_conv");                                                                       \
+  }                                                                                                              \
   if (dtype == D && w_dtype == WD && vec) {                                                                      \
     auto kern = taps == 4 ? causal_conv_vec_kernel<T, TW, 4> : causal_conv_vec_kernel<T, TW, 0>;                 \
     kern<<<vgrid, threads, 0, stream>>>(static_cast<const T*>(x), x_stride, static_cast<const TW*>(w), static_cast<const TW*>(bias), \
@@ -228,8 +299,11 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(
 // of 32 channels: the products u_b . Ra[b]^T and u_b . Ri[b]^T are bfloat16 x bfloat16 with float32
 // accumulation (every product of two bfloat16 numbers is exact in float32, so only the order of
 // the sum differs from the kernel above); sigmoids, decays and roots are float32 as there.
-// A wave owns 16 output channels of a block and 64 tokens; the weights come in the checkpoint's
-// own layout [block][out][in], whose rows are the A operand as they lie.
+// A wave owns 16 output channels of a block and 64 tokens (few: 16); the weights come in the checkpoint's
+// own layout [block][out][in], whose rows are the A operand as they lie.  Few tokens are bound by a wave's own chain: all of the
+// weights' rows (up to 256 channels) and what the end reads are asked for at once, and of up to 4 (8) tokens each lane finishes one (two)
+// of the numbers that the products leave four of in a quarter (half) of the lanes.  Four tokens, 10 blocks of 256, us in a replayed step:
+// 6.5 -> 4.4 (8 tokens 6.7 -> 4.9, 16 7.1 -> 5.8; 17 and more go as 64 do).
 typedef __bf16 rg_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float rg_f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t rg_u32x4_t __attribute__((ext_vector_type(4)));
@@ -238,11 +312,22 @@ union RgFrag {
   rg_bf16x8_t v;
 };
 
+__device__ __forceinline__ void rglru_gate(float ra, float ri, float decay, float u, float& a, float& b) {
+  const float rg = 1.f / (1.f + expf(-ra));
+  const float ig = 1.f / (1.f + expf(-ri));
+  const float log_a = -decay * rg;
+  a = expf(log_a);
+  b = sqrtf(fmaxf(-expm1f(2.f * log_a), 0.f)) * ig * u;
+}
+
+// MT: tiles of 16 tokens a wave; E: the numbers a lane finishes of each (4, or less where 4 E tokens are all there are)
+template <int MT, int E>
 __global__ __launch_bounds__(256) void rglru_gates_mfma_kernel(
     const bf16_t* __restrict__ u, const bf16_t* __restrict__ wa, const bf16_t* __restrict__ ba,
     const bf16_t* __restrict__ wi, const bf16_t* __restrict__ bi, const bf16_t* __restrict__ lam, float rate,
     float* __restrict__ a_out, float* __restrict__ b_out, int n_tokens, int channels, int block_size) {
-  constexpr int MT = 4;
+  static_assert(E == 4 || MT == 1, "few tokens are one tile");
+  constexpr int AHEAD = MT == 1 ? 8 : 1;  // steps of 32 channels asked for at once
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, r = lane % 16, g = lane / 16;
   const int n0 = blockIdx.x * 16 * MT, b = blockIdx.y;
   const int o0 = (blockIdx.z * 4 + wave) * 16;  // first output channel of the wave within the block
@@ -257,45 +342,73 @@ __global__ __launch_bounds__(256) void rglru_gates_mfma_kernel(
   rg_f32x4_t acc_a[MT], acc_i[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc_a[m] = acc_i[m] = rg_f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < block_size; k0 += 32) {
-    RgFrag fa, fi, fu[MT];
-    fa.u = *reinterpret_cast<const rg_u32x4_t*>(wa_row + k0);
-    fi.u = *reinterpret_cast<const rg_u32x4_t*>(wi_row + k0);
+  // lane (r, g) will hold, for token 16m + r, the channels o0 + 4g .. 4g + 3; with E < 4 it takes channels 4g + E (r / 4E) .. of token r % 4E
+  constexpr int TOK = 4 * E;
+  const int tok = r % TOK, first = E == 4 ? 0 : E * (r / TOK);
+  const int c0 = b * block_size + o0 + 4 * g + first;
+  uint32_t ends[3][E], ue[MT][E];  // what the end reads, as it lies in memory
 #pragma unroll
-    for (int m = 0; m < MT; ++m) fu[m].u = *reinterpret_cast<const rg_u32x4_t*>(ur[m] + k0);
+  for (int i = 0; i < E; ++i) {
+    ends[0][i] = ba[c0 + i], ends[1][i] = bi[c0 + i], ends[2][i] = lam[c0 + i];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      acc_a[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa.v, fu[m].v, acc_a[m], 0, 0, 0);
-      acc_i[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fi.v, fu[m].v, acc_i[m], 0, 0, 0);
+    for (int m = 0; m < MT; ++m) ue[m][i] = u[static_cast<size_t>(min(n0 + 16 * m + tok, n_tokens - 1)) * channels + c0 + i];
+  }
+  for (int k0 = 0; k0 < block_size; k0 += 32 * AHEAD) {
+    RgFrag fa[AHEAD], fi[AHEAD], fu[AHEAD][MT];
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) {
+      const int k = min(k0 + 32 * s, block_size - 32);  // (steps past the last read it again, unused)
+      fa[s].u = *reinterpret_cast<const rg_u32x4_t*>(wa_row + k);
+      fi[s].u = *reinterpret_cast<const rg_u32x4_t*>(wi_row + k);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) fu[s][m].u = *reinterpret_cast<const rg_u32x4_t*>(ur[m] + k);
+    }
+    if (AHEAD > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) {
+      if (AHEAD > 1) asm volatile("" ::"v"(fa[s].u), "v"(fi[s].u), "v"(fu[s][0].u));  // (or the loads go under the condition, and wait there)
+      if (s == 0 || k0 + 32 * s < block_size) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          acc_a[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[s].v, fu[s][m].v, acc_a[m], 0, 0, 0);
+          acc_i[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fi[s].v, fu[s][m].v, acc_i[m], 0, 0, 0);
+        }
+      }
     }
   }
-  // lane (r, g) holds, for token 16m + r, the channels o0 + 4g .. 4g + 3
-  const int c0 = b * block_size + o0 + 4 * g;
-  float bav[4], biv[4], decay[4];
+  if (E < 4) {
+    float ta[E] = {}, ti[E] = {};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    bav[i] = bf16_to_f32(ba[c0 + i]);
-    biv[i] = bf16_to_f32(bi[c0 + i]);
-    decay[i] = rate * softplus_f32(bf16_to_f32(lam[c0 + i]));
+    for (int i = 0; i < 4; ++i) {
+      const float xa = __shfl(acc_a[0][i], tok + 16 * g, 64), xi = __shfl(acc_i[0][i], tok + 16 * g, 64);
+      if (i - i % E == first) ta[i % E] = xa, ti[i % E] = xi;
+    }
+#pragma unroll
+    for (int i = 0; i < E; ++i) acc_a[0][i] = ta[i], acc_i[0][i] = ti[i];
+  }
+  float bav[E], biv[E], decay[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    if (MT == 1) asm volatile("" ::"v"(ends[0][i]), "v"(ends[1][i]), "v"(ends[2][i]), "v"(ue[0][i]));
+    bav[i] = __uint_as_float(ends[0][i] << 16);
+    biv[i] = __uint_as_float(ends[1][i] << 16);
+    decay[i] = rate * softplus_f32(__uint_as_float(ends[2][i] << 16));
   }
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    const int n = n0 + 16 * m + r;
+    const int n = n0 + 16 * m + tok;
     if (n >= n_tokens) continue;
-    const uint2 uw = *reinterpret_cast<const uint2*>(u + static_cast<size_t>(n) * channels + c0);
-    const float uv[4] = {__uint_as_float(uw.x << 16), __uint_as_float(uw.x & 0xffff0000u), __uint_as_float(uw.y << 16),
-                         __uint_as_float(uw.y & 0xffff0000u)};
-    float av[4], bv[4];
+    const size_t at = static_cast<size_t>(n) * channels + c0;
+    float av[E], bv[E];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float rg = 1.f / (1.f + expf(-(acc_a[m][i] + bav[i])));
-      const float ig = 1.f / (1.f + expf(-(acc_i[m][i] + biv[i])));
-      const float log_a = -decay[i] * rg;
-      av[i] = expf(log_a);
-      bv[i] = sqrtf(fmaxf(-expm1f(2.f * log_a), 0.f)) * ig * uv[i];
+    for (int i = 0; i < E; ++i) rglru_gate(acc_a[m][i] + bav[i], acc_i[m][i] + biv[i], decay[i], __uint_as_float(ue[m][i] << 16), av[i], bv[i]);
+    if constexpr (E == 4) {
+      *reinterpret_cast<float4*>(a_out + at) = make_float4(av[0], av[1], av[2], av[3]);
+      *reinterpret_cast<float4*>(b_out + at) = make_float4(bv[0], bv[1], bv[2], bv[3]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < E; ++i) a_out[at + i] = av[i], b_out[at + i] = bv[i];
     }
-    *reinterpret_cast<float4*>(a_out + static_cast<size_t>(n) * channels + c0) = make_float4(av[0], av[1], av[2], av[3]);
-    *reinterpret_cast<float4*>(b_out + static_cast<size_t>(n) * channels + c0) = make_float4(bv[0], bv[1], bv[2], bv[3]);
   }
 }
 
@@ -316,9 +429,12 @@ extern "C" int yk_rglru_gates(const void* u, int dtype, const void* wa_t, const 
       reinterpret_cast<uintptr_t>(u) % 16 == 0 && reinterpret_cast<uintptr_t>(wa) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(wi) % 16 == 0 && reinterpret_cast<uintptr_t>(a_out) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(b_out) % 16 == 0) {
-    dim3 mgrid((n_tokens + 63) / 64, blocks, (block_size + 63) / 64);
+    const int tokens = n_tokens <= 16 ? 16 : 64;
+    dim3 mgrid((n_tokens + tokens - 1) / tokens, blocks, (block_size + 63) / 64);
     YK_REQUIRE(mgrid.z <= 65535, "rglru_gates: blocks too wide for one launch");
-    rglru_gates_mfma_kernel<<<mgrid, 256, 0, stream>>>(
+    auto kern = n_tokens <= 4 ? rglru_gates_mfma_kernel<1, 1> : n_tokens <= 8 ? rglru_gates_mfma_kernel<1, 2> :
+                n_tokens <= 16 ? rglru_gates_mfma_kernel<1, 4> : rglru_gates_mfma_kernel<4, 4>;
+    kern<<<mgrid, 256, 0, stream>>>(
         static_cast<const bf16_t*>(u), static_cast<const bf16_t*>(wa), static_cast<const bf16_t*>(ba),
         static_cast<const bf16_t*>(wi), static_cast<const bf16_t*>(bi), static_cast<const bf16_t*>(lam), rate, a_out, b_out,
         n_tokens, channels, block_size);
@@ -364,23 +480,30 @@ __global__ void rglru_scan_kernel(const float* __restrict__ a, const float* __re
   if (c >= channels) return;
   const int q0 = seq_qstart[seq], ql = seq_qlen[seq], slot = state_slots[seq];
   float S = s_state[static_cast<size_t>(slot) * channels + c];
+  // the convolution's last inputs as they will be, oldest first: what is left of the old ones, then the span's.  Three of them (four taps)
+  // are asked for here, beside what the walk waits for; one after the other behind it they cost as much again.
+  const int keep = taps - 1;
+  T* hist = conv_state + static_cast<size_t>(slot) * keep * channels + c;
+  auto kept = [&](int i) { return i + ql < keep ? hist + static_cast<size_t>(i + ql) * channels : x + static_cast<size_t>(q0 + i + ql - keep) * x_stride + c; };
+  T next[3];
+  if (keep == 3) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) next[i] = *kept(i);
+  }
   for (int t = 0; t < ql; ++t) {
     const size_t idx = static_cast<size_t>(q0 + t) * channels + c;
-    S = fmaf(a[idx], S, b[idx]);
-    const float yv = to_f32<T>(y[static_cast<size_t>(q0 + t) * y_stride + c]);
-    out[idx] = from_f32<T>(S * act_gelu_tanh(yv));
+    const float at = a[idx], bt = b[idx];
+    const T yt = y[static_cast<size_t>(q0 + t) * y_stride + c];
+    __builtin_amdgcn_sched_barrier(0);  // (all three asked for before the first is waited for)
+    S = fmaf(at, S, bt);
+    out[idx] = from_f32<T>(S * act_gelu_tanh(to_f32<T>(yt)));
   }
   s_state[static_cast<size_t>(slot) * channels + c] = S;
-  // the convolution's last taps - 1 inputs, oldest first: what is left of the old ones, then the span's
-  const int keep = taps - 1;
-  if (keep > 0) {
-    T* hist = conv_state + static_cast<size_t>(slot) * keep * channels;
-    if (ql >= keep) {
-      for (int i = 0; i < keep; ++i) hist[static_cast<size_t>(i) * channels + c] = x[static_cast<size_t>(q0 + ql - keep + i) * x_stride + c];
-    } else {
-      for (int i = 0; i < keep - ql; ++i) hist[static_cast<size_t>(i) * channels + c] = hist[static_cast<size_t>(i + ql) * channels + c];
-      for (int i = 0; i < ql; ++i) hist[static_cast<size_t>(keep - ql + i) * channels + c] = x[static_cast<size_t>(q0 + i) * x_stride + c];
-    }
+  if (keep == 3) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) hist[static_cast<size_t>(i) * channels] = next[i];
+  } else {  // (ascending: a row is read before it is overwritten)
+    for (int i = 0; i < keep; ++i) hist[static_cast<size_t>(i) * channels] = *kept(i);
   }
 }
 

@@ -28,6 +28,7 @@
 // weight shared by the heads, times silu or the sigmoid of a gate column), and the shift of a convolution's kept
 // inputs by a span.
 #include <algorithm>
+#include <climits>
 
 #include "common.h"
 
@@ -356,6 +357,8 @@ struct ScanArgs {
   int beta_stride, beta_col, by_step;
   const float *skip, *bonus;
   int chunk;
+  int per_kv;  // heads that share a kv head, and what to divide by it with (linear_state_token_kernel)
+  uint32_t per_kv_inverse;
 };
 
 template <typename T, int TPC, int ROWS, int KIND>
@@ -576,18 +579,30 @@ __global__ __launch_bounds__(256) void linear_state_scan_fast_kernel(const T* __
 
 // Steps of single tokens: all state traffic and no walk.  A workgroup takes 64 columns of a (request, head)'s S, thread (row group, four
 // columns) every sixteenth row of them 16 bytes at a time, so a wave reads rows in pieces of 256 bytes (a column a group of
-// lanes, as above, reads them in pieces of 16 to 64); all of S is asked for before the token's inputs are, and both sums over
-// the decayed S meet once, in registers and then over the four waves in LDS.  Longer spans stay right: a token after the other.
-// Eight requests, us in a replayed step: 8 heads of 256 x 512 gated 59 -> 12.9 (67 MB of states read and written), 32 of 128 x 128 with the
-// delta rule 17.4 -> 8.9, 16 with decays per channel 10.2 -> 7.9; 64 requests of 4 heads of 256 x 512 222 -> 41.
-__device__ __forceinline__ void token_load4(const float* p, float* v) {
-  const float4 x = *reinterpret_cast<const float4*>(p);
-  v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+// lanes, as above, reads them in pieces of 16 to 64), and both sums over the decayed S meet once, in registers and then over the
+// four waves in LDS.  Small ones are bound by their chain of waits: the first token's inputs are asked for before S is (loads come
+// back in their order), all without conditions of their own, so that norms and decays are made while S is on its way.  Longer spans
+// stay right: a token after the other.
+// Eight requests, us in a replayed step (before the order of its loads): 8 heads of 256 x 512 gated 9.3 (10.4; 67 MB of states read and
+// written), 32 of 128 x 128 with the delta rule 6.7 (7.3), 16 with decays per channel 5.1 (5.7), 32 of 64 x 64 with a bonus 3.4 (3.6); 64
+// requests of 4 heads of 256 x 512 40 (40); a column a group of lanes, as above, takes 59, 17.4, 10.2 and 222 of the first three and the last.
+template <typename T>
+struct TokenFour {
+  typedef uint32_t Raw __attribute__((ext_vector_type(sizeof(T))));  // four elements as they lie in memory
+};
+__device__ __forceinline__ uint32_t token_raw(float x) { return __float_as_uint(x); }
+__device__ __forceinline__ uint32_t token_raw(bf16_t x) { return x; }
+template <typename T>
+__device__ __forceinline__ float token_value(uint32_t raw) {
+  return __uint_as_float(sizeof(T) == 2 ? raw << 16 : raw);
 }
-__device__ __forceinline__ void token_load4(const bf16_t* p, float* v) {
-  const uint2 w = *reinterpret_cast<const uint2*>(p);
-  v[0] = __uint_as_float(w.x << 16); v[1] = __uint_as_float(w.x & 0xffff0000u);
-  v[2] = __uint_as_float(w.y << 16); v[3] = __uint_as_float(w.y & 0xffff0000u);
+__device__ __forceinline__ void token_four(TokenFour<float>::Raw x, float* v) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(x[e]);
+}
+__device__ __forceinline__ void token_four(TokenFour<bf16_t>::Raw x, float* v) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(e % 2 ? x[e / 2] & 0xffff0000u : x[e / 2] << 16);
 }
 
 template <typename T, int D, int KIND>
@@ -596,46 +611,73 @@ __global__ __launch_bounds__(256) void linear_state_token_kernel(const T* __rest
   constexpr bool CH = KIND & kScanChannel, DELTA = KIND & kScanDelta, FIRST = KIND & kScanReadFirst;
   constexpr int ROWS = D / 16;
   __shared__ __attribute__((aligned(16))) float ks[D], qs[D], as[CH ? D : 1], red[2][4][64], sums[4][4];
-  const int seq = blockIdx.x, h = blockIdx.y, kvh = h / (g.n_heads / g.n_kv), vdim = g.vdim;
+  typedef typename TokenFour<T>::Raw Raw4;
+  const int seq = blockIdx.x, h = blockIdx.y, vdim = g.vdim;
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, group = threadIdx.x / 16, col = 64 * blockIdx.z + 4 * (threadIdx.x % 16);
-  const int q0 = g.seq_qstart[seq], ql = g.seq_qlen[seq];
+  const int q0 = g.seq_qstart[seq], ql = g.seq_qlen[seq], state_slot = g.state_slots[seq];
+  const int kvh = g.per_kv == 1 ? h : divide_by(h, g.per_kv, g.per_kv_inverse);
+  arguments_now(g.decay, g.decay_p0, g.decay_p1, g.beta);
+  asm volatile("" ::"s"(q0), "s"(state_slot), "s"(g.skip), "s"(g.bonus));
   if (ql <= 0) return;
-  float* S_head = state + (static_cast<size_t>(g.state_slots[seq]) * g.n_heads + h) * D * vdim + col;
-  float S[ROWS][4];
+  const int i = min(static_cast<int>(threadIdx.x), D - 1);  // (threads beyond the channels read the last and use nothing)
+  // a decay that is given per head has no logits: its own value stands in for them
+  const bool logits = g.decay_mode != 4;
+  const float* z_col = logits ? g.decay + g.decay_col + (CH ? h * D + i : h) : g.decay_p0 + h;
+  const size_t z_stride = logits ? g.decay_stride : 0;
+  const float *bias_at = CH ? (g.decay_mode == 2 ? g.decay_p1 : g.decay_p0) + h * D + i : (g.decay_mode == 0 ? g.decay_p1 : g.decay_p0) + h,
+              *skip_at = (g.skip != nullptr ? g.skip : g.decay_p0) + h;
+  uint32_t q_raw, k_raw, beta_raw = 0;
+  Raw4 v_raw;
+  float z;
+  auto ask = [&](size_t n) {
+    const T* row = qkv + n * g.qkv_stride;
+    q_raw = token_raw(row[g.q_col + kvh * D + i]);
+    k_raw = token_raw(row[g.k_col + kvh * D + i]);
+    z = z_col[n * z_stride];
+    v_raw = *reinterpret_cast<const Raw4*>(row + g.v_col + h * vdim + col);
+    if (DELTA) {
+      const size_t at = n * g.beta_stride + g.beta_col + h;
+      if (beta_rows != nullptr) beta_raw = token_raw(beta_rows[at]);
+      else beta_raw = token_raw(g.beta[at]);
+    }
+  };
+  ask(q0);
+  const float bias = *bias_at, head_p0 = g.decay_p0[h], skip_raw = *skip_at, bonus = FIRST ? g.bonus[h * D + i] : 0.f;
+  float* S_head = state + (static_cast<size_t>(state_slot) * g.n_heads + h) * D * vdim + col;
+  TokenFour<float>::Raw S_raw[ROWS];
 #pragma unroll
-  for (int r = 0; r < ROWS; ++r) token_load4(S_head + static_cast<size_t>(group + 16 * r) * vdim, S[r]);
-  const float skip_h = g.skip != nullptr ? g.skip[h] : 0.f;
-  const float dec_rate = CH && g.decay_mode == 2 ? expf(g.decay_p0[h]) : 1.f;
-
+  for (int r = 0; r < ROWS; ++r) S_raw[r] = *reinterpret_cast<const TokenFour<float>::Raw*>(S_head + static_cast<size_t>(group + 16 * r) * vdim);
+  __builtin_amdgcn_sched_barrier(0);
+  const float skip_h = g.skip != nullptr ? skip_raw : 0.f;
+  const float dec_rate = CH && g.decay_mode == 2 ? expf(head_p0) : 1.f;
+  float S[ROWS][4];
   for (int t = 0; t < ql; ++t) {
     const size_t n = static_cast<size_t>(q0) + t;
-    const T* row = qkv + n * g.qkv_stride;
-    float v[4];
-    token_load4(row + g.v_col + h * vdim + col, v);
-    if (t > 0) __syncthreads();
+    if (t > 0) {
+      ask(n);
+      __syncthreads();
+    }
+    asm volatile("" : "+v"(q_raw), "+v"(k_raw));
     float q = 0.f, k = 0.f, w = 0.f;
-    const int i = threadIdx.x;
-    if (i < D) {
-      q = to_f32<T>(row[g.q_col + kvh * D + i]);
-      k = to_f32<T>(row[g.k_col + kvh * D + i]);
-      w = FIRST ? q * g.bonus[h * D + i] * k : q * k;
+    if (threadIdx.x < D) {
+      q = token_value<T>(q_raw);
+      k = token_value<T>(k_raw);
+      w = FIRST ? q * bonus * k : q * k;
       qs[i] = q;
       ks[i] = k;
-      if (CH) as[i] = channel_decay(g.decay[n * g.decay_stride + g.decay_col + h * D + i] + (g.decay_mode == 2 ? g.decay_p1 : g.decay_p0)[h * D + i], g.decay_mode,
-                                    g.tau, dec_rate);
+      if (CH) as[i] = channel_decay(z + bias, g.decay_mode, g.tau, dec_rate);
     }
     const float wave_q = wave_sum(q * q), wave_k = wave_sum(k * k), wave_w = wave_sum(w);
     if (lane == 0) sums[wave][0] = wave_q, sums[wave][1] = wave_k, sums[wave][2] = wave_w;
     float a = 1.f, strength = 1.f;
     if (!CH) {
-      const float step = g.decay_mode == 0 ? softplus_f32(g.decay[n * g.decay_stride + g.decay_col + h] + g.decay_p1[h]) : 1.f;
-      a = g.decay_mode == 4 ? g.decay_p0[h] : expf(-expf(g.decay_p0[h]) * step);
+      const float step = g.decay_mode == 0 ? softplus_f32(z + bias) : 1.f;
+      a = g.decay_mode == 4 ? head_p0 : expf(-expf(head_p0) * step);
       if (g.by_step) strength = step;
     }
-    if (DELTA) {
-      const size_t at = n * g.beta_stride + g.beta_col + h;
-      strength = 1.f / (1.f + expf(-(beta_rows != nullptr ? to_f32<T>(beta_rows[at]) : g.beta[at])));
-    }
+    if (DELTA) strength = 1.f / (1.f + expf(-(beta_rows != nullptr ? token_value<T>(beta_raw) : token_value<float>(beta_raw))));
+    float v[4];
+    token_four(v_raw, v);
     __syncthreads();
     float mq = g.q_scale, mk = 1.f;
     if (g.unit_eps >= 0.f) {
@@ -644,6 +686,10 @@ __global__ __launch_bounds__(256) void linear_state_token_kernel(const T* __rest
     }
     const float kq = ((sums[0][2] + sums[1][2]) + (sums[2][2] + sums[3][2])) * (mq * mk);
     float pk[2][4] = {}, pq[2][4] = {};
+    if (t == 0) {
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) token_four(S_raw[r], S[r]);
+    }
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
       const float ar = CH ? as[group + 16 * r] : a, kr = ks[group + 16 * r], qr = qs[group + 16 * r];
@@ -761,7 +807,8 @@ extern "C" int yk_linear_state_scan(const void* qkv, int qkv_stride, int dtype, 
   if (n_tokens == n_seqs && (dim == 64 || dim == 128 || dim == 256) && vdim % 64 == 0 && qkv_stride % 8 == 0 && v_col % 8 == 0 && al16(qkv) &&
       al16(state) && al16(out) && kind != kScanReadFirst && (skip == nullptr || kind == 0)) {
     const ScanArgs g{seq_qstart, seq_qlen, state_slots, qkv_stride, n_heads, n_kv, dim, vdim, q_col, k_col, v_col, q_scale, unit_eps, decay_mode, 0, decay,
-                     decay_stride, decay_col, decay_p0, decay_p1, tau, beta, beta_stride, beta_col, write_mode == 2, skip, bonus, 1};
+                     decay_stride, decay_col, decay_p0, decay_p1, tau, beta, beta_stride, beta_col, write_mode == 2, skip, bonus, 1,
+                     n_heads / n_kv, inverse_of(n_heads / n_kv)};
     const dim3 token_grid(n_seqs, n_heads, vdim / 64);
 #define YK_TOKEN(T, D, KIND)                                                                                                    \
   if (dim == D && kind == KIND) {                                                                                               \
@@ -791,7 +838,7 @@ extern "C" int yk_linear_state_scan(const void* qkv, int qkv_stride, int dtype, 
     }
     const ScanArgs g{seq_qstart, seq_qlen, state_slots, qkv_stride, n_heads, n_kv, dim, vdim, q_col, k_col, v_col, q_scale, unit_eps,
                      decay_mode, given, given ? decays : decay, given ? n_heads * dim : decay_stride, given ? 0 : decay_col, decay_p0, decay_p1, tau,
-                     beta, beta_stride, beta_col, write_mode == 2, skip, bonus, chunk};
+                     beta, beta_stride, beta_col, write_mode == 2, skip, bonus, chunk, n_heads / n_kv, inverse_of(n_heads / n_kv)};
     const size_t fast_lds = sizeof(float) * ((chunk + 2) * ((per_channel ? 3 : 2) * (dp + 4) + 4 + cols) + dp);
     YK_REQUIRE(fast_lds <= 128 * 1024, "linear_state_scan: the staged tokens do not fit in LDS");
 #define YK_FAST(T, TPC, KIND)                                                                                                   \
@@ -944,7 +991,8 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* __res
 }
 
 // The same in pieces of four elements, a thread holding P of them: everything is asked for before the sum.  LANES threads a part: as few
-// as hold it in one piece each up to a wave, which holds up to 1,024 elements in four, beyond it a workgroup.  Bound by memory where the
+// as hold it in one piece each up to a wave, which holds up to 1,024 elements in four, beyond it a workgroup.  Few parts are bound by what one waits for: a decode step of eight tokens, by
+// the trace, 16 parts of 128 4.9 -> 4.1 us without 64-bit divisions and conditions on loads.  Bound by memory where the
 // parts are many (bfloat16 gates and results, us, with its launch): 3,241 tokens of 16 parts of 128 12.9, where a wave a part with four pieces
 // a thread, three of them empty, took 46 for the gates' exponentials of nothing; 2,048 tokens of 32 parts of 64 7.8 (53), 16 of 128 8.4
 // (28), 8 of 256 8.0 (15.8), 4 of 512 8.1 (10.1), 2 of 1,024 8.1 (8.2).
@@ -972,29 +1020,33 @@ __device__ __forceinline__ float hn_sum(float v, float* scratch) {
 template <typename TW, typename TG, typename TO, int LANES, int P>
 __global__ __launch_bounds__(256) void gated_head_norm_vec_kernel(const float* __restrict__ o, const TW* __restrict__ w, float eps,
                                                                   const TG* __restrict__ gate, int gate_stride, int gate_col, int n_heads,
-                                                                  int vdim, TO* __restrict__ out, size_t total, int w_stride, int gate_first,
-                                                                  int gate_act) {
+                                                                  int vdim, TO* __restrict__ out, int total, int w_stride, int gate_first,
+                                                                  int gate_act, uint32_t heads_inverse) {
   __shared__ float scratch[17];
-  const size_t wanted = blockIdx.x * static_cast<size_t>(256 / LANES) + threadIdx.x / LANES;
-  const size_t item = min(wanted, total - 1);  // (threads past the end repeat the last part and store nothing)
+  const int wanted = blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+  const int item = min(wanted, total - 1);  // (threads past the end repeat the last part and store nothing)
   const int t = threadIdx.x % LANES;
-  const size_t n = item / n_heads;
-  const int h = static_cast<int>(item % n_heads);
-  const float* row = o + item * vdim;
-  const TG* g = gate + n * gate_stride + gate_col + h * vdim;
+  const int n = n_heads == 1 ? item : divide_by(item, n_heads, heads_inverse), h = item - n * n_heads;
+  const float* row = o + static_cast<size_t>(item) * vdim;
+  const TG* g = gate + static_cast<size_t>(n) * gate_stride + gate_col + h * vdim;
+  const TW* wh = w + static_cast<size_t>(h) * w_stride;
   float4 v[P], a[P], m[P];
   float ss = 0.f;
+  // (asked for without conditions, each of which would be a wait; pieces beyond the part read its last)
 #pragma unroll
   for (int p = 0; p < P; ++p) {
-    const int c = 4 * (t + p * LANES);
-    v[p] = a[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int c = min(4 * (t + p * LANES), vdim - 4);
+    v[p] = hn_load4<float>(row + c);
+    a[p] = hn_load4<TG>(g + c);
     m[p] = make_float4(1.f, 1.f, 1.f, 1.f);
-    if (c < vdim) {
-      v[p] = hn_load4<float>(row + c);
-      a[p] = hn_load4<TG>(g + c);
-      if (w != nullptr) m[p] = hn_load4<TW>(w + static_cast<size_t>(h) * w_stride + c);
-    }
   }
+  if (w != nullptr) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) m[p] = hn_load4<TW>(wh + min(4 * (t + p * LANES), vdim - 4));
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+    if (4 * (t + p * LANES) >= vdim) v[p] = a[p] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     a[p] = make_float4(head_gate_act(a[p].x, gate_act), head_gate_act(a[p].y, gate_act), head_gate_act(a[p].z, gate_act), head_gate_act(a[p].w, gate_act));
@@ -1009,7 +1061,7 @@ __global__ __launch_bounds__(256) void gated_head_norm_vec_kernel(const float* _
     if (c < vdim && wanted < total) {
       float4 y = make_float4(v[p].x * inv * m[p].x, v[p].y * inv * m[p].y, v[p].z * inv * m[p].z, v[p].w * inv * m[p].w);
       if (!gate_first) y.x *= a[p].x, y.y *= a[p].y, y.z *= a[p].z, y.w *= a[p].w;
-      hn_store4(out + item * vdim + c, y);
+      hn_store4(out + static_cast<size_t>(item) * vdim + c, y);
     }
   }
 }
@@ -1025,11 +1077,12 @@ extern "C" int yk_gated_head_norm(const float* o, const void* w, int w_dtype, fl
   const int grid = static_cast<int>((total + 3) / 4);
   const int w_stride = w_per_part ? vdim : 0;
   auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const bool vec = vdim % 4 == 0 && vdim <= 4096 && gate_stride % 4 == 0 && gate_col % 4 == 0 && al16(o) && al16(w) && al16(gate) && al16(out);
+  const bool vec = vdim % 4 == 0 && vdim <= 4096 && gate_stride % 4 == 0 && gate_col % 4 == 0 && al16(o) && al16(w) && al16(gate) && al16(out) &&
+                   total <= static_cast<size_t>(INT_MAX) - 256;
 #define YK_VEC(TW, TG, TO, LANES, P)                                                                                  \
   gated_head_norm_vec_kernel<TW, TG, TO, LANES, P><<<static_cast<unsigned>((total + 256 / LANES - 1) / (256 / LANES)), 256, 0, stream>>>( \
       o, static_cast<const TW*>(w), eps, static_cast<const TG*>(gate), gate_stride, gate_col, n_heads, vdim,          \
-      static_cast<TO*>(out), total, w_stride, gate_first, gate_act)
+      static_cast<TO*>(out), static_cast<int>(total), w_stride, gate_first, gate_act, inverse_of(n_heads))
 #define YK_CASE(WD, TW, GD, TG, OD, TO)                                                                               \
   if (w_dtype == WD && gate_dtype == GD && out_dtype == OD) {                                                         \
     if (vec && vdim > 1024) YK_VEC(TW, TG, TO, 256, 4);                                                               \
