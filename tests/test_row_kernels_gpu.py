@@ -293,3 +293,35 @@ def test_gated_recurrence_of_few_tokens(n, blocks, size):
     close(Sd, want_S, 2e-5)
     close(got, want_S[slots] * torch.nn.functional.gelu(y.double(), approximate="tanh"), 2.0 ** -8)
     assert torch.equal(kd.cpu(), want_kept)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [3, 21])
+@pytest.mark.parametrize("head_dim,value_dim,rotary,page,interleaved", [(2, 6, 2, 1, False), (66, 62, 34, 3, True), (128, 64, 128, 8, False), (130, 128, 64, 8, True),
+                                                                        (256, 256, 256, 16, False)])
+def test_projection_rows_at_the_ends_of_a_wave(dtype, n, head_dim, value_dim, rotary, page, interleaved):
+    """Heads that end inside a lane's first piece, at a wave's end and in the last piece, pages of one token; then the same queries turned
+    back and gated.  Float32: norms of up to 256 elements and two products a turn, 4e-6; bfloat16: rounded once or twice, 2^-7 of the largest."""
+    from yalis_amd.parts.base import Rotation
+
+    o, g, H, G = ops(), torch.Generator().manual_seed(head_dim + n), 3, 2
+    qkv = torch.randn(n, H * head_dim + G * (head_dim + value_dim), generator=g).to(dtype)
+    bias = torch.randn(qkv.shape[1], generator=g)
+    positions = torch.randint(0, 40, (n,), generator=g, dtype=torch.int32)
+    slots = torch.randperm(4 * page + n, generator=g)[:n].to(torch.int32)
+    qn, kn = (torch.rand(head_dim, generator=g) + 0.5).to(dtype), (torch.rand(head_dim, generator=g) + 0.5).to(dtype)
+    table = lambda width: [f(torch.arange(40.0)[:, None] * 100.0 ** (-torch.arange(width // 2) / (width // 2))) for f in (torch.cos, torch.sin)]
+    rot, vrot = (Rotation(*table(w), w, inter) for w, inter in ((rotary, interleaved), (value_dim, not interleaved)))
+    on = lambda r: Rotation(r.cos.cuda(), r.sin.cuda(), r.rotary_dim, r.interleaved)
+    n_pages = (4 * page + n) // page + 1
+    pages = lambda d: (torch.zeros(n_pages, G, page, head_dim, dtype=dtype, device=d), torch.zeros(n_pages, G, value_dim, page, dtype=dtype, device=d))
+    (k, v), (kr, vr) = pages("cuda"), pages("cpu")
+    got = o.qkv_prepare(qkv.cuda(), H, G, head_dim, value_dim, positions.cuda(), dtype, q_norm=qn.cuda(), k_norm=kn.cuda(), qk_eps=1e-6, rotation=on(rot),
+                        value_norm_eps=1e-6, value_rotation=on(vrot), k_cache=k, v_cache=v, slots=slots.cuda(), page_size=page, bias=bias.cuda())
+    want = R.qkv_prepare(qkv, H, G, head_dim, value_dim, positions, dtype, q_norm=qn, k_norm=kn, qk_eps=1e-6, rotation=rot, value_norm_eps=1e-6,
+                         value_rotation=vrot, k_cache=kr, v_cache=vr, slots=slots, page_size=page, bias=bias)
+    if o.masked_pages_tiled(dtype, head_dim, value_dim, page):
+        k, v = R.untile_cache(k, v)
+    tol = 4e-6 if dtype == torch.float32 else 2.0 ** -7
+    for a, b in ((got, want), (k, kr), (v, vr)):
+        close(a, b.to(a.dtype), tol)

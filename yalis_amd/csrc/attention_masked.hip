@@ -49,10 +49,124 @@ __device__ __forceinline__ float rotated_element(const float* buf, int i, int ro
   return rot_second(buf[i - half], buf[i], cos_row[i - half], sign * sin_row[i - half]);
 }
 
+// What both kernels make of a token's head before it turns, a wave each: the sum of its slices, the bias, the norm and the row's scale in
+// val (element lane + 64 i; zeros beyond len), and the cosines and sines it will turn by.  NI: pieces of 64 that hold the longest head.
+// Bound by what one waits for: the position comes with the arguments' loads, and the row, its weights, bias and scale, then the tables'
+// rows are all asked for before the first is used, none under a condition that differs between lanes (a wait for each: a head of 128
+// in four pieces 12 of them, one after the other).  By the trace, 24 heads of 128, normed, turned, in tiled pages: 4 tokens 5.9 -> 3.5 us,
+// 2,801 in groups of eight 49 -> 33.
+template <int NI>
+struct HeadValues {
+  float val[NI], cv[NI], sv[NI];
+  int rot = 0, inter = 0;
+};
+__device__ __forceinline__ uint32_t head_raw(float x) { return __float_as_uint(x); }
+__device__ __forceinline__ uint32_t head_raw(bf16_t x) { return x; }
+template <typename T>
+__device__ __forceinline__ float head_value(uint32_t x) {
+  return __uint_as_float(sizeof(T) == 2 ? x << 16 : x);
+}
+template <int NI, typename TS, typename TW>
+__device__ __forceinline__ HeadValues<NI> head_values(
+    const TS* row, int n_splits, size_t split_stride, int round_sum, int kind, int col0, int n, int len, int k_col0, int pos,
+    const TW* q_norm_w, const TW* k_norm_w, int qk_norm, float qk_eps, const float* cos_t, const float* sin_t, int rotary_dim, int interleaved,
+    int max_pos, int v_norm, float v_eps, const float* v_cos, const float* v_sin, int v_interleaved, int v_max_pos, const float* bias,
+    const float* row_scales) {
+  HeadValues<NI> x;
+  const int lane = threadIdx.x % 64;
+  int at[NI];
+  uint32_t raw[NI], wr[NI], br[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    at[i] = min(lane + 64 * i, len - 1);
+    raw[i] = head_raw(row[at[i]]);
+  }
+  asm volatile("" ::"s"(pos));  // (here at the latest, or it is asked for where the tables are)
+  // weights: of the head's elements, or as wide as the projection
+  const TW* w = kind == 2 || qk_norm == 0 ? nullptr : kind == 0 ? q_norm_w : k_norm_w;
+  if (w != nullptr) {
+    if (qk_norm == 2) w += kind == 0 ? col0 : col0 - k_col0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) wr[i] = head_raw(w[at[i]]);
+  }
+  if (bias != nullptr) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) br[i] = head_raw(bias[col0 + at[i]]);
+  }
+  float rs = 1.f;
+  const bool scaled = kind != 2 && row_scales != nullptr;
+  if (scaled) rs = row_scales[2 * static_cast<size_t>(n) + kind];
+  const float *cr = nullptr, *sr = nullptr;
+  if (kind == 2) {
+    if (v_cos != nullptr) {
+      x.rot = len, x.inter = v_interleaved;
+      cr = v_cos, sr = v_sin;
+    }
+  } else if (rotary_dim > 0) {
+    x.rot = rotary_dim, x.inter = interleaved;
+    cr = cos_t, sr = sin_t;
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i) x.cv[i] = 1.f, x.sv[i] = 0.f;
+  if (x.rot > 0) {
+    const int half = x.rot / 2;
+    const size_t first = static_cast<size_t>(min(pos, (kind == 2 ? v_max_pos : max_pos) - 1)) * half;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int d = min(lane + 64 * i, x.rot - 1), m = x.inter ? d / 2 : (d < half ? d : d - half);
+      x.cv[i] = cr[first + m];
+      x.sv[i] = sr[first + m];
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) x.val[i] = 0.f + head_value<TS>(raw[i]);
+  for (int s = 1; s < n_splits; ++s)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x.val[i] += to_f32<TS>(row[s * split_stride + at[i]]);
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    float v = as_output(x.val[i], round_sum);
+    if (bias != nullptr) v += __uint_as_float(br[i]);
+    v = lane + 64 * i < len ? v : 0.f;
+    x.val[i] = v;
+    ss = fmaf(v, v, ss);
+  }
+  if (kind == 2 ? v_norm != 0 : qk_norm == 1) {
+    ss = wave_sum(ss);
+    const float inv = 1.f / sqrtf(ss / static_cast<float>(len) + (kind == 2 ? v_eps : qk_eps));
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x.val[i] = x.val[i] * inv * (w != nullptr ? head_value<TW>(wr[i]) : 1.f);
+  } else if (kind != 2 && qk_norm == 2) {  // (over the whole projection: its inverse root mean square is part of the row's scale)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x.val[i] *= head_value<TW>(wr[i]);
+  }
+  if (scaled) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x.val[i] *= rs;
+  }
+  return x;
+}
+// element d of a head that lies in LDS, turned by its pair's angle
+__device__ __forceinline__ float head_turned(float mine, const float* buf, int d, int rot, int inter, float c, float s) {
+  if (rot == 0) return mine;
+  const int half = rot / 2;
+  const bool first = inter ? d % 2 == 0 : d < half, turns = d < rot;
+  const float other = buf[!turns ? d : inter ? d ^ 1 : first ? d + half : d - half];
+  const float a = first ? mine : other, b = first ? other : mine, x = rot_first(a, b, c, s), y = rot_second(a, b, c, s);
+  return turns ? (first ? x : y) : mine;
+}
+// a wave's own LDS: written before, read behind
+__device__ __forceinline__ void head_in_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace
 
 // A workgroup of four waves takes four heads of a token (a wave a head).
-template <typename TS, typename T, typename TW>
+template <typename TS, typename T, typename TW, int NI>
 __global__ __launch_bounds__(256) void qkv_prepare_kernel(
     const TS* __restrict__ src, int n_splits, size_t split_stride, int round_sum, int src_stride,
     T* __restrict__ q_out, int q_stride, int n_heads, int n_kv, int head_dim, int v_dim,
@@ -61,13 +175,12 @@ __global__ __launch_bounds__(256) void qkv_prepare_kernel(
     int interleaved, int max_pos, int v_norm, float v_eps, const float* __restrict__ v_cos,
     const float* __restrict__ v_sin, int v_interleaved, int v_max_pos, T* __restrict__ k_cache,
     T* __restrict__ v_cache, const int32_t* __restrict__ slots, int page_size, int tiled,
-    const float* __restrict__ bias, const float* __restrict__ row_scales, int v_from_k, int q_maps) {
-  __shared__ float bufs[4][kMaxHead];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const float* __restrict__ bias, const float* __restrict__ row_scales, int v_from_k, int q_maps, uint32_t page_inverse) {
+  __shared__ float bufs[4][64 * NI];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   float* buf = bufs[wave];
-  const int n = blockIdx.x, n_slots = n_heads + 2 * n_kv;
-  const bool live = blockIdx.y * 4 + wave < n_slots;  // (a wave beyond the heads works on the last one and stores nothing)
-  const int slot_y = min(static_cast<int>(blockIdx.y) * 4 + wave, n_slots - 1);
+  const int n = blockIdx.x, n_slots = n_heads + 2 * n_kv, slot_y = blockIdx.y * 4 + wave;
+  if (slot_y >= n_slots) return;
   const int kind = slot_y < n_heads ? 0 : (slot_y < n_heads + n_kv ? 1 : 2);  // q, k, v
   const int len = kind == 2 ? v_dim : head_dim;
   int col0;
@@ -75,107 +188,40 @@ __global__ __launch_bounds__(256) void qkv_prepare_kernel(
   else if (kind == 1) col0 = n_heads * head_dim + (slot_y - n_heads) * head_dim;
   else if (v_from_k) col0 = n_heads * head_dim + (slot_y - n_heads - n_kv) * head_dim;  // the key head's own columns
   else col0 = (n_heads + n_kv) * head_dim + (slot_y - n_heads - n_kv) * v_dim;
-  const TS* row = src + static_cast<size_t>(n) * src_stride + col0;
-  // the position, this lane's cosines and sines and the token's slot are asked for before the row
-  // is: three waits for memory one behind the other (position, table, row) become two side by side
-  const int pos = positions[n];
-  const float *cr = nullptr, *sr = nullptr;
-  int rot = 0, inter = 0;
-  if (kind == 2) {
-    if (v_cos != nullptr) {
-      const int p = min(pos, v_max_pos - 1);
-      rot = v_dim, inter = v_interleaved;
-      cr = v_cos + static_cast<size_t>(p) * (v_dim / 2);
-      sr = v_sin + static_cast<size_t>(p) * (v_dim / 2);
-    }
-  } else if (rotary_dim > 0) {
-    const int p = min(pos, max_pos - 1);
-    rot = rotary_dim, inter = interleaved;
-    cr = cos_t + static_cast<size_t>(p) * (rotary_dim / 2);
-    sr = sin_t + static_cast<size_t>(p) * (rotary_dim / 2);
-  }
-  float cv[4], sv[4];
+  const int pos = positions[n], slot = kind != 0 ? slots[n] : 0;
+  arguments_now(q_norm_w, k_norm_w, k_cache, v_cache);
+  arguments_now(cos_t, sin_t, v_cos, v_sin);
+  arguments_now(bias, row_scales);
+  const HeadValues<NI> x = head_values<NI, TS, TW>(src + static_cast<size_t>(n) * src_stride + col0, n_splits, split_stride, round_sum, kind, col0, n, len,
+                                                   n_heads * head_dim, pos, q_norm_w, k_norm_w, qk_norm, qk_eps, cos_t, sin_t, rotary_dim,
+                                                   interleaved, max_pos, v_norm, v_eps, v_cos, v_sin, v_interleaved, v_max_pos, bias, row_scales);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = lane + 64 * i;
-    cv[i] = 1.f, sv[i] = 0.f;
-    if (d < rot) {
-      const int m = inter ? d / 2 : (d < rot / 2 ? d : d - rot / 2);
-      cv[i] = cr[m];
-      sv[i] = sr[m];
-    }
-  }
-  const int slot = kind != 0 ? slots[n] : 0;
-  float val[4];
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = lane + 64 * i;
-    float v = 0.f;
-    if (d < len) {
-      for (int s = 0; s < n_splits; ++s) v += to_f32<TS>(row[s * split_stride + d]);
-      v = as_output(v, round_sum);
-      if (bias != nullptr) v += bias[col0 + d];
-    }
-    val[i] = v;
-    ss = fmaf(v, v, ss);
-  }
-  const bool normed = kind == 2 ? v_norm != 0 : qk_norm == 1;
-  if (normed) {
-    ss = wave_sum(ss);
-    const float inv = 1.f / sqrtf(ss / static_cast<float>(len) + (kind == 2 ? v_eps : qk_eps));
-    const TW* w = kind == 0 ? q_norm_w : (kind == 1 ? k_norm_w : nullptr);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = lane + 64 * i;
-      if (d < len) val[i] = val[i] * inv * (w != nullptr ? to_f32<TW>(w[d]) : 1.f);
-    }
-  } else if (kind != 2 && qk_norm == 2) {
-    // the norm over the whole projection: weights as wide as the projection; the inverse root mean square over
-    // all heads is part of the row's scale below
-    const TW* w = kind == 0 ? q_norm_w + col0 : k_norm_w + (col0 - n_heads * head_dim);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = lane + 64 * i;
-      if (d < len) val[i] *= to_f32<TW>(w[d]);
-    }
-  }
-  if (kind != 2 && row_scales != nullptr) {
-    const float rs = row_scales[2 * static_cast<size_t>(n) + kind];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) val[i] *= rs;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = lane + 64 * i;
-    if (d < len) buf[d] = val[i];
-  }
-  __syncthreads();
+  for (int i = 0; i < NI; ++i)
+    if (lane + 64 * i < len) buf[lane + 64 * i] = x.val[i];
+  head_in_lds();
   size_t base = 0;
   int off = 0;
   if (kind != 0) {
-    const int page = slot / page_size, g = kind == 1 ? slot_y - n_heads : slot_y - n_heads - n_kv;
-    off = slot % page_size;
+    const int page = page_size == 1 ? slot : divide_by(slot, page_size, page_inverse), g = kind == 1 ? slot_y - n_heads : slot_y - n_heads - n_kv;
+    off = slot - page * page_size;
     base = (static_cast<size_t>(page) * n_kv + g) * page_size * (kind == 1 ? head_dim : v_dim);
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NI; ++i) {
     const int d = lane + 64 * i;
-    if (d >= len || !live) continue;
-    float v = buf[d];
-    if (d < rot) {  // the pair's other element from LDS, the angle from the registers
-      if (inter)
-        v = (d % 2 == 0) ? rot_first(buf[d], buf[d + 1], cv[i], sv[i]) : rot_second(buf[d - 1], buf[d], cv[i], sv[i]);
+    if (d >= len) continue;
+    const float v = head_turned(x.val[i], buf, d, x.rot, x.inter, x.cv[i], x.sv[i]);
+    if (kind == 0) {
+      T* out = q_out + static_cast<size_t>(n) * q_stride + static_cast<size_t>(col0) * q_maps + d;
+      if (q_maps == 1) *out = from_f32<T>(v);
       else
-        v = d < rot / 2 ? rot_first(buf[d], buf[d + rot / 2], cv[i], sv[i]) : rot_second(buf[d - rot / 2], buf[d], cv[i], sv[i]);
-    }
-    if (kind == 0)
-      for (int mp = 0; mp < q_maps; ++mp)  // a row per map, zeros where the other maps' elements are
-        q_out[static_cast<size_t>(n) * q_stride + static_cast<size_t>(col0) * q_maps + mp * head_dim + d] = from_f32<T>(d / (head_dim / q_maps) == mp ? v : 0.f);
-    else if (kind == 1)
+        for (int mp = 0; mp < q_maps; ++mp)  // a row per map, zeros where the other maps' elements are
+          out[mp * head_dim] = from_f32<T>(d / (head_dim / q_maps) == mp ? v : 0.f);
+    } else if (kind == 1) {
       k_cache[base + cache_k_offset(tiled, page_size, head_dim, off, d)] = from_f32<T>(v);
-    else
+    } else {
       v_cache[base + cache_v_offset(tiled, page_size, v_dim, off, d)] = from_f32<T>(v);
+    }
   }
 }
 
@@ -185,7 +231,7 @@ __global__ __launch_bounds__(256) void qkv_prepare_kernel(
 // slots run on from a multiple of eight within a page, the eight tokens' values of one element as
 // one piece of the transposed page (a token at a time stores each value two bytes wide into a
 // row of its own, 128 bytes from the next).
-template <typename TS, typename TW>
+template <typename TS, typename TW, int NI>
 __global__ __launch_bounds__(512) void qkv_prepare8_kernel(
     const TS* __restrict__ src, int n_splits, size_t split_stride, int round_sum, int src_stride,
     bf16_t* __restrict__ q_out, int q_stride, int n_heads, int n_kv, int head_dim, int v_dim,
@@ -194,11 +240,11 @@ __global__ __launch_bounds__(512) void qkv_prepare8_kernel(
     int interleaved, int max_pos, int v_norm, float v_eps, const float* __restrict__ v_cos,
     const float* __restrict__ v_sin, int v_interleaved, int v_max_pos, bf16_t* __restrict__ k_cache,
     bf16_t* __restrict__ v_cache, const int32_t* __restrict__ slots, int page_size, int tiled, int n_tokens,
-    const float* __restrict__ bias, const float* __restrict__ row_scales, int v_from_k, int q_maps) {
-  __shared__ float bufs[8][kMaxHead];
-  __shared__ __attribute__((aligned(16))) bf16_t outs[8][kMaxHead];
+    const float* __restrict__ bias, const float* __restrict__ row_scales, int v_from_k, int q_maps, uint32_t page_inverse) {
+  __shared__ float bufs[8][64 * NI];
+  __shared__ __attribute__((aligned(16))) bf16_t outs[8][64 * NI];
   __shared__ int slot_s[8];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   float* buf = bufs[wave];
   const int n0 = blockIdx.x * 8, n_live = min(8, n_tokens - n0);
   const int n = min(n0 + wave, n_tokens - 1);  // (a wave beyond the tokens repeats the last one; nothing of it is stored)
@@ -210,116 +256,46 @@ __global__ __launch_bounds__(512) void qkv_prepare8_kernel(
   else if (kind == 1) col0 = n_heads * head_dim + (slot_y - n_heads) * head_dim;
   else if (v_from_k) col0 = n_heads * head_dim + (slot_y - n_heads - n_kv) * head_dim;  // the key head's own columns
   else col0 = (n_heads + n_kv) * head_dim + (slot_y - n_heads - n_kv) * v_dim;
-  const TS* row = src + static_cast<size_t>(n) * src_stride + col0;
-  const int pos = positions[n];
-  const float *cr = nullptr, *sr = nullptr;
-  int rot = 0, inter = 0;
-  if (kind == 2) {
-    if (v_cos != nullptr) {
-      const int p = min(pos, v_max_pos - 1);
-      rot = v_dim, inter = v_interleaved;
-      cr = v_cos + static_cast<size_t>(p) * (v_dim / 2);
-      sr = v_sin + static_cast<size_t>(p) * (v_dim / 2);
-    }
-  } else if (rotary_dim > 0) {
-    const int p = min(pos, max_pos - 1);
-    rot = rotary_dim, inter = interleaved;
-    cr = cos_t + static_cast<size_t>(p) * (rotary_dim / 2);
-    sr = sin_t + static_cast<size_t>(p) * (rotary_dim / 2);
-  }
-  float cv[4], sv[4];
+  const int pos = positions[n], slot = kind != 0 ? slots[n] : 0;
+  arguments_now(q_norm_w, k_norm_w, k_cache, v_cache);
+  arguments_now(cos_t, sin_t, v_cos, v_sin);
+  arguments_now(bias, row_scales);
+  const HeadValues<NI> x = head_values<NI, TS, TW>(src + static_cast<size_t>(n) * src_stride + col0, n_splits, split_stride, round_sum, kind, col0, n, len,
+                                                   n_heads * head_dim, pos, q_norm_w, k_norm_w, qk_norm, qk_eps, cos_t, sin_t, rotary_dim,
+                                                   interleaved, max_pos, v_norm, v_eps, v_cos, v_sin, v_interleaved, v_max_pos, bias, row_scales);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NI; ++i)
+    if (lane + 64 * i < len) buf[lane + 64 * i] = x.val[i];
+  head_in_lds();
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
     const int d = lane + 64 * i;
-    cv[i] = 1.f, sv[i] = 0.f;
-    if (d < rot) {
-      const int m = inter ? d / 2 : (d < rot / 2 ? d : d - rot / 2);
-      cv[i] = cr[m];
-      sv[i] = sr[m];
-    }
+    if (d < len) outs[wave][d] = f32_to_bf16(head_turned(x.val[i], buf, d, x.rot, x.inter, x.cv[i], x.sv[i]));
   }
-  if (lane == 0) slot_s[wave] = kind != 0 ? slots[n] : 0;
-  float val[4];
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = lane + 64 * i;
-    float v = 0.f;
-    if (d < len) {
-      for (int s = 0; s < n_splits; ++s) v += to_f32<TS>(row[s * split_stride + d]);
-      v = as_output(v, round_sum);
-      if (bias != nullptr) v += bias[col0 + d];
-    }
-    val[i] = v;
-    ss = fmaf(v, v, ss);
-  }
-  const bool normed = kind == 2 ? v_norm != 0 : qk_norm == 1;
-  if (normed) {
-    ss = wave_sum(ss);
-    const float inv = 1.f / sqrtf(ss / static_cast<float>(len) + (kind == 2 ? v_eps : qk_eps));
-    const TW* w = kind == 0 ? q_norm_w : (kind == 1 ? k_norm_w : nullptr);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = lane + 64 * i;
-      if (d < len) val[i] = val[i] * inv * (w != nullptr ? to_f32<TW>(w[d]) : 1.f);
-    }
-  } else if (kind != 2 && qk_norm == 2) {
-    // the norm over the whole projection: weights as wide as the projection; the inverse root mean square over
-    // all heads is part of the row's scale below
-    const TW* w = kind == 0 ? q_norm_w + col0 : k_norm_w + (col0 - n_heads * head_dim);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int d = lane + 64 * i;
-      if (d < len) val[i] *= to_f32<TW>(w[d]);
-    }
-  }
-  if (kind != 2 && row_scales != nullptr) {
-    const float rs = row_scales[2 * static_cast<size_t>(n) + kind];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) val[i] *= rs;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = lane + 64 * i;
-    if (d < len) buf[d] = val[i];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = lane + 64 * i;
-    if (d >= len) continue;
-    float v = buf[d];
-    if (d < rot) {
-      if (inter)
-        v = (d % 2 == 0) ? rot_first(buf[d], buf[d + 1], cv[i], sv[i]) : rot_second(buf[d - 1], buf[d], cv[i], sv[i]);
-      else
-        v = d < rot / 2 ? rot_first(buf[d], buf[d + rot / 2], cv[i], sv[i]) : rot_second(buf[d - rot / 2], buf[d], cv[i], sv[i]);
-    }
-    outs[wave][d] = f32_to_bf16(v);
-  }
-  __syncthreads();
-  const int pieces = len / 8;  // (len is a multiple of 8 here)
+  head_in_lds();
+  const int pieces = len / 8;  // (len is a multiple of 8 here; queries and keys: a wave stores its own token's)
   if (kind == 0) {
-    for (int idx = threadIdx.x; idx < n_live * pieces; idx += blockDim.x) {
-      const int t = idx / pieces, p = idx % pieces;
+    if (wave >= n_live || lane >= pieces) return;
+    const uint4 row = *reinterpret_cast<const uint4*>(&outs[wave][8 * lane]);
+    bf16_t* out = q_out + static_cast<size_t>(n) * q_stride + static_cast<size_t>(col0) * q_maps + 8 * lane;
+    if (q_maps == 1) *reinterpret_cast<uint4*>(out) = row;
+    else
       for (int mp = 0; mp < q_maps; ++mp)  // a row per map, zeros where the other maps' elements are
-        *reinterpret_cast<uint4*>(q_out + static_cast<size_t>(n0 + t) * q_stride + static_cast<size_t>(col0) * q_maps + mp * head_dim + 8 * p) =
-            p / (pieces / q_maps) == mp ? *reinterpret_cast<const uint4*>(&outs[t][8 * p]) : make_uint4(0u, 0u, 0u, 0u);
-    }
+        *reinterpret_cast<uint4*>(out + mp * head_dim) = lane / (pieces / q_maps) == mp ? row : make_uint4(0u, 0u, 0u, 0u);
     return;
   }
   const int g = kind == 1 ? slot_y - n_heads : slot_y - n_heads - n_kv;
   const size_t slab = static_cast<size_t>(page_size) * len;
   if (kind == 1) {
-    for (int idx = threadIdx.x; idx < n_live * pieces; idx += blockDim.x) {
-      const int t = idx / pieces, p = idx % pieces;
-      const int slot = slot_s[t];
-      const size_t base = (static_cast<size_t>(slot / page_size) * n_kv + g) * slab;
-      *reinterpret_cast<uint4*>(k_cache + base + cache_k_offset(tiled, page_size, head_dim, slot % page_size, 8 * p)) =
-          *reinterpret_cast<const uint4*>(&outs[t][8 * p]);
-    }
+    if (wave >= n_live || lane >= pieces) return;
+    const int page = page_size == 1 ? slot : divide_by(slot, page_size, page_inverse);
+    const size_t base = (static_cast<size_t>(page) * n_kv + g) * slab;
+    *reinterpret_cast<uint4*>(k_cache + base + cache_k_offset(tiled, page_size, head_dim, slot - page * page_size, 8 * lane)) =
+        *reinterpret_cast<const uint4*>(&outs[wave][8 * lane]);
     return;
   }
+  if (lane == 0) slot_s[wave] = slot;
+  __syncthreads();
   bool together = n_live == 8 && slot_s[0] % 8 == 0;
 #pragma unroll
   for (int t = 1; t < 8; ++t) together = together && slot_s[t] == slot_s[0] + t;
@@ -367,18 +343,21 @@ extern "C" int yk_qkv_prepare(const void* src, int src_dtype, int n_splits, int 
   YK_REQUIRE(n_heads + 2 * n_kv <= 65535, "qkv_prepare: too many heads for one launch");
   if (n_tokens == 0) return 0;
   const size_t stride = static_cast<size_t>(n_tokens) * src_stride;
+  const bool two = head_dim <= 128 && v_dim <= 128;
+  const uint32_t page_inverse = page_size > 0 ? inverse_of(page_size) : 0;
   auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   if (act_dtype == YK_BF16 && n_tokens >= 16 && head_dim % (8 * q_maps) == 0 && v_dim % 8 == 0 && q_stride % 8 == 0 && page_size % 8 == 0 &&
       al16(q_out) && al16(k_cache) && al16(v_cache) && (norm_w_dtype == YK_BF16 || norm_w_dtype == YK_F32)) {
     dim3 grid8((n_tokens + 7) / 8, n_heads + 2 * n_kv);
 #define YK_CASE8(SD, TS, WD, TW)                                                                              \
   if (src_dtype == SD && (norm_w_dtype == WD || (q_norm_w == nullptr && k_norm_w == nullptr && WD == YK_F32))) { \
-    qkv_prepare8_kernel<TS, TW><<<grid8, 512, 0, stream>>>(                                                    \
+    auto kern = two ? qkv_prepare8_kernel<TS, TW, 2> : qkv_prepare8_kernel<TS, TW, 4>;                          \
+    kern<<<grid8, 512, 0, stream>>>(                                                                           \
         static_cast<const TS*>(src), n_splits, stride, round_sum, src_stride, static_cast<bf16_t*>(q_out), q_stride, \
         n_heads, n_kv, head_dim, v_dim, positions, static_cast<const TW*>(q_norm_w),                           \
         static_cast<const TW*>(k_norm_w), qk_norm, qk_eps, cos_t, sin_t, rotary_dim, interleaved, max_pos,      \
         v_norm, v_eps, v_cos, v_sin, v_interleaved, v_max_pos, static_cast<bf16_t*>(k_cache),                  \
-        static_cast<bf16_t*>(v_cache), slots, page_size, tiled, n_tokens, bias, row_scales, v_from_k, q_maps);         \
+        static_cast<bf16_t*>(v_cache), slots, page_size, tiled, n_tokens, bias, row_scales, v_from_k, q_maps, page_inverse); \
     return yk_check_launch("qkv_prepare (8 tokens)");                                                          \
   }
     YK_CASE8(YK_F32, float, YK_F32, float)
@@ -390,12 +369,13 @@ extern "C" int yk_qkv_prepare(const void* src, int src_dtype, int n_splits, int 
   dim3 grid(n_tokens, (n_heads + 2 * n_kv + 3) / 4), block(256);
 #define YK_CASE(SD, TS, AD, T, WD, TW)                                                                       \
   if (src_dtype == SD && act_dtype == AD && (norm_w_dtype == WD || (q_norm_w == nullptr && k_norm_w == nullptr && WD == YK_F32))) { \
-    qkv_prepare_kernel<TS, T, TW><<<grid, block, 0, stream>>>(                                                \
+    auto kern = two ? qkv_prepare_kernel<TS, T, TW, 2> : qkv_prepare_kernel<TS, T, TW, 4>;                     \
+    kern<<<grid, block, 0, stream>>>(                                                                         \
         static_cast<const TS*>(src), n_splits, stride, round_sum, src_stride, static_cast<T*>(q_out), q_stride,  \
         n_heads, n_kv, head_dim, v_dim, positions, static_cast<const TW*>(q_norm_w),                          \
         static_cast<const TW*>(k_norm_w), qk_norm, qk_eps, cos_t, sin_t, rotary_dim, interleaved, max_pos,     \
         v_norm, v_eps, v_cos, v_sin, v_interleaved, v_max_pos, static_cast<T*>(k_cache), static_cast<T*>(v_cache), \
-        slots, page_size, tiled, bias, row_scales, v_from_k, q_maps);                                                 \
+        slots, page_size, tiled, bias, row_scales, v_from_k, q_maps, page_inverse);                             \
     return yk_check_launch("qkv_prepare");                                                                    \
   }
   YK_CASE(YK_F32, float, YK_F32, float, YK_F32, float)
@@ -668,29 +648,50 @@ extern "C" int yk_attn_masked(const void* q, int q_stride, void* out, const void
   return yk_fail("attn_masked: unsupported dtype combination");
 }
 
-template <typename T, typename TG>
+// Bound by its chain of waits, as head_values is: the row, the tables' and the gate are asked for before the row goes through LDS.
+// 16 heads of 128, by the trace: 4 tokens 4.1 -> 2.3 us.
+template <typename T, typename TG, int NI>
 __global__ __launch_bounds__(64) void attn_finish_kernel(
     T* __restrict__ out, const int32_t* __restrict__ positions, int v_dim, int n_heads, const float* __restrict__ v_cos,
     const float* __restrict__ v_sin, int v_interleaved, int v_max_pos, const TG* __restrict__ gate_src, int gate_splits,
     size_t gate_split_stride, int gate_round, int gate_stride, int gate_col0, int gate_elems) {
-  __shared__ float os[kMaxHead];
-  const int n = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+  __shared__ float os[64 * NI];
+  const int n = blockIdx.x, h = blockIdx.y, lane = threadIdx.x, pos = v_cos != nullptr ? positions[n] : 0;
   T* orow = out + (static_cast<size_t>(n) * n_heads + h) * v_dim;
-  for (int d = lane; d < v_dim; d += 64) os[d] = to_f32<T>(orow[d]);
-  __syncthreads();
-  float gate = 1.f;
-  const size_t gate_at = static_cast<size_t>(n) * gate_stride + gate_col0 + static_cast<size_t>(h) * gate_elems;
-  if (gate_src != nullptr && gate_elems == 1) gate = head_gate<TG>(gate_src, gate_splits, gate_split_stride, gate_round, gate_at);
-  const float *cr = nullptr, *sr = nullptr;
-  if (v_cos != nullptr) {
-    const int p = min(positions[n], v_max_pos - 1);
-    cr = v_cos + static_cast<size_t>(p) * (v_dim / 2);
-    sr = v_sin + static_cast<size_t>(p) * (v_dim / 2);
+  int at[NI];
+  uint32_t raw[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    at[i] = min(lane + 64 * i, v_dim - 1);
+    raw[i] = head_raw(orow[at[i]]);
   }
-  for (int d = lane; d < v_dim; d += 64) {
-    const float v = cr != nullptr ? rotated_element(os, d, v_dim, v_interleaved, cr, sr, -1.f) : os[d];
-    if (gate_src != nullptr && gate_elems > 1) gate = head_gate<TG>(gate_src, gate_splits, gate_split_stride, gate_round, gate_at + d);
-    orow[d] = from_f32<T>(v * gate);
+  asm volatile("" ::"s"(pos));
+  float cv[NI], sv[NI], gate[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) cv[i] = 1.f, sv[i] = 0.f, gate[i] = 1.f;
+  if (v_cos != nullptr) {
+    const int half = v_dim / 2;
+    const size_t first = static_cast<size_t>(min(pos, v_max_pos - 1)) * half;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int m = v_interleaved ? at[i] / 2 : (at[i] < half ? at[i] : at[i] - half);
+      cv[i] = v_cos[first + m];
+      sv[i] = v_sin[first + m];
+    }
+  }
+  if (gate_src != nullptr) {
+    const size_t gate_at = static_cast<size_t>(n) * gate_stride + gate_col0 + static_cast<size_t>(h) * gate_elems;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      gate[i] = i > 0 && gate_elems == 1 ? gate[0] : head_gate<TG>(gate_src, gate_splits, gate_split_stride, gate_round, gate_at + (gate_elems == 1 ? 0 : at[i]));
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i) os[lane + 64 * i] = head_value<T>(raw[i]);
+  head_in_lds();
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int d = lane + 64 * i;
+    if (d < v_dim) orow[d] = from_f32<T>(head_turned(head_value<T>(raw[i]), os, d, v_cos != nullptr ? v_dim : 0, v_interleaved, cv[i], -sv[i]) * gate[i]);
   }
 }
 
@@ -706,7 +707,8 @@ extern "C" int yk_attn_finish(void* out, int dtype, const int32_t* positions, in
   const size_t gstride = static_cast<size_t>(n_tokens) * gate_stride;
 #define YK_CASE(D, T, GD, TG)                                                                          \
   if (dtype == D && (gate_src == nullptr ? GD == D : gate_dtype == GD)) {                               \
-    attn_finish_kernel<T, TG><<<grid, block, 0, stream>>>(static_cast<T*>(out), positions, v_dim, n_heads, v_cos, v_sin, \
+    auto kern = v_dim <= 128 ? attn_finish_kernel<T, TG, 2> : attn_finish_kernel<T, TG, 4>;              \
+    kern<<<grid, block, 0, stream>>>(static_cast<T*>(out), positions, v_dim, n_heads, v_cos, v_sin, \
                                                           v_interleaved, v_max_pos, static_cast<const TG*>(gate_src),   \
                                                           gate_splits, gstride, gate_round, gate_stride, gate_col0,     \
                                                           gate_elems);                                                  \
