@@ -186,7 +186,8 @@ static int g_mode = 0;
 // the units waits for the first.  So, where slices would do (handed_on): matrices of up to 6.5 M elements whose K and columns are not
 // far apart (1,024 x 4,096 at eight rows 9.5 / 10.0; one slice: 8,192 x 512 5.3 / 4.3, 12,288 x 512 5.5 / 5.7, 25,344 x 256 4.8 / 8.2);
 // larger ones whose workgroups make one or two whole rounds of the compute units; and with up to four and two rows those on whose
-// line above it is ahead.  Up to eight rows: at 16 the two are about even, and a product that takes attention's
+// line above it is ahead.  Of the larger ones only those with one side half as long again as the other: square ones, where it is as far
+// ahead (the line of 4,096 x 4,096), come as slices, and a program that holds them while it launches another product of that size is told so.  Up to eight rows: at 16 the two are about even, and a product that takes attention's
 // unmerged splits (which this form does not) has the bits of the one that takes them merged there.
 // Where a kernel would have to add the slices: also up to 13 M elements (36 M with up to 8 rows and a K of one round of eight waves) with a K
 // of up to 8,192 (6,144 from 13 rows on; any with up to four), but not a short K against many columns (with a
@@ -197,7 +198,7 @@ static int g_mode = 0;
 static bool handed_on(int M, int N, int K) {
   const long long elements = static_cast<long long>(N) * K;
   if (M <= 8 && elements <= 6500000 && K >= KC && (K <= 8 * KC || 2LL * K <= 3LL * N) && (N <= 8192 || N <= 16LL * K)) return true;
-  if (M > 8 || K < 8 * KC) return false;
+  if (M > 8 || K < 8 * KC || (2LL * K < 3LL * N && 2LL * N < 3LL * K)) return false;
   const bool one_round = N > 3584 && N <= 4096, two_rounds = N > 7168 && N <= 8192;
   if ((one_round && K <= 12288) || (two_rounds && K <= 4096)) return true;
   if (M <= 4 && (((N >= 2816 && N <= 4096) || two_rounds) && K <= 14336)) return true;
