@@ -325,3 +325,35 @@ def test_projection_rows_at_the_ends_of_a_wave(dtype, n, head_dim, value_dim, ro
     tol = 4e-6 if dtype == torch.float32 else 2.0 ** -7
     for a, b in ((got, want), (k, kr), (v, vr)):
         close(a, b.to(a.dtype), tol)
+
+
+@pytest.mark.parametrize("chunk", [1, 7, 8, 9, 64])
+def test_gated_recurrence_of_ragged_chunks(chunk):
+    """Chunks of less than, exactly and just over the tokens that are asked for at once, cut anywhere: against float64 token by token, 2e-5
+    for the kept state (as above; a decay is at most 1, so errors do not grow along the span)."""
+    o, g, blocks, size = ops(), torch.Generator().manual_seed(chunk), 2, 32
+    spans, c = [33, 1, 40, 71], blocks * size
+    n, slots = sum(spans), [3, 1, 4, 2]
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    u, y, x, ba, bi, lam = r(n, c), r(n, c), r(n, c), r(c), r(c), r(c)
+    wa, wi = ((torch.randn(blocks, size, size, generator=g) / size ** 0.5).bfloat16() for _ in range(2))
+    S, kept = torch.randn(len(spans) + 1, c, generator=g), r(len(spans) + 1, 3, c)
+    product = lambda m, b: torch.einsum("nbk,bok->nbo", u.double().view(n, blocks, size), m.double()).reshape(n, c) + b.double()
+    log_a = -torch.nn.functional.softplus(lam.double()) * torch.sigmoid(product(wa, ba))
+    b = torch.sqrt(-torch.expm1(2 * log_a)) * torch.sigmoid(product(wi, bi)) * u.double()
+    want_S, want, want_kept, rows, first_chunk, first = S.double(), [], kept.clone(), [], [0], 0
+    for i, (slot, length) in enumerate(zip(slots, spans)):
+        for t in range(first, first + length):
+            want_S[slot] = torch.exp(log_a[t]) * want_S[slot] + b[t]
+            want.append(want_S[slot].clone())
+        want_kept[slot] = torch.cat([kept[slot], x[first: first + length]])[-3:]
+        rows += [(i, first + t, min(chunk, length - t)) for t in range(0, length, chunk)]
+        first_chunk.append(len(rows))
+        first += length
+    dev = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    t, Sd, kd = (lambda m: m.transpose(1, 2).contiguous().cuda()), S.cuda(), kept.cuda()
+    got = o.rglru(u.cuda(), y.cuda(), x.cuda(), t(wa), ba.cuda(), t(wi), bi.cuda(), lam.cuda(), 1.0, Sd, kd, 4, _spans(spans, slots), wa=wa.cuda(), wi=wi.cuda(),
+                  chunks=dev(rows), seq_chunk0=dev(first_chunk))
+    close(Sd, want_S, 2e-5)
+    close(got, torch.stack(want) * torch.nn.functional.gelu(y.double(), approximate="tanh"), 2.0 ** -8)
+    assert torch.equal(kd.cpu(), want_kept)
