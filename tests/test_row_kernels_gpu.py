@@ -1,4 +1,4 @@
-"""Norms and activations whose threads hold one or two pieces of a row, at rows that do not fill their threads."""
+"""Kernels of a step's rows (norms, activations, slices, few-row products, experts of few pairs, heads, recurrences) at sizes that do not fill their threads."""
 import math
 
 import pytest
