@@ -237,6 +237,34 @@ def test_experts_of_few_pairs(n, top, experts, hidden, ff):
         assert torch.equal(got2[top:], got[top:])  # (its own rows: the pair's clamps drop a NaN)
 
 
+@pytest.mark.parametrize("dtype,n,top,experts", [(torch.bfloat16, 5, 2, 3), (torch.bfloat16, 40, 2, 16), (torch.bfloat16, 100, 1, 2), (torch.bfloat16, 200, 1, 2),
+                                                 (torch.float32, 5, 2, 3)])  # pairs that route themselves, tiles of 16, 64 and 128 pairs, the general form
+def test_experts_out_of_range_are_the_nearest(dtype, n, top, experts):
+    """Numbers below zero and beyond the last expert in the table: the rows that the first and the last expert give, in the same bits."""
+    o, g = ops(), torch.Generator().manual_seed(n)
+    hidden, ff = 64, 96
+    x = torch.randn(n, hidden, generator=g).to(dtype).cuda()
+    ids = torch.randint(0, 30, (n,), generator=g, dtype=torch.int32).cuda()
+    table = torch.randint(-3, experts + 4, (30, top), generator=g, dtype=torch.int32)
+    table[0, 0], table[1, 0] = -2 ** 31, 2 ** 31 - 1
+    wgu = (torch.randn(experts, 2, ff, hidden, generator=g) / hidden ** 0.5).to(dtype).cuda()
+    wd = (torch.randn(experts, hidden, ff, generator=g) / ff ** 0.5).to(dtype).cuda()
+    got = o.moe_experts(x, ids, table.cuda(), wgu, wd, "silu")
+    assert torch.equal(got, o.moe_experts(x, ids, table.clamp(0, experts - 1).cuda(), wgu, wd, "silu"))
+
+
+def test_more_experts_than_are_offered():
+    """4,097 experts are refused, of however few pairs."""
+    from yalis_amd.ops.hip import KernelError
+
+    o, bf = ops(), torch.bfloat16
+    for n in (2, 70):
+        table = torch.zeros(n, 1, dtype=torch.int32, device="cuda")
+        with pytest.raises(KernelError, match="4,096 experts"):
+            o.moe_experts(torch.zeros(n, 32, dtype=bf, device="cuda"), None, table, torch.zeros(4097, 2, 32, 32, dtype=bf, device="cuda"),
+                          torch.zeros(4097, 32, 32, dtype=bf, device="cuda"), "silu")
+
+
 def _spans(spans, slots):
     from types import SimpleNamespace
 

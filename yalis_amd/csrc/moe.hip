@@ -21,6 +21,9 @@
 #include "common.h"
 
 // ------------------------------------------------------------------------------- routing
+// an expert's number from a table; one out of range is the nearest that there is, as token ids are (it is an address later)
+__device__ __forceinline__ int expert_of(int e, int n_experts) { return min(max(e, 0), n_experts - 1); }
+
 __global__ __launch_bounds__(1024) void moe_route_kernel(
     const int32_t* __restrict__ token_ids, const int32_t* __restrict__ table, int vocab, int top, int n_experts,
     int n_pairs, int tile_rows, int32_t* __restrict__ order, int32_t* __restrict__ slot_expert,
@@ -33,7 +36,7 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(
   for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) {
     int id = token_ids != nullptr ? token_ids[i / top] : i / top;  // (no ids: the table has a row per token of the step)
     id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
-    const int e = table[static_cast<size_t>(id) * top + i % top];
+    const int e = expert_of(table[static_cast<size_t>(id) * top + i % top], n_experts);
     atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
@@ -68,7 +71,7 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(
   for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) {
     int id = token_ids != nullptr ? token_ids[i / top] : i / top;  // (no ids: the table has a row per token of the step)
     id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
-    const int e = table[static_cast<size_t>(id) * top + i % top];
+    const int e = expert_of(table[static_cast<size_t>(id) * top + i % top], n_experts);
     const int at = atomicAdd(&cnt[e], 1);
     order[at] = i;
     slot_expert[at] = e;
@@ -677,6 +680,7 @@ struct FewPairs {
   const int32_t *token_ids, *table;  // as moe_route takes them
   int vocab, top, n_pairs;
   uint32_t top_inverse;  // inverse_of(top), for top > 1
+  int n_experts;
 };
 __device__ __forceinline__ int pair_token(const FewPairs& p, int pair) { return p.top > 1 ? divide_by(pair, p.top, p.top_inverse) : pair; }
 // whether tile t is somebody's; then its expert, its pairs' count and the pair of the lane's row lane % 16 (rows beyond them repeat the last)
@@ -685,7 +689,7 @@ __device__ __forceinline__ bool few_pairs_tile(const FewPairs& p, int t, int& e,
   int id = token;
   if (p.token_ids != nullptr) id = p.token_ids[token];
   id = id < 0 ? 0 : (id >= p.vocab ? p.vocab - 1 : id);
-  const int mine = p.table[static_cast<size_t>(id) * p.top + (i - token * p.top)];
+  const int mine = expert_of(p.table[static_cast<size_t>(id) * p.top + (i - token * p.top)], p.n_experts);
   e = __builtin_amdgcn_readlane(mine, t);
   const bool with = lane < p.n_pairs && mine == e;
   const unsigned long long all = __ballot(with);
@@ -754,8 +758,9 @@ template <int FT, int WAVES, int DEPTH, bool GATED>
 __global__ __launch_bounds__(64 * WAVES) void moe_gate_up_few_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
                                                               const int32_t* __restrict__ token_ids, const int32_t* __restrict__ table, int n_pairs,
                                                               int n_groups, uint32_t groups_inverse, int top, int vocab, uint32_t top_inverse,
-                                                              int x_stride, int x_per_token, int hidden, int ff, int kind, float p0, float p1) {
-  const FewPairs pairs{token_ids, table, vocab, top, n_pairs, top_inverse};
+                                                              int x_stride, int x_per_token, int hidden, int ff, int kind, float p0, float p1,
+                                                              int n_experts) {
+  const FewPairs pairs{token_ids, table, vocab, top, n_pairs, top_inverse, n_experts};
   int t, group;
   few_pairs_place(n_groups, groups_inverse, t, group);
   if (t >= n_pairs) return;
@@ -798,8 +803,8 @@ template <int FT, int WAVES, int DEPTH>
 __global__ __launch_bounds__(64 * WAVES) void moe_down_few_kernel(const bf16_t* __restrict__ y, const bf16_t* __restrict__ w, float* __restrict__ out,
                                                            const int32_t* __restrict__ token_ids, const int32_t* __restrict__ table, int n_pairs,
                                                            int n_groups, uint32_t groups_inverse, int top, int vocab, uint32_t top_inverse, int hidden,
-                                                           int ff) {
-  const FewPairs pairs{token_ids, table, vocab, top, n_pairs, top_inverse};
+                                                           int ff, int n_experts) {
+  const FewPairs pairs{token_ids, table, vocab, top, n_pairs, top_inverse, n_experts};
   int t, group;
   few_pairs_place(n_groups, groups_inverse, t, group);
   if (t >= n_pairs) return;
@@ -834,10 +839,11 @@ extern "C" int yk_moe_few_pairs_ok(int n_pairs, int hidden, int ff, int x_stride
 
 // Both products of up to 64 pairs, bfloat16 throughout but the float32 rows that come out.  token_ids, table, vocab, top: as moe_route; x has a
 // row per token (x_per_token) or per pair; y [n_pairs, ff] scratch.
-extern "C" int yk_moe_few_pairs(const int32_t* token_ids, const int32_t* table, int vocab, int top, int n_pairs, const void* x, int x_stride,
+extern "C" int yk_moe_few_pairs(const int32_t* token_ids, const int32_t* table, int vocab, int top, int n_experts, int n_pairs, const void* x, int x_stride,
                                 int x_per_token, const void* w_gate_up, const void* w_down, int hidden, int ff, int gated, int kind, float p0,
                                 float p1, void* y, float* rows, hipStream_t stream) {
-  YK_REQUIRE(vocab >= 1 && top >= 1 && hidden > 0 && ff > 0 && x_stride >= hidden, "moe_few_pairs: bad sizes");
+  YK_REQUIRE(vocab >= 1 && top >= 1 && n_experts >= 1 && hidden > 0 && ff > 0 && x_stride >= hidden, "moe_few_pairs: bad sizes");
+  YK_REQUIRE(n_experts <= 4096, "moe_few_pairs: more than 4,096 experts");  // (as moe_route)
   YK_REQUIRE(kind >= 0 && kind < (gated ? YK_GATED_KINDS : YK_PLAIN_KINDS), "moe_few_pairs: unknown activation");
   YK_REQUIRE(yk_moe_few_pairs_ok(n_pairs, hidden, ff, x_stride), "moe_few_pairs: up to 64 pairs, sizes in multiples of 32");
   YK_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(w_down) && aligned16(y) && aligned16(rows), "moe_few_pairs: operands must be 16-byte aligned");
@@ -850,13 +856,13 @@ extern "C" int yk_moe_few_pairs(const int32_t* token_ids, const int32_t* table, 
     const int groups = (ff + 16 * GF - 1) / (16 * GF);                                                                                  \
     moe_gate_up_few_kernel<GF, GW, GD, GATED><<<static_cast<unsigned>(n_pairs * groups), 64 * GW, 0, stream>>>(                          \
         xb, wg, yb, token_ids, table, n_pairs, groups, groups > 1 ? inverse_of(groups) : 0u, top, vocab, top_inverse, x_stride, x_per_token, \
-        hidden, ff, kind, p0, p1);                                                                                                      \
+        hidden, ff, kind, p0, p1, n_experts);                                                                                           \
   }
 #define YK_DN(DF, DW, DD)                                                                                                               \
   {                                                                                                                                     \
     const int groups = (hidden + 16 * DF - 1) / (16 * DF);                                                                              \
     moe_down_few_kernel<DF, DW, DD><<<static_cast<unsigned>(n_pairs * groups), 64 * DW, 0, stream>>>(                                    \
-        yb, wd, rows, token_ids, table, n_pairs, groups, groups > 1 ? inverse_of(groups) : 0u, top, vocab, top_inverse, hidden, ff);    \
+        yb, wd, rows, token_ids, table, n_pairs, groups, groups > 1 ? inverse_of(groups) : 0u, top, vocab, top_inverse, hidden, ff, n_experts); \
   }
   // One tile of 16 features a workgroup and eight steps ahead (us of both products, 16 experts of 1,024 in width 2,048, pairs of four tokens with 6
   // distinct experts / 16 experts' pairs of 4,096 with 12: two tiles of gate rows 20.3 / 64.7, sixteen steps 19.7 / 65.2, eight waves 22.7 / 60.6, this 19.7 / 56.8).

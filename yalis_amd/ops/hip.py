@@ -197,7 +197,7 @@ _SIGNATURES = {
     ),
     "yk_moe_few_pairs_ok": ([_c_int, _c_int, _c_int, _c_int], _c_int),
     "yk_moe_few_pairs": (
-        [_vp, _vp, _c_int, _c_int, _c_int, _vp, _c_int, _c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _vp, _vp, _vp],
+        [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp, _c_int, _c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _vp, _vp, _vp],
         _c_int,
     ),
     "yk_moe_down": ([_vp, _c_int, _vp, _c_int, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _vp], _c_int),
@@ -288,7 +288,7 @@ _LATER_SIGNATURES = {
         "yk_probe_mfma_bf16": ([_c_int, _c_int, _vp, _vp], _c_int),
     },
 }
-_ABI = 29
+_ABI = 30
 
 # Rows of x up to which the hand-written matrix-core kernel runs a bfloat16 product;
 # above it the vendor library does.
@@ -2356,7 +2356,7 @@ class HipOps:
             y = torch.empty((pairs, ff), dtype=bf, device=dev)
             self._check(
                 self.lib.yk_moe_few_pairs(
-                    _ptr(token_ids), table.data_ptr(), vocab, top, pairs, x.data_ptr(), x.stride(0), int(x_top > 1), w_gate_up.data_ptr(),
+                    _ptr(token_ids), table.data_ptr(), vocab, top, experts, pairs, x.data_ptr(), x.stride(0), int(x_top > 1), w_gate_up.data_ptr(),
                     w_down.data_ptr(), hidden, ff, int(gated), kind, p0, p1, y.data_ptr(), rows.data_ptr(), self._stream(),
                 )
             )
