@@ -237,6 +237,25 @@ def test_experts_of_few_pairs(n, top, experts, hidden, ff):
         assert torch.equal(got2[top:], got[top:])  # (its own rows: the pair's clamps drop a NaN)
 
 
+@pytest.mark.parametrize("steps", [1, 4, 5, 7, 8, 9, 13, 20, 28, 29, 33, 36, 61])  # of 32: one to four waves with some, one to sixteen a wave, last waves with fewer or none
+def test_experts_of_few_pairs_at_any_depth(steps):
+    """Both products at every remainder of what a wave asks for at once: the bits of the sorted pairs' form, which walks K two steps at a time."""
+    o, g = ops(), torch.Generator(device="cuda").manual_seed(steps)
+    n, top, experts, k = 12, 2, 5, 32 * steps
+    for hidden, ff in ((k, 64), (64, k)):
+        x = torch.randn(n, hidden, device="cuda", generator=g).bfloat16()
+        table = torch.rand(n, experts, device="cuda", generator=g).argsort(-1)[:, :top].to(torch.int32).contiguous()
+        ids = torch.arange(n, dtype=torch.int32, device="cuda")
+        wgu = (torch.randn(experts, 2, ff, hidden, device="cuda", generator=g) / hidden ** 0.5).bfloat16()
+        wd = (torch.randn(experts, hidden, ff, device="cuda", generator=g) / ff ** 0.5).bfloat16()
+        got, ask = o.moe_experts(x, ids, table, wgu, wd, "silu"), o._ask
+        o._ask = lambda name, *args: 0 if name == "yk_moe_few_pairs_ok" else ask(name, *args)
+        try:
+            assert torch.equal(got, o.moe_experts(x, ids, table, wgu, wd, "silu"))
+        finally:
+            del o._ask
+
+
 @pytest.mark.parametrize("dtype,n,top,experts", [(torch.bfloat16, 5, 2, 3), (torch.bfloat16, 40, 2, 16), (torch.bfloat16, 100, 1, 2), (torch.bfloat16, 200, 1, 2),
                                                  (torch.float32, 5, 2, 3)])  # pairs that route themselves, tiles of 16, 64 and 128 pairs, the general form
 def test_experts_out_of_range_are_the_nearest(dtype, n, top, experts):

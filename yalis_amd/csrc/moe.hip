@@ -704,7 +704,10 @@ __device__ __forceinline__ bool few_pairs_tile(const FewPairs& p, int t, int& e,
 }
 
 // acc[n] += 16 rows of w[n] . 16 rows of x over n_steps steps of 32 along K, DEPTH of them asked for ahead: a unit that runs one
-// such workgroup has as many bytes in flight as its waves ask for, and two steps are 32 KiB of them.
+// such workgroup has as many bytes in flight as its waves ask for, and two steps are 32 KiB of them.  Fewer steps than DEPTH (a K of less
+// than 1,024 over four waves, and the last wave's of one that does not divide) are all asked for at once too, those beyond the last read again and unused:
+// one after the other, a wait each, both products of 16 experts' 48 pairs, us: 992 in width 2,048 56.4 (now 49.4), 1,056 56.0 (52.8), 384 in width
+// 4,096 53.4 (51.6); 14 experts' 32 pairs of 512 in width 896 18.6 (16.8).
 template <int NW, int DEPTH>
 __device__ __forceinline__ void few_pairs_product(const bf16_t* const (&w)[NW], const bf16_t* x, int n_steps, f32x4_t (&acc)[NW]) {
   MoeFrag a[DEPTH][NW], b[DEPTH];
@@ -718,11 +721,20 @@ __device__ __forceinline__ void few_pairs_product(const bf16_t* const (&w)[NW], 
     for (int n = 0; n < NW; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[slot][n].v, b[slot].v, acc[n], 0, 0, 0);
   };
   if (n_steps < DEPTH) {
-    for (int s = 0; s < n_steps; ++s) {
-      ask(0, s);
-      multiply(0);
+    if constexpr (DEPTH > 1) {
+      if (n_steps <= DEPTH / 2) return few_pairs_product<NW, DEPTH / 2>(w, x, n_steps, acc);
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) ask(d, min(d, n_steps - 1));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+#pragma unroll
+        for (int n = 0; n < NW; ++n) asm volatile("" ::"v"(a[d][n].u));  // (or the loads go under the condition, and wait there)
+        asm volatile("" ::"v"(b[d].u));
+        if (d < n_steps) multiply(d);
+      }
     }
-    return;
+    return;  // (a wave without a step)
   }
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) ask(d, d);
