@@ -11,7 +11,7 @@ from yalis_amd.ops.build import CSRC
 # The number that libraries and bindings compare when a library is loaded, and the entry points that it stands for.  Where one of
 # these changes, the number goes up (yk_abi_version in runtime.hip, _ABI in ops/hip.py): a library built before would read its
 # arguments from the wrong places.
-ENTRY_POINTS = (30, "b4f356b4df2e3909")
+ENTRY_POINTS = (31, "f92e1e712e204564")
 
 
 def prototypes():

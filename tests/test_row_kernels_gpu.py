@@ -256,6 +256,30 @@ def test_experts_of_few_pairs_at_any_depth(steps):
             del o._ask
 
 
+# both sides of every line of yk_moe_few_pairs_ok: tokens, choices a token, experts, width, ff
+@pytest.mark.parametrize("n,top,experts,hidden,ff,few", [
+    (16, 2, 17, 4096, 1024, True), (16, 2, 16, 4096, 1024, False), (16, 2, 4, 4096, 1024, True), (16, 2, 5, 4096, 1024, False),
+    (12, 2, 8, 4096, 992, True), (12, 2, 8, 4096, 1024, False), (25, 1, 8, 4096, 992, False), (16, 2, 8, 2048, 1024, True), (16, 2, 8, 2080, 1024, False), (32, 1, 2, 2048, 96, True), (33, 1, 9, 2048, 96, True),
+    (33, 1, 8, 2048, 96, False), (33, 1, 9, 2080, 96, False), (64, 1, 2, 1024, 96, True), (64, 1, 15, 1056, 96, False), (64, 1, 16, 1056, 96, True),
+    (65, 1, 33, 96, 96, False)])
+def test_which_pairs_route_themselves(n, top, experts, hidden, ff, few):
+    """The rule's answer, and the same bits in either form."""
+    o, g = ops(), torch.Generator(device="cuda").manual_seed(n + hidden)
+    x = torch.randn(n, hidden, device="cuda", generator=g).bfloat16()
+    table = torch.rand(n, experts, device="cuda", generator=g).argsort(-1)[:, :top].to(torch.int32).contiguous()
+    wgu = (torch.randn(experts, 2, ff, hidden, device="cuda", generator=g) / hidden ** 0.5).bfloat16()
+    wd = (torch.randn(experts, hidden, ff, device="cuda", generator=g) / ff ** 0.5).bfloat16()
+    assert bool(o._ask("yk_moe_few_pairs_ok", n * top, experts, hidden, ff, hidden)) == few
+    forms, ask = [], o._ask
+    try:
+        for take in (0, int(n * top <= 64)):
+            o._ask = lambda name, *args: take if name == "yk_moe_few_pairs_ok" else ask(name, *args)
+            forms.append(o.moe_experts(x, None, table, wgu, wd, "silu", input_per_token=True))
+    finally:
+        del o._ask
+    assert torch.equal(*forms) and torch.equal(forms[0], o.moe_experts(x, None, table, wgu, wd, "silu", input_per_token=True))
+
+
 @pytest.mark.parametrize("dtype,n,top,experts", [(torch.bfloat16, 5, 2, 3), (torch.bfloat16, 40, 2, 16), (torch.bfloat16, 100, 1, 2), (torch.bfloat16, 200, 1, 2),
                                                  (torch.float32, 5, 2, 3)])  # pairs that route themselves, tiles of 16, 64 and 128 pairs, the general form
 def test_experts_out_of_range_are_the_nearest(dtype, n, top, experts):

@@ -844,9 +844,19 @@ __global__ __launch_bounds__(64 * WAVES) void moe_down_few_kernel(const bf16_t* 
   }
 }
 
-// Whether the products of so many pairs route themselves.
-extern "C" int yk_moe_few_pairs_ok(int n_pairs, int hidden, int ff, int x_stride) {
-  return n_pairs >= 1 && n_pairs <= 64 && yk_moe_mfma_ok(hidden, ff, x_stride) ? 1 : 0;
+static bool few_pairs_fit(int n_pairs, int hidden, int ff, int x_stride) { return n_pairs >= 1 && n_pairs <= 64 && yk_moe_mfma_ok(hidden, ff, x_stride); }
+
+// Whether the products of so many pairs route themselves.  That saves a launch and its list, some 10 us, and costs a look at the pairs for
+// every pair's tile (those that are not the first of 16 of an expert's are nobody's) and tiles of 16 features where sorted pairs take 32
+// and 64: the wider the rows and the more pairs an expert has, the less is left.  Parts of the sorted form's time at widths of 1,024, 2,048, 3,072 and
+// 4,096, ff 256 to 2,048, 2 to 32 experts: up to 32 pairs in width 2,048 and less 0.35 to 1.03, beyond with up to four experts 0.38 to 1.03 and with fewer
+// than two pairs an expert 0.59 to 1.03, with more 1.0 to 1.12 (32 pairs of 16 experts of 384 in 4,096 1.12, of 8 of 1,024 1.11; 24 pairs of 8 of
+// 256 and 512 0.63 and 0.86); 48 and 64 pairs in width 1,024 0.58 to 1.01, in 2,048 0.82 to 1.04 with up to four pairs an expert and up to 1.17 with more
+// (8 experts of 2,048; 2 of 512 1.10), in 3,072 and 4,096 0.65 to 1.21.
+extern "C" int yk_moe_few_pairs_ok(int n_pairs, int n_experts, int hidden, int ff, int x_stride) {
+  if (!few_pairs_fit(n_pairs, hidden, ff, x_stride)) return 0;
+  if (n_pairs <= 32) return hidden <= 2048 || n_experts <= 4 || n_pairs < 2 * n_experts || (ff < 1024 && n_pairs <= 24);
+  return hidden <= 1024 || (hidden <= 2048 && n_pairs <= 4 * n_experts);
 }
 
 // Both products of up to 64 pairs, bfloat16 throughout but the float32 rows that come out.  token_ids, table, vocab, top: as moe_route; x has a
@@ -857,7 +867,7 @@ extern "C" int yk_moe_few_pairs(const int32_t* token_ids, const int32_t* table, 
   YK_REQUIRE(vocab >= 1 && top >= 1 && n_experts >= 1 && hidden > 0 && ff > 0 && x_stride >= hidden, "moe_few_pairs: bad sizes");
   YK_REQUIRE(n_experts <= 4096, "moe_few_pairs: more than 4,096 experts");  // (as moe_route)
   YK_REQUIRE(kind >= 0 && kind < (gated ? YK_GATED_KINDS : YK_PLAIN_KINDS), "moe_few_pairs: unknown activation");
-  YK_REQUIRE(yk_moe_few_pairs_ok(n_pairs, hidden, ff, x_stride), "moe_few_pairs: up to 64 pairs, sizes in multiples of 32");
+  YK_REQUIRE(few_pairs_fit(n_pairs, hidden, ff, x_stride), "moe_few_pairs: up to 64 pairs, sizes in multiples of 32");
   YK_REQUIRE(aligned16(x) && aligned16(w_gate_up) && aligned16(w_down) && aligned16(y) && aligned16(rows), "moe_few_pairs: operands must be 16-byte aligned");
   const uint32_t top_inverse = top > 1 ? inverse_of(top) : 0u;
   const bf16_t *xb = static_cast<const bf16_t*>(x), *wg = static_cast<const bf16_t*>(w_gate_up), *wd = static_cast<const bf16_t*>(w_down);

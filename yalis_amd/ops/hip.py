@@ -195,7 +195,7 @@ _SIGNATURES = {
          _c_float, _vp, _c_int, _vp],
         _c_int,
     ),
-    "yk_moe_few_pairs_ok": ([_c_int, _c_int, _c_int, _c_int], _c_int),
+    "yk_moe_few_pairs_ok": ([_c_int, _c_int, _c_int, _c_int, _c_int], _c_int),
     "yk_moe_few_pairs": (
         [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp, _c_int, _c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _vp, _vp, _vp],
         _c_int,
@@ -288,7 +288,7 @@ _LATER_SIGNATURES = {
         "yk_probe_mfma_bf16": ([_c_int, _c_int, _vp, _vp], _c_int),
     },
 }
-_ABI = 30
+_ABI = 31
 
 # Rows of x up to which the hand-written matrix-core kernel runs a bfloat16 product;
 # above it the vendor library does.
@@ -2350,7 +2350,7 @@ class HipOps:
         # tiles of 128 or 64 pairs where an expert has that many on average, else of 16
         tile_rows = 128 if pairs >= 96 * experts else (64 if pairs >= 48 * experts else 16)
         bf = torch.bfloat16
-        if (tile_rows == 16 and x.dtype == bf and w_gate_up.dtype == bf and w_down.dtype == bf and self._ask("yk_moe_few_pairs_ok", pairs, hidden, ff, x.stride(0))
+        if (tile_rows == 16 and x.dtype == bf and w_gate_up.dtype == bf and w_down.dtype == bf and self._ask("yk_moe_few_pairs_ok", pairs, experts, hidden, ff, x.stride(0))
                 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0 and w_down.data_ptr() % 16 == 0):
             # few pairs route themselves: no kernel before the products
             y = torch.empty((pairs, ff), dtype=bf, device=dev)
