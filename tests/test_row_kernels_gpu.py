@@ -205,6 +205,20 @@ def test_few_rows_in_one_workgroup_by_rows_of_x(m, n, k):
     assert torch.equal(got, torch.stack([w[:, (r * 37 + k // 2) % k] for r in range(m)]))
 
 
+def test_few_rows_far_apart():
+    """Rows of x that reach over 2^31 elements: the bits of the same rows side by side, as a product, with a bias and with pairs."""
+    o, g, bf = ops(), torch.Generator(device="cuda").manual_seed(3), torch.bfloat16
+    m, n, k, apart = 3, 1024, 264, 2 ** 30 + 8
+    wide = torch.empty(m, apart, dtype=bf, device="cuda")
+    wide[:, :k] = torch.randn(m, k, device="cuda", generator=g)
+    x, w, bias = wide[:, :k], torch.randn(n, k, device="cuda", generator=g).to(bf), torch.randn(n, device="cuda", generator=g)
+    near = x.contiguous()
+    for out in (torch.float32, bf):
+        assert torch.equal(o.linear(x, w, out), o.linear(near, w, out)) and torch.equal(o.gemm_cols(x, w, out), o.gemm_cols(near, w, out))
+        assert torch.equal(o.linear(x, w, out, bias=bias), o.linear(near, w, out, bias=bias))
+    assert torch.equal(o.gate_up_act(x, w, 8, "silu", bf), o.gate_up_act(near, w, 8, "silu", bf))
+
+
 @pytest.mark.parametrize("n,top,experts", [(1, 1, 2), (1, 4, 4), (4, 2, 16), (5, 3, 7), (16, 4, 32), (33, 1, 2), (64, 1, 2), (21, 3, 3)])
 @pytest.mark.parametrize("hidden,ff", [(32, 32), (96, 64), (160, 288), (1056, 1024), (2048, 96)])  # fewer steps of 32 than waves, than are asked for ahead, more
 def test_experts_of_few_pairs(n, top, experts, hidden, ff):

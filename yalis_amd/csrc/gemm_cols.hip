@@ -237,7 +237,15 @@ extern "C" int yk_gemm_cols(const void* x, const void* w, void* y, int y_dtype, 
   YK_REQUIRE(!gated || (N % 16 == 0 && kind >= 0 && kind < YK_GATED_KINDS), "gemm_cols: a gated product needs N % 16 == 0 and a known pair");
   YK_REQUIRE(!bias || bias_dtype == YK_F32 || bias_dtype == YK_BF16, "gemm_cols: unsupported bias dtype");
   if (M == 0) return 0;
-  YK_REQUIRE(static_cast<long long>(M - 1) * ldx + K < 1ll << 31, "gemm_cols: the rows of x must lie within 4 GiB");
+  if (static_cast<long long>(M - 1) * ldx + K >= 1ll << 31) {  // the kernel's offsets into x have 32 bits: rows that far apart go one by one (the same sums)
+    for (int m = 0; m < M; ++m) {
+      const int rc = yk_gemm_cols(static_cast<const bf16_t*>(x) + static_cast<size_t>(m) * ldx, w,
+                                  static_cast<char*>(y) + static_cast<size_t>(m) * ldy * (y_dtype == YK_F32 ? 4 : 2), y_dtype, 1, N, K, ldx, ldw, ldy, bias,
+                                  bias_dtype, gated, kind, p0, p1, stream);
+      if (rc) return rc;
+    }
+    return 0;
+  }
   const Finish f{gated, kind, p0, p1, bias, bias_dtype == YK_F32};
   const unsigned tiles = (N + 15) / 16;
   const int n_chunks = (K + KC - 1) / KC;
