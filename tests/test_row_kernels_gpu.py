@@ -116,6 +116,22 @@ CONSUMERS = {
 }
 
 
+# rows and widths whose pieces of four end in a workgroup, a wave and a row; 64 rows take slices by rows, more of them by pieces; 6 and 258 the general kernel
+@pytest.mark.parametrize("rows", [1, 3, 64, 65, 1027])
+@pytest.mark.parametrize("inter,group", [(4, 0), (6, 0), (96, 4), (256, 0), (258, 0), (1020, 0), (1028, 4), (1028, 0), (3076, 0)])
+def test_gated_pairs_of_any_rows(rows, inter, group):
+    """The plain pairs of the slices' sum (float32 exp: 2e-6; rounded once: 2^-8), and the bits of that sum itself at any number of slices."""
+    o, g = ops(), torch.Generator().manual_seed(rows + inter)
+    for slices in (1, 2, 3, 8, 9):
+        parts = torch.randn(slices, rows, 2 * inter, generator=g)
+        for dtype in (torch.float32, torch.bfloat16):
+            whole = in_order(parts, dtype)
+            got = o.gated_act(SplitSum(parts.cuda(), dtype) if slices > 1 else whole.cuda(), "silu", dtype, group=group)
+            assert torch.equal(got, o.gated_act(whole.cuda(), "silu", dtype, group=group))
+            assert torch.equal(got, o.gated_act(whole.to(dtype).cuda(), "silu", dtype, group=group))
+            close(got, R.gated_act_general(whole, "silu", dtype, group), 2e-6 if dtype == torch.float32 else 2.0 ** -8)
+
+
 @pytest.mark.parametrize("consumer", CONSUMERS)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,width", [(3, 4), (3, 516), (2, 4096), (2, 6148), (1025, 520)])  # one piece of a row a thread, two and four
