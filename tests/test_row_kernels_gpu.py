@@ -112,8 +112,25 @@ CONSUMERS = {
     "sandwich_norm": lambda o, res, d, w, rows: o.sandwich_norm(res, d, (w, w, 1e-5, True), 0.5, (w, None, 1e-5, False), None, torch.float32),
     "sandwich_norm rows": lambda o, res, d, w, rows: o.sandwich_norm(res, d, None, 1.0, (w, w, 1e-5, True), rows, torch.bfloat16),
     "activation": lambda o, res, d, w, rows: o.activation(d, "relu2", torch.float32),
-    "gated_act": lambda o, res, d, w, rows: o.gated_act(d, "silu", torch.float32) if d.shape[1] % 8 == 0 else torch.zeros(1),
+    "gated_act": lambda o, res, d, w, rows: o.gated_act(d, "silu", torch.float32),
 }
+
+
+# rows that fill the chip (one piece a thread and two), rows of three and of four pieces
+@pytest.mark.parametrize("consumer,n,width", [(c, n, w) for c in CONSUMERS for n, w in ((300, 1028), (1025, 1028), (1025, 256))]
+                         + [(c, 2, w) for c in ("add_rmsnorm", "gather_add_rmsnorm", "rmsnorm", "norm_add") for w in (10244, 14340)]
+                         + [(c, 2, 16384) for c in ("add_rmsnorm", "gather_add_rmsnorm", "rmsnorm")])
+def test_slices_of_many_and_wide_rows(consumer, n, width):
+    """As above where fewer slices are asked for at once: the bits of the sum itself."""
+    o, g = ops(), torch.Generator(device="cuda").manual_seed(width + n)
+    call, w = CONSUMERS[consumer], torch.rand(width, device="cuda", generator=g) + 0.5
+    rows = torch.tensor([n - 1, 0, n // 2], dtype=torch.int32, device="cuda")
+    for slices in (2, 3, 4, 5, 8, 9):
+        t, res = torch.randn(slices, n, width, device="cuda", generator=g), torch.randn(n, width, device="cuda", generator=g)
+        for dtype in (torch.float32, torch.bfloat16):
+            first, second = res.clone(), res.clone()
+            got, want = call(o, first, SplitSum(t, dtype), w, rows), call(o, second, in_order(t, dtype), w, rows)
+            assert same(got, want) and same(first, second), slices
 
 
 # rows and widths whose pieces of four end in a workgroup, a wave and a row; 64 rows take slices by rows, more of them by pieces; 6 and 258 the general kernel

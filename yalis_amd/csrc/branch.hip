@@ -59,13 +59,13 @@ __global__ __launch_bounds__(256) void norm_add_kernel(
 // to memory and back each way.  Behind copies of 16 MB and of its input in a replayed graph, four rows of 2,048 in bfloat16 alone / with two expert
 // rows, us: with 256 threads whose loads waited one for another 3.6 / 4.6, now 2.0 / 2.3.
 constexpr uint32_t ROW_ROUND = 1u << 16, ROW_UNIT = 1u << 17;  // `how`: bits 0-15 slices; 19-23 waves
-template <typename TS, typename TW, int P>
+template <typename TS, typename TW, int P, SlicesAtOnce HOW>
 __global__ __launch_bounds__(1024) void norm_add_vec_kernel(float* __restrict__ residual, const TS* __restrict__ src,
                                                             const float* __restrict__ pairs, const TW* __restrict__ w,
                                                             bf16_t* __restrict__ out, int width, uint32_t how, int top,
                                                             uint32_t split_stride, float pair_weight, float eps) {
   __shared__ float scratch[16];
-  constexpr int G = P == 1 ? 8 : 4, GS = sizeof(TS) == 2 ? 1 : G;  // expert rows and slices asked for at once
+  constexpr int G = P == 4 ? 1 : HOW == kFewRows ? 8 / P : slices_at_once<HOW, P>, GS = sizeof(TS) == 2 ? 1 : G;  // expert rows and slices asked for at once
   const int n_splits = how & 0xffffu, waves = (how >> 19) & 31, round_sum = (how & ROW_ROUND) != 0;
   const size_t n = blockIdx.x;
   float4 rs[P];
@@ -89,14 +89,14 @@ __global__ __launch_bounds__(1024) void norm_add_vec_kernel(float* __restrict__ 
   for (int k = 0; k < P; ++k) v[k] = es[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   if (src != nullptr) {
     join_slices<GS, P, TS>(d, n_splits, v);
-    join_rest<GS, P, TS>(p, at, n_splits, split_stride, v);
+    if constexpr (HOW != kOneSlice || P == 4) join_rest<GS, P, TS>(p, at, n_splits, split_stride, v);
 #pragma unroll
     for (int k = 0; k < P; ++k)
       v[k] = make_float4(as_output(v[k].x, round_sum), as_output(v[k].y, round_sum), as_output(v[k].z, round_sum), as_output(v[k].w, round_sum));
   }
   if (pairs != nullptr) {
     join_slices<G, P, float>(e, top, es);
-    join_rest<G, P, float>(q, at, top, width, es);
+    if constexpr (HOW != kOneSlice || P == 4) join_rest<G, P, float>(q, at, top, width, es);
 #pragma unroll
     for (int k = 0; k < P; ++k)
       v[k] = make_float4(fmaf(pair_weight, es[k].x, v[k].x), fmaf(pair_weight, es[k].y, v[k].y), fmaf(pair_weight, es[k].z, v[k].z),
@@ -157,15 +157,20 @@ extern "C" int yk_norm_add(float* residual, const void* src, int src_dtype, int 
   const int pieces = (width / 4 + threads - 1) / threads;
   const uint32_t how = static_cast<uint32_t>(n_splits & 0xffff) | (round_sum ? ROW_ROUND : 0u) | (unit_offset ? ROW_UNIT : 0u) |
                        static_cast<uint32_t>(threads / 64) << 19;
-#define YK_VEC(TS, TW, P)                                                                                    \
-  norm_add_vec_kernel<TS, TW, P><<<n_rows, threads, 0, stream>>>(                                            \
+  const SlicesAtOnce at_once = slices_how(std::max(n_splits, pairs ? top : 0), n_rows);
+#define YK_VEC(TS, TW, P, HOW)                                                                               \
+  norm_add_vec_kernel<TS, TW, P, HOW><<<n_rows, threads, 0, stream>>>(                                            \
       residual, static_cast<const TS*>(src), pairs, static_cast<const TW*>(w), static_cast<bf16_t*>(out), width, how, top, \
       static_cast<uint32_t>(stride), pair_weight, eps)
 #define YK_CASE(SD, TS, WD, TW)                                                                            \
   if ((src == nullptr || src_dtype == SD) && w_dtype == WD) {                                                \
-    if (vec && pieces <= 1) YK_VEC(TS, TW, 1);                                                               \
-    else if (vec && pieces <= 2) YK_VEC(TS, TW, 2);                                                          \
-    else if (vec) YK_VEC(TS, TW, 4);                                                                         \
+    if (vec && pieces <= 1 && at_once == kOneSlice) YK_VEC(TS, TW, 1, kOneSlice);                            \
+    else if (vec && pieces <= 1 && at_once == kManyRows) YK_VEC(TS, TW, 1, kManyRows);                       \
+    else if (vec && pieces <= 1) YK_VEC(TS, TW, 1, kFewRows);                                                \
+    else if (vec && pieces <= 2 && at_once == kOneSlice) YK_VEC(TS, TW, 2, kOneSlice);                       \
+    else if (vec && pieces <= 2 && at_once == kManyRows) YK_VEC(TS, TW, 2, kManyRows);                       \
+    else if (vec && pieces <= 2) YK_VEC(TS, TW, 2, kFewRows);                                                \
+    else if (vec) YK_VEC(TS, TW, 4, kOneSlice); /* (one at a time: what the registers hold) */               \
     else                                                                                                     \
       norm_add_kernel<TS, TW, bf16_t><<<n_rows, 256, lds, stream>>>(                                         \
           residual, static_cast<const TS*>(src), n_splits, stride, round_sum, pairs, top, pair_weight,       \
@@ -226,7 +231,7 @@ __device__ __forceinline__ float4 scaled4(float4 a, float s) { return make_float
 // eight slices / two bfloat16 terms with their own norms, us: with loads that waited one for another 2.3 / 3.3 / 3.9, now 2.2 / 3.1 / 3.1.
 // `how`: bits 0-7 and 8-15 the terms' slices; 19-23 waves; and the bits below
 constexpr uint32_t SUM_ROUND_A = 1u << 16, SUM_ROUND_B = 1u << 17, SUM_UNIT = 1u << 18, SUM_AW = 1u << 24, SUM_BW = 1u << 25, SUM_CW = 1u << 26;
-template <typename TW, bool A16, int B, int P>
+template <typename TW, bool A16, int B, int P, SlicesAtOnce HOW>
 __global__ __launch_bounds__(1024) void sum_norm_vec_kernel(float* __restrict__ residual, const void* __restrict__ a_src,
                                                             const void* __restrict__ b_src, const TW* __restrict__ w,
                                                             bf16_t* __restrict__ out, int width, uint32_t how, uint32_t stride,
@@ -235,7 +240,7 @@ __global__ __launch_bounds__(1024) void sum_norm_vec_kernel(float* __restrict__ 
                                                             float b_eps) {
   using TA = std::conditional_t<A16, bf16_t, float>;
   using TB = std::conditional_t<B == 2, bf16_t, float>;
-  constexpr int GA = A16 ? 1 : P == 1 ? 8 : 4, GB = B != 1 ? 1 : P == 1 ? 8 : 4;  // slices asked for at once
+  constexpr int G = HOW == kFewRows ? 8 : HOW == kManyRows ? 4 : 1, GA = A16 ? 1 : G, GB = B != 1 ? 1 : G;  // slices asked for at once
   __shared__ float scratch[3][16];
   const int na = how & 0xff, nb = (how >> 8) & 0xff, waves = (how >> 19) & 31;
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(1024) void sum_norm_vec_kernel(float* __restrict__ 
 #pragma unroll
     for (int k = 0; k < P; ++k) s[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     join_slices<G, P, T>(d, slices, s);
-    join_rest<G, P, T>(p, at, slices, stride, s);
+    if constexpr (HOW != kOneSlice) join_rest<G, P, T>(p, at, slices, stride, s);
     if constexpr (sizeof(T) == 4) {
 #pragma unroll
       for (int k = 0; k < P; ++k)
@@ -393,17 +398,21 @@ extern "C" int yk_sum_norm(float* residual, const void* a_src, int a_dtype, int 
   const bool vec = width % 4 == 0 && width <= 4096 && al(residual) && al(a_src) && al(b_src) && al(a_w) && al(b_w) && al(channel_w) &&
                    al(w) && al(out) && a_splits <= 255 && b_splits <= 255 && stride < size_t{1} << 32;
   // a piece a thread for few rows, two where rows fill the chip (eight rows of 2,048: 6.2 -> 4.2 us with twice the threads)
-  const int pieces = n_rows < 1024 ? 1 : 2, threads = (width / 4 + 64 * pieces - 1) / (64 * pieces) * 64;
+  const int threads = n_rows >= 1024 ? (width / 4 + 127) / 128 * 64 : (width / 4 + 63) / 64 * 64, pieces = 4 * threads < width ? 2 : 1;
   const uint32_t how = static_cast<uint32_t>(a_splits & 0xff) | static_cast<uint32_t>(b_splits & 0xff) << 8 | (a_round ? SUM_ROUND_A : 0u) |
                        (b_round ? SUM_ROUND_B : 0u) | (unit_offset ? SUM_UNIT : 0u) | static_cast<uint32_t>(threads / 64) << 19 |
                        (a_w ? SUM_AW : 0u) | (has_b && b_w ? SUM_BW : 0u) | (channel_w ? SUM_CW : 0u);
-#define YK_VEC(TW, A16, B, P)                                                                                              \
-  sum_norm_vec_kernel<TW, A16, B, P><<<n_rows, threads, 0, stream>>>(                                                      \
+  const SlicesAtOnce at_once = slices_how(std::max(a_splits, has_b ? b_splits : 1), n_rows);
+#define YK_VEC(TW, A16, B, P, HOW)                                                                                         \
+  sum_norm_vec_kernel<TW, A16, B, P, (A16 && B != 1 ? kOneSlice : HOW)><<<n_rows, threads, 0, stream>>>(                   \
       residual, a_src, b_src, static_cast<const TW*>(w), static_cast<bf16_t*>(out), width, how, static_cast<uint32_t>(stride), residual_scale, \
       static_cast<const TW*>(a_w), static_cast<const TW*>(b_w), static_cast<const TW*>(channel_w), branch_scale, eps, a_eps, b_eps)
-#define YK_VEC_P(TW, A16, B)              \
-  if (pieces == 1) YK_VEC(TW, A16, B, 1); \
-  else YK_VEC(TW, A16, B, 2)
+#define YK_VEC_P(TW, A16, B)                                                         \
+  if (pieces == 1 && at_once == kOneSlice) YK_VEC(TW, A16, B, 1, kOneSlice);         \
+  else if (pieces == 1 && at_once == kManyRows) YK_VEC(TW, A16, B, 1, kManyRows);    \
+  else if (pieces == 1) YK_VEC(TW, A16, B, 1, kFewRows);                             \
+  else if (at_once == kOneSlice) YK_VEC(TW, A16, B, 2, kOneSlice);                   \
+  else YK_VEC(TW, A16, B, 2, kManyRows) /* (1,024 rows and more) */
 #define YK_VEC_B(TW, A16)                 \
   if (!has_b) { YK_VEC_P(TW, A16, 0); }   \
   else if (tb.bf16) { YK_VEC_P(TW, A16, 2); } \

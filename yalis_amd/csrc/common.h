@@ -211,13 +211,18 @@ __device__ __forceinline__ void join_rest(const T* p, const uint32_t (&at)[IT], 
     }
   }
 }
-// slices in flight at a time for IT pieces a thread: what the registers hold
-template <typename T, int IT>
-constexpr int slices_at_once = sizeof(T) == 2 ? 1 : IT == 1 ? 16 : IT == 2 ? 8 : 4;
-// The sum over n >= 1 slices of IT pieces of four values, `at` elements from p.
-template <int IT, typename T>
+// Slices asked for at a time by a kernel with IT pieces a thread, where rows are few and where they fill the chip.  Few rows are bound by their waits,
+// many by how many waves a unit holds: registers of slices that are not there, or more than a workgroup of 1,024 threads has (128), cost more
+// than waits.  With the registers of many slices everywhere / now, float32 rows, us: one row of 10,240 and its residual's norm (spilled) 8.2 / 3.9, 2,048 of
+// them 86 / 43, 500 of 8,192 9.7 / 7.7, 2,048 normed alone 21.4 / 17.0; 1,023 rows of 4,096 as two terms 15.8 / 11.7.
+enum SlicesAtOnce { kOneSlice, kManyRows, kFewRows };
+template <SlicesAtOnce HOW, int IT>
+constexpr int slices_at_once = HOW == kOneSlice ? 1 : HOW == kManyRows ? (IT == 1 ? 4 : 2) : (IT == 1 ? 16 : 8);
+inline SlicesAtOnce slices_how(int n_splits, size_t n_rows) { return n_splits <= 1 ? kOneSlice : n_rows > 256 ? kManyRows : kFewRows; }
+// The sum over n >= 1 slices (kOneSlice: one) of IT pieces of four values, `at` elements from p.
+template <SlicesAtOnce HOW, int IT, typename T>
 __device__ __forceinline__ void sum_slices(const T* p, const uint32_t (&at)[IT], int n, size_t stride, float4 (&s)[IT]) {
-  constexpr int SL = slices_at_once<T, IT>;
+  constexpr int SL = slices_at_once<HOW, IT>;
 #pragma unroll
   for (int k = 0; k < IT; ++k) s[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   do {
@@ -226,7 +231,7 @@ __device__ __forceinline__ void sum_slices(const T* p, const uint32_t (&at)[IT],
     join_slices<SL, IT, T>(d, n, s);
     p += SL * stride;
     n -= SL;
-  } while (sizeof(T) == 4 && n > 0);  // (slices are float32)
+  } while (SL > 1 && n > 0);
 }
 // Arguments that did not come with the launch, asked for here and not where they are first used, one wait after the other.
 __device__ __forceinline__ void arguments_now(const void* a, const void* b = nullptr, const void* c = nullptr, const void* d = nullptr) {

@@ -257,9 +257,9 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ residual, const TD* __res
 // one row of 2,048 2.58 / 1.90, with 8 slices 3.33 / 2.60, 16 4.35 / 3.24; eight rows 2.85 / 1.88, 3.61 / 2.63, 4.71 / 3.26; eight rows of 4,096 3.65 / 2.39, with 8 slices
 // 4.32 / 3.48.
 // `how` (one word, so that the arguments every row needs fit what comes with the launch): the bits below.
-constexpr int NORM_IT_MAX = 8;
+constexpr int NORM_IT_MAX = 4;
 constexpr uint32_t NORM_ROUND = 1u << 16, NORM_UNIT = 1u << 17, NORM_ROW = 1u << 18;  // bits 0-15: slices (0: no delta); 19-23: waves
-template <typename TD, typename TW, typename TO, int NORM_IT, bool FRESH>
+template <typename TD, typename TW, typename TO, int NORM_IT, bool FRESH, SlicesAtOnce HOW>
 __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(
     float* __restrict__ residual, const TD* __restrict__ delta, const TW* __restrict__ weight, TO* __restrict__ out, int width,
     uint32_t how, uint32_t split_stride, float eps, const int32_t* __restrict__ rows, const int32_t* __restrict__ table_ids,
@@ -282,7 +282,26 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(
   }
   if (FRESH || n_splits > 0) {
     float4 ds[NORM_IT];
-    sum_slices<NORM_IT, TD>(del, at, n_splits, split_stride, ds);
+    if constexpr (NORM_IT < 3 || HOW == kOneSlice) {
+      sum_slices<HOW, NORM_IT, TD>(del, at, n_splits, split_stride, ds);
+    } else {
+      // rows of more than 8,192: four slices of a piece at a time, and none of pieces that the row does not have (they are up to half of
+      // them; 8 slices of 10,240 5.8 us, with what is beyond the row read again 7.1)
+#pragma unroll
+      for (int it = 0; it < NORM_IT; ++it) ds[it] = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int s0 = 0; s0 < n_splits; s0 += 4) {
+#pragma unroll
+        for (int it = 0; it < NORM_IT; ++it) {
+          if ((static_cast<int>(threadIdx.x) + it * 64 * waves) * 4 >= width) continue;
+          float4 d[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) d[j] = four_at<TD>(del + static_cast<size_t>(min(s0 + j, n_splits - 1)) * split_stride + at[it]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (s0 + j < n_splits) ds[it].x += d[j].x, ds[it].y += d[j].y, ds[it].z += d[j].z, ds[it].w += d[j].w;
+        }
+      }
+    }
 #pragma unroll
     for (int it = 0; it < NORM_IT; ++it) {
       v[it].x += as_output(ds[it].x, round_sum);
@@ -333,7 +352,7 @@ static int launch_add_rmsnorm(float* residual, const void* delta, int n_splits, 
   const bool aligned = width % 4 == 0 && reinterpret_cast<uintptr_t>(residual) % 16 == 0 && reinterpret_cast<uintptr_t>(add_row) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(delta) % 16 == 0 && reinterpret_cast<uintptr_t>(weight) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(out) % 16 == 0 && split_stride % 4 == 0;
-  if (aligned && width <= 4 * NORM_IT_MAX * 512 && n_splits < 1 << 16 && split_stride < size_t{1} << 32) {
+  if (aligned && width <= 4 * NORM_IT_MAX * 1024 && n_splits < 1 << 16 && split_stride < size_t{1} << 32) {
     // one four-wide chunk per thread where the row allows (faster than two at 8 rows), at most
     // 1,024 threads; with rows enough to fill the GPU several times over, two chunks per thread:
     // twice the rows are in flight on a compute unit and a row's sum meets half the waves
@@ -344,17 +363,22 @@ static int launch_add_rmsnorm(float* residual, const void* delta, int n_splits, 
     const uint32_t how = (delta ? static_cast<uint32_t>(n_splits) : 0u) | (round_sum ? NORM_ROUND : 0u) | (unit_offset ? NORM_UNIT : 0u) |
                          (add_row ? NORM_ROW : 0u) | static_cast<uint32_t>(threads / 64) << 19;
     const bool fresh = table_ids || !residual;
-#define YK_NORM(IT, FRESH)                                                                                                         \
-    add_rmsnorm_vec_kernel<TD, TW, TO, IT, FRESH><<<n_rows, threads, 0, stream>>>(                                                 \
+    const SlicesAtOnce at_once = slices_how(n_splits, n_rows);
+#define YK_NORM(IT, FRESH, HOW)                                                                                                    \
+    add_rmsnorm_vec_kernel<TD, TW, TO, IT, FRESH, HOW><<<n_rows, threads, 0, stream>>>(                                            \
         residual, static_cast<const TD*>(delta), static_cast<const TW*>(weight), static_cast<TO*>(out), width, how,                \
         static_cast<uint32_t>(split_stride), eps, rows, table_ids, table_rows, add_row)
-#define YK_NORM_IT(IT)             \
-    if (fresh) YK_NORM(IT, true);  \
-    else YK_NORM(IT, false)
-    if (pieces <= 1) YK_NORM_IT(1);
-    else if (pieces <= 2) YK_NORM_IT(2);
-    else if (pieces <= 4) YK_NORM_IT(4);
-    else YK_NORM_IT(8);
+#define YK_NORM_HOW(IT, FRESH)                                         \
+    if (sizeof(TD) == 2 || at_once == kOneSlice) YK_NORM(IT, FRESH, kOneSlice); /* (slices are float32) */ \
+    else if (at_once == kManyRows) YK_NORM(IT, FRESH, (sizeof(TD) == 2 ? kOneSlice : kManyRows)); \
+    else YK_NORM(IT, FRESH, (sizeof(TD) == 2 ? kOneSlice : IT == 4 ? kManyRows : kFewRows))
+#define YK_NORM_IT(IT)                   \
+    if (fresh) { YK_NORM_HOW(IT, true); } \
+    else { YK_NORM_HOW(IT, false); }
+    if (pieces <= 1) { YK_NORM_IT(1) }
+    else if (pieces <= 2) { YK_NORM_IT(2) }
+    else { YK_NORM_IT(4) }
+#undef YK_NORM_HOW
 #undef YK_NORM_IT
 #undef YK_NORM
   } else {
@@ -736,7 +760,7 @@ __global__ __launch_bounds__(256) void gated_act_slices_kernel(const float* __re
   const uint32_t gate = gate_col(j, inter, group);
   const uint32_t at[2] = {gate, gate + static_cast<uint32_t>(up_offset(inter, group))};
   float4 s[2];
-  sum_slices<2, float>(gu + static_cast<size_t>(blockIdx.x) * 2 * inter, at, n_splits, split_stride, s);
+  sum_slices<kFewRows, 2, float>(gu + static_cast<size_t>(blockIdx.x) * 2 * inter, at, n_splits, split_stride, s);
   const float4 y = gated_four(s[0], s[1], round_sum, act, p0, p1);
   if (first < static_cast<uint32_t>(inter)) put_four<TO>(out + static_cast<size_t>(blockIdx.x) * inter + j, y);
 }

@@ -628,7 +628,7 @@ __global__ __launch_bounds__(256) void reduce_splits_vec_kernel(const float* __r
   const uint32_t first = blockIdx.x * 256, i = min(first + threadIdx.x, pieces - 1);
   const uint32_t at[1] = {4 * (i - first)};
   float4 v[1];
-  sum_slices<1, float>(part + 4 * static_cast<size_t>(first), at, splits, 4 * static_cast<size_t>(pieces), v);
+  sum_slices<kFewRows, 1, float>(part + 4 * static_cast<size_t>(first), at, splits, 4 * static_cast<size_t>(pieces), v);
   if (first + threadIdx.x < pieces) put_four<TO>(y + static_cast<size_t>(i / per_row) * ldy + 4 * (i % per_row), v[0]);
 }
 

@@ -116,13 +116,13 @@ __device__ __forceinline__ float4 piece_norm(float4 v, NormStats st, float4 w, f
 // `how`: bits 0-15 slices; 19-23 waves; and these
 constexpr uint32_t SN_ROUND = 1u << 16, SN_CENTER_A = 1u << 17, SN_CENTER_B = 1u << 18, SN_ROWS = 1u << 24, SN_BIAS_A = 1u << 25,
                    SN_BIAS_B = 1u << 26;
-template <typename TS, typename TW, typename TO, int P>
+template <typename TS, typename TW, typename TO, int P, SlicesAtOnce HOW>
 __global__ __launch_bounds__(1024) void sandwich_norm_vec_kernel(float* __restrict__ residual, const TS* __restrict__ src,
                                                                  const TW* __restrict__ wa, const TW* __restrict__ wb,
                                                                  TO* __restrict__ out, int width, uint32_t how, uint32_t split_stride,
                                                                  float scale, const TW* __restrict__ ba, const TW* __restrict__ bb,
                                                                  const int32_t* __restrict__ rows, float eps_a, float eps_b) {
-  constexpr int SL = sizeof(TS) == 2 ? 1 : P == 1 ? 8 : 4;  // slices asked for at once
+  constexpr int SL = HOW == kFewRows ? 8 / P : slices_at_once<HOW, P>;  // slices asked for at once
   __shared__ float scratch[4][16];
   const int n_splits = how & 0xffffu, waves = (how >> 19) & 31, round_sum = (how & SN_ROUND) != 0;
   const size_t n = blockIdx.x;
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(1024) void sandwich_norm_vec_kernel(float* __restri
   }
   if (src != nullptr) {
     join_slices<SL, P, TS>(d, n_splits, br);
-    join_rest<SL, P, TS>(p, at, n_splits, split_stride, br);
+    if constexpr (HOW != kOneSlice) join_rest<SL, P, TS>(p, at, n_splits, split_stride, br);
 #pragma unroll
     for (int k = 0; k < P; ++k)
       br[k] = make_float4(as_output(br[k].x, round_sum), as_output(br[k].y, round_sum), as_output(br[k].z, round_sum),
@@ -217,19 +217,22 @@ extern "C" int yk_sandwich_norm(float* residual, const void* src, int src_dtype,
                    al(bb) && al(out) && n_splits < 1 << 16 && stride < size_t{1} << 32;
   // a piece a thread for few rows, two where rows fill the chip: eight rows of 4,096 11.1 -> 6.2 us, 2,048 rows of 2,048 24 -> 15 us
   // against 256 threads with up to four pieces each (whose slices were then added one round trip after the other)
-  const int pieces = n_rows >= 1024 ? 2 : 1;
-  const int threads = (width / 4 + 64 * pieces - 1) / (64 * pieces) * 64;
+  const int threads = n_rows >= 1024 ? (width / 4 + 127) / 128 * 64 : (width / 4 + 63) / 64 * 64, pieces = 4 * threads < width ? 2 : 1;
   const uint32_t how = static_cast<uint32_t>(n_splits & 0xffff) | (round_sum ? SN_ROUND : 0u) | (center_a ? SN_CENTER_A : 0u) |
                        (center_b ? SN_CENTER_B : 0u) | static_cast<uint32_t>(threads / 64) << 19 | (rows ? SN_ROWS : 0u) |
                        (wa && ba ? SN_BIAS_A : 0u) | (wb && bb ? SN_BIAS_B : 0u);
-#define YK_VEC(TS, TW, TO, P)                                                                                     \
-  sandwich_norm_vec_kernel<TS, TW, TO, P><<<n_rows, threads, 0, stream>>>(                                        \
+  const SlicesAtOnce at_once = slices_how(n_splits, n_rows);
+#define YK_VEC(TS, TW, TO, P, HOW)                                                                                \
+  sandwich_norm_vec_kernel<TS, TW, TO, P, (sizeof(TS) == 2 ? kOneSlice : HOW)><<<n_rows, threads, 0, stream>>>(                                        \
       residual, static_cast<const TS*>(src), static_cast<const TW*>(wa), static_cast<const TW*>(wb), static_cast<TO*>(out), width, how, \
       static_cast<uint32_t>(stride), scale, static_cast<const TW*>(ba), static_cast<const TW*>(bb), rows, eps_a, eps_b)
 #define YK_CASE(SD, TS, WD, TW, OD, TO)                                                                           \
   if ((src == nullptr || src_dtype == SD) && w_dtype == WD && (out == nullptr || out_dtype == OD)) {              \
-    if (vec && pieces == 1) YK_VEC(TS, TW, TO, 1);                                                                \
-    else if (vec && pieces == 2) YK_VEC(TS, TW, TO, 2);                                                           \
+    if (vec && pieces == 1 && at_once == kOneSlice) YK_VEC(TS, TW, TO, 1, kOneSlice);                             \
+    else if (vec && pieces == 1 && at_once == kManyRows) YK_VEC(TS, TW, TO, 1, kManyRows);                        \
+    else if (vec && pieces == 1) YK_VEC(TS, TW, TO, 1, kFewRows);                                                 \
+    else if (vec && at_once == kOneSlice) YK_VEC(TS, TW, TO, 2, kOneSlice);                                       \
+    else if (vec) YK_VEC(TS, TW, TO, 2, kManyRows); /* (1,024 rows and more) */                                   \
     else                                                                                                          \
     sandwich_norm_kernel<TS, TW, TO><<<n_rows, 256, lds, stream>>>(                                               \
         residual, static_cast<const TS*>(src), n_splits, stride, round_sum, static_cast<const TW*>(wa),           \
@@ -269,14 +272,14 @@ __global__ void activation_kernel(const TS* __restrict__ src, int n_splits, size
   }
 }
 
-// The same, four elements a thread and all its slices (up to 16) asked for at once (2,048 rows of 8,192: 39 -> 18 us).
-template <typename TS, typename TO>
+// The same, four elements a thread; all its slices (up to 16) asked for at once where the launch is small (2,048 rows of 8,192: 39 -> 18 us).
+template <typename TS, typename TO, SlicesAtOnce HOW>
 __global__ __launch_bounds__(256) void activation_vec_kernel(const TS* __restrict__ src, int n_splits, size_t split_stride, int round_sum, int kind,
                                                              TO* __restrict__ out, size_t pieces) {
   const size_t first = blockIdx.x * static_cast<size_t>(256);
   const uint32_t at[1] = {4 * static_cast<uint32_t>(min(static_cast<size_t>(threadIdx.x), pieces - 1 - first))};
   float4 v[1];
-  sum_slices<1, TS>(src + 4 * first, at, n_splits, split_stride, v);
+  sum_slices<HOW, 1, TS>(src + 4 * first, at, n_splits, split_stride, v);
   if (first + threadIdx.x < pieces)
     put_four<TO>(out + 4 * first + at[0], make_float4(act_plain(as_output(v[0].x, round_sum), kind), act_plain(as_output(v[0].y, round_sum), kind),
                                                       act_plain(as_output(v[0].z, round_sum), kind), act_plain(as_output(v[0].w, round_sum), kind)));
@@ -289,11 +292,14 @@ extern "C" int yk_activation(const void* src, int src_dtype, int n_splits, int r
   if (total == 0) return 0;
   const int grid = static_cast<int>(std::min<size_t>((total + 255) / 256, 1 << 20));
   const bool vec = total % 4 == 0 && total < (1ull << 40) && (reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+#define YK_VEC(TS, TO, HOW)                                                                                         \
+  activation_vec_kernel<TS, TO, HOW><<<(total / 4 + 255) / 256, 256, 0, stream>>>(                                 \
+      static_cast<const TS*>(src), n_splits, total, round_sum, kind, static_cast<TO*>(out), total / 4)
 #define YK_CASE(SD, TS, OD, TO)                                                                                    \
   if (src_dtype == SD && out_dtype == OD) {                                                                        \
-    if (vec)                                                                                                       \
-      activation_vec_kernel<TS, TO><<<(total / 4 + 255) / 256, 256, 0, stream>>>(                                  \
-          static_cast<const TS*>(src), n_splits, total, round_sum, kind, static_cast<TO*>(out), total / 4);        \
+    if (vec && n_splits == 1) YK_VEC(TS, TO, kOneSlice);                                                           \
+    else if (vec && total > 1 << 18) YK_VEC(TS, TO, (sizeof(TS) == 2 ? kOneSlice : kManyRows));                    \
+    else if (vec) YK_VEC(TS, TO, (sizeof(TS) == 2 ? kOneSlice : kFewRows));                                        \
     else                                                                                                           \
       activation_kernel<TS, TO><<<grid, 256, 0, stream>>>(static_cast<const TS*>(src), n_splits, total, round_sum, kind, \
                                                           static_cast<TO*>(out), total);                           \
@@ -303,6 +309,7 @@ extern "C" int yk_activation(const void* src, int src_dtype, int n_splits, int r
   YK_CASE(YK_F32, float, YK_BF16, bf16_t)
   YK_CASE(YK_BF16, bf16_t, YK_BF16, bf16_t)
 #undef YK_CASE
+#undef YK_VEC
   return yk_fail("activation: unsupported dtype combination");
 }
 
