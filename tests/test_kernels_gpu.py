@@ -297,6 +297,15 @@ def test_products_with_their_own_end_are_no_further_from_64_bits(ops, n, k):
     (8, 17576, 2048, True, False), (8, 17584, 2048, False, False), (8, 16384, 1024, True, False), (8, 16400, 1024, False, False),
     (8, 1040, 8192, True, False), (8, 1040, 8200, False, False), (4, 1040, 8200, True, False), (12, 1040, 6152, True, False), (13, 1040, 6152, False, False),
     (16, 2112, 6144, True, False), (16, 2120, 6144, False, False),
+    # beyond 6.5 M elements: a K of eight chunks, sides that are no square, rounds of the compute units, up to four rows and two
+    (8, 4096, 2040, True, False), (8, 4096, 2048, True, True), (9, 4096, 2048, True, False), (8, 4096, 2728, True, True), (8, 4096, 2736, True, False),
+    (8, 4096, 6136, False, False), (8, 4096, 6144, True, True), (8, 4096, 12288, True, True), (8, 4096, 12296, False, False), (9, 4096, 8192, False, False),
+    (8, 3584, 8192, False, False), (8, 3600, 8192, True, True), (8, 4112, 8192, False, False), (8, 7168, 4096, False, False), (8, 7184, 4096, True, True),
+    (8, 8192, 4096, True, True), (8, 8192, 4104, False, False), (8, 8208, 4096, False, False), (4, 2800, 8192, False, False), (4, 2816, 8192, True, True),
+    (5, 2816, 8192, False, False), (4, 3072, 14336, True, True), (4, 3072, 14344, False, False), (4, 8192, 8200, False, False), (4, 8192, 12296, True, True),
+    (4, 2048, 5632, True, True), (5, 2048, 5632, True, False), (4, 2048, 5640, True, False), (4, 2032, 5632, True, False),
+    (2, 2048, 8192, True, True), (3, 2048, 8192, False, False), (2, 2048, 8200, False, False), (2, 1024, 4096, True, True), (2, 1024, 4104, True, False),
+    (2, 14336, 2048, True, False), (2, 14352, 2048, True, True), (2, 16384, 2048, True, True), (3, 16384, 2048, True, False), (2, 16384, 2056, False, False),
 ])
 def test_where_products_have_their_own_end(ops, m, n, k, whole, handed_on):
     """Which of the two forms a product takes, told by the order of its sums, and the same value as the other up to that."""

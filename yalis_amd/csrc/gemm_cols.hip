@@ -183,11 +183,20 @@ static int g_mode = 0;
 // A workgroup of 16 columns reads x once for them, four times as often a column as the other form, and
 // ends with a barrier and a few sums: both count the more, the more rows x has and the more workgroups a compute unit runs one
 // after another; few columns are few workgroups, whose walk over a long K nothing divides further; and a second round that fills a part of
-// the units waits for the first.  So, where slices would do (handed_on): matrices of up to 6.5 M elements whose K and columns are not
-// far apart (1,024 x 4,096 at eight rows 9.5 / 10.0; one slice: 8,192 x 512 5.3 / 4.3, 12,288 x 512 5.5 / 5.7, 25,344 x 256 4.8 / 8.2);
-// larger ones whose workgroups make one or two whole rounds of the compute units; and with up to four and two rows those on whose
-// line above it is ahead.  Of the larger ones only those with one side half as long again as the other: square ones, where it is as far
-// ahead (the line of 4,096 x 4,096), come as slices, and a program that holds them while it launches another product of that size is told so.  Up to eight rows: at 16 the two are about even, and a product that takes attention's
+// the units waits for the first.  So, where slices would do (handed_on), up to eight rows:
+//   - matrices of up to 6.5 M elements whose K and columns are not far apart (1,024 x 4,096 at eight rows 9.5 / 10.0; one slice: 8,192 x 512
+//     5.3 / 4.3, 12,288 x 512 5.5 / 5.7, 25,344 x 256 4.8 / 8.2);
+//   - larger ones whose workgroups make one or two rounds of the compute units with an eighth of them idle or fewer (as above, slices / this: 4,112 x
+//     8,192 19.2 / 23.6, 8,208 x 4,096 20.2 / 21.6; 3,584 and 3,600 x 8,192 16.8 / 16.5 and 17.2 / 17.2, 7,168 and 7,680 x 4,096 17.2 / 17.5 and 18.1 / 17.8),
+//     up to where the two meet (4,096 x 11,008 22.9 / 21.2, 12,288 22.6 / 22.9, 13,312 23.7 / 23.8; 8,192 x 4,096 18.9 / 18.2, 4,864 20.1 / 20.7);
+//   - up to four rows as far as that line lies then (4,096 x 14,336 24.6 / 23.8, 16,384 26.8 / 27.0; 2,048 x 5,120 11.3 / 11.1, 5,888 11.7 / 11.7; between 2,560 and
+//     2,816 columns, and with five rows, it is 3 to 8 % ahead some way beyond); up to two rows (2,048 x 8,192 12.7 / 12.5, 9,216 13.6 / 13.6;
+//     1,024 x 4,096 9.1 / 8.7, 5,120 9.6 / 10.1; 16,384 x 2,048 20.2 / 18.4, 2,304 21.3 / 20.7);
+//   - of the larger ones only those with one side half as long again as the other.  That is no line of speed: square ones are ahead here too (one, four and
+//     eight rows: 3,072 x 3,072 11.0, 11.2, 11.4 / 9.1, 9.9, 10.4; 4,096 x 4,096 12.2, 12.7, 13.2 / 11.2, 11.6, 12.0; 4,096 x 6,136 16.4, 17.0, 17.4 / 14.0, 14.8, 15.7).
+//     It is the price of an interface: products of this shape come as slices in the library's workspace, and a program that holds them while
+//     it launches the next product is told so.
+// At 16 rows the two are about even, and a product that takes attention's
 // unmerged splits (which this form does not) has the bits of the one that takes them merged there.
 // Where a kernel would have to add the slices: also up to 13 M elements (36 M with up to 8 rows and a K of one round of eight waves) with a K
 // of up to 8,192 (6,144 from 13 rows on; any with up to four), but not a short K against many columns (with a
@@ -199,11 +208,14 @@ static bool handed_on(int M, int N, int K) {
   const long long elements = static_cast<long long>(N) * K;
   if (M <= 8 && elements <= 6500000 && K >= KC && (K <= 8 * KC || 2LL * K <= 3LL * N) && (N <= 8192 || N <= 16LL * K)) return true;
   if (M > 8 || K < 8 * KC || (2LL * K < 3LL * N && 2LL * N < 3LL * K)) return false;
-  const bool one_round = N > 3584 && N <= 4096, two_rounds = N > 7168 && N <= 8192;
+  constexpr int UNITS = 256;  // compute units, a workgroup of 16 columns each
+  const int tiles = (N + 15) / 16;
+  auto rounds = [&](int r) { return tiles > r * UNITS - r * UNITS / 8 && tiles <= r * UNITS; };
+  const bool one_round = rounds(1), two_rounds = rounds(2);
   if ((one_round && K <= 12288) || (two_rounds && K <= 4096)) return true;
   if (M <= 4 && (((N >= 2816 && N <= 4096) || two_rounds) && K <= 14336)) return true;
   if (M <= 4 && N >= 2048 && N < 2816 && K <= 5632) return true;
-  return M <= 2 && ((N <= 2048 && K <= 4LL * N) || (N > 14336 && N <= 16384 && K <= 8 * KC));
+  return M <= 2 && ((N <= 2048 && K <= 4LL * N) || (rounds(4) && K <= 8 * KC));
 }
 
 extern "C" int yk_gemm_cols_ok(int M, int N, int K, int slices_do) {

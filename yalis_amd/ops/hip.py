@@ -695,9 +695,9 @@ class HipOps:
         bfloat16 products of up to 16 rows run in one of two forms whose sums run in different orders (``gemm_cols`` and
         K slices).  Which of them may depend on what is asked for: where slices need a kernel of their own to add them, more
         sizes are ``gemm_cols``'s (``yk_gemm_cols_ok``).  A product has the same bits whole, as slices, with a bias added
-        afterwards or in ``gate_up_act`` where it is ``gemm_cols``'s even as slices (most products of up to 8 rows, 6.5 M elements
-        of w and 1,024 rows of w or more) and where it is never (fewer rows of w, more than 16 of x, large matrices); between
-        these only up to rounding.  More than 64 rows of bfloat16 are ``gemm_block``'s, ``gemm_tile``'s or the vendor library's by size
+        afterwards or in ``gate_up_act`` where it is ``gemm_cols``'s even as slices (up to 8 rows of x and 1,024 rows of w or more: most
+        matrices of up to 6.5 M elements, and larger ones that are not square and whose rows fill the compute units, up to 16,384 of them
+        and a K of 14,336) and where it is never (fewer rows of w, more than 16 of x, other large matrices); between these only up to rounding.  More than 64 rows of bfloat16 are ``gemm_block``'s, ``gemm_tile``'s or the vendor library's by size
         and by whether slices will do; float32 is ``gemm_fma``'s."""
         if bias is not None:
             if isinstance(x, torch.Tensor):
